@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define HSTU_BLOCK_ABI_VERSION 3
+#define HSTU_BLOCK_ABI_VERSION 4
 
 typedef enum HstuBlockStatus {
   HSTU_BLOCK_OK = 0,
@@ -68,6 +68,8 @@ typedef struct HstuNormGateArgs {
   int64_t a_stride, u_stride, out_stride;
   const void* gamma;
   const void* beta;
+  const int32_t* seq_offsets; /* or null.  Given: out is a padded batch [rows / L][L], sequence b's rows are those of `a` */
+  int32_t L, reserved0;       /* from row seq_offsets[b] on, rows past its end (seq_offsets[b + 1]) are zeros; no gate then */
 } HstuNormGateArgs;
 
 int hstu_norm_gate_fwd(const HstuNormGateArgs* args, void* stream);
@@ -104,6 +106,11 @@ typedef struct HstuNormGateBwdArgs {
   float* dbeta;
   void* workspace;
   size_t workspace_bytes;
+  const void* u_pre;          /* or null.  Given: u = silu(u_pre), and du is the gradient of u_pre (u's, rounded, times silu') */
+  int64_t u_pre_stride;
+  const void* add;            /* or null.  Given: added to the rounded da (a gradient that reaches `a` another way) */
+  int64_t add_stride;
+  const int32_t* row_map;     /* or null.  Given: row r of dout is at row row_map[r] of its buffer */
 } HstuNormGateBwdArgs;
 
 size_t hstu_norm_gate_bwd_workspace_bytes(int64_t rows, int32_t width);
@@ -164,9 +171,88 @@ typedef struct HstuEmbedNormArgs {
   const void* gamma;
   const void* beta;
   void* out;
+  const int32_t* row_map; /* or null.  Given: row r takes entry row_map[r] of ids (hstu_pack_plan) */
+  int32_t L;              /* with positions null and pos_table given: the position is that entry's index modulo L */
+  int32_t round_steps;    /* 1: the scaled row and the sum are each rounded to bf16 (what separate steps leave); 0: one rounding */
 } HstuEmbedNormArgs;
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* args, void* stream);
+/* Its gradients for the gradient g->dout of its result: g->da, the gradient of the summed rows x_t (bf16 [rows, width]), and
+ * g->dgamma, g->dbeta; of `g` only those, dout's and da's strides and the workspace are read, of `a` everything but out.
+ * row_map applies to the gather, not to dout. */
+int hstu_embed_norm_bwd(const HstuEmbedNormArgs* a, const HstuNormGateBwdArgs* g, void* stream);
+
+/* The gradient of a gathered table, all of it: out[v, :] = the sum of scale * g[t, :] over the rows t whose key is v, added in the
+ * order of the rows with every term and partial sum rounded to bf16 (the bits of torch's gather backward; rows of up to 64
+ * elements: partial sums in fp32); zeros for keys without a row.  The key is the id (or position) as hstu_embed_norm_fwd finds it, clamped
+ * into [0, keys).  out: bf16 [keys, width] contiguous. */
+typedef struct HstuEmbedGradArgs {
+  uint32_t struct_size;   /* sizeof(HstuEmbedGradArgs) */
+  uint32_t version;       /* HSTU_BLOCK_ABI_VERSION    */
+  int64_t rows, keys;
+  int32_t width;
+  float scale;
+  const void* g;
+  int64_t g_stride;
+  const int64_t* ids;
+  const int64_t* positions;
+  const int32_t* row_map;
+  int32_t L, by_position; /* by_position: the keys are positions (positions, or the entry's index modulo L) */
+  void* out;
+  void* workspace;
+  size_t workspace_bytes;
+} HstuEmbedGradArgs;
+
+size_t hstu_embed_grad_workspace_bytes(int64_t rows, int64_t keys, int32_t width);
+int hstu_embed_grad(const HstuEmbedGradArgs* args, void* stream);
+
+/* Packing a padded batch [B, L] of the given lengths (int32 or int64 [B], clamped to [0, L]): seq_offsets int32 [B + 1],
+ * row_map int32 [B L] (its first *total entries: the padded row of each packed token), total: one int32 that the device can
+ * write (pinned host memory will do). */
+int hstu_pack_plan(const void* lens, int32_t lens_are_64bit, int32_t B, int32_t L, int32_t* seq_offsets, int32_t* row_map, int32_t* total, void* stream);
+/* Lengths of an end-padded batch from its byte mask [B, L]; *bad becomes 1 when a row is not non-zero bytes followed by zeros
+ * (and stays as it was otherwise). */
+int hstu_mask_lengths(const uint8_t* mask, int32_t B, int32_t L, int32_t* lens, int32_t* bad, void* stream);
+/* d[r, :] *= silu'(pre[r, :]) in place, bf16 rows of `width` elements. */
+int hstu_silu_bwd(void* d, int64_t d_stride, const void* pre, int64_t pre_stride, int64_t rows, int32_t width, void* stream);
+
+/* The block's matrix products without a library: bf16 operands, fp32 accumulation, one rounding.
+ *   HSTU_GEMM_NN   out[M, N] = act(x[M, K] w[K, N] + c + bias)    a projection (recml/layers/keras/hstu.py:444-449, 473-474)
+ *   HSTU_GEMM_NT   out[M, K] = x[M, N] w[K, N]^T                  the gradient of its input
+ *   HSTU_GEMM_TN   w[K, N]   = x[M, K]^T y[M, N]                  the gradient of its weight (w written)
+ * The weight comes as `slabs` matrices [K, N / slabs], contiguous each, side by side along N (the U, Q, K and V kernels
+ * of a block); the other operands are single matrices with a row stride.  NN: bias [N], c [M, N] (row stride c_stride) and
+ * `pre` (bf16 [M, N] contiguous: the value before the activation, which then applies to the rounded value) may be null; out is contiguous.
+ * N, K, N / slabs and the row strides multiples of 8, pointers 16-byte aligned.  TN sums a long M in parts: `workspace`
+ * of hstu_gemm_workspace_bytes(op, M, N, K) bytes, owned by the caller; the parts are added in a fixed order. */
+#define HSTU_GEMM_NN 0
+#define HSTU_GEMM_NT 1
+#define HSTU_GEMM_TN 2
+#define HSTU_GEMM_MAX_SLABS 4
+typedef struct HstuGemmArgs {
+  uint32_t struct_size;   /* sizeof(HstuGemmArgs)      */
+  uint32_t version;       /* HSTU_BLOCK_ABI_VERSION    */
+  int32_t op;
+  int32_t activation;     /* NN: 1 = silu, 0 = none */
+  int64_t M;
+  int32_t N, K;
+  int32_t slabs, reserved0;
+  const void* x;
+  int64_t x_stride;
+  const void* w[HSTU_GEMM_MAX_SLABS];
+  const void* y;
+  int64_t y_stride;
+  const void* bias;
+  const void* c;
+  int64_t c_stride;
+  void* out;
+  void* pre;
+  void* workspace;
+  size_t workspace_bytes;
+} HstuGemmArgs;
+
+size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K);
+int hstu_gemm(const HstuGemmArgs* args, void* stream);
 
 int hstu_block_abi_version(void);
 const char* hstu_block_last_error(void);

@@ -9,7 +9,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("RECML_AMD_BLOCK_LIB") or os.path.join(_HERE, "lib", "libhstu_block.so")
 
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 EXPORTS = (
     "hstu_block_abi_version",
@@ -20,6 +20,14 @@ EXPORTS = (
     "hstu_gemm_silu_fwd",
     "hstu_gemm_silu_workspace_bytes",
     "hstu_embed_norm_fwd",
+    "hstu_embed_norm_bwd",
+    "hstu_embed_grad",
+    "hstu_embed_grad_workspace_bytes",
+    "hstu_pack_plan",
+    "hstu_mask_lengths",
+    "hstu_silu_bwd",
+    "hstu_gemm",
+    "hstu_gemm_workspace_bytes",
 )
 
 
@@ -32,6 +40,7 @@ class HstuNormGateArgs(C.Structure):
       ("a", C.c_void_p), ("u", C.c_void_p), ("out", C.c_void_p),
       ("a_stride", C.c_int64), ("u_stride", C.c_int64), ("out_stride", C.c_int64),
       ("gamma", C.c_void_p), ("beta", C.c_void_p),
+      ("seq_offsets", C.c_void_p), ("L", C.c_int32), ("reserved0", C.c_int32),
   ]
 
 
@@ -46,6 +55,8 @@ class HstuNormGateBwdArgs(C.Structure):
       ("da_stride", C.c_int64), ("du_stride", C.c_int64),
       ("gamma", C.c_void_p), ("beta", C.c_void_p), ("dgamma", C.c_void_p), ("dbeta", C.c_void_p),
       ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
+      ("u_pre", C.c_void_p), ("u_pre_stride", C.c_int64), ("add", C.c_void_p), ("add_stride", C.c_int64),
+      ("row_map", C.c_void_p),
   ]
 
 
@@ -63,6 +74,25 @@ class HstuGemmSiluArgs(C.Structure):
   ]
 
 
+class HstuGemmArgs(C.Structure):
+  """Field-for-field image of `struct HstuGemmArgs`."""
+
+  _fields_ = [
+      ("struct_size", C.c_uint32), ("version", C.c_uint32),
+      ("op", C.c_int32), ("activation", C.c_int32),
+      ("M", C.c_int64), ("N", C.c_int32), ("K", C.c_int32),
+      ("slabs", C.c_int32), ("reserved0", C.c_int32),
+      ("x", C.c_void_p), ("x_stride", C.c_int64), ("w", C.c_void_p * 4),
+      ("y", C.c_void_p), ("y_stride", C.c_int64),
+      ("bias", C.c_void_p), ("c", C.c_void_p), ("c_stride", C.c_int64),
+      ("out", C.c_void_p), ("pre", C.c_void_p),
+      ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
+  ]
+
+
+GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2
+
+
 class HstuEmbedNormArgs(C.Structure):
   """Field-for-field image of `struct HstuEmbedNormArgs`."""
 
@@ -74,6 +104,20 @@ class HstuEmbedNormArgs(C.Structure):
       ("vocab", C.c_int64), ("table_stride", C.c_int64),
       ("positions", C.c_void_p), ("pos_table", C.c_void_p), ("n_positions", C.c_int64),
       ("gamma", C.c_void_p), ("beta", C.c_void_p), ("out", C.c_void_p),
+      ("row_map", C.c_void_p), ("L", C.c_int32), ("round_steps", C.c_int32),
+  ]
+
+
+class HstuEmbedGradArgs(C.Structure):
+  """Field-for-field image of `struct HstuEmbedGradArgs`."""
+
+  _fields_ = [
+      ("struct_size", C.c_uint32), ("version", C.c_uint32),
+      ("rows", C.c_int64), ("keys", C.c_int64), ("width", C.c_int32), ("scale", C.c_float),
+      ("g", C.c_void_p), ("g_stride", C.c_int64),
+      ("ids", C.c_void_p), ("positions", C.c_void_p), ("row_map", C.c_void_p),
+      ("L", C.c_int32), ("by_position", C.c_int32),
+      ("out", C.c_void_p), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
   ]
 
 
@@ -107,6 +151,10 @@ def load():
     lib.hstu_gemm_silu_fwd.argtypes = [C.POINTER(HstuGemmSiluArgs), C.c_void_p]
     lib.hstu_gemm_silu_workspace_bytes.restype = C.c_size_t
     lib.hstu_gemm_silu_workspace_bytes.argtypes = []
+    lib.hstu_gemm.restype = C.c_int
+    lib.hstu_gemm.argtypes = [C.POINTER(HstuGemmArgs), C.c_void_p]
+    lib.hstu_gemm_workspace_bytes.restype = C.c_size_t
+    lib.hstu_gemm_workspace_bytes.argtypes = [C.c_int32, C.c_int64, C.c_int32, C.c_int32]
     lib.hstu_embed_norm_fwd.restype = C.c_int
     lib.hstu_embed_norm_fwd.argtypes = [C.POINTER(HstuEmbedNormArgs), C.c_void_p]
     ver = lib.hstu_block_abi_version()

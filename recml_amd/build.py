@@ -13,12 +13,16 @@ LIB_PATH = os.path.join(LIB_DIR, "libhstu_attn.so")
 SOURCES = [os.path.join(_HERE, "csrc", "hstu_attn.hip")]
 # the block-side steps live in a library of their own: they bring hipBLASLt along, the attention does not
 BLOCK_LIB_PATH = os.path.join(LIB_DIR, "libhstu_block.so")
-BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip")]
+BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip"), os.path.join(_HERE, "csrc", "hstu_gemm.hip")]
 BLOCK_LINK = ["-lhipblaslt"]
 INCLUDE = os.path.join(ROOT, "include")
 # the block's microbenchmark: a stand-alone program (its own main), evidence for what bounds the kernel
 MICRO_PATH = os.path.join(LIB_DIR, "micro_fwd_stream")
 MICRO_SOURCES = [os.path.join(_HERE, "csrc", "micro_fwd_stream.hip")]
+
+# the native host side: a Python extension module over both libraries
+NATIVE_PATH = os.path.join(LIB_DIR, "_native.so")
+NATIVE_SOURCES = [os.path.join(_HERE, "csrc", "native.cpp")]
 
 # -packed-fp32-ops is switched off for the device pass: packed fp32
 # instructions are not wanted in these kernels.  The host pass does not know
@@ -59,6 +63,26 @@ def build_block_library(verbose: bool = False) -> str:
   return _compile(BLOCK_SOURCES, BLOCK_LIB_PATH, BLOCK_LINK, verbose=verbose)
 
 
+def build_native(verbose: bool = False) -> str:
+  """Compiles the native host side into recml_amd/lib/_native.so (host code only; links the two libraries above)."""
+  import sysconfig
+  import torch
+  troot = os.path.dirname(torch.__file__)
+  tinc = os.path.join(troot, "include")
+  tmp = NATIVE_PATH + ".tmp"
+  cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", INCLUDE,
+         "-I", tinc, "-I", os.path.join(tinc, "torch", "csrc", "api", "include"), "-I", "/opt/rocm/include",
+         "-I", sysconfig.get_paths()["include"], "-o", tmp, *NATIVE_SOURCES, "-L", LIB_DIR, "-l:libhstu_attn.so", "-l:libhstu_block.so",
+         "-L", os.path.join(troot, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+  res = subprocess.run(cmd, capture_output=True, text=True)
+  if res.returncode != 0:
+    raise RuntimeError("g++ failed:\n" + res.stdout + res.stderr)
+  if verbose:
+    print(res.stderr)
+  os.replace(tmp, NATIVE_PATH)
+  return NATIVE_PATH
+
+
 def build_microbench(verbose: bool = False) -> str:
   """Compiles the forward block's microbenchmark into recml_amd/lib/micro_fwd_stream (an executable)."""
   os.makedirs(LIB_DIR, exist_ok=True)
@@ -77,4 +101,5 @@ def build_microbench(verbose: bool = False) -> str:
 if __name__ == "__main__":
   print(build_library(verbose=True))
   print(build_block_library(verbose=True))
+  print(build_native(verbose=True))
   print(build_microbench(verbose=True))

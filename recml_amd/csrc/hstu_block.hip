@@ -26,16 +26,13 @@
 #include <tuple>
 
 #include "hstu_block.h"
+#include "hstu_block_common.h"
 
 namespace {
-
-typedef __bf16 bf16_t;
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
 thread_local char g_err[512] = "";
+}
 
-int fail(int code, const char* fmt, ...) {
+int block_fail(int code, const char* fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
@@ -43,26 +40,19 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
-__device__ __forceinline__ void unpack8(const uint4& v, float (&f)[8]) {
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = __builtin_bit_cast(float, w[i] << 16);
-    f[2 * i + 1] = __builtin_bit_cast(float, w[i] & 0xffff0000u);
-  }
+int block_allow_lds(const void* fn, int bytes, int* granted) {
+  constexpr int kMaxDev = 64;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(e));
+  if (dev >= 0 && dev < kMaxDev && __atomic_load_n(&granted[dev], __ATOMIC_ACQUIRE) >= bytes) return HSTU_BLOCK_OK;
+  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes of LDS): %s", bytes, hipGetErrorString(e));
+  if (dev >= 0 && dev < kMaxDev) __atomic_store_n(&granted[dev], bytes, __ATOMIC_RELEASE);
+  return HSTU_BLOCK_OK;
 }
 
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  floatx2 f = {lo, hi};
-  bf16x2 r = __builtin_convertvector(f, bf16x2);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-  return v;
-}
+namespace {
 
 struct NormGateParams {
   const bf16_t* a;
@@ -71,24 +61,43 @@ struct NormGateParams {
   const bf16_t* gamma;
   const bf16_t* beta;
   int64_t rows, a_stride, u_stride, out_stride;
+  // out is a padded batch [rows / L][L] whose sequence b starts at row seq_offsets[b] of `a`; rows past a sequence's end
+  // are zeros (null: row r of `a` is row r of `out`)
+  const int32_t* seq_offsets;
+  int32_t L;
   int32_t width;
   float eps;
 };
 
-// One wavefront per row; lane l owns the 8-element pieces l, l + 64, ... of the row (CH of them at most).
-template <int CH>
+// LPR lanes per row (a row of up to 64, 128, 256 elements takes 8, 16, 32 lanes, so that a wavefront holds 8, 4, 2 of them;
+// longer ones a whole wavefront); lane l of a row owns its 8-element pieces l, l + LPR, ... (CH of them at most).
+template <int CH, int LPR>
 __global__ __launch_bounds__(256) void hstu_norm_gate(const NormGateParams p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int RPW = 64 / LPR;
+  const int lane = threadIdx.x & (LPR - 1);
+  const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + ((threadIdx.x & 63) / LPR);
   if (row >= p.rows) return;
-  const bf16_t* ar = p.a + row * p.a_stride;
-  const bf16_t* ur = p.u ? p.u + row * p.u_stride : nullptr;   // no gate: the plain layer norm
+  int64_t src = row;
   bf16_t* orow = p.out + row * p.out_stride;
+  if (p.seq_offsets) {
+    const int b = (int)(row / p.L), i = (int)(row - (int64_t)b * p.L), o0 = p.seq_offsets[b];
+    src = o0 + i;
+    if (i >= p.seq_offsets[b + 1] - o0) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int e = (c * LPR + lane) * 8;
+        if (e < p.width) *(uint4*)(orow + e) = uint4{0u, 0u, 0u, 0u};
+      }
+      return;
+    }
+  }
+  const bf16_t* ar = p.a + src * p.a_stride;
+  const bf16_t* ur = p.u ? p.u + row * p.u_stride : nullptr;   // no gate: the plain layer norm
   float x[CH][8];
   float sum = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
       unpack8(*(const uint4*)(ar + e), x[c]);
 #pragma unroll
@@ -98,11 +107,11 @@ __global__ __launch_bounds__(256) void hstu_norm_gate(const NormGateParams p) {
       for (int i = 0; i < 8; ++i) x[c][i] = 0.f;
     }
   }
-  const float mean = wave_sum(sum) / (float)p.width;
+  const float mean = group_sum<LPR>(sum) / (float)p.width;
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -111,10 +120,10 @@ __global__ __launch_bounds__(256) void hstu_norm_gate(const NormGateParams p) {
       }
     }
   }
-  const float rstd = __builtin_amdgcn_rsqf(wave_sum(ss) / (float)p.width + p.eps);
+  const float rstd = __builtin_amdgcn_rsqf(group_sum<LPR>(ss) / (float)p.width + p.eps);
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
       float g[8], b[8], uu[8];
       unpack8(*(const uint4*)(p.gamma + e), g);
@@ -128,12 +137,7 @@ __global__ __launch_bounds__(256) void hstu_norm_gate(const NormGateParams p) {
       float y[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) y[i] = uu[i] * __builtin_fmaf((x[c][i] - mean) * rstd, g[i], b[i]);
-      uint4 o;
-      o.x = pack2(y[0], y[1]);
-      o.y = pack2(y[2], y[3]);
-      o.z = pack2(y[4], y[5]);
-      o.w = pack2(y[6], y[7]);
-      *(uint4*)(orow + e) = o;
+      *(uint4*)(orow + e) = pack8(y);
     }
   }
 }
@@ -147,7 +151,19 @@ struct NormGateBwdParams {
   bf16_t* da;
   bf16_t* du;
   float* partial;          // [gridDim.x][2 * width]: each workgroup's sums for dgamma, then for dbeta
-  int64_t rows, a_stride, u_stride, dout_stride, da_stride, du_stride;
+  const bf16_t* u_pre;     // u = silu(u_pre), and du is the gradient of u_pre; or null
+  const bf16_t* add;       // added to da (the gradient that reaches `a` past the norm); or null
+  const int32_t* row_map;  // row r of dout is row row_map[r] of the buffer; or null
+  // a = scale * table[ids[r]] + pos_table[row % L] instead of rows of `a` (the model's front end; a is null then); r = the
+  // row, or row_map's entry for it, which then does not apply to dout
+  const int64_t* ids;
+  const int64_t* positions;
+  const bf16_t* table;
+  const bf16_t* pos_table;
+  int64_t vocab, table_stride, n_positions;
+  float scale;
+  int32_t L, round_steps;
+  int64_t rows, a_stride, u_stride, dout_stride, da_stride, du_stride, u_pre_stride, add_stride;
   int32_t width;
   float eps;
 };
@@ -156,32 +172,56 @@ struct NormGateBwdParams {
 //   du = g * (gamma * xhat + beta),  gn = g * u  (the gradient at the normalised row; gn = g without a gate)
 //   dgamma += gn * xhat,  dbeta += gn           (summed over the rows)
 //   da = rstd * (gn gamma - mean_w(gn gamma) - xhat * mean_w(gn gamma xhat))
-// One wavefront per row as in the forward, a workgroup walking over rows with the grid's stride: the row,
+// Rows on lanes as in the forward, a workgroup walking over rows with the grid's stride: the row,
 // its gradient and the gate are read once, da and du written once (5 x width x 2 bytes per row, the
 // bound).  The two column sums stay in registers over a wave's rows, are added across the workgroup's
 // four waves through LDS and leave as one partial row per workgroup; hstu_colsum adds those in a fixed
 // order, so the result does not depend on the timing of the run.
-template <int CH>
+// EMB: the rows are the front end's gathered ones.
+template <int CH, int LPR, bool EMB>
 __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParams p) {
-  __shared__ float red[4][CH * 512];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __shared__ float red[4][CH * LPR * 8];
+  constexpr int RPW = 64 / LPR;
+  const int lane = threadIdx.x & (LPR - 1), w = threadIdx.x >> 6;
   const float inv_w = 1.f / (float)p.width;
   float dg[CH][8], db[CH][8];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
 #pragma unroll
     for (int i = 0; i < 8; ++i) dg[c][i] = db[c][i] = 0.f;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + w; row < p.rows; row += (int64_t)gridDim.x * 4) {
-    const bf16_t* ar = p.a + row * p.a_stride;
-    const bf16_t* gr = p.dout + row * p.dout_stride;
+  for (int64_t row = ((int64_t)blockIdx.x * 4 + w) * RPW + ((threadIdx.x & 63) / LPR); row < p.rows; row += (int64_t)gridDim.x * 4 * RPW) {
+    const bf16_t *ar = nullptr, *pr = nullptr;
+    int64_t grow = row;
+    if constexpr (EMB) {
+      const int64_t at = p.row_map ? p.row_map[row] : row;
+      int64_t id = p.ids[at];
+      id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
+      ar = p.table + id * p.table_stride;
+      if (p.pos_table) {
+        int64_t ps = p.positions ? p.positions[row] : at % p.L;
+        ps = ps < 0 ? 0 : (ps >= p.n_positions ? p.n_positions - 1 : ps);
+        pr = p.pos_table + ps * (int64_t)p.width;
+      }
+    } else {
+      ar = p.a + row * p.a_stride;
+      if (p.row_map) grow = p.row_map[row];
+    }
+    const bf16_t* gr = p.dout + grow * p.dout_stride;
     float x[CH][8], g[CH][8];
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int e = (c * 64 + lane) * 8;
+      const int e = (c * LPR + lane) * 8;
       if (e < p.width) {
         unpack8(*(const uint4*)(ar + e), x[c]);
         unpack8(*(const uint4*)(gr + e), g[c]);
+        if constexpr (EMB) {
+          float pe[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          if (pr) unpack8(*(const uint4*)(pr + e), pe);
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            x[c][i] = p.round_steps ? round_bf16(round_bf16(x[c][i] * p.scale) + pe[i]) : __builtin_fmaf(x[c][i], p.scale, pe[i]);
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) sum += x[c][i];
       } else {
@@ -189,11 +229,11 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
         for (int i = 0; i < 8; ++i) x[c][i] = g[c][i] = 0.f;
       }
     }
-    const float mean = wave_sum(sum) * inv_w;
+    const float mean = group_sum<LPR>(sum) * inv_w;
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int e = (c * 64 + lane) * 8;
+      const int e = (c * LPR + lane) * 8;
       if (e < p.width) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -202,11 +242,11 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
         }
       }
     }
-    const float rstd = __builtin_amdgcn_rsqf(wave_sum(ss) * inv_w + p.eps);
+    const float rstd = __builtin_amdgcn_rsqf(group_sum<LPR>(ss) * inv_w + p.eps);
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int e = (c * 64 + lane) * 8;
+      const int e = (c * LPR + lane) * 8;
       if (e < p.width) {
         float gm[8];
         unpack8(*(const uint4*)(p.gamma + e), gm);
@@ -219,12 +259,13 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
             y[i] = g[c][i] * __builtin_fmaf((x[c][i] - mean) * rstd, gm[i], bt[i]);
             g[c][i] *= uu[i];
           }
-          uint4 o;
-          o.x = pack2(y[0], y[1]);
-          o.y = pack2(y[2], y[3]);
-          o.z = pack2(y[4], y[5]);
-          o.w = pack2(y[6], y[7]);
-          *(uint4*)(p.du + row * p.du_stride + e) = o;
+          if (p.u_pre) {
+            float z[8];
+            unpack8(*(const uint4*)(p.u_pre + row * p.u_pre_stride + e), z);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = round_bf16(y[i]) * silu_grad(z[i]);     // (du in bf16, as the attention's dq, dk, dv are)
+          }
+          *(uint4*)(p.du + row * p.du_stride + e) = pack8(y);
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -240,21 +281,22 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
         }
       }
     }
-    const float c1 = wave_sum(s1) * inv_w, c2 = wave_sum(s2) * inv_w;
+    const float c1 = group_sum<LPR>(s1) * inv_w, c2 = group_sum<LPR>(s2) * inv_w;
     bf16_t* dr = p.da + row * p.da_stride;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int e = (c * 64 + lane) * 8;
+      const int e = (c * LPR + lane) * 8;
       if (e < p.width) {
         float y[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) y[i] = rstd * (g[c][i] - c1 - x[c][i] * c2);
-        uint4 o;
-        o.x = pack2(y[0], y[1]);
-        o.y = pack2(y[2], y[3]);
-        o.z = pack2(y[4], y[5]);
-        o.w = pack2(y[6], y[7]);
-        *(uint4*)(dr + e) = o;
+        if (!EMB && p.add) {
+          float more[8];
+          unpack8(*(const uint4*)(p.add + row * p.add_stride + e), more);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) y[i] = round_bf16(y[i]) + more[i];      // (each share a bf16 gradient of its own)
+        }
+        *(uint4*)(dr + e) = pack8(y);
       }
     }
   }
@@ -265,7 +307,13 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
 #pragma unroll
     for (int c = 0; c < CH; ++c)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) red[w][(c * 64 + lane) * 8 + i] = half == 0 ? dg[c][i] : db[c][i];
+      for (int i = 0; i < 8; ++i) {
+        float v = half == 0 ? dg[c][i] : db[c][i];
+        // (the row groups of a wave hold the same columns)
+#pragma unroll
+        for (int d = 32; d >= LPR; d >>= 1) v += __shfl_xor(v, d, 64);
+        if ((threadIdx.x & 63) < LPR) red[w][(c * LPR + lane) * 8 + i] = v;
+      }
     __syncthreads();
     for (int col = threadIdx.x; col < p.width; col += 256)
       part[half * p.width + col] = (red[0][col] + red[1][col]) + (red[2][col] + red[3][col]);
@@ -304,9 +352,12 @@ __global__ __launch_bounds__(1024) void hstu_colsum(const float* __restrict__ pa
   }
 }
 
+// lanes per row of the norm kernels
+int lanes_per_row(int width) { return width <= 64 ? 8 : width <= 128 ? 16 : width <= 256 ? 32 : 64; }
+
 // workgroups of the backward kernel for this many rows (each walks over rows with the grid's stride)
-int norm_gate_bwd_blocks(int64_t rows) {
-  const int64_t nb = (rows + 3) / 4;
+int norm_gate_bwd_blocks(int64_t rows, int width) {
+  const int64_t per = 4 * (64 / lanes_per_row(width)), nb = (rows + per - 1) / per;
   return (int)(nb < 1 ? 1 : (nb > 1024 ? 1024 : nb));
 }
 
@@ -318,24 +369,29 @@ struct EmbedNormParams {
   const bf16_t* gamma;
   const bf16_t* beta;
   bf16_t* out;
+  const int32_t* row_map;  // token r takes entry row_map[r] of ids (its row in the padded batch), or null: entry r
+  int32_t L;               // with positions null: the position is that entry's index modulo L
   int64_t rows, vocab, table_stride, n_positions;
   int32_t width;
   float eps, scale;
+  int32_t round_steps;     // the scaled row and the sum are each rounded to bf16, as separate steps would leave them
 };
 
-// One wavefront per token: its table row (and position row) is gathered into registers, normalised
+// Rows on lanes as in hstu_norm_gate: a token's table row (and position row) is gathered into registers, normalised
 // there and written once.
-template <int CH>
+template <int CH, int LPR>
 __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int RPW = 64 / LPR;
+  const int lane = threadIdx.x & (LPR - 1);
+  const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + ((threadIdx.x & 63) / LPR);
   if (row >= p.rows) return;
-  int64_t id = p.ids[row];
+  const int64_t at = p.row_map ? p.row_map[row] : row;
+  int64_t id = p.ids[at];
   id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
   const bf16_t* er = p.table + id * p.table_stride;
   const bf16_t* pr = nullptr;
   if (p.pos_table) {
-    int64_t ps = p.positions[row];
+    int64_t ps = p.positions ? p.positions[row] : at % p.L;
     ps = ps < 0 ? 0 : (ps >= p.n_positions ? p.n_positions - 1 : ps);
     pr = p.pos_table + ps * (int64_t)p.width;
   }
@@ -343,18 +399,14 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
   float sum = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
       unpack8(*(const uint4*)(er + e), x[c]);
-      if (pr) {
-        float pe[8];
-        unpack8(*(const uint4*)(pr + e), pe);
+      float pe[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (pr) unpack8(*(const uint4*)(pr + e), pe);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[c][i] = __builtin_fmaf(x[c][i], p.scale, pe[i]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[c][i] *= p.scale;
-      }
+      for (int i = 0; i < 8; ++i)
+        x[c][i] = p.round_steps ? round_bf16(round_bf16(x[c][i] * p.scale) + pe[i]) : __builtin_fmaf(x[c][i], p.scale, pe[i]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) sum += x[c][i];
     } else {
@@ -362,11 +414,11 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
       for (int i = 0; i < 8; ++i) x[c][i] = 0.f;
     }
   }
-  const float mean = wave_sum(sum) / (float)p.width;
+  const float mean = group_sum<LPR>(sum) / (float)p.width;
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -375,28 +427,361 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
       }
     }
   }
-  const float rstd = __builtin_amdgcn_rsqf(wave_sum(ss) / (float)p.width + p.eps);
+  const float rstd = __builtin_amdgcn_rsqf(group_sum<LPR>(ss) / (float)p.width + p.eps);
   bf16_t* orow = p.out + row * (int64_t)p.width;
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int e = (c * 64 + lane) * 8;
+    const int e = (c * LPR + lane) * 8;
     if (e < p.width) {
       float g[8], b[8], y[8];
       unpack8(*(const uint4*)(p.gamma + e), g);
       unpack8(*(const uint4*)(p.beta + e), b);
 #pragma unroll
       for (int i = 0; i < 8; ++i) y[i] = __builtin_fmaf((x[c][i] - mean) * rstd, g[i], b[i]);
-      uint4 o;
-      o.x = pack2(y[0], y[1]);
-      o.y = pack2(y[2], y[3]);
-      o.z = pack2(y[4], y[5]);
-      o.w = pack2(y[6], y[7]);
-      *(uint4*)(orow + e) = o;
+      *(uint4*)(orow + e) = pack8(y);
     }
   }
 }
 
-bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+// ---- a batch's packing --------------------------------------------------
+
+// Where the tokens of a padded batch go when it is packed: offsets[b] = the sum of the lengths before b, row_map[t] = the
+// padded row b L + i of packed token t, total = the number of tokens.  One workgroup per sequence; each adds up the lengths
+// before its own (B of them: at most a few loads per thread).
+template <typename T>
+__global__ __launch_bounds__(256) void hstu_pack_plan_kernel(const T* __restrict__ lens, int B, int L, int32_t* __restrict__ offsets,
+                                                      int32_t* __restrict__ row_map, int32_t* __restrict__ total) {
+  __shared__ int part[4];
+  const int b = blockIdx.x, tid = threadIdx.x;
+  auto len = [&](int x) {
+    const int64_t n = (int64_t)lens[x];
+    return (int)(n < 0 ? 0 : (n > L ? L : n));
+  };
+  int sum = 0;
+  for (int x = tid; x < b; x += 256) sum += len(x);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+  if ((tid & 63) == 0) part[tid >> 6] = sum;
+  __syncthreads();
+  const int off = part[0] + part[1] + part[2] + part[3], n = len(b);
+  if (tid == 0) {
+    offsets[b] = off;
+    if (b == B - 1) {
+      offsets[B] = off + n;
+      *total = off + n;
+    }
+  }
+  for (int i = tid; i < n; i += 256) row_map[off + i] = b * L + i;
+}
+
+// Lengths of an end-padded batch from its mask (bytes, one row per wavefront); *bad is raised by a row that is not a
+// run of non-zero bytes followed by zeros.
+__global__ __launch_bounds__(256) void hstu_mask_lengths_kernel(const uint8_t* __restrict__ mask, int B, int L, int32_t* __restrict__ lens,
+                                                         int32_t* __restrict__ bad) {
+  const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (b >= B) return;
+  const uint8_t* row = mask + (int64_t)b * L;
+  int n = 0, last = -1;
+  for (int i = lane; i < L; i += 64) {
+    const bool on = row[i] != 0;
+    n += on ? 1 : 0;
+    last = on ? i : last;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    n += __shfl_xor(n, d, 64);
+    const int o = __shfl_xor(last, d, 64);
+    last = last > o ? last : o;
+  }
+  if (lane == 0) {
+    lens[b] = n;
+    if (last + 1 != n) *bad = 1;
+  }
+}
+
+// ---- gradients of the embedding tables ----------------------------------
+
+// The gradient of rows gathered from a table: out[v] = the sum of scale * g[t] over the tokens t with key(t) = v, v in [0, V), and
+// zeros for the others.  Keys are ids (clamped like the gather) or, with L, positions.  The terms of a key are added in the order
+// of the tokens and every partial sum is rounded to bf16 (rows of up to 64 elements: kept in fp32): the arithmetic of torch's
+// gather backward, whose kernel did this before (one wavefront per 32 table columns' run of tokens, reading and writing the sum in memory
+// for every token: 3.5 ms of a training step of 78 k tokens over 100 k popular and unpopular items, and as much for the positions).
+//   A popular key has thousands of tokens and most have none or one.  The tokens are put in order by key (counted, room reserved
+// per key, placed: no sort of the whole), a key's run is put in order by token, and the runs are summed in registers: short ones by
+// one wavefront each, long ones by one wavefront per 128 columns with 64 rows in flight (the chain of additions is 20 cycles a
+// row, the memory latency behind it over a thousand).
+constexpr int EG_SHORT = 32;         // tokens of a run that one wavefront orders and sums by itself
+constexpr int EG_WINDOW = 1 << 19;   // tokens whose bits fit the LDS of the ordering of a long run
+struct EmbedGradParams {
+  const bf16_t* g;
+  bf16_t* out;
+  const int64_t* ids;
+  const int64_t* positions;
+  const int32_t* row_map;
+  int64_t T, V, g_stride, out_stride;
+  int32_t L, width, by_position;
+  float scale;
+  int32_t* count;      // [V]: tokens of a key, then where its run starts
+  int32_t* rank;       // [T]: a token's place in its run
+  int32_t* order;      // [T]: tokens by key
+  int32_t* heads;      // [4]: tokens placed, short runs, long runs
+  int4* shorts;        // {key, first place, tokens, -}
+  int4* longs;
+  int32_t* sorted;     // [T]: the long runs' tokens in order
+};
+__device__ __forceinline__ int64_t eg_key(const EmbedGradParams& p, int64_t t) {
+  const int64_t at = p.row_map ? p.row_map[t] : t;
+  int64_t k = p.by_position ? (p.positions ? p.positions[t] : at % p.L) : p.ids[at];
+  return k < 0 ? 0 : (k >= p.V ? p.V - 1 : k);
+}
+__global__ __launch_bounds__(256) void hstu_eg_clear(const EmbedGradParams p) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < p.V) p.count[i] = 0;
+  if (i < 4) p.heads[i] = 0;
+}
+__global__ __launch_bounds__(256) void hstu_eg_count(const EmbedGradParams p) {
+  // one addition per wavefront and key: the tokens of a popular key would otherwise queue at its counter one by one
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int key = t < p.T ? (int)eg_key(p, t) : -1;
+  int leader = lane, rank = 0, members = 0;
+  uint64_t left = __builtin_amdgcn_ballot_w64(key >= 0);
+  while (left) {
+    const int first = __builtin_ctzll(left);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(key == __builtin_amdgcn_readlane(key, first));
+    if ((same >> lane) & 1) {
+      leader = first;
+      rank = __builtin_popcountll(same & ((1ull << lane) - 1));
+      members = __builtin_popcountll(same);
+    }
+    left &= ~same;
+  }
+  int base = 0;
+  if (key >= 0 && leader == lane) base = atomicAdd(&p.count[key], members);
+  base = __shfl(base, leader, 64);
+  if (t < p.T) p.rank[t] = base + rank;
+}
+// Each workgroup reserves room for its 256 keys with one addition per counter, and clears the rows of those without a token.
+__global__ __launch_bounds__(256) void hstu_eg_reserve(const EmbedGradParams p) {
+  __shared__ int sums[4][3], base[3];
+  const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int n = v < p.V ? p.count[v] : 0;
+  const int mine[3] = {n, n > 0 && n <= EG_SHORT ? 1 : 0, n > EG_SHORT ? 1 : 0};
+  int at[3];
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    int s = mine[x];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(s, d, 64);
+      s += lane >= d ? o : 0;
+    }
+    at[x] = s - mine[x];
+    if (lane == 63) sums[w][x] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) base[threadIdx.x] = atomicAdd(&p.heads[threadIdx.x], sums[0][threadIdx.x] + sums[1][threadIdx.x] + sums[2][threadIdx.x] + sums[3][threadIdx.x]);
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    at[x] += base[x];
+    for (int y = 0; y < w; ++y) at[x] += sums[y][x];
+  }
+  if (n > 0) {
+    p.count[v] = at[0];
+    const int4 run = {(int)v, at[0], n, 0};
+    if (n <= EG_SHORT) p.shorts[at[1]] = run; else p.longs[at[2]] = run;
+  }
+  // the rows of keys without a token, the whole wave one at a time
+  uint64_t empty = __builtin_amdgcn_ballot_w64(v < p.V && n == 0);
+  const int64_t v0 = v - lane;
+  while (empty) {
+    const int x = __builtin_ctzll(empty);
+    empty &= empty - 1;
+    bf16_t* o = p.out + (v0 + x) * p.out_stride;
+    for (int e = 8 * lane; e < p.width; e += 512) *(uint4*)(o + e) = uint4{0u, 0u, 0u, 0u};
+  }
+}
+__global__ __launch_bounds__(256) void hstu_eg_place(const EmbedGradParams p) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < p.T) p.order[p.count[eg_key(p, t)] + p.rank[t]] = (int32_t)t;
+}
+// One wavefront per short run: its tokens in order by counting the smaller ones, then their rows, four in flight.
+__global__ __launch_bounds__(256) void hstu_eg_short(const EmbedGradParams p) {
+  __shared__ int tokens[4][EG_SHORT];
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (i >= p.heads[1]) return;
+  const int4 run = p.shorts[i];
+  const int n = run.z;
+  const int mine = lane < n ? p.order[run.y + lane] : 0x7fffffff;
+  int r = 0;
+  for (int x = 0; x < n; ++x) r += __shfl(mine, x, 64) < mine ? 1 : 0;
+  if (lane < n) tokens[w][r] = mine;
+  __builtin_amdgcn_wave_barrier();
+  for (int e = 8 * lane; e < p.width; e += 512) {
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < n; x += 4) {
+      uint4 v[4];
+#pragma unroll
+      for (int y = 0; y < 4; ++y) v[y] = *(const uint4*)(p.g + (int64_t)tokens[w][x + y < n ? x + y : x] * p.g_stride + e);
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        if (x + y < n) {
+          float f[8];
+          unpack8(v[y], f);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            s[k] += p.scale == 1.f ? f[k] : round_bf16(f[k] * p.scale);
+            s[k] = p.width > 64 ? round_bf16(s[k]) : s[k];
+          }
+        }
+      }
+    }
+    *(uint4*)(p.out + (int64_t)run.x * p.out_stride + e) = pack8(s);
+  }
+}
+// One workgroup per long run: its tokens' bits set in LDS, read back in order.
+__global__ __launch_bounds__(256) void hstu_eg_order(const EmbedGradParams p) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t bits[];
+  __shared__ int sums[4];
+  if ((int)blockIdx.x >= p.heads[2]) return;
+  const int4 run = p.longs[blockIdx.x];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int done = 0;
+  for (int64_t t0 = 0; t0 < p.T; t0 += EG_WINDOW) {
+    const int span = (int)(p.T - t0 < EG_WINDOW ? p.T - t0 : EG_WINDOW), words = (span + 31) >> 5;
+    for (int x = tid; x < words; x += 256) bits[x] = 0u;
+    __syncthreads();
+    for (int x = tid; x < run.z; x += 256) {
+      const int64_t t = p.order[run.y + x] - t0;
+      if (t >= 0 && t < span) atomicOr(&bits[t >> 5], 1u << (t & 31));
+    }
+    __syncthreads();
+    // every thread a stretch of words: count, prefix sum, write
+    const int per = (words + 255) / 256, x0 = tid * per < words ? tid * per : words, x1 = x0 + per < words ? x0 + per : words;
+    int c = 0;
+    for (int x = x0; x < x1; ++x) c += __builtin_popcount(bits[x]);
+    int s = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(s, d, 64);
+      s += lane >= d ? o : 0;
+    }
+    if (lane == 63) sums[w] = s;
+    __syncthreads();
+    int at = done + s - c;
+    for (int y = 0; y < w; ++y) at += sums[y];
+    for (int x = x0; x < x1; ++x) {
+      uint32_t m = bits[x];
+      while (m) {
+        p.sorted[run.y + at++] = (int32_t)(t0 + 32 * x + __builtin_ctz(m));
+        m &= m - 1;
+      }
+    }
+    done += sums[0] + sums[1] + sums[2] + sums[3];
+    __syncthreads();
+  }
+}
+// One wavefront per long run and 128 columns, two columns per lane, 64 rows in flight (32 in registers, 32 being added).
+// WIDE: partial sums rounded to bf16.
+template <bool WIDE, bool SCALED>
+__global__ __launch_bounds__(64) void hstu_eg_long(const EmbedGradParams p) {
+  if ((int)blockIdx.x >= p.heads[2]) return;
+  const int4 run = p.longs[blockIdx.x];
+  const int lane = threadIdx.x, e = blockIdx.y * 128 + 2 * lane;
+  const int32_t* tok = p.sorted + run.y;
+  const bool on = e < p.width;
+  const bf16_t* g = p.g + (on ? e : 0);
+  float s0 = 0.f, s1 = 0.f;
+  constexpr int DEPTH = 32;
+  uint32_t a[DEPTH], b[DEPTH];
+  // A lane holds one of 64 tokens.  Tokens are loaded ahead of the rows that are in flight while they come: loads return in
+  // order, so that waiting for tokens behind rows would empty the pipeline at every batch.
+  auto tokens = [&](int x) { return tok[x + lane < run.z ? x + lane : 0]; };
+  auto fetch = [&](uint32_t (&v)[DEPTH], int held, int from) {
+#pragma unroll
+    for (int y = 0; y < DEPTH; ++y) v[y] = *(const uint32_t*)(g + (int64_t)__builtin_amdgcn_readlane(held, from + y) * p.g_stride);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add = [&](const uint32_t (&v)[DEPTH], int n) {
+#pragma unroll
+    for (int y = 0; y < DEPTH; ++y) {
+      const uint32_t u = y < n ? v[y] : 0u;      // past the run's end: zeros
+      float f0 = __builtin_bit_cast(float, u << 16), f1 = __builtin_bit_cast(float, u & 0xffff0000u);
+      if (SCALED) { f0 = round_bf16(f0 * p.scale); f1 = round_bf16(f1 * p.scale); }
+      s0 += f0;
+      s1 += f1;
+      if (WIDE) {
+        const uint32_t r = pack2(s0, s1);
+        s0 = __builtin_bit_cast(float, r << 16);
+        s1 = __builtin_bit_cast(float, r & 0xffff0000u);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int now = tokens(0), next = tokens(64);
+  fetch(a, now, 0);
+  for (int x = 0; x < run.z; x += 2 * DEPTH) {
+    const int later = tokens(x + 128);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(b, now, DEPTH);
+    add(a, run.z - x);
+    fetch(a, next, 0);
+    add(b, run.z - x - DEPTH);
+    now = next;
+    next = later;
+  }
+  if (on) *(uint32_t*)(p.out + (int64_t)run.x * p.out_stride + e) = pack2(s0, s1);
+}
+
+template <bool EMB>
+void launch_norm_bwd(const NormGateBwdParams& p, int nb, hipStream_t st) {
+  const dim3 grid((unsigned)nb), block(256);
+  const int lpr = lanes_per_row(p.width), ch = (p.width + 511) / 512;
+  if (lpr == 8) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 8, EMB>), grid, block, 0, st, p);
+  else if (lpr == 16) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 16, EMB>), grid, block, 0, st, p);
+  else if (lpr == 32) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 32, EMB>), grid, block, 0, st, p);
+  else if (ch <= 1) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 64, EMB>), grid, block, 0, st, p);
+  else if (ch <= 2) hipLaunchKernelGGL((hstu_norm_gate_bwd<2, 64, EMB>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((hstu_norm_gate_bwd<4, 64, EMB>), grid, block, 0, st, p);
+}
+
+struct EmbedGradPlan {
+  int64_t shorts, longs;         // most there can be
+  size_t count, rank, order, heads, short_list, long_list, sorted, total;
+};
+EmbedGradPlan embed_grad_plan(int64_t T, int64_t V) {
+  EmbedGradPlan w;
+  auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  w.longs = T / (EG_SHORT + 1) < V ? T / (EG_SHORT + 1) : V;
+  w.shorts = T < V ? T : V;
+  size_t at = 0;
+  w.count = at; at += up((size_t)V * 4);
+  w.rank = at; at += up((size_t)T * 4);
+  w.order = at; at += up((size_t)T * 4);
+  w.heads = at; at += 256;
+  w.short_list = at; at += up((size_t)w.shorts * 16);
+  w.long_list = at; at += up((size_t)w.longs * 16);
+  w.sorted = at; at += up((size_t)T * 4);
+  w.total = at;
+  return w;
+}
+
+// ---- SiLU's gradient in place: d *= silu'(pre), rows of `width` elements with strides
+__global__ __launch_bounds__(256) void hstu_silu_bwd_kernel(bf16_t* d, const bf16_t* pre, int64_t rows, int width, int64_t d_stride, int64_t pre_stride) {
+  const int pieces = width / 8;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / pieces;
+  if (row >= rows) return;
+  const int e = (int)(i - row * pieces) * 8;
+  float x[8], z[8];
+  unpack8(*(const uint4*)(d + row * d_stride + e), x);
+  unpack8(*(const uint4*)(pre + row * pre_stride + e), z);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) x[k] *= silu_grad(z[k]);
+  *(uint4*)(d + row * d_stride + e) = pack8(x);
+}
 
 // ---- hipBLASLt side -------------------------------------------------------
 
@@ -442,148 +827,281 @@ int hstu_block_abi_version(void) { return HSTU_BLOCK_ABI_VERSION; }
 const char* hstu_block_last_error(void) { return g_err; }
 
 int hstu_norm_gate_fwd(const HstuNormGateArgs* a, void* stream) {
-  if (!a) return fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuNormGateArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
-    return fail(HSTU_BLOCK_ERR_VERSION, "norm-gate args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "norm-gate args struct_size/version (%u/%u) do not match this library (%zu/%d)",
                 a->struct_size, a->version, sizeof(HstuNormGateArgs), HSTU_BLOCK_ABI_VERSION);
   if (a->rows < 0 || a->width < 8 || a->width > 8192 || (a->width & 7))
-    return fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0 and width a multiple of 8 in [8, 8192] expected, got rows=%lld width=%d",
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0 and width a multiple of 8 in [8, 8192] expected, got rows=%lld width=%d",
                 (long long)a->rows, a->width);
   g_err[0] = 0;
   if (a->rows == 0) return HSTU_BLOCK_OK;
-  if (!a->a || !a->out || !a->gamma || !a->beta) return fail(HSTU_BLOCK_ERR_NULL, "a, out, gamma and beta must be non-null");
-  if (!aligned16(a->a) || !aligned16(a->u) || !aligned16(a->out) || !aligned16(a->gamma) || !aligned16(a->beta) ||
+  if (!a->a || !a->out || !a->gamma || !a->beta) return block_fail(HSTU_BLOCK_ERR_NULL, "a, out, gamma and beta must be non-null");
+  if (!block_aligned16(a->a) || !block_aligned16(a->u) || !block_aligned16(a->out) || !block_aligned16(a->gamma) || !block_aligned16(a->beta) ||
       (a->a_stride & 7) || (a->out_stride & 7) || a->a_stride < a->width || a->out_stride < a->width ||
       (a->u && ((a->u_stride & 7) || a->u_stride < a->width)))
-    return fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
-  if ((a->rows + 3) / 4 > 0x7fffffffLL) return fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
+  if ((a->rows + 3) / 4 > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
+  if (a->seq_offsets && (a->u || a->L < 1)) return block_fail(HSTU_BLOCK_ERR_SHAPE, "a padded output takes L >= 1 and no gate");
   NormGateParams p;
   p.a = (const bf16_t*)a->a; p.u = (const bf16_t*)a->u; p.out = (bf16_t*)a->out;
   p.gamma = (const bf16_t*)a->gamma; p.beta = (const bf16_t*)a->beta;
   p.rows = a->rows; p.a_stride = a->a_stride; p.u_stride = a->u_stride; p.out_stride = a->out_stride;
   p.width = a->width; p.eps = a->eps;
-  const dim3 grid((unsigned)((a->rows + 3) / 4)), block(256);
+  p.seq_offsets = a->seq_offsets; p.L = a->L;
   hipStream_t st = (hipStream_t)stream;
-  const int ch = (a->width + 511) / 512;
-  if (ch <= 1) hipLaunchKernelGGL(hstu_norm_gate<1>, grid, block, 0, st, p);
-  else if (ch <= 2) hipLaunchKernelGGL(hstu_norm_gate<2>, grid, block, 0, st, p);
-  else if (ch <= 4) hipLaunchKernelGGL(hstu_norm_gate<4>, grid, block, 0, st, p);
-  else hipLaunchKernelGGL(hstu_norm_gate<16>, grid, block, 0, st, p);
+  const int lpr = lanes_per_row(a->width), per = 4 * (64 / lpr), ch = (a->width + 511) / 512;
+  const dim3 grid((unsigned)((a->rows + per - 1) / per)), block(256);
+  if (lpr == 8) hipLaunchKernelGGL((hstu_norm_gate<1, 8>), grid, block, 0, st, p);
+  else if (lpr == 16) hipLaunchKernelGGL((hstu_norm_gate<1, 16>), grid, block, 0, st, p);
+  else if (lpr == 32) hipLaunchKernelGGL((hstu_norm_gate<1, 32>), grid, block, 0, st, p);
+  else if (ch <= 1) hipLaunchKernelGGL((hstu_norm_gate<1, 64>), grid, block, 0, st, p);
+  else if (ch <= 2) hipLaunchKernelGGL((hstu_norm_gate<2, 64>), grid, block, 0, st, p);
+  else if (ch <= 4) hipLaunchKernelGGL((hstu_norm_gate<4, 64>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((hstu_norm_gate<16, 64>), grid, block, 0, st, p);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate kernel launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 
 size_t hstu_norm_gate_bwd_workspace_bytes(int64_t rows, int32_t width) {
   if (rows < 0 || width < 8) return 0;
-  return (size_t)norm_gate_bwd_blocks(rows) * 2u * (size_t)width * sizeof(float);
+  return (size_t)norm_gate_bwd_blocks(rows, width) * 2u * (size_t)width * sizeof(float);
 }
 
 int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
-  if (!a) return fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuNormGateBwdArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
-    return fail(HSTU_BLOCK_ERR_VERSION, "norm-gate backward args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "norm-gate backward args struct_size/version (%u/%u) do not match this library (%zu/%d)",
                 a->struct_size, a->version, sizeof(HstuNormGateBwdArgs), HSTU_BLOCK_ABI_VERSION);
   if (a->rows < 0 || a->width < 8 || a->width > 2048 || (a->width & 7))
-    return fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0 and width a multiple of 8 in [8, 2048] expected, got rows=%lld width=%d",
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0 and width a multiple of 8 in [8, 2048] expected, got rows=%lld width=%d",
                 (long long)a->rows, a->width);
   g_err[0] = 0;
-  if (!a->dgamma || !a->dbeta) return fail(HSTU_BLOCK_ERR_NULL, "dgamma and dbeta must be non-null");
+  if (!a->dgamma || !a->dbeta) return block_fail(HSTU_BLOCK_ERR_NULL, "dgamma and dbeta must be non-null");
   hipStream_t st = (hipStream_t)stream;
-  const int nb = a->rows == 0 ? 0 : norm_gate_bwd_blocks(a->rows);
+  const int nb = a->rows == 0 ? 0 : norm_gate_bwd_blocks(a->rows, a->width);
   if (nb > 0) {
-    if (!a->a || !a->dout || !a->da || !a->gamma || !a->beta) return fail(HSTU_BLOCK_ERR_NULL, "a, dout, da, gamma and beta must be non-null");
-    if ((a->u == nullptr) != (a->du == nullptr)) return fail(HSTU_BLOCK_ERR_NULL, "u and du go together (both null: the plain layer norm)");
-    if (!aligned16(a->a) || !aligned16(a->u) || !aligned16(a->dout) || !aligned16(a->da) || !aligned16(a->du) ||
-        !aligned16(a->gamma) || !aligned16(a->beta) ||
+    if (!a->a || !a->dout || !a->da || !a->gamma || !a->beta) return block_fail(HSTU_BLOCK_ERR_NULL, "a, dout, da, gamma and beta must be non-null");
+    if ((a->u == nullptr) != (a->du == nullptr)) return block_fail(HSTU_BLOCK_ERR_NULL, "u and du go together (both null: the plain layer norm)");
+    if (!block_aligned16(a->a) || !block_aligned16(a->u) || !block_aligned16(a->dout) || !block_aligned16(a->da) || !block_aligned16(a->du) ||
+        !block_aligned16(a->gamma) || !block_aligned16(a->beta) ||
         (a->a_stride & 7) || (a->dout_stride & 7) || (a->da_stride & 7) ||
         a->a_stride < a->width || a->dout_stride < a->width || a->da_stride < a->width ||
         (a->u && ((a->u_stride & 7) || (a->du_stride & 7) || a->u_stride < a->width || a->du_stride < a->width)))
-      return fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
+      return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
     const size_t need = hstu_norm_gate_bwd_workspace_bytes(a->rows, a->width);
     if (!a->workspace || a->workspace_bytes < need || ((uintptr_t)a->workspace & 3u))
-      return fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_norm_gate_bwd_workspace_bytes), got %zu", need,
+      return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_norm_gate_bwd_workspace_bytes), got %zu", need,
                   a->workspace ? a->workspace_bytes : (size_t)0);
-    NormGateBwdParams p;
+    if ((a->u_pre && (!a->u || !block_aligned16(a->u_pre) || (a->u_pre_stride & 7) || a->u_pre_stride < a->width)) ||
+        (a->add && (!block_aligned16(a->add) || (a->add_stride & 7) || a->add_stride < a->width)))
+      return block_fail(HSTU_BLOCK_ERR_SHAPE, "u_pre (with a gate) and add: 16-byte aligned, row strides multiples of 8 elements and >= width");
+    NormGateBwdParams p = {};
+    p.u_pre = (const bf16_t*)a->u_pre; p.u_pre_stride = a->u_pre_stride;
+    p.add = (const bf16_t*)a->add; p.add_stride = a->add_stride; p.row_map = a->row_map;
     p.a = (const bf16_t*)a->a; p.u = (const bf16_t*)a->u; p.dout = (const bf16_t*)a->dout;
     p.gamma = (const bf16_t*)a->gamma; p.beta = (const bf16_t*)a->beta;
     p.da = (bf16_t*)a->da; p.du = (bf16_t*)a->du; p.partial = (float*)a->workspace;
     p.rows = a->rows; p.a_stride = a->a_stride; p.u_stride = a->u_stride; p.dout_stride = a->dout_stride;
     p.da_stride = a->da_stride; p.du_stride = a->du_stride; p.width = a->width; p.eps = a->eps;
-    const dim3 grid((unsigned)nb), block(256);
-    const int ch = (a->width + 511) / 512;
-    if (ch <= 1) hipLaunchKernelGGL(hstu_norm_gate_bwd<1>, grid, block, 0, st, p);
-    else if (ch <= 2) hipLaunchKernelGGL(hstu_norm_gate_bwd<2>, grid, block, 0, st, p);
-    else hipLaunchKernelGGL(hstu_norm_gate_bwd<4>, grid, block, 0, st, p);
+    launch_norm_bwd<false>(p, nb, st);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate backward kernel launch: %s", hipGetErrorString(e));
+    if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate backward kernel launch: %s", hipGetErrorString(e));
   }
   hipLaunchKernelGGL(hstu_colsum, dim3((unsigned)((2 * a->width + 31) / 32)), dim3(1024), 0, st, (const float*)a->workspace, nb, a->width,
                      a->dgamma, a->dbeta);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(HSTU_BLOCK_ERR_LAUNCH, "column-sum kernel launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "column-sum kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
-  if (!a) return fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuEmbedNormArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
-    return fail(HSTU_BLOCK_ERR_VERSION, "embed-norm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "embed-norm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
                 a->struct_size, a->version, sizeof(HstuEmbedNormArgs), HSTU_BLOCK_ABI_VERSION);
   if (a->rows < 0 || a->width < 8 || a->width > 8192 || (a->width & 7) || a->vocab < 1)
-    return fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, vocab >= 1 and width a multiple of 8 in [8, 8192] expected, got rows=%lld vocab=%lld width=%d",
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, vocab >= 1 and width a multiple of 8 in [8, 8192] expected, got rows=%lld vocab=%lld width=%d",
                 (long long)a->rows, (long long)a->vocab, a->width);
   g_err[0] = 0;
   if (a->rows == 0) return HSTU_BLOCK_OK;
-  if (!a->ids || !a->table || !a->out || !a->gamma || !a->beta) return fail(HSTU_BLOCK_ERR_NULL, "ids, table, out, gamma and beta must be non-null");
-  if ((a->pos_table != nullptr) != (a->positions != nullptr) || (a->pos_table && a->n_positions < 1))
-    return fail(HSTU_BLOCK_ERR_NULL, "pos_table and positions go together (with n_positions >= 1)");
-  if (!aligned16(a->table) || !aligned16(a->pos_table) || !aligned16(a->out) || !aligned16(a->gamma) || !aligned16(a->beta) ||
+  if (!a->ids || !a->table || !a->out || !a->gamma || !a->beta) return block_fail(HSTU_BLOCK_ERR_NULL, "ids, table, out, gamma and beta must be non-null");
+  if ((a->pos_table != nullptr) != (a->positions != nullptr || a->L > 0) || (a->pos_table && a->n_positions < 1) || a->L < 0)
+    return block_fail(HSTU_BLOCK_ERR_NULL, "pos_table and positions (or L) go together (with n_positions >= 1)");
+  if (!block_aligned16(a->table) || !block_aligned16(a->pos_table) || !block_aligned16(a->out) || !block_aligned16(a->gamma) || !block_aligned16(a->beta) ||
       (a->table_stride & 7) || a->table_stride < a->width)
-    return fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, table_stride a multiple of 8 elements and >= width");
-  if ((a->rows + 3) / 4 > 0x7fffffffLL) return fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, table_stride a multiple of 8 elements and >= width");
+  if ((a->rows + 3) / 4 > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
   EmbedNormParams p;
   p.ids = a->ids; p.positions = a->positions;
   p.table = (const bf16_t*)a->table; p.pos_table = (const bf16_t*)a->pos_table;
   p.gamma = (const bf16_t*)a->gamma; p.beta = (const bf16_t*)a->beta; p.out = (bf16_t*)a->out;
   p.rows = a->rows; p.vocab = a->vocab; p.table_stride = a->table_stride; p.n_positions = a->n_positions;
   p.width = a->width; p.eps = a->eps; p.scale = a->scale;
-  const dim3 grid((unsigned)((a->rows + 3) / 4)), block(256);
+  p.row_map = a->row_map; p.L = a->L; p.round_steps = a->round_steps;
   hipStream_t st = (hipStream_t)stream;
-  const int ch = (a->width + 511) / 512;
-  if (ch <= 1) hipLaunchKernelGGL(hstu_embed_norm<1>, grid, block, 0, st, p);
-  else if (ch <= 2) hipLaunchKernelGGL(hstu_embed_norm<2>, grid, block, 0, st, p);
-  else if (ch <= 4) hipLaunchKernelGGL(hstu_embed_norm<4>, grid, block, 0, st, p);
-  else hipLaunchKernelGGL(hstu_embed_norm<16>, grid, block, 0, st, p);
+  const int lpr = lanes_per_row(a->width), per = 4 * (64 / lpr), ch = (a->width + 511) / 512;
+  const dim3 grid((unsigned)((a->rows + per - 1) / per)), block(256);
+  if (lpr == 8) hipLaunchKernelGGL((hstu_embed_norm<1, 8>), grid, block, 0, st, p);
+  else if (lpr == 16) hipLaunchKernelGGL((hstu_embed_norm<1, 16>), grid, block, 0, st, p);
+  else if (lpr == 32) hipLaunchKernelGGL((hstu_embed_norm<1, 32>), grid, block, 0, st, p);
+  else if (ch <= 1) hipLaunchKernelGGL((hstu_embed_norm<1, 64>), grid, block, 0, st, p);
+  else if (ch <= 2) hipLaunchKernelGGL((hstu_embed_norm<2, 64>), grid, block, 0, st, p);
+  else if (ch <= 4) hipLaunchKernelGGL((hstu_embed_norm<4, 64>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((hstu_embed_norm<16, 64>), grid, block, 0, st, p);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(HSTU_BLOCK_ERR_LAUNCH, "embed-norm kernel launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "embed-norm kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+int hstu_embed_norm_bwd(const HstuEmbedNormArgs* a, const HstuNormGateBwdArgs* g, void* stream) {
+  if (!a || !g) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (a->struct_size != sizeof(HstuEmbedNormArgs) || a->version != HSTU_BLOCK_ABI_VERSION || g->struct_size != sizeof(HstuNormGateBwdArgs) ||
+      g->version != HSTU_BLOCK_ABI_VERSION)
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "embed-norm backward args do not match this library");
+  if (a->rows < 0 || a->width < 8 || a->width > 2048 || (a->width & 7) || a->vocab < 1 || a->L < 0)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, vocab >= 1 and width a multiple of 8 in [8, 2048] expected");
+  if (!g->dgamma || !g->dbeta) return block_fail(HSTU_BLOCK_ERR_NULL, "dgamma and dbeta must be non-null");
+  hipStream_t st = (hipStream_t)stream;
+  const int nb = a->rows == 0 ? 0 : norm_gate_bwd_blocks(a->rows, a->width);
+  if (nb > 0) {
+    if (!a->ids || !a->table || !a->gamma || !g->dout || !g->da) return block_fail(HSTU_BLOCK_ERR_NULL, "ids, table, gamma, dout and da must be non-null");
+    if ((a->pos_table != nullptr) != (a->positions != nullptr || a->L > 0) || (a->pos_table && a->n_positions < 1))
+      return block_fail(HSTU_BLOCK_ERR_NULL, "pos_table and positions (or L) go together (with n_positions >= 1)");
+    if (!block_aligned16(a->table) || !block_aligned16(a->pos_table) || !block_aligned16(a->gamma) || !block_aligned16(g->dout) || !block_aligned16(g->da) ||
+        (a->table_stride & 7) || a->table_stride < a->width || (g->dout_stride & 7) || g->dout_stride < a->width || (g->da_stride & 7) ||
+        g->da_stride < a->width)
+      return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
+    const size_t need = hstu_norm_gate_bwd_workspace_bytes(a->rows, a->width);
+    if (!g->workspace || g->workspace_bytes < need || ((uintptr_t)g->workspace & 3u))
+      return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_norm_gate_bwd_workspace_bytes)", need);
+    NormGateBwdParams p = {};
+    p.ids = a->ids; p.positions = a->positions; p.table = (const bf16_t*)a->table; p.pos_table = (const bf16_t*)a->pos_table;
+    p.vocab = a->vocab; p.table_stride = a->table_stride; p.n_positions = a->n_positions; p.scale = a->scale; p.L = a->L; p.round_steps = a->round_steps;
+    p.row_map = a->row_map;
+    p.dout = (const bf16_t*)g->dout; p.dout_stride = g->dout_stride; p.da = (bf16_t*)g->da; p.da_stride = g->da_stride;
+    p.gamma = (const bf16_t*)a->gamma; p.partial = (float*)g->workspace;
+    p.rows = a->rows; p.width = a->width; p.eps = a->eps;
+    launch_norm_bwd<true>(p, nb, st);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "embed-norm backward kernel launch: %s", hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(hstu_colsum, dim3((unsigned)((2 * a->width + 31) / 32)), dim3(1024), 0, st, (const float*)g->workspace, nb, a->width,
+                     g->dgamma, g->dbeta);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "column-sum kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+size_t hstu_embed_grad_workspace_bytes(int64_t rows, int64_t keys, int32_t width) {
+  return rows < 0 || keys < 1 || width < 8 ? 0 : embed_grad_plan(rows, keys).total;
+}
+
+int hstu_embed_grad(const HstuEmbedGradArgs* a, void* stream) {
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (a->struct_size != sizeof(HstuEmbedGradArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "embedding gradient args do not match this library");
+  if (a->rows < 0 || a->rows > 0x7fffffff || a->keys < 1 || a->keys > 0x7fffffff || a->width < 8 || (a->width & 7) || a->L < 0)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, keys >= 1 and width a multiple of 8 expected");
+  if (!a->out || !block_aligned16(a->out) || (a->rows && (!a->g || !block_aligned16(a->g))) || (a->g_stride & 7) || a->g_stride < a->width)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "g and out must be 16-byte aligned, g_stride a multiple of 8 elements and >= width");
+  if (a->rows && !(a->by_position ? (a->positions || a->L > 0) : a->ids != nullptr)) return block_fail(HSTU_BLOCK_ERR_NULL, "the keys are missing");
+  const EmbedGradPlan w = embed_grad_plan(a->rows, a->keys);
+  if (!a->workspace || a->workspace_bytes < w.total || ((uintptr_t)a->workspace & 255u))
+    return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_embed_grad_workspace_bytes), 256-byte aligned", w.total);
+  char* base = (char*)a->workspace;
+  EmbedGradParams p = {};
+  p.g = (const bf16_t*)a->g; p.out = (bf16_t*)a->out; p.ids = a->ids; p.positions = a->positions; p.row_map = a->row_map;
+  p.T = a->rows; p.V = a->keys; p.g_stride = a->g_stride; p.out_stride = a->width; p.L = a->L; p.width = a->width; p.by_position = a->by_position;
+  p.scale = a->scale;
+  p.count = (int32_t*)(base + w.count); p.rank = (int32_t*)(base + w.rank); p.order = (int32_t*)(base + w.order); p.heads = (int32_t*)(base + w.heads);
+  p.shorts = (int4*)(base + w.short_list); p.longs = (int4*)(base + w.long_list); p.sorted = (int32_t*)(base + w.sorted);
+  hipStream_t st = (hipStream_t)stream;
+  const unsigned bv = (unsigned)((p.V + 255) / 256), bt = (unsigned)((p.T + 255) / 256);
+  hipLaunchKernelGGL(hstu_eg_clear, dim3(bv), dim3(256), 0, st, p);
+  if (bt) hipLaunchKernelGGL(hstu_eg_count, dim3(bt), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(hstu_eg_reserve, dim3(bv), dim3(256), 0, st, p);
+  if (bt) {
+    hipLaunchKernelGGL(hstu_eg_place, dim3(bt), dim3(256), 0, st, p);
+    if (w.longs) {
+      // (the long runs first: the longest of them is the last to end)
+      const int64_t span = p.T < EG_WINDOW ? p.T : EG_WINDOW;
+      const int lds = (int)((span + 31) / 32 * 4);
+      static int granted[64];
+      if (int rc = block_allow_lds((const void*)hstu_eg_order, EG_WINDOW / 8, granted)) return rc;
+      hipLaunchKernelGGL(hstu_eg_order, dim3((unsigned)w.longs), dim3(256), lds, st, p);
+      const dim3 grid((unsigned)w.longs, (unsigned)((p.width + 127) / 128));
+      const bool wide = p.width > 64, scaled = p.scale != 1.f;
+      if (wide && scaled) hipLaunchKernelGGL((hstu_eg_long<true, true>), grid, dim3(64), 0, st, p);
+      else if (wide) hipLaunchKernelGGL((hstu_eg_long<true, false>), grid, dim3(64), 0, st, p);
+      else if (scaled) hipLaunchKernelGGL((hstu_eg_long<false, true>), grid, dim3(64), 0, st, p);
+      else hipLaunchKernelGGL((hstu_eg_long<false, false>), grid, dim3(64), 0, st, p);
+    }
+    hipLaunchKernelGGL(hstu_eg_short, dim3((unsigned)((w.shorts + 3) / 4)), dim3(256), 0, st, p);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "embedding gradient launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+int hstu_pack_plan(const void* lens, int32_t lens_are_64bit, int32_t B, int32_t L, int32_t* seq_offsets, int32_t* row_map, int32_t* total, void* stream) {
+  if (!lens || !seq_offsets || !row_map || !total) return block_fail(HSTU_BLOCK_ERR_NULL, "lens, seq_offsets, row_map and total must be non-null");
+  if (B < 1 || L < 1 || (int64_t)B * L > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad batch B=%d L=%d", B, L);
+  hipStream_t st = (hipStream_t)stream;
+  if (lens_are_64bit) hipLaunchKernelGGL(hstu_pack_plan_kernel<int64_t>, dim3((unsigned)B), dim3(256), 0, st, (const int64_t*)lens, B, L, seq_offsets, row_map, total);
+  else hipLaunchKernelGGL(hstu_pack_plan_kernel<int32_t>, dim3((unsigned)B), dim3(256), 0, st, (const int32_t*)lens, B, L, seq_offsets, row_map, total);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "pack plan launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+int hstu_mask_lengths(const uint8_t* mask, int32_t B, int32_t L, int32_t* lens, int32_t* bad, void* stream) {
+  if (!mask || !lens || !bad) return block_fail(HSTU_BLOCK_ERR_NULL, "mask, lens and bad must be non-null");
+  if (B < 1 || L < 1) return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad batch B=%d L=%d", B, L);
+  hipLaunchKernelGGL(hstu_mask_lengths_kernel, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, (hipStream_t)stream, mask, B, L, lens, bad);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "mask lengths launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+int hstu_silu_bwd(void* d, int64_t d_stride, const void* pre, int64_t pre_stride, int64_t rows, int32_t width, void* stream) {
+  if (rows < 0 || width < 8 || (width & 7) || (d_stride & 7) || (pre_stride & 7) || d_stride < width || pre_stride < width)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, width and row strides multiples of 8 expected");
+  if (rows == 0) return HSTU_BLOCK_OK;
+  if (!d || !pre || !block_aligned16(d) || !block_aligned16(pre)) return block_fail(HSTU_BLOCK_ERR_NULL, "d and pre must be 16-byte aligned");
+  const int64_t n = rows * (width / 8);
+  hipLaunchKernelGGL(hstu_silu_bwd_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (bf16_t*)d, (const bf16_t*)pre, rows, width,
+                     d_stride, pre_stride);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "silu backward launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 
 size_t hstu_gemm_silu_workspace_bytes(void) { return kBlasWorkspace; }
 
 int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
-  if (!a) return fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuGemmSiluArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
-    return fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
                 a->struct_size, a->version, sizeof(HstuGemmSiluArgs), HSTU_BLOCK_ABI_VERSION);
   if (a->M < 0 || a->N < 1 || a->K < 1 || a->M > 0x7fffffffLL || a->x_stride < a->K)
-    return fail(HSTU_BLOCK_ERR_SHAPE, "bad shape M=%lld N=%d K=%d x_stride=%lld", (long long)a->M, a->N, a->K, (long long)a->x_stride);
-  if (a->activation != 0 && a->activation != 1) return fail(HSTU_BLOCK_ERR_SHAPE, "activation must be 0 (none) or 1 (silu)");
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad shape M=%lld N=%d K=%d x_stride=%lld", (long long)a->M, a->N, a->K, (long long)a->x_stride);
+  if (a->activation != 0 && a->activation != 1) return block_fail(HSTU_BLOCK_ERR_SHAPE, "activation must be 0 (none) or 1 (silu)");
   g_err[0] = 0;
   if (a->M == 0) return HSTU_BLOCK_OK;
-  if (!a->x || !a->w || !a->out) return fail(HSTU_BLOCK_ERR_NULL, "x, w and out must be non-null");
+  if (!a->x || !a->w || !a->out) return block_fail(HSTU_BLOCK_ERR_NULL, "x, w and out must be non-null");
   // the kernel picked for a shape is kept and reused for every later call of that shape: it may assume what
   // the first call's pointers offered, so every call has to offer it
-  if (!aligned16(a->x) || !aligned16(a->w) || !aligned16(a->out) || !aligned16(a->bias) || !aligned16(a->workspace) || (a->x_stride & 7))
-    return fail(HSTU_BLOCK_ERR_SHAPE, "x, w, out, bias and workspace must be 16-byte aligned and x_stride a multiple of 8 elements");
-  if (a->c && (!aligned16(a->c) || (a->c_stride & 7) || a->c_stride < a->N))
-    return fail(HSTU_BLOCK_ERR_SHAPE, "c must be 16-byte aligned with a row stride that is a multiple of 8 elements and >= N");
-  if (a->workspace_bytes && !a->workspace) return fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace_bytes without a workspace");
+  if (!block_aligned16(a->x) || !block_aligned16(a->w) || !block_aligned16(a->out) || !block_aligned16(a->bias) || !block_aligned16(a->workspace) || (a->x_stride & 7))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "x, w, out, bias and workspace must be 16-byte aligned and x_stride a multiple of 8 elements");
+  if (a->c && (!block_aligned16(a->c) || (a->c_stride & 7) || a->c_stride < a->N))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "c must be 16-byte aligned with a row stride that is a multiple of 8 elements and >= N");
+  if (a->workspace_bytes && !a->workspace) return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace_bytes without a workspace");
   int dev = 0;
   hipError_t he = hipGetDevice(&dev);
-  if (he != hipSuccess) return fail(HSTU_BLOCK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(he));
-  if (dev < 0 || dev >= 64) return fail(HSTU_BLOCK_ERR_LAUNCH, "device index %d out of range", dev);
+  if (he != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(he));
+  if (dev < 0 || dev >= 64) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "device index %d out of range", dev);
 
   BlasState& bs = blas();
   GemmPlan plan;
@@ -592,7 +1110,7 @@ int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
     std::lock_guard<std::mutex> lock(bs.mu);
     if (!bs.handle[dev]) {
       const hipblasStatus_t st = hipblasLtCreate(&bs.handle[dev]);
-      if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtCreate: %s", blas_str(st));
+      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtCreate: %s", blas_str(st));
     }
     handle = bs.handle[dev];
     const auto key = std::make_tuple(dev, a->M, a->N, a->K, a->x_stride, a->bias ? 1 : 0, a->activation, a->workspace_bytes,
@@ -618,7 +1136,7 @@ int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
       } part;
       GemmPlan& np = part.p;
       hipblasStatus_t st = hipblasLtMatmulDescCreate(&np.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F);
-      if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescCreate: %s", blas_str(st));
+      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescCreate: %s", blas_str(st));
       // every attribute is checked: a rejected epilogue or bias type would otherwise come back as "no kernel",
       // or as a product without its epilogue
       auto set_desc = [&](hipblasLtMatmulDescAttributes_t attr, const void* val, size_t bytes) {
@@ -638,23 +1156,23 @@ int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
         if (st == HIPBLAS_STATUS_SUCCESS) st = set_desc(HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &a->bias, sizeof(void*));
       }
       if (st != HIPBLAS_STATUS_SUCCESS)
-        return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (epilogue %d, bias %d): %s", (int)epi, a->bias ? 1 : 0, blas_str(st));
+        return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (epilogue %d, bias %d): %s", (int)epi, a->bias ? 1 : 0, blas_str(st));
       st = hipblasLtMatrixLayoutCreate(&np.la, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->K, (int64_t)a->N);
       if (st == HIPBLAS_STATUS_SUCCESS) st = hipblasLtMatrixLayoutCreate(&np.lb, HIP_R_16BF, (uint64_t)a->K, (uint64_t)a->M, a->x_stride);
       if (st == HIPBLAS_STATUS_SUCCESS) st = hipblasLtMatrixLayoutCreate(&np.lc, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->M, (int64_t)a->N);
       if (st == HIPBLAS_STATUS_SUCCESS && a->c)
         st = hipblasLtMatrixLayoutCreate(&np.lres, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->M, a->c_stride);
-      if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatrixLayoutCreate: %s", blas_str(st));
+      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatrixLayoutCreate: %s", blas_str(st));
       st = hipblasLtMatmulPreferenceCreate(&part.pref);
-      if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceCreate: %s", blas_str(st));
+      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceCreate: %s", blas_str(st));
       const uint64_t ws = a->workspace_bytes;
       st = hipblasLtMatmulPreferenceSetAttribute(part.pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws));
-      if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceSetAttribute: %s", blas_str(st));
+      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceSetAttribute: %s", blas_str(st));
       hipblasLtMatmulHeuristicResult_t res[1];
       int found = 0;
       st = hipblasLtMatmulAlgoGetHeuristic(handle, np.desc, np.la, np.lb, a->c ? np.lres : np.lc, np.lc, part.pref, 1, res, &found);
       if (st != HIPBLAS_STATUS_SUCCESS || found < 1)
-        return fail(HSTU_BLOCK_ERR_BLAS, "hipBLASLt has no kernel for M=%lld N=%d K=%d with this epilogue (%s)",
+        return block_fail(HSTU_BLOCK_ERR_BLAS, "hipBLASLt has no kernel for M=%lld N=%d K=%d with this epilogue (%s)",
                     (long long)a->M, a->N, a->K, blas_str(st));
       np.algo = res[0].algo;
       np.workspace = res[0].workspaceSize;
@@ -676,14 +1194,14 @@ int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
     // and the product is enqueued before it is released
     if (a->bias) {
       const hipblasStatus_t sb = hipblasLtMatmulDescSetAttribute(plan.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &a->bias, sizeof(void*));
-      if (sb != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (bias pointer): %s", blas_str(sb));
+      if (sb != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (bias pointer): %s", blas_str(sb));
     }
     // (with c: D = alpha A B + beta C with C = c and beta = 1, the output written elsewhere)
     const float alpha = 1.0f, beta = a->c ? 1.0f : 0.0f;
     const hipblasStatus_t st = hipblasLtMatmul(handle, plan.desc, &alpha, a->w, plan.la, a->x, plan.lb, &beta, a->c ? a->c : a->out,
                                                a->c ? plan.lres : plan.lc, a->out, plan.lc, &plan.algo, a->workspace, a->workspace_bytes,
                                                (hipStream_t)stream);
-    if (st != HIPBLAS_STATUS_SUCCESS) return fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmul: %s", blas_str(st));
+    if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmul: %s", blas_str(st));
   }
   return HSTU_BLOCK_OK;
 }

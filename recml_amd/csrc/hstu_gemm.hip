@@ -1,0 +1,493 @@
+// The matrix products of an HSTU block on the matrix cores of gfx950, in bf16 with fp32 accumulation.
+//
+//   HSTU_GEMM_NN   out[m, n] = act(sum_k x[m, k] w[k, n] + bias[n] + c[m, n])     a projection
+//   HSTU_GEMM_NT   out[m, k] = sum_n x[m, n] w[k, n]                              the gradient of its input
+//   HSTU_GEMM_TN   out[k, n] = sum_m x[m, k] y[m, n]                              the gradient of its weight
+//
+// The weight (NN, NT) and the weight's gradient (TN) may come as several matrices side by side along n ("slabs": the
+// U, Q, K and V kernels of a block), so nobody concatenates them.  See hstu_gemm_kernel for the layout of the work.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "hstu_block.h"
+#include "hstu_block_common.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) short4v* lds_short4_ptr;
+
+constexpr int GEMM_BK = 32;          // contraction depth of a stage
+constexpr int GEMM_THREADS = 256;
+
+struct GemmParams {
+  const bf16_t* q;                   // the operand of the output's rows
+  const bf16_t* p[HSTU_GEMM_MAX_SLABS];   // the operand of its columns, as slabs
+  bf16_t* out[HSTU_GEMM_MAX_SLABS];
+  float* partial;                    // split contraction: [split][rows][cols] sums instead of `out`
+  bf16_t* pre;                       // the value before the activation is stored here as well (or null)
+  const bf16_t* bias;
+  const bf16_t* c;
+  int64_t q_stride, p_stride, out_stride, c_stride;
+  int32_t rows, cols, depth;         // of the product: output rows and columns, contraction
+  int32_t slab, out_slab;            // width of a slab of `p` (along the weight's n) and of `out` (along its columns)
+  int32_t splits, depth_per_split;
+  int32_t row_tiles, col_tiles;
+  int32_t activation;
+};
+
+// 256 bytes of zeros: what lanes whose element lies outside an operand load.
+__device__ __attribute__((aligned(256))) unsigned char gemm_zeros[256];
+
+__device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_addr_wave_uniform) {
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr_wave_uniform);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(base), "v"(src) : "memory", "m0");
+}
+
+#define HSTU_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | ((((n) >> 4) & 3) << 14)) | 0x0F70)
+
+// One workgroup: a tile of 64 MB output rows x 64 NB output columns, four waves of 32 MB x 32 NB.  The contraction runs in
+// stages of 32 through a three-stage LDS ring filled by direct global -> LDS loads (two stages in flight, one barrier
+// per stage).  The product is formed transposed (columns as the matrix instruction's rows): a lane then holds four
+// consecutive columns of one output row.
+//   An operand stored along the contraction (Q_T / P_T false) lies in LDS as rows of 64 bytes, 16-byte chunk c of row r at
+// c ^ (r / 4 % 4): a fragment is one ds_read_b128 per lane, 16 rows reach all 64 banks.  One stored across it (x and dz in
+// the weight's gradient, the weight itself in the forward) lies as 32 rows of 128 columns, chunk c at c ^ 4 (r % 4), and is
+// transposed on the way out by ds_read_b64_tr_b16, two per fragment.
+//   Why 256 x 128 (MB 4, NB 2): with 64 x 64 per wave the four SIMDs' fragments take all of the LDS bandwidth (128 bytes a
+// clock) at full matrix rate, with 128 x 64 three quarters of it; 128 accumulators leave two workgroups per CU, so that one's
+// barriers and stores run under the other's products.
+template <int MB, int NB, bool Q_T, bool P_T, int STAGES = 3>
+__global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmParams g) {
+  constexpr int TM = 64 * MB, TN = 64 * NB;
+  constexpr int Q_BYTES = TM * GEMM_BK * 2, P_BYTES = TN * GEMM_BK * 2, STAGE = Q_BYTES + P_BYTES;
+  constexpr int LQ = Q_BYTES / 4096, LP = P_BYTES / 4096;      // direct loads of 1 KB per wave
+  static_assert(LQ >= 1 && LP >= 1, "a stage is at least one load per wave and operand");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const uint32_t smem_lds = __builtin_amdgcn_groupstaticsize();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+
+  // Workgroups go to the eight XCDs in turn: the column tiles of a row tile (which share the row operand) follow each
+  // other on one XCD; with a split contraction all tiles of a split do.
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  int rt, ct, split = 0;
+  if (g.splits > 1) {
+    const int per = g.row_tiles * g.col_tiles;
+    split = (j / per) * 8 + xcd;
+    const int t = j % per;
+    rt = t / g.col_tiles;
+    ct = t - rt * g.col_tiles;
+    if (split >= g.splits) return;
+  } else {
+    rt = (j / g.col_tiles) * 8 + xcd;
+    ct = j % g.col_tiles;
+    if (rt >= g.row_tiles) return;
+  }
+  const int m0 = rt * TM, n0 = ct * TN;
+  const int k_begin = split * g.depth_per_split;
+  const int k_end = k_begin + g.depth_per_split < g.depth ? k_begin + g.depth_per_split : g.depth;
+  const int nt = (k_end - k_begin + GEMM_BK - 1) / GEMM_BK;
+
+  // ---- what each lane loads: piece i of an operand is 1 KB of LDS, lane l of it 16 bytes at 16 l.
+  //   along:  row = 16 piece + l / 4, physical chunk l % 4           (advance: 32 elements per stage)
+  //   across: panel of 128 columns, row = 4 (piece % 8) + l / 16, physical chunk l % 16    (advance: 32 rows per stage)
+  // A source past the operand's end is the page of zeros.
+  // Small tiles (64 columns) across the contraction: rows of 64 columns, 8 rows per piece, chunk c at c ^ 4 (r / 2 % 2).
+  struct Src { int outer, k; };      // index along the output's axis, and along the contraction
+  auto src_of = [&](bool across, int tile, int piece) {
+    Src s;
+    if (!across) {
+      const int row = 16 * piece + (lane >> 2);
+      s.outer = row;
+      s.k = 8 * ((lane & 3) ^ ((row >> 2) & 3));
+    } else if (tile >= 128) {
+      const int panel = piece >> 3, row = 4 * (piece & 7) + (lane >> 4);
+      s.outer = 128 * panel + 8 * ((lane & 15) ^ (4 * (row & 3)));
+      s.k = row;
+    } else {
+      const int row = 8 * piece + (lane >> 3);
+      s.outer = 8 * ((lane & 7) ^ (4 * ((row >> 1) & 1)));
+      s.k = row;
+    }
+    return s;
+  };
+  const char* qp[LQ];
+  const char* pp[LP];
+  int qk[LQ], pk[LP];                // contraction index of the lane's next load; past k_end: zeros
+  int ps[LP], pc[LP];                // P along the contraction in slabs: slab and column within it
+  int po[LP];
+#pragma unroll
+  for (int i = 0; i < LQ; ++i) {
+    const Src s = src_of(Q_T, TM, w * LQ + i);
+    const int m = m0 + s.outer;
+    qk[i] = m < g.rows ? k_begin + s.k : 0x3fffffff;
+    qp[i] = (const char*)(Q_T ? g.q + (int64_t)(k_begin + s.k) * g.q_stride + m : g.q + (int64_t)m * g.q_stride + k_begin + s.k);
+  }
+#pragma unroll
+  for (int i = 0; i < LP; ++i) {
+    const Src s = src_of(P_T, TN, w * LP + i);
+    const int n = n0 + s.outer;
+    pk[i] = n < g.cols ? k_begin + s.k : 0x3fffffff;
+    if (P_T) {
+      // across the contraction: the column decides the slab, once (TN: y is one matrix, its slab the whole width)
+      const int sl = n < g.cols ? n / g.slab : 0;
+      pp[i] = (const char*)(g.p[sl] + (int64_t)(k_begin + s.k) * g.p_stride + (n - sl * g.slab));
+      ps[i] = pc[i] = po[i] = 0;
+    } else {
+      ps[i] = (k_begin + s.k) / g.slab;
+      pc[i] = k_begin + s.k - ps[i] * g.slab;
+      po[i] = n;
+      const int sl = ps[i] < HSTU_GEMM_MAX_SLABS ? ps[i] : 0;
+      pp[i] = (const char*)((sl == 0 ? g.p[0] : sl == 1 ? g.p[1] : sl == 2 ? g.p[2] : g.p[3]) + (int64_t)n * g.p_stride + pc[i]);
+    }
+  }
+  const int64_t q_step = Q_T ? (int64_t)GEMM_BK * g.q_stride * 2 : GEMM_BK * 2;
+  const int64_t p_step = (int64_t)GEMM_BK * g.p_stride * 2;
+  constexpr int NLOAD = LQ + LP;     // of a stage, per wave
+  auto issue_one = [&](int st, int i) {
+    const uint32_t base = smem_lds + (uint32_t)st * STAGE;
+    if (i < LQ) {
+      const void* src = qk[i] < k_end ? (const void*)qp[i] : (const void*)(gemm_zeros + 16 * (lane & 15));
+      lds_dma16(src, base + 1024u * (w * LQ + i));
+      qp[i] += q_step;
+      qk[i] += GEMM_BK;
+      return;
+    }
+    i -= LQ;
+    const void* src = pk[i] < k_end ? (const void*)pp[i] : (const void*)(gemm_zeros + 16 * (lane & 15));
+    lds_dma16(src, base + Q_BYTES + 1024u * (w * LP + i));
+    pk[i] += GEMM_BK;
+    if (P_T) {
+      pp[i] += p_step;
+    } else {
+      // along the contraction, and on to the next slab where this one ends (selects: a branch here would cut the products
+      // around it into separate schedules)
+      pc[i] += GEMM_BK;
+      const bool over = pc[i] >= g.slab;
+      pc[i] -= over ? g.slab : 0;
+      const int64_t hop = ps[i] == 0 ? g.p[1] - g.p[0] : ps[i] == 1 ? g.p[2] - g.p[1] : g.p[3] - g.p[2];
+      pp[i] += GEMM_BK * 2 + (over ? (hop - g.slab) * 2 : 0);
+      ps[i] += over ? 1 : 0;
+    }
+  };
+
+  // ---- fragments: lane (index l32 of a block of 32, half hh) holds contraction elements 16 s + 8 hh .. + 7
+  const int wm = w & 1, wn = w >> 1;
+  const int gi = lane & 15;
+  auto frag = [&](bool across, int tile, const unsigned char* base, int block, int s) -> bf16x8 {
+    if (!across) {
+      const int r = 32 * block + l32;
+      return *(const bf16x8*)(base + r * 64 + (((2 * s + hh) ^ ((r >> 2) & 3)) * 16));
+    }
+    const int row = 16 * s + 8 * hh + (gi >> 2);
+    const int c2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
+    const unsigned char* at;
+    int pitch;
+    if (tile >= 128) {
+      const int panel = block >> 2, ob = block & 3;
+      pitch = 256;
+      at = base + panel * (GEMM_BK * 256) + row * 256 + (4 * (ob ^ (gi >> 2)) + c2) * 16 + 8 * (gi & 1);
+    } else {
+      pitch = 128;
+      at = base + row * 128 + ((4 * ((block & 1) ^ ((row >> 1) & 1)) + c2)) * 16 + 8 * (gi & 1);
+    }
+    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at));
+    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at + 4 * pitch));
+    struct { short4v a, b; } both = {lo, hi};
+    return __builtin_bit_cast(bf16x8, both);
+  };
+
+  floatx16 acc[NB][MB];
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+
+  static_assert((STAGES - 1) * NLOAD <= 63 && STAGES >= 2 && STAGES <= 4, "vmcnt range");
+  struct Frags { bf16x8 p[NB], q[MB]; };
+  auto load = [&](int st, int s, Frags& f) {
+    const unsigned char* qb = smem + st * STAGE;
+    const unsigned char* pb = qb + Q_BYTES;
+#pragma unroll
+    for (int a = 0; a < NB; ++a) f.p[a] = frag(P_T, TN, pb, wn * NB + a, s);
+#pragma unroll
+    for (int b = 0; b < MB; ++b) f.q[b] = frag(Q_T, TM, qb, wm * MB + b, s);
+  };
+  // One sub-step's products; with `refill` the loads of the stage that takes place `st` go out between them: issued
+  // back to back they would hold the wave up (the CU's memory front end takes one every 16 cycles from all its waves).
+  auto products = [&](const Frags& f, auto refill_, int st) {
+    constexpr bool refill = decltype(refill_)::value;
+    int next = 0;
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int a = 0; a < NB; ++a) {
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.p[a], f.q[b], acc[a][b], 0, 0, 0);
+        if constexpr (refill) {
+          const int due = ((b * NB + a + 1) * NLOAD) / (MB * NB);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < NLOAD; ++i)
+            if (i >= next && i < due) issue_one(st, i);
+          __builtin_amdgcn_sched_barrier(0);
+          next = due;
+        }
+      }
+  };
+  // Stages past the contraction's end are loaded too (zeros), so that every wait counts the same number of younger loads.
+#pragma unroll
+  for (int t = 0; t < STAGES; ++t)
+#pragma unroll
+    for (int i = 0; i < NLOAD; ++i) issue_one(t, i);
+  // A stage's two sub-steps of 16: the fragments of each are asked for ahead of the products of the one before it, so that
+  // the matrix pipe has work while they come.  The order is fixed by scheduling barriers.
+  Frags fa, fb;
+  HSTU_WAIT_VMCNT((STAGES - 1) * NLOAD);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  load(0, 0, fa);
+  int st = 0;
+  for (int t = 0; t < nt; ++t) {
+    load(st, 1, fb);
+    __builtin_amdgcn_sched_barrier(0);
+    products(fa, std::false_type{}, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // (fb is here: the stage's last read is done, and behind the barrier everyone's is: its place can be refilled)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    HSTU_WAIT_VMCNT((STAGES - 2) * NLOAD);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int next = st + 1 >= STAGES ? 0 : st + 1;
+    load(next, 0, fa);
+    __builtin_amdgcn_sched_barrier(0);
+    products(fb, std::true_type{}, st);
+    __builtin_amdgcn_sched_barrier(0);
+    st = next;
+  }
+  HSTU_WAIT_VMCNT(0);
+  __syncthreads();
+
+  // ---- out: blocks of 32 rows x 32 NB columns through the wave's own LDS (fp32, rows 16 bytes apart from a multiple of 256:
+  // conflict-free both ways), then whole row pieces of 8 columns per lane
+  constexpr int W = 32 * NB, PITCH = W * 4 + 16;
+  unsigned char* stage = smem + w * (32 * PITCH);
+  constexpr int LPR = W / 8, RPI = 64 / LPR;        // lanes per row, rows per instruction
+  const int rr = lane / LPR, cc = lane - rr * LPR;
+  const int n = n0 + wn * W + 8 * cc;
+  float bias[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) bias[i] = 0.f;
+  if (g.bias && n < g.cols) unpack8(*(const uint4*)(g.bias + n), bias);
+  const int osl = (g.partial || n >= g.cols) ? 0 : n / g.out_slab;
+#pragma unroll
+  for (int b = 0; b < MB; ++b) {
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const float4 v = {acc[a][b][4 * q4], acc[a][b][4 * q4 + 1], acc[a][b][4 * q4 + 2], acc[a][b][4 * q4 + 3]};
+        *(float4*)(stage + l32 * PITCH + (32 * a + 8 * q4 + 4 * hh) * 4) = v;
+      }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = RPI * i + rr;
+      const int m = m0 + wm * 32 * MB + 32 * b + row;
+      const float4 v0 = *(const float4*)(stage + row * PITCH + 32 * cc), v1 = *(const float4*)(stage + row * PITCH + 32 * cc + 16);
+      if (m < g.rows && n < g.cols) {
+        float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        if (g.partial) {
+          float* o = g.partial + ((int64_t)split * g.rows + m) * g.cols + n;
+          *(float4*)o = v0;
+          *(float4*)(o + 4) = v1;
+        } else {
+          if (g.c) {
+            float cv[8];
+            unpack8(*(const uint4*)(g.c + (int64_t)m * g.c_stride + n), cv);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] += cv[e];
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] += bias[e];
+          bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)m * g.out_stride + (n - osl * g.out_slab);
+          if (g.pre) {
+            // (the activation of the stored value, which is what its gradient is taken at)
+            const uint4 z = pack8(x);
+            *(uint4*)(g.pre + (int64_t)m * g.out_stride + n) = z;
+            unpack8(z, x);
+          }
+          if (g.activation) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = silu(x[e]);
+          }
+          *(uint4*)o = pack8(x);
+        }
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Sums the partial products of a split contraction in the order of the splits and rounds them once.
+__global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
+  const int64_t per = (int64_t)g.rows * g.cols;
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (e >= per) return;
+  float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < g.splits; ++s) {
+    const float4 a = *(const float4*)(g.partial + s * per + e), b = *(const float4*)(g.partial + s * per + e + 4);
+    x[0] += a.x; x[1] += a.y; x[2] += a.z; x[3] += a.w;
+    x[4] += b.x; x[5] += b.y; x[6] += b.z; x[7] += b.w;
+  }
+  const int m = (int)(e / g.cols), n = (int)(e - (int64_t)m * g.cols), sl = n / g.out_slab;
+  bf16_t* o = (sl == 0 ? g.out[0] : sl == 1 ? g.out[1] : sl == 2 ? g.out[2] : g.out[3]) + (int64_t)m * g.out_stride + (n - sl * g.out_slab);
+  *(uint4*)o = pack8(x);
+}
+
+template <int MB, int NB, bool Q_T, bool P_T, int STAGES = 3>
+int launch(const GemmParams& p, hipStream_t st) {
+  constexpr int TM = 64 * MB, TN = 64 * NB;
+  constexpr int ring = STAGES * (TM + TN) * GEMM_BK * 2, out = 4 * 32 * (32 * NB * 4 + 16);
+  constexpr int smem = ring > out ? ring : out;
+  static int granted[64];
+  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES>, smem, granted)) return rc;
+  GemmParams g = p;
+  g.row_tiles = (g.rows + TM - 1) / TM;
+  g.col_tiles = (g.cols + TN - 1) / TN;
+  const int64_t tiles = (int64_t)g.row_tiles * g.col_tiles;
+  const int64_t blocks = g.splits > 1 ? 8LL * ((g.splits + 7) / 8) * tiles : 8LL * ((g.row_tiles + 7) / 8) * g.col_tiles;
+  if (blocks > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "grid too large");
+  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES>), dim3((unsigned)blocks), dim3(GEMM_THREADS), smem, st, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
+template <bool Q_T, bool P_T>
+int launch_sized(const GemmParams& p, hipStream_t st, int tile) {
+  if (tile == 2) return launch<4, 2, Q_T, P_T>(p, st);
+  if (tile == 1) return launch<2, 2, Q_T, P_T>(p, st);
+  return launch<1, 1, Q_T, P_T>(p, st);
+}
+
+int64_t tiles_of(int64_t rows, int64_t cols, int tm, int tn) { return ((rows + tm - 1) / tm) * ((cols + tn - 1) / tn); }
+
+// The tile of a product: 256 x 128 has the most products per byte of LDS traffic, 128 x 128 leaves room for a third workgroup
+// per CU, whose loads cover the others' starts and stores.  Long contractions take the first (78 k x 2048 x 2048: 692 us
+// against 775), short ones the second (78 k x 512 x 2048: 255 us against 262); products of few tiles go down to 64 x 64.
+int pick_tile(int64_t rows, int64_t cols, int64_t depth) {
+  if (depth >= 1024 && tiles_of(rows, cols, 256, 128) >= 512) return 2;
+  if (tiles_of(rows, cols, 128, 128) >= 384) return 1;
+  return 0;
+}
+
+// Splits of a weight gradient's contraction (rows M of the batch): enough workgroups for the chip, whole stages, at least
+// 256 rows each.
+int pick_splits(int64_t rows, int64_t cols, int64_t depth, int* tile) {
+  const int t = tiles_of(rows, cols, 256, 128) >= 8 ? 2 : (tiles_of(rows, cols, 128, 128) >= 4 ? 1 : 0);
+  *tile = t;
+  const int64_t tiles = t == 2 ? tiles_of(rows, cols, 256, 128) : (t == 1 ? tiles_of(rows, cols, 128, 128) : tiles_of(rows, cols, 64, 64));
+  int64_t s = (512 + tiles - 1) / tiles;
+  const int64_t most = depth / 256;
+  s = s < most ? s : most;
+  s = s < 1 ? 1 : (s > 64 ? 64 : s);
+  if (s > 1) s = (s + 7) / 8 * 8;              // (a split is one XCD's work)
+  return (int)s;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K) {
+  if (op != HSTU_GEMM_TN || M < 1 || N < 1 || K < 1) return 0;
+  int tile;
+  const int s = pick_splits(K, N, M, &tile);
+  return s > 1 ? (size_t)s * (size_t)K * (size_t)N * sizeof(float) : 0;
+}
+
+int hstu_gemm(const HstuGemmArgs* a, void* stream) {
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (a->struct_size != sizeof(HstuGemmArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+                      a->struct_size, a->version, sizeof(HstuGemmArgs), HSTU_BLOCK_ABI_VERSION);
+  if (a->op < HSTU_GEMM_NN || a->op > HSTU_GEMM_TN) return block_fail(HSTU_BLOCK_ERR_SHAPE, "unknown op %d", a->op);
+  if (a->M < 0 || a->M > 0x3fffffff || a->N < 8 || a->K < 8 || (a->N & 7) || (a->K & 7) || a->slabs < 1 || a->slabs > HSTU_GEMM_MAX_SLABS ||
+      a->N % a->slabs || (a->N / a->slabs & 7))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "N, K and the slabs must be multiples of 8: got M=%lld N=%d K=%d in %d slabs", (long long)a->M, a->N, a->K,
+                      a->slabs);
+  const int slab = a->N / a->slabs;
+  const bool tn = a->op == HSTU_GEMM_TN;
+  if ((a->x_stride & 7) || a->x_stride < (a->op == HSTU_GEMM_NT ? a->N : a->K))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "x_stride must be a multiple of 8 and cover a row, got %lld", (long long)a->x_stride);
+  if (a->M == 0 && !tn) return HSTU_BLOCK_OK;
+  bool ok = block_aligned16(a->x) && block_aligned16(a->bias) && block_aligned16(a->c) && block_aligned16(a->pre) && (a->x || a->M == 0);
+  for (int i = 0; i < a->slabs; ++i) ok = ok && a->w[i] && block_aligned16(a->w[i]);
+  if (tn) ok = ok && (a->y || a->M == 0) && block_aligned16(a->y) && (a->y_stride & 7) == 0 && a->y_stride >= a->N;
+  else ok = ok && a->out && block_aligned16(a->out) && (!a->c || ((a->c_stride & 7) == 0 && a->c_stride >= a->N));
+  if (!ok) return block_fail(HSTU_BLOCK_ERR_SHAPE, "operands must be present, 16-byte aligned, with row strides of whole 16-byte pieces");
+  if (a->op != HSTU_GEMM_NN && (a->bias || a->c || a->pre || a->activation))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "bias, c, pre and the activation belong to the forward product");
+  hipStream_t st = (hipStream_t)stream;
+  GemmParams p = {};
+  p.q = (const bf16_t*)a->x;
+  p.q_stride = a->x_stride;
+  p.splits = 1;
+  p.slab = slab;
+  p.bias = (const bf16_t*)a->bias; p.c = (const bf16_t*)a->c; p.c_stride = a->c_stride;
+  p.pre = (bf16_t*)a->pre;
+  p.activation = a->activation;
+  if (tn) {
+    p.rows = a->K; p.cols = a->N; p.depth = (int32_t)a->M;
+    p.p[0] = (const bf16_t*)a->y; p.p_stride = a->y_stride;
+    p.slab = a->N;                       // y is one matrix; the slabs are the output's
+    p.out_slab = slab;
+    for (int i = 0; i < a->slabs; ++i) p.out[i] = (bf16_t*)const_cast<void*>(a->w[i]);
+    p.out_stride = slab;
+    int tile;
+    p.splits = pick_splits(a->K, a->N, a->M, &tile);
+    p.depth_per_split = p.depth;
+    if (p.splits == 1) return launch_sized<true, true>(p, st, tile);
+    const size_t need = hstu_gemm_workspace_bytes(a->op, a->M, a->N, a->K);
+    if (!a->workspace || a->workspace_bytes < need || !block_aligned16(a->workspace))
+      return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_gemm_workspace_bytes), got %zu", need,
+                        a->workspace ? a->workspace_bytes : (size_t)0);
+    p.partial = (float*)a->workspace;
+    const int per = ((p.depth + p.splits - 1) / p.splits + GEMM_BK - 1) / GEMM_BK * GEMM_BK;
+    p.depth_per_split = per;
+    if (int rc = launch_sized<true, true>(p, st, tile)) return rc;
+    const int64_t n8 = (int64_t)p.rows * p.cols / 8;
+    hipLaunchKernelGGL(hstu_gemm_reduce, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm reduction launch: %s", hipGetErrorString(e));
+    return HSTU_BLOCK_OK;
+  }
+  // (one slab may be narrower than a stage, several may not: the kernel moves on by at most one per stage)
+  if (a->op == HSTU_GEMM_NT && a->slabs > 1 && slab < GEMM_BK)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "slabs of at least %d columns are needed here, got %d", GEMM_BK, slab);
+  for (int i = 0; i < HSTU_GEMM_MAX_SLABS; ++i) p.p[i] = (const bf16_t*)a->w[i < a->slabs ? i : a->slabs - 1];
+  p.p_stride = slab;
+  p.rows = (int32_t)a->M;
+  p.out[0] = (bf16_t*)a->out;
+  if (a->op == HSTU_GEMM_NN) {
+    p.cols = p.out_slab = a->N;
+    p.out_stride = a->N;
+    p.depth = p.depth_per_split = a->K;
+    return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth));
+  }
+  p.cols = p.out_slab = a->K;
+  p.out_stride = a->K;
+  p.depth = p.depth_per_split = a->N;
+  return launch_sized<false, false>(p, st, pick_tile(p.rows, p.cols, p.depth));
+}
+
+}  // extern "C"

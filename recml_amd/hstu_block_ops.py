@@ -16,6 +16,7 @@ import ctypes as C
 import torch
 
 from recml_amd import _lib_block
+from recml_amd import _native
 
 _workspaces = {}
 
@@ -63,11 +64,15 @@ def _norm_gate_fwd(attn, u, gamma, beta, eps):
   return out
 
 
-def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None):
+def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None, u_pre=None, add=None):
   """Gradients of u * layer_norm(attn) (of layer_norm(attn) with u=None) for the gradient `dout` of the
   result: (d_attn, d_u, d_gamma, d_beta); d_attn and d_u bf16 shaped like attn, d_gamma and d_beta fp32
   [W], summed over the rows in a fixed order.  `du_out`: where to write d_u (a slice of the gradient
-  of a fused projection, say) instead of a new tensor.  W up to 2048."""
+  of a fused projection, say) instead of a new tensor.  `u_pre`: u is silu(u_pre), and d_u its gradient.
+  `add`: added to d_attn (a gradient that reaches attn another way).  W up to 2048."""
+  got = _native.norm_gate_bwd(attn, u, gamma, beta, dout, eps, du_out, u_pre, add)
+  if got is not None:
+    return got
   for n, t in (("attn", attn), ("gamma", gamma), ("beta", beta), ("dout", dout)) + ((("u", u),) if u is not None else ()):
     _check(n, t)
   if dout.shape != attn.shape or (u is not None and u.shape != attn.shape):
@@ -92,6 +97,18 @@ def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None)
         raise ValueError("du_out must be shaped like attn with a contiguous last axis")
     d2 = du if du.dim() == 2 else du.view(-1, W)     # raises if the leading axes do not collapse: a copy would lose the writes
     a.u, a.u_stride, a.du, a.du_stride = u2.data_ptr(), u2.stride(0), d2.data_ptr(), d2.stride(0)
+  if u_pre is not None:
+    _check("u_pre", u_pre)
+    if u is None or u_pre.shape != attn.shape:
+      raise ValueError("u_pre goes with u and is shaped like it")
+    z2 = _rows(u_pre, "u_pre")
+    a.u_pre, a.u_pre_stride = z2.data_ptr(), z2.stride(0)
+  if add is not None:
+    _check("add", add)
+    if add.shape != attn.shape:
+      raise ValueError("add must be shaped like attn")
+    add2 = _rows(add, "add")
+    a.add, a.add_stride = add2.data_ptr(), add2.stride(0)
   g, b = gamma.reshape(-1).contiguous(), beta.reshape(-1).contiguous()
   if g.numel() != W or b.numel() != W:
     raise ValueError(f"gamma and beta must have {W} entries")
@@ -106,6 +123,9 @@ def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None)
   if rc != 0:
     _raise(lib, rc, "hstu_norm_gate_bwd")
   return da, du, dgb[0], dgb[1]
+
+
+_OWN_NORM_GATE_BWD = norm_gate_bwd    # (how the native graph nodes tell it from something put in its place)
 
 
 class _NormGateFn(torch.autograd.Function):
@@ -227,6 +247,45 @@ def gemm_silu(x, w, bias=None, activation: bool = True, residual=None):
   if rc != 0:
     _raise(lib, rc, "hstu_gemm_silu_fwd")
   return out
+
+
+def block_gemm(op, x, ws, *, y=None, bias=None, residual=None, activation=False, want_pre=False):
+  """The block's matrix products on the package's own kernels (include/hstu_block.h: hstu_gemm).
+
+  op GEMM_NN: act(x @ w + residual + bias), with the value before the activation as a second result when
+  `want_pre`; GEMM_NT: x @ w.T; GEMM_TN: x.T @ y written into the matrices of `ws`.  `ws`: one to four contiguous
+  [K, N / len(ws)] matrices side by side along N."""
+  M, N = x.shape[0], ws[0].shape[1] * len(ws)
+  K = ws[0].shape[0]
+  a = _lib_block.HstuGemmArgs()
+  a.struct_size, a.version = C.sizeof(_lib_block.HstuGemmArgs), _lib_block.ABI_VERSION
+  a.op, a.activation, a.M, a.N, a.K, a.slabs = op, 1 if activation else 0, M, N, K, len(ws)
+  a.x, a.x_stride = x.data_ptr(), x.stride(0)
+  for i, w in enumerate(ws):
+    a.w[i] = w.data_ptr()
+  lib = _lib_block.load()
+  out = pre = ws_buf = None
+  if op == _lib_block.GEMM_TN:
+    a.y, a.y_stride = y.data_ptr(), y.stride(0)
+    need = lib.hstu_gemm_workspace_bytes(op, M, N, K)
+    if need:
+      ws_buf = torch.empty(need, dtype=torch.uint8, device=x.device)
+      a.workspace, a.workspace_bytes = ws_buf.data_ptr(), need
+  else:
+    out = torch.empty((M, N if op == _lib_block.GEMM_NN else K), dtype=x.dtype, device=x.device)
+    a.out = out.data_ptr()
+    if want_pre:
+      pre = torch.empty_like(out)
+      a.pre = pre.data_ptr()
+    if bias is not None:
+      a.bias = bias.data_ptr()
+    if residual is not None:
+      a.c, a.c_stride = residual.data_ptr(), residual.stride(0)
+  with torch.cuda.device(x.device):
+    rc = lib.hstu_gemm(C.byref(a), C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream))
+  if rc != 0:
+    _raise(lib, rc, "hstu_gemm")
+  return (out, pre) if want_pre else out
 
 
 def embed_norm(ids, table, gamma, beta, eps: float = 1e-6, *, scale: float = 1.0, positions=None, pos_table=None):

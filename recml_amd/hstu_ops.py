@@ -1,7 +1,8 @@
 """HSTU pointwise-SiLU attention forward on MI355X: host-side operator.
 
 Three entry points, each a thin argument check over one C call
-(`hstu_attn_fwd`, include/hstu_attn.h):
+(`hstu_attn_fwd`, include/hstu_attn.h), made by the native host side
+(recml_amd/csrc/native.cpp) when the arguments are ready as they are:
 
   hstu_attention              the full op: padded or jagged Q/K/V, per-sequence
                               lengths, relative-position and timestamp bias
@@ -26,6 +27,7 @@ import numpy as np
 import torch
 
 from recml_amd import _lib
+from recml_amd import _native
 
 
 class MaskType(str, enum.Enum):
@@ -126,6 +128,11 @@ class AttentionBatch:
     else:
       self._prepared = None
       self._pending = (sig, tensors)
+
+  def _keep_native(self, signature, workspace, reused, tensors):
+    """What the native block call prepared or reused (its signature is bytes: never equal to one of the Python side's)."""
+    self._prepared, self._buf, self._tensors = signature or None, workspace, tensors
+    self.prepared_calls += 1 if reused else 0
 
   def _commit(self):
     if self._pending is not None:
@@ -398,6 +405,12 @@ def hstu_attention(q, k, v, *, seq_lens=None, seq_offsets=None, max_len=None,
   Returns:
     Tensor shaped like q with v's head dim and v's dtype.
   """
+  if batch is None:
+    got = _native.attention(q, k, v, seq_lens, seq_offsets, max_len, n, alpha, causal, pos_bias, timestamps, ts_bias, ts_bucket_size,
+                            q_segment_ids, kv_segment_ids, sliding_window_size, mask, bias, out, q_scale, k_scale,
+                            dropout_p, dropout_seed, False)
+    if got is not None:
+      return got
   _check_gpu("q", q)
   _check_gpu("v", v)
   if out is None:
@@ -500,6 +513,9 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
   return dq, dk, dv, dpos, dts
 
 
+_OWN_ATTENTION_BWD = hstu_attention_bwd    # (how the native graph nodes tell it from something put in its place)
+
+
 def dropout_keep(seed, p, b, h, H, i, j) -> bool:
   """Whether the weight of (sequence b, head h of H, query i, key j) survives dropout with this seed and
   rate: the library's own rule, evaluated on the host (no GPU needed)."""
@@ -560,7 +576,24 @@ def hstu_attention_autograd(q, k, v, *, pos_bias=None, ts_bias=None, bias=None, 
   """hstu_attention as a differentiable torch op: gradients for q, k, v, the bias tables pos_bias
   and ts_bias, and a dense `bias` (its gradient is dS summed over the heads, and over the batch
   when the bias is shared by it)."""
+  if kwargs.keys() <= _NATIVE_AUTOGRAD:
+    got = _native_autograd(q, k, v, pos_bias, ts_bias, bias, **kwargs)
+    if got is not None:
+      return got
   return _HstuAttentionFn.apply(q, k, v, pos_bias, ts_bias, bias, kwargs)
+
+
+def _native_autograd(q, k, v, pos_bias, ts_bias, bias, seq_lens=None, seq_offsets=None, max_len=None, n=None, alpha=1.0, causal=True,
+                     timestamps=None, ts_bucket_size=0.301, q_segment_ids=None, kv_segment_ids=None, sliding_window_size=None,
+                     mask=None, dropout_p=0.0, dropout_seed=0):
+  """The differentiable call through the native host side; None when its arguments need the Python one."""
+  return _native.attention(q, k, v, seq_lens, seq_offsets, max_len, n, alpha, causal, pos_bias, timestamps, ts_bias, ts_bucket_size,
+                           q_segment_ids, kv_segment_ids, sliding_window_size, mask, bias, None, None, None,
+                           dropout_p, dropout_seed, True)
+
+
+_NATIVE_AUTOGRAD = frozenset(("seq_lens", "seq_offsets", "max_len", "n", "alpha", "causal", "timestamps", "ts_bucket_size",
+                              "q_segment_ids", "kv_segment_ids", "sliding_window_size", "mask", "dropout_p", "dropout_seed"))
 
 
 def pointwise_splash_attention(

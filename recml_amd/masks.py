@@ -21,6 +21,9 @@ def make_causal_mask(mask: torch.Tensor, dtype=torch.float32) -> torch.Tensor:
   return torch.tril(make_attention_mask(mask, dtype=dtype))
 
 
+NOT_END_PADDED = "padding mask is not end-padded; pass an explicit mask instead"
+
+
 def lengths_from_padding_mask(mask: torch.Tensor) -> torch.Tensor:
   """Lengths of an END-padded batch ([B, L] of 0/1 with all 1s first).
 
@@ -32,5 +35,5 @@ def lengths_from_padding_mask(mask: torch.Tensor) -> torch.Tensor:
   L = m.shape[-1]
   prefix = torch.arange(L, device=m.device).unsqueeze(0) < lens.unsqueeze(-1)
   if not bool((prefix == m).all()):
-    raise ValueError("padding mask is not end-padded; pass an explicit mask instead")
+    raise ValueError(NOT_END_PADDED)
   return lens
