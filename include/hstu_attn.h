@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define HSTU_ATTN_ABI_VERSION 3
+#define HSTU_ATTN_ABI_VERSION 4
 
 /* Tensor layouts of q, k, v, out. */
 enum HstuLayout {
@@ -179,6 +179,10 @@ typedef struct HstuAttnFwdArgs {
   float dropout_p;        /* in [0, 1)                                        */
   uint32_t reserved0;     /* 0                                                */
   uint64_t dropout_seed;
+  /* Row pitch of `mask` (bytes) and of `dense_bias` (floats); 0: Lkv, a contiguous matrix.  The matrix-core kernels
+   * fetch rows in 16-byte pieces: a matrix whose Lkv does not allow that can be handed over with rows a few elements
+   * longer (hstu_attn_pad_rows makes such a copy; at most 15 more, zeros there).  ddense_bias stays [.., L, Lkv]. */
+  int64_t mask_pitch, bias_pitch;
 } HstuAttnFwdArgs;
 
 /* Whether dropout keeps pair (query i, key j) of sequence b and head h (of H
@@ -186,6 +190,10 @@ typedef struct HstuAttnFwdArgs {
  * checkers.  i and j count from the start of the sequence.  Always 1 for
  * dropout_p = 0. */
 int hstu_attn_dropout_keep(uint64_t dropout_seed, float dropout_p, int32_t b, int32_t h, int32_t H, int32_t i, int32_t j);
+
+/* Copies `rows` rows of n elements (of 1 or 4 bytes) to rows `pitch` elements apart, zeros behind each; a pitch of whole
+ * 16-byte pieces, dst 16-byte aligned.  Enqueued on `stream`. */
+int hstu_attn_pad_rows(const void* src, void* dst, int64_t rows, int32_t n, int32_t pitch, int32_t element_bytes, void* stream);
 
 /* ABI version of the loaded library (HSTU_ATTN_ABI_VERSION at build time). */
 int hstu_attn_abi_version(void);

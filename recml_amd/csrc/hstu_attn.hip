@@ -101,6 +101,7 @@ struct Params {
   int32_t B, L, Lkv, H, d_qk, d_v;
   int32_t jagged, causal, mask_mode, window;
   int32_t mask_batched, dense_bias_batched, pos_heads, ts_heads;
+  int32_t mask_pitch, bias_pitch;   // bytes and floats from one row of the keep-mask and of the dense bias to the next
   int32_t ts_nb;
   float ts_bucket_size;
   float alpha, inv_n;
@@ -2362,7 +2363,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
     __shared__ int mr_lo[4], mr_hi[4];
     __shared__ unsigned int kbits[MASK_PRES_MAX_KT];      // per key tile: which of the tile's four 32-row steps keep a pair there
     const int nb = p.mask_batched ? p.B : 1;
-    const int ppr = p.Lkv / 16;
+    const int ppr = p.mask_pitch / 16;
     const int n_kt = (p.Lkv + BM - 1) / BM;
     const bool pres_on = p.mask_pres && n_kt <= MASK_PRES_MAX_KT;
     uint8_t* pres = (uint8_t*)(mrange_out + 2 * (int64_t)nb * p.n_qtiles);
@@ -2370,7 +2371,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
       const int b = tile / p.n_qtiles, qt = tile - b * p.n_qtiles;
       const int r0 = qt * BM;
       const int rows = p.L - r0 < BM ? p.L - r0 : BM;
-      const uint4* mg = (const uint4*)(p.mask + ((int64_t)b * p.L + r0) * p.Lkv);
+      const uint4* mg = (const uint4*)(p.mask + ((int64_t)b * p.L + r0) * p.mask_pitch);
       const int n = rows * ppr;
       int lo = 0x7fffffff, hi = 0;
       if (pres_on) {
@@ -2739,7 +2740,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       // 4w .. 4w+3 (8 rows each, the rows of its own queries); lane l of a piece lands at row l / 8,
       // physical chunk l % 8.  Rows past L and keys past Lkv re-read the last row / the last four keys:
       // finite data for logits that are masked by their index.
-      const float* dbg = p.dense_bias + (p.dense_bias_batched ? (int64_t)c_.b * p.L * p.Lkv : 0);
+      const float* dbg = p.dense_bias + (p.dense_bias_batched ? (int64_t)c_.b * p.L * p.bias_pitch : 0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = 4 * w + r;
@@ -2747,19 +2748,19 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
         int gr = c_.q0 + row;
         gr = gr < p.L - 1 ? gr : p.L - 1;
         int col = kv0 + 4 * (pc ^ (row & 7));
-        col = col < p.Lkv - 4 ? col : p.Lkv - 4;
-        lds_dma16(dbg, ((uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col) * 4u, Db() + j * 1024);
+        col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
+        lds_dma16(dbg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Db() + j * 1024);
       }
     }
     if (DENSE & 2) {
       // Mask tile: row r at LDS byte 32 r; wave w brings its own 32 rows, two lanes per row.
-      const uint8_t* mg = p.mask + (p.mask_batched ? (int64_t)c_.b * p.L * p.Lkv : 0);
+      const uint8_t* mg = p.mask + (p.mask_batched ? (int64_t)c_.b * p.L * p.mask_pitch : 0);
       const int row = 32 * w + (lane >> 1);
       int gr = c_.q0 + row;
       gr = gr < p.L - 1 ? gr : p.L - 1;
       int col = kv0 + 16 * (lane & 1);
-      col = col < p.Lkv - 16 ? col : p.Lkv - 16;
-      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col, Dm() + w * 1024);
+      col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
+      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Dm() + w * 1024);
     }
   };
   // The lane's share of the dense operands that have landed: 16 bias values (keys 8g + 4hh .. +3 of its
@@ -3839,26 +3840,26 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     if (MSK) {
       // the wave's own 32 rows of the step's mask tile, two lanes per row; rows past L and the second half of a last
       // step of 16 keys re-read bytes inside the matrix (those pairs are masked by their index)
-      const uint8_t* mg = p.mask + (p.mask_batched ? (int64_t)b * p.L * p.Lkv : 0);
+      const uint8_t* mg = p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0);
       int gr = r0 + (lane >> 1);
       gr = gr < p.L - 1 ? gr : p.L - 1;
       int col = kv0 + 16 * (lane & 1);
-      col = col < p.Lkv - 16 ? col : p.Lkv - 16;
-      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col, Mk(st) + w * 1024);
+      col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
+      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Mk(st) + w * 1024);
     }
     if (DB) {
       // the wave's own 32 rows of the step's bias tile in four pieces of 8 rows: row r at byte 128 r, lane l of a piece
       // lands at row l / 8, physical chunk l % 8, and fetches the logical chunk the swizzle maps there.  Rows past L
       // and keys past Lkv re-read the last row / the last four keys (those pairs are masked by their index).
-      const float* bg = p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0);
+      const float* bg = p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 32 * w + 8 * r + (lane >> 3), pc = lane & 7;
         int gr = q0 + row;
         gr = gr < p.L - 1 ? gr : p.L - 1;
         int col = kv0 + 4 * (pc ^ (row & 7));
-        col = col < p.Lkv - 4 ? col : p.Lkv - 4;
-        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
+        col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
+        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
       }
     }
   };
@@ -4502,24 +4503,24 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
     if (MSK) {
       // rows 8w .. 8w + 7 of the step's mask tile, eight lanes per row (16 bytes each = this tile's 128 keys); rows past
       // L and pieces past Lkv re-read bytes inside the matrix (those pairs are masked by their index)
-      const uint8_t* mg = (const uint8_t*)scalar_ptr(p.mask + (p.mask_batched ? (int64_t)b * p.L * p.Lkv : 0));
+      const uint8_t* mg = (const uint8_t*)scalar_ptr(p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0));
       int gr = qbs + 8 * w + (lane >> 3);
       gr = gr < p.L - 1 ? gr : p.L - 1;
       int col = kv0 + 16 * (lane & 7);
-      col = col < p.Lkv - 16 ? col : p.Lkv - 16;
-      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col, Mk(st) + w * 1024);
+      col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
+      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Mk(st) + w * 1024);
     }
     if (DB) {
       // rows 8w .. 8w + 7 of the step's bias tile in four pieces of two rows (512 bytes a row = this tile's 128 keys);
       // rows past L and pieces past Lkv re-read values inside the matrix (those pairs are masked by their index)
-      const float* bg = (const float*)scalar_ptr(p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0));
+      const float* bg = (const float*)scalar_ptr(p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0));
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         int gr = qbs + 8 * w + 2 * r + (lane >> 5);
         gr = gr < p.L - 1 ? gr : p.L - 1;
         int col = kv0 + 4 * (lane & 31);
-        col = col < p.Lkv - 4 ? col : p.Lkv - 4;
-        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.Lkv + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
+        col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
+        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
       }
     }
   };
@@ -4920,6 +4921,9 @@ int effective_window(const HstuAttnFwdArgs* a) {
   return (a->window >= 0 && a->window < longest) ? a->window : -1;
 }
 
+// The row pitch of a dense operand: the caller's, or that of a contiguous [.., L, Lkv] matrix.
+int dense_pitch(const HstuAttnFwdArgs* a, int64_t pitch) { return pitch ? (int)pitch : a->Lkv; }
+
 // Whether the matrix-core kernel covers these arguments (dtype aside: bf16, or fp8 q/k).
 bool mfma_eligible(const HstuAttnFwdArgs* a) {
   const int kb = a->qk_dtype == HSTU_DTYPE_FP8_E4M3FN ? 1 : 2;   // bytes per q / k element
@@ -4932,9 +4936,9 @@ bool mfma_eligible(const HstuAttnFwdArgs* a) {
   const bool dense = a->mask || a->dense_bias;
   const bool dense_ok = !dense ||
       (kb == 2 && !a->pos_tab && !a->ts_tab && a->mask_mode != HSTU_MASK_SEGMENT &&
-       (!a->dense_bias || (a->Lkv % 4 == 0 && aligned16(a->dense_bias))) &&
-       (!a->mask || (a->Lkv % 16 == 0 && aligned16(a->mask))) &&
-       (int64_t)a->L * a->Lkv * 4 < (1LL << 32));
+       (!a->dense_bias || (dense_pitch(a, a->bias_pitch) % 4 == 0 && aligned16(a->dense_bias))) &&
+       (!a->mask || (dense_pitch(a, a->mask_pitch) % 16 == 0 && aligned16(a->mask))) &&
+       (int64_t)a->L * (a->Lkv + 15) * 4 < (1LL << 32));
   // keys and queries of different lengths: the padded layout without the table biases (whose geometry needs one length)
   const bool len_ok = a->L == a->Lkv || (a->layout == HSTU_LAYOUT_PADDED && !a->pos_tab && !a->ts_tab);
   const bool opts_ok = seg_ok && dense_ok && len_ok &&
@@ -4962,6 +4966,10 @@ int validate(const HstuAttnFwdArgs* a) {
                                    HSTU_FWD_RESIDENT_WORKGROUPS | HSTU_FWD_COMPILER_SCHEDULED_BLOCKS;
   if ((uint32_t)a->flags & ~known_flags) return fail(HSTU_ERR_SHAPE, "unknown bits in flags: 0x%x", (unsigned)a->flags);
   if (!(a->dropout_p >= 0.0f && a->dropout_p < 1.0f)) return fail(HSTU_ERR_SHAPE, "dropout_p must be in [0, 1), got %g", (double)a->dropout_p);
+  if (a->mask_pitch != 0 && (a->mask_pitch < a->Lkv || a->mask_pitch > a->Lkv + 15)) return fail(HSTU_ERR_SHAPE, "mask_pitch must be 0 or in [Lkv, Lkv + 15], got %lld", (long long)a->mask_pitch);
+  if (a->bias_pitch != 0 && (a->bias_pitch < a->Lkv || a->bias_pitch > a->Lkv + 15)) return fail(HSTU_ERR_SHAPE, "bias_pitch must be 0 or in [Lkv, Lkv + 15], got %lld", (long long)a->bias_pitch);
+  if ((a->mask_pitch > a->Lkv || a->bias_pitch > a->Lkv) && !mfma_eligible(a))
+    return fail(HSTU_ERR_SHAPE, "rows of a dense operand further apart than Lkv are for the matrix-core kernel's calls");
   if (a->reserved0 != 0u) return fail(HSTU_ERR_SHAPE, "reserved0 must be 0");
   const bool empty = a->B == 0 || (a->layout == HSTU_LAYOUT_JAGGED && a->total_tokens == 0);
   if (!empty && (!a->q || !a->k || !a->v || !a->out))
@@ -5122,6 +5130,7 @@ Params make_params(const HstuAttnFwdArgs* a) {
   p.causal = a->causal != 0;
   p.mask_mode = p.jagged ? HSTU_MASK_LENGTH : a->mask_mode;
   p.window = effective_window(a);
+  p.mask_pitch = dense_pitch(a, a->mask_pitch); p.bias_pitch = dense_pitch(a, a->bias_pitch);
   p.mask_batched = a->mask_batched; p.dense_bias_batched = a->dense_bias_batched;
   p.pos_heads = a->pos_heads; p.ts_heads = a->ts_heads;
   p.ts_nb = a->ts_num_buckets;
@@ -5516,6 +5525,21 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
 #endif
 }
 
+// Rows of n elements to rows `pitch` apart, zeros in between: one workgroup per row and 256 16-byte pieces of it.
+template <typename T>
+__global__ __launch_bounds__(256) void hstu_pad_rows(const T* __restrict__ src, T* __restrict__ dst, int64_t rows, int n, int pitch) {
+  constexpr int PER = 16 / sizeof(T);
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * PER;
+  if (c >= pitch) return;
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    const T* s = src + row * n;
+    T v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) v[i] = c + i < n ? s[c + i] : (T)0;
+    *(uint4*)(dst + row * pitch + c) = *(const uint4*)v;
+  }
+}
+
 }  // namespace
 
 // Scratch of hstu_attn_fwd_noalloc: the workspace of a forward call, built into the library so that
@@ -5570,6 +5594,20 @@ int hstu_attn_bucket_thresholds(float bucket_size, int32_t* thresholds, int coun
   return law.reach + 1;
 }
 
+int hstu_attn_pad_rows(const void* src, void* dst, int64_t rows, int32_t n, int32_t pitch, int32_t element_bytes, void* stream) {
+  if (rows < 0 || n < 1 || pitch < n || (element_bytes != 1 && element_bytes != 4) || (pitch * element_bytes & 15))
+    return fail(HSTU_ERR_SHAPE, "pad_rows: rows >= 0, pitch >= n of whole 16-byte pieces and elements of 1 or 4 bytes expected");
+  if (rows == 0) return HSTU_OK;
+  if (!src || !dst || !aligned16(dst)) return fail(HSTU_ERR_NULL, "pad_rows: src and a 16-byte aligned dst are needed");
+  const int pieces = pitch * element_bytes / 16;
+  const dim3 grid((unsigned)(rows < 65536 ? rows : 65536), (unsigned)((pieces + 255) / 256)), block(pieces < 256 ? ((pieces + 63) / 64 * 64) : 256);
+  if (element_bytes == 1) hipLaunchKernelGGL(hstu_pad_rows<uint8_t>, grid, block, 0, (hipStream_t)stream, (const uint8_t*)src, (uint8_t*)dst, rows, n, pitch);
+  else hipLaunchKernelGGL(hstu_pad_rows<float>, grid, block, 0, (hipStream_t)stream, (const float*)src, (float*)dst, rows, n, pitch);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "pad_rows launch: %s", hipGetErrorString(e));
+  return HSTU_OK;
+}
+
 const char* hstu_attn_fwd_variant(const HstuAttnFwdArgs* args) {
   if (validate(args) != HSTU_OK) return "invalid";
   switch (pick_variant(args)) {
@@ -5615,6 +5653,8 @@ int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) {
   if (p.dbias && !p.dense_bias) return fail(HSTU_ERR_NULL, "ddense_bias needs the forward's dense_bias");
   hipStream_t st = (hipStream_t)stream;
   if (bwd_mfma_eligible(args)) return launch_bwd_mfma(args, p, st);
+  if (f->mask_pitch > f->Lkv || f->bias_pitch > f->Lkv)
+    return fail(HSTU_ERR_SHAPE, "rows of a dense operand further apart than Lkv are for the matrix-core kernels' calls");
   // (the general kernels sum the bucket table's gradient in LDS first, one float per entry)
   if (p.dts && p.ts_tab && p.ts_nb > 4095)
     return fail(HSTU_ERR_SHAPE, "the gradient of a timestamp table of more than 4096 entries is not supported, got %d", p.ts_nb + 1);

@@ -1,0 +1,55 @@
+"""Dense masks and biases whose rows are no whole 16-byte pieces, in bf16 on the matrix-core kernels.
+
+The host side gives such a matrix longer rows (hstu_attn_pad_rows) when that is all that keeps a call off the matrix-core
+kernels; lengths around the kernels' tiles (32 keys, 128 rows) and around the pieces (4 floats, 16 mask bytes)."""
+
+import numpy as np
+import pytest
+import torch
+
+import recml_amd
+from oracle import hstu_oracle as O
+
+pytestmark = pytest.mark.gpu
+bf = torch.bfloat16
+
+
+def _dev(x, dtype=None):
+  t = torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")
+  return t if dtype is None else t.to(dtype)
+
+
+def _rel(a, b):
+  return np.abs(a - b).max() / max(np.abs(b).max(), 1e-30)
+
+
+@pytest.mark.parametrize("L", [1, 15, 33, 127, 131, 248, 302])
+@pytest.mark.parametrize("d,with_mask,with_bias,shared", [(64, True, True, False), (32, True, False, True), (128, False, True, False), (128, True, True, True)])
+def test_dense_rows_of_any_length(gpu, L, d, with_mask, with_bias, shared):
+  rng = np.random.default_rng(100 * L + d)
+  B, H = 2, 2
+  q, k, v, dout = (O.round_bf16(rng.standard_normal((B, L, H, d)).astype(np.float32) * 0.4) for _ in range(4))
+  nb = 1 if shared else B
+  mask = (rng.random((nb, L, L)) > 0.3) & (np.arange(L)[None, None, :] <= np.arange(L)[None, :, None]) if with_mask else None
+  if mask is not None and shared:
+    mask = mask[0]
+  bias = (rng.standard_normal((nb, L, L)) * 0.4).astype(np.float32) if with_bias else None
+  kw = dict(n=float(L), alpha=0.3, causal=not with_mask)
+  ref = O.hstu_attention_ref(q, k, v, mask=mask, bias=bias, **kw)
+  want = O.hstu_attention_bwd_ref(q, k, v, dout, mask=mask, bias=bias, bias_grad=with_bias, **kw)
+  gk = dict(kw, mask=None if mask is None else _dev(mask))
+  bt = None if bias is None else _dev(bias).requires_grad_(True)
+  ts = [_dev(x, bf).requires_grad_(True) for x in (q, k, v)]
+  out = recml_amd.hstu_attention_autograd(*ts, bias=bt, **gk)
+  out.backward(_dev(dout, bf))
+  variant = []
+  again = recml_amd.hstu_attention_bwd(*(t.detach() for t in ts), _dev(dout, bf), bias=None if bt is None else bt.detach(), bias_grad=with_bias,
+                                       _variant_out=variant, **gk)
+  torch.cuda.synchronize()
+  assert variant == ["hstu_bwd_mfma_bf16"]
+  assert _rel(out.detach().float().cpu().numpy(), ref) <= 2e-2
+  for nm, t, g, w in zip(("dq", "dk", "dv"), ts, again[:3], want[:3]):
+    assert torch.equal(t.grad, g), nm                      # both host sides, the same kernels
+    assert _rel(g.float().cpu().numpy(), w) <= 2e-2, nm
+  if with_bias:
+    assert _rel(bt.grad.cpu().numpy(), want[5]) <= 2e-2
