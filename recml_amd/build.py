@@ -10,7 +10,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(_HERE)
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libhstu_attn.so")
-SOURCES = [os.path.join(_HERE, "csrc", "hstu_attn.hip")]
+SOURCES = [os.path.join(_HERE, "csrc", "hstu_attn.hip"), os.path.join(_HERE, "csrc", "hstu_f32.hip")]
 # the block-side steps live in a library of their own: they bring hipBLASLt along, the attention does not
 BLOCK_LIB_PATH = os.path.join(LIB_DIR, "libhstu_block.so")
 BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip"), os.path.join(_HERE, "csrc", "hstu_gemm.hip")]

@@ -58,165 +58,16 @@
 
 #include <type_traits>
 
-#include "hstu_attn.h"
+#include "hstu_attn_common.h"
+
+using namespace hstu;
 
 namespace {
-
-typedef __bf16 bf16_t;
-typedef bf16_t bf16x8 __attribute__((ext_vector_type(8)));
-typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-struct Params {
-  const void* q;
-  const void* k;
-  const void* v;
-  void* out;
-  int64_t q_sb, q_st, q_sh;
-  int64_t k_sb, k_st, k_sh;
-  int64_t v_sb, v_st, v_sh;
-  int64_t o_sb, o_st, o_sh;
-  const int32_t* seq_lens;
-  const int32_t* seq_offsets;
-  const int32_t* q_seg;
-  const int32_t* kv_seg;
-  const uint8_t* mask;
-  const float* dense_bias;
-  const float* pos_tab;
-  const float* ts_tab;
-  const int64_t* ts;
-  const float* pos_scaled;   // workspace: log2(e) * pos_tab, zero-padded (MFMA kernel)
-  // workspace of the MFMA kernel's timestamp path: per sequence, 1 when max - min timestamp fits
-  // 31 bits; then timestamps minus the sequence minimum as int32, and their (min, max) per 32-key tile
-  const int32_t* ts_ok;
-  const int32_t* ts_rel;
-  const int32_t* ts_range;
-  const int4* ts_keyed;      // workspace: the bucket tables [heads][3 KB], see TsKeys
-  const void* ws_base;       // start of the workspace (all of the above lie within 4 GB of it)
-  const float* q_scale;      // [H] or null: dequantisation scales of fp8 q / k
-  const float* k_scale;
-  int64_t ts_sb;
-  int32_t B, L, Lkv, H, d_qk, d_v;
-  int32_t jagged, causal, mask_mode, window;
-  int32_t mask_batched, dense_bias_batched, pos_heads, ts_heads;
-  int32_t mask_pitch, bias_pitch;   // bytes and floats from one row of the keep-mask and of the dense bias to the next
-  int32_t ts_nb;
-  float ts_bucket_size;
-  float alpha, inv_n;
-  int32_t n_qtiles;
-  // Key-range splitting (MFMA forward; off when split_cap == 0): hstu_prepare, which sees the lengths,
-  // shares a query tile with more steps than twice a slot's average load between up to MAX_CHUNKS workgroups,
-  // each covering a contiguous part of the keys and leaving its fp32 partial O^T in `partial`; the
-  // workgroup that arrives last at the tile's counter sums them and writes the rows.
-  int32_t split_cap;         // chunk slots of the partial buffer (per head)
-  int32_t n_slots;           // workgroups that run at once per XCD (what the split decision balances for)
-  const int32_t* mask_range; // workspace: per (mask batch, query tile) the first 32-key step with a kept pair and one past the last
-  int32_t persist;           // forward: resident workgroups that loop over the work list
-  int32_t no_stream;         // forward: interior steps through the compiler-scheduled block code too (a comparison switch)
-  int32_t mask_pres;         // the preparation also fills the dense mask's presence table (the backward asks for it)
-  // Dropout on the attention weights: pair (b, h, i, j) is kept when drop_hash(...) >= drop_thr (0: no dropout).
-  // The survivors' scale 1 / (1 - p) is folded into inv_n by the host.
-  uint32_t drop_thr, drop_key;
-  // Timestamp descriptors (matrix-core forward at d = 128; null = none): one 16-bit word per (32-key step, query
-  // row), [step][row] with `ts_desc_pitch` rows per step, built by hstu_prepare (ts_desc_block) for every head and layer of
-  // a batch; and per (128-row tile, chunk of TS_DESC_CHUNK steps) the first step in which some row needs the per-pair
-  // lookup (INT32_MAX: none).
-  const uint16_t* ts_desc;
-  const int32_t* ts_tquads;
-  int32_t ts_desc_pitch;
-  int32_t ts_desc_tiles;     // tile slots of ts_tquads
-  int32_t ts_desc_chunks;    // entries per tile slot: chunks of TS_DESC_CHUNK steps
-  float* partial;            // [chunk slot][head][BM x d_v floats in register order]
-  uint32_t* ctr;             // workspace: [0, 8) draw counters of the XCDs, [8] workgroups done, then from
-                             // CTR_RESERVED on one arrival counter per (chunk slot, head); all zero between launches
-  // Work list built on the device by hstu_prepare (MFMA kernel; null = workgroups enumerate every
-  // possible (sequence, tile) and most exit): sched[0] = number of items, then from
-  // sched[4] on one int4 per (sequence, query tile, chunk) that has work:
-  // {b | first chunk slot << 14, qt | chunk << 16 | chunks << 24, first token, stored length}.
-  const int32_t* sched;
-  // backward pass: gradient of out in, gradients of q, k, v out (layouts of out, q, k, v), and
-  // fp32 table gradients that are accumulated into (null = not wanted)
-  const void* dout;
-  void* dq;
-  void* dk;
-  void* dv;
-  float* dpos;
-  float* dts;
-  float* dbias;              // gradient of the dense bias (general backward), or null
-  int64_t items_max;         // capacity of the list (sizes the grid)
-};
-
-// Per-sequence geometry shared by both kernels.
-struct Seq {
-  int n_q;        // query rows that produce output
-  int n_kv;       // keys that may be attended
-  int rows;       // rows of the output tile space (L, or n_b when jagged)
-  int64_t tok0;   // first token of the sequence in the token axis
-  int64_t bq, bk, bv, bo;  // element offsets of (token 0, head h)
-  int64_t ts0;    // element offset of timestamp 0
-  int n_ts;       // timestamps addressable for this sequence
-};
-
-// o0: first token (jagged layout); nraw: the sequence's length as stored (offset difference or
-// seq_lens entry; ignored for the padded layout without a length mask).
-__device__ __forceinline__ Seq seq_from(const Params& p, int b, int h, int o0, int nraw) {
-  Seq s;
-  if (p.jagged) {
-    int n = nraw;
-    n = n < 0 ? 0 : (n > p.L ? p.L : n);
-    s.n_q = n; s.n_kv = n; s.rows = n; s.tok0 = o0;
-    s.bq = (int64_t)o0 * p.q_st + (int64_t)h * p.q_sh;
-    s.bk = (int64_t)o0 * p.k_st + (int64_t)h * p.k_sh;
-    s.bv = (int64_t)o0 * p.v_st + (int64_t)h * p.v_sh;
-    s.bo = (int64_t)o0 * p.o_st + (int64_t)h * p.o_sh;
-  } else {
-    int nq = p.L, nk = p.Lkv;
-    if (p.mask_mode == HSTU_MASK_LENGTH) {
-      int n = nraw;
-      n = n < 0 ? 0 : n;
-      nq = n < p.L ? n : p.L;
-      nk = n < p.Lkv ? n : p.Lkv;
-    }
-    s.n_q = nq; s.n_kv = nk; s.rows = p.L; s.tok0 = 0;
-    s.bq = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
-    s.bk = (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
-    s.bv = (int64_t)b * p.v_sb + (int64_t)h * p.v_sh;
-    s.bo = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
-  }
-  if (p.ts_sb != 0) { s.ts0 = (int64_t)b * p.ts_sb; s.n_ts = p.L; }
-  else              { s.ts0 = s.tok0;               s.n_ts = s.n_kv; }
-  return s;
-}
-
-__device__ __forceinline__ void seq_raw(const Params& p, int b, int& o0, int& nraw) {
-  o0 = 0;
-  nraw = p.L;
-  if (p.jagged) {
-    o0 = p.seq_offsets[b];
-    nraw = p.seq_offsets[b + 1] - o0;
-  } else if (p.mask_mode == HSTU_MASK_LENGTH) {
-    nraw = p.seq_lens[b];
-  }
-}
-
-__device__ __forceinline__ Seq seq_info(const Params& p, int b, int h) {
-  int o0, nraw;
-  seq_raw(p, b, o0, nraw);
-  return seq_from(p, b, h, o0, nraw);
-}
-
-__device__ __forceinline__ float ldf(const float* p) { return *p; }
-__device__ __forceinline__ float ldf(const bf16_t* p) { return (float)*p; }
-__device__ __forceinline__ void stf(float* p, float x) { *p = x; }
-__device__ __forceinline__ void stf(bf16_t* p, float x) { *p = (bf16_t)x; }
 
 // ---------------------------------------------------------------------------
 // General kernel: fp32 FMA arithmetic, every option.
 // ---------------------------------------------------------------------------
 
-constexpr float LOG2E = 1.4426950408889634f;
 constexpr int GT = 32;       // query rows and keys per tile
 constexpr int GMAXX = 32;    // d_v / 8 accumulators per thread, d_v <= 256
 // floats of the general backward's timestamp-bucket histogram in LDS: one per table entry, a multiple of four
@@ -399,34 +250,6 @@ __device__ __forceinline__ void general_dense_col(const Params& p, int b, int i0
     int i = i0 + 8 * (r >> 2) + 4 * hh + (r & 3);
     v[r] = col[(int64_t)(i < p.L - 1 ? i : p.L - 1) * p.Lkv];
   }
-}
-// Dropout's keep rule: a counter-based hash of (seed, b, h, i, j), the same on the host, in every kernel and in
-// the CPU oracle.  drop_seed_key folds the 64-bit seed (host, once per call), drop_bh_key the sequence and the
-// head (once per work item), drop_keep the pair: two multiply-add steps on the indices, of which a kernel hoists
-// the one that is fixed for its lane, then drop_keep_mixed.
-__host__ __device__ inline uint32_t drop_seed_key(uint64_t seed) {
-  uint32_t z = (uint32_t)seed ^ 0x9E3779B9u;
-  z = (z ^ (z >> 16)) * 0x85EBCA6Bu;
-  z ^= (uint32_t)(seed >> 32);
-  z = (z ^ (z >> 13)) * 0xC2B2AE35u;
-  return z ^ (z >> 16);
-}
-__host__ __device__ inline uint32_t drop_bh_key(uint32_t key, uint32_t bh) {
-  uint32_t z = key + bh * 0x9E3779B1u;
-  z = (z ^ (z >> 15)) * 0x2C1B3C6Du;
-  return z ^ (z >> 13);
-}
-constexpr uint32_t DROP_CI = 0x85EBCA77u, DROP_CJ = 0xC2B2AE3Du;
-// ij = kbh + i * DROP_CI + j * DROP_CJ (wrapping)
-// (two multiplications with one fold of the high half onto the low half between them: the comparison reads the product
-// from its top bits down, which depend on every bit of ij; seven instructions per pair with the index step and the select)
-__host__ __device__ inline bool drop_keep_mixed(uint32_t ij, uint32_t thr) {
-  uint32_t z = ij * 0x2C1B3C6Du;
-  z = (z ^ (z >> 16)) * 0x297A2D39u;
-  return z >= thr;
-}
-__host__ __device__ inline bool drop_keep(uint32_t kbh, uint32_t i, uint32_t j, uint32_t thr) {
-  return drop_keep_mixed(kbh + i * DROP_CI + j * DROP_CJ, thr);
 }
 // The 16 values a lane holds in a 32 x 32 block sit at offsets c(r) = 8 (r / 4) + r % 4 along the axis that is not the
 // lane's own: ij0 carries everything else, `step` is that axis's multiplier.  One value after the other on purpose (the
@@ -4843,13 +4666,17 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
 
 thread_local char g_err[512] = "";
 
-int fail(int code, const char* fmt, ...) {
+}  // namespace
+
+int hstu::fail(int code, const char* fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
   return code;
 }
+
+namespace {
 
 enum Variant { V_INVALID = 0, V_GENERAL_F32, V_GENERAL_BF16, V_MFMA_BF16, V_MFMA_FP8 };
 
@@ -4859,7 +4686,6 @@ enum Variant { V_INVALID = 0, V_GENERAL_F32, V_GENERAL_BF16, V_MFMA_BF16, V_MFMA
 // kernels and the CPU oracle share.  `keys` is the part of the matrix-core kernels' keyed table that does
 // not depend on the bias values, `keyed_ok` whether that table can represent this bucket size (at most
 // one boundary per key range, bucket indices within the backward's histogram).
-constexpr int LAW_THR_LEN = 256;
 struct BucketLaw {
   float size;
   bool valid, keyed_ok;
@@ -4911,6 +4737,16 @@ const BucketLaw& bucket_law(float size_f) {
   law.valid = true;
   return law;
 }
+
+}  // namespace
+
+int hstu::bucket_thresholds(float bucket_size, const int32_t** thr) {
+  const BucketLaw& law = bucket_law(bucket_size);
+  *thr = law.thr;
+  return law.reach;
+}
+
+namespace {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -5160,6 +4996,7 @@ int allow_lds(const void* fn, int bytes, int* granted /* [kMaxDev] */) {
 
 template <typename T>
 int launch_general(const Params& p, hipStream_t st) {
+  if (f32_takes(p, sizeof(T) == 2, false)) return f32_launch_fwd(p, sizeof(T) == 2, st);
   const bool small = p.d_qk <= 128 && p.d_v <= 128;
   if (p.B > 65535 || (p.L + 127) / 128 > 65535)
     return fail(HSTU_ERR_SHAPE, "the general kernel takes at most 65535 sequences and 65535 tiles of 128 rows per call (B = %d, L = %d)", p.B, p.L);
@@ -5220,6 +5057,7 @@ bool general_bwd_bf16_products(const Params& p) {
 // where the rows allow), larger ones by the FMA kernels.
 template <typename T>
 int launch_bwd(const Params& p, hipStream_t st) {
+  if (f32_takes(p, sizeof(T) == 2, true)) return f32_launch_bwd(p, sizeof(T) == 2, st);
   if (p.B > 65535) return fail(HSTU_ERR_SHAPE, "the general backward takes at most 65535 sequences per call, got %d", p.B);
   if (p.d_qk <= 128 && p.d_v <= 128) {
     // (each wave's block of dS goes through LDS for the position table's diagonal sums and for the dense bias's row-wise adds)
