@@ -3500,17 +3500,24 @@ template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ float dpp_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xf, true));
 }
-// sum of v over the 64 lanes, the same value in every lane (all lanes must be active)
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_f<0x111>(v);
-  v += dpp_f<0x112>(v);
-  v += dpp_f<0x114>(v);
-  v += dpp_f<0x118>(v);
-  v += dpp_f<0x142, 0xa>(v);
-  v += dpp_f<0x143, 0xc>(v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+// v of the lane CTRL names for the upper 32 lanes (0 where there is none), `lower` for the others
+template <int CTRL>
+__device__ __forceinline__ float dpp_upper(float lower, float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, lower), __builtin_bit_cast(int, v), CTRL, 0xc, 0xf, true));
 }
-
+// a's upper 32 lanes against b's lower 32; a's odd rows of 16 against b's even ones
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  const unsigned x = r[0], y = r[1];       // (a bit cast of a vector's element takes element 0)
+  a = __builtin_bit_cast(float, x);
+  b = __builtin_bit_cast(float, y);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  const unsigned x = r[0], y = r[1];       // (a bit cast of a vector's element takes element 0)
+  a = __builtin_bit_cast(float, x);
+  b = __builtin_bit_cast(float, y);
+}
 // float atomic add on an LDS location given by an ordinary pointer (named as LDS for the compiler: on
 // a pointer of unknown address space it builds a run-time dispatch that some instantiations miscompile)
 typedef __attribute__((address_space(3))) float* lds_float_ptr;
@@ -3748,6 +3755,9 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
   const int vc2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
   const int c_lo = vc2 ^ hh, c_hi = vc2 ^ (hh + 2);
 
+  // (timestamp-table gradient: the lane's bucket of the last block and what is summed for it)
+  int sum_bucket = 0;
+  float sum_s = 0.f;
   auto block = [&](int t) {
     const int st = t % NSTAGE;
     const int kbs = t * BN;
@@ -3776,11 +3786,11 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     // lane holds S^T[kv = kbs + 8g + 4hh + tt][q = qrow], r = 4g + tt
     float u[16];
     // for the table gradients: either this lane's 16 pairs are in bucket bk_lane >= 0, those with a bit
-    // in far_bits in the next one (then every lane of the wave has such a pair of buckets), or bkp holds
+    // before `cut` in the next one (then every lane of the wave has such a pair of buckets), or bkp holds
     // the 16 buckets, one byte each (bucket < TS_TAB_LEN <= 255)
     uint32_t bkp[4] = {0u, 0u, 0u, 0u};
-    uint32_t far_bits = 0u;
-    int bk_lane = -1;
+    int bk_lane = -1, cut = (int)0x80000000;
+    bool far_keys = false;
     if (POS) {
       const int xb = 4 * hh + (BM - 1) - 32 * w - m;
       const int sft = xb & 3;
@@ -3825,7 +3835,8 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           // bucket exactly when tq - tk >= thr, i.e. tk <= tq - thr (a lane whose ends share a bucket
           // must not flag any key: the next bucket's sum would take its dS)
           const float add_near = en.v_near, add_far = en.v_far;
-          const int cut = en.b_far != en.b_near ? tq32 - en.thr : (int)0x80000000;
+          cut = en.b_far != en.b_near ? tq32 - en.thr : (int)0x80000000;
+          far_keys = true;
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
@@ -3834,7 +3845,6 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
             u[4 * g + 1] += f1 ? add_far : add_near;
             u[4 * g + 2] += f2 ? add_far : add_near;
             u[4 * g + 3] += f3 ? add_far : add_near;
-            if (TG) far_bits |= ((uint32_t)f0 | ((uint32_t)f1 << 1) | ((uint32_t)f2 << 2) | ((uint32_t)f3 << 3)) << (4 * g);
           }
           bk_lane = en.b_near;
         } else {
@@ -3944,59 +3954,67 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
       }
     }
     if (want_dpos) {
-      // Pair (row m, key offset c = 8g + 4hh + tt) lies on diagonal c - m.  Lane j takes, for each of
-      // its 16 offsets, the value of row (j + c) mod 32 of its half: all 16 are then on diagonal -j or,
-      // where j + c wrapped, 32 - j.  The two sums are completed with the other half's and added to
-      // the wave's ring: lanes of the lower half own -j, lanes of the upper half 32 - j.
-      // (the lane's index enters through a register the compiler cannot see through: it would otherwise
-      // keep the 16 permute addresses of the loop below in registers across the whole key loop, which
-      // this kernel does not have)
-      int jj = m + 4 * hh;
-      if (D == 128) asm volatile("" : "+v"(jj));        // (smaller head dims have the 16 registers)
-      const int half4 = (lane & 32) << 2;
-      float s_all = 0.f, s_low = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c0 = 8 * (r >> 2) + (r & 3);
-        const int addr = (((jj + c0) & 31) << 2) | half4;
-        const float rv = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(addr, __builtin_bit_cast(int, ds[r])));
-        s_all += rv;
-        s_low += (jj + c0 < 32) ? rv : 0.f;
-      }
-      const float s_high = s_all - s_low;
-      const float mine = hh ? s_high : s_low, theirs = hh ? s_low : s_high;
-      const float got = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, theirs)));
+      // Pair (row m, key offset c = 8g + 4hh + tt) lies on diagonal c - m.  Within a row of 16 lanes (p = m % 16, query half
+      // qh = m / 16) a shift by c0 % 16, c0 = c - 4hh, brings a register's values onto diagonals 16 k - p + 4hh - 16 qh: k = c0 / 16
+      // for the lanes it keeps, one more for those that come in from the other end, so three sums take all of them, by
+      // additions whose operand is shifted on the way (31, where a lane permute per value took 16 of them and as many selects).
+      float t0 = 0.f, t1 = 0.f, t2 = 0.f;
+#define HSTU_DIAG(G, T) { \
+      constexpr int cp = 8 * ((G) & 1) + (T); \
+      const float v = ds[4 * (G) + (T)]; \
+      const float keepv = cp == 0 ? v : dpp_f<0x100 + (cp == 0 ? 1 : cp)>(v); \
+      const float wrapv = cp == 0 ? 0.f : dpp_f<0x110 + (cp == 0 ? 1 : 16 - cp)>(v); \
+      if constexpr ((G) < 2) { t0 += keepv; if constexpr (cp != 0) t1 += wrapv; } \
+      else { t1 += keepv; if constexpr (cp != 0) t2 += wrapv; } }
+      HSTU_DIAG(0, 0) HSTU_DIAG(0, 1) HSTU_DIAG(0, 2) HSTU_DIAG(0, 3)
+      HSTU_DIAG(1, 0) HSTU_DIAG(1, 1) HSTU_DIAG(1, 2) HSTU_DIAG(1, 3)
+      HSTU_DIAG(2, 0) HSTU_DIAG(2, 1) HSTU_DIAG(2, 2) HSTU_DIAG(2, 3)
+      HSTU_DIAG(3, 0) HSTU_DIAG(3, 1) HSTU_DIAG(3, 2) HSTU_DIAG(3, 3)
+#undef HSTU_DIAG
+      // the upper half's four lanes further on (rows 2 and 3 only): then both halves are on 16 k - p - 16 qh
+      const float w0 = t0, w1 = t1;
+      t0 = dpp_upper<0x104>(t0, w0);
+      t1 = dpp_upper<0x104>(t1, w1) + dpp_upper<0x11c>(0.f, w0);
+      t2 = dpp_upper<0x104>(t2, t2) + dpp_upper<0x11c>(0.f, w1);
+      // the halves' sums; then rows [k = 0, 1, 2, -] of the lower query half in `lo`, of the upper in `up`, which lies one k
+      // further down: diagonal 16 i - 16 - p in row i of the total
+      swap32(t0, t1);
+      float lo = t0 + t1, up = 0.f;
+      swap32(t2, up);
+      up += t2;
+      swap32(lo, up);
+      swap16(lo, up);
+      const float diag = up + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane - 16) & 63) << 2, __builtin_bit_cast(int, lo)));
       // the workgroup's ring of diagonal sums: this wave's diagonal X is the workgroup's X + 96 - 32 w (a lane per
       // slot within the instruction; other waves may add to the same slots, hence the atomic form)
-      lds_atomic_add(TgBase + ((kbs + 127 - m + 32 * hh - 32 * w) & (TG_WG_RING - 1)), mine + got);
+      lds_atomic_add(TgBase + ((kbs + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_WG_RING - 1)), diag);
     }
     if (want_dts) {
       float* hist = TgBase + NWAVES * TG_RING;
       if (bk_lane >= 0) {
-        float s_near = 0.f, s_far = 0.f;
+        // A lane's bucket changes with the step only now and then (the nearer the keys, the smaller): its sum stays in a
+        // register until it does, and reaches the histogram then, by an LDS atomic of the lanes concerned.
+        float s_near = ((ds[0] + ds[1]) + (ds[2] + ds[3])) + ((ds[4] + ds[5]) + (ds[6] + ds[7])) +
+                       (((ds[8] + ds[9]) + (ds[10] + ds[11])) + ((ds[12] + ds[13]) + (ds[14] + ds[15])));
+        if (far_keys) {
+          const int32_t* tk = Tk(st);
+          float s_far = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const bool far = (far_bits >> r) & 1u;
-          s_near += far ? 0.f : ds[r];
-          s_far += far ? ds[r] : 0.f;
-        }
-        // lanes with the same bucket are summed together, one bucket value per round
-        const bool any_far = __builtin_amdgcn_ballot_w64(far_bits != 0u) != 0;
-        bool done = false;
-        for (;;) {
-          const uint64_t act = __builtin_amdgcn_ballot_w64(!done);
-          if (act == 0) break;
-          const int leader = __builtin_ctzll(act);
-          const int b0 = __builtin_amdgcn_readlane(bk_lane, leader);
-          const bool mine = !done && bk_lane == b0;
-          const float a = wave_sum(mine ? s_near : 0.f);
-          const float c = any_far ? wave_sum(mine ? s_far : 0.f) : 0.f;
-          if (lane == 0) {
-            lds_atomic_add(&hist[b0], a);
-            if (any_far) lds_atomic_add(&hist[b0 + 1], c);
+          for (int g = 0; g < 4; ++g) {
+            const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
+            s_far += (kk.x <= cut ? ds[4 * g] : 0.f) + (kk.y <= cut ? ds[4 * g + 1] : 0.f);
+            s_far += (kk.z <= cut ? ds[4 * g + 2] : 0.f) + (kk.w <= cut ? ds[4 * g + 3] : 0.f);
           }
-          done = done || mine;
+          s_near -= s_far;
+          if (sum_bucket == bk_lane + 1) sum_s += s_far;
+          else if (s_far != 0.f) lds_atomic_add(&hist[bk_lane + 1], s_far);
         }
+        if (sum_bucket != bk_lane) {
+          if (sum_s != 0.f) lds_atomic_add(&hist[sum_bucket], sum_s);
+          sum_bucket = bk_lane;
+          sum_s = 0.f;
+        }
+        sum_s += s_near;
       } else {
         // LDS atomics cost by the lane: neighbouring keys mostly share a bucket, so each run of equal
         // buckets is summed first, and runs that add nothing (masked pairs) are skipped
@@ -4080,7 +4098,8 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     flush_diag(32 * t_last + 64 * w);
   }
   if (want_dts) {
-    // every wave is past the loop's last barrier: the histogram is complete
+    if (sum_s != 0.f) lds_atomic_add(TgBase + NWAVES * TG_RING + sum_bucket, sum_s);
+    __syncthreads();                     // the histogram is complete
     const float* hist = TgBase + NWAVES * TG_RING;
     for (int e = tid; e < TS_TAB_LEN; e += MFMA_THREADS) {
       const float val = hist[e];
@@ -4122,16 +4141,23 @@ __device__ __forceinline__ void mfma_acc(floatx16& acc, bf16x8 a, bf16x8 b) {
 }
 
 // Ring depth of the dK/dV kernel (see there).
-constexpr int dkv_stages(int d, bool dense_bias) { return (d == 128 && !dense_bias) ? 6 : NSTAGE; }
+constexpr int dkv_stages(int d, bool dense_bias, bool wide) { return (d == 128 && !dense_bias && !wide) ? 6 : NSTAGE; }
 
-template <int D>
+// WIDE (d = 128 without a dense bias, other than the stream's instance): eight waves, two per SIMD.  Waves w and w + 4
+// share 32 keys and take the even and the odd steps; K and V come from LDS (in registers next to the accumulators of 32
+// keys they leave room for one wave per SIMD only, which ran every block's products, vector part and waits one after the
+// other), and at the end the two waves exchange halves of their sums.
+template <int D, bool WIDE>
 struct DkvShape {
-  static constexpr bool ACC_ASM = D == 128;
-  static constexpr int DSPLIT = 1;                       // waves per 32 keys
-  static constexpr int NW = NWAVES * DSPLIT;             // waves per workgroup
+  static constexpr bool ACC_ASM = D == 128 && !WIDE;
+  static constexpr int QSPLIT = WIDE ? 2 : 1;            // waves per 32 keys
+  static constexpr int NW = NWAVES * QSPLIT;             // waves per workgroup
   static constexpr int THREADS = 64 * NW;
-  static constexpr int DW = D / DSPLIT;                  // channels of dK / dV per wave
+  static constexpr int KV_BYTES = WIDE ? 2 * BM * D * 2 : 0;   // K and V rows of the tile
 };
+constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dense_bias) {
+  return d == 128 && !dense_bias && (pos || ts || seg || mask);
+}
 
 // MSK: the dense keep-mask as in the other backward kernel; here a step's tile is 32 query rows x this workgroup's
 // 128 keys (wave w fetches rows 8w .. 8w + 7 of it, 128 bytes each), a lane reads the 16 bytes of its key's column,
@@ -4140,14 +4166,15 @@ struct DkvShape {
 // reads the 16 values of its key's column (consecutive lanes, consecutive words: no swizzle needed).  The bias's
 // gradient is the other kernel's business.
 template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false>
-__global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) void hstu_bwd_dkv_mfma(const Params p) {
-  using SH = DkvShape<D>;
-  constexpr int NW = SH::NW, THREADS = SH::THREADS, DW = SH::DW;
+__global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB)>::THREADS), ((D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB)) || DB ? 1 : 2))
+void hstu_bwd_dkv_mfma(const Params p) {
+  constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB);
+  using SH = DkvShape<D, WIDE>;
+  constexpr int NW = SH::NW, THREADS = SH::THREADS;
   constexpr bool ACC_ASM = SH::ACC_ASM;
   // A pair of blocks that needs no mask runs as one hand-scheduled instruction stream (hstu_bwd_stream_d128.inc,
   // written by gen_bwd_stream.py): the vector part of one block behind the matrix instructions of the other.
-  constexpr bool STREAM = D == 128 && !POS && !TS && !SEG && !MSK && !DB && SH::DSPLIT == 1;
-  constexpr int DVBW = DW / 32;          // 32-channel blocks of dK / dV per wave
+  constexpr bool STREAM = D == 128 && !POS && !TS && !SEG && !MSK && !DB;
   using SM = MfmaSmem<D, 2>;
   constexpr int CPR = SM::CPR;
   constexpr int QCH = D / 16;
@@ -4158,10 +4185,10 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   // Ring depth: 4 stages (two pairs of steps: one at work, one on its way), or 6 where the workgroup has the CU's
   // LDS to itself anyway (d = 128) and the stages are small enough: the loads of a pair then have the time of two
   // pairs to arrive, which the hand-scheduled pairs need (one pair's time is less than a trip to memory).
-  constexpr int NST = dkv_stages(D, DB);
+  constexpr int NST = dkv_stages(D, DB, WIDE);
   constexpr int AHEAD = NST - 2;           // steps between a load and its use
   static_assert((NST - 1) * NDMA <= 63, "vmcnt range");
-  static_assert(!(MSK || DB) || (!POS && !TS && !SEG && SH::DSPLIT == 1), "dense operands come without the table biases and the segment ids");
+  static_assert(!(MSK || DB) || (!POS && !TS && !SEG), "dense operands come without the table biases and the segment ids");
   // timestamp operands of a step: 36 int32 query-side timestamps (rows qbs .. qbs + 35), then the
   // (min, max) of timestamp tiles t and t + 1
   constexpr int TQ_LANES = BN / 4 + 2;
@@ -4181,6 +4208,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   auto Wc = [&](int st) { return (float*)(smem + BIAS_OFF + st * BIAS_STAGE); };
   auto Tq = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0)); };
   const unsigned char* TsKey = smem + BIAS_OFF + NST * BIAS_STAGE;   // the keyed bucket table of this head
+  unsigned char* const KvLds = smem + BIAS_OFF + NST * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0);   // WIDE: [K | V], 128 rows each, swizzled like the tiles
 
   Work wk;
   if (!work_of_block(p, blockIdx.x, wk)) return;
@@ -4198,7 +4226,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   const int lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = w8 % NWAVES;            // which 32 keys of the tile
-  const int dh = w8 / NWAVES;           // which part of the channels
+  const int qh = w8 / NWAVES;           // WIDE: which step of a pair
   const int m = lane & 31, hh = lane >> 5;
   const char* __restrict__ qg = (const char*)scalar_ptr((const char*)p.q + s.bq * 2);
   const char* __restrict__ dog = (const char*)scalar_ptr((const char*)p.dout + s.bo * 2);
@@ -4259,7 +4287,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
         hi = hi > lo ? hi : lo;
       }
     } else {
-      general_mask_live_steps<false>(p, b, kv0, tid, lo, hi);
+      general_mask_live_steps<false>(p, b, kv0, tid & 255, lo, hi);    // (WIDE: both halves the same)
     }
     t_lo = lo;
     nt = hi > lo ? hi : lo;
@@ -4359,10 +4387,22 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   for (int i = 0; i < AHEAD; ++i)
     if (t_lo + i < nt) dma_step(t_lo + i);
 
-  // K and V fragments of this lane's key (B operands)
+  // K and V fragments of this lane's key (B operands); WIDE: the tile's rows in LDS (rows past the sequence repeat its last)
   typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-  uintx4 hs_k[QCH], hs_v[QCH];
-  {
+  uintx4 hs_k[WIDE ? 1 : QCH], hs_v[WIDE ? 1 : QCH];
+  if constexpr (WIDE) {
+    const char* kg = (const char*)scalar_ptr((const char*)p.k + s.bk * 2);
+    const char* vg = (const char*)scalar_ptr((const char*)p.v + s.bv * 2);
+    constexpr int PIECES = BM * D * 2 / 1024;
+    for (int i = w8; i < PIECES; i += NW) {
+      const int c = 64 * i + lane, row = c / CPR, pc = c - row * CPR;
+      int grow = kv0 + row;
+      grow = grow < s.n_kv - 1 ? grow : s.n_kv - 1;
+      const uint32_t sw = (uint32_t)((pc ^ swz_rt<D>(row)) * 16);
+      lds_dma16(kg, (uint32_t)grow * ((uint32_t)p.k_st * 2u) + sw, KvLds + i * 1024);
+      lds_dma16(vg, (uint32_t)grow * ((uint32_t)p.v_st * 2u) + sw, KvLds + BM * D * 2 + i * 1024);
+    }
+  } else {
     uint4 kfr[QCH], vfr[QCH];
     const char* kp = (const char*)p.k + (s.bk + (int64_t)kcol * p.k_st) * 2 + 16 * hh;
     const char* vp = (const char*)p.v + (s.bv + (int64_t)kcol * p.v_st) * 2 + 16 * hh;
@@ -4396,9 +4436,9 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
     asm volatile("" ::"v"(tk), "v"(tk32));
   }
 
-  floatx16 dka[DVBW], dva[DVBW];
+  floatx16 dka[DVB], dva[DVB];
 #pragma unroll
-  for (int i = 0; i < DVBW; ++i) {
+  for (int i = 0; i < DVB; ++i) {
     if (ACC_ASM) {
       mfma_acc_zero<STREAM>(dka[i]);
       mfma_acc_zero<STREAM>(dva[i]);
@@ -4420,7 +4460,41 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
     const int st = (t - t_lo) % NST;      // (a pair of steps starts at an even stage)
     const int qbs = t * BN;
     const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // The block's bucket or pair of buckets first: its chain of table reads runs under the products.  The time differences
+    // of this lane's key to the step's rows lie between those to the smallest and to the largest timestamp of the two tiles
+    // the rows come from.
+    TsEnds en;
+    bool one_bucket = false, two_buckets = false;
+    if (TS && ts32) {
+      const int4 rg = *(const int4*)(Tq(st) + 4 * (TQ_LANES - 1));
+      const int t_min = rg.x < rg.z ? rg.x : rg.z, t_max = rg.y > rg.w ? rg.y : rg.w;
+      en = ts_ends(TsKey, t_min - tk32, t_max - tk32);
+      one_bucket = __builtin_amdgcn_ballot_w64(!en.same) == 0;
+      two_buckets = __builtin_amdgcn_ballot_w64(!en.two) == 0;
+    }
     floatx16 sacc, dpacc;
+    if constexpr (WIDE) {
+      // Row m of each tile against row 32 w + m of the keys'.  The two chains take turns, and the fragments of a product are
+      // asked for two products ahead (left to itself the compiler has no registers for more than the next one, and every
+      // product waits for LDS): the order is fixed by scheduling barriers.
+      const unsigned char* const qr = (const unsigned char*)Qs(st) + m * (D * 2);
+      const unsigned char* const kr = KvLds + (32 * w + m) * (D * 2);
+      uint4 af[3], bf[3];
+      auto ask = [&](int i) __attribute__((always_inline)) {          // product i: S for even i, dP for odd, channels 16 (i / 2) ..
+        const int at = ((2 * (i >> 1) + hh) ^ gk) * 16;
+        af[i % 3] = *(const uint4*)(qr + at + (i & 1) * SM::K_BYTES);
+        bf[i % 3] = *(const uint4*)(kr + at + (i & 1) * (BM * D * 2));
+      };
+      ask(0);
+      ask(1);
+#pragma unroll
+      for (int i = 0; i < 2 * QCH; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < 2 * QCH) ask(i + 2);
+        floatx16& d = (i & 1) ? dpacc : sacc;
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i % 3]), __builtin_bit_cast(bf16x8, bf[i % 3]), i < 2 ? zero : d, 0, 0, 0);
+      }
+    } else {
     {
       uint4 af[QCH];
       const unsigned char* ar = (const unsigned char*)Qs(st) + m * (D * 2);
@@ -4440,6 +4514,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
       for (int ks = 0; ks < QCH; ++ks)
         dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[ks]), __builtin_bit_cast(bf16x8, hs_v[ks]),
                                                         ks == 0 ? zero : dpacc, 0, 0, 0);
+    }
     }
     float u[16];
     if (POS) {
@@ -4475,45 +4550,58 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
         return iq < qbs ? qbs : iq;                 // only for rows past the sequence (masked below)
       };
       if (ts32) {
-        // the time differences of this lane's key to the step's rows lie between those to the
-        // smallest and to the largest timestamp of the two tiles the rows come from
-        const int4 rg = *(const int4*)(tqs + 4 * (TQ_LANES - 1));
-        const int t_min = rg.x < rg.z ? rg.x : rg.z, t_max = rg.y > rg.w ? rg.y : rg.w;
-        const TsEnds en = ts_ends(TsKey, t_min - tk32, t_max - tk32);
-        if (__builtin_amdgcn_ballot_w64(!en.same) == 0) {
+        if (one_bucket) {
           const float add = en.v_near;
 #pragma unroll
           for (int r = 0; r < 16; ++r) u[r] += add;
-        } else if (__builtin_amdgcn_ballot_w64(!en.two) == 0) {
-          // one bucket boundary at most: the farther bucket exactly when tq - tk >= thr
-          const float add_near = en.v_near, add_far = en.v_far;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) u[r] += tqs[tq_at(r) - qbs] - tk32 >= en.thr ? add_far : add_near;
         } else {
+          // the 16 rows' timestamps: away from the sequence's end four consecutive words per group, one further on than an
+          // aligned read has them
+          int tqv[16];
+          if (qbs + BN < s.n_ts) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) u[r] += ts_value(ts_look(TsKey, tqs[tq_at(r) - qbs] - tk32));
+            for (int g = 0; g < 4; ++g) {
+              const int4 a = *(const int4*)(tqs + 8 * g + 4 * hh);
+              tqv[4 * g] = a.y; tqv[4 * g + 1] = a.z; tqv[4 * g + 2] = a.w;
+              tqv[4 * g + 3] = tqs[8 * g + 4 * hh + 4];
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tqv[r] = tqs[tq_at(r) - qbs];
+          }
+          if (two_buckets) {
+            // one bucket boundary at most: the farther bucket exactly when tq - tk >= thr (none of the three is negative)
+            const float add_near = en.v_near, add_far = en.v_far;
+            const uint32_t cut = (uint32_t)en.thr + (uint32_t)tk32;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) u[r] += (uint32_t)tqv[r] >= cut ? add_far : add_near;
+          } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) u[r] += ts_value(ts_look(TsKey, tqv[r] - tk32));
+          }
         }
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r) u[r] += ts_value(ts_look(TsKey, ts_clip64(tsg[tq_at(r)] - tk)));
       }
     }
-    // transposed fragments of dO (for dV) and of Q (for dK)
-    uint4 otf[2][DVBW], qtf[2][DVBW];
-    {
-      const bf16_t* orr = Os(st) + vrow * D + 4 * (gi & 1);
-      const bf16_t* qrr = Qs(st) + vrow * D + 4 * (gi & 1);
+    // transposed fragments of dO (for dV) and of Q (for dK); WIDE: ahead of their products
+    const bf16_t* const orr = Os(st) + vrow * D + 4 * (gi & 1);
+    const bf16_t* const qrr = Qs(st) + vrow * D + 4 * (gi & 1);
+    auto frag_tr = [&](const bf16_t* rows, int cc, int dvb) __attribute__((always_inline)) {
+      const int cb = 4 * (dvb ^ swz_rt_group<D>(gi));
+      const uint2 lo = lds_read_tr(rows + (16 * cc) * D + (cb + c_lo) * 8);
+      const uint2 hi = lds_read_tr(rows + (16 * cc + 8) * D + (cb + c_hi) * 8);
+      return uint4{lo.x, lo.y, hi.x, hi.y};
+    };
+    uint4 otf[2][WIDE ? 1 : DVB], qtf[2][WIDE ? 1 : DVB];
+    if constexpr (!WIDE) {
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-        for (int dvb = 0; dvb < DVBW; ++dvb) {
-          const int cb = 4 * ((dh * DVBW + dvb) ^ swz_rt_group<D>(gi));
-          uint2 lo = lds_read_tr(orr + (16 * cc) * D + (cb + c_lo) * 8);
-          uint2 hi = lds_read_tr(orr + (16 * cc + 8) * D + (cb + c_hi) * 8);
-          otf[cc][dvb] = uint4{lo.x, lo.y, hi.x, hi.y};
-          lo = lds_read_tr(qrr + (16 * cc) * D + (cb + c_lo) * 8);
-          hi = lds_read_tr(qrr + (16 * cc + 8) * D + (cb + c_hi) * 8);
-          qtf[cc][dvb] = uint4{lo.x, lo.y, hi.x, hi.y};
+        for (int dvb = 0; dvb < DVB; ++dvb) {
+          otf[cc][dvb] = frag_tr(orr, cc, dvb);
+          qtf[cc][dvb] = frag_tr(qrr, cc, dvb);
         }
     }
     float pv[16], ds[16];
@@ -4568,6 +4656,29 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
       drop_apply16(pv, ds, drop_bh_key(p.drop_key, (uint32_t)b * (uint32_t)p.H + (uint32_t)h) + (uint32_t)kcol * DROP_CJ +
                                (uint32_t)(qbs + 4 * hh) * DROP_CI, DROP_CI, p.drop_thr);
     }
+    if constexpr (WIDE) {
+      // the accumulating products, dV and dK in turn, their fragments two products ahead
+      uint4 pk[2], dk4[2], tf[3];
+#pragma unroll
+      for (int cc = 0; cc < 2; ++cc) {
+        pk[cc] = uint4{pack_bf16(pv[8 * cc + 0], pv[8 * cc + 1]), pack_bf16(pv[8 * cc + 2], pv[8 * cc + 3]),
+                       pack_bf16(pv[8 * cc + 4], pv[8 * cc + 5]), pack_bf16(pv[8 * cc + 6], pv[8 * cc + 7])};
+        dk4[cc] = uint4{pack_bf16(ds[8 * cc + 0], ds[8 * cc + 1]), pack_bf16(ds[8 * cc + 2], ds[8 * cc + 3]),
+                        pack_bf16(ds[8 * cc + 4], ds[8 * cc + 5]), pack_bf16(ds[8 * cc + 6], ds[8 * cc + 7])};
+      }
+      auto ask = [&](int i) __attribute__((always_inline)) { tf[i % 3] = frag_tr((i & 1) ? qrr : orr, i / (2 * DVB), (i >> 1) % DVB); };
+      ask(0);
+      ask(1);
+#pragma unroll
+      for (int i = 0; i < 4 * DVB; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < 4 * DVB) ask(i + 2);
+        const bf16x8 bb = __builtin_bit_cast(bf16x8, (i & 1) ? dk4[i / (2 * DVB)] : pk[i / (2 * DVB)]);
+        floatx16& d = (i & 1) ? dka[(i >> 1) % DVB] : dva[(i >> 1) % DVB];
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf[i % 3]), bb, d, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
       uint4 pk, dk4;
@@ -4581,7 +4692,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
       dk4.w = pack_bf16(ds[8 * cc + 6], ds[8 * cc + 7]);
       const bf16x8 pb = __builtin_bit_cast(bf16x8, pk), db = __builtin_bit_cast(bf16x8, dk4);
 #pragma unroll
-      for (int dvb = 0; dvb < DVBW; ++dvb) {
+      for (int dvb = 0; dvb < DVB; ++dvb) {
         if (ACC_ASM) {
           mfma_acc<STREAM>(dva[dvb], __builtin_bit_cast(bf16x8, otf[cc][dvb]), pb);
           mfma_acc<STREAM>(dka[dvb], __builtin_bit_cast(bf16x8, qtf[cc][dvb]), db);
@@ -4590,6 +4701,7 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
           dka[dvb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, qtf[cc][dvb]), db, dka[dvb], 0, 0, 0);
         }
       }
+    }
     }
     // The compiler does not know of the matrix instructions above: whatever it puts behind them (a copy of an
     // accumulator at a join of two paths, say) must find the last product's result in place.
@@ -4634,6 +4746,11 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   };
   auto block_pair = [&](int t) __attribute__((always_inline)) {
     const int n_sent = send_ahead(t);
+    if constexpr (WIDE) {
+      if (t + qh < nt && wave_live && t + qh >= t_wave && t + qh <= t_wave_end) block(t + qh);
+      end_of_pair(n_sent);
+      return;
+    }
     if (wave_live && t >= t_wave && t <= t_wave_end) block(t);
     if (t + 1 < nt && wave_live && t + 1 >= t_wave && t + 1 <= t_wave_end) block(t + 1);
     end_of_pair(n_sent);
@@ -4655,9 +4772,38 @@ __global__ __launch_bounds__(DkvShape<D>::THREADS, (D == 128 || DB) ? 1 : 2) voi
   for (; t < nt; t += 2) block_pair(t);
 
   if (ACC_ASM) asm volatile("s_nop 15\n\ts_nop 15");   // the last product has left the pipeline before its result is read
-  unsigned char* ot = smem + w8 * (32 * DW * 2);
-  store_rows<DW>(dka, p.alpha * p.inv_n, ot, dkg + dh * DW, p.k_st, r0, s.n_kv, s.rows, lane);
-  store_rows<DW>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg + dh * DW, p.v_st, r0, s.n_kv, s.rows, lane);
+  if constexpr (WIDE) {
+    // The pair of waves on the same keys: the first sums and stores dK, the second dV; each hands the other's half over
+    // through LDS (16 KB a wave; the loop's last barrier is behind everyone).
+    float4* const give = (float4*)(smem + w8 * (64 * D * 2));
+    float4* const take = (float4*)(smem + (w8 ^ NWAVES) * (64 * D * 2));
+    auto swap_halves = [&](floatx16 (&mine)[DVB], const floatx16 (&other)[DVB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < DVB; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) give[(4 * i + g) * 64 + lane] = float4{other[i][4 * g], other[i][4 * g + 1], other[i][4 * g + 2], other[i][4 * g + 3]};
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < DVB; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 v = take[(4 * i + g) * 64 + lane];
+          mine[i][4 * g] += v.x; mine[i][4 * g + 1] += v.y; mine[i][4 * g + 2] += v.z; mine[i][4 * g + 3] += v.w;
+        }
+    };
+    unsigned char* const ot = (unsigned char*)take;       // (read by this wave alone)
+    if (qh == 0) {
+      swap_halves(dka, dva);
+      store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, p.k_st, r0, s.n_kv, s.rows, lane);
+    } else {
+      swap_halves(dva, dka);
+      store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, p.v_st, r0, s.n_kv, s.rows, lane);
+    }
+  } else {
+    unsigned char* ot = smem + w8 * (32 * D * 2);
+    store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, p.k_st, r0, s.n_kv, s.rows, lane);
+    store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, p.v_st, r0, s.n_kv, s.rows, lane);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -5309,10 +5455,11 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   const int smem = MfmaSmem<D, 2>::total(POS, TS, SEG) + (MSK ? NSTAGE * MfmaSmem<D, 2>::DM_BYTES : 0) +
                    (DB ? NSTAGE * MfmaSmem<D, 2>::DB_BYTES : 0);
   const int smem_q = smem + (TG ? BWD_TG_BYTES : 0);
-  constexpr int nst_kv = dkv_stages(D, DB);
+  using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB)>;
+  constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB));
   const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + (MSK ? nst_kv * MfmaSmem<D, 2>::DM_BYTES : 0) +
                       (DB ? nst_kv * MfmaSmem<D, 2>::DB_BYTES : 0) +
-                      (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
+                      SH::KV_BYTES + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
   static int granted_q[64], granted_kv[64];
   if (int rc = allow_lds((const void*)hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>, smem_q, granted_q)) return rc;
   if (int rc = allow_lds((const void*)hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>, smem_kv, granted_kv)) return rc;
@@ -5321,7 +5468,7 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   hipLaunchKernelGGL((hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>), dim3((unsigned)blocks), dim3(MFMA_THREADS), smem_q, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dq kernel launch: %s", hipGetErrorString(e));
-  hipLaunchKernelGGL((hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>), dim3((unsigned)blocks), dim3(DkvShape<D>::THREADS), smem_kv, st, p);
+  hipLaunchKernelGGL((hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>), dim3((unsigned)blocks), dim3(SH::THREADS), smem_kv, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dk/dv kernel launch: %s", hipGetErrorString(e));
   return HSTU_OK;
