@@ -49,6 +49,17 @@ __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_addr_wav
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(base), "v"(src) : "memory", "m0");
 }
 
+// The same with a scalar base and a 32-bit lane offset.
+__device__ __forceinline__ void lds_dma16(const char* base_uniform, uint32_t off, uint32_t lds_addr_wave_uniform) {
+  const uint32_t to = __builtin_amdgcn_readfirstlane(lds_addr_wave_uniform);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(to), "v"(off), "s"(base_uniform) : "memory", "m0");
+}
+__device__ __forceinline__ const char* scalar_ptr(const void* p) {
+  const uint64_t v = (uint64_t)(uintptr_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (const char*)(uintptr_t)(((uint64_t)hi << 32) | lo);
+}
+
 #define HSTU_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | ((((n) >> 4) & 3) << 14)) | 0x0F70)
 
 // One workgroup: a tile of 64 MB output rows x 64 NB output columns, four waves of 32 MB x 32 NB.  The contraction runs in
@@ -62,7 +73,11 @@ __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_addr_wav
 //   Why 256 x 128 (MB 4, NB 2): with 64 x 64 per wave the four SIMDs' fragments take all of the LDS bandwidth (128 bytes a
 // clock) at full matrix rate, with 128 x 64 three quarters of it; 128 accumulators leave two workgroups per CU, so that one's
 // barriers and stores run under the other's products.
-template <int MB, int NB, bool Q_T, bool P_T, int STAGES = 3>
+//   UNIFORM: a tile's columns of P (a stage's, where P lies along the contraction) are in one slab.  A load is then a scalar base
+// that moves on with the stage and a lane offset that never changes; rows and columns past an operand's end repeat its last
+// (what they give is not stored), and only the stage that crosses the contraction's end tests its elements.  Per-lane
+// pointers, counters and slab hops were three of the ten vector instructions behind every matrix instruction.
+template <int MB, int NB, bool Q_T, bool P_T, int STAGES, bool UNIFORM>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmParams g) {
   constexpr int TM = 64 * MB, TN = 64 * NB;
   constexpr int Q_BYTES = TM * GEMM_BK * 2, P_BYTES = TN * GEMM_BK * 2, STAGE = Q_BYTES + P_BYTES;
@@ -148,11 +163,72 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmPa
       pp[i] = (const char*)((sl == 0 ? g.p[0] : sl == 1 ? g.p[1] : sl == 2 ? g.p[2] : g.p[3]) + (int64_t)n * g.p_stride + pc[i]);
     }
   }
+  // (UNIFORM: lane offsets; the scalar bases follow from the stage)
+  uint32_t qo[LQ], uo[LP];
+  const char *q_base = nullptr, *p_base = nullptr;
+  int u_k = k_begin, u_slab = 0, u_col = 0;      // contraction index of the next stage to load; P along it: its slab and column there
+  if constexpr (UNIFORM) {
+#pragma unroll
+    for (int i = 0; i < LQ; ++i) {
+      Src s = src_of(Q_T, TM, w * LQ + i);
+      const int most = g.rows - (Q_T ? 8 : 1) - m0;
+      s.outer = s.outer < most ? s.outer : most;
+      qo[i] = Q_T ? (uint32_t)(s.k * (int)g.q_stride + s.outer) * 2u : (uint32_t)(s.outer * (int)g.q_stride + s.k) * 2u;
+      qk[i] = s.k;
+    }
+#pragma unroll
+    for (int i = 0; i < LP; ++i) {
+      Src s = src_of(P_T, TN, w * LP + i);
+      const int most = g.cols - (P_T ? 8 : 1) - n0;
+      s.outer = s.outer < most ? s.outer : most;
+      uo[i] = P_T ? (uint32_t)(s.k * (int)g.p_stride + s.outer) * 2u : (uint32_t)(s.outer * (int)g.p_stride + s.k) * 2u;
+      pk[i] = s.k;
+    }
+    q_base = scalar_ptr(Q_T ? g.q + (int64_t)k_begin * g.q_stride + m0 : g.q + (int64_t)m0 * g.q_stride + k_begin);
+    if (P_T) {
+      const int sl = n0 / g.slab;
+      p_base = scalar_ptr(g.p[sl] + (int64_t)k_begin * g.p_stride + (n0 - sl * g.slab));
+    } else {
+      u_slab = k_begin / g.slab;
+      u_col = k_begin - u_slab * g.slab;
+      p_base = scalar_ptr(g.p[u_slab] + (int64_t)n0 * g.p_stride + u_col);
+    }
+  }
   const int64_t q_step = Q_T ? (int64_t)GEMM_BK * g.q_stride * 2 : GEMM_BK * 2;
   const int64_t p_step = (int64_t)GEMM_BK * g.p_stride * 2;
   constexpr int NLOAD = LQ + LP;     // of a stage, per wave
   auto issue_one = [&](int st, int i) {
     const uint32_t base = smem_lds + (uint32_t)st * STAGE;
+    if constexpr (UNIFORM) {
+      const bool whole = u_k + GEMM_BK <= k_end;
+      const uint32_t to = i < LQ ? base + 1024u * (w * LQ + i) : base + Q_BYTES + 1024u * (w * LP + i - LQ);
+      const char* from = i < LQ ? q_base : p_base;
+      const uint32_t off = i < LQ ? qo[i < LQ ? i : 0] : uo[i < LQ ? 0 : i - LQ];
+      if (whole) {
+        lds_dma16(from, off, to);
+      } else {
+        const int k = u_k + (i < LQ ? qk[i < LQ ? i : 0] : pk[i < LQ ? 0 : i - LQ]);
+        lds_dma16(k < k_end ? (const void*)(from + off) : (const void*)(gemm_zeros + 16 * (lane & 15)), to);
+      }
+      if (i == NLOAD - 1) {       // on to the next stage (past the end the bases stay: everything there is zeros)
+        u_k += GEMM_BK;
+        if (u_k < k_end) {
+          q_base += q_step;
+          if (P_T) {
+            p_base += p_step;
+          } else {
+            u_col += GEMM_BK;
+            p_base += GEMM_BK * 2;
+            if (u_col >= g.slab) {
+              u_col = 0;
+              ++u_slab;
+              p_base = scalar_ptr(g.p[u_slab] + (int64_t)n0 * g.p_stride);
+            }
+          }
+        }
+      }
+      return;
+    }
     if (i < LQ) {
       const void* src = qk[i] < k_end ? (const void*)qp[i] : (const void*)(gemm_zeros + 16 * (lane & 15));
       lds_dma16(src, base + 1024u * (w * LQ + i));
@@ -316,8 +392,10 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmPa
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] += cv[e];
           }
+          if (g.bias) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] += bias[e];
+            for (int e = 0; e < 8; ++e) x[e] += bias[e];
+          }
           bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)m * g.out_stride + (n - osl * g.out_slab);
           if (g.pre) {
             // (the activation of the stored value, which is what its gradient is taken at)
@@ -353,23 +431,32 @@ __global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
   *(uint4*)o = pack8(x);
 }
 
+template <int MB, int NB, bool Q_T, bool P_T, int STAGES, bool UNIFORM>
+int launch_as(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
+  static int granted[64];
+  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES, UNIFORM>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES, UNIFORM>), dim3(blocks), dim3(GEMM_THREADS), smem, st, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+
 template <int MB, int NB, bool Q_T, bool P_T, int STAGES = 3>
 int launch(const GemmParams& p, hipStream_t st) {
   constexpr int TM = 64 * MB, TN = 64 * NB;
   constexpr int ring = STAGES * (TM + TN) * GEMM_BK * 2, out = 4 * 32 * (32 * NB * 4 + 16);
   constexpr int smem = ring > out ? ring : out;
-  static int granted[64];
-  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES>, smem, granted)) return rc;
   GemmParams g = p;
   g.row_tiles = (g.rows + TM - 1) / TM;
   g.col_tiles = (g.cols + TN - 1) / TN;
   const int64_t tiles = (int64_t)g.row_tiles * g.col_tiles;
   const int64_t blocks = g.splits > 1 ? 8LL * ((g.splits + 7) / 8) * tiles : 8LL * ((g.row_tiles + 7) / 8) * g.col_tiles;
   if (blocks > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "grid too large");
-  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES>), dim3((unsigned)blocks), dim3(GEMM_THREADS), smem, st, g);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
-  return HSTU_BLOCK_OK;
+  // one slab per tile (per stage, along the contraction); lane offsets within 32 bits
+  const bool one_slab = P_T ? (g.slab >= g.cols || g.slab % TN == 0) : g.slab % GEMM_BK == 0;
+  const int64_t widest = (int64_t)(TM > TN ? TM : TN) * (g.q_stride > g.p_stride ? g.q_stride : g.p_stride) * 2;
+  if (one_slab && widest < (1LL << 31)) return launch_as<MB, NB, Q_T, P_T, STAGES, true>(g, (unsigned)blocks, smem, st);
+  return launch_as<MB, NB, Q_T, P_T, STAGES, false>(g, (unsigned)blocks, smem, st);
 }
 
 template <bool Q_T, bool P_T>
@@ -382,10 +469,12 @@ int launch_sized(const GemmParams& p, hipStream_t st, int tile) {
 int64_t tiles_of(int64_t rows, int64_t cols, int tm, int tn) { return ((rows + tm - 1) / tm) * ((cols + tn - 1) / tn); }
 
 // The tile of a product: 256 x 128 has the most products per byte of LDS traffic, 128 x 128 leaves room for a third workgroup
-// per CU, whose loads cover the others' starts and stores.  Long contractions take the first (78 k x 2048 x 2048: 692 us
-// against 775), short ones the second (78 k x 512 x 2048: 255 us against 262); products of few tiles go down to 64 x 64.
+// per CU, whose loads cover the others' starts and stores.  Long contractions take the first (74 k x 2048 to 512 columns: 196 us
+// against 214), and so do short ones with tiles enough for six rounds over the chip (74 k x 512 to 2048 columns: 270 us against
+// 281; to 512 columns 76 against 68); products of few tiles go down to 64 x 64.  (256 x 256 with one wave per SIMD, 128 x 128
+// per wave: 310 and 220 us.)
 int pick_tile(int64_t rows, int64_t cols, int64_t depth) {
-  if (depth >= 1024 && tiles_of(rows, cols, 256, 128) >= 512) return 2;
+  if (tiles_of(rows, cols, 256, 128) >= (depth >= 1024 ? 512 : 3072)) return 2;
   if (tiles_of(rows, cols, 128, 128) >= 384) return 1;
   return 0;
 }

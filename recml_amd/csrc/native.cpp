@@ -570,11 +570,11 @@ void gemm(int op, int64_t M, Rows x, std::initializer_list<const Tensor*> ws, in
   block_check(hstu_gemm(&g, stream_of(like)), "hstu_gemm");
 }
 
-// d [M, N] w^T for a weight [K, N] in slabs: the package's kernel for the small ones, torch's product for the large ones
-// (78 k x 512 x 2048: 235 us here, 197 us there; 10 k x 256 x 1024: the same; below, its launch alone takes longer).
+// d [M, N] w^T for a weight [K, N] in slabs: the package's kernel for small products and short contractions, torch's product for
+// the others (74 k x 512 to 512: 60 us here, 93 us there; 74 k x 2048 to 512: 196 us here, 158 us there).
 Tensor input_gradient(const Tensor& d, std::initializer_list<const Tensor*> ws, int64_t K, int64_t N) {
   const int64_t M = d.size(0), slab = N / (int64_t)ws.size();
-  if (2.0 * (double)M * (double)N * (double)K < 6e9 && (ws.size() == 1 || slab >= 32)) {
+  if ((N <= 1024 || 2.0 * (double)M * (double)N * (double)K < 6e9) && (ws.size() == 1 || slab >= 32)) {
     const Tensor out = fresh(d, {M, K});
     gemm(HSTU_GEMM_NT, M, {d.const_data_ptr(), N}, ws, K, N, out);
     return out;
