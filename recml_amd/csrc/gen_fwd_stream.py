@@ -56,7 +56,7 @@ class Regs:
   """The stream's own registers from v[base] up.  With `alias` the K fragments share registers with
   the V fragments of keys 0..15 and with the position window (96 registers), else 128."""
 
-  def __init__(self, base: int, alias: bool, lag: bool = False, ts: bool = False):
+  def __init__(self, base: int, alias: bool, lag: bool = False, ts: bool = False, f8: bool = False):
     assert base % 4 == 0
     self.base = base
     b = base
@@ -77,9 +77,10 @@ class Regs:
     self.e = b; b += 8            # the SiLU's temporaries
     self.p0 = b; b += 4           # P, keys 0..15 (B operand)
     self.p1 = b; b += 4           # P, keys 16..31
-    self.kf = b; b += 32          # K fragments 0..7
+    self.kf = b; b += 16 if f8 else 32   # K fragments 0..7 (8-bit elements: two registers each)
     self.vfb = b; b += 16         # V fragments of keys 16..31
     if alias:
+      assert not f8
       self.vfa = self.kf          # V fragments of keys 0..15: the registers of K fragments 0..3
       self.posw = self.kf + 16    # position window: those of K fragments 4..7
     else:
@@ -136,6 +137,10 @@ class Stream:
     return "".join(f'      "{l}\\n\\t"\n' for l in self.lines)
 
 
+def mfma_f8(dst: str, a: str, b: str, c: str) -> str:
+  return f"v_mfma_f32_32x32x16_fp8_fp8 {dst}, {a}, {b}, {c}"
+
+
 def mfma(dst: str, a: str, b: str, c: str) -> str:
   return f"v_mfma_f32_32x32x16_bf16 {dst}, {a}, {b}, {c}"
 
@@ -157,14 +162,20 @@ LDS_SLOTS_DEEP = {-1: ["k0", "k1"], 1: ["va0"], 2: ["va1"], 5: ["vb0"], 6: ["vb1
 
 class Gen:
   def __init__(self, pos: bool, dma: bool, base: int = 160, alias: bool = True, lds_slots=None, valu: str = "phases", ablate=(),
-               lag: bool = False, pos_slot: int = 11, ts: bool = False):
+               lag: bool = False, pos_slot: int = 11, ts: bool = False, f8: bool = False):
+    # f8: q and k in 8 bits.  Half the K tile and fragment registers, one direct load per wave and K tile; a 16-byte read
+    # brings the fragments of two products.
+    self.f8 = f8
+    self.k_bytes = K_BYTES // 2 if f8 else K_BYTES
+    self.stage = STAGE - K_BYTES + self.k_bytes
+    self.k_loads = 1 if f8 else 2
     self.pos = pos
     self.ts = ts
     self.dma = dma
     self.lag = lag
     self.pos_slot = pos_slot
     self.parity = 0               # lag schedule: which P buffer the iteration at hand writes
-    self.R = Regs(140 if lag else base, alias, lag, ts)
+    self.R = Regs(140 if lag else base, alias, lag, ts, f8)
     self.S = Stream(ablate)
     self.alias = alias
     self.lds_slots = lds_slots or (LDS_SLOTS_ALIAS if alias else LDS_SLOTS_DEEP)
@@ -217,15 +228,25 @@ class Gen:
       if "nok" in self.ablate:
         S.tag_index[f"k{ks}"] = S.lds_done
         continue
+      if self.f8:
+        if ks % 2 == 0: S.lds(f"ds_read_b128 {R.r(R.kf + 2 * ks, 4)}, {self.ka(ks // 2)} offset:{kst * self.stage}", f"k{ks}")
+        else: S.tag_index[f"k{ks}"] = S.tag_index[f"k{ks - 1}"]
+        continue
       dst = R.dummy if "ldsdummy" in self.ablate else R.kf + 4 * ks
       S.lds(f"ds_read_b128 {R.r(dst, 4)}, {self.ka(ks)} offset:{kst * STAGE}", f"k{ks}")
+
+  def logit_product(self, ks: int) -> str:
+    R = self.R
+    c = "0" if ks == 0 else R.r(R.sacc, 16)
+    if self.f8: return mfma_f8(R.r(R.sacc, 16), R.r(R.kf + 2 * ks, 2), self.q(ks), c)
+    return mfma(R.r(R.sacc, 16), R.r(R.kf + 4 * ks, 4), self.q(ks), c)
 
   def v_reads(self, vst: int, cc: int, dvbs):
     R, S = self.R, self.S
     dst0 = R.vfa if cc == 0 else R.vfb
     for d in dvbs:
       for x in range(2):
-        off = vst * STAGE + (16 * cc + 8 * x) * D * 2
+        off = vst * self.stage + (16 * cc + 8 * x) * D * 2
         S.lds(f"ds_read_b64_tr_b16 {R.r(dst0 + 4 * d + 2 * x, 2)}, {self.va(d)} offset:{off}", f"v{cc}{d}{x}")
 
   def pos_reads(self, kst: int):
@@ -297,7 +318,7 @@ class Gen:
         ks = slot - 4
         if not last:
           S.need(f"k{ks}")
-          S.emit(mfma(R.r(R.sacc, 16), R.r(R.kf + 4 * ks, 4), self.q(ks), "0" if ks == 0 else R.r(R.sacc, 16)))
+          S.emit(self.logit_product(ks))
       else:
         d = slot - 12
         S.need(f"v0{d}0", f"v0{d}1")
@@ -443,7 +464,7 @@ class Gen:
     """Direct loads of one step's K tile (and position window) into ring stage st; the scalar pointers
     s[90:91] (K rows) and s[94:95] (window) then move on by one step."""
     L = []
-    for r in range(2): self._load(L, "%[kdst]", st * STAGE + r * 1024, f"%[koff{r}]", "s[90:91]")
+    for r in range(self.k_loads): self._load(L, "%[kdst]", st * self.stage + r * 1024, f"%[koff{r}]", "s[90:91]")
     L.append("s_add_u32 s90, s90, %[kstep]")
     L.append("s_addc_u32 s91, s91, 0")
     if self.ts:
@@ -468,7 +489,7 @@ class Gen:
     for ahead in (3, 4): L += self.dma_k_side((vst + ahead) % NSTAGE)
     for ahead in (2, 3):
       st = (vst + ahead) % NSTAGE
-      for r in range(2): self._load(L, "%[vdst]", st * STAGE + r * 1024, f"%[voff{r}]", "s[92:93]")
+      for r in range(2): self._load(L, "%[vdst]", st * self.stage + r * 1024, f"%[voff{r}]", "s[92:93]")
       L.append("s_add_u32 s92, s92, %[vstep]")
       L.append("s_addc_u32 s93, s93, 0")
     return L
@@ -488,15 +509,17 @@ class Gen:
     self.k_reads(kst, 0, 8)
     for ks in range(8):
       S.need(f"k{ks}")
-      S.emit(mfma(R.r(R.sacc, 16), R.r(R.kf + 4 * ks, 4), self.q(ks), "0" if ks == 0 else R.r(R.sacc, 16)))
+      S.emit(self.logit_product(ks))
     if self.pos: self.pos_reads(kst)
     if self.ts:
       self.desc_read(kst)
       self.desc_unpack()
       self.value_read()
-    # the scale + bias instructions read the accumulator: 11 wait states behind the last matrix instruction
+    # the scale + bias instructions read the accumulator: 11 wait states behind the last matrix instruction (8-bit operands: as
+    # many again, whatever that instruction's number of passes)
     S.emit("s_nop 7")
     S.emit("s_nop 3")
+    if self.f8: S.emit("s_nop 7")
 
   def tail(self):
     """The product still pending after the last iteration, then wait states until the accumulators may be read."""
@@ -558,7 +581,7 @@ def full_variant(pos: bool, base: int, **kw) -> Gen:
       it(vst, first_of_pair=True, dma_lines=lines)
       if first and pair == 0:
         # this wave's share of step 2's K side has landed once at most the pair's own loads are in flight
-        own = (3 if (pos or g.ts) else 2) * 2 + 2 * 2
+        own = (g.k_loads + (1 if (pos or g.ts) else 0)) * 2 + 2 * 2
         S.emit(f"s_waitcnt vmcnt({own})")
         S.emit("s_barrier")
       else:
@@ -579,12 +602,12 @@ def full_variant(pos: bool, base: int, **kw) -> Gen:
   return g
 
 
-def loads_only_variant(pos: bool, ts: bool) -> Gen:
+def loads_only_variant(pos: bool, ts: bool, f8: bool = False) -> Gen:
   """What a wave without query rows (all 32 past the sequence's end) runs in place of full_variant: its share of the
   direct loads, the waits for them and every barrier of the workgroup, in the same order and number, and nothing else.
   A pair's loads go to ring stages whose last readers finished before the barrier that starts the pair, so they may
   all go out right behind it."""
-  g = Gen(pos, dma=True, base=152 if ts else 160, ts=ts, **PRODUCT)     # (the register window goes unused)
+  g = Gen(pos, dma=True, base=144 if f8 else 152 if ts else 160, ts=ts, f8=f8, **(PRODUCT_F8 if f8 else PRODUCT))     # (the register window goes unused)
   g.loads_only = True
   S = g.S = Stream()
   S.emit("s_mov_b64 s[90:91], %[kp]")
@@ -598,7 +621,7 @@ def loads_only_variant(pos: bool, ts: bool) -> Gen:
       if first and pair == 0: lines = g.dma_k_side(2) + lines
       for l in lines: S.emit(l)
       if first and pair == 0:
-        own = (3 if (pos or ts) else 2) * 2 + 2 * 2
+        own = (g.k_loads + (1 if (pos or ts) else 0)) * 2 + 2 * 2
         S.emit(f"s_waitcnt vmcnt({own})")
         S.emit("s_barrier")
       S.emit("s_waitcnt vmcnt(0)")
@@ -619,7 +642,7 @@ def loads_only_variant(pos: bool, ts: bool) -> Gen:
 def asm_statement(g: Gen) -> str:
   if getattr(g, "loads_only", False):
     ins = ['[kdst] "s"(hs_kdst)', '[vdst] "s"(hs_vdst)', '[kstep] "s"(hs_kstep)', '[vstep] "s"(hs_vstep)']
-    ins += [f'[koff{r}] "v"(hs_koff[{r}])' for r in range(2)] + [f'[voff{r}] "v"(hs_voff[{r}])' for r in range(2)]
+    ins += [f'[koff{r}] "v"(hs_koff[{r}])' for r in range(g.k_loads)] + [f'[voff{r}] "v"(hs_voff[{r}])' for r in range(2)]
     ins += ['[kp] "s"(hs_kp)', '[vp] "s"(hs_vp)']
     outs = ['[n] "+s"(hs_n)']
     if g.ts:
@@ -632,7 +655,7 @@ def asm_statement(g: Gen) -> str:
             f"      : {', '.join(outs)}\n      : {', '.join(ins)}\n      : {', '.join(clob)});\n")
   ins = ['[alpha] "s"(hs_alpha)']
   ins += [f'[q{ks}] "v"(hs_q[{ks}])' for ks in range(8)]
-  ins += [f'[ka{ks}] "v"(hs_ka[{ks}])' for ks in range(8)]
+  ins += [f'[ka{ks}] "v"(hs_ka[{ks}])' for ks in range(4 if g.f8 else 8)]
   ins += [f'[va{d}] "v"(hs_va[{d}])' for d in range(4)]
   if g.pos: ins.append('[pa] "v"(hs_pa)')
   if g.ts:
@@ -644,7 +667,7 @@ def asm_statement(g: Gen) -> str:
   clob = ['"memory"', '"scc"'] + clob_extra + [f'"{c}"' for c in g.R.clobbers()]
   if g.dma:
     ins += ['[kdst] "s"(hs_kdst)', '[vdst] "s"(hs_vdst)', '[kstep] "s"(hs_kstep)', '[vstep] "s"(hs_vstep)']
-    ins += [f'[koff{r}] "v"(hs_koff[{r}])' for r in range(2)] + [f'[voff{r}] "v"(hs_voff[{r}])' for r in range(2)]
+    ins += [f'[koff{r}] "v"(hs_koff[{r}])' for r in range(g.k_loads)] + [f'[voff{r}] "v"(hs_voff[{r}])' for r in range(2)]
     ins += ['[kp] "s"(hs_kp)', '[vp] "s"(hs_vp)']
     clob += ['"m0"'] + [f'"s{i}"' for i in range(90, 96)]
     if g.ts:
@@ -662,6 +685,8 @@ def statement(g: Gen, name: str) -> str:
 
 # What the product build takes (measured against the alternatives by --experiments).
 PRODUCT = dict(alias=True, valu="phases")
+# (8-bit q and k leave the registers for the V fragments and the window to have their own)
+PRODUCT_F8 = dict(alias=False, valu="phases")
 
 
 def experiments(base_alias: int, base_deep: int):
@@ -708,7 +733,9 @@ def main():
            "#define HSTU_STREAM_COMPUTE_ONLY 1\n#define HSTU_STREAM_COMPUTE_ONLY_POS 2\n#define HSTU_STREAM_FULL 3\n#define HSTU_STREAM_FULL_POS 4\n"
            "#define HSTU_STREAM_FULL_TS 5\n#define HSTU_STREAM_FULL_POS_TS 6\n"
            "#define HSTU_STREAM_LOADS_ONLY 7\n#define HSTU_STREAM_LOADS_ONLY_POS 8\n#define HSTU_STREAM_LOADS_ONLY_TS 9\n"
-           "#define HSTU_STREAM_LOADS_ONLY_POS_TS 10\n"]
+           "#define HSTU_STREAM_LOADS_ONLY_POS_TS 10\n"
+           "#define HSTU_STREAM_FULL_F8 11\n#define HSTU_STREAM_FULL_POS_F8 12\n"
+           "#define HSTU_STREAM_LOADS_ONLY_F8 13\n#define HSTU_STREAM_LOADS_ONLY_POS_F8 14\n"]
   parts.append(statement(compute_only_variant(False, a.base, **PRODUCT), "HSTU_STREAM_COMPUTE_ONLY"))
   parts.append(statement(compute_only_variant(True, a.base, **PRODUCT), "HSTU_STREAM_COMPUTE_ONLY_POS"))
   parts.append(statement(full_variant(False, a.base, **PRODUCT), "HSTU_STREAM_FULL"))
@@ -719,6 +746,9 @@ def main():
   parts.append(statement(loads_only_variant(True, False), "HSTU_STREAM_LOADS_ONLY_POS"))
   parts.append(statement(loads_only_variant(False, True), "HSTU_STREAM_LOADS_ONLY_TS"))
   parts.append(statement(loads_only_variant(True, True), "HSTU_STREAM_LOADS_ONLY_POS_TS"))    # (another pitch of the bias stages)
+  for pos in (False, True):
+    parts.append(statement(full_variant(pos, a.base - 16, f8=True, **PRODUCT_F8), "HSTU_STREAM_FULL_POS_F8" if pos else "HSTU_STREAM_FULL_F8"))
+    parts.append(statement(loads_only_variant(pos, False, f8=True), "HSTU_STREAM_LOADS_ONLY_POS_F8" if pos else "HSTU_STREAM_LOADS_ONLY_F8"))
   with open(a.out, "w") as f:
     f.write("".join(parts))
   print("wrote", a.out)

@@ -3062,7 +3062,8 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   // (Not in the resident-workgroup instances with timestamps: what those keep across their loop over items and
   // what the stream clobbers do not fit the register file together, and the compiler's spills cost the block code
   // more than the stream gains.  Calls with timestamp descriptors take one workgroup per item instead.)
-  constexpr bool STREAM = D == 128 && !F8 && !SEG && DENSE == 0 && PAIRS && !(TS && PERSIST);
+  // (8-bit q and k: the same stream with its logits' products and K tiles in 8 bits, without timestamps.)
+  constexpr bool STREAM = D == 128 && !(F8 && TS) && !SEG && DENSE == 0 && PAIRS && !(TS && PERSIST);
   auto stream_quads = [&]() -> int {
     if constexpr (!STREAM) return 0;
     const Params pf = fresh();
@@ -3095,12 +3096,16 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       const int gk = SM::swz_k(m), gi = lane & 15, vrow = 4 * hh + (gi >> 2), gq = SM::swz_v(vrow) >> 2;
       const int vc2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
       typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-      uintx4 hs_q[8];
+      typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+      typename std::conditional<F8, uintx2, uintx4>::type hs_q[8];
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) hs_q[ks] = uintx4{qf[ks].x, qf[ks].y, qf[ks].z, qf[ks].w};
-      uint32_t hs_ka[8], hs_va[4];
+      for (int ks = 0; ks < 8; ++ks) {
+        if constexpr (F8) hs_q[ks] = ks & 1 ? uintx2{qf[ks / 2].z, qf[ks / 2].w} : uintx2{qf[ks / 2].x, qf[ks / 2].y};
+        else hs_q[ks] = uintx4{qf[ks].x, qf[ks].y, qf[ks].z, qf[ks].w};
+      }
+      uint32_t hs_ka[QCH], hs_va[4];
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) hs_ka[ks] = smem_lds + (uint32_t)(m * 256 + (((2 * ks + hh) ^ gk) * 16));
+      for (int ks = 0; ks < QCH; ++ks) hs_ka[ks] = smem_lds + (uint32_t)(m * (D * KB) + (((2 * ks + hh) ^ gk) * 16));
 #pragma unroll
       for (int d = 0; d < 4; ++d) hs_va[d] = smem_lds + (uint32_t)(SM::K_BYTES + vrow * 256 + 8 * (gi & 1) + vc2 * 16 + ((d ^ gq) & 3) * 64);
       const int xb = 4 * hh + (BM - 1) - 32 * w - m, sft = xb & 3;
@@ -3109,10 +3114,11 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
         const int c = 64 * (2 * w + r) + lane, row = c / 16, pc = c - row * 16;
-        hs_koff[r] = (uint32_t)row * kst_bytes + (uint32_t)((pc ^ SM::swz_k(row)) * 16);
+        const int ck = 64 * (LDK * w + r % LDK) + lane, krow = ck / KCPR, kpc = ck - krow * KCPR;
+        hs_koff[r] = (uint32_t)krow * kst_bytes + (uint32_t)((kpc ^ SM::swz_k(krow)) * 16);
         hs_voff[r] = (uint32_t)row * vst_bytes + (uint32_t)((pc ^ SM::swz_v(row)) * 16);
       }
-      const uint32_t hs_kdst = __builtin_amdgcn_readfirstlane(smem_lds + (uint32_t)(2 * w * 1024));
+      const uint32_t hs_kdst = __builtin_amdgcn_readfirstlane(smem_lds + (uint32_t)(LDK * w * 1024));
       const uint32_t hs_vdst = __builtin_amdgcn_readfirstlane(smem_lds + (uint32_t)(SM::K_BYTES + 2 * w * 1024));
       const uint32_t hs_kstep = (uint32_t)BN * kst_bytes, hs_vstep = (uint32_t)BN * vst_bytes;
       const char* hs_kp = cx.kg + (size_t)(t_lo + 2) * hs_kstep;
@@ -3142,7 +3148,15 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       floatx16 (&hs_o)[DVB] = o;
       if (wave_last < 0) {
         // a wave whose 32 rows lie past the sequence's end: its share of the loads and every barrier, nothing else
-        if constexpr (POS && TS) {
+        if constexpr (F8 && POS) {
+#define HSTU_STREAM_VARIANT HSTU_STREAM_LOADS_ONLY_POS_F8
+#include "hstu_fwd_stream_d128.inc"
+#undef HSTU_STREAM_VARIANT
+        } else if constexpr (F8) {
+#define HSTU_STREAM_VARIANT HSTU_STREAM_LOADS_ONLY_F8
+#include "hstu_fwd_stream_d128.inc"
+#undef HSTU_STREAM_VARIANT
+        } else if constexpr (POS && TS) {
 #define HSTU_STREAM_VARIANT HSTU_STREAM_LOADS_ONLY_POS_TS
 #include "hstu_fwd_stream_d128.inc"
 #undef HSTU_STREAM_VARIANT
@@ -3159,6 +3173,14 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
 #include "hstu_fwd_stream_d128.inc"
 #undef HSTU_STREAM_VARIANT
         }
+      } else if constexpr (F8 && POS) {
+#define HSTU_STREAM_VARIANT HSTU_STREAM_FULL_POS_F8
+#include "hstu_fwd_stream_d128.inc"
+#undef HSTU_STREAM_VARIANT
+      } else if constexpr (F8) {
+#define HSTU_STREAM_VARIANT HSTU_STREAM_FULL_F8
+#include "hstu_fwd_stream_d128.inc"
+#undef HSTU_STREAM_VARIANT
       } else if constexpr (POS && TS) {
 #define HSTU_STREAM_VARIANT HSTU_STREAM_FULL_POS_TS
 #include "hstu_fwd_stream_d128.inc"
