@@ -2345,8 +2345,14 @@ constexpr bool fwd_takes_ts_desc(int d, bool ts, bool f8, bool seg, int dense) {
 #include "hstu_fwd_stream_d128.inc"   // (the variants' names; the statements are expanded inside the kernel)
 #include "hstu_bwd_stream_d128.inc"
 
-template <int D, bool POS, bool TS, bool F8, bool SEG = false, int DENSE = 0, bool PERSIST = false>
+// WHOLE: a small call with a position table alone takes the table as the caller gave it.  The part of it that a tile's rows and
+// at most WHOLE_KEYS keys meet is scaled and laid out in LDS once, in the four shifted copies that the steps read; nothing is left
+// for hstu_prepare then, whose launch cost such a call as much as a third of the kernel.
+constexpr int WHOLE_KEYS = 512;
+constexpr int WHOLE_COPY = (WHOLE_KEYS + BM + 4) * 4;      // bytes of one copy
+template <int D, bool POS, bool TS, bool F8, bool SEG = false, int DENSE = 0, bool PERSIST = false, bool WHOLE = false>
 __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Params p) {
+  static_assert(!WHOLE || (POS && !TS && !SEG && DENSE == 0 && !PERSIST), "the whole window is for the position table alone");
   constexpr int KB = F8 ? 1 : 2;       // bytes per q / k element
   using SM = MfmaSmem<D, KB>;
   constexpr int CPR = SM::CPR;
@@ -2362,7 +2368,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   constexpr int NSTAGE = fwd_stages(D, DENSE);   // the ring depth of this kernel (shadows the backward kernels' constant)
   static_assert(BM * BN * 4 / 1024 == 4 * NWAVES && BM * BN / 1024 == NWAVES, "dense tiles: 4 + 1 pieces per wave");
   // direct loads per wave per step
-  constexpr int NDMA = LDK + LD + ((POS || TS) ? 1 : 0) + (SEG ? 1 : 0);
+  constexpr int NDMA = LDK + LD + (((POS && !WHOLE) || TS) ? 1 : 0) + (SEG ? 1 : 0);
   constexpr int NDENSE = ((DENSE & 1) ? 4 : 0) + ((DENSE & 2) ? 1 : 0);     // the dense operands' loads, counted apart
   static_assert((NSTAGE - 1) * NDMA + NDENSE <= 63, "vmcnt range");
   static_assert(DENSE == 0 || (!POS && !TS && !SEG && !F8), "dense operands come without table biases, segment ids and fp8");
@@ -2381,13 +2387,13 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   // its window copy and, in the four lanes behind it, its own rows' descriptors.
   constexpr bool TSD = fwd_takes_ts_desc(D, TS, F8, SEG, DENSE);
   constexpr int DESC_WAVE = 64;                                      // 32 descriptors of 2 bytes
-  constexpr int CS = TSD ? (POS ? SM::POS_COPY : 0) + DESC_WAVE : SM::POS_COPY;   // from one wave's copy to the next
-  constexpr int BIAS_STAGE = SM::bias_stage(POS, TS, SEG) + (TSD ? NWAVES * DESC_WAVE : 0);
+  constexpr int CS = WHOLE ? WHOLE_COPY : TSD ? (POS ? SM::POS_COPY : 0) + DESC_WAVE : SM::POS_COPY;   // from one wave's copy to the next
+  constexpr int BIAS_STAGE = WHOLE ? 0 : SM::bias_stage(POS, TS, SEG) + (TSD ? NWAVES * DESC_WAVE : 0);
   auto Wc = [&](int st) { return (float*)(smem + BIAS_OFF + st * BIAS_STAGE); };
   auto Tk = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (TSD ? NWAVES * CS : (POS ? SM::POS_BYTES : 0))); };
   auto Sg = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + SM::bias_stage(POS, TS)); };
   const unsigned char* TsKey = smem + BIAS_OFF + NSTAGE * BIAS_STAGE;   // the keyed bucket table of this head
-  constexpr int DENSE_OFF = BIAS_OFF + NSTAGE * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0);
+  constexpr int DENSE_OFF = BIAS_OFF + NSTAGE * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0) + (WHOLE ? 4 * WHOLE_COPY : 0);
   constexpr int DENSE_STAGE = SM::dense_stage(DENSE);
   constexpr int XCH_OFF = DENSE_OFF + DENSE_STAGE;   // 16 bytes for values one lane hands to the workgroup
   auto Db = [&]() { return smem + DENSE_OFF; };
@@ -2537,7 +2543,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       lds_dma16(c_.vg, voff, Vs(st) + j * 512);
     }
     }
-    if ((POS || TS) && (part & 1) != 0) {
+    if (((POS && !WHOLE) || TS) && (part & 1) != 0) {
       // one more load per wave brings the bias operands (bias_lane)
       bool on;
       const uint32_t off = bias_lane(c_, t, on, lane);
@@ -2761,7 +2767,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
     if (POS) {
       const int xb = 4 * hh + (BM - 1) - 32 * w - m;
       const int sft = xb & 3;
-      const float* wrow = (const float*)((const unsigned char*)Wc(st) + sft * CS) + (xb - sft);
+      const float* wrow = (const float*)((const unsigned char*)Wc(st) + sft * CS) + (xb - sft) + (WHOLE ? kbs : 0);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         float4 bv = *(const float4*)(wrow + 8 * g);
@@ -3063,7 +3069,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   // what the stream clobbers do not fit the register file together, and the compiler's spills cost the block code
   // more than the stream gains.  Calls with timestamp descriptors take one workgroup per item instead.)
   // (8-bit q and k: the same stream with its logits' products and K tiles in 8 bits, without timestamps.)
-  constexpr bool STREAM = D == 128 && !(F8 && TS) && !SEG && DENSE == 0 && PAIRS && !(TS && PERSIST);
+  constexpr bool STREAM = D == 128 && !(F8 && TS) && !SEG && DENSE == 0 && PAIRS && !(TS && PERSIST) && !WHOLE;
   auto stream_quads = [&]() -> int {
     if constexpr (!STREAM) return 0;
     const Params pf = fresh();
@@ -3216,10 +3222,31 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
     // prologue follows behind the Q fragments, whose wait covers every load issued before it: behind
     // all of the prologue it held up the first block until everything had landed.
     if (TS) load_ts_table(h);
+    constexpr int WHOLE_PER = WHOLE ? (WHOLE_KEYS + BM + MFMA_THREADS - 1) / MFMA_THREADS : 1;
+    float whole[WHOLE_PER];
+    if constexpr (WHOLE) {
+      // window[x] = pos[(L - 1) - (q0 + 127) + x] for key x + row - (q0 + 127)
+      const float* tab = p.pos_tab + (int64_t)(p.pos_heads > 1 ? h : 0) * (2 * p.L - 1);
+#pragma unroll
+      for (int i = 0; i < WHOLE_PER; ++i) {
+        int at = (p.L - 1) - (q0 + BM - 1) + tid + MFMA_THREADS * i;
+        at = at < 0 ? 0 : (at > 2 * p.L - 2 ? 2 * p.L - 2 : at);       // (pairs outside the table are masked)
+        whole[i] = tab[at];
+      }
+    }
     if (t_lo < nt) dma_step(cx, t_lo, std::integral_constant<int, 0>{});
     if (DENSE != 0 && t_lo < nt) dense_refill(cx, t_lo);
     load_q(first);
     settle_q();
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int i = 0; i < WHOLE_PER; ++i) {
+        const int x = tid + MFMA_THREADS * i;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (x - c >= 0 && x < WHOLE_KEYS + BM) *(float*)(smem + BIAS_OFF + c * WHOLE_COPY + 4 * (x - c)) = whole[i] * LOG2E;
+      }
+    }
     if (t_lo + 1 < nt) dma_step(cx, t_lo + 1, std::integral_constant<int, 1>{});
     if constexpr (NSTAGE > 3 && !PAIRS) {
       if (t_lo + 2 < nt) dma_step(cx, t_lo + 2, std::integral_constant<int, 2>{});
@@ -5315,18 +5342,18 @@ int launch_bwd(const Params& p, hipStream_t st) {
   return HSTU_OK;
 }
 
-template <int D, bool POS, bool TS, bool F8, bool SEG = false, int DENSE = 0, bool PERSIST = false>
+template <int D, bool POS, bool TS, bool F8, bool SEG = false, int DENSE = 0, bool PERSIST = false, bool WHOLE = false>
 int launch_mfma_inst(const Params& p, hipStream_t st) {
-  const int smem = MfmaSmem<D, F8 ? 1 : 2>::total(POS, TS, SEG, DENSE, fwd_stages(D, DENSE)) + FWD_XCH_BYTES +
+  const int smem = MfmaSmem<D, F8 ? 1 : 2>::total(POS && !WHOLE, TS, SEG, DENSE, fwd_stages(D, DENSE)) + FWD_XCH_BYTES + (WHOLE ? 4 * WHOLE_COPY : 0) +
                    (fwd_takes_ts_desc(D, TS, F8, SEG, DENSE) ? fwd_stages(D, DENSE) * NWAVES * 64 : 0);
   static int granted[64];
-  if (int rc = allow_lds((const void*)hstu_fwd_mfma_bf16<D, POS, TS, F8, SEG, DENSE, PERSIST>, smem, granted)) return rc;
+  if (int rc = allow_lds((const void*)hstu_fwd_mfma_bf16<D, POS, TS, F8, SEG, DENSE, PERSIST, WHOLE>, smem, granted)) return rc;
   hipError_t e;
   long long blocks = mfma_grid(p);
   // resident workgroups: as many as run at once, fewer when the list cannot be longer than that
   if (PERSIST && blocks > 8LL * p.n_slots) blocks = 8LL * p.n_slots;
   if (blocks > 0x7fffffffLL) return fail(HSTU_ERR_SHAPE, "grid too large");
-  hipLaunchKernelGGL((hstu_fwd_mfma_bf16<D, POS, TS, F8, SEG, DENSE, PERSIST>), dim3((unsigned)blocks), dim3(MFMA_THREADS), smem, st, p);
+  hipLaunchKernelGGL((hstu_fwd_mfma_bf16<D, POS, TS, F8, SEG, DENSE, PERSIST, WHOLE>), dim3((unsigned)blocks), dim3(MFMA_THREADS), smem, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "mfma kernel launch: %s", hipGetErrorString(e));
   return HSTU_OK;
@@ -5354,6 +5381,7 @@ int launch_mfma_d(const Params& p, hipStream_t st) {
       return launch_mfma_inst<D, false, false, false, false, 0, true>(p, st);
     }
   }
+  if (p.whole_window) return launch_mfma_inst<D, true, false, F8, false, 0, false, true>(p, st);
   if (pos && ts) return launch_mfma_inst<D, true, true, F8>(p, st);
   if (pos) return launch_mfma_inst<D, true, false, F8>(p, st);
   if (ts) return launch_mfma_inst<D, false, true, F8>(p, st);
@@ -5704,6 +5732,11 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // the split capacity adapts to the workspace the caller brought (never below what the call needs)
       const WorkspacePlan ws = plan_workspace(args, true, args->workspace ? args->workspace_bytes : 0);
       Params q = p;
+      // A call without a work list, with a position table and nothing else to prepare, whose tiles' windows fit LDS: the
+      // kernel takes the table itself, and the preparation is not launched.
+      q.whole_window = ws.sched_bytes == 0 && q.pos_tab && !q.ts_tab && !q.mask && !q.dense_bias && q.mask_mode != HSTU_MASK_SEGMENT &&
+                       q.Lkv <= WHOLE_KEYS;
+      if (q.whole_window && !(args->flags & HSTU_FWD_PREPARE_ONLY)) return f8 ? launch_mfma<true>(q, st) : launch_mfma<false>(q, st);
       if (int rc2 = setup_workspace(args, ws, q, st)) return rc2;
       if (args->flags & HSTU_FWD_PREPARE_ONLY) return HSTU_OK;
       // Resident workgroups over the work list, where that loop is built (d = 128 in bf16, lengths or no mask)
