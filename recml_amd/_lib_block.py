@@ -157,6 +157,10 @@ def load():
     lib.hstu_gemm_workspace_bytes.argtypes = [C.c_int32, C.c_int64, C.c_int32, C.c_int32]
     lib.hstu_embed_norm_fwd.restype = C.c_int
     lib.hstu_embed_norm_fwd.argtypes = [C.POINTER(HstuEmbedNormArgs), C.c_void_p]
+    lib.hstu_embed_grad.restype = C.c_int
+    lib.hstu_embed_grad.argtypes = [C.POINTER(HstuEmbedGradArgs), C.c_void_p]
+    lib.hstu_embed_grad_workspace_bytes.restype = C.c_size_t
+    lib.hstu_embed_grad_workspace_bytes.argtypes = [C.c_int64, C.c_int64, C.c_int32]
     ver = lib.hstu_block_abi_version()
     if ver != ABI_VERSION:
       raise RuntimeError(f"libhstu_block.so has ABI {ver}, expected {ABI_VERSION}")

@@ -1,0 +1,75 @@
+"""The block's own matrix products around their tiles, stages, slabs and splits, and the sums of a gathered table's gradient
+around their runs, against fp32 products and exact sums."""
+
+import ctypes as C
+
+import pytest
+import torch
+
+from recml_amd import _lib_block
+from recml_amd import hstu_block_ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _normal(g, *shape):
+  return torch.randn(shape, generator=g).to(torch.bfloat16).to("cuda:0")
+
+
+def _close(got, want):
+  want = want.cpu()
+  assert (got.float().cpu() - want).abs().max() <= 8e-3 * want.abs().max().clamp(min=1e-3)
+
+
+@pytest.mark.parametrize("M,N,K,slabs", [
+    (1, 8, 8, 1),              # one piece of one tile
+    (65, 72, 40, 1),           # a row past a tile of 64, a contraction that is no whole stage
+    (300, 32, 16, 4),          # slabs narrower than a stage: the weight along the contraction is one matrix then
+    (257, 160, 136, 4),        # slabs of 40: a stage that crosses from one into the next
+    (1000, 512, 128, 4),       # slabs of whole tiles
+    (6200, 1024, 136, 2),      # 128 x 128 tiles
+    (33000, 512, 1024, 4),     # 256 x 128 tiles, a long contraction, a split weight gradient whose last part is short
+])
+def test_block_products(gpu, M, N, K, slabs):
+  g = torch.Generator().manual_seed(M + N)
+  x, y, bias, res = _normal(g, M, K), _normal(g, M, N), _normal(g, N), _normal(g, M, N)
+  x = torch.cat([x, x], 1)[:, :K]                                     # rows further apart than they are long
+  ws = [_normal(g, K, N // slabs) * 0.1 for _ in range(slabs)]
+  w = torch.cat(ws, 1).float()
+  want = x.float() @ w + res.float() + bias.float()
+  out, pre = ops.block_gemm(_lib_block.GEMM_NN, x, ws, bias=bias, residual=res, activation=True, want_pre=True)
+  _close(pre, want)
+  _close(out, torch.nn.functional.silu(pre.float()))
+  _close(ops.block_gemm(_lib_block.GEMM_NN, x, ws), x.float() @ w)
+  if slabs == 1 or N // slabs >= 32:
+    _close(ops.block_gemm(_lib_block.GEMM_NT, y, ws), y.float() @ w.t())
+  grads = [torch.full_like(t, float("nan")) for t in ws]
+  ops.block_gemm(_lib_block.GEMM_TN, x, grads, y=y)
+  _close(torch.cat(grads, 1), x.float().t() @ y.float())
+
+
+@pytest.mark.parametrize("rows,keys,width", [(0, 5, 8), (1, 1, 8), (700, 1, 136), (3000, 40, 64), (3000, 5000, 72), (4097, 257, 128)])
+@pytest.mark.parametrize("scale", [1.0, 2.0])
+def test_gathered_table_gradient(gpu, rows, keys, width, scale):
+  """Small whole numbers: every partial sum is exact, whatever is rounded when."""
+  g = torch.Generator().manual_seed(rows + keys)
+  ids = torch.exp(torch.rand(rows, generator=g).double() * torch.log(torch.tensor(float(keys)))).long() - 1
+  ids = ids.clamp(0, keys - 1)
+  grad = torch.randint(0, 2, (rows, width), generator=g) * 2 - 1
+  grad[torch.rand(rows, generator=g) < 0.7] = 0
+  want = torch.zeros(keys, width, dtype=torch.long).index_add_(0, ids, grad) * int(scale)
+  assert want.abs().max() < 256
+  dev = torch.device("cuda:0")
+  d, idd = grad.to(torch.bfloat16).to(dev), ids.to(dev)
+  out = torch.full((keys, width), float("nan"), dtype=torch.bfloat16, device=dev)
+  lib = _lib_block.load()
+  ws = torch.empty(lib.hstu_embed_grad_workspace_bytes(rows, keys, width) + 256, dtype=torch.uint8, device=dev)
+  a = _lib_block.HstuEmbedGradArgs()
+  a.struct_size, a.version = C.sizeof(a), _lib_block.ABI_VERSION
+  a.rows, a.keys, a.width, a.scale = rows, keys, width, scale
+  a.g, a.g_stride, a.ids, a.out = d.data_ptr(), width, idd.data_ptr(), out.data_ptr()
+  a.workspace = (ws.data_ptr() + 255) // 256 * 256
+  a.workspace_bytes = ws.numel() - (a.workspace - ws.data_ptr())
+  assert lib.hstu_embed_grad(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+  torch.cuda.synchronize()
+  assert torch.equal(out.cpu().long(), want)
