@@ -4043,18 +4043,29 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
       if (bk_lane >= 0) {
         // A lane's bucket changes with the step only now and then (the nearer the keys, the smaller): its sum stays in a
         // register until it does, and reaches the histogram then, by an LDS atomic of the lanes concerned.
-        float s_near = ((ds[0] + ds[1]) + (ds[2] + ds[3])) + ((ds[4] + ds[5]) + (ds[6] + ds[7])) +
-                       (((ds[8] + ds[9]) + (ds[10] + ds[11])) + ((ds[12] + ds[13]) + (ds[14] + ds[15])));
-        if (far_keys) {
+        float s_near;
+        if (!far_keys) {
+          s_near = ((ds[0] + ds[1]) + (ds[2] + ds[3])) + ((ds[4] + ds[5]) + (ds[6] + ds[7])) +
+                   (((ds[8] + ds[9]) + (ds[10] + ds[11])) + ((ds[12] + ds[13]) + (ds[14] + ds[15])));
+        } else {
+          // (two sums of their own: the near one as what the far one leaves of the total would lose its digits where the far
+          // keys outweigh it, and all of them to one infinity among those)
           const int32_t* tk = Tk(st);
           float s_far = 0.f;
+          s_near = 0.f;
+          auto add = [&](int key, float v) {
+            const bool far = key <= cut;
+            s_far += far ? v : 0.f;
+            s_near += far ? 0.f : v;
+          };
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
-            s_far += (kk.x <= cut ? ds[4 * g] : 0.f) + (kk.y <= cut ? ds[4 * g + 1] : 0.f);
-            s_far += (kk.z <= cut ? ds[4 * g + 2] : 0.f) + (kk.w <= cut ? ds[4 * g + 3] : 0.f);
+            add(kk.x, ds[4 * g]);
+            add(kk.y, ds[4 * g + 1]);
+            add(kk.z, ds[4 * g + 2]);
+            add(kk.w, ds[4 * g + 3]);
           }
-          s_near -= s_far;
           if (sum_bucket == bk_lane + 1) sum_s += s_far;
           else if (s_far != 0.f) lds_atomic_add(&hist[bk_lane + 1], s_far);
         }
