@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define HSTU_BLOCK_ABI_VERSION 4
+#define HSTU_BLOCK_ABI_VERSION 5
 
 typedef enum HstuBlockStatus {
   HSTU_BLOCK_OK = 0,
@@ -174,13 +174,12 @@ typedef struct HstuEmbedNormArgs {
   const int32_t* row_map; /* or null.  Given: row r takes entry row_map[r] of ids (hstu_pack_plan) */
   int32_t L;              /* with positions null and pos_table given: the position is that entry's index modulo L */
   int32_t round_steps;    /* 1: the scaled row and the sum are each rounded to bf16 (what separate steps leave); 0: one rounding */
+  void* sums;             /* or null (with round_steps only): x_t is stored here as well, bf16 [rows, width], for the gradients: */
+                          /* hstu_norm_gate_bwd on these rows gives the gradient at x_t, whatever becomes of the tables */
+  int64_t* keys;          /* or null: the row of `table` that each row took, [rows] (the keys of hstu_embed_grad) */
 } HstuEmbedNormArgs;
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* args, void* stream);
-/* Its gradients for the gradient g->dout of its result: g->da, the gradient of the summed rows x_t (bf16 [rows, width]), and
- * g->dgamma, g->dbeta; of `g` only those, dout's and da's strides and the workspace are read, of `a` everything but out.
- * row_map applies to the gather, not to dout. */
-int hstu_embed_norm_bwd(const HstuEmbedNormArgs* a, const HstuNormGateBwdArgs* g, void* stream);
 
 /* The gradient of a gathered table, all of it: out[v, :] = the sum of scale * g[t, :] over the rows t whose key is v, added in the
  * order of the rows with every term and partial sum rounded to bf16 (the bits of torch's gather backward; rows of up to 64

@@ -9,7 +9,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("RECML_AMD_BLOCK_LIB") or os.path.join(_HERE, "lib", "libhstu_block.so")
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 EXPORTS = (
     "hstu_block_abi_version",
@@ -20,7 +20,6 @@ EXPORTS = (
     "hstu_gemm_silu_fwd",
     "hstu_gemm_silu_workspace_bytes",
     "hstu_embed_norm_fwd",
-    "hstu_embed_norm_bwd",
     "hstu_embed_grad",
     "hstu_embed_grad_workspace_bytes",
     "hstu_pack_plan",
@@ -105,6 +104,7 @@ class HstuEmbedNormArgs(C.Structure):
       ("positions", C.c_void_p), ("pos_table", C.c_void_p), ("n_positions", C.c_int64),
       ("gamma", C.c_void_p), ("beta", C.c_void_p), ("out", C.c_void_p),
       ("row_map", C.c_void_p), ("L", C.c_int32), ("round_steps", C.c_int32),
+      ("sums", C.c_void_p), ("keys", C.c_void_p),
   ]
 
 

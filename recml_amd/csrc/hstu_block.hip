@@ -154,15 +154,6 @@ struct NormGateBwdParams {
   const bf16_t* u_pre;     // u = silu(u_pre), and du is the gradient of u_pre; or null
   const bf16_t* add;       // added to da (the gradient that reaches `a` past the norm); or null
   const int32_t* row_map;  // row r of dout is row row_map[r] of the buffer; or null
-  // a = scale * table[ids[r]] + pos_table[row % L] instead of rows of `a` (the model's front end; a is null then); r = the
-  // row, or row_map's entry for it, which then does not apply to dout
-  const int64_t* ids;
-  const int64_t* positions;
-  const bf16_t* table;
-  const bf16_t* pos_table;
-  int64_t vocab, table_stride, n_positions;
-  float scale;
-  int32_t L, round_steps;
   int64_t rows, a_stride, u_stride, dout_stride, da_stride, du_stride, u_pre_stride, add_stride;
   int32_t width;
   float eps;
@@ -177,8 +168,7 @@ struct NormGateBwdParams {
 // bound).  The two column sums stay in registers over a wave's rows, are added across the workgroup's
 // four waves through LDS and leave as one partial row per workgroup; hstu_colsum adds those in a fixed
 // order, so the result does not depend on the timing of the run.
-// EMB: the rows are the front end's gathered ones.
-template <int CH, int LPR, bool EMB>
+template <int CH, int LPR>
 __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParams p) {
   __shared__ float red[4][CH * LPR * 8];
   constexpr int RPW = 64 / LPR;
@@ -190,22 +180,8 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
 #pragma unroll
     for (int i = 0; i < 8; ++i) dg[c][i] = db[c][i] = 0.f;
   for (int64_t row = ((int64_t)blockIdx.x * 4 + w) * RPW + ((threadIdx.x & 63) / LPR); row < p.rows; row += (int64_t)gridDim.x * 4 * RPW) {
-    const bf16_t *ar = nullptr, *pr = nullptr;
-    int64_t grow = row;
-    if constexpr (EMB) {
-      const int64_t at = p.row_map ? p.row_map[row] : row;
-      int64_t id = p.ids[at];
-      id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
-      ar = p.table + id * p.table_stride;
-      if (p.pos_table) {
-        int64_t ps = p.positions ? p.positions[row] : at % p.L;
-        ps = ps < 0 ? 0 : (ps >= p.n_positions ? p.n_positions - 1 : ps);
-        pr = p.pos_table + ps * (int64_t)p.width;
-      }
-    } else {
-      ar = p.a + row * p.a_stride;
-      if (p.row_map) grow = p.row_map[row];
-    }
+    const bf16_t* ar = p.a + row * p.a_stride;
+    const int64_t grow = p.row_map ? p.row_map[row] : row;
     const bf16_t* gr = p.dout + grow * p.dout_stride;
     float x[CH][8], g[CH][8];
     float sum = 0.f;
@@ -215,13 +191,6 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
       if (e < p.width) {
         unpack8(*(const uint4*)(ar + e), x[c]);
         unpack8(*(const uint4*)(gr + e), g[c]);
-        if constexpr (EMB) {
-          float pe[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          if (pr) unpack8(*(const uint4*)(pr + e), pe);
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            x[c][i] = p.round_steps ? round_bf16(round_bf16(x[c][i] * p.scale) + pe[i]) : __builtin_fmaf(x[c][i], p.scale, pe[i]);
-        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) sum += x[c][i];
       } else {
@@ -290,7 +259,7 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
         float y[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) y[i] = rstd * (g[c][i] - c1 - x[c][i] * c2);
-        if (!EMB && p.add) {
+        if (p.add) {
           float more[8];
           unpack8(*(const uint4*)(p.add + row * p.add_stride + e), more);
 #pragma unroll
@@ -375,10 +344,13 @@ struct EmbedNormParams {
   int32_t width;
   float eps, scale;
   int32_t round_steps;     // the scaled row and the sum are each rounded to bf16, as separate steps would leave them
+  bf16_t* sums;            // the rows before the norm, for the gradients; or null
+  int64_t* keys;           // the table rows taken, for the gradients; or null
 };
 
 // Rows on lanes as in hstu_norm_gate: a token's table row (and position row) is gathered into registers, normalised
-// there and written once.
+// there and written once.  In training the gathered rows and their ids are stored next to it (as many bytes again): the
+// backward then works on its own copies, so that neither the ids nor the tables have to stay as they were until it runs.
 template <int CH, int LPR>
 __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) {
   constexpr int RPW = 64 / LPR;
@@ -388,6 +360,7 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
   const int64_t at = p.row_map ? p.row_map[row] : row;
   int64_t id = p.ids[at];
   id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
+  if (p.keys && lane == 0) p.keys[row] = id;
   const bf16_t* er = p.table + id * p.table_stride;
   const bf16_t* pr = nullptr;
   if (p.pos_table) {
@@ -407,6 +380,7 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         x[c][i] = p.round_steps ? round_bf16(round_bf16(x[c][i] * p.scale) + pe[i]) : __builtin_fmaf(x[c][i], p.scale, pe[i]);
+      if (p.sums) *(uint4*)(p.sums + row * (int64_t)p.width + e) = pack8(x[c]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) sum += x[c][i];
     } else {
@@ -735,16 +709,15 @@ __global__ __launch_bounds__(64) void hstu_eg_long(const EmbedGradParams p) {
   if (on) *(uint32_t*)(p.out + (int64_t)run.x * p.out_stride + e) = pack2(s0, s1);
 }
 
-template <bool EMB>
 void launch_norm_bwd(const NormGateBwdParams& p, int nb, hipStream_t st) {
   const dim3 grid((unsigned)nb), block(256);
   const int lpr = lanes_per_row(p.width), ch = (p.width + 511) / 512;
-  if (lpr == 8) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 8, EMB>), grid, block, 0, st, p);
-  else if (lpr == 16) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 16, EMB>), grid, block, 0, st, p);
-  else if (lpr == 32) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 32, EMB>), grid, block, 0, st, p);
-  else if (ch <= 1) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 64, EMB>), grid, block, 0, st, p);
-  else if (ch <= 2) hipLaunchKernelGGL((hstu_norm_gate_bwd<2, 64, EMB>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((hstu_norm_gate_bwd<4, 64, EMB>), grid, block, 0, st, p);
+  if (lpr == 8) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 8>), grid, block, 0, st, p);
+  else if (lpr == 16) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 16>), grid, block, 0, st, p);
+  else if (lpr == 32) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 32>), grid, block, 0, st, p);
+  else if (ch <= 1) hipLaunchKernelGGL((hstu_norm_gate_bwd<1, 64>), grid, block, 0, st, p);
+  else if (ch <= 2) hipLaunchKernelGGL((hstu_norm_gate_bwd<2, 64>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((hstu_norm_gate_bwd<4, 64>), grid, block, 0, st, p);
 }
 
 struct EmbedGradPlan {
@@ -905,7 +878,7 @@ int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
     p.da = (bf16_t*)a->da; p.du = (bf16_t*)a->du; p.partial = (float*)a->workspace;
     p.rows = a->rows; p.a_stride = a->a_stride; p.u_stride = a->u_stride; p.dout_stride = a->dout_stride;
     p.da_stride = a->da_stride; p.du_stride = a->du_stride; p.width = a->width; p.eps = a->eps;
-    launch_norm_bwd<false>(p, nb, st);
+    launch_norm_bwd(p, nb, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate backward kernel launch: %s", hipGetErrorString(e));
   }
@@ -932,6 +905,7 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   if (!block_aligned16(a->table) || !block_aligned16(a->pos_table) || !block_aligned16(a->out) || !block_aligned16(a->gamma) || !block_aligned16(a->beta) ||
       (a->table_stride & 7) || a->table_stride < a->width)
     return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, table_stride a multiple of 8 elements and >= width");
+  if (a->sums && (!a->round_steps || !block_aligned16(a->sums))) return block_fail(HSTU_BLOCK_ERR_SHAPE, "sums go with round_steps and are 16-byte aligned");
   if ((a->rows + 3) / 4 > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
   EmbedNormParams p;
   p.ids = a->ids; p.positions = a->positions;
@@ -940,6 +914,7 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   p.rows = a->rows; p.vocab = a->vocab; p.table_stride = a->table_stride; p.n_positions = a->n_positions;
   p.width = a->width; p.eps = a->eps; p.scale = a->scale;
   p.row_map = a->row_map; p.L = a->L; p.round_steps = a->round_steps;
+  p.sums = (bf16_t*)a->sums; p.keys = a->keys;
   hipStream_t st = (hipStream_t)stream;
   const int lpr = lanes_per_row(a->width), per = 4 * (64 / lpr), ch = (a->width + 511) / 512;
   const dim3 grid((unsigned)((a->rows + per - 1) / per)), block(256);
@@ -952,45 +927,6 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   else hipLaunchKernelGGL((hstu_embed_norm<16, 64>), grid, block, 0, st, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "embed-norm kernel launch: %s", hipGetErrorString(e));
-  return HSTU_BLOCK_OK;
-}
-
-int hstu_embed_norm_bwd(const HstuEmbedNormArgs* a, const HstuNormGateBwdArgs* g, void* stream) {
-  if (!a || !g) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
-  if (a->struct_size != sizeof(HstuEmbedNormArgs) || a->version != HSTU_BLOCK_ABI_VERSION || g->struct_size != sizeof(HstuNormGateBwdArgs) ||
-      g->version != HSTU_BLOCK_ABI_VERSION)
-    return block_fail(HSTU_BLOCK_ERR_VERSION, "embed-norm backward args do not match this library");
-  if (a->rows < 0 || a->width < 8 || a->width > 2048 || (a->width & 7) || a->vocab < 1 || a->L < 0)
-    return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, vocab >= 1 and width a multiple of 8 in [8, 2048] expected");
-  if (!g->dgamma || !g->dbeta) return block_fail(HSTU_BLOCK_ERR_NULL, "dgamma and dbeta must be non-null");
-  hipStream_t st = (hipStream_t)stream;
-  const int nb = a->rows == 0 ? 0 : norm_gate_bwd_blocks(a->rows, a->width);
-  if (nb > 0) {
-    if (!a->ids || !a->table || !a->gamma || !g->dout || !g->da) return block_fail(HSTU_BLOCK_ERR_NULL, "ids, table, gamma, dout and da must be non-null");
-    if ((a->pos_table != nullptr) != (a->positions != nullptr || a->L > 0) || (a->pos_table && a->n_positions < 1))
-      return block_fail(HSTU_BLOCK_ERR_NULL, "pos_table and positions (or L) go together (with n_positions >= 1)");
-    if (!block_aligned16(a->table) || !block_aligned16(a->pos_table) || !block_aligned16(a->gamma) || !block_aligned16(g->dout) || !block_aligned16(g->da) ||
-        (a->table_stride & 7) || a->table_stride < a->width || (g->dout_stride & 7) || g->dout_stride < a->width || (g->da_stride & 7) ||
-        g->da_stride < a->width)
-      return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, row strides multiples of 8 elements and >= width");
-    const size_t need = hstu_norm_gate_bwd_workspace_bytes(a->rows, a->width);
-    if (!g->workspace || g->workspace_bytes < need || ((uintptr_t)g->workspace & 3u))
-      return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace of %zu bytes needed (hstu_norm_gate_bwd_workspace_bytes)", need);
-    NormGateBwdParams p = {};
-    p.ids = a->ids; p.positions = a->positions; p.table = (const bf16_t*)a->table; p.pos_table = (const bf16_t*)a->pos_table;
-    p.vocab = a->vocab; p.table_stride = a->table_stride; p.n_positions = a->n_positions; p.scale = a->scale; p.L = a->L; p.round_steps = a->round_steps;
-    p.row_map = a->row_map;
-    p.dout = (const bf16_t*)g->dout; p.dout_stride = g->dout_stride; p.da = (bf16_t*)g->da; p.da_stride = g->da_stride;
-    p.gamma = (const bf16_t*)a->gamma; p.partial = (float*)g->workspace;
-    p.rows = a->rows; p.width = a->width; p.eps = a->eps;
-    launch_norm_bwd<true>(p, nb, st);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "embed-norm backward kernel launch: %s", hipGetErrorString(e));
-  }
-  hipLaunchKernelGGL(hstu_colsum, dim3((unsigned)((2 * a->width + 31) / 32)), dim3(1024), 0, st, (const float*)g->workspace, nb, a->width,
-                     g->dgamma, g->dbeta);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "column-sum kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 

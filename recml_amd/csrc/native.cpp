@@ -780,37 +780,49 @@ void fill_embed(HstuEmbedNormArgs& a, const EmbedCall& c, const Tensor& table, c
   a.round_steps = c.training ? 1 : 0;
 }
 
-Tensor table_gradient(const EmbedCall& c, const Tensor& g, const Tensor& table, bool by_position) {
-  const Tensor out = fresh(table, {table.size(0), table.size(1)});
+// The gradient of the front end's table [keys, W], or (by position) of its position table, for the gradient `g` of the rows that were
+// summed from them.
+struct TableGradient {
+  int64_t keys, L;
+  double scale;
+  bool by_position;
+};
+Tensor table_gradient(const TableGradient& t, const Tensor& g, const Tensor& ids, const Tensor& row_map) {
+  const int64_t W = g.size(1);
+  const Tensor out = fresh(g, {t.keys, W});
   HstuEmbedGradArgs a;
   memset(&a, 0, sizeof(a));
   a.struct_size = sizeof(a);
   a.version = HSTU_BLOCK_ABI_VERSION;
-  a.rows = c.T; a.keys = table.size(0); a.width = (int32_t)table.size(1);
-  a.scale = by_position ? 1.0f : (float)c.scale;
-  a.g = g.const_data_ptr(); a.g_stride = table.size(1);
-  a.ids = c.ids.const_data_ptr<int64_t>();
-  if (c.row_map.defined()) a.row_map = c.row_map.const_data_ptr<int32_t>();
-  a.L = (int32_t)c.L; a.by_position = by_position ? 1 : 0;
+  a.rows = g.size(0); a.keys = t.keys; a.width = (int32_t)W;
+  a.scale = (float)t.scale;
+  a.g = g.const_data_ptr(); a.g_stride = W;
+  if (ids.defined()) a.ids = ids.const_data_ptr<int64_t>();
+  if (row_map.defined()) a.row_map = row_map.const_data_ptr<int32_t>();
+  a.L = (int32_t)t.L; a.by_position = t.by_position ? 1 : 0;
   a.out = out.data_ptr();
   const int64_t ws = (int64_t)hstu_embed_grad_workspace_bytes(a.rows, a.keys, a.width);
-  const Tensor buf = at::empty({ws}, table.options().dtype(at::kByte).requires_grad(false));
+  const Tensor buf = at::empty({ws}, g.options().dtype(at::kByte));
   a.workspace = buf.data_ptr(); a.workspace_bytes = (size_t)ws;
-  block_check(hstu_embed_grad(&a, stream_of(table)), "hstu_embed_grad");
+  block_check(hstu_embed_grad(&a, stream_of(g)), "hstu_embed_grad");
   return out;
 }
 
+torch::autograd::SavedVariable keep(const Tensor& t) { return torch::autograd::SavedVariable(t, false); }
+
+// Works on the forward's own copies of the gathered rows and their keys: the caller's ids and tables may be refilled or updated
+// before it runs.
 struct EmbedBackward : public torch::autograd::Node {
-  torch::autograd::SavedVariable table, pos_table, gamma, beta;
-  bool has_pos = false;
-  EmbedCall call;
+  torch::autograd::SavedVariable rows, keys, row_map, gamma, beta;
+  bool packed = false;
+  int64_t vocab = 0, positions = 0, L = 0;     // positions = 0: no position table
+  double eps = 0.0, scale = 1.0;
 
   std::string name() const override { return "HstuEmbedBackward"; }
 
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
-    for (auto* s : {&table, &pos_table, &gamma, &beta}) s->reset_data();
-    call = EmbedCall();
+    for (auto* s : {&rows, &keys, &row_map, &gamma, &beta}) s->reset_data();
   }
 
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
@@ -818,27 +830,19 @@ struct EmbedBackward : public torch::autograd::Node {
     const at::NoGradGuard no_grad;
     torch::autograd::variable_list r(4);
     if (!grads[0].defined()) return r;
-    const Tensor t = table.unpack(), pt = has_pos ? pos_table.unpack() : Tensor(), ga = gamma.unpack(), be = beta.unpack();
-    const c10::DeviceGuard guard(t.device());
-    const int64_t W = t.size(1);
-    Tensor dout = grads[0].contiguous().view({call.T, W});
+    const Tensor x = rows.unpack(), ids = keys.unpack(), ga = gamma.unpack(), be = beta.unpack(), map = packed ? row_map.unpack() : Tensor();
+    const c10::DeviceGuard guard(x.device());
+    const int64_t T = x.size(0), W = x.size(1);
+    Tensor dout = grads[0].contiguous().view({T, W});
     if (!aligned(dout)) dout = dout.clone();
-    HstuEmbedNormArgs a;
-    fill_embed(a, call, t, pt, ga, be);
-    const Tensor da = fresh(t, {call.T, W});
-    HstuNormGateBwdArgs g;
-    memset(&g, 0, sizeof(g));
-    g.struct_size = sizeof(g);
-    g.version = HSTU_BLOCK_ABI_VERSION;
-    g.dout = dout.const_data_ptr(); g.dout_stride = W; g.da = da.data_ptr(); g.da_stride = W;
-    const Tensor sums = at::empty({2, W}, t.options().dtype(at::kFloat).requires_grad(false));
-    g.dgamma = sums.data_ptr<float>(); g.dbeta = g.dgamma + W;
-    const int64_t ws = (int64_t)hstu_norm_gate_bwd_workspace_bytes(call.T, (int32_t)W);
-    const Tensor buf = at::empty({std::max<int64_t>(ws, 16)}, t.options().dtype(at::kByte).requires_grad(false));
-    g.workspace = buf.data_ptr(); g.workspace_bytes = (size_t)buf.numel();
-    block_check(hstu_embed_norm_bwd(&a, &g, stream_of(t)), "hstu_embed_norm_bwd");
-    if (task_should_compute_output(0)) r[0] = table_gradient(call, da, t, false);
-    if (has_pos && task_should_compute_output(1)) r[1] = table_gradient(call, da, pt, true);
+    const Tensor da = fresh(x, {T, W});
+    NormGrad n;
+    n.a = {x.const_data_ptr(), W};
+    n.dout = {dout.const_data_ptr(), W};
+    n.da = da.data_ptr(); n.da_stride = W;
+    const Tensor sums = norm_backward(n, ga, be, T, W, eps);
+    if (task_should_compute_output(0)) r[0] = table_gradient({vocab, 0, scale, false}, da, ids, Tensor());
+    if (positions && task_should_compute_output(1)) r[1] = table_gradient({positions, L, 1.0, true}, da, Tensor(), map);
     if (task_should_compute_output(2)) r[2] = sums[0].to(ga.scalar_type()).view(ga.sizes());
     if (task_should_compute_output(3)) r[3] = sums[1].to(be.scalar_type()).view(be.sizes());
     return r;
@@ -1012,8 +1016,6 @@ PyObject* guarded(F&& f) {
   }
 }
 
-torch::autograd::SavedVariable keep(const Tensor& t) { return torch::autograd::SavedVariable(t, false); }
-
 // block(tokens [.., D], params, heads, head_dim, eps, alpha, n, seq_lens, seq_offsets, max_len, pos, timestamps, ts_tab, mask, bias,
 //       dropout_p, dropout_seed, prepared, workspace, differentiable) -> (out, signature, workspace, reused) or None
 // Padded tokens [B, L, D], or packed ones [T, D] with seq_offsets.
@@ -1172,23 +1174,34 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     c.training = graph;
     if (D % 8 || D > (graph ? 2048 : 8192) || c.T < 1 || c.L < 1 || gamma.numel() != D || beta.numel() != D || c.ids.numel() > (1 << 30) ||
         (graph && (table.size(0) > (1 << 30)))) Py_RETURN_NONE;
-    Tensor out;
+    Tensor out, sums, keys;
     without_lock(table, [&] {
       out = packed ? fresh(table, {c.T, D}) : fresh(table, {c.ids.size(0), c.L, D});
       HstuEmbedNormArgs e;
       fill_embed(e, c, table, pos_table, gamma, beta);
       e.out = out.data_ptr();
+      if (graph) {
+        sums = fresh(table, {c.T, D});
+        keys = at::empty({c.T}, c.ids.options());
+        e.sums = sums.data_ptr();
+        e.keys = keys.data_ptr<int64_t>();
+      }
       block_check(hstu_embed_norm_fwd(&e, stream_of(table)), "hstu_embed_norm_fwd");
       return true;
     });
     if (graph) {
       auto node = std::shared_ptr<EmbedBackward>(new EmbedBackward(), torch::autograd::deleteNode);
       node->set_next_edges(torch::autograd::collect_next_edges(table, pos_table, gamma, beta));
-      node->table = keep(table);
-      if ((node->has_pos = pos_table.defined())) node->pos_table = keep(pos_table);
+      node->rows = keep(sums);
+      node->keys = keep(keys);
+      if ((node->packed = packed)) node->row_map = keep(c.row_map);
       node->gamma = keep(gamma);
       node->beta = keep(beta);
-      node->call = std::move(c);
+      node->vocab = table.size(0);
+      node->positions = pos_table.defined() ? pos_table.size(0) : 0;
+      node->L = c.L;
+      node->eps = c.eps;
+      node->scale = c.scale;
       torch::autograd::set_history(out, node);
     }
     return THPVariable_Wrap(std::move(out));
