@@ -183,7 +183,7 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* args, void* stream);
 
 /* The gradient of a gathered table, all of it: out[v, :] = the sum of scale * g[t, :] over the rows t whose key is v, added in the
  * order of the rows with every term and partial sum rounded to bf16 (the bits of torch's gather backward; rows of up to 64
- * elements: partial sums in fp32); zeros for keys without a row.  The key is the id (or position) as hstu_embed_norm_fwd finds it, clamped
+ * elements, and by_position = 2: partial sums in fp32); zeros for keys without a row.  The key is the id (or position) as hstu_embed_norm_fwd finds it, clamped
  * into [0, keys).  out: bf16 [keys, width] contiguous. */
 typedef struct HstuEmbedGradArgs {
   uint32_t struct_size;   /* sizeof(HstuEmbedGradArgs) */
@@ -196,7 +196,7 @@ typedef struct HstuEmbedGradArgs {
   const int64_t* ids;
   const int64_t* positions;
   const int32_t* row_map;
-  int32_t L, by_position; /* by_position: the keys are positions (positions, or the entry's index modulo L) */
+  int32_t L, by_position; /* by_position 1 or 2: the keys are positions (positions, or the entry's index modulo L) */
   void* out;
   void* workspace;
   size_t workspace_bytes;

@@ -494,6 +494,7 @@ struct EmbedGradParams {
   const int32_t* row_map;
   int64_t T, V, g_stride, out_stride;
   int32_t L, width, by_position;
+  int32_t round_sums;  // every partial sum rounded to bf16
   float scale;
   int32_t* count;      // [V]: tokens of a key, then where its run starts
   int32_t* rank;       // [T]: a token's place in its run
@@ -607,7 +608,7 @@ __global__ __launch_bounds__(256) void hstu_eg_short(const EmbedGradParams p) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
             s[k] += p.scale == 1.f ? f[k] : round_bf16(f[k] * p.scale);
-            s[k] = p.width > 64 ? round_bf16(s[k]) : s[k];
+            s[k] = p.round_sums ? round_bf16(s[k]) : s[k];
           }
         }
       }
@@ -951,6 +952,8 @@ int hstu_embed_grad(const HstuEmbedGradArgs* a, void* stream) {
   p.g = (const bf16_t*)a->g; p.out = (bf16_t*)a->out; p.ids = a->ids; p.positions = a->positions; p.row_map = a->row_map;
   p.T = a->rows; p.V = a->keys; p.g_stride = a->g_stride; p.out_stride = a->width; p.L = a->L; p.width = a->width; p.by_position = a->by_position;
   p.scale = a->scale;
+  // (a position's rows in a padded batch were not gathered but broadcast: that gradient is one fp32 sum, rounded once)
+  p.round_sums = a->width > 64 && a->by_position != 2;
   p.count = (int32_t*)(base + w.count); p.rank = (int32_t*)(base + w.rank); p.order = (int32_t*)(base + w.order); p.heads = (int32_t*)(base + w.heads);
   p.shorts = (int4*)(base + w.short_list); p.longs = (int4*)(base + w.long_list); p.sorted = (int32_t*)(base + w.sorted);
   hipStream_t st = (hipStream_t)stream;
@@ -968,7 +971,7 @@ int hstu_embed_grad(const HstuEmbedGradArgs* a, void* stream) {
       if (int rc = block_allow_lds((const void*)hstu_eg_order, EG_WINDOW / 8, granted)) return rc;
       hipLaunchKernelGGL(hstu_eg_order, dim3((unsigned)w.longs), dim3(256), lds, st, p);
       const dim3 grid((unsigned)w.longs, (unsigned)((p.width + 127) / 128));
-      const bool wide = p.width > 64, scaled = p.scale != 1.f;
+      const bool wide = p.round_sums != 0, scaled = p.scale != 1.f;
       if (wide && scaled) hipLaunchKernelGGL((hstu_eg_long<true, true>), grid, dim3(64), 0, st, p);
       else if (wide) hipLaunchKernelGGL((hstu_eg_long<true, false>), grid, dim3(64), 0, st, p);
       else if (scaled) hipLaunchKernelGGL((hstu_eg_long<false, true>), grid, dim3(64), 0, st, p);

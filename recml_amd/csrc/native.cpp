@@ -785,7 +785,7 @@ void fill_embed(HstuEmbedNormArgs& a, const EmbedCall& c, const Tensor& table, c
 struct TableGradient {
   int64_t keys, L;
   double scale;
-  bool by_position;
+  int by_position;               // as in HstuEmbedGradArgs
 };
 Tensor table_gradient(const TableGradient& t, const Tensor& g, const Tensor& ids, const Tensor& row_map) {
   const int64_t W = g.size(1);
@@ -799,7 +799,7 @@ Tensor table_gradient(const TableGradient& t, const Tensor& g, const Tensor& ids
   a.g = g.const_data_ptr(); a.g_stride = W;
   if (ids.defined()) a.ids = ids.const_data_ptr<int64_t>();
   if (row_map.defined()) a.row_map = row_map.const_data_ptr<int32_t>();
-  a.L = (int32_t)t.L; a.by_position = t.by_position ? 1 : 0;
+  a.L = (int32_t)t.L; a.by_position = t.by_position;
   a.out = out.data_ptr();
   const int64_t ws = (int64_t)hstu_embed_grad_workspace_bytes(a.rows, a.keys, a.width);
   const Tensor buf = at::empty({ws}, g.options().dtype(at::kByte));
@@ -841,8 +841,9 @@ struct EmbedBackward : public torch::autograd::Node {
     n.dout = {dout.const_data_ptr(), W};
     n.da = da.data_ptr(); n.da_stride = W;
     const Tensor sums = norm_backward(n, ga, be, T, W, eps);
-    if (task_should_compute_output(0)) r[0] = table_gradient({vocab, 0, scale, false}, da, ids, Tensor());
-    if (positions && task_should_compute_output(1)) r[1] = table_gradient({positions, L, 1.0, true}, da, Tensor(), map);
+    if (task_should_compute_output(0)) r[0] = table_gradient({vocab, 0, scale, 0}, da, ids, Tensor());
+    // (packed rows gather their positions; in a padded batch the table's rows are broadcast over the sequences: one fp32 sum then)
+    if (positions && task_should_compute_output(1)) r[1] = table_gradient({positions, L, 1.0, packed ? 1 : 2}, da, Tensor(), map);
     if (task_should_compute_output(2)) r[2] = sums[0].to(ga.scalar_type()).view(ga.sizes());
     if (task_should_compute_output(3)) r[3] = sums[1].to(be.scalar_type()).view(be.sizes());
     return r;

@@ -44,3 +44,24 @@ def test_gradients_do_not_depend_on_what_becomes_of_the_inputs(gpu, jagged, chan
   got = _grads(model, out, dout)
   for name in want:
     assert torch.equal(got[name], want[name]), name
+
+
+@pytest.mark.parametrize("rows", [32, 192])
+def test_position_gradient_of_a_padded_batch_is_one_sum(gpu, rows):
+  """The position table is broadcast over a padded batch: its gradient against the front end in float64.  Each row's gradient is rounded
+  to bf16 (2^-9 of it at most, independently) and the sum over the batch once more: 2^-8 in all; rounded at every addition it would be
+  7e-3 off for 32 sequences and 1.7e-2 for 192."""
+  g = torch.Generator().manual_seed(rows)
+  model = recml_amd.HSTU(vocab_size=500, max_positions=8, model_dim=128, num_heads=2, num_layers=0, add_head=False, dtype=BF, device=DEV, seed=3)
+  model.requires_grad_(True)
+  ids = torch.randint(0, 500, (rows, 8), generator=g).to(DEV)
+  dout = torch.randn((rows, 8, 128), generator=g).to(DEV).to(BF)
+  # (one norm alone: the model's closing norm on top of it would hide the front end's rounding behind its own)
+  x = recml_amd._native.embed(ids, model.item_embedding, model.position_embedding, model.final_norm_gamma, model.final_norm_beta, 1e-6, 1.0, None, 0, True)
+  got = torch.autograd.grad(x, model.position_embedding, dout)[0].double()
+  table, pos = model.item_embedding.detach().double(), model.position_embedding.detach().double().requires_grad_(True)
+  summed = table[ids] + pos
+  summed = summed + (summed.to(BF).double() - summed).detach()
+  out = torch.nn.functional.layer_norm(summed, (128,), eps=1e-6)
+  want = torch.autograd.grad(out, pos, dout.double())[0]
+  assert (got - want).norm() <= 2.0 ** -8 * want.norm()

@@ -73,3 +73,33 @@ def test_gathered_table_gradient(gpu, rows, keys, width, scale):
   assert lib.hstu_embed_grad(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
   torch.cuda.synchronize()
   assert torch.equal(out.cpu().long(), want)
+
+
+@pytest.mark.parametrize("B,L,keys,width,by_position", [(128, 9, 9, 72, 2), (192, 3, 5, 136, 2), (20, 40, 40, 128, 2), (128, 9, 9, 64, 1), (30, 7, 9, 136, 1)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_position_table_gradient(gpu, B, L, keys, width, by_position, packed):
+  """The keys are positions, of every entry or of those a row map names.  by_position 2: an fp32 sum rounded once, so at most half a unit
+  in the last of its 8 bits off (and what B additions in fp32 leave); by_position 1: exact on whole numbers below 256."""
+  g = torch.Generator().manual_seed(B + L)
+  rows = torch.arange(B * L) if not packed else (torch.rand(B * L, generator=g) < 0.6).nonzero().squeeze(1)
+  T, dev = rows.numel(), torch.device("cuda:0")
+  grad = torch.randn((T, width), generator=g).to(torch.bfloat16) if by_position == 2 else torch.randint(-1, 2, (T, width), generator=g).to(torch.bfloat16)
+  want = torch.zeros(keys, width, dtype=torch.float64).index_add_(0, rows % L, grad.double())
+  d, rm = grad.to(dev), rows.to(torch.int32).to(dev)
+  out = torch.full((keys, width), float("nan"), dtype=torch.bfloat16, device=dev)
+  lib = _lib_block.load()
+  ws = torch.empty(lib.hstu_embed_grad_workspace_bytes(T, keys, width) + 256, dtype=torch.uint8, device=dev)
+  a = _lib_block.HstuEmbedGradArgs()
+  a.struct_size, a.version = C.sizeof(a), _lib_block.ABI_VERSION
+  a.rows, a.keys, a.width, a.scale = T, keys, width, 1.0
+  a.g, a.g_stride, a.out, a.L, a.by_position = d.data_ptr(), width, out.data_ptr(), L, by_position
+  if packed:
+    a.row_map = rm.data_ptr()
+  a.workspace = (ws.data_ptr() + 255) // 256 * 256
+  a.workspace_bytes = ws.numel() - (a.workspace - ws.data_ptr())
+  assert lib.hstu_embed_grad(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+  got = out.cpu().double()
+  if by_position == 2:
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + B * 2.0 ** -21).all()
+  else:
+    assert want.abs().max() < 256 and torch.equal(got, want)
