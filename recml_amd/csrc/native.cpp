@@ -1169,7 +1169,8 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     const int64_t D = table.size(1);
     c.L = c.ids.size(1);
     const bool packed = c.row_map.defined();
-    if (packed && (!plain(c.row_map, dev, at::kInt) || c.row_map.numel() < c.T)) Py_RETURN_NONE;
+    // (the map's entries index ids: one with more entries is another batch's)
+    if (packed && (!plain(c.row_map, dev, at::kInt) || c.row_map.numel() < c.T || c.row_map.numel() > c.ids.numel())) Py_RETURN_NONE;
     if (!packed) c.T = c.ids.numel();
     const bool graph = a[9] == Py_True && wants_grad({&table, &pos_table, &gamma, &beta});
     c.training = graph;

@@ -327,7 +327,8 @@ class HSTU(torch.nn.Module):
     B, L = inputs.shape
     # which padded row each packed token comes from: found once (the one host wait of the packing: the token count) and used for
     # every gather and for the scatter at the end
-    got = _native.pack(seq_lens, L)
+    # (lengths of another batch size are not for the kernels: torch's shape checks below report them)
+    got = _native.pack(seq_lens, L) if seq_lens.shape == (B,) else None
     if got is None:
       lens = seq_lens.to(torch.int64).clamp(0, L)
       valid = torch.arange(L, device=inputs.device)[None, :] < lens[:, None]          # [B, L]

@@ -65,3 +65,12 @@ def test_position_gradient_of_a_padded_batch_is_one_sum(gpu, rows):
   out = torch.nn.functional.layer_norm(summed, (128,), eps=1e-6)
   want = torch.autograd.grad(out, pos, dout.double())[0]
   assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("count", [2, 5])
+@pytest.mark.parametrize("grad", [False, True])
+def test_lengths_of_another_batch_size_are_refused(gpu, count, grad):
+  """Packing is by the lengths: more of them than there are sequences would have the gather read past the ids."""
+  model = _model()
+  with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+    model(_inputs()[0], seq_lens=torch.full((count,), 7, dtype=torch.int32, device=DEV), jagged=True)
