@@ -152,7 +152,8 @@ int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* args, void* stream);
  * (row stride table_stride), pos_table: bf16 [n_positions, width] contiguous or
  * null, ids / positions: int64 [rows] (positions null with pos_table null),
  * out: bf16 [rows, width] contiguous.  Indices outside their table are clamped
- * into it (the reference's gather on an accelerator does the same).  width a
+ * into it (the reference's gather on an accelerator does the same) or, with
+ * `outside`, reported.  width a
  * multiple of 8 up to 8192; pointers and table_stride multiples of 8 elements. */
 typedef struct HstuEmbedNormArgs {
   uint32_t struct_size;   /* sizeof(HstuEmbedNormArgs) */
@@ -177,6 +178,8 @@ typedef struct HstuEmbedNormArgs {
   void* sums;             /* or null (with round_steps only): x_t is stored here as well, bf16 [rows, width], for the gradients: */
                           /* hstu_norm_gate_bwd on these rows gives the gradient at x_t, whatever becomes of the tables */
   int64_t* keys;          /* or null: the row of `table` that each row took, [rows] (the keys of hstu_embed_grad) */
+  int32_t* outside;       /* or null: indices are clamped.  Given (one int32 that the device can write): negative ids count from the */
+                          /* table's end, and the word becomes 1 when an id or a position lies outside its table (it is clamped then) */
 } HstuEmbedNormArgs;
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* args, void* stream);

@@ -104,7 +104,7 @@ class HstuEmbedNormArgs(C.Structure):
       ("positions", C.c_void_p), ("pos_table", C.c_void_p), ("n_positions", C.c_int64),
       ("gamma", C.c_void_p), ("beta", C.c_void_p), ("out", C.c_void_p),
       ("row_map", C.c_void_p), ("L", C.c_int32), ("round_steps", C.c_int32),
-      ("sums", C.c_void_p), ("keys", C.c_void_p),
+      ("sums", C.c_void_p), ("keys", C.c_void_p), ("outside", C.c_void_p),
   ]
 
 

@@ -48,5 +48,5 @@ def _first_call(name):
   return call
 
 
-_FUNCTIONS = ("attention", "block", "embed", "final_norm", "linear", "pack", "mask_lengths", "mask_is_prefix", "norm_gate_bwd")
-attention, block, embed, final_norm, linear, pack, mask_lengths, mask_is_prefix, norm_gate_bwd = (_first_call(n) for n in _FUNCTIONS)
+_FUNCTIONS = ("attention", "block", "embed", "final_norm", "linear", "pack", "mask_lengths", "raised", "norm_gate_bwd")
+attention, block, embed, final_norm, linear, pack, mask_lengths, raised, norm_gate_bwd = (_first_call(n) for n in _FUNCTIONS)

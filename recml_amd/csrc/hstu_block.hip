@@ -346,6 +346,7 @@ struct EmbedNormParams {
   int32_t round_steps;     // the scaled row and the sum are each rounded to bf16, as separate steps would leave them
   bf16_t* sums;            // the rows before the norm, for the gradients; or null
   int64_t* keys;           // the table rows taken, for the gradients; or null
+  int32_t* outside;        // raised where an index lies outside its table; or null
 };
 
 // Rows on lanes as in hstu_norm_gate: a token's table row (and position row) is gathered into registers, normalised
@@ -359,12 +360,17 @@ __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) 
   if (row >= p.rows) return;
   const int64_t at = p.row_map ? p.row_map[row] : row;
   int64_t id = p.ids[at];
+  if (p.outside) {
+    id += id < 0 ? p.vocab : 0;
+    if (id < 0 || id >= p.vocab) *p.outside = 1;
+  }
   id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
   if (p.keys && lane == 0) p.keys[row] = id;
   const bf16_t* er = p.table + id * p.table_stride;
   const bf16_t* pr = nullptr;
   if (p.pos_table) {
     int64_t ps = p.positions ? p.positions[row] : at % p.L;
+    if (p.outside && (ps < 0 || ps >= p.n_positions)) *p.outside = 1;
     ps = ps < 0 ? 0 : (ps >= p.n_positions ? p.n_positions - 1 : ps);
     pr = p.pos_table + ps * (int64_t)p.width;
   }
@@ -915,7 +921,7 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   p.rows = a->rows; p.vocab = a->vocab; p.table_stride = a->table_stride; p.n_positions = a->n_positions;
   p.width = a->width; p.eps = a->eps; p.scale = a->scale;
   p.row_map = a->row_map; p.L = a->L; p.round_steps = a->round_steps;
-  p.sums = (bf16_t*)a->sums; p.keys = a->keys;
+  p.sums = (bf16_t*)a->sums; p.keys = a->keys; p.outside = a->outside;
   hipStream_t st = (hipStream_t)stream;
   const int lpr = lanes_per_row(a->width), per = 4 * (64 / lpr), ch = (a->width + 511) / 512;
   const dim3 grid((unsigned)((a->rows + per - 1) / per)), block(256);

@@ -1151,7 +1151,59 @@ PyObject* norm_gate_bwd(PyObject*, PyObject* const* a, Py_ssize_t count) {
   });
 }
 
-// embed(ids, table, pos_table, gamma, beta, eps, scale, row_map, tokens, differentiable) -> [tokens, D] (or shaped like ids) or None
+// A word in pinned host memory that a kernel writes, and the event behind that kernel.
+struct Word {
+  Tensor host;
+  hipEvent_t done = nullptr;
+  explicit Word(const Tensor& like) {
+    host = at::empty({1}, like.options().dtype(at::kInt).device(at::kCPU).pinned_memory(true).requires_grad(false));
+    *host.data_ptr<int32_t>() = 0;
+    TORCH_CHECK(hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
+  }
+  Word(const Word&) = delete;
+  void record(void* stream) { TORCH_CHECK(hipEventRecord(done, (hipStream_t)stream) == hipSuccess, "hipEventRecord failed"); }
+  int32_t wait() {
+    TORCH_CHECK(hipEventSynchronize(done) == hipSuccess, "hipEventSynchronize failed");
+    return *(volatile int32_t*)host.data_ptr<int32_t>();
+  }
+  ~Word() {
+    // (the word must not go back to the pool while the kernel may still write it)
+    if (done) {
+      (void)hipEventSynchronize(done);
+      (void)hipEventDestroy(done);
+    }
+  }
+};
+
+void drop_word(PyObject* capsule) { delete (Word*)PyCapsule_GetPointer(capsule, "recml_amd.word"); }
+
+// Hands a word over to Python as a ticket: raised(ticket) says whether its kernel raised it.
+PyObject* ticket_of(std::unique_ptr<Word> word) {
+  PyObject* const capsule = PyCapsule_New(word.get(), "recml_amd.word", drop_word);
+  if (capsule) word.release();
+  return capsule;
+}
+
+PyObject* raised(PyObject*, PyObject* ticket) {
+  return guarded([&]() -> PyObject* {
+    Word* const word = (Word*)PyCapsule_GetPointer(ticket, "recml_amd.word");
+    if (!word) return nullptr;
+    int32_t value;
+    Py_BEGIN_ALLOW_THREADS
+    value = word->wait();
+    Py_END_ALLOW_THREADS
+    return PyBool_FromLong(value != 0);
+  });
+}
+
+bool capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+// embed(ids, table, pos_table, gamma, beta, eps, scale, row_map, tokens, differentiable) -> (rows [tokens, D] (or shaped like ids), ticket)
+// or None.  Without gradients indices are clamped into their tables and the ticket is None; with them they are taken as torch's indexing
+// takes them, and raised(ticket) says that one lay outside.  (A captured step has no ticket: nobody can ask while it is captured.)
 PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
   if (count != 10) {
     PyErr_SetString(PyExc_TypeError, "embed takes 10 arguments");
@@ -1173,10 +1225,13 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (packed && (!plain(c.row_map, dev, at::kInt) || c.row_map.numel() < c.T || c.row_map.numel() > c.ids.numel())) Py_RETURN_NONE;
     if (!packed) c.T = c.ids.numel();
     const bool graph = a[9] == Py_True && wants_grad({&table, &pos_table, &gamma, &beta});
+    // (a padded batch longer than the position table: torch's addition reports it)
+    if (graph && !packed && pos_table.defined() && pos_table.size(0) < c.L) Py_RETURN_NONE;
     c.training = graph;
     if (D % 8 || D > (graph ? 2048 : 8192) || c.T < 1 || c.L < 1 || gamma.numel() != D || beta.numel() != D || c.ids.numel() > (1 << 30) ||
         (graph && (table.size(0) > (1 << 30)))) Py_RETURN_NONE;
     Tensor out, sums, keys;
+    std::unique_ptr<Word> outside;
     without_lock(table, [&] {
       out = packed ? fresh(table, {c.T, D}) : fresh(table, {c.ids.size(0), c.L, D});
       HstuEmbedNormArgs e;
@@ -1187,8 +1242,13 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
         keys = at::empty({c.T}, c.ids.options());
         e.sums = sums.data_ptr();
         e.keys = keys.data_ptr<int64_t>();
+        if (!capturing(stream_of(table))) {
+          outside = std::make_unique<Word>(table);
+          e.outside = outside->host.data_ptr<int32_t>();
+        }
       }
       block_check(hstu_embed_norm_fwd(&e, stream_of(table)), "hstu_embed_norm_fwd");
+      if (outside) outside->record(stream_of(table));
       return true;
     });
     if (graph) {
@@ -1206,7 +1266,8 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
       node->scale = c.scale;
       torch::autograd::set_history(out, node);
     }
-    return THPVariable_Wrap(std::move(out));
+    PyObject* const ticket = outside ? ticket_of(std::move(outside)) : (Py_INCREF(Py_None), Py_None);
+    return ticket ? Py_BuildValue("(NN)", THPVariable_Wrap(std::move(out)), ticket) : nullptr;
   });
 }
 
@@ -1282,30 +1343,6 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t count) {
   });
 }
 
-// A word in pinned host memory that a kernel writes, and the event behind that kernel.
-struct Word {
-  Tensor host;
-  hipEvent_t done = nullptr;
-  explicit Word(const Tensor& like) {
-    host = at::empty({1}, like.options().dtype(at::kInt).device(at::kCPU).pinned_memory(true).requires_grad(false));
-    *host.data_ptr<int32_t>() = 0;
-    TORCH_CHECK(hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
-  }
-  Word(const Word&) = delete;
-  void record(void* stream) { TORCH_CHECK(hipEventRecord(done, (hipStream_t)stream) == hipSuccess, "hipEventRecord failed"); }
-  int32_t wait() {
-    TORCH_CHECK(hipEventSynchronize(done) == hipSuccess, "hipEventSynchronize failed");
-    return *(volatile int32_t*)host.data_ptr<int32_t>();
-  }
-  ~Word() {
-    // (the word must not go back to the pool while the kernel may still write it)
-    if (done) {
-      (void)hipEventSynchronize(done);
-      (void)hipEventDestroy(done);
-    }
-  }
-};
-
 // pack(lens, length) -> (seq_offsets, row_map, tokens) of the batch's packed form, or None.  Waits for the token count.
 PyObject* pack(PyObject*, PyObject* const* a, Py_ssize_t count) {
   if (count != 2) {
@@ -1333,10 +1370,8 @@ PyObject* pack(PyObject*, PyObject* const* a, Py_ssize_t count) {
   });
 }
 
-void drop_word(PyObject* capsule) { delete (Word*)PyCapsule_GetPointer(capsule, "recml_amd.word"); }
-
-// mask_lengths(mask [B, L] of bytes) -> (lengths int32 [B], ticket) or None; mask_is_prefix(ticket) -> whether every row was
-// end-padded.  Two steps, so that the work on the lengths is enqueued before anyone waits.
+// mask_lengths(mask [B, L] of bytes) -> (lengths int32 [B], ticket) or None; raised(ticket) -> whether a row was not end-padded.
+// Two steps, so that the work on the lengths is enqueued before anyone waits.
 PyObject* mask_lengths(PyObject*, PyObject* const* a, Py_ssize_t count) {
   if (count != 1) {
     PyErr_SetString(PyExc_TypeError, "mask_lengths takes 1 argument");
@@ -1347,33 +1382,17 @@ PyObject* mask_lengths(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (!tensor_arg(a[0], &mask) || !mask.defined() || !mask.is_cuda() || mask.dim() != 2 || mask.size(0) < 1 || mask.size(1) < 1 || !mask.is_contiguous() ||
         (mask.scalar_type() != at::kBool && mask.scalar_type() != at::kByte) || mask.numel() > 0x7fffffff) Py_RETURN_NONE;
     Tensor lens;
-    Word* const word = without_lock(mask, [&]() -> Word* {
+    auto word = without_lock(mask, [&] {
       lens = at::empty({mask.size(0)}, mask.options().dtype(at::kInt));
       auto bad = std::make_unique<Word>(mask);
       void* const st = stream_of(mask);
       block_check(hstu_mask_lengths((const uint8_t*)mask.const_data_ptr(), (int32_t)mask.size(0), (int32_t)mask.size(1), lens.data_ptr<int32_t>(),
                                     bad->host.data_ptr<int32_t>(), st), "hstu_mask_lengths");
       bad->record(st);
-      return bad.release();
+      return bad;
     });
-    PyObject* const capsule = PyCapsule_New(word, "recml_amd.word", drop_word);
-    if (!capsule) {
-      delete word;
-      return nullptr;
-    }
-    return Py_BuildValue("(NN)", THPVariable_Wrap(lens), capsule);
-  });
-}
-
-PyObject* mask_is_prefix(PyObject*, PyObject* ticket) {
-  return guarded([&]() -> PyObject* {
-    Word* const word = (Word*)PyCapsule_GetPointer(ticket, "recml_amd.word");
-    if (!word) return nullptr;
-    int32_t bad;
-    Py_BEGIN_ALLOW_THREADS
-    bad = word->wait();
-    Py_END_ALLOW_THREADS
-    return PyBool_FromLong(bad == 0);
+    PyObject* const ticket = ticket_of(std::move(word));
+    return ticket ? Py_BuildValue("(NN)", THPVariable_Wrap(lens), ticket) : nullptr;
   });
 }
 
@@ -1401,7 +1420,7 @@ PyMethodDef methods[] = {
     HSTU_FAST(linear, "A matrix product with gradients."),
     HSTU_FAST(pack, "The packed form of a padded batch."),
     HSTU_FAST(mask_lengths, "Lengths of an end-padded batch from its mask."),
-    {"mask_is_prefix", mask_is_prefix, METH_O, "Whether the mask behind a mask_lengths ticket was end-padded."},
+    {"raised", raised, METH_O, "Whether the kernel behind a ticket found what it looks for (waits for that kernel)."},
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -264,11 +264,13 @@ class HSTU(torch.nn.Module):
 
   def _front_end(self, ids, row_map=None, tokens=0):
     """Gather, scale, position embedding and final_norm (hstu.py:593-601): in bf16 on a GPU one pass, and one each for the
-    gradients of the norm and of the tables.  ids [B, L]; the packed form with `row_map` (its `tokens` first entries)."""
+    gradients of the norm and of the tables.  ids [B, L]; the packed form with `row_map` (its `tokens` first entries).
+    Returns the rows and, with gradients, a ticket for _check_indices."""
     table, positions = self.item_embedding, self.position_embedding
     scale = self.model_dim ** 0.5 if self.scale_by_sqrt_dim else 1.0
-    x = _native.embed(ids if ids.dtype == torch.int64 and ids.is_contiguous() else ids.to(torch.int64).contiguous(), table, positions,
+    got = _native.embed(ids if ids.dtype == torch.int64 and ids.is_contiguous() else ids.to(torch.int64).contiguous(), table, positions,
                       self.final_norm_gamma, self.final_norm_beta, self.eps, scale, row_map, tokens, True)
+    x, ticket = (None, None) if got is None else got
     if x is None:
       where = None if row_map is None else row_map[:tokens].to(torch.int64)
       x = table[ids if where is None else ids.reshape(-1)[where]]
@@ -277,7 +279,14 @@ class HSTU(torch.nn.Module):
       if positions is not None:
         x = x + (positions[: ids.shape[1]] if where is None else positions[where % ids.shape[1]])
       x = self._final_norm(x)
-    return F.dropout(x, self.dropout, self.training) if self.training and self.dropout > 0.0 else x
+    return (F.dropout(x, self.dropout, self.training) if self.training and self.dropout > 0.0 else x), ticket
+
+  def _check_indices(self, ticket):
+    """Raises where the front end met an id outside the vocabulary or a position past the table (in training; inference clamps them).
+    Asked when the rest of the forward is enqueued: the answer is there by then."""
+    if ticket is not None and _native.raised(ticket):
+      raise IndexError(f"an item id lies outside the vocabulary of {self.item_embedding.shape[0]}"
+                       + ("" if self.position_embedding is None else f", or a position past the {self.position_embedding.shape[0]} there are"))
 
   def _head(self, x):
     out = _native.linear(x, self.reverse_embedding, True)
@@ -308,7 +317,7 @@ class HSTU(torch.nn.Module):
     if jagged:
       out = self._forward_jagged(inputs, seq_lens, pos_bias, timestamps, ts_bias)
     else:
-      x = self._front_end(inputs)
+      x, outside = self._front_end(inputs)
       # every block sees the same lengths, timestamps and tables: the attention prepares them once
       batch = hstu_ops.AttentionBatch()
       for block in self.decoder_blocks:
@@ -319,7 +328,8 @@ class HSTU(torch.nn.Module):
       out = self._final_norm(x)
       if self.reverse_embedding is not None:
         out = self._head(out)
-    if ticket is not None and not _native.mask_is_prefix(ticket):
+      self._check_indices(outside)
+    if ticket is not None and _native.raised(ticket):
       raise ValueError(masks.NOT_END_PADDED)
     return out
 
@@ -338,7 +348,7 @@ class HSTU(torch.nn.Module):
       tokens = rows.numel()
     else:
       offsets, rows, tokens = got
-    x = self._front_end(inputs, rows, tokens)
+    x, outside = self._front_end(inputs, rows, tokens)
     ts = None if timestamps is None else timestamps.reshape(-1).index_select(0, rows[:tokens])
     batch = hstu_ops.AttentionBatch()
     for block in self.decoder_blocks:
@@ -346,9 +356,11 @@ class HSTU(torch.nn.Module):
     if self.reverse_embedding is None:
       out = _native.final_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps, offsets, rows, B, L, True)
       if out is not None:
+        self._check_indices(outside)
         return out
     x = self._final_norm(x)
     if self.reverse_embedding is not None:
       x = self._head(x)
+    self._check_indices(outside)
     out = torch.zeros((B * L, x.shape[-1]), dtype=x.dtype, device=x.device)
     return out.index_copy(0, rows[:tokens].to(torch.int64), x).reshape(B, L, x.shape[-1])

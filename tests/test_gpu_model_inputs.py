@@ -57,7 +57,7 @@ def test_position_gradient_of_a_padded_batch_is_one_sum(gpu, rows):
   ids = torch.randint(0, 500, (rows, 8), generator=g).to(DEV)
   dout = torch.randn((rows, 8, 128), generator=g).to(DEV).to(BF)
   # (one norm alone: the model's closing norm on top of it would hide the front end's rounding behind its own)
-  x = recml_amd._native.embed(ids, model.item_embedding, model.position_embedding, model.final_norm_gamma, model.final_norm_beta, 1e-6, 1.0, None, 0, True)
+  x = model._front_end(ids)[0]
   got = torch.autograd.grad(x, model.position_embedding, dout)[0].double()
   table, pos = model.item_embedding.detach().double(), model.position_embedding.detach().double().requires_grad_(True)
   summed = table[ids] + pos
@@ -74,3 +74,42 @@ def test_lengths_of_another_batch_size_are_refused(gpu, count, grad):
   model = _model()
   with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
     model(_inputs()[0], seq_lens=torch.full((count,), 7, dtype=torch.int32, device=DEV), jagged=True)
+
+
+@pytest.mark.parametrize("jagged", [False, True])
+def test_ids_out_of_the_vocabulary(gpu, jagged):
+  """With gradients ids are taken as torch's indexing takes them: negative ones count from the end, others are an error.  Without,
+  they are clamped."""
+  model = _model()
+  ids, lens, dout = _inputs()
+  last, negative = ids.clone(), ids.clone()
+  last[0, 3], negative[0, 3] = V - 1, -1
+  want = _grads(model, model(last, seq_lens=lens, jagged=jagged), dout)
+  got = _grads(model, model(negative, seq_lens=lens, jagged=jagged), dout)
+  assert all(torch.equal(got[n], want[n]) for n in want)
+  for bad in (V, -V - 1):
+    out_of_range = ids.clone()
+    out_of_range[0, 3] = bad
+    with pytest.raises(IndexError):
+      model(out_of_range, seq_lens=lens, jagged=jagged)
+    with torch.no_grad():
+      clamped = model(out_of_range.clamp(0, V - 1), seq_lens=lens, jagged=jagged)
+      assert torch.equal(model(out_of_range, seq_lens=lens, jagged=jagged), clamped)
+  # past the sequences' ends packed ids are never read
+  out_of_range = ids.clone()
+  out_of_range[2, 5] = V
+  if jagged:
+    assert model(out_of_range, seq_lens=lens, jagged=True).isfinite().all()
+
+
+def test_positions_past_the_table(gpu):
+  """A batch longer than the position table: an error with gradients, in the packed form where a token reaches past it."""
+  model = _model()
+  g = torch.Generator().manual_seed(1)
+  ids = torch.randint(1, V, (B, L + 8), generator=g).to(DEV)
+  lens = lambda n: torch.tensor([n, 17, 1], dtype=torch.int32, device=DEV)
+  with pytest.raises(RuntimeError):
+    model(ids, seq_lens=lens(L))
+  assert model(ids, seq_lens=lens(L), jagged=True).isfinite().all()
+  with pytest.raises(IndexError):
+    model(ids, seq_lens=lens(L + 1), jagged=True)
