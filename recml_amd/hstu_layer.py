@@ -127,13 +127,16 @@ class HSTUBlock(torch.nn.Module):
     make_causal_mask does for an end-padded batch) with optional bias tables;
     or, for the reference's calling convention, a dense `attention_mask`
     [B, L, L] and optional `attention_bias` [B, L, L]
-    (recml/layers/keras/hstu.py:422-440).  `batch`: an `hstu_ops.AttentionBatch` shared with the
+    (recml/layers/keras/hstu.py:422-440), beside which lengths and tables are not looked at.  `batch`: an `hstu_ops.AttentionBatch` shared with the
     other blocks that see the same lengths, timestamps and tables.  `dropout_seed`: in training mode
     with a dropout rate, the seed of this call's keep pattern (default: drawn from torch's generator).
     """
     drop = self._dropout_kw(dropout_seed)
     B, L, D = inputs.shape
     H, hd = self.num_heads, self.head_dim
+    if attention_mask is not None:
+      # the mask stands in place of the lengths, and the dense bias in place of the tables (hstu.py:422-440)
+      seq_lens = pos_bias = timestamps = ts_bias = None
     out = self._native_steps(inputs, L, batch, drop, pos_bias, timestamps, ts_bias, seq_lens=seq_lens,
                              attention_mask=attention_mask, attention_bias=attention_bias)
     if out is not None:
