@@ -52,7 +52,7 @@ def _norm_gate_fwd(attn, u, gamma, beta, eps):
   a.a_stride, a.out_stride = a2.stride(0), W
   if u2 is not None:
     a.u, a.u_stride = u2.data_ptr(), u2.stride(0)
-  g, b = gamma.reshape(-1).contiguous(), beta.reshape(-1).contiguous()
+  g, b = _vector(gamma), _vector(beta)
   if g.numel() != W or b.numel() != W:
     raise ValueError(f"gamma and beta must have {W} entries")
   a.gamma, a.beta = g.data_ptr(), b.data_ptr()
@@ -109,7 +109,7 @@ def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None,
       raise ValueError("add must be shaped like attn")
     add2 = _rows(add, "add")
     a.add, a.add_stride = add2.data_ptr(), add2.stride(0)
-  g, b = gamma.reshape(-1).contiguous(), beta.reshape(-1).contiguous()
+  g, b = _vector(gamma), _vector(beta)
   if g.numel() != W or b.numel() != W:
     raise ValueError(f"gamma and beta must have {W} entries")
   a.gamma, a.beta = g.data_ptr(), b.data_ptr()
@@ -181,16 +181,23 @@ def layer_norm(x, gamma, beta, eps: float = 1e-6):
 
 
 def _rows(t, name):
-  """[..., W] -> a [rows, W] view with one row stride (a copy when the layout does not allow it)."""
+  """[..., W] -> a [rows, W] view with one row stride of whole 16-byte pieces (a copy when the layout does not allow it)."""
   W = t.shape[-1]
   if t.stride(-1) != 1:
     t = t.contiguous()
-  try:
-    return t.view(-1, W) if t.dim() != 2 else t
-  except RuntimeError:
-    pass
-  # leading axes of a strided slice: [T, W] slices are 2-d already; anything else is flattened by a copy
-  return t.reshape(-1, W)
+  if t.dim() != 2:
+    try:
+      t = t.view(-1, W)
+    except RuntimeError:
+      # leading axes of a strided slice: [T, W] slices are 2-d already; anything else is flattened by a copy
+      t = t.reshape(-1, W)
+  return t if t.data_ptr() % 16 == 0 and (t.stride(0) % 8 == 0 or W % 8) else t.clone(memory_format=torch.contiguous_format)
+
+
+def _vector(t):
+  """A norm's scale or offset as the kernels read it: contiguous, on a 16-byte boundary (a copy when it is not)."""
+  t = t.reshape(-1).contiguous()
+  return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def gemm_silu(x, w, bias=None, activation: bool = True, residual=None):
@@ -315,7 +322,7 @@ def embed_norm(ids, table, gamma, beta, eps: float = 1e-6, *, scale: float = 1.0
     pt, pf = pos_table.contiguous(), positions.reshape(-1).contiguous()
     keep += [pt, pf]
     a.positions, a.pos_table, a.n_positions = pf.data_ptr(), pt.data_ptr(), pt.shape[0]
-  g, b = gamma.reshape(-1).contiguous(), beta.reshape(-1).contiguous()
+  g, b = _vector(gamma), _vector(beta)
   if g.numel() != W or b.numel() != W:
     raise ValueError(f"gamma and beta must have {W} entries")
   a.gamma, a.beta, a.out = g.data_ptr(), b.data_ptr(), out.data_ptr()

@@ -33,6 +33,7 @@ import torch
 import torch.nn.functional as F
 
 from recml_amd import _native
+from recml_amd import hstu_block_ops
 from recml_amd import hstu_ops
 from recml_amd import masks
 
@@ -48,6 +49,66 @@ def _attention(q, k, v, *, pos_bias=None, ts_bias=None, batch=None, **kw):
   if _wants_grad(q, k, v, pos_bias, ts_bias, kw.get("bias")):
     return hstu_ops.hstu_attention_autograd(q, k, v, pos_bias=pos_bias, ts_bias=ts_bias, **kw)
   return hstu_ops.hstu_attention(q, k, v, pos_bias=pos_bias, ts_bias=ts_bias, batch=batch, **kw)
+
+
+class _AttentionGateFn(torch.autograd.Function):
+  """gated = u * layer_norm(attention(q, k, v)) on the four slices of ONE projection uqkv [..., 4, H, hd]
+  (contiguous, bf16), with every gradient through the HIP kernels, which write dq, dk, dv and du straight
+  into the slices of one gradient tensor shaped like the projection."""
+
+  @staticmethod
+  def forward(ctx, uqkv, gamma, beta, pos_bias, ts_bias, eps, batch, kwargs):
+    uqkv = uqkv.contiguous()            # (the backward mirrors this layout for the gradient)
+    u, q, k, v = uqkv.unbind(dim=-3)
+    attn = hstu_ops.hstu_attention(q, k, v, pos_bias=pos_bias, ts_bias=ts_bias, batch=batch, **kwargs)
+    W = q.shape[-2] * q.shape[-1]
+    gated = hstu_block_ops.norm_gate(attn.reshape(-1, W).detach(), u.reshape(-1, W).detach(), gamma.detach().reshape(-1),
+                                     beta.detach().reshape(-1), eps)
+    ctx.save_for_backward(uqkv, attn, gamma, beta, *(t for t in (pos_bias, ts_bias) if t is not None))
+    ctx.has = (pos_bias is not None, ts_bias is not None)
+    ctx.eps, ctx.kwargs = eps, kwargs
+    return gated.reshape(*uqkv.shape[:-3], W)
+
+  @staticmethod
+  def backward(ctx, dgated):
+    uqkv, attn, gamma, beta, *rest = ctx.saved_tensors
+    pos = rest.pop(0) if ctx.has[0] else None
+    ts = rest.pop(0) if ctx.has[1] else None
+    u, q, k, v = uqkv.unbind(dim=-3)
+    W = q.shape[-2] * q.shape[-1]
+    d_uqkv = torch.empty_like(uqkv)                     # uqkv is contiguous: the same strides
+    du, dq, dk, dv = d_uqkv.unbind(dim=-3)
+    du2 = du.reshape(-1, W)
+    assert du2.data_ptr() == du.data_ptr()              # a view: the kernel writes into d_uqkv
+    d_attn, _, dg, db = hstu_block_ops.norm_gate_bwd(attn.reshape(-1, W), u.reshape(-1, W), gamma.reshape(-1), beta.reshape(-1),
+                                                     dgated.reshape(-1, W).contiguous(), ctx.eps, du_out=du2)
+    # needs_input_grad follows forward's arguments: uqkv, gamma, beta, pos_bias, ts_bias, ...
+    want_tables = (pos is not None and ctx.needs_input_grad[3]) or (ts is not None and ctx.needs_input_grad[4])
+    _, _, _, dpos, dts = hstu_ops.hstu_attention_bwd(q, k, v, d_attn.reshape(attn.shape), pos_bias=pos, ts_bias=ts,
+                                                     table_grads=want_tables, grads_out=(dq, dk, dv), **ctx.kwargs)
+    cast = lambda g, t: None if g is None else g.to(t.dtype)
+    return (d_uqkv, dg.to(gamma.dtype).reshape(gamma.shape), db.to(beta.dtype).reshape(beta.shape),
+            cast(dpos, pos) if pos is not None else None, cast(dts, ts) if ts is not None else None, None, None, None)
+
+
+class _OutputProjectionFn(torch.autograd.Function):
+  """gated @ W (+ bias) + residual with the residual as the product's C operand (recml/layers/keras/hstu.py:473-474):
+  torch's addmm copies the residual into the output before the product.  The gradients are two plain products."""
+
+  @staticmethod
+  def forward(ctx, gated, w, bias, residual):
+    ctx.save_for_backward(gated, w)
+    ctx.has_bias = bias is not None
+    return hstu_block_ops.gemm_silu(gated, w, bias, False, residual=residual)
+
+  @staticmethod
+  def backward(ctx, dout):
+    gated, w = ctx.saved_tensors
+    need = ctx.needs_input_grad
+    d_gated = dout @ w.t() if need[0] else None
+    d_w = gated.t() @ dout if need[1] else None
+    d_bias = dout.sum(0) if (ctx.has_bias and need[2]) else None
+    return d_gated, d_w, d_bias, dout if need[3] else None
 
 
 def _glorot_uniform(shape, fan_in, fan_out, generator, dtype, device):
@@ -141,36 +202,49 @@ class HSTUBlock(torch.nn.Module):
                              attention_mask=attention_mask, attention_bias=attention_bias)
     if out is not None:
       return out
-    x = F.layer_norm(inputs, (D,), self.input_ln_gamma, self.input_ln_beta, self.eps)
-    u, q, k, v = self._project(x.reshape(B * L, D), (B, L)).unbind(dim=2)
+    alpha, n = self._alpha_n(L)
+    if attention_mask is None and attention_bias is None and self._fused_training(inputs, pos_bias, ts_bias):
+      return self._train_steps(inputs.reshape(B * L, D), (B, L), pos_bias, ts_bias, batch,
+                               dict(seq_lens=seq_lens, n=n, alpha=alpha, timestamps=timestamps, **drop)).reshape(B, L, D)
+    fused = self._fused_inference(inputs, pos_bias, ts_bias, attention_bias)
+    u, q, k, v = self._project(self._input_norm(inputs, fused).reshape(B * L, D), (B, L), fused).unbind(dim=2)
     if attention_mask is not None:
       # the reference's calling convention: a dense [B, L, L] mask and bias (training: forward and backward kernels,
       # the gradient of a dense bias included)
       attn = hstu_ops.pointwise_attention(q, k, v, attention_mask, attention_bias,
                                           scaled_pointwise_attn=self.scaled_pointwise_attn, batch=batch, **drop)
     else:
-      alpha, n = self._alpha_n(L)
       attn = _attention(q, k, v, seq_lens=seq_lens, n=n, alpha=alpha, pos_bias=pos_bias,
                         timestamps=timestamps, ts_bias=ts_bias, bias=attention_bias, batch=batch, **drop)
-    return self._gate_and_output(attn.reshape(B * L, H * hd), u.reshape(B * L, H * hd), inputs.reshape(B * L, D)).reshape(B, L, D)
+    return self._gate_and_output(attn.reshape(B * L, H * hd), u.reshape(B * L, H * hd), inputs.reshape(B * L, D), fused).reshape(B, L, D)
 
   def _alpha_n(self, L):
     """The logit scale and the normaliser (recml/layers/keras/hstu.py:365-378)."""
     return (1.0 / math.sqrt(self.head_dim), 1.0) if self.scaled_pointwise_attn else (1.0, float(L))
 
-  def _project(self, x, lead):
-    """U, Q, K, V of normalised rows in torch: [*lead, 4, H, hd]."""
-    w, b = self._uqkv_weights()
-    uqkv = x @ w
-    if b is not None:
-      uqkv = uqkv + b
-    return F.silu(uqkv).reshape(*lead, 4, self.num_heads, self.head_dim)
+  def _input_norm(self, t, fused):
+    if fused:
+      return hstu_block_ops.layer_norm(t, self.input_ln_gamma, self.input_ln_beta, self.eps)
+    return F.layer_norm(t, (self.hidden_dim,), self.input_ln_gamma, self.input_ln_beta, self.eps)
 
-  def _gate_and_output(self, attn, u, residual):
-    """Attention norm, U gate, output product and residual in torch, on rows."""
+  def _project(self, x, lead, fused):
+    """U, Q, K, V of normalised rows: [*lead, 4, H, hd].  `fused`: the activation in the product's epilogue."""
+    w, b = self._uqkv_weights()
+    if fused:
+      uqkv = hstu_block_ops.gemm_silu(x, w, b, True)
+    else:
+      uqkv = x @ w
+      uqkv = F.silu(uqkv if b is None else uqkv + b)
+    return uqkv.reshape(*lead, 4, self.num_heads, self.head_dim)
+
+  def _gate_and_output(self, attn, u, residual, fused):
+    """Attention norm, U gate, output product and residual, on rows.  `fused`: norm and gate in one pass, rounded once, and the
+    residual as the product's C operand."""
     W = attn.shape[-1]
-    normed = F.layer_norm(attn, (W,), self.attn_ln_gamma.reshape(-1), self.attn_ln_beta.reshape(-1), self.eps)
-    out = (u * normed) @ self.output_kernel.reshape(W, self.hidden_dim)
+    gamma, beta, w = self.attn_ln_gamma.reshape(-1), self.attn_ln_beta.reshape(-1), self.output_kernel.reshape(W, self.hidden_dim)
+    if fused:
+      return hstu_block_ops.gemm_silu(hstu_block_ops.norm_gate(attn, u, gamma, beta, self.eps), w, self.output_bias, False, residual=residual)
+    out = (u * F.layer_norm(attn, (W,), gamma, beta, self.eps)) @ w
     if self.use_bias:
       out = out + self.output_bias
     return out + residual
@@ -178,9 +252,28 @@ class HSTUBlock(torch.nn.Module):
   def _wants_grad(self, *tensors) -> bool:
     return torch.is_grad_enabled() and (any(p is not None and p.requires_grad for p in self._parameters.values()) or _wants_grad(*tensors))
 
+  def _fused_inference(self, t, *bias_inputs) -> bool:
+    """Whether the steps of hstu_block_ops apply where the native call does not: bf16 on a GPU, nothing asking for gradients, widths
+    the norm kernels take."""
+    D = self.hidden_dim
+    return t.is_cuda and t.dtype == torch.bfloat16 and D % 8 == 0 and D <= 8192 and not self._wants_grad(t, *bias_inputs)
+
   def _fused_training(self, t, *bias_inputs) -> bool:
-    """Whether a call that asks for gradients may take the fused steps."""
-    return True
+    """Whether the training form of the fused steps (native, or _train_steps) applies: bf16 on a GPU, something asking for a gradient,
+    widths the norm kernels' backward takes."""
+    D, W = self.hidden_dim, self.num_heads * self.head_dim
+    return (t.is_cuda and t.dtype == torch.bfloat16 and self._wants_grad(t, *bias_inputs)
+            and D % 8 == 0 and W % 8 == 0 and D <= 2048 and W <= 2048)
+
+  def _train_steps(self, tokens, lead, pos_bias, ts_bias, batch, attn_kw):
+    """The block on rows [T, D] with gradients where the native call does not apply (head dims or parameters that are not laid out for
+    it): norms, attention and gate through the HIP kernels, the products and the projections' SiLU in torch.  `lead`: the leading
+    shape of the attention's tensors ((B, L) padded, (T,) packed)."""
+    x = hstu_block_ops.layer_norm(tokens, self.input_ln_gamma, self.input_ln_beta, self.eps)
+    uqkv = self._project(x, lead, False)
+    gated = _AttentionGateFn.apply(uqkv, self.attn_ln_gamma, self.attn_ln_beta, pos_bias, ts_bias, self.eps, batch, attn_kw)
+    W = self.num_heads * self.head_dim
+    return _OutputProjectionFn.apply(gated.reshape(-1, W), self.output_kernel.reshape(W, self.hidden_dim), self.output_bias, tokens)
 
   def _native_steps(self, tokens, length, batch, drop, pos_bias, timestamps, ts_bias, seq_lens=None, seq_offsets=None,
                     attention_mask=None, attention_bias=None):
@@ -224,12 +317,15 @@ class HSTUBlock(torch.nn.Module):
     out = self._native_steps(tokens, int(max_len), batch, drop, pos_bias, timestamps, ts_bias, seq_offsets=seq_offsets)
     if out is not None:
       return out
-    x = F.layer_norm(tokens, (D,), self.input_ln_gamma, self.input_ln_beta, self.eps)
-    u, q, k, v = self._project(x, (T,)).unbind(dim=1)
     alpha, n = self._alpha_n(max_len)
+    if self._fused_training(tokens, pos_bias, ts_bias):
+      return self._train_steps(tokens, (T,), pos_bias, ts_bias, batch,
+                               dict(seq_offsets=seq_offsets, max_len=max_len, n=n, alpha=alpha, timestamps=timestamps, **drop))
+    fused = self._fused_inference(tokens, pos_bias, ts_bias)
+    u, q, k, v = self._project(self._input_norm(tokens, fused), (T,), fused).unbind(dim=1)
     attn = _attention(q, k, v, seq_offsets=seq_offsets, max_len=max_len, n=n, alpha=alpha,
                       pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch, **drop)
-    return self._gate_and_output(attn.reshape(T, H * hd), u.reshape(T, H * hd), tokens)
+    return self._gate_and_output(attn.reshape(T, H * hd), u.reshape(T, H * hd), tokens, fused)
 
 
 class HSTU(torch.nn.Module):
@@ -263,25 +359,39 @@ class HSTU(torch.nn.Module):
 
   def _final_norm(self, x):
     out = _native.final_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps, None, None, 0, 0, True)
-    return F.layer_norm(x, (self.model_dim,), self.final_norm_gamma, self.final_norm_beta, self.eps) if out is None else out
+    if out is not None:
+      return out
+    D = self.model_dim
+    training = _wants_grad(x, self.final_norm_gamma, self.final_norm_beta)
+    if x.is_cuda and x.dtype == torch.bfloat16 and D % 8 == 0 and D <= (2048 if training else 8192):
+      return hstu_block_ops.layer_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps)
+    return F.layer_norm(x, (D,), self.final_norm_gamma, self.final_norm_beta, self.eps)
 
   def _front_end(self, ids, row_map=None, tokens=0):
     """Gather, scale, position embedding and final_norm (hstu.py:593-601): in bf16 on a GPU one pass, and one each for the
     gradients of the norm and of the tables.  ids [B, L]; the packed form with `row_map` (its `tokens` first entries).
     Returns the rows and, with gradients, a ticket for _check_indices."""
     table, positions = self.item_embedding, self.position_embedding
-    scale = self.model_dim ** 0.5 if self.scale_by_sqrt_dim else 1.0
+    scale, length = self.model_dim ** 0.5 if self.scale_by_sqrt_dim else 1.0, ids.shape[1]
     got = _native.embed(ids if ids.dtype == torch.int64 and ids.is_contiguous() else ids.to(torch.int64).contiguous(), table, positions,
                       self.final_norm_gamma, self.final_norm_beta, self.eps, scale, row_map, tokens, True)
     x, ticket = (None, None) if got is None else got
     if x is None:
       where = None if row_map is None else row_map[:tokens].to(torch.int64)
-      x = table[ids if where is None else ids.reshape(-1)[where]]
-      if self.scale_by_sqrt_dim:
-        x = x * scale
-      if positions is not None:
-        x = x + (positions[: ids.shape[1]] if where is None else positions[where % ids.shape[1]])
-      x = self._final_norm(x)
+      ids = ids if where is None else ids.reshape(-1)[where]
+      if table.is_cuda and table.dtype == torch.bfloat16 and not _wants_grad(table, positions, self.final_norm_gamma, self.final_norm_beta):
+        at = None
+        if positions is not None:
+          at = torch.arange(length, device=ids.device).expand(ids.shape).contiguous() if where is None else where % length
+        x = hstu_block_ops.embed_norm(ids.to(torch.int64), table, self.final_norm_gamma, self.final_norm_beta, self.eps, scale=scale,
+                                      positions=at, pos_table=positions)
+      else:
+        x = table[ids]
+        if self.scale_by_sqrt_dim:
+          x = x * scale
+        if positions is not None:
+          x = x + (positions[:length] if where is None else positions[where % length])
+        x = self._final_norm(x)
     return (F.dropout(x, self.dropout, self.training) if self.training and self.dropout > 0.0 else x), ticket
 
   def _check_indices(self, ticket):

@@ -42,3 +42,51 @@ def test_a_dense_mask_stands_alone(gpu):
   trained = blk(x, attention_mask=mask, **more)
   # (bf16 on both sides, rounded at different steps: 2^-8 each)
   assert (trained.detach() - want).float().norm() <= 2e-2 * want.float().norm()
+
+
+def _off_native(kind):
+  """A block that the native call does not take, and its inputs' width."""
+  if kind == "head dim 4":
+    return _block(40, 10), 40
+  blk = _block()
+  if kind == "weights laid out across":
+    blk.u_kernel.data = blk.u_kernel.data.permute(2, 1, 0).contiguous().permute(2, 1, 0)
+  else:
+    flat = torch.zeros(D + 1, dtype=BF, device=DEV)
+    flat[1:] = 1.0
+    blk.input_ln_gamma.data, blk.attn_ln_gamma.data = flat[1:], flat[1:].view(H, HD)
+  return blk, D
+
+
+@pytest.mark.parametrize("kind", ["head dim 4", "weights laid out across", "norm scales off a 16-byte boundary"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_blocks_beside_the_native_call_keep_the_fused_steps(gpu, monkeypatch, kind, packed):
+  """In bf16 the norm and the gate are one pass with one rounding, with and without gradients, also where the native call does not
+  apply; against torch's steps, which round the normed rows by themselves (2^-8 apart per step)."""
+  blk, width = _off_native(kind)
+  x, lens, *_ = _inputs(width)
+  valid = torch.arange(L, device=DEV)[None] < lens[:, None]
+  offsets = torch.tensor(np.concatenate([[0], np.cumsum(lens.cpu().numpy())]), dtype=torch.int32, device=DEV)
+  if packed:
+    x = x[valid].contiguous()
+  call = lambda t: blk.forward_jagged(t, offsets, L) if packed else blk(t, seq_lens=lens)
+  norms, gates = [], []
+  fwd, bwd = hstu_block_ops._norm_gate_fwd, hstu_block_ops.norm_gate_bwd
+  monkeypatch.setattr(hstu_block_ops, "_norm_gate_fwd", lambda *a: norms.append(a[1] is not None) or fwd(*a))
+  monkeypatch.setattr(hstu_block_ops, "norm_gate_bwd", lambda *a, **k: gates.append(a[1] is not None) or bwd(*a, **k))
+  scored = call(x)
+  assert norms == [False, True]                       # the input norm, then the attention norm with the gate
+  blk.requires_grad_(True)
+  dout = torch.randn(x.shape, generator=torch.Generator().manual_seed(9)).to(DEV).to(BF)
+  wrt = [x.requires_grad_(True), *blk.parameters()]
+  trained = call(x)
+  got = torch.autograd.grad(trained, wrt, dout)
+  assert norms == [False, True] * 2 and gates == [True, False]
+  blk._fused_training = lambda *a: False
+  plain = call(x)
+  want = torch.autograd.grad(plain, wrt, dout)
+  assert len(norms) == 4
+  close = lambda a, b, tol: (a.float() - b.float()).norm() <= tol * b.float().norm()
+  assert close(scored, plain.detach(), 1e-2) and close(trained.detach(), plain.detach(), 1e-2)
+  for g, w, name in zip(got, want, ["x", *dict(blk.named_parameters())]):
+    assert close(g, w, 3e-2), name
