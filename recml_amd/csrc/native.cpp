@@ -1060,15 +1060,18 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
     Tensor out, normed, pre, uqkv, attn, gated;
     const bool ok = without_lock(tokens, [&] {
       const int64_t T = c.T, D = c.D, W = c.H * c.hd;
+      uqkv = fresh(tokens, {T, 4, c.H, c.hd});
+      if (c.L) attn = fresh(tokens, {c.B, c.L, c.H, c.hd});
+      else attn = fresh(tokens, {T, c.H, c.hd});
+      // (a call whose attention the Python side has to take is found here, before any of its work)
+      HstuAttnFwdArgs probe;
+      if (!fill(probe, projection_slice(uqkv, c, 1), projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
       normed = fresh(tokens, {T, D});
       norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
-      uqkv = fresh(tokens, {T, 4, c.H, c.hd});
       if (graph) pre = at::empty_like(uqkv);
       Tensor pb;
       if (p[P_UB].defined()) pb = at::cat({p[P_UB].view({W}), p[P_QB].view({W}), p[P_KB].view({W}), p[P_VB].view({W})});
       gemm(HSTU_GEMM_NN, T, {normed.const_data_ptr(), D}, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W, uqkv, pb, {nullptr, 0}, true, pre);
-      if (c.L) attn = fresh(tokens, {c.B, c.L, c.H, c.hd});
-      else attn = fresh(tokens, {T, c.H, c.hd});
       if (!forward_into(attn, projection_slice(uqkv, c, 1), projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), pos, ts_tab, bias, o,
                         share ? &shared : nullptr)) return false;
       gated = fresh(tokens, {T, W});

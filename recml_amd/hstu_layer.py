@@ -42,6 +42,11 @@ def _wants_grad(*tensors) -> bool:
   return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
 
 
+def _ready(t, dtype):
+  """A lengths, timestamps or table tensor as the kernels read it."""
+  return t if not isinstance(t, torch.Tensor) or (t.dtype == dtype and t.is_contiguous()) else t.to(dtype).contiguous()
+
+
 def _attention(q, k, v, *, pos_bias=None, ts_bias=None, batch=None, **kw):
   """The attention op, differentiable when anything it reads wants a gradient: through the HIP
   backward kernels for q, k, v, the bias tables and a dense bias.  `batch`: the per-batch preparation
@@ -284,6 +289,11 @@ class HSTUBlock(torch.nn.Module):
     grad = self._wants_grad(tokens, pos_bias, ts_bias, attention_bias)
     if grad and not self._fused_training(tokens, pos_bias, ts_bias):
       return None
+    # (torch's default integers, 16-bit tables: converted here, by the first block of a batch for all of them; a table's conversion is
+    # part of the graph)
+    ready = _ready if batch is None else batch.ready
+    seq_lens, seq_offsets, timestamps = ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64)
+    pos_bias, ts_bias = (_ready(t, torch.float32) if grad else ready(t, torch.float32) for t in (pos_bias, ts_bias))
     P = self._parameters
     params = (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], P.get("u_bias"), P.get("q_bias"),
               P.get("k_bias"), P.get("v_bias"), P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], P.get("output_bias"))

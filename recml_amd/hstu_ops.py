@@ -128,6 +128,7 @@ class AttentionBatch:
     self._prepared = None     # signature the workspace was prepared for
     self._pending = None
     self._tensors = ()        # keeps the signature's tensors alive (their addresses are part of it)
+    self._converted = []      # [what a tensor was, the tensor, it as the kernels read it]: tensors of other types than theirs
     self.prepared_calls = 0   # calls that skipped the preparation
 
   @staticmethod
@@ -139,6 +140,18 @@ class AttentionBatch:
     # (tensors made under torch.inference_mode() carry no version counter, and reading it raises)
     version = -1 if t.is_inference() else t._version
     return (t.data_ptr(), version, tuple(t.shape), tuple(t.stride()), t.dtype)
+
+  def ready(self, t, dtype):
+    """`t` as a contiguous tensor of `dtype`: itself, or a copy that later calls with the same tensor, unmodified, share."""
+    if not isinstance(t, torch.Tensor) or (t.dtype == dtype and t.is_contiguous()):
+      return t
+    was = (self._ident(t), dtype)
+    for known, _, copy in self._converted:
+      if known == was:
+        return copy
+    copy = t.detach().to(dtype).contiguous()
+    self._converted = self._converted[-7:] + [(was, t, copy)]
+    return copy
 
   def _attach(self, args, keep, sig, tensors):
     ws = _lib.load().hstu_attn_fwd_workspace_bytes(C.byref(args))

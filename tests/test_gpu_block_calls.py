@@ -90,3 +90,61 @@ def test_blocks_beside_the_native_call_keep_the_fused_steps(gpu, monkeypatch, ki
   assert close(scored, plain.detach(), 1e-2) and close(trained.detach(), plain.detach(), 1e-2)
   for g, w, name in zip(got, want, ["x", *dict(blk.named_parameters())]):
     assert close(g, w, 3e-2), name
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("grad", [False, True])
+def test_other_integer_and_table_types_take_the_native_call(gpu, monkeypatch, packed, grad):
+  """torch's default integers for lengths and offsets, 32-bit timestamps, a bf16 table, one whose rows are strided: the same bits as with
+  the kernels' own types, through the native call, and table gradients in the tables' own types."""
+  blk = _block().requires_grad_(grad)
+  x, lens, pos, ts, tsb = _inputs()
+  pos16 = pos.to(BF)
+  wide = torch.zeros((H, 2 * 129), device=DEV)
+  wide[:, ::2] = tsb
+  ts = ts - ts.min()
+  offsets = torch.tensor(np.concatenate([[0], np.cumsum(lens.cpu().numpy())]), dtype=torch.int32, device=DEV)
+  if packed:
+    valid = torch.arange(L, device=DEV)[None] < lens[:, None]
+    x, ts = x[valid].contiguous(), ts[valid].contiguous()
+  call = lambda lens, offsets, **kw: blk.forward_jagged(x, offsets, L, **kw) if packed else blk(x, seq_lens=lens, **kw)
+  seen = []
+  native = recml_amd._native.block
+  monkeypatch.setattr(recml_amd._native, "block", lambda *a: (seen.append(native(*a)), seen[-1])[1])
+  plain = [t.requires_grad_(grad) for t in (pos16.float(), tsb.clone())]
+  given = [t.requires_grad_(grad) for t in (pos16, wide[:, ::2])]
+  want = call(lens, offsets, pos_bias=plain[0], timestamps=ts, ts_bias=plain[1])
+  got = call(lens.long(), offsets.long(), pos_bias=given[0], timestamps=ts.int(), ts_bias=given[1])
+  assert len(seen) == 2 and all(s is not None for s in seen)
+  assert torch.equal(got, want)
+  if grad:
+    dout = torch.randn(x.shape, generator=torch.Generator().manual_seed(9)).to(DEV).to(BF)
+    params = list(blk.parameters())
+    a, b = torch.autograd.grad(got, [*given, *params], dout), torch.autograd.grad(want, [*plain, *params], dout)
+    assert a[0].dtype == BF
+    # (the tables' sums are added to by atomics, in no fixed order)
+    assert (a[0].float() - b[0]).abs().max() <= 2.0 ** -8 * b[0].abs().max() and (a[1] - b[1]).abs().max() <= 1e-5 * b[1].abs().max()
+    assert all(torch.equal(p, q) for p, q in zip(a[2:], b[2:]))
+
+
+def test_converted_lengths_are_shared_and_not_outlived(gpu, monkeypatch):
+  """The blocks of a model share one preparation from 64-bit lengths too, and lengths changed in place are seen."""
+  from recml_amd import hstu_ops
+  made = []
+
+  class Batch(hstu_ops.AttentionBatch):
+    def __init__(self):
+      super().__init__()
+      made.append(self)
+
+  monkeypatch.setattr(hstu_ops, "AttentionBatch", Batch)
+  model = recml_amd.HSTU(vocab_size=50, max_positions=L, model_dim=D, num_heads=H, num_layers=3, dtype=BF, device=DEV, add_head=False, seed=1)
+  ids = torch.randint(1, 50, (B, L), generator=torch.Generator().manual_seed(4)).to(DEV)
+  lens, pos = _inputs()[1:3]
+  assert torch.equal(model(ids, seq_lens=lens.long(), pos_bias=pos), model(ids, seq_lens=lens, pos_bias=pos))
+  assert [b.prepared_calls for b in made] == [2, 2]
+  blk, batch, wide = _block(), hstu_ops.AttentionBatch(), lens.long()
+  x = _inputs()[0]
+  blk(x, seq_lens=wide, pos_bias=pos, batch=batch)
+  wide.fill_(30)
+  assert torch.equal(blk(x, seq_lens=wide, pos_bias=pos, batch=batch), blk(x, seq_lens=torch.full_like(lens, 30), pos_bias=pos))
