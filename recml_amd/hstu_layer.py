@@ -254,8 +254,17 @@ class HSTUBlock(torch.nn.Module):
       out = out + self.output_bias
     return out + residual
 
+  def _weights(self):
+    """The block's parameters as the native call takes them: whatever stands under their names (a parametrization or a pruning mask
+    puts a tensor of its own there)."""
+    P = self._parameters
+    of = lambda name: P[name] if name in P else getattr(self, name)
+    biases = (of("u_bias"), of("q_bias"), of("k_bias"), of("v_bias")) if self.use_bias else (None,) * 4
+    return (of("input_ln_gamma"), of("input_ln_beta"), of("u_kernel"), of("q_kernel"), of("k_kernel"), of("v_kernel"), *biases,
+            of("attn_ln_gamma"), of("attn_ln_beta"), of("output_kernel"), of("output_bias") if self.use_bias else None)
+
   def _wants_grad(self, *tensors) -> bool:
-    return torch.is_grad_enabled() and (any(p is not None and p.requires_grad for p in self._parameters.values()) or _wants_grad(*tensors))
+    return torch.is_grad_enabled() and _wants_grad(*self._weights(), *tensors)
 
   def _fused_inference(self, t, *bias_inputs) -> bool:
     """Whether the steps of hstu_block_ops apply where the native call does not: bf16 on a GPU, nothing asking for gradients, widths
@@ -286,7 +295,8 @@ class HSTUBlock(torch.nn.Module):
     GPU, parameters ready as they are.  None where it does not apply: fp32, a dense mask or bias with gradients, ..."""
     if tokens.dtype != torch.bfloat16 or not tokens.is_cuda:
       return None
-    grad = self._wants_grad(tokens, pos_bias, ts_bias, attention_bias)
+    weights = self._weights()
+    grad = _wants_grad(tokens, *weights, pos_bias, ts_bias, attention_bias)
     if grad and not self._fused_training(tokens, pos_bias, ts_bias):
       return None
     # (torch's default integers, 16-bit tables: converted here, by the first block of a batch for all of them; a table's conversion is
@@ -294,11 +304,8 @@ class HSTUBlock(torch.nn.Module):
     ready = _ready if batch is None else batch.ready
     seq_lens, seq_offsets, timestamps = ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64)
     pos_bias, ts_bias = (_ready(t, torch.float32) if grad else ready(t, torch.float32) for t in (pos_bias, ts_bias))
-    P = self._parameters
-    params = (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], P.get("u_bias"), P.get("q_bias"),
-              P.get("k_bias"), P.get("v_bias"), P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], P.get("output_bias"))
     alpha, n = self._alpha_n(length)
-    got = _native.block(tokens.contiguous(), params, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
+    got = _native.block(tokens.contiguous(), weights, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
                         None if seq_offsets is None else length, pos_bias, timestamps, ts_bias, attention_mask, attention_bias,
                         drop.get("dropout_p", 0.0), drop.get("dropout_seed", 0),
                         False if batch is None else batch._prepared, None if batch is None else batch._buf, grad)

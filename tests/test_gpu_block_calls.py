@@ -4,6 +4,8 @@ what is computed, whatever the types and layouts of lengths, tables and paramete
 import numpy as np
 import pytest
 import torch
+import torch.nn.utils.parametrize
+import torch.nn.utils.prune
 
 import recml_amd
 from recml_amd import hstu_block_ops
@@ -148,3 +150,40 @@ def test_converted_lengths_are_shared_and_not_outlived(gpu, monkeypatch):
   blk(x, seq_lens=wide, pos_bias=pos, batch=batch)
   wide.fill_(30)
   assert torch.equal(blk(x, seq_lens=wide, pos_bias=pos, batch=batch), blk(x, seq_lens=torch.full_like(lens, 30), pos_bias=pos))
+
+
+class _Doubled(torch.nn.Module):
+  def forward(self, w):
+    return 2.0 * w
+
+
+@pytest.mark.parametrize("how", ["parametrize", "prune", "prune a bias"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_parametrized_and_pruned_blocks(gpu, how, packed):
+  """torch.nn.utils.parametrize and prune take a parameter's name out of the module's parameters and put a tensor there: the same as a
+  block with that tensor, and the gradient reaches the parameter behind it."""
+  x, lens, *_ = _inputs()
+  offsets = torch.tensor([0, L, L + 41, L + 42], dtype=torch.int32, device=DEV)
+  call = lambda blk: blk.forward_jagged(x[:, 0].repeat(50, 1)[: L + 42].contiguous(), offsets, L) if packed else blk(x, seq_lens=lens)
+  blk, plain = _block(use_bias=True), _block(use_bias=True)
+  for b in (blk, plain):
+    b.requires_grad_(True)
+    b.q_bias.data += 0.25
+  if how == "parametrize":
+    torch.nn.utils.parametrize.register_parametrization(blk, "u_kernel", _Doubled(), unsafe=True)
+    behind, shown = blk.parametrizations.u_kernel.original, plain.u_kernel
+    shown.data *= 2.0
+    factor = torch.full_like(shown, 2.0)
+  else:
+    name = "output_kernel" if how == "prune" else "q_bias"
+    factor = (torch.rand(getattr(blk, name).shape, generator=torch.Generator().manual_seed(1)) < 0.5).to(DEV).to(BF)
+    torch.nn.utils.prune.custom_from_mask(blk, name, factor)
+    behind, shown = getattr(blk, name + "_orig"), getattr(plain, name)
+    shown.data *= factor
+  got, want = call(blk), call(plain)
+  assert torch.equal(got, want)
+  dout = torch.randn(got.shape, generator=torch.Generator().manual_seed(9)).to(DEV).to(BF)
+  a, b = torch.autograd.grad(got, behind, dout)[0], torch.autograd.grad(want, shown, dout)[0]
+  assert torch.equal(a, b * factor)
+  with torch.no_grad():
+    assert torch.equal(call(blk), call(plain))
