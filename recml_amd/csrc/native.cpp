@@ -15,6 +15,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <hip/hip_runtime.h>
 #include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/edge.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -924,6 +925,14 @@ struct LinearBackward : public torch::autograd::Node {
 // Python
 // ---------------------------------------------------------------------------
 
+// Runs `f`; an exception becomes the Python one of its type (torch.OutOfMemoryError, IndexError, an error of a hook, ...).
+template <typename F>
+PyObject* guarded(F&& f) {
+  HANDLE_TH_ERRORS
+  return f();
+  END_HANDLE_TH_ERRORS
+}
+
 enum Arg { A_Q, A_K, A_V, A_SEQ_LENS, A_SEQ_OFFSETS, A_MAX_LEN, A_N, A_ALPHA, A_CAUSAL, A_POS, A_TS, A_TS_TAB, A_BUCKET, A_QSEG, A_KVSEG, A_WINDOW,
            A_MASK, A_BIAS, A_OUT, A_QSCALE, A_KSCALE, A_DROP_P, A_DROP_SEED, A_GRAD, A_COUNT };
 
@@ -934,7 +943,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count) {
     PyErr_Format(PyExc_TypeError, "attention takes %d arguments, got %zd", (int)A_COUNT, count);
     return nullptr;
   }
-  try {
+  return guarded([&]() -> PyObject* {
     Tensor q, k, v, pos, ts_tab, bias, out;
     Options o;
     for (int i : {A_Q, A_K, A_V})
@@ -989,10 +998,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count) {
       torch::autograd::set_history(out, node);
     }
     return THPVariable_Wrap(std::move(out));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
+  });
 }
 
 // Runs `f` without the interpreter's lock, on the tensor's device, outside of any graph.
@@ -1007,15 +1013,6 @@ auto without_lock(const Tensor& t, F&& f) {
   return f();
 }
 
-template <typename F>
-PyObject* guarded(F&& f) {
-  try {
-    return f();
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
-}
 
 // block(tokens [.., D], params, heads, head_dim, eps, alpha, n, seq_lens, seq_offsets, max_len, pos, timestamps, ts_tab, mask, bias,
 //       dropout_p, dropout_seed, prepared, workspace, differentiable) -> (out, signature, workspace, reused) or None
