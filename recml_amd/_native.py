@@ -9,9 +9,18 @@ from __future__ import annotations
 import importlib.util
 import os
 
+import torch
+from torch.autograd import forward_ad
+
 from recml_amd import _lib, _lib_block
 
 PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_native.so")
+
+
+def has_tangent(*tensors) -> bool:
+  """Whether one of the tensors carries a forward-mode tangent: the kernels' results have none, so such a call goes through the
+  autograd functions, which refuse it."""
+  return any(isinstance(t, torch.Tensor) and forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 def _load():

@@ -482,6 +482,14 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
   return false;
 }
 
+// Whether a tensor carries a forward-mode tangent.  The kernels give none for their results: such a call goes the Python way, whose
+// torch steps carry tangents on and whose autograd functions refuse them.
+bool dual(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->defined() && t->_fw_grad(0).defined()) return true;
+  return false;
+}
+
 // ---------------------------------------------------------------------------
 // block steps
 // ---------------------------------------------------------------------------
@@ -903,11 +911,11 @@ struct LinearBackward : public torch::autograd::Node {
 
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    const at::NoGradGuard no_grad;
     torch::autograd::variable_list r(2);
     if (!grads[0].defined()) return r;
     const Tensor a = x.unpack(), b = w.unpack();
     const c10::DeviceGuard guard(a.device());
+    const at::NoGradGuard no_grad;
     const int64_t K = b.size(0), N = b.size(1), M = a.numel() / K;
     Tensor d = grads[0].contiguous().view({M, N});
     if (!aligned(d)) d = d.clone();
@@ -966,6 +974,7 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (causal < 0) return nullptr;
     o.causal = causal != 0;
     const bool graph = args[A_GRAD] == Py_True && wants_grad({&q, &k, &v, &pos, &ts_tab, &bias});
+    if (args[A_GRAD] == Py_True && dual({&q, &k, &v, &pos, &ts_tab, &bias})) Py_RETURN_NONE;
     if (!q.is_cuda() || q.dim() < 1 || v.dim() != q.dim() || (graph && (out.defined() || q.scalar_type() == at::kFloat8_e4m3fn))) Py_RETURN_NONE;
     bool ok;
     {
@@ -1054,6 +1063,9 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
       return any;
     }();
     if ((graph && (o.mask.defined() || bias.defined())) || !block_ready(tokens, p, c, graph)) Py_RETURN_NONE;
+    for (const Tensor& t : p)
+      if (dual({&t})) Py_RETURN_NONE;
+    if (dual({&tokens, &pos, &ts_tab, &bias})) Py_RETURN_NONE;
     Tensor out, normed, pre, uqkv, attn, gated;
     const bool ok = without_lock(tokens, [&] {
       const int64_t T = c.T, D = c.D, W = c.H * c.hd;
@@ -1214,7 +1226,7 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     Tensor table, pos_table, gamma, beta;
     if (!tensor_arg(a[0], &c.ids) || !tensor_arg(a[1], &table) || !tensor_arg(a[2], &pos_table) || !tensor_arg(a[3], &gamma) || !tensor_arg(a[4], &beta) ||
         !float_arg(a[5], &c.eps) || !float_arg(a[6], &c.scale) || !tensor_arg(a[7], &c.row_map) || !long_arg(a[8], &c.T)) Py_RETURN_NONE;
-    if (!c.ids.defined() || !table.defined() || !table.is_cuda()) Py_RETURN_NONE;
+    if (!c.ids.defined() || !table.defined() || !table.is_cuda() || dual({&table, &pos_table, &gamma, &beta})) Py_RETURN_NONE;
     const auto dev = table.device();
     if (!plain(c.ids, dev, at::kLong) || c.ids.dim() != 2 || !ready(table, dev) || table.dim() != 2 || !ready(gamma, dev) || !ready(beta, dev) ||
         (pos_table.defined() && (!ready(pos_table, dev) || pos_table.dim() != 2 || pos_table.size(1) != table.size(1)))) Py_RETURN_NONE;
@@ -1284,7 +1296,7 @@ PyObject* final_norm(PyObject*, PyObject* const* a, Py_ssize_t count) {
     int64_t B, L;
     if (!tensor_arg(a[0], &x) || !tensor_arg(a[1], &gamma) || !tensor_arg(a[2], &beta) || !float_arg(a[3], &eps) || !tensor_arg(a[4], &seq_offsets) ||
         !tensor_arg(a[5], &row_map) || !long_arg(a[6], &B) || !long_arg(a[7], &L)) Py_RETURN_NONE;
-    if (!x.defined() || !x.is_cuda() || x.dim() < 2) Py_RETURN_NONE;
+    if (!x.defined() || !x.is_cuda() || x.dim() < 2 || dual({&x, &gamma, &beta})) Py_RETURN_NONE;
     const auto dev = x.device();
     const int64_t D = x.size(-1), rows = x.numel() / (D ? D : 1);
     const bool graph = a[8] == Py_True && wants_grad({&x, &gamma, &beta});
@@ -1320,7 +1332,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t count) {
   }
   return guarded([&]() -> PyObject* {
     Tensor x, w;
-    if (!tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) || !x.defined() || !w.defined() || !x.is_cuda() || x.dim() < 2 || w.dim() != 2) Py_RETURN_NONE;
+    if (!tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) || !x.defined() || !w.defined() || !x.is_cuda() || x.dim() < 2 || w.dim() != 2 ||
+        dual({&x, &w})) Py_RETURN_NONE;
     const auto dev = x.device();
     const int64_t K = w.size(0), N = w.size(1), M = x.numel() / (K ? K : 1);
     if (!ready(x, dev) || !ready(w, dev) || x.size(-1) != K || K % 8 || N % 8 || K < 8 || N < 8 || M < 1 || M > (1 << 30) || N > (1 << 30)) Py_RETURN_NONE;

@@ -165,7 +165,7 @@ def norm_gate(attn, u, gamma, beta, eps: float = 1e-6):
   and whose leading axes collapse to one row stride (a slice of a fused projection does);
   gamma, beta: [W].  Differentiable in all four (W up to 2048 then: wider rows with a gradient wanted
   raise here, not at backward time)."""
-  if _wants_grad(attn, u, gamma, beta):
+  if _wants_grad(attn, u, gamma, beta) or _native.has_tangent(attn, u, gamma, beta):
     _check_grad_width(attn.shape[-1])
     return _NormGateFn.apply(attn, u, gamma, beta, eps)
   return _norm_gate_fwd(attn, u, gamma, beta, eps)
@@ -174,7 +174,7 @@ def norm_gate(attn, u, gamma, beta, eps: float = 1e-6):
 def layer_norm(x, gamma, beta, eps: float = 1e-6):
   """layer_norm(x) over the last axis (keras LayerNormalization as the block's input norm uses it,
   recml/layers/keras/hstu.py:442): the same kernels without the gate.  Differentiable in x, gamma, beta."""
-  if _wants_grad(x, gamma, beta):
+  if _wants_grad(x, gamma, beta) or _native.has_tangent(x, gamma, beta):
     _check_grad_width(x.shape[-1])
     return _NormGateFn.apply(x, None, gamma, beta, eps)
   return _norm_gate_fwd(x, None, gamma, beta, eps)

@@ -42,6 +42,11 @@ def _wants_grad(*tensors) -> bool:
   return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
 
 
+def _differentiates(*tensors) -> bool:
+  """Whether a gradient is asked for in either mode."""
+  return _wants_grad(*tensors) or _native.has_tangent(*tensors)
+
+
 def _ready(t, dtype):
   """A lengths, timestamps or table tensor as the kernels read it."""
   return t if not isinstance(t, torch.Tensor) or (t.dtype == dtype and t.is_contiguous()) else t.to(dtype).contiguous()
@@ -51,7 +56,7 @@ def _attention(q, k, v, *, pos_bias=None, ts_bias=None, batch=None, **kw):
   """The attention op, differentiable when anything it reads wants a gradient: through the HIP
   backward kernels for q, k, v, the bias tables and a dense bias.  `batch`: the per-batch preparation
   shared by the layers (inference only)."""
-  if _wants_grad(q, k, v, pos_bias, ts_bias, kw.get("bias")):
+  if _differentiates(q, k, v, pos_bias, ts_bias, kw.get("bias")):
     return hstu_ops.hstu_attention_autograd(q, k, v, pos_bias=pos_bias, ts_bias=ts_bias, **kw)
   return hstu_ops.hstu_attention(q, k, v, pos_bias=pos_bias, ts_bias=ts_bias, batch=batch, **kw)
 
@@ -264,7 +269,7 @@ class HSTUBlock(torch.nn.Module):
             of("attn_ln_gamma"), of("attn_ln_beta"), of("output_kernel"), of("output_bias") if self.use_bias else None)
 
   def _wants_grad(self, *tensors) -> bool:
-    return torch.is_grad_enabled() and _wants_grad(*self._weights(), *tensors)
+    return _differentiates(*self._weights(), *tensors)
 
   def _fused_inference(self, t, *bias_inputs) -> bool:
     """Whether the steps of hstu_block_ops apply where the native call does not: bf16 on a GPU, nothing asking for gradients, widths
@@ -379,7 +384,7 @@ class HSTU(torch.nn.Module):
     if out is not None:
       return out
     D = self.model_dim
-    training = _wants_grad(x, self.final_norm_gamma, self.final_norm_beta)
+    training = _differentiates(x, self.final_norm_gamma, self.final_norm_beta)
     if x.is_cuda and x.dtype == torch.bfloat16 and D % 8 == 0 and D <= (2048 if training else 8192):
       return hstu_block_ops.layer_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps)
     return F.layer_norm(x, (D,), self.final_norm_gamma, self.final_norm_beta, self.eps)
@@ -396,7 +401,8 @@ class HSTU(torch.nn.Module):
     if x is None:
       where = None if row_map is None else row_map[:tokens].to(torch.int64)
       ids = ids if where is None else ids.reshape(-1)[where]
-      if table.is_cuda and table.dtype == torch.bfloat16 and not _wants_grad(table, positions, self.final_norm_gamma, self.final_norm_beta):
+      if table.is_cuda and table.dtype == torch.bfloat16 and not _differentiates(table, positions, self.final_norm_gamma,
+                                                                                              self.final_norm_beta):
         at = None
         if positions is not None:
           at = torch.arange(length, device=ids.device).expand(ids.shape).contiguous() if where is None else where % length

@@ -39,3 +39,30 @@ def test_out_of_memory_keeps_its_type(little_memory, grad):
   x = torch.zeros((1, 1 << 16, 128), dtype=BF, device=DEV)
   with pytest.raises(torch.OutOfMemoryError):
     blk(x, seq_lens=torch.tensor([5], dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_forward_mode_is_refused_not_dropped(gpu, grad):
+  """The kernels give no tangents: a dual tensor anywhere in a differentiable call is refused, as torch's autograd functions refuse it."""
+  lens = torch.tensor([40, 7], dtype=torch.int32, device=DEV)
+  q = _randn(2, 40, 2, 64)
+  pos = _randn(2, 79, std=0.1, dtype=torch.float32)
+  blk = _block().requires_grad_(grad)
+  x = _randn(2, 40, 128)
+  gamma, beta = torch.ones(128, dtype=BF, device=DEV), torch.zeros(128, dtype=BF, device=DEV)
+  model = recml_amd.HSTU(vocab_size=50, max_positions=40, model_dim=128, num_heads=2, num_layers=1, dtype=BF, device=DEV, seed=1, add_head=False)
+  model.requires_grad_(grad)
+  ids = torch.randint(1, 50, (2, 40), generator=torch.Generator().manual_seed(4)).to(DEV)
+  with torch.autograd.forward_ad.dual_level():
+    dual = lambda t: torch.autograd.forward_ad.make_dual(t.detach(), torch.ones_like(t))
+    calls = [lambda: recml_amd.hstu_attention_autograd(dual(q), q, q, seq_lens=lens),
+             lambda: recml_amd.hstu_attention_autograd(q, q, q, seq_lens=lens, pos_bias=dual(pos)),
+             lambda: blk(dual(x), seq_lens=lens), lambda: blk(x, seq_lens=lens, pos_bias=dual(pos)),
+             lambda: blk.forward_jagged(dual(x[0]), torch.tensor([0, 40], dtype=torch.int32, device=DEV), 40),
+             lambda: recml_amd.layer_norm(dual(x), gamma, beta), lambda: recml_amd.norm_gate(x, x, dual(gamma), beta),
+             lambda: model(ids, seq_lens=lens, pos_bias=dual(pos[0]))]
+    for i, call in enumerate(calls):
+      with pytest.raises(NotImplementedError):
+        call()
+        pytest.fail(f"call {i} took a dual tensor")
+
