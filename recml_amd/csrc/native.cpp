@@ -897,7 +897,7 @@ struct FinalNormBackward : public torch::autograd::Node {
   }
 };
 
-// x [M, K] w [K, N] with gradients.
+// x [M, K] w [K, N] with gradients, and theirs where they are asked for (create_graph: torch's products then).
 struct LinearBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable x, w;
 
@@ -915,6 +915,11 @@ struct LinearBackward : public torch::autograd::Node {
     if (!grads[0].defined()) return r;
     const Tensor a = x.unpack(), b = w.unpack();
     const c10::DeviceGuard guard(a.device());
+    if (at::GradMode::is_enabled()) {
+      if (task_should_compute_output(0)) r[0] = at::matmul(grads[0], b.t());
+      if (task_should_compute_output(1)) r[1] = at::matmul(a.flatten(0, -2).t(), grads[0].flatten(0, -2));
+      return r;
+    }
     const at::NoGradGuard no_grad;
     const int64_t K = b.size(0), N = b.size(1), M = a.numel() / K;
     Tensor d = grads[0].contiguous().view({M, N});

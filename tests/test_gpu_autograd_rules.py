@@ -66,3 +66,20 @@ def test_forward_mode_is_refused_not_dropped(gpu, grad):
         call()
         pytest.fail(f"call {i} took a dual tensor")
 
+
+def test_the_head_carries_tangents_and_second_derivatives(gpu):
+  """The output head stands for x @ w, which has both.  bf16 products of 64 and 96 terms, rounded once on either side: 2^-8."""
+  model = recml_amd.HSTU(vocab_size=96, max_positions=8, model_dim=64, num_heads=1, num_layers=0, dtype=BF, device=DEV, seed=1)
+  model.requires_grad_(True)
+  x, t, v, u = _randn(3, 8, 64, seed=1).requires_grad_(True), _randn(3, 8, 64, seed=2), _randn(3, 8, 96, seed=3), _randn(3, 8, 64, seed=4)
+  w = model.reverse_embedding
+  close = lambda a, b: (a.float() - b.float()).norm() <= 2.0 ** -8 * b.float().norm()
+  with torch.autograd.forward_ad.dual_level():
+    tangent = torch.autograd.forward_ad.unpack_dual(model._head(torch.autograd.forward_ad.make_dual(x.detach(), t))).tangent
+    assert tangent is not None and close(tangent, t.float() @ w.detach().float())
+  y = model._head(x)
+  gx, gw = torch.autograd.grad(y, [x, w], v, create_graph=True)
+  assert close(gx, v.float() @ w.detach().float().t())
+  got = torch.autograd.grad([gx, gw], [w, x], [u, torch.ones_like(gw)])
+  assert close(got[0], u.reshape(-1, 64).float().t() @ v.reshape(-1, 96).float())
+  assert close(got[1], v.float() @ torch.ones(96, 64, device=DEV))
