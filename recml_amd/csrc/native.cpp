@@ -213,8 +213,8 @@ bool fill(HstuAttnFwdArgs& a, const Tensor& q, const Tensor& k, const Tensor& v,
 }
 
 // Gives a dense mask or bias whose rows cannot be fetched 16 bytes at a time longer rows, where that is all that keeps the call
-// off the matrix-core kernels (B=16, L=1000, H=8, d=64 with gradients: 1.22 ms there, 0.38 on the matrix cores).  The copies stay
-// in `o`, for the backward.
+// off the matrix-core kernels (B=16, L=1000, H=8, d=64 with gradients: 1.22 ms there, 0.38 on the matrix cores).  The copies are
+// left in `o`, for the backward; copies found there are used.
 void pad_dense(HstuAttnFwdArgs& a, Options& o, const Tensor& like) {
   if ((!a.mask && !a.dense_bias) || a.qk_dtype != HSTU_DTYPE_BF16 || a.L != a.Lkv) return;
   auto on_mfma = [](const HstuAttnFwdArgs& x) { return !strcmp(hstu_attn_fwd_variant(&x), "hstu_fwd_mfma_bf16"); };
@@ -385,15 +385,15 @@ void gradient_buffers(const Tensor (&t)[3], Tensor (&g)[3]) {
 }
 
 struct AttentionBackward : public torch::autograd::Node {
-  torch::autograd::SavedVariable q, k, v, pos, ts_tab, bias;
+  torch::autograd::SavedVariable q, k, v, pos, ts_tab, bias, mask_rows, bias_rows;
   Options opts;
-  bool has_pos = false, has_ts = false, has_bias = false;
+  bool has_pos = false, has_ts = false, has_bias = false, has_mask_rows = false, has_bias_rows = false;
 
   std::string name() const override { return "HstuAttentionBackward"; }
 
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
-    for (auto* s : {&q, &k, &v, &pos, &ts_tab, &bias}) s->reset_data();
+    for (auto* s : {&q, &k, &v, &pos, &ts_tab, &bias, &mask_rows, &bias_rows}) s->reset_data();
     opts = Options();
   }
 
@@ -439,7 +439,10 @@ struct AttentionBackward : public torch::autograd::Node {
     // (the forward struct's `out` is not read by the backward, which takes dout's strides from it)
     TORCH_CHECK(dout.scalar_type() == t[2].scalar_type() && fill(b.fwd, t[0], t[1], t[2], dout, p, tt, bs, opts),
                 "the gradient of hstu_attention's result does not fit the call");
-    pad_dense(b.fwd, opts, t[0]);
+    Options rows = opts;
+    if (has_mask_rows) rows.mask_rows = mask_rows.unpack();
+    if (has_bias_rows) rows.bias_rows = bias_rows.unpack();
+    pad_dense(b.fwd, rows, t[0]);
     const Tensor scratch = scratch_for(b.fwd, t[0]);
     Tensor g[3];
     gradient_buffers(t, g);
@@ -663,10 +666,14 @@ struct NormOp {
   }
 };
 
+// A tensor kept for the backward, the forward's own intermediates included: this way torch's saved-tensor hooks see it (checkpointing
+// and offloading replace it).
+torch::autograd::SavedVariable keep(const Tensor& t) { return torch::autograd::SavedVariable(t, false); }
+
 struct BlockBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable tokens, params[P_COUNT], pos, ts_tab;
   bool has[P_COUNT] = {}, has_pos = false, has_ts = false;
-  Tensor normed, pre, uqkv, attn, gated;       // of the forward
+  torch::autograd::SavedVariable saved_normed, saved_pre, saved_uqkv, saved_attn, saved_gated;       // of the forward
   BlockCall call;
 
   std::string name() const override { return "HstuBlockBackward"; }
@@ -675,9 +682,7 @@ struct BlockBackward : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     tokens.reset_data();
     for (auto& p : params) p.reset_data();
-    pos.reset_data();
-    ts_tab.reset_data();
-    normed = pre = uqkv = attn = gated = Tensor();
+    for (auto* x : {&pos, &ts_tab, &saved_normed, &saved_pre, &saved_uqkv, &saved_attn, &saved_gated}) x->reset_data();
     call.opts = Options();
   }
 
@@ -687,8 +692,8 @@ struct BlockBackward : public torch::autograd::Node {
     const at::NoGradGuard no_grad;
     torch::autograd::variable_list r(1 + P_COUNT + 2);
     if (!grads[0].defined()) return r;
-    TORCH_CHECK(uqkv.defined(), "Trying to backward through the block a second time: its saved tensors are gone (pass retain_graph=True)");
-    const Tensor x = tokens.unpack();
+    const Tensor x = tokens.unpack(), normed = saved_normed.unpack(), pre = saved_pre.unpack(), uqkv = saved_uqkv.unpack(), attn = saved_attn.unpack(),
+                 gated = saved_gated.unpack();
     const c10::DeviceGuard guard(x.device());
     Tensor p[P_COUNT];
     for (int i = 0; i < P_COUNT; ++i)
@@ -817,8 +822,6 @@ Tensor table_gradient(const TableGradient& t, const Tensor& g, const Tensor& ids
   return out;
 }
 
-torch::autograd::SavedVariable keep(const Tensor& t) { return torch::autograd::SavedVariable(t, false); }
-
 // Works on the forward's own copies of the gathered rows and their keys: the caller's ids and tables may be refilled or updated
 // before it runs.
 struct EmbedBackward : public torch::autograd::Node {
@@ -861,16 +864,15 @@ struct EmbedBackward : public torch::autograd::Node {
 
 // The closing norm, from packed tokens to the padded batch (or rows to rows).
 struct FinalNormBackward : public torch::autograd::Node {
-  torch::autograd::SavedVariable x, gamma, beta;
-  Tensor row_map;
+  torch::autograd::SavedVariable x, gamma, beta, row_map;
+  bool packed = false;
   double eps = 0.0;
 
   std::string name() const override { return "HstuFinalNormBackward"; }
 
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
-    for (auto* s : {&x, &gamma, &beta}) s->reset_data();
-    row_map = Tensor();
+    for (auto* s : {&x, &gamma, &beta, &row_map}) s->reset_data();
   }
 
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
@@ -888,7 +890,7 @@ struct FinalNormBackward : public torch::autograd::Node {
     n.a = {a.const_data_ptr(), W};
     n.dout = {dout.const_data_ptr(), W};
     n.da = da.data_ptr(); n.da_stride = W;
-    n.row_map = row_map;
+    if (packed) n.row_map = row_map.unpack();
     const Tensor sums = norm_backward(n, ga, be, rows, W, eps);
     if (task_should_compute_output(0)) r[0] = da;
     if (task_should_compute_output(1)) r[1] = sums[0].to(ga.scalar_type()).view(ga.sizes());
@@ -1008,6 +1010,9 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count) {
       if (node->has_pos) node->pos = torch::autograd::SavedVariable(pos, false);
       if (node->has_ts) node->ts_tab = torch::autograd::SavedVariable(ts_tab, false);
       if (node->has_bias) node->bias = torch::autograd::SavedVariable(bias, false);
+      if ((node->has_mask_rows = o.mask_rows.defined())) node->mask_rows = torch::autograd::SavedVariable(o.mask_rows, false);
+      if ((node->has_bias_rows = o.bias_rows.defined())) node->bias_rows = torch::autograd::SavedVariable(o.bias_rows, false);
+      o.mask_rows = o.bias_rows = Tensor();
       node->opts = std::move(o);
       torch::autograd::set_history(out, node);
     }
@@ -1109,11 +1114,11 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
         if ((node->has[i] = p[i].defined())) node->params[i] = keep(p[i]);
       if ((node->has_pos = pos.defined())) node->pos = keep(pos);
       if ((node->has_ts = ts_tab.defined())) node->ts_tab = keep(ts_tab);
-      node->normed = std::move(normed);
-      node->pre = std::move(pre);
-      node->uqkv = std::move(uqkv);
-      node->attn = std::move(attn);
-      node->gated = std::move(gated);
+      node->saved_normed = keep(normed);
+      node->saved_pre = keep(pre);
+      node->saved_uqkv = keep(uqkv);
+      node->saved_attn = keep(attn);
+      node->saved_gated = keep(gated);
       node->call = std::move(c);
       torch::autograd::set_history(out, node);
     }
@@ -1321,7 +1326,7 @@ PyObject* final_norm(PyObject*, PyObject* const* a, Py_ssize_t count) {
       node->x = keep(x);
       node->gamma = keep(gamma);
       node->beta = keep(beta);
-      if (unpack) node->row_map = row_map;
+      if ((node->packed = unpack)) node->row_map = keep(row_map);
       node->eps = eps;
       torch::autograd::set_history(out, node);
     }

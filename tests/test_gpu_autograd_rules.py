@@ -83,3 +83,65 @@ def test_the_head_carries_tangents_and_second_derivatives(gpu):
   got = torch.autograd.grad([gx, gw], [w, x], [u, torch.ones_like(gw)])
   assert close(got[0], u.reshape(-1, 64).float().t() @ v.reshape(-1, 96).float())
   assert close(got[1], v.float() @ torch.ones(96, 64, device=DEV))
+
+
+def _bytes(t):
+  return t.numel() * t.element_size()
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_saved_tensor_hooks_see_what_the_block_keeps(gpu, packed):
+  """The block's intermediates (the normed rows, the projection before and after its activation, the attention and the gated rows: 11 x
+  tokens x D) go through torch's saved-tensor hooks: save_on_cpu leaves none of them on the GPU, and the gradients are the same bits."""
+  T, D = 4096, 128
+  blk = _block().requires_grad_(True)
+  x = _randn(T, D).requires_grad_(True)
+  offsets = torch.arange(0, T + 1, 512, dtype=torch.int32, device=DEV)
+  call = lambda: blk.forward_jagged(x, offsets, 512) if packed else blk(x.view(8, 512, D), seq_lens=torch.full((8,), 512, dtype=torch.int32, device=DEV))
+  dout = _randn(*call().shape, seed=3)
+  want = torch.autograd.grad(call(), [x, *blk.parameters()], dout)
+  held = []
+  for hooks in (None, torch.autograd.graph.save_on_cpu()):
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    if hooks is None:
+      out = call()
+    else:
+      with hooks:
+        out = call()
+    held.append(torch.cuda.memory_allocated() - before)
+    got = torch.autograd.grad(out, [x, *blk.parameters()], dout)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    del out, got
+  assert held[0] >= 11 * _bytes(x) and held[1] <= 2 * _bytes(x)
+
+
+def test_checkpointing_a_block_frees_and_recomputes(gpu):
+  """torch.utils.checkpoint without reentry replaces what is saved: nothing but the output stays, and the gradients are the same bits,
+  dropout included (its seed comes from torch's generator, which checkpointing restores)."""
+  from torch.utils.checkpoint import checkpoint
+  T, D = 4096, 128
+  blk = _block(dropout=0.2).requires_grad_(True)
+  x = _randn(8, 512, D).requires_grad_(True)
+  lens = torch.full((8,), 500, dtype=torch.int32, device=DEV)
+  dout = _randn(8, 512, D, seed=3)
+  torch.manual_seed(11)
+  want = torch.autograd.grad(blk(x, seq_lens=lens), [x, *blk.parameters()], dout)
+  torch.manual_seed(11)
+  torch.cuda.synchronize()
+  before = torch.cuda.memory_allocated()
+  out = checkpoint(lambda t: blk(t, seq_lens=lens), x, use_reentrant=False)
+  assert torch.cuda.memory_allocated() - before <= 2 * _bytes(x)
+  got = torch.autograd.grad(out, [x, *blk.parameters()], dout)
+  assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_a_second_backward_needs_the_graph_kept(gpu):
+  blk = _block().requires_grad_(True)
+  x = _randn(2, 40, 128).requires_grad_(True)
+  out = blk(x, seq_lens=torch.tensor([40, 9], dtype=torch.int32, device=DEV))
+  dout = _randn(2, 40, 128, seed=1)
+  a = torch.autograd.grad(out, x, dout, retain_graph=True)[0]
+  assert torch.equal(torch.autograd.grad(out, x, dout)[0], a)
+  with pytest.raises(RuntimeError, match="second time"):
+    torch.autograd.grad(out, x, dout)
