@@ -670,6 +670,21 @@ struct NormOp {
 // and offloading replace it).
 torch::autograd::SavedVariable keep(const Tensor& t) { return torch::autograd::SavedVariable(t, false); }
 
+// How far back a block's backward has to go, by what wants a gradient (`wanted(i)`: the i-th of tokens, the parameters, pos, ts_tab).
+struct BlockWants {
+  bool kernels = false, input, projections, attention, gate;
+  template <typename F>
+  explicit BlockWants(F&& wanted) {
+    bool biases = false;
+    for (int i = P_U; i <= P_V; ++i) kernels = kernels || wanted(1 + i);
+    for (int i = P_UB; i <= P_VB; ++i) biases = biases || wanted(1 + i);
+    input = wanted(0) || wanted(1 + P_IN_G) || wanted(1 + P_IN_B);
+    projections = kernels || biases || input;
+    attention = projections || wanted(1 + P_COUNT) || wanted(1 + P_COUNT + 1);
+    gate = attention || wanted(1 + P_ATTN_G) || wanted(1 + P_ATTN_B);
+  }
+};
+
 struct BlockBackward : public torch::autograd::Node {
   torch::autograd::SavedVariable tokens, params[P_COUNT], pos, ts_tab;
   bool has[P_COUNT] = {}, has_pos = false, has_ts = false;
@@ -686,41 +701,45 @@ struct BlockBackward : public torch::autograd::Node {
     call.opts = Options();
   }
 
-  // Gradients in the order of the edges: tokens, the parameters, pos, ts_tab.
+  // Gradients in the order of the edges: tokens, the parameters, pos, ts_tab.  The steps are undone from the output on, as far as a
+  // gradient is asked for behind them.
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const at::NoGradGuard no_grad;
     torch::autograd::variable_list r(1 + P_COUNT + 2);
     if (!grads[0].defined()) return r;
-    const Tensor x = tokens.unpack(), normed = saved_normed.unpack(), pre = saved_pre.unpack(), uqkv = saved_uqkv.unpack(), attn = saved_attn.unpack(),
-                 gated = saved_gated.unpack();
+    const BlockWants w([&](int i) { return task_should_compute_output(i); });
+    const Tensor x = tokens.unpack();
     const c10::DeviceGuard guard(x.device());
     Tensor p[P_COUNT];
     for (int i = 0; i < P_COUNT; ++i)
       if (has[i]) p[i] = params[i].unpack();
-    const Tensor pt = has_pos ? pos.unpack() : Tensor(), tt = has_ts ? ts_tab.unpack() : Tensor();
     const int64_t T = call.T, D = call.D, W = call.H * call.hd;
     auto want = [&](int i) { return task_should_compute_output(1 + i); };
     Tensor dout = grads[0].contiguous().view({T, D});
     if (!aligned(dout)) dout = dout.clone();
     // output product
     const Tensor wo = p[P_OUT].view({W, D});
-    const Tensor d_gated = input_gradient(dout, {&wo}, W, D);
     if (want(P_OUT)) {
-      const Tensor g = fresh(p[P_OUT], p[P_OUT].sizes());
+      const Tensor g = fresh(p[P_OUT], p[P_OUT].sizes()), gated = saved_gated.unpack();
       gemm(HSTU_GEMM_TN, T, {gated.const_data_ptr(), W}, {&g}, W, D, Tensor(), Tensor(), {nullptr, 0}, false, Tensor(), {dout.const_data_ptr(), D});
       r[1 + P_OUT] = g;
     }
     if (has[P_OUT_B] && want(P_OUT_B)) r[1 + P_OUT_B] = dout.sum(0);
+    if (!w.gate) return r;
     // attention norm and gate: du lands in the projection's gradient, already through its SiLU
+    const Tensor d_gated = input_gradient(dout, {&wo}, W, D);
+    const Tensor pre = saved_pre.unpack(), uqkv = saved_uqkv.unpack(), attn = saved_attn.unpack();
     const Tensor d_uqkv = at::empty_like(uqkv);
     auto rows_of = [&](const Tensor& t, int64_t stride) { return t.as_strided({T, W}, {stride, 1}, t.storage_offset()); };
     const NormOp gate(rows_of(attn, W), rows_of(uqkv, 4 * W), p[P_ATTN_G], p[P_ATTN_B], d_gated, call.eps, rows_of(d_uqkv, 4 * W), rows_of(pre, 4 * W),
                       Tensor());
-    const Tensor d_attn = gate.da.view(attn.sizes());
     if (want(P_ATTN_G)) r[1 + P_ATTN_G] = gate.dgamma.to(at::kBFloat16).view(p[P_ATTN_G].sizes());
     if (want(P_ATTN_B)) r[1 + P_ATTN_B] = gate.dbeta.to(at::kBFloat16).view(p[P_ATTN_B].sizes());
+    if (!w.attention) return r;
     // attention: dq, dk, dv land next to it
+    const Tensor d_attn = gate.da.view(attn.sizes());
+    const Tensor pt = has_pos ? pos.unpack() : Tensor(), tt = has_ts ? ts_tab.unpack() : Tensor();
     {
       const Tensor q = projection_slice(uqkv, call, 1), k = projection_slice(uqkv, call, 2), v = projection_slice(uqkv, call, 3);
       HstuAttnBwdArgs b;
@@ -746,13 +765,13 @@ struct BlockBackward : public torch::autograd::Node {
       if (has_pos && want(P_COUNT)) r[1 + P_COUNT] = dpos;
       if (has_ts && want(P_COUNT + 1)) r[1 + P_COUNT + 1] = dts;
     }
+    if (!w.projections) return r;
     block_check(hstu_silu_bwd((void*)at_column(d_uqkv, W), 4 * W, at_column(pre, W), 4 * W, T, (int32_t)(3 * W), stream_of(x)), "hstu_silu_bwd");
     // projections
     const Tensor dz = d_uqkv.view({T, 4 * W});
-    bool any = false;
-    for (int i = P_U; i <= P_V; ++i) any = any || want(i);
-    if (any) {
+    if (w.kernels) {
       const Tensor gu = fresh(p[P_U], p[P_U].sizes()), gq = fresh(gu, gu.sizes()), gk = fresh(gu, gu.sizes()), gv = fresh(gu, gu.sizes());
+      const Tensor normed = saved_normed.unpack();
       gemm(HSTU_GEMM_TN, T, {normed.const_data_ptr(), D}, {&gu, &gq, &gk, &gv}, D, 4 * W, Tensor(), Tensor(), {nullptr, 0}, false, Tensor(),
            {dz.const_data_ptr(), 4 * W});
       r[1 + P_U] = gu; r[1 + P_Q] = gq; r[1 + P_K] = gk; r[1 + P_V] = gv;
@@ -761,7 +780,7 @@ struct BlockBackward : public torch::autograd::Node {
       const Tensor g = dz.sum(0).view({4, call.H, call.hd});
       for (int i = 0; i < 4; ++i) r[1 + P_UB + i] = g[i];
     }
-    if (task_should_compute_output(0) || want(P_IN_G) || want(P_IN_B)) {
+    if (w.input) {
       const Tensor d_normed = input_gradient(dz, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W);
       // (with the residual's share added)
       const NormOp in(x.view({T, D}), Tensor(), p[P_IN_G], p[P_IN_B], d_normed, call.eps, Tensor(), Tensor(), dout);
@@ -1114,11 +1133,19 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
         if ((node->has[i] = p[i].defined())) node->params[i] = keep(p[i]);
       if ((node->has_pos = pos.defined())) node->pos = keep(pos);
       if ((node->has_ts = ts_tab.defined())) node->ts_tab = keep(ts_tab);
-      node->saved_normed = keep(normed);
-      node->saved_pre = keep(pre);
-      node->saved_uqkv = keep(uqkv);
-      node->saved_attn = keep(attn);
-      node->saved_gated = keep(gated);
+      // (only what the gradients asked for read)
+      auto wanted = [&](int i) {
+        const Tensor& t = i == 0 ? tokens : i <= P_COUNT ? p[i - 1] : i == P_COUNT + 1 ? pos : ts_tab;
+        return t.defined() && t.requires_grad();
+      };
+      const BlockWants w(wanted);
+      if (w.kernels) node->saved_normed = keep(normed);
+      if (w.gate) {
+        node->saved_pre = keep(pre);
+        node->saved_uqkv = keep(uqkv);
+        node->saved_attn = keep(attn);
+      }
+      if (wanted(1 + P_OUT)) node->saved_gated = keep(gated);
       node->call = std::move(c);
       torch::autograd::set_history(out, node);
     }

@@ -145,3 +145,33 @@ def test_a_second_backward_needs_the_graph_kept(gpu):
   assert torch.equal(torch.autograd.grad(out, x, dout)[0], a)
   with pytest.raises(RuntimeError, match="second time"):
     torch.autograd.grad(out, x, dout)
+
+
+@pytest.mark.parametrize("part", ["output_kernel", "output_bias", "attn_ln_beta", "pos", "k_kernel", "v_bias", "input_ln_gamma", "x"])
+def test_frozen_parts_are_not_differentiated(gpu, part):
+  """A gradient is taken back only as far as something behind wants it, and only what that reads is kept: the same bits as with
+  everything trained, and for the parts behind the gate neither the projection nor its gradient (8 x tokens x D) is there."""
+  T, D = 4096, 128
+  blk = _block(use_bias=True)
+  x = _randn(8, 512, D)
+  lens = torch.full((8,), 500, dtype=torch.int32, device=DEV)
+  pos = _randn(2, 1023, std=0.1, dtype=torch.float32)
+  dout = _randn(8, 512, D, seed=3)
+  named = dict(blk.named_parameters(), x=x, pos=pos)
+  for t in named.values():
+    t.requires_grad_(True)
+  want = dict(zip(named, torch.autograd.grad(blk(x, seq_lens=lens, pos_bias=pos), list(named.values()), dout)))[part]
+  for t in named.values():
+    t.requires_grad_(False)
+  named[part].requires_grad_(True)
+  torch.cuda.synchronize()
+  before = torch.cuda.memory_allocated()
+  out = blk(x, seq_lens=lens, pos_bias=pos)
+  held = torch.cuda.memory_allocated() - before
+  torch.cuda.reset_peak_memory_stats()
+  got = torch.autograd.grad(out, named[part], dout)[0]
+  peak = torch.cuda.max_memory_allocated() - before
+  # (the position table's gradient is added up by atomics, in no fixed order)
+  assert torch.equal(got, want) if part != "pos" else (got - want).abs().max() <= 1e-5 * want.abs().max()
+  if part.startswith("output"):
+    assert held <= 3 * _bytes(x) and peak <= 4 * _bytes(x)
