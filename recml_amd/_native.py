@@ -31,8 +31,6 @@ def _load():
   spec = importlib.util.spec_from_file_location("recml_amd.lib._native", PATH)
   module = importlib.util.module_from_spec(spec)
   spec.loader.exec_module(module)
-  from recml_amd import hstu_block_ops, hstu_ops
-  module.set_operators(vars(hstu_ops), hstu_ops._OWN_ATTENTION_BWD, vars(hstu_block_ops), hstu_block_ops._OWN_NORM_GATE_BWD)
   return module
 
 

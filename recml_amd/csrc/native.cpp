@@ -311,58 +311,6 @@ Tensor like_output(const Tensor& q, const Tensor& v) {
 // autograd
 // ---------------------------------------------------------------------------
 
-// The package's Python operators that the graph nodes stand for.  A node runs the C call directly as long as the operator
-// is the package's own; where a program has put something else in its place (to count or check the calls), that is called.
-struct Operator {
-  const char* name;
-  PyObject* space = nullptr;       // the module's namespace
-  PyObject* own = nullptr;         // the operator as the package defines it
-
-  // What stands there instead of the package's own (a new reference), or null.  With the interpreter's lock.
-  PyObject* other() const {
-    PyObject* const now = space ? PyDict_GetItemString(space, name) : nullptr;
-    if (!now || now == own) return nullptr;
-    Py_INCREF(now);
-    return now;
-  }
-};
-Operator op_attention_bwd{"hstu_attention_bwd"}, op_norm_gate_bwd{"norm_gate_bwd"};
-
-struct Lock {
-  PyGILState_STATE state = PyGILState_Ensure();
-  ~Lock() { PyGILState_Release(state); }
-};
-
-PyObject* wrap(const Tensor& t) {
-  if (t.defined()) return THPVariable_Wrap(t);
-  Py_RETURN_NONE;
-}
-
-// Calls fn(*args, **kw) (all references taken) and gives back its tuple's tensors.
-std::vector<Tensor> call_operator(PyObject* fn, PyObject* args, PyObject* kw) {
-  PyObject* const got = fn && args && kw ? PyObject_Call(fn, args, kw) : nullptr;
-  std::vector<Tensor> out;
-  std::string why;
-  if (got && PyTuple_Check(got)) {
-    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(got); ++i) {
-      PyObject* const x = PyTuple_GET_ITEM(got, i);
-      out.push_back(THPVariable_Check(x) ? THPVariable_Unpack(x) : Tensor());
-    }
-  } else {
-    why = "an operator of the backward did not return a tuple";
-    if (PyErr_Occurred()) {
-      PyObject *type, *value, *trace;
-      PyErr_Fetch(&type, &value, &trace);
-      PyObject* const text = value ? PyObject_Str(value) : nullptr;
-      if (text && PyUnicode_Check(text)) why = PyUnicode_AsUTF8(text);
-      for (PyObject* o : {text, type, value, trace}) Py_XDECREF(o);
-    }
-  }
-  for (PyObject* o : {got, kw, args, fn}) Py_XDECREF(o);
-  TORCH_CHECK(why.empty(), why);
-  return out;
-}
-
 // dq, dk, dv with the strides of q, k, v.  Slices of one projection get slices of one buffer laid out like it (mirrored
 // one by one each would span nearly all of the projection).
 void gradient_buffers(const Tensor (&t)[3], Tensor (&g)[3]) {
@@ -406,32 +354,6 @@ struct AttentionBackward : public torch::autograd::Node {
     const Tensor p = has_pos ? pos.unpack() : Tensor(), tt = has_ts ? ts_tab.unpack() : Tensor(), bs = has_bias ? bias.unpack() : Tensor();
     const c10::DeviceGuard guard(t[0].device());
     const Tensor dout = grads[0].contiguous();
-    {
-      const Lock lock;
-      if (PyObject* const fn = op_attention_bwd.other()) {
-        const bool tables = (has_pos && task_should_compute_output(3)) || (has_ts && task_should_compute_output(4));
-        const bool grad_bias = has_bias && task_should_compute_output(5);
-        PyObject* const args = Py_BuildValue("(NNNN)", wrap(t[0]), wrap(t[1]), wrap(t[2]), wrap(dout));
-        PyObject* const kw = Py_BuildValue(
-            "{s:N,s:N,s:d,s:N,s:N,s:N,s:N,s:d,s:N,s:N,s:N,s:N,s:d,s:K,s:N,s:N}", "seq_lens", wrap(opts.seq_lens), "seq_offsets", wrap(opts.seq_offsets),
-            "alpha", opts.alpha, "causal", PyBool_FromLong(opts.causal), "pos_bias", wrap(p), "timestamps", wrap(opts.timestamps), "ts_bias", wrap(tt),
-            "ts_bucket_size", opts.bucket_size, "q_segment_ids", wrap(opts.q_seg), "kv_segment_ids", wrap(opts.kv_seg), "mask", wrap(opts.mask), "bias",
-            wrap(bs), "dropout_p", opts.dropout_p, "dropout_seed", (unsigned long long)opts.dropout_seed, "table_grads", PyBool_FromLong(tables),
-            "bias_grad", PyBool_FromLong(grad_bias));
-        auto also = [&](const char* name, PyObject* value) {
-          if (kw) PyDict_SetItemString(kw, name, value);
-          Py_XDECREF(value);
-        };
-        if (opts.max_len >= 0) also("max_len", PyLong_FromLongLong(opts.max_len));
-        if (opts.n > 0.0) also("n", PyFloat_FromDouble(opts.n));
-        if (opts.window >= 0) also("sliding_window_size", PyLong_FromLongLong(opts.window));
-        std::vector<Tensor> got = call_operator(fn, args, kw);
-        got.resize(6);
-        for (int i = 0; i < 6; ++i)
-          if (task_should_compute_output(i)) result[i] = got[i];
-        return result;
-      }
-    }
     HstuAttnBwdArgs b;
     memset(&b, 0, sizeof(b));
     b.struct_size = sizeof(b);
@@ -637,17 +559,6 @@ struct NormOp {
   Tensor da, dgamma, dbeta;
   NormOp(const Tensor& attn, const Tensor& u, const Tensor& gamma, const Tensor& beta, const Tensor& dout, double eps, const Tensor& du_out,
          const Tensor& u_pre, const Tensor& add) {
-    {
-      const Lock lock;
-      if (PyObject* const fn = op_norm_gate_bwd.other()) {
-        PyObject* const args = Py_BuildValue("(NNNNNd)", wrap(attn), wrap(u), wrap(gamma.view({gamma.numel()})), wrap(beta.view({beta.numel()})), wrap(dout), eps);
-        PyObject* const kw = Py_BuildValue("{s:N,s:N,s:N}", "du_out", wrap(du_out), "u_pre", wrap(u_pre), "add", wrap(add));
-        const std::vector<Tensor> got = call_operator(fn, args, kw);
-        TORCH_CHECK(got.size() == 4, "norm_gate_bwd returns four tensors");
-        da = got[0]; dgamma = got[2]; dbeta = got[3];
-        return;
-      }
-    }
     const int64_t rows = attn.size(0), W = attn.size(1);
     da = fresh(attn, {rows, W});
     NormGrad n;
@@ -1446,23 +1357,10 @@ PyObject* mask_lengths(PyObject*, PyObject* const* a, Py_ssize_t count) {
   });
 }
 
-// set_operators(hstu_ops' namespace, hstu_attention_bwd, hstu_block_ops' namespace, norm_gate_bwd)
-PyObject* set_operators(PyObject*, PyObject* const* a, Py_ssize_t count) {
-  if (count != 4 || !PyDict_Check(a[0]) || !PyDict_Check(a[2])) {
-    PyErr_SetString(PyExc_TypeError, "set_operators takes two namespaces, each with its operator");
-    return nullptr;
-  }
-  for (int i = 0; i < 4; ++i) Py_INCREF(a[i]);       // (for as long as the module lives)
-  op_attention_bwd.space = a[0]; op_attention_bwd.own = a[1];
-  op_norm_gate_bwd.space = a[2]; op_norm_gate_bwd.own = a[3];
-  Py_RETURN_NONE;
-}
-
 PyMethodDef methods[] = {
     {"attention", (PyCFunction)(void (*)(void))attention, METH_FASTCALL,
      "One attention forward on arguments that are ready for the kernels; None when they are not."},
 #define HSTU_FAST(name, doc) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, doc}
-    HSTU_FAST(set_operators, "The Python operators behind the graph nodes."),
     HSTU_FAST(block, "One HSTU block forward (differentiable where asked)."),
     HSTU_FAST(norm_gate_bwd, "The gradients of the norm and gate step."),
     HSTU_FAST(embed, "The model's front end: gather, position embedding, layer norm."),

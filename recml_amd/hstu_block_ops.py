@@ -125,7 +125,7 @@ def norm_gate_bwd(attn, u, gamma, beta, dout, eps: float = 1e-6, *, du_out=None,
   return da, du, dgb[0], dgb[1]
 
 
-_OWN_NORM_GATE_BWD = norm_gate_bwd    # (how the native graph nodes tell it from something put in its place)
+_OWN_NORM_GATE_BWD = norm_gate_bwd    # (where a program puts another operator in its place, that one is called: no native node then)
 
 
 class _NormGateFn(torch.autograd.Function):

@@ -302,7 +302,8 @@ class HSTUBlock(torch.nn.Module):
       return None
     weights = self._weights()
     grad = _wants_grad(tokens, *weights, pos_bias, ts_bias, attention_bias)
-    if grad and not self._fused_training(tokens, pos_bias, ts_bias):
+    if grad and not (self._fused_training(tokens, pos_bias, ts_bias) and hstu_ops.hstu_attention_bwd is hstu_ops._OWN_ATTENTION_BWD
+                     and hstu_block_ops.norm_gate_bwd is hstu_block_ops._OWN_NORM_GATE_BWD):
       return None
     # (torch's default integers, 16-bit tables: converted here, by the first block of a batch for all of them; a table's conversion is
     # part of the graph)

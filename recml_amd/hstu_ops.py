@@ -560,7 +560,7 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
   return dq, dk, dv, dpos, dts
 
 
-_OWN_ATTENTION_BWD = hstu_attention_bwd    # (how the native graph nodes tell it from something put in its place)
+_OWN_ATTENTION_BWD = hstu_attention_bwd    # (where a program puts another operator in its place, that one is called: no native node then)
 
 
 def dropout_keep(seed, p, b, h, H, i, j) -> bool:
@@ -623,7 +623,7 @@ def hstu_attention_autograd(q, k, v, *, pos_bias=None, ts_bias=None, bias=None, 
   """hstu_attention as a differentiable torch op: gradients for q, k, v, the bias tables pos_bias
   and ts_bias, and a dense `bias` (its gradient is dS summed over the heads, and over the batch
   when the bias is shared by it)."""
-  if kwargs.keys() <= _NATIVE_AUTOGRAD:
+  if kwargs.keys() <= _NATIVE_AUTOGRAD and hstu_attention_bwd is _OWN_ATTENTION_BWD:
     got = _native_autograd(q, k, v, pos_bias, ts_bias, bias, **kwargs)
     if got is not None:
       return got

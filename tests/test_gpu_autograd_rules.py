@@ -174,4 +174,5 @@ def test_frozen_parts_are_not_differentiated(gpu, part):
   # (the position table's gradient is added up by atomics, in no fixed order)
   assert torch.equal(got, want) if part != "pos" else (got - want).abs().max() <= 1e-5 * want.abs().max()
   if part.startswith("output"):
-    assert held <= 3 * _bytes(x) and peak <= 4 * _bytes(x)
+    # (a bias's column sum is torch's, which brings 4 MB of scratch, 4 x tokens x D here)
+    assert held <= 3 * _bytes(x) and peak <= 7 * _bytes(x)
