@@ -33,6 +33,9 @@
 extern "C" {
 #endif
 
+/* Version 4 added mask_pitch and bias_pitch at the end of HstuAttnFwdArgs.  Callers built against version 3 are taken as
+ * they are: their structs say so in struct_size and version, and what they do not have is zero.  Any other pair that does
+ * not match is refused (HSTU_ERR_VERSION). */
 #define HSTU_ATTN_ABI_VERSION 4
 
 /* Tensor layouts of q, k, v, out. */

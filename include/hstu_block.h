@@ -36,6 +36,10 @@
 extern "C" {
 #endif
 
+/* Versions since 3 added members at the end of HstuNormGateArgs, HstuNormGateBwdArgs and HstuEmbedNormArgs (4: seq_offsets and L;
+ * u_pre, add and row_map; row_map, L and round_steps; 5: sums, keys and outside) and functions; 5 took hstu_embed_norm_bwd away.
+ * Callers built against 3 or 4 are taken as they are: their structs say so in struct_size and version, and what they do not have
+ * is zero.  Any other pair that does not match is refused (HSTU_BLOCK_ERR_VERSION). */
 #define HSTU_BLOCK_ABI_VERSION 5
 
 typedef enum HstuBlockStatus {

@@ -4999,6 +4999,34 @@ bool mfma_eligible(const HstuAttnFwdArgs* a) {
   return d_ok && opts_ok && align_ok && off_ok;
 }
 
+// Structs of callers that were built against version 3 of the ABI: what they end with is a prefix of what they are now (the forward's;
+// the backward's embeds it).  They are read as today's with zeros in what they do not have; any other struct is taken as it is.
+constexpr size_t FWD_ARGS_V3 = offsetof(HstuAttnFwdArgs, mask_pitch);
+constexpr size_t BWD_ARGS_V3 = sizeof(HstuAttnBwdArgs) - (sizeof(HstuAttnFwdArgs) - FWD_ARGS_V3);
+const HstuAttnFwdArgs* today(const HstuAttnFwdArgs* a, HstuAttnFwdArgs& own) {
+  if (!a || a->version != 3 || a->struct_size != FWD_ARGS_V3) return a;
+  memset(&own, 0, sizeof(own));
+  memcpy(&own, a, FWD_ARGS_V3);
+  own.struct_size = sizeof(own);
+  own.version = HSTU_ATTN_ABI_VERSION;
+  return &own;
+}
+const HstuAttnBwdArgs* today(const HstuAttnBwdArgs* a, HstuAttnBwdArgs& own) {
+  if (!a || a->version != 3 || a->struct_size != BWD_ARGS_V3) return a;
+  constexpr size_t head = offsetof(HstuAttnBwdArgs, fwd) + FWD_ARGS_V3, tail = sizeof(HstuAttnBwdArgs) - offsetof(HstuAttnBwdArgs, dout);
+  static_assert(head + tail == BWD_ARGS_V3, "the backward's struct of version 3: the forward's of that version between head and tail");
+  memset(&own, 0, sizeof(own));
+  memcpy(&own, a, head);
+  memcpy((char*)&own + offsetof(HstuAttnBwdArgs, dout), (const char*)a + head, tail);
+  own.struct_size = sizeof(own);
+  own.version = HSTU_ATTN_ABI_VERSION;
+  if (own.fwd.version == 3 && own.fwd.struct_size == FWD_ARGS_V3) {
+    own.fwd.struct_size = sizeof(own.fwd);
+    own.fwd.version = HSTU_ATTN_ABI_VERSION;
+  }
+  return &own;
+}
+
 int validate(const HstuAttnFwdArgs* a) {
   if (!a) return fail(HSTU_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuAttnFwdArgs) || a->version != HSTU_ATTN_ABI_VERSION)
@@ -5629,6 +5657,8 @@ int hstu_attn_dropout_keep(uint64_t dropout_seed, float dropout_p, int32_t b, in
 const char* hstu_attn_last_error(void) { return g_err; }
 
 size_t hstu_attn_fwd_workspace_bytes(const HstuAttnFwdArgs* args) {
+  HstuAttnFwdArgs own;
+  args = today(args, own);
   if (validate(args) != HSTU_OK) return 0;
   return plan_workspace(args).total();
 }
@@ -5655,6 +5685,8 @@ int hstu_attn_pad_rows(const void* src, void* dst, int64_t rows, int32_t n, int3
 }
 
 const char* hstu_attn_fwd_variant(const HstuAttnFwdArgs* args) {
+  HstuAttnFwdArgs own;
+  args = today(args, own);
   if (validate(args) != HSTU_OK) return "invalid";
   switch (pick_variant(args)) {
     case V_GENERAL_F32: return "hstu_fwd_general<float>";
@@ -5666,6 +5698,8 @@ const char* hstu_attn_fwd_variant(const HstuAttnFwdArgs* args) {
 }
 
 const char* hstu_attn_bwd_variant(const HstuAttnBwdArgs* args) {
+  HstuAttnBwdArgs own;
+  args = today(args, own);
   if (!args || args->struct_size != sizeof(HstuAttnBwdArgs) || args->version != HSTU_ATTN_ABI_VERSION) return "invalid";
   HstuAttnFwdArgs probe = args->fwd;
   if (!probe.out) probe.out = (void*)args->dout;
@@ -5678,6 +5712,8 @@ const char* hstu_attn_bwd_variant(const HstuAttnBwdArgs* args) {
 }
 
 int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) {
+  HstuAttnBwdArgs own;
+  args = today(args, own);
   if (!args) return fail(HSTU_ERR_NULL, "args is null");
   if (args->struct_size != sizeof(HstuAttnBwdArgs) || args->version != HSTU_ATTN_ABI_VERSION)
     return fail(HSTU_ERR_VERSION, "backward args struct_size/version (%u/%u) do not match this library (%zu/%d)",
@@ -5708,6 +5744,8 @@ int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) {
 }
 
 int hstu_attn_fwd_noalloc(const HstuAttnFwdArgs* args, void* stream) {
+  HstuAttnFwdArgs own;
+  args = today(args, own);
   int rc = validate(args);
   if (rc != HSTU_OK) return rc;
   HstuAttnFwdArgs a = *args;
@@ -5727,6 +5765,8 @@ int hstu_attn_fwd_noalloc(const HstuAttnFwdArgs* args, void* stream) {
 }
 
 int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
+  HstuAttnFwdArgs own;
+  args = today(args, own);
   int rc = validate(args);
   if (rc != HSTU_OK) return rc;
   g_err[0] = 0;

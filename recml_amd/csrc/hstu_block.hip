@@ -807,6 +807,8 @@ int hstu_block_abi_version(void) { return HSTU_BLOCK_ABI_VERSION; }
 const char* hstu_block_last_error(void) { return g_err; }
 
 int hstu_norm_gate_fwd(const HstuNormGateArgs* a, void* stream) {
+  HstuNormGateArgs own;
+  a = block_today(a, own, offsetof(HstuNormGateArgs, seq_offsets), sizeof(HstuNormGateArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuNormGateArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "norm-gate args struct_size/version (%u/%u) do not match this library (%zu/%d)",
@@ -850,6 +852,8 @@ size_t hstu_norm_gate_bwd_workspace_bytes(int64_t rows, int32_t width) {
 }
 
 int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
+  HstuNormGateBwdArgs own;
+  a = block_today(a, own, offsetof(HstuNormGateBwdArgs, u_pre), sizeof(HstuNormGateBwdArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuNormGateBwdArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "norm-gate backward args struct_size/version (%u/%u) do not match this library (%zu/%d)",
@@ -897,6 +901,8 @@ int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
 }
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
+  HstuEmbedNormArgs own;
+  a = block_today(a, own, offsetof(HstuEmbedNormArgs, row_map), offsetof(HstuEmbedNormArgs, sums));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuEmbedNormArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "embed-norm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
@@ -942,6 +948,8 @@ size_t hstu_embed_grad_workspace_bytes(int64_t rows, int64_t keys, int32_t width
 }
 
 int hstu_embed_grad(const HstuEmbedGradArgs* a, void* stream) {
+  HstuEmbedGradArgs own;
+  a = block_today(a, own, 0, sizeof(HstuEmbedGradArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuEmbedGradArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "embedding gradient args do not match this library");
@@ -1026,6 +1034,8 @@ int hstu_silu_bwd(void* d, int64_t d_stride, const void* pre, int64_t pre_stride
 size_t hstu_gemm_silu_workspace_bytes(void) { return kBlasWorkspace; }
 
 int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
+  HstuGemmSiluArgs own;
+  a = block_today(a, own, sizeof(HstuGemmSiluArgs), sizeof(HstuGemmSiluArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuGemmSiluArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",

@@ -4,7 +4,11 @@
 #define HSTU_BLOCK_COMMON_H_
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
+#include <string.h>
+
+#include "hstu_block.h"
 
 // Stores the message that hstu_block_last_error() returns on this thread; returns `code`.
 __attribute__((visibility("hidden"))) int block_fail(int code, const char* fmt, ...);
@@ -12,6 +16,18 @@ __attribute__((visibility("hidden"))) int block_fail(int code, const char* fmt, 
 __attribute__((visibility("hidden"))) int block_allow_lds(const void* fn, int bytes, int* granted);
 
 namespace {
+
+// The arguments as this version has them: a struct of versions 3 or 4 (of the given sizes: prefixes of today's) with zeros in
+// what it does not have, any other as it is.
+template <typename A>
+const A* block_today(const A* a, A& own, size_t v3, size_t v4) {
+  if (!a || !((a->version == 3 && a->struct_size == v3) || (a->version == 4 && a->struct_size == v4))) return a;
+  memset(&own, 0, sizeof(own));
+  memcpy(&own, a, a->struct_size);
+  own.struct_size = sizeof(own);
+  own.version = HSTU_BLOCK_ABI_VERSION;
+  return &own;
+}
 
 typedef __bf16 bf16_t;
 typedef float floatx2 __attribute__((ext_vector_type(2)));

@@ -505,6 +505,8 @@ size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K) {
 }
 
 int hstu_gemm(const HstuGemmArgs* a, void* stream) {
+  HstuGemmArgs own;
+  a = block_today(a, own, 0, sizeof(HstuGemmArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
   if (a->struct_size != sizeof(HstuGemmArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
     return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
