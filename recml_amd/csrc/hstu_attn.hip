@@ -5464,15 +5464,22 @@ int slots_per_xcd(const Params& p, int32_t* out) {
   return HSTU_OK;
 }
 
-// Points the workspace fields of `q` into the caller's buffer as `ws` lays it out and enqueues the
-// kernel that fills it (unless the caller says it is filled already).
-int setup_workspace(const HstuAttnFwdArgs* args, const WorkspacePlan& ws, Params& q, hipStream_t st) {
-  q.split_cap = ws.split_cap;
+// Whether the caller's buffer is what hstu_attn_fwd_workspace_bytes asks for.
+int check_workspace(const HstuAttnFwdArgs* args, const WorkspacePlan& ws) {
   if (!ws.total()) return HSTU_OK;
   if (!args->workspace || args->workspace_bytes < ws.total())
     return fail(HSTU_ERR_WORKSPACE, "workspace of %zu bytes needed (see hstu_attn_fwd_workspace_bytes), got %zu",
                 ws.total(), args->workspace ? args->workspace_bytes : (size_t)0);
   if (((uintptr_t)args->workspace & 255u) != 0) return fail(HSTU_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  return HSTU_OK;
+}
+
+// Points the workspace fields of `q` into the caller's buffer as `ws` lays it out and enqueues the
+// kernel that fills it (unless the caller says it is filled already).
+int setup_workspace(const HstuAttnFwdArgs* args, const WorkspacePlan& ws, Params& q, hipStream_t st) {
+  q.split_cap = ws.split_cap;
+  if (int rc = check_workspace(args, ws)) return rc;
+  if (!ws.total()) return HSTU_OK;
   char* base = (char*)args->workspace;
   if (ws.bias_total() >= (1ull << 32)) return fail(HSTU_ERR_WORKSPACE, "workspace of %zu bytes is beyond what the kernel addresses", ws.bias_total());
   float* pos_out = ws.pos_bytes ? (float*)base : nullptr;
@@ -5787,6 +5794,8 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // kernel takes the table itself, and the preparation is not launched.
       q.whole_window = ws.sched_bytes == 0 && q.pos_tab && !q.ts_tab && !q.mask && !q.dense_bias && q.mask_mode != HSTU_MASK_SEGMENT &&
                        q.Lkv <= WHOLE_KEYS;
+      // (a buffer that is missing is an error all the same: which calls use it is not the caller's to know)
+      if (int rc2 = check_workspace(args, ws)) return rc2;
       if (q.whole_window && !(args->flags & HSTU_FWD_PREPARE_ONLY)) return f8 ? launch_mfma<true>(q, st) : launch_mfma<false>(q, st);
       if (int rc2 = setup_workspace(args, ws, q, st)) return rc2;
       if (args->flags & HSTU_FWD_PREPARE_ONLY) return HSTU_OK;
