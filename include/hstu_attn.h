@@ -184,7 +184,8 @@ typedef struct HstuAttnFwdArgs {
   uint64_t dropout_seed;
   /* Row pitch of `mask` (bytes) and of `dense_bias` (floats); 0: Lkv, a contiguous matrix.  The matrix-core kernels
    * fetch rows in 16-byte pieces: a matrix whose Lkv does not allow that can be handed over with rows a few elements
-   * longer (hstu_attn_pad_rows makes such a copy; at most 15 more, zeros there).  ddense_bias stays [.., L, Lkv]. */
+   * longer (hstu_attn_pad_rows makes such a copy; at most 15 more, zeros there).  ddense_bias stays [.., L, Lkv].  A forward
+   * call with a pitch multiplies its weights as two bf16 parts (16 bits), as the general kernel multiplies them in 32 bits. */
   int64_t mask_pitch, bias_pitch;
 } HstuAttnFwdArgs;
 

@@ -2332,6 +2332,9 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
 // registers at the start of the step and at once asks for step t + 1 into the same bytes -- no other
 // wave is involved, and the loads have the whole block and the barrier to land.  With a three-stage K / V
 // ring that is 68 KB at d = 128: two workgroups per CU.  A block whose mask tile is all zero is skipped.
+// Bit 2: the second product takes the activated weights as two bf16 parts, the rounded value and what the rounding left, instead of
+// the rounded value alone.  This is for calls whose rows were made longer for this kernel (mask_pitch, bias_pitch): the general kernel,
+// which they would otherwise take, multiplies 32-bit weights.
 // Ring depth of the forward kernel.  Up to d = 64 a wave needs at most 128 registers, so four
 // workgroups fit a CU once their LDS does: three stages (two steps in flight behind the one being
 // computed) instead of four take the d = 64 kernel with a position table from 43 KB to 32 KB, three
@@ -2911,6 +2914,23 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
 #pragma unroll
       for (int dvb = 0; dvb < DVB; ++dvb)
         o[dvb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[cc][dvb]), pb, o[dvb], 0, 0, 0);
+      if constexpr ((DENSE & 4) != 0) {
+        // (an infinite weight has no second part)
+        const uint32_t w2[4] = {pk.x, pk.y, pk.z, pk.w};
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const float hi = __builtin_bit_cast(float, (r & 1) ? w2[r >> 1] & 0xffff0000u : w2[r >> 1] << 16);
+          e[r] = __builtin_fabsf(hi) < __builtin_inff() ? e[r] - hi : 0.f;
+        }
+        pk.x = pack_bf16(e[0], e[1]);
+        pk.y = pack_bf16(e[2], e[3]);
+        pk.z = pack_bf16(e[4], e[5]);
+        pk.w = pack_bf16(e[6], e[7]);
+        const bf16x8 pl = __builtin_bit_cast(bf16x8, pk);
+#pragma unroll
+        for (int dvb = 0; dvb < DVB; ++dvb)
+          o[dvb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[cc][dvb]), pl, o[dvb], 0, 0, 0);
+      }
     }
   };
 
@@ -5201,6 +5221,7 @@ Params make_params(const HstuAttnFwdArgs* a) {
   p.mask_mode = p.jagged ? HSTU_MASK_LENGTH : a->mask_mode;
   p.window = effective_window(a);
   p.mask_pitch = dense_pitch(a, a->mask_pitch); p.bias_pitch = dense_pitch(a, a->bias_pitch);
+  p.weights_in_parts = a->mask_pitch != 0 || a->bias_pitch != 0;
   p.mask_batched = a->mask_batched; p.dense_bias_batched = a->dense_bias_batched;
   p.pos_heads = a->pos_heads; p.ts_heads = a->ts_heads;
   p.ts_nb = a->ts_num_buckets;
@@ -5402,9 +5423,15 @@ template <int D, bool F8>
 int launch_mfma_d(const Params& p, hipStream_t st) {
   const bool pos = p.pos_tab != nullptr, ts = p.ts_tab != nullptr;
   if (!F8 && (p.mask || p.dense_bias)) {
-    if (p.mask && p.dense_bias) return launch_mfma_inst<D, false, false, false, false, 3>(p, st);
-    if (p.mask) return launch_mfma_inst<D, false, false, false, false, 2>(p, st);
-    return launch_mfma_inst<D, false, false, false, false, 1>(p, st);
+    const int kind = (p.dense_bias ? 1 : 0) + (p.mask ? 2 : 0) + (p.weights_in_parts ? 4 : 0);
+    switch (kind) {
+      case 1: return launch_mfma_inst<D, false, false, false, false, 1>(p, st);
+      case 2: return launch_mfma_inst<D, false, false, false, false, 2>(p, st);
+      case 3: return launch_mfma_inst<D, false, false, false, false, 3>(p, st);
+      case 5: return launch_mfma_inst<D, false, false, false, false, 5>(p, st);
+      case 6: return launch_mfma_inst<D, false, false, false, false, 6>(p, st);
+      default: return launch_mfma_inst<D, false, false, false, false, 7>(p, st);
+    }
   }
   if (!F8 && p.mask_mode == HSTU_MASK_SEGMENT) {
     if (pos && ts) return launch_mfma_inst<D, true, true, false, true>(p, st);

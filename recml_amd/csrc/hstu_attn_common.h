@@ -49,6 +49,7 @@ struct Params {
   int32_t jagged, causal, mask_mode, window;
   int32_t mask_batched, dense_bias_batched, pos_heads, ts_heads;
   int32_t mask_pitch, bias_pitch;   // bytes and floats from one row of the keep-mask and of the dense bias to the next
+  int32_t weights_in_parts;         // the matrix-core forward: activated weights as two bf16 parts in the second product
   int32_t ts_nb;
   float ts_bucket_size;
   float alpha, inv_n;

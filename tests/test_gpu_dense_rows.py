@@ -53,3 +53,32 @@ def test_dense_rows_of_any_length(gpu, L, d, with_mask, with_bias, shared):
     assert _rel(g.float().cpu().numpy(), w) <= 2e-2, nm
   if with_bias:
     assert _rel(bt.grad.cpu().numpy(), want[5]) <= 2e-2
+
+
+def _beside(x):
+  """The same values in rows that are no whole 16 bytes apart: such a call is the general kernel's."""
+  B, L, H, d = x.shape
+  buf = torch.zeros((B, L, H * d + 4), dtype=bf, device="cuda:0")
+  buf[:, :, : H * d] = x.reshape(B, L, H * d)
+  return buf[:, :, : H * d].unflatten(2, (H, d))
+
+
+@pytest.mark.parametrize("L", [67, 258, 1002])
+@pytest.mark.parametrize("d,with_mask,with_bias", [(64, True, True), (32, True, False), (128, False, True), (128, True, True)])
+def test_weights_of_longer_rows_keep_their_bits(gpu, L, d, with_mask, with_bias):
+  """Against 64 bits the matrix-core kernel is no further off than the general kernel, which multiplies 32-bit weights and which took
+  these calls: both leave the output's rounding, sqrt(1/12) 2^-8 or so.  2 % is what the weights' second rounding, at 2^-17, and the
+  order of the sums may add; weights rounded once to bf16 are 15 % and more further off."""
+  rng = np.random.default_rng(L + d)
+  B, H = 2, 2
+  q, k, v = (O.round_bf16(rng.standard_normal((B, L, H, d)).astype(np.float32) * 0.4) for _ in range(3))
+  mask = (rng.random((B, L, L)) > 0.3) & (np.arange(L)[None, None, :] <= np.arange(L)[None, :, None]) if with_mask else None
+  bias = (rng.standard_normal((B, L, L)) * 0.4).astype(np.float32) if with_bias else None
+  kw = dict(n=float(L), alpha=0.3, causal=not with_mask)
+  want = O.hstu_attention_ref(q, k, v, mask=mask, bias=bias, dtype=np.float64, **kw)
+  gk = dict(kw, mask=None if mask is None else _dev(mask), bias=None if bias is None else _dev(bias))
+  ts = [_dev(x, bf) for x in (q, k, v)]
+  err = lambda *t: np.linalg.norm(recml_amd.hstu_attention(*t, **gk).double().cpu().numpy() - want) / np.linalg.norm(want)
+  here, general = err(*ts), err(*(_beside(t) for t in ts))
+  assert here <= 1.02 * general, (here, general)
+
