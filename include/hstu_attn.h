@@ -195,8 +195,9 @@ typedef struct HstuAttnFwdArgs {
  * dropout_p = 0. */
 int hstu_attn_dropout_keep(uint64_t dropout_seed, float dropout_p, int32_t b, int32_t h, int32_t H, int32_t i, int32_t j);
 
-/* Copies `rows` rows of n elements (of 1 or 4 bytes) to rows `pitch` elements apart, zeros behind each; a pitch of whole
- * 16-byte pieces, dst 16-byte aligned.  Enqueued on `stream`. */
+/* Copies `rows` rows of n elements (bytes, or floats) to rows `pitch` elements apart, zeros behind each; a pitch of whole
+ * 16-byte pieces, dst 16-byte aligned.  Finite floats beyond +-2.3e38 (a mask by the lowest value) become +-2.3e38.  Enqueued
+ * on `stream`. */
 int hstu_attn_pad_rows(const void* src, void* dst, int64_t rows, int32_t n, int32_t pitch, int32_t element_bytes, void* stream);
 
 /* ABI version of the loaded library (HSTU_ATTN_ABI_VERSION at build time). */

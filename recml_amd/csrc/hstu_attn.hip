@@ -5643,7 +5643,15 @@ __global__ __launch_bounds__(256) void hstu_pad_rows(const T* __restrict__ src, 
     const T* s = src + row * n;
     T v[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) v[i] = c + i < n ? s[c + i] : (T)0;
+    for (int i = 0; i < PER; ++i) {
+      v[i] = c + i < n ? s[c + i] : (T)0;
+      if constexpr (sizeof(T) == 4) {
+        // A bias of a float's lowest value is a mask.  The matrix-core kernels scale it by log2(e), past which it would be infinite and its
+        // weight NaN; the general kernels, whose calls these are, take it as it is.
+        const float a = __builtin_fabsf(v[i]);
+        v[i] = a > 2.3e38f && a < __builtin_inff() ? __builtin_copysignf(2.3e38f, v[i]) : v[i];
+      }
+    }
     *(uint4*)(dst + row * pitch + c) = *(const uint4*)v;
   }
 }

@@ -82,3 +82,19 @@ def test_weights_of_longer_rows_keep_their_bits(gpu, L, d, with_mask, with_bias)
   here, general = err(*ts), err(*(_beside(t) for t in ts))
   assert here <= 1.02 * general, (here, general)
 
+
+@pytest.mark.parametrize("d", [32, 128])
+def test_a_mask_by_the_lowest_value(gpu, d):
+  """A bias of finfo.min where a pair is not to count: weights of exactly 0, and gradients of 0, not NaN."""
+  rng = np.random.default_rng(d)
+  B, L, H = 2, 131, 2
+  q, k, v, dout = (_dev(O.round_bf16(rng.standard_normal((B, L, H, d)).astype(np.float32) * 0.4), bf) for _ in range(4))
+  mask = rng.random((B, L, L)) > 0.3
+  low = _dev(np.where(mask, 0.0, np.finfo(np.float32).min).astype(np.float32)).requires_grad_(True)
+  grads = []
+  for bias, m in ((low, None), (torch.zeros_like(low).requires_grad_(True), _dev(mask))):
+    ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    out = recml_amd.hstu_attention_autograd(*ts, n=float(L), causal=False, mask=m, bias=bias)
+    grads.append([out.detach(), *torch.autograd.grad(out, [*ts, bias], dout)])
+  for a, b in zip(*grads):
+    assert a.isfinite().all() and (a.float() - b.float()).norm() <= 2.0 ** -8 * b.float().norm()
