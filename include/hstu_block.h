@@ -7,8 +7,8 @@
  *                         the normalised input with their activation
  *                         (hstu.py:444-449, the EinsumDense layers of :281-330
  *                         with activation="silu"), as ONE matrix product with
- *                         the activation applied by the product's epilogue
- *                         (hipBLASLt) instead of a pass of its own.
+ *                         the activation in its epilogue instead of a pass of
+ *                         its own (hstu_gemm's kernels).
  *   hstu_norm_gate_fwd    out = u * layer_norm(attn): the layer norm over
  *                         (heads, head_dim) of the attention output and the U
  *                         gate (hstu.py:471-472) in one pass over memory.
@@ -49,7 +49,7 @@ typedef enum HstuBlockStatus {
   HSTU_BLOCK_ERR_SHAPE = -4,
   HSTU_BLOCK_ERR_WORKSPACE = -5,
   HSTU_BLOCK_ERR_LAUNCH = -6,
-  HSTU_BLOCK_ERR_BLAS = -7      /* hipBLASLt has no kernel for the request, or failed */
+  HSTU_BLOCK_ERR_BLAS = -7      /* no longer returned (the products were a library's once) */
 } HstuBlockStatus;
 
 /* out[t, :] = u[t, :] * (gamma * (a[t, :] - mean_t) * rstd_t + beta), mean and
@@ -123,12 +123,11 @@ int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* args, void* stream);
 /* out[m, n] = silu(sum_k x[m, k] w[k, n] + bias[n]); x: bf16 [M, K] (row stride
  * x_stride), w: bf16 [K, N] contiguous, bias: bf16 [N] or null, out: bf16
  * [M, N] contiguous; with `c` (bf16 [M, N], row stride c_stride, 16-byte aligned,
- * c_stride a multiple of 8) out = act(x w + c + bias).  fp32 accumulation.  `workspace` (device memory, may be
- * null) is handed to hipBLASLt; hstu_gemm_silu_workspace_bytes() says how much
- * it would like.  The descriptor and the chosen algorithm of a shape are kept
- * by the library after the first call with it: every call must therefore offer
- * what the first did, so x, w, bias, out and workspace must be 16-byte aligned
- * and x_stride a multiple of 8 elements (HSTU_BLOCK_ERR_SHAPE otherwise). */
+ * c_stride a multiple of 8) out = act(x w + c + bias).  fp32 accumulation, one
+ * rounding.  x, w, bias, out and workspace must be 16-byte aligned and x_stride
+ * a multiple of 8 elements (HSTU_BLOCK_ERR_SHAPE otherwise); N and K multiples
+ * of 8 run on the matrix cores, others element by element.  `workspace` is not
+ * used and may be null. */
 typedef struct HstuGemmSiluArgs {
   uint32_t struct_size;   /* sizeof(HstuGemmSiluArgs)  */
   uint32_t version;       /* HSTU_BLOCK_ABI_VERSION    */

@@ -135,7 +135,7 @@ def load():
       return _lib
     if not os.path.exists(LIB_PATH):
       raise RuntimeError(
-          f"{LIB_PATH} is missing: build it with `python -m recml_amd.build` (needs hipcc and hipBLASLt)")
+          f"{LIB_PATH} is missing: build it with `python -m recml_amd.build` (needs hipcc)")
     lib = C.CDLL(LIB_PATH)
     lib.hstu_block_abi_version.restype = C.c_int
     lib.hstu_block_abi_version.argtypes = []

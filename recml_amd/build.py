@@ -11,10 +11,9 @@ ROOT = os.path.dirname(_HERE)
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libhstu_attn.so")
 SOURCES = [os.path.join(_HERE, "csrc", "hstu_attn.hip"), os.path.join(_HERE, "csrc", "hstu_f32.hip")]
-# the block-side steps live in a library of their own: they bring hipBLASLt along, the attention does not
+# the block-side steps live in a library of their own
 BLOCK_LIB_PATH = os.path.join(LIB_DIR, "libhstu_block.so")
 BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip"), os.path.join(_HERE, "csrc", "hstu_gemm.hip")]
-BLOCK_LINK = ["-lhipblaslt"]
 INCLUDE = os.path.join(ROOT, "include")
 # the block's microbenchmark: a stand-alone program (its own main), evidence for what bounds the kernel
 MICRO_PATH = os.path.join(LIB_DIR, "micro_fwd_stream")
@@ -40,10 +39,10 @@ def hipcc() -> str:
   return exe
 
 
-def _compile(sources, out, link=(), verbose=False) -> str:
+def _compile(sources, out, verbose=False) -> str:
   os.makedirs(LIB_DIR, exist_ok=True)
   tmp = out + ".tmp"
-  cmd = [hipcc(), *HIPCC_FLAGS, "-I", INCLUDE, "-o", tmp, *sources, *link]
+  cmd = [hipcc(), *HIPCC_FLAGS, "-I", INCLUDE, "-o", tmp, *sources]
   res = subprocess.run(cmd, capture_output=True, text=True)
   if res.returncode != 0:
     raise RuntimeError("hipcc failed:\n" + res.stdout + res.stderr)
@@ -60,7 +59,7 @@ def build_library(verbose: bool = False) -> str:
 
 def build_block_library(verbose: bool = False) -> str:
   """Compiles the block-side steps into recml_amd/lib/libhstu_block.so."""
-  return _compile(BLOCK_SOURCES, BLOCK_LIB_PATH, BLOCK_LINK, verbose=verbose)
+  return _compile(BLOCK_SOURCES, BLOCK_LIB_PATH, verbose=verbose)
 
 
 def build_native(verbose: bool = False) -> str:

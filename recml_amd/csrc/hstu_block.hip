@@ -8,22 +8,15 @@
 //   hstu_norm_gate_bwd  the gradients of that step (and, without a gate, of a plain layer norm): one
 //                    pass over the row, its gradient and the gate; column sums for dgamma / dbeta in
 //                    registers, one partial row per workgroup, added in a fixed order by hstu_colsum.
-//   gemm + silu      out = silu(x W + bias)       (hstu.py:444-449)
-//                    hipBLASLt matrix product with the activation in its epilogue.
 //   hstu_embed_norm  out = layer_norm(scale * table[ids] + pos_table[positions])   (hstu.py:593-601)
 //                    the same one-wave-per-row scheme with a gathered row: one read of the table row
 //                    (and of the small position table, which stays in cache), one write.
 
 #include <hip/hip_runtime.h>
-#include <hipblaslt/hipblaslt.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
-
-#include <map>
-#include <mutex>
-#include <tuple>
 
 #include "hstu_block.h"
 #include "hstu_block_common.h"
@@ -39,6 +32,8 @@ int block_fail(int code, const char* fmt, ...) {
   va_end(ap);
   return code;
 }
+
+void block_clear_error() { g_err[0] = 0; }
 
 int block_allow_lds(const void* fn, int bytes, int* granted) {
   constexpr int kMaxDev = 64;
@@ -763,41 +758,6 @@ __global__ __launch_bounds__(256) void hstu_silu_bwd_kernel(bf16_t* d, const bf1
   *(uint4*)(d + row * d_stride + e) = pack8(x);
 }
 
-// ---- hipBLASLt side -------------------------------------------------------
-
-constexpr size_t kBlasWorkspace = 32u << 20;
-
-struct GemmPlan {
-  hipblasLtMatmulDesc_t desc = nullptr;
-  hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, lc = nullptr, lres = nullptr;   // lres: the C operand when it is not the output
-  hipblasLtMatmulAlgo_t algo;
-  size_t workspace = 0;
-};
-
-struct BlasState {
-  std::mutex mu;
-  hipblasLtHandle_t handle[64] = {};
-  // (device, M, N, K, x_stride, bias?, activation, workspace offered, row stride of c or 0) -> plan
-  std::map<std::tuple<int, int64_t, int, int, int64_t, int, int, size_t, int64_t>, GemmPlan> plans;
-};
-
-BlasState& blas() {
-  static BlasState s;
-  return s;
-}
-
-const char* blas_str(hipblasStatus_t st) {
-  switch (st) {
-    case HIPBLAS_STATUS_SUCCESS: return "success";
-    case HIPBLAS_STATUS_NOT_INITIALIZED: return "not initialized";
-    case HIPBLAS_STATUS_ALLOC_FAILED: return "allocation failed";
-    case HIPBLAS_STATUS_INVALID_VALUE: return "invalid value";
-    case HIPBLAS_STATUS_NOT_SUPPORTED: return "not supported";
-    case HIPBLAS_STATUS_EXECUTION_FAILED: return "execution failed";
-    default: return "error";
-  }
-}
-
 }  // namespace
 
 extern "C" {
@@ -1028,136 +988,6 @@ int hstu_silu_bwd(void* d, int64_t d_stride, const void* pre, int64_t pre_stride
                      d_stride, pre_stride);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "silu backward launch: %s", hipGetErrorString(e));
-  return HSTU_BLOCK_OK;
-}
-
-size_t hstu_gemm_silu_workspace_bytes(void) { return kBlasWorkspace; }
-
-int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
-  HstuGemmSiluArgs own;
-  a = block_today(a, own, sizeof(HstuGemmSiluArgs), sizeof(HstuGemmSiluArgs));
-  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
-  if (a->struct_size != sizeof(HstuGemmSiluArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
-    return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
-                a->struct_size, a->version, sizeof(HstuGemmSiluArgs), HSTU_BLOCK_ABI_VERSION);
-  if (a->M < 0 || a->N < 1 || a->K < 1 || a->M > 0x7fffffffLL || a->x_stride < a->K)
-    return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad shape M=%lld N=%d K=%d x_stride=%lld", (long long)a->M, a->N, a->K, (long long)a->x_stride);
-  if (a->activation != 0 && a->activation != 1) return block_fail(HSTU_BLOCK_ERR_SHAPE, "activation must be 0 (none) or 1 (silu)");
-  g_err[0] = 0;
-  if (a->M == 0) return HSTU_BLOCK_OK;
-  if (!a->x || !a->w || !a->out) return block_fail(HSTU_BLOCK_ERR_NULL, "x, w and out must be non-null");
-  // the kernel picked for a shape is kept and reused for every later call of that shape: it may assume what
-  // the first call's pointers offered, so every call has to offer it
-  if (!block_aligned16(a->x) || !block_aligned16(a->w) || !block_aligned16(a->out) || !block_aligned16(a->bias) || !block_aligned16(a->workspace) || (a->x_stride & 7))
-    return block_fail(HSTU_BLOCK_ERR_SHAPE, "x, w, out, bias and workspace must be 16-byte aligned and x_stride a multiple of 8 elements");
-  if (a->c && (!block_aligned16(a->c) || (a->c_stride & 7) || a->c_stride < a->N))
-    return block_fail(HSTU_BLOCK_ERR_SHAPE, "c must be 16-byte aligned with a row stride that is a multiple of 8 elements and >= N");
-  if (a->workspace_bytes && !a->workspace) return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace_bytes without a workspace");
-  int dev = 0;
-  hipError_t he = hipGetDevice(&dev);
-  if (he != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(he));
-  if (dev < 0 || dev >= 64) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "device index %d out of range", dev);
-
-  BlasState& bs = blas();
-  GemmPlan plan;
-  hipblasLtHandle_t handle;
-  {
-    std::lock_guard<std::mutex> lock(bs.mu);
-    if (!bs.handle[dev]) {
-      const hipblasStatus_t st = hipblasLtCreate(&bs.handle[dev]);
-      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtCreate: %s", blas_str(st));
-    }
-    handle = bs.handle[dev];
-    const auto key = std::make_tuple(dev, a->M, a->N, a->K, a->x_stride, a->bias ? 1 : 0, a->activation, a->workspace_bytes,
-                                     a->c ? a->c_stride : (int64_t)0);
-    auto it = bs.plans.find(key);
-    if (it == bs.plans.end()) {
-      // row-major out[M, N] = x[M, K] w[K, N] is, in the column-major terms of the library,
-      // out^T [N x M] = w^T [N x K] x^T [K x M] with leading dimensions N, x_stride and N
-      // (built in a holder that frees whatever exists of the plan on every early return)
-      struct Partial {
-        GemmPlan p{};
-        hipblasLtMatmulPreference_t pref = nullptr;
-        bool keep = false;
-        ~Partial() {
-          if (pref) hipblasLtMatmulPreferenceDestroy(pref);
-          if (keep) return;
-          if (p.la) hipblasLtMatrixLayoutDestroy(p.la);
-          if (p.lb) hipblasLtMatrixLayoutDestroy(p.lb);
-          if (p.lc) hipblasLtMatrixLayoutDestroy(p.lc);
-          if (p.lres) hipblasLtMatrixLayoutDestroy(p.lres);
-          if (p.desc) hipblasLtMatmulDescDestroy(p.desc);
-        }
-      } part;
-      GemmPlan& np = part.p;
-      hipblasStatus_t st = hipblasLtMatmulDescCreate(&np.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F);
-      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescCreate: %s", blas_str(st));
-      // every attribute is checked: a rejected epilogue or bias type would otherwise come back as "no kernel",
-      // or as a product without its epilogue
-      auto set_desc = [&](hipblasLtMatmulDescAttributes_t attr, const void* val, size_t bytes) {
-        return hipblasLtMatmulDescSetAttribute(np.desc, attr, val, bytes);
-      };
-      const hipblasOperation_t op_n = HIPBLAS_OP_N;
-      st = set_desc(HIPBLASLT_MATMUL_DESC_TRANSA, &op_n, sizeof(op_n));
-      if (st == HIPBLAS_STATUS_SUCCESS) st = set_desc(HIPBLASLT_MATMUL_DESC_TRANSB, &op_n, sizeof(op_n));
-      hipblasLtEpilogue_t epi = HIPBLASLT_EPILOGUE_DEFAULT;
-      if (a->activation == 1) epi = a->bias ? HIPBLASLT_EPILOGUE_SWISH_BIAS_EXT : HIPBLASLT_EPILOGUE_SWISH_EXT;
-      else if (a->bias) epi = HIPBLASLT_EPILOGUE_BIAS;
-      if (st == HIPBLAS_STATUS_SUCCESS) st = set_desc(HIPBLASLT_MATMUL_DESC_EPILOGUE, &epi, sizeof(epi));
-      if (st == HIPBLAS_STATUS_SUCCESS && a->bias) {
-        const hipDataType bt = HIP_R_16BF;
-        st = set_desc(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &bt, sizeof(bt));
-        // the heuristic looks at the pointer's presence; the real one is set on every call below
-        if (st == HIPBLAS_STATUS_SUCCESS) st = set_desc(HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &a->bias, sizeof(void*));
-      }
-      if (st != HIPBLAS_STATUS_SUCCESS)
-        return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (epilogue %d, bias %d): %s", (int)epi, a->bias ? 1 : 0, blas_str(st));
-      st = hipblasLtMatrixLayoutCreate(&np.la, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->K, (int64_t)a->N);
-      if (st == HIPBLAS_STATUS_SUCCESS) st = hipblasLtMatrixLayoutCreate(&np.lb, HIP_R_16BF, (uint64_t)a->K, (uint64_t)a->M, a->x_stride);
-      if (st == HIPBLAS_STATUS_SUCCESS) st = hipblasLtMatrixLayoutCreate(&np.lc, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->M, (int64_t)a->N);
-      if (st == HIPBLAS_STATUS_SUCCESS && a->c)
-        st = hipblasLtMatrixLayoutCreate(&np.lres, HIP_R_16BF, (uint64_t)a->N, (uint64_t)a->M, a->c_stride);
-      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatrixLayoutCreate: %s", blas_str(st));
-      st = hipblasLtMatmulPreferenceCreate(&part.pref);
-      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceCreate: %s", blas_str(st));
-      const uint64_t ws = a->workspace_bytes;
-      st = hipblasLtMatmulPreferenceSetAttribute(part.pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws));
-      if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulPreferenceSetAttribute: %s", blas_str(st));
-      hipblasLtMatmulHeuristicResult_t res[1];
-      int found = 0;
-      st = hipblasLtMatmulAlgoGetHeuristic(handle, np.desc, np.la, np.lb, a->c ? np.lres : np.lc, np.lc, part.pref, 1, res, &found);
-      if (st != HIPBLAS_STATUS_SUCCESS || found < 1)
-        return block_fail(HSTU_BLOCK_ERR_BLAS, "hipBLASLt has no kernel for M=%lld N=%d K=%d with this epilogue (%s)",
-                    (long long)a->M, a->N, a->K, blas_str(st));
-      np.algo = res[0].algo;
-      np.workspace = res[0].workspaceSize;
-      if (bs.plans.size() >= 256) {
-        for (auto& kv : bs.plans) {
-          hipblasLtMatrixLayoutDestroy(kv.second.la);
-          hipblasLtMatrixLayoutDestroy(kv.second.lb);
-          hipblasLtMatrixLayoutDestroy(kv.second.lc);
-          if (kv.second.lres) hipblasLtMatrixLayoutDestroy(kv.second.lres);
-          hipblasLtMatmulDescDestroy(kv.second.desc);
-        }
-        bs.plans.clear();
-      }
-      it = bs.plans.emplace(key, np).first;
-      part.keep = true;
-    }
-    plan = it->second;
-    // the descriptor is shared by every call of this shape: the bias pointer is set under the lock
-    // and the product is enqueued before it is released
-    if (a->bias) {
-      const hipblasStatus_t sb = hipblasLtMatmulDescSetAttribute(plan.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &a->bias, sizeof(void*));
-      if (sb != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmulDescSetAttribute (bias pointer): %s", blas_str(sb));
-    }
-    // (with c: D = alpha A B + beta C with C = c and beta = 1, the output written elsewhere)
-    const float alpha = 1.0f, beta = a->c ? 1.0f : 0.0f;
-    const hipblasStatus_t st = hipblasLtMatmul(handle, plan.desc, &alpha, a->w, plan.la, a->x, plan.lb, &beta, a->c ? a->c : a->out,
-                                               a->c ? plan.lres : plan.lc, a->out, plan.lc, &plan.algo, a->workspace, a->workspace_bytes,
-                                               (hipStream_t)stream);
-    if (st != HIPBLAS_STATUS_SUCCESS) return block_fail(HSTU_BLOCK_ERR_BLAS, "hipblasLtMatmul: %s", blas_str(st));
-  }
   return HSTU_BLOCK_OK;
 }
 

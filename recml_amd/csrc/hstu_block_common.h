@@ -12,6 +12,7 @@
 
 // Stores the message that hstu_block_last_error() returns on this thread; returns `code`.
 __attribute__((visibility("hidden"))) int block_fail(int code, const char* fmt, ...);
+__attribute__((visibility("hidden"))) void block_clear_error();
 // Raises the dynamic-LDS limit of a kernel, once per device (`granted`: 64 entries of the caller).
 __attribute__((visibility("hidden"))) int block_allow_lds(const void* fn, int bytes, int* granted);
 

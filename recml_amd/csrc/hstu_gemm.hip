@@ -493,9 +493,101 @@ int pick_splits(int64_t rows, int64_t cols, int64_t depth, int* tile) {
   return (int)s;
 }
 
+// out = act(x w + c + bias) for widths that the kernel above cannot fetch 16 bytes at a time: element by element, fp32 products.  (One
+// workgroup per 64 x 64 outputs, 16 of the contraction at a time through LDS, 4 x 4 outputs per thread.)
+struct PlainParams {
+  const bf16_t *x, *w, *bias, *c;
+  bf16_t* out;
+  int64_t x_stride, c_stride;
+  int32_t M, N, K, activation, col_tiles;
+};
+__global__ __launch_bounds__(256) void hstu_gemm_plain(const PlainParams p) {
+  __shared__ float xs[16][65], ws[16][65];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int m0 = (int)(blockIdx.x / p.col_tiles) * 64, n0 = (int)(blockIdx.x % p.col_tiles) * 64;
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < p.K; k0 += 16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = tid + 256 * i;
+      const int xr = e >> 4, xk = e & 15, wk = e >> 6, wc = e & 63;
+      xs[xk][xr] = m0 + xr < p.M && k0 + xk < p.K ? (float)p.x[(int64_t)(m0 + xr) * p.x_stride + k0 + xk] : 0.f;
+      ws[wk][wc] = n0 + wc < p.N && k0 + wk < p.K ? (float)p.w[(int64_t)(k0 + wk) * p.N + n0 + wc] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(xs[k][ty + 16 * i], ws[k][tx + 16 * j], acc[i][j]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int m = m0 + ty + 16 * i, n = n0 + tx + 16 * j;
+      if (m < p.M && n < p.N) {
+        float v = acc[i][j];
+        if (p.c) v += (float)p.c[(int64_t)m * p.c_stride + n];
+        if (p.bias) v += (float)p.bias[n];
+        p.out[(int64_t)m * p.N + n] = (bf16_t)(p.activation ? silu(v) : v);
+      }
+    }
+}
+
 }  // namespace
 
 extern "C" {
+
+// (nothing is needed; callers that ask are given a size they can allocate)
+size_t hstu_gemm_silu_workspace_bytes(void) { return 256; }
+
+int hstu_gemm_silu_fwd(const HstuGemmSiluArgs* a, void* stream) {
+  HstuGemmSiluArgs own;
+  a = block_today(a, own, sizeof(HstuGemmSiluArgs), sizeof(HstuGemmSiluArgs));
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (a->struct_size != sizeof(HstuGemmSiluArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)",
+                      a->struct_size, a->version, sizeof(HstuGemmSiluArgs), HSTU_BLOCK_ABI_VERSION);
+  if (a->M < 0 || a->N < 1 || a->K < 1 || a->M > 0x7fffffffLL || a->x_stride < a->K)
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad shape M=%lld N=%d K=%d x_stride=%lld", (long long)a->M, a->N, a->K, (long long)a->x_stride);
+  if (a->activation != 0 && a->activation != 1) return block_fail(HSTU_BLOCK_ERR_SHAPE, "activation must be 0 (none) or 1 (silu)");
+  block_clear_error();
+  if (a->M == 0) return HSTU_BLOCK_OK;
+  if (!a->x || !a->w || !a->out) return block_fail(HSTU_BLOCK_ERR_NULL, "x, w and out must be non-null");
+  if (!block_aligned16(a->x) || !block_aligned16(a->w) || !block_aligned16(a->out) || !block_aligned16(a->bias) || !block_aligned16(a->workspace) || (a->x_stride & 7))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "x, w, out, bias and workspace must be 16-byte aligned and x_stride a multiple of 8 elements");
+  if (a->c && (!block_aligned16(a->c) || (a->c_stride & 7) || a->c_stride < a->N))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "c must be 16-byte aligned with a row stride that is a multiple of 8 elements and >= N");
+  if (a->workspace_bytes && !a->workspace) return block_fail(HSTU_BLOCK_ERR_WORKSPACE, "workspace_bytes without a workspace");
+  constexpr int64_t PART = 1 << 28;              // rows of a launch: 32-bit indices
+  for (int64_t m0 = 0; m0 < a->M; m0 += PART) {
+    const int64_t rows = a->M - m0 < PART ? a->M - m0 : PART;
+    const bf16_t* x = (const bf16_t*)a->x + m0 * a->x_stride;
+    const bf16_t* c = a->c ? (const bf16_t*)a->c + m0 * a->c_stride : nullptr;
+    bf16_t* out = (bf16_t*)a->out + m0 * a->N;
+    if (a->N % 8 == 0 && a->K % 8 == 0) {
+      HstuGemmArgs g;
+      memset(&g, 0, sizeof(g));
+      g.struct_size = sizeof(g); g.version = HSTU_BLOCK_ABI_VERSION;
+      g.op = HSTU_GEMM_NN; g.activation = a->activation;
+      g.M = rows; g.N = a->N; g.K = a->K; g.slabs = 1;
+      g.x = x; g.x_stride = a->x_stride; g.w[0] = const_cast<void*>(a->w); g.bias = a->bias; g.c = c; g.c_stride = a->c_stride; g.out = out;
+      if (int rc = hstu_gemm(&g, stream)) return rc;
+      continue;
+    }
+    PlainParams p = {x, (const bf16_t*)a->w, (const bf16_t*)a->bias, c, out, a->x_stride, a->c_stride, (int32_t)rows, a->N, a->K, a->activation, 0};
+    p.col_tiles = (a->N + 63) / 64;
+    const int64_t blocks = (rows + 63) / 64 * p.col_tiles;
+    if (blocks > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "grid too large");
+    hipLaunchKernelGGL(hstu_gemm_plain, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
+  }
+  return HSTU_BLOCK_OK;
+}
 
 size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K) {
   if (op != HSTU_GEMM_TN || M < 1 || N < 1 || K < 1) return 0;

@@ -18,8 +18,6 @@ import torch
 from recml_amd import _lib_block
 from recml_amd import _native
 
-_workspaces = {}
-
 
 def _check(name, t, dtype=torch.bfloat16):
   if not isinstance(t, torch.Tensor) or not t.is_cuda:
@@ -203,12 +201,14 @@ def _vector(t):
 def gemm_silu(x, w, bias=None, activation: bool = True, residual=None):
   """silu(x @ w + bias) (or without the activation): x [M, K] bf16 (row stride free), w [K, N] contiguous,
   bias [N] or None -> [M, N] bf16.  `residual` [M, N] bf16 (row stride free) is added to the product as
-  its C operand, before bias and activation: the block's `+ inputs` without a pass (or a copy) of its own."""
+  its C operand, before bias and activation: the block's `+ inputs` without a pass (or a copy) of its own.
+  On the package's own kernels (74 k x 512 to 2048 columns: 257 us, hipBLASLt's product with the same epilogue 242; 20 k x 1024 to
+  4096: 187 and 168).  The library's product has faulted the GPU at 6400 x 2048 to 8192 and at 74 k x 1024 to 4096 columns."""
   _check("x", x)
   _check("w", w)
   if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[0]:
     raise ValueError(f"x [M, K] and w [K, N] expected, got {tuple(x.shape)} and {tuple(w.shape)}")
-  # the library wants 16-byte aligned operands and a row stride that keeps rows so
+  # the kernels want 16-byte aligned operands and a row stride that keeps rows so
   # (`contiguous()` returns a dense tensor as it is, misaligned or not: a view that starts off a 16-byte
   # boundary needs a copy of its own)
   if x.stride(1) != 1 or x.stride(0) % 8:
@@ -222,11 +222,6 @@ def gemm_silu(x, w, bias=None, activation: bool = True, residual=None):
   N = w.shape[1]
   out = torch.empty((M, N), dtype=x.dtype, device=x.device)
   lib = _lib_block.load()
-  key = (x.device.index, torch.cuda.current_stream(x.device).cuda_stream)
-  ws = _workspaces.get(key)
-  if ws is None:
-    ws = torch.empty(lib.hstu_gemm_silu_workspace_bytes(), dtype=torch.uint8, device=x.device)
-    _workspaces[key] = ws
   a = _lib_block.HstuGemmSiluArgs()
   a.struct_size, a.version = C.sizeof(_lib_block.HstuGemmSiluArgs), _lib_block.ABI_VERSION
   a.M, a.N, a.K, a.activation = M, N, K, 1 if activation else 0
@@ -239,7 +234,6 @@ def gemm_silu(x, w, bias=None, activation: bool = True, residual=None):
     if bias.data_ptr() % 16:
       bias = bias.clone()
     a.bias = bias.data_ptr()
-  a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
   if residual is not None:
     _check("residual", residual)
     if tuple(residual.shape) != (M, N):

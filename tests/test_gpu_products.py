@@ -103,3 +103,22 @@ def test_position_table_gradient(gpu, B, L, keys, width, by_position, packed):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + B * 2.0 ** -21).all()
   else:
     assert want.abs().max() < 256 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (5, 8, 7), (64, 20, 12), (65, 17, 65), (130, 40, 100)])
+@pytest.mark.parametrize("act", [False, True])
+def test_products_of_widths_that_are_no_multiple_of_8(gpu, M, K, N, act):
+  """Element by element, fp32 sums and one rounding: 2^-8 of the result, and 2^-20 of the terms' magnitudes for the sums' order."""
+  g = torch.Generator().manual_seed(M + N)
+  wide = torch.full((M, (K + 15) // 8 * 8), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+  wide[:, :K] = _normal(g, M, K)
+  x, w, bias = wide[:, :K], _normal(g, K, N), _normal(g, N)
+  res = torch.full((M, (N + 15) // 8 * 8), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+  res[:, :N] = _normal(g, M, N)
+  res = res[:, :N]
+  for b, r in ((None, None), (bias, None), (bias, res)):
+    want = x.double() @ w.double() + (0 if b is None else b.double()) + (0 if r is None else r.double())
+    size = x.double().abs() @ w.double().abs() + 2
+    want = torch.nn.functional.silu(want) if act else want
+    got = ops.gemm_silu(x, w, b, act, residual=r).double()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all()
