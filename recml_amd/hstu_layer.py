@@ -448,29 +448,37 @@ class HSTU(torch.nn.Module):
     elif seq_lens is None:
       if padding_mask is None:
         raise ValueError("Either `attention_mask`, `padding_mask` or `seq_lens` must be set.")
-      # (whether the mask is end-padded is asked when the work on it is enqueued: `ticket`)
+      # Whether the mask is end-padded is known once its kernel has run (`ticket`).  It is asked before anything random is drawn, in the
+      # packed form behind the packing's own wait, and otherwise when the first block is enqueued: the answer is there by then, where
+      # waiting for it first leaves a small batch's GPU idle (32 x 50 x 64, 4 blocks: 164 us a call, 133 this way).
       got = _native.mask_lengths(padding_mask)
       seq_lens, ticket = got if got is not None else (masks.lengths_from_padding_mask(padding_mask), None)
     if jagged:
-      out = self._forward_jagged(inputs, seq_lens, pos_bias, timestamps, ts_bias)
-    else:
-      x, outside = self._front_end(inputs)
-      # every block sees the same lengths, timestamps and tables: the attention prepares them once
-      batch = hstu_ops.AttentionBatch()
-      for block in self.decoder_blocks:
-        if attention_mask is not None:
-          x = block(x, attention_mask=attention_mask, batch=batch)
-        else:
-          x = block(x, seq_lens=seq_lens, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch)
-      out = self._final_norm(x)
-      if self.reverse_embedding is not None:
-        out = self._head(out)
-      self._check_indices(outside)
-    if ticket is not None and _native.raised(ticket):
-      raise ValueError(masks.NOT_END_PADDED)
+      return self._forward_jagged(inputs, seq_lens, pos_bias, timestamps, ts_bias, ticket)
+    if self.training and self.dropout > 0.0:
+      ticket = self._check_mask(ticket)
+    x, outside = self._front_end(inputs)
+    # every block sees the same lengths, timestamps and tables: the attention prepares them once
+    batch = hstu_ops.AttentionBatch()
+    for block in self.decoder_blocks:
+      if attention_mask is not None:
+        x = block(x, attention_mask=attention_mask, batch=batch)
+      else:
+        x = block(x, seq_lens=seq_lens, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch)
+      ticket = self._check_mask(ticket)
+    out = self._final_norm(x)
+    if self.reverse_embedding is not None:
+      out = self._head(out)
+    self._check_mask(ticket)
+    self._check_indices(outside)
     return out
 
-  def _forward_jagged(self, inputs, seq_lens, pos_bias, timestamps, ts_bias):
+  def _check_mask(self, ticket):
+    """Raises where the padding mask behind the ticket was not end-padded; there is nothing left to ask afterwards."""
+    if ticket is not None and _native.raised(ticket):
+      raise ValueError(masks.NOT_END_PADDED)
+
+  def _forward_jagged(self, inputs, seq_lens, pos_bias, timestamps, ts_bias, ticket):
     B, L = inputs.shape
     # which padded row each packed token comes from: found once (the one host wait of the packing: the token count) and used for
     # every gather and for the scatter at the end
@@ -485,6 +493,7 @@ class HSTU(torch.nn.Module):
       tokens = rows.numel()
     else:
       offsets, rows, tokens = got
+    self._check_mask(ticket)
     x, outside = self._front_end(inputs, rows, tokens)
     ts = None if timestamps is None else timestamps.reshape(-1).index_select(0, rows[:tokens])
     batch = hstu_ops.AttentionBatch()
