@@ -267,11 +267,8 @@ void sign(std::string& to, const Tensor& t) {
   for (int64_t i = 0; i < t.dim(); ++i) { put(t.size(i)); put(t.stride(i)); }
 }
 
-// The forward into `out`; false: the Python side takes the call (and reports what is wrong with it).
-bool forward_into(const Tensor& out, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pos, const Tensor& ts_tab, const Tensor& bias,
-                  Options& o, Shared* shared = nullptr) {
-  HstuAttnFwdArgs a;
-  if (!fill(a, q, k, v, out, pos, ts_tab, bias, o)) return false;
+// The forward that fill() has described; false: the Python side takes the call (and reports what is wrong with it).
+bool forward(HstuAttnFwdArgs& a, const Tensor& q, const Tensor& pos, const Tensor& ts_tab, const Tensor& bias, Options& o, Shared* shared = nullptr) {
   pad_dense(a, o, q);
   if (!shared) {
     const Tensor buf = scratch_for(a, q);
@@ -920,7 +917,8 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count) {
         const c10::DeviceGuard guard(q.device());
         const at::NoGradGuard no_grad;
         if (!out.defined()) out = like_output(q, v);
-        ok = forward_into(out, q, k, v, pos, ts_tab, bias, o);
+        HstuAttnFwdArgs a;
+        ok = fill(a, q, k, v, out, pos, ts_tab, bias, o) && forward(a, q, pos, ts_tab, bias, o);
       } catch (...) {
         PyEval_RestoreThread(saved);
         throw;
@@ -1013,16 +1011,16 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
       if (c.L) attn = fresh(tokens, {c.B, c.L, c.H, c.hd});
       else attn = fresh(tokens, {T, c.H, c.hd});
       // (a call whose attention the Python side has to take is found here, before any of its work)
-      HstuAttnFwdArgs probe;
-      if (!fill(probe, projection_slice(uqkv, c, 1), projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
+      HstuAttnFwdArgs a;
+      const Tensor q = projection_slice(uqkv, c, 1);
+      if (!fill(a, q, projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
       normed = fresh(tokens, {T, D});
       norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
       if (graph) pre = at::empty_like(uqkv);
       Tensor pb;
       if (p[P_UB].defined()) pb = at::cat({p[P_UB].view({W}), p[P_QB].view({W}), p[P_KB].view({W}), p[P_VB].view({W})});
       gemm(HSTU_GEMM_NN, T, {normed.const_data_ptr(), D}, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W, uqkv, pb, {nullptr, 0}, true, pre);
-      if (!forward_into(attn, projection_slice(uqkv, c, 1), projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), pos, ts_tab, bias, o,
-                        share ? &shared : nullptr)) return false;
+      if (!forward(a, q, pos, ts_tab, bias, o, share ? &shared : nullptr)) return false;
       gated = fresh(tokens, {T, W});
       norm(gated, {attn.const_data_ptr(), W}, {uqkv.const_data_ptr(), 4 * W}, p[P_ATTN_G], p[P_ATTN_B], T, W, c.eps);
       out = fresh(tokens, tokens.sizes());

@@ -262,11 +262,15 @@ class HSTUBlock(torch.nn.Module):
   def _weights(self):
     """The block's parameters as the native call takes them: whatever stands under their names (a parametrization or a pruning mask
     puts a tensor of its own there)."""
-    P = self._parameters
-    of = lambda name: P[name] if name in P else getattr(self, name)
-    biases = (of("u_bias"), of("q_bias"), of("k_bias"), of("v_bias")) if self.use_bias else (None,) * 4
-    return (of("input_ln_gamma"), of("input_ln_beta"), of("u_kernel"), of("q_kernel"), of("k_kernel"), of("v_kernel"), *biases,
-            of("attn_ln_gamma"), of("attn_ln_beta"), of("output_kernel"), of("output_bias") if self.use_bias else None)
+    try:
+      P = self._parameters               # (a module's attribute lookup costs four times the dictionary's)
+      biases = (P["u_bias"], P["q_bias"], P["k_bias"], P["v_bias"], P["output_bias"]) if self.use_bias else (None,) * 5
+      return (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], *biases[:4],
+              P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], biases[4])
+    except KeyError:
+      biases = (self.u_bias, self.q_bias, self.k_bias, self.v_bias, self.output_bias) if self.use_bias else (None,) * 5
+      return (self.input_ln_gamma, self.input_ln_beta, self.u_kernel, self.q_kernel, self.k_kernel, self.v_kernel, *biases[:4],
+              self.attn_ln_gamma, self.attn_ln_beta, self.output_kernel, biases[4])
 
   def _wants_grad(self, *tensors) -> bool:
     return _differentiates(*self._weights(), *tensors)
@@ -305,21 +309,29 @@ class HSTUBlock(torch.nn.Module):
     if grad and not (self._fused_training(tokens, pos_bias, ts_bias) and hstu_ops.hstu_attention_bwd is hstu_ops._OWN_ATTENTION_BWD
                      and hstu_block_ops.norm_gate_bwd is hstu_block_ops._OWN_NORM_GATE_BWD):
       return None
-    # (torch's default integers, 16-bit tables: converted here, by the first block of a batch for all of them; a table's conversion is
-    # part of the graph)
-    ready = _ready if batch is None else batch.ready
-    seq_lens, seq_offsets, timestamps = ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64)
-    pos_bias, ts_bias = (_ready(t, torch.float32) if grad else ready(t, torch.float32) for t in (pos_bias, ts_bias))
     alpha, n = self._alpha_n(length)
-    got = _native.block(tokens.contiguous(), weights, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
-                        None if seq_offsets is None else length, pos_bias, timestamps, ts_bias, attention_mask, attention_bias,
-                        drop.get("dropout_p", 0.0), drop.get("dropout_seed", 0),
-                        False if batch is None else batch._prepared, None if batch is None else batch._buf, grad)
+    given = (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias)
+
+    def call(seq_lens, seq_offsets, timestamps, pos_bias, ts_bias):
+      return _native.block(tokens.contiguous(), weights, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
+                           None if seq_offsets is None else length, pos_bias, timestamps, ts_bias, attention_mask, attention_bias,
+                           drop.get("dropout_p", 0.0), drop.get("dropout_seed", 0),
+                           False if batch is None else batch._prepared, None if batch is None else batch._buf, grad)
+
+    got = call(*given)
+    if got is None:
+      # (declined before any work.  torch's default integers, 16-bit tables: converted, by the first block of a batch for all of them; a
+      # table's conversion is part of the graph)
+      ready = _ready if batch is None else batch.ready
+      table = _ready if grad else ready
+      was, given = given, (ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64),
+                           table(pos_bias, torch.float32), table(ts_bias, torch.float32))
+      got = call(*given) if any(x is not y for x, y in zip(was, given)) else None
     if got is None:
       return None
     out, signature, workspace, reused = got
     if batch is not None:
-      batch._keep_native(signature, workspace, reused, (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias, attention_mask))
+      batch._keep_native(signature, workspace, reused, (*given, attention_mask))
     return out
 
   def _uqkv_weights(self):
