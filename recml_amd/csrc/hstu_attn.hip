@@ -4073,18 +4073,13 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           const int32_t* tk = Tk(st);
           float s_far = 0.f;
           s_near = 0.f;
-          auto add = [&](int key, float v) {
-            const bool far = key <= cut;
-            s_far += far ? v : 0.f;
-            s_near += far ? 0.f : v;
-          };
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
-            add(kk.x, ds[4 * g]);
-            add(kk.y, ds[4 * g + 1]);
-            add(kk.z, ds[4 * g + 2]);
-            add(kk.w, ds[4 * g + 3]);
+            const bool f0 = kk.x <= cut, f1 = kk.y <= cut, f2 = kk.z <= cut, f3 = kk.w <= cut;
+            const float *v = ds + 4 * g;
+            s_far += ((f0 ? v[0] : 0.f) + (f1 ? v[1] : 0.f)) + ((f2 ? v[2] : 0.f) + (f3 ? v[3] : 0.f));
+            s_near += ((f0 ? 0.f : v[0]) + (f1 ? 0.f : v[1])) + ((f2 ? 0.f : v[2]) + (f3 ? 0.f : v[3]));
           }
           if (sum_bucket == bk_lane + 1) sum_s += s_far;
           else if (s_far != 0.f) lds_atomic_add(&hist[bk_lane + 1], s_far);

@@ -262,15 +262,17 @@ class HSTUBlock(torch.nn.Module):
   def _weights(self):
     """The block's parameters as the native call takes them: whatever stands under their names (a parametrization or a pruning mask
     puts a tensor of its own there)."""
+    P = self._parameters                 # (a module's attribute lookup costs four times the dictionary's)
     try:
-      P = self._parameters               # (a module's attribute lookup costs four times the dictionary's)
-      biases = (P["u_bias"], P["q_bias"], P["k_bias"], P["v_bias"], P["output_bias"]) if self.use_bias else (None,) * 5
-      return (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], *biases[:4],
-              P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], biases[4])
+      if not self.use_bias:
+        return (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], None, None, None, None,
+                P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], None)
+      return (P["input_ln_gamma"], P["input_ln_beta"], P["u_kernel"], P["q_kernel"], P["k_kernel"], P["v_kernel"], P["u_bias"], P["q_bias"],
+              P["k_bias"], P["v_bias"], P["attn_ln_gamma"], P["attn_ln_beta"], P["output_kernel"], P["output_bias"])
     except KeyError:
-      biases = (self.u_bias, self.q_bias, self.k_bias, self.v_bias, self.output_bias) if self.use_bias else (None,) * 5
-      return (self.input_ln_gamma, self.input_ln_beta, self.u_kernel, self.q_kernel, self.k_kernel, self.v_kernel, *biases[:4],
-              self.attn_ln_gamma, self.attn_ln_beta, self.output_kernel, biases[4])
+      biases = (self.u_bias, self.q_bias, self.k_bias, self.v_bias) if self.use_bias else (None,) * 4
+      return (self.input_ln_gamma, self.input_ln_beta, self.u_kernel, self.q_kernel, self.k_kernel, self.v_kernel, *biases,
+              self.attn_ln_gamma, self.attn_ln_beta, self.output_kernel, self.output_bias if self.use_bias else None)
 
   def _wants_grad(self, *tensors) -> bool:
     return _differentiates(*self._weights(), *tensors)
@@ -310,28 +312,25 @@ class HSTUBlock(torch.nn.Module):
                      and hstu_block_ops.norm_gate_bwd is hstu_block_ops._OWN_NORM_GATE_BWD):
       return None
     alpha, n = self._alpha_n(length)
-    given = (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias)
-
-    def call(seq_lens, seq_offsets, timestamps, pos_bias, ts_bias):
-      return _native.block(tokens.contiguous(), weights, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
-                           None if seq_offsets is None else length, pos_bias, timestamps, ts_bias, attention_mask, attention_bias,
-                           drop.get("dropout_p", 0.0), drop.get("dropout_seed", 0),
-                           False if batch is None else batch._prepared, None if batch is None else batch._buf, grad)
-
-    got = call(*given)
+    got = _native.block(tokens.contiguous(), weights, self.num_heads, self.head_dim, self.eps, alpha, n, seq_lens, seq_offsets,
+                        None if seq_offsets is None else length, pos_bias, timestamps, ts_bias, attention_mask, attention_bias,
+                        drop.get("dropout_p", 0.0), drop.get("dropout_seed", 0),
+                        False if batch is None else batch._prepared, None if batch is None else batch._buf, grad)
     if got is None:
       # (declined before any work.  torch's default integers, 16-bit tables: converted, by the first block of a batch for all of them; a
       # table's conversion is part of the graph)
       ready = _ready if batch is None else batch.ready
       table = _ready if grad else ready
-      was, given = given, (ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64),
-                           table(pos_bias, torch.float32), table(ts_bias, torch.float32))
-      got = call(*given) if any(x is not y for x, y in zip(was, given)) else None
-    if got is None:
-      return None
+      given = seq_lens, seq_offsets, timestamps, pos_bias, ts_bias
+      seq_lens, seq_offsets, timestamps = ready(seq_lens, torch.int32), ready(seq_offsets, torch.int32), ready(timestamps, torch.int64)
+      pos_bias, ts_bias = table(pos_bias, torch.float32), table(ts_bias, torch.float32)
+      if all(x is y for x, y in zip(given, (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias))):
+        return None
+      return self._native_steps(tokens, length, batch, drop, pos_bias, timestamps, ts_bias, seq_lens, seq_offsets, attention_mask,
+                                attention_bias)
     out, signature, workspace, reused = got
     if batch is not None:
-      batch._keep_native(signature, workspace, reused, (*given, attention_mask))
+      batch._keep_native(signature, workspace, reused, (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias, attention_mask))
     return out
 
   def _uqkv_weights(self):
@@ -477,7 +476,8 @@ class HSTU(torch.nn.Module):
         x = block(x, attention_mask=attention_mask, batch=batch)
       else:
         x = block(x, seq_lens=seq_lens, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch)
-      ticket = self._check_mask(ticket)
+      if ticket is not None:
+        ticket = self._check_mask(ticket)
     out = self._final_norm(x)
     if self.reverse_embedding is not None:
       out = self._head(out)
