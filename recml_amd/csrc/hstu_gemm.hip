@@ -472,7 +472,9 @@ int64_t tiles_of(int64_t rows, int64_t cols, int tm, int tn) { return ((rows + t
 // per CU, whose loads cover the others' starts and stores.  Long contractions take the first (74 k x 2048 to 512 columns: 196 us
 // against 214), and so do short ones with tiles enough for six rounds over the chip (74 k x 512 to 2048 columns: 270 us against
 // 281; to 512 columns 76 against 68); products of few tiles go down to 64 x 64.  (256 x 256 with one wave per SIMD, 128 x 128
-// per wave: 310 and 220 us.)
+// per wave: 310 and 220 us.)  Both sides were timed before the loads of UNIFORM; with them the chosen tiles take 187 and 257 us.
+// Widths of 256 to 2048, 1.6 k to 131 k rows, with these lines in the library product's time: a projection 1.0 - 1.2, the output product
+// 1.4, input gradients 0.9 - 1.8, weight gradients 0.5 - 2.7 (the worst at 1.6 k rows x 1024 columns).
 int pick_tile(int64_t rows, int64_t cols, int64_t depth) {
   if (tiles_of(rows, cols, 256, 128) >= (depth >= 1024 ? 512 : 3072)) return 2;
   if (tiles_of(rows, cols, 128, 128) >= 384) return 1;
