@@ -23,7 +23,6 @@ typedef short short4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4v* lds_short4_ptr;
 
 constexpr int GEMM_BK = 32;          // contraction depth of a stage
-constexpr int GEMM_THREADS = 256;
 
 struct GemmParams {
   const bf16_t* q;                   // the operand of the output's rows
@@ -62,7 +61,15 @@ __device__ __forceinline__ const char* scalar_ptr(const void* p) {
 
 #define HSTU_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | ((((n) >> 4) & 3) << 14)) | 0x0F70)
 
-// One workgroup: a tile of 64 MB output rows x 64 NB output columns, four waves of 32 MB x 32 NB.  The contraction runs in
+// 16 bytes that this launch does not read again: not kept in this XCD's L2, where the operands are (the reader is a later launch,
+// on any XCD).  74 k x 512 -> 2048, out alone / with the pre-activation: 240 -> 213, 282 -> 226 us.
+__device__ __forceinline__ void store_past_cache(bf16_t* to, const uint4& v) {
+  typedef uint32_t words __attribute__((ext_vector_type(4)));
+  const words x = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(x, (words*)to);
+}
+
+// One workgroup: a tile of 64 MB output rows x 32 NB WN output columns, 2 x WN waves of 32 MB x 32 NB.  The contraction runs in
 // stages of 32 through a three-stage LDS ring filled by direct global -> LDS loads (two stages in flight, one barrier
 // per stage).  The product is formed transposed (columns as the matrix instruction's rows): a lane then holds four
 // consecutive columns of one output row.
@@ -70,18 +77,23 @@ __device__ __forceinline__ const char* scalar_ptr(const void* p) {
 // c ^ (r / 4 % 4): a fragment is one ds_read_b128 per lane, 16 rows reach all 64 banks.  One stored across it (x and dz in
 // the weight's gradient, the weight itself in the forward) lies as 32 rows of 128 columns, chunk c at c ^ 4 (r % 4), and is
 // transposed on the way out by ds_read_b64_tr_b16, two per fragment.
-//   Why 256 x 128 (MB 4, NB 2): with 64 x 64 per wave the four SIMDs' fragments take all of the LDS bandwidth (128 bytes a
-// clock) at full matrix rate, with 128 x 64 three quarters of it; 128 accumulators leave two workgroups per CU, so that one's
-// barriers and stores run under the other's products.
+//   Why 128 x 64 per wave (MB 4, NB 2): with 64 x 64 the four SIMDs' fragments take all of the LDS bandwidth (128 bytes a clock) at
+// full matrix rate, with 128 x 64 three quarters of it, and the direct loads' writes come on top: 72 KB per 512 clocks in a tile of
+// 256 x 128, 131 KB per 1024 in one of 256 x 256 (WN 4), whose main loop is the faster one (1290 against 1100 TFLOP/s over long
+// contractions); 256 x 128 leaves two workgroups per CU, so that one's stores run under the other's products.  Without its epilogue
+// 74 k x 512 -> 2048 takes 139 us, with it 194: the stores burst at a tile's end.
 //   UNIFORM: a tile's columns of P (a stage's, where P lies along the contraction) are in one slab.  A load is then a scalar base
 // that moves on with the stage and a lane offset that never changes; rows and columns past an operand's end repeat its last
 // (what they give is not stored), and only the stage that crosses the contraction's end tests its elements.  Per-lane
 // pointers, counters and slab hops were three of the ten vector instructions behind every matrix instruction.
-template <int MB, int NB, bool Q_T, bool P_T, int STAGES, bool UNIFORM>
-__global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmParams g) {
-  constexpr int TM = 64 * MB, TN = 64 * NB;
+//   OUT: what the epilogue does, known to the compiler where it is one of the products of a block: a branch between its steps keeps
+// it from ordering them across pieces (74 k x 512 -> 2048 with the activation 235 us, 194 without).
+enum { OUT_PLAIN, OUT_SILU, OUT_PRE_SILU, OUT_ADD, OUT_PARTIAL, OUT_ANY };
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT>
+__global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams g) {
+  constexpr int TM = 64 * MB, TN = 32 * NB * WN, WAVES = 2 * WN;
   constexpr int Q_BYTES = TM * GEMM_BK * 2, P_BYTES = TN * GEMM_BK * 2, STAGE = Q_BYTES + P_BYTES;
-  constexpr int LQ = Q_BYTES / 4096, LP = P_BYTES / 4096;      // direct loads of 1 KB per wave
+  constexpr int LQ = Q_BYTES / (1024 * WAVES), LP = P_BYTES / (1024 * WAVES);      // direct loads of 1 KB per wave
   static_assert(LQ >= 1 && LP >= 1, "a stage is at least one load per wave and operand");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const uint32_t smem_lds = __builtin_amdgcn_groupstaticsize();
@@ -94,12 +106,20 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmPa
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   int rt, ct, split = 0;
   if (g.splits > 1) {
+    // (fewer splits than XCDs, 2 or 4: each has 4 or 2 of them, which take its tiles in turn)
     const int per = g.row_tiles * g.col_tiles;
-    split = (j / per) * 8 + xcd;
-    const int t = j % per;
+    int t;
+    if (g.splits < 8) {
+      split = xcd & (g.splits - 1);
+      t = j * (8 / g.splits) + xcd / g.splits;
+      if (t >= per) return;
+    } else {
+      split = (j / per) * 8 + xcd;
+      t = j % per;
+      if (split >= g.splits) return;
+    }
     rt = t / g.col_tiles;
     ct = t - rt * g.col_tiles;
-    if (split >= g.splits) return;
   } else {
     rt = (j / g.col_tiles) * 8 + xcd;
     ct = j % g.col_tiles;
@@ -374,42 +394,68 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void hstu_gemm_kernel(const GemmPa
         *(float4*)(stage + l32 * PITCH + (32 * a + 8 * q4 + 4 * hh) * 4) = v;
       }
     __builtin_amdgcn_wave_barrier();
+    // (the steps below over all pieces of the block at a time: a piece by itself is a chain of dependent transcendentals with
+    // nothing beside it, 240 us where this takes 204 at 74 k x 512 -> 2048)
+    constexpr int PIECES = 32 / RPI;
+    float x[PIECES][8];
 #pragma unroll
-    for (int i = 0; i < 32 / RPI; ++i) {
-      const int row = RPI * i + rr;
-      const int m = m0 + wm * 32 * MB + 32 * b + row;
-      const float4 v0 = *(const float4*)(stage + row * PITCH + 32 * cc), v1 = *(const float4*)(stage + row * PITCH + 32 * cc + 16);
-      if (m < g.rows && n < g.cols) {
-        float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-        if (g.partial) {
-          float* o = g.partial + ((int64_t)split * g.rows + m) * g.cols + n;
-          *(float4*)o = v0;
-          *(float4*)(o + 4) = v1;
-        } else {
-          if (g.c) {
-            float cv[8];
-            unpack8(*(const uint4*)(g.c + (int64_t)m * g.c_stride + n), cv);
+    for (int i = 0; i < PIECES; ++i) {
+      const unsigned char* at = stage + (RPI * i + rr) * PITCH + 32 * cc;
+      const float4 v0 = *(const float4*)at, v1 = *(const float4*)(at + 16);
+      x[i][0] = v0.x; x[i][1] = v0.y; x[i][2] = v0.z; x[i][3] = v0.w;
+      x[i][4] = v1.x; x[i][5] = v1.y; x[i][6] = v1.z; x[i][7] = v1.w;
+    }
+    const int mb = m0 + wm * 32 * MB + 32 * b + rr;      // the lane's row of piece 0
+    auto inside = [&](int i) { return mb + RPI * i < g.rows && n < g.cols; };
+    if constexpr (OUT == OUT_PARTIAL) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] += cv[e];
-          }
-          if (g.bias) {
+      for (int i = 0; i < PIECES; ++i)
+        if (inside(i)) {
+          float* o = g.partial + ((int64_t)split * g.rows + mb + RPI * i) * g.cols + n;
+          *(float4*)o = float4{x[i][0], x[i][1], x[i][2], x[i][3]};
+          *(float4*)(o + 4) = float4{x[i][4], x[i][5], x[i][6], x[i][7]};
+        }
+    } else {
+      if (OUT == OUT_ADD || (OUT == OUT_ANY && g.c)) {
+        uint4 cr[PIECES];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] += bias[e];
-          }
-          bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)m * g.out_stride + (n - osl * g.out_slab);
-          if (g.pre) {
-            // (the activation of the stored value, which is what its gradient is taken at)
-            const uint4 z = pack8(x);
-            *(uint4*)(g.pre + (int64_t)m * g.out_stride + n) = z;
-            unpack8(z, x);
-          }
-          if (g.activation) {
+        for (int i = 0; i < PIECES; ++i) {
+          cr[i] = uint4{0u, 0u, 0u, 0u};
+          if (inside(i)) cr[i] = *(const uint4*)(g.c + (int64_t)(mb + RPI * i) * g.c_stride + n);
+        }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = silu(x[e]);
-          }
-          *(uint4*)o = pack8(x);
+        for (int i = 0; i < PIECES; ++i) {
+          float cv[8];
+          unpack8(cr[i], cv);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[i][e] += cv[e];
         }
       }
+      if (!Q_T && P_T) {        // (zeros without one)
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[i][e] += bias[e];
+      }
+      if (OUT == OUT_PRE_SILU || (OUT == OUT_ANY && g.pre)) {
+        // (the activation of the stored value, which is what its gradient is taken at)
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+          const uint4 z = pack8(x[i]);
+          if (inside(i)) store_past_cache(g.pre + (int64_t)(mb + RPI * i) * g.out_stride + n, z);
+          unpack8(z, x[i]);
+        }
+      }
+      if (OUT == OUT_SILU || OUT == OUT_PRE_SILU || (OUT == OUT_ANY && g.activation)) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[i][e] = silu(x[i][e]);
+      }
+      bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)mb * g.out_stride + (n - osl * g.out_slab);
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i)
+        if (inside(i)) store_past_cache(o + (int64_t)(RPI * i) * g.out_stride, pack8(x[i]));
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -431,68 +477,105 @@ __global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
   *(uint4*)o = pack8(x);
 }
 
-template <int MB, int NB, bool Q_T, bool P_T, int STAGES, bool UNIFORM>
-int launch_as(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT>
+int launch_out(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
   static int granted[64];
-  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES, UNIFORM>, smem, granted)) return rc;
-  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, Q_T, P_T, STAGES, UNIFORM>), dim3(blocks), dim3(GEMM_THREADS), smem, st, g);
+  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT>), dim3(blocks), dim3(128 * WN), smem, st, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 
-template <int MB, int NB, bool Q_T, bool P_T, int STAGES = 3>
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM>
+int launch_as(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
+  if constexpr (Q_T) {
+    if (g.partial) return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_PARTIAL>(g, blocks, smem, st);
+  } else if constexpr (P_T) {
+    if constexpr (UNIFORM) {
+      if (!g.c && !g.pre && g.activation) return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_SILU>(g, blocks, smem, st);
+      if (!g.c && g.pre && g.activation) return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_PRE_SILU>(g, blocks, smem, st);
+      if (g.c && !g.pre && !g.activation) return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_ADD>(g, blocks, smem, st);
+    }
+    if (g.c || g.pre || g.activation) return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_ANY>(g, blocks, smem, st);
+  }
+  return launch_out<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT_PLAIN>(g, blocks, smem, st);
+}
+
+// One slab per tile (per stage, along the contraction); lane offsets within 32 bits.
+bool uniform(const GemmParams& g, bool p_t, int tm, int tn) {
+  const bool one_slab = p_t ? (g.slab >= g.cols || g.slab % tn == 0) : g.slab % GEMM_BK == 0;
+  const int64_t widest = (int64_t)(tm > tn ? tm : tn) * (g.q_stride > g.p_stride ? g.q_stride : g.p_stride) * 2;
+  return one_slab && widest < (1LL << 31);
+}
+
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES = 3>
 int launch(const GemmParams& p, hipStream_t st) {
-  constexpr int TM = 64 * MB, TN = 64 * NB;
-  constexpr int ring = STAGES * (TM + TN) * GEMM_BK * 2, out = 4 * 32 * (32 * NB * 4 + 16);
+  constexpr int TM = 64 * MB, TN = 32 * NB * WN;
+  constexpr int ring = STAGES * (TM + TN) * GEMM_BK * 2, out = 2 * WN * 32 * (32 * NB * 4 + 16);
   constexpr int smem = ring > out ? ring : out;
   GemmParams g = p;
   g.row_tiles = (g.rows + TM - 1) / TM;
   g.col_tiles = (g.cols + TN - 1) / TN;
   const int64_t tiles = (int64_t)g.row_tiles * g.col_tiles;
-  const int64_t blocks = g.splits > 1 ? 8LL * ((g.splits + 7) / 8) * tiles : 8LL * ((g.row_tiles + 7) / 8) * g.col_tiles;
+  const int64_t blocks = g.splits >= 8 ? 8LL * ((g.splits + 7) / 8) * tiles
+                         : g.splits > 1 ? 8LL * ((tiles * g.splits + 7) / 8) : 8LL * ((g.row_tiles + 7) / 8) * g.col_tiles;
   if (blocks > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "grid too large");
-  // one slab per tile (per stage, along the contraction); lane offsets within 32 bits
-  const bool one_slab = P_T ? (g.slab >= g.cols || g.slab % TN == 0) : g.slab % GEMM_BK == 0;
-  const int64_t widest = (int64_t)(TM > TN ? TM : TN) * (g.q_stride > g.p_stride ? g.q_stride : g.p_stride) * 2;
-  if (one_slab && widest < (1LL << 31)) return launch_as<MB, NB, Q_T, P_T, STAGES, true>(g, (unsigned)blocks, smem, st);
-  return launch_as<MB, NB, Q_T, P_T, STAGES, false>(g, (unsigned)blocks, smem, st);
+  if (uniform(g, P_T, TM, TN)) return launch_as<MB, NB, WN, Q_T, P_T, STAGES, true>(g, (unsigned)blocks, smem, st);
+  if constexpr (WN == 4) return launch<4, 2, 2, Q_T, P_T>(p, st);
+  else return launch_as<MB, NB, WN, Q_T, P_T, STAGES, false>(g, (unsigned)blocks, smem, st);
 }
 
 template <bool Q_T, bool P_T>
 int launch_sized(const GemmParams& p, hipStream_t st, int tile) {
-  if (tile == 2) return launch<4, 2, Q_T, P_T>(p, st);
-  if (tile == 1) return launch<2, 2, Q_T, P_T>(p, st);
-  return launch<1, 1, Q_T, P_T>(p, st);
+  if (tile == 3) return launch<4, 2, 4, Q_T, P_T>(p, st);
+  if (tile == 2) return launch<4, 2, 2, Q_T, P_T>(p, st);
+  if (tile == 1) return launch<2, 2, 2, Q_T, P_T>(p, st);
+  return launch<1, 1, 2, Q_T, P_T>(p, st);
 }
 
 int64_t tiles_of(int64_t rows, int64_t cols, int tm, int tn) { return ((rows + tm - 1) / tm) * ((cols + tn - 1) / tn); }
 
-// The tile of a product: 256 x 128 has the most products per byte of LDS traffic, 128 x 128 leaves room for a third workgroup
-// per CU, whose loads cover the others' starts and stores.  Long contractions take the first (74 k x 2048 to 512 columns: 196 us
-// against 214), and so do short ones with tiles enough for six rounds over the chip (74 k x 512 to 2048 columns: 270 us against
-// 281; to 512 columns 76 against 68); products of few tiles go down to 64 x 64.  (256 x 256 with one wave per SIMD, 128 x 128
-// per wave: 310 and 220 us.)  Both sides were timed before the loads of UNIFORM; with them the chosen tiles take 187 and 257 us.
-// Widths of 256 to 2048, 1.6 k to 131 k rows, with these lines in the library product's time: a projection 1.0 - 1.2, the output product
-// 1.4, input gradients 0.9 - 1.8, weight gradients 0.5 - 2.7 (the worst at 1.6 k rows x 1024 columns).
-int pick_tile(int64_t rows, int64_t cols, int64_t depth) {
-  if (tiles_of(rows, cols, 256, 128) >= (depth >= 1024 ? 512 : 3072)) return 2;
-  if (tiles_of(rows, cols, 128, 128) >= 384) return 1;
-  return 0;
+// What a product of `tiles` tiles over a contraction of `depth` takes, in microseconds: the CUs run side by side, and one that has n
+// workgroups to run needs n times their share of its pipes, but no less than one workgroup by itself takes from its first load to
+// its last store.  The constants are a fit to widths of 64 to 2048 and 400 to 131 k rows, every product with every tile: the choice
+// by them takes 1.2 % more than the best of the four at each size (the lines by tile counts before it: 12 %).
+constexpr int GEMM_TILES = 4;
+struct TileCost { int rows, cols; double alone, alone_k, share, share_k, added; };    // added: with an operand that is added to the product
+constexpr TileCost TILE_COST[GEMM_TILES] = {
+    {64, 64, 4.3, 0.0061, 0.7, 0.0043, 0.1},        // most workgroups: few rows
+    {128, 128, 5.8, 0.0102, 2.6, 0.0089, 0.5},      // three workgroups per CU: 6400 x 1024 -> 1024 24 us (256 x 128: 28, 64 x 64: 33)
+    {256, 128, 7.7, 0.0146, 4.8, 0.0150, 1.0},      // two: 19200 x 512 -> 2048 61 us (256 x 256: 64, 128 x 128: 64)
+    {256, 256, 0.0, 0.0, 7.7, 0.0210, 6.0},         // one: 74 k x 512 -> 2048 194 us (256 x 128: 204), 74 k x 2048 -> 2048 558 (628)
+};
+double tile_cost(int t, int64_t rows, int64_t cols, double depth, int splits, bool add) {
+  const TileCost& c = TILE_COST[t];
+  const double n = (double)((tiles_of(rows, cols, c.rows, c.cols) * splits + 255) / 256);
+  const double alone = c.alone + c.alone_k * depth, share = n * (c.share + c.share_k * depth + (add ? c.added : 0.0));
+  return alone > share ? alone : share;
 }
 
-// Splits of a weight gradient's contraction (rows M of the batch): enough workgroups for the chip, whole stages, at least
-// 256 rows each.
+int pick_tile(int64_t rows, int64_t cols, int64_t depth, bool widest, bool add) {
+  int best = 0;
+  for (int t = 1; t < (widest ? GEMM_TILES : GEMM_TILES - 1); ++t)
+    if (tile_cost(t, rows, cols, (double)depth, 1, add) < tile_cost(best, rows, cols, (double)depth, 1, add)) best = t;
+  return best;
+}
+
+// Tile and splits of a weight gradient, whose contraction is the batch's rows: a split's partial sums are written, read and added (a
+// launch, 0.155 us a megabyte, 0.24 a split).  Powers of two, so that whole XCDs share a split; at least 128 rows each.  With
+// every (tile, splits) of the sweep timed the choice takes 1.8 % more than the best (the lines before it 36 %: they took eight
+// splits where two or none do; 1600 rows, 1024 -> 4096: 62 -> 23 us).
 int pick_splits(int64_t rows, int64_t cols, int64_t depth, int* tile) {
-  const int t = tiles_of(rows, cols, 256, 128) >= 8 ? 2 : (tiles_of(rows, cols, 128, 128) >= 4 ? 1 : 0);
-  *tile = t;
-  const int64_t tiles = t == 2 ? tiles_of(rows, cols, 256, 128) : (t == 1 ? tiles_of(rows, cols, 128, 128) : tiles_of(rows, cols, 64, 64));
-  int64_t s = (512 + tiles - 1) / tiles;
-  const int64_t most = depth / 256;
-  s = s < most ? s : most;
-  s = s < 1 ? 1 : (s > 64 ? 64 : s);
-  if (s > 1) s = (s + 7) / 8 * 8;              // (a split is one XCD's work)
-  return (int)s;
+  int splits = 1;
+  double least = 1e300;
+  for (int s = 1; s <= 64 && (s == 1 || depth / s >= 128); s *= 2)
+    for (int t = 0; t < GEMM_TILES; ++t) {
+      double c = tile_cost(t, rows, cols, (double)depth / s, s, false);
+      if (s > 1) c += 2.4 + 0.155 * 8e-6 * s * (double)rows * (double)cols + 0.24 * s;
+      if (c < least) { least = c; splits = s; *tile = t; }
+    }
+  return splits;
 }
 
 // out = act(x w + c + bias) for widths that the kernel above cannot fetch 16 bytes at a time: element by element, fp32 products.  (One
@@ -667,12 +750,12 @@ int hstu_gemm(const HstuGemmArgs* a, void* stream) {
     p.cols = p.out_slab = a->N;
     p.out_stride = a->N;
     p.depth = p.depth_per_split = a->K;
-    return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth));
+    return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, true, 256, 256), p.c != nullptr));
   }
   p.cols = p.out_slab = a->K;
   p.out_stride = a->K;
   p.depth = p.depth_per_split = a->N;
-  return launch_sized<false, false>(p, st, pick_tile(p.rows, p.cols, p.depth));
+  return launch_sized<false, false>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, false, 256, 256), false));
 }
 
 }  // extern "C"

@@ -28,7 +28,11 @@ def _close(got, want):
     (257, 160, 136, 4),        # slabs of 40: a stage that crosses from one into the next
     (1000, 512, 128, 4),       # slabs of whole tiles
     (6200, 1024, 136, 2),      # 128 x 128 tiles
-    (33000, 512, 1024, 4),     # 256 x 128 tiles, a long contraction, a split weight gradient whose last part is short
+    (33000, 512, 1024, 4),     # 256 x 128 tiles of a weight's gradient, a long contraction, a last split that is short
+    (6300, 2048, 520, 1),      # 256 x 256 tiles, the last of both axes short; a stage that the contraction ends in
+    (6300, 2048, 512, 4),      # the same over slabs
+    (9000, 2056, 1032, 1),     # a weight's gradient in four splits, whose 45 tiles two XCDs each share
+    (4100, 2056, 2056, 1),     # and in two
 ])
 def test_block_products(gpu, M, N, K, slabs):
   g = torch.Generator().manual_seed(M + N)
