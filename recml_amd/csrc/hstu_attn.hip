@@ -3513,6 +3513,15 @@ __device__ __forceinline__ constexpr int swz_rt(int row) {
 template <int D>
 __device__ __forceinline__ constexpr int swz_rt_group(int gi) { return D == 128 ? (gi >> 2) : D == 64 ? ((gi >> 3) & 1) : 0; }
 
+// The lane's number, worked out where it is asked for.  The backward kernels with timestamps have no register left for what only
+// their bucket lookups need of it: kept across the loop it is spilled, and the reload's wait is a wait for every direct load in
+// flight (the two kernels together 4130 -> 4000 us at B = 64, L = 2048, d = 128).
+__device__ __forceinline__ int lane_again() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
 // sigma and f' from u = x log2(e): returns sigma(x), stores f'(x)
 __device__ __forceinline__ float silu_grad_log2(float u, float* fprime) {
   const float e = __builtin_amdgcn_exp2f(-u);
@@ -3555,12 +3564,12 @@ __device__ __forceinline__ void store_rows(const floatx16 (&acc)[D / 32], float 
   }
 }
 
-// Extra LDS of the dQ kernel when it also sums table gradients: a ring of TG_RING diagonal sums per
-// wave, then one sum per bucket for the workgroup.  Kept this small on purpose: with both biases at
-// d = 128 the kernel's LDS is 78 KB, and two workgroups must still fit a CU's 160 KB.
-constexpr int TG_RING = 128;
-constexpr int TG_WG_RING = 256;      // the workgroup's ring of diagonal sums (within the NWAVES * TG_RING floats set aside)
-constexpr int BWD_TG_BYTES = (NWAVES * TG_RING + TS_TAB_LEN) * 4;
+// Extra LDS of the dQ kernel when it also sums table gradients: two rings of diagonal sums, then TG_COPIES sums per bucket for the
+// workgroup.  Kept this small on purpose: with both biases at d = 128 the kernel's LDS is 79.95 KB, and two workgroups must
+// still fit a CU's 160 KB.
+constexpr int TG_RING = 256;
+constexpr int TG_COPIES = 2;         // of the bucket sums, by lane: neighbouring lanes' adds to one bucket do not wait for each other
+constexpr int BWD_TG_BYTES = (2 * TG_RING + TG_COPIES * TS_TAB_LEN) * 4;
 
 // v of the lane `CTRL` names (data-parallel-primitive controls of the vector ALU: 0x110 + n = n lanes
 // down within a row of 16, 0x142 / 0x143 = lane 15 of the previous row / lane 31 to the rows that
@@ -3587,6 +3596,12 @@ __device__ __forceinline__ void swap16(float& a, float& b) {
   a = __builtin_bit_cast(float, x);
   b = __builtin_bit_cast(float, y);
 }
+// v of a lane of the lower 32 and of its partner 32 further on, added, for the lower one; 0 for the upper
+__device__ __forceinline__ float both_halves(float v) {
+  float z = 0.f;
+  swap32(v, z);
+  return v + z;
+}
 // float atomic add on an LDS location given by an ordinary pointer (named as LDS for the compiler: on
 // a pointer of unknown address space it builds a run-time dispatch that some instantiations miscompile)
 typedef __attribute__((address_space(3))) float* lds_float_ptr;
@@ -3595,13 +3610,18 @@ __device__ __forceinline__ void lds_atomic_add(float* lds_location, float v) {
 }
 
 // TG: also accumulate the table gradients.  Every pair adds its dS to the entry of each table its
-// logit read; LDS float atomics with many lanes on one address turned out to cost about 4 cycles per
-// lane, so the sums are formed in registers first and reach LDS one lane per address.
+// logit read; an LDS float atomic costs the CU's LDS about 3 cycles per lane, on one address or on 64 (a block's 64 diagonal sums
+// added that way: 190 cycles of it), so the sums are formed in registers first, and the diagonal ones reach LDS by reads and writes.
 // Position table: pair (q, key) of a workgroup lies on diagonal X = key - q + (q0 + 127) >= 0.  A block's
 // 32 x 32 pairs are brought onto their 63 diagonals by lane permutes (see the block), one value per
-// lane, and added to the workgroup's ring of sums.  The blocks of a pair of steps (t, t + 1) only touch
-// X in [32 t, 32 t + 192), so everything below 32 (t + 2) is final after the pair's barrier: at the start
+// lane.  The upper 32 of them are the lower 32 of the wave's next block: they wait for it in a register, and a block adds 32
+// finished sums of its wave to a ring, by a read and a write: waves 0 and 2 to one, 1 and 3 to the other.  Two waves of a ring
+// are on different slots in every pair of steps (t, t + 1), 32 t + 96 - 32 w .. + 64 for wave w, and a pair's barrier lies between
+// one wave's turn at a slot and the other's.  Everything below 32 (t + 2) is final after the pair's barrier: at the start
 // of the next pair one wave adds those 64 diagonals to the table in memory and clears them.
+// (B = 64 at L = 2048, H = 8, d = 128, both tables, this kernel: 2370 us with an atomic per lane and block for the diagonals and per
+// half row for the buckets, one product's registers for the fragments and a spilled lane number; 1800 us as it is.  d = 64, 78 k
+// tokens, the position table: 250 and 222.)
 // Bucket table: where each lane has one bucket for the whole block (or two neighbours), lanes with
 // the same bucket are summed across the wave and one lane adds the sum to the workgroup's
 // histogram (an LDS atomic, but of one lane); only blocks with more buckets per lane use one
@@ -3773,7 +3793,7 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
   if (t_lo < nt) dma_step(t_lo);
   if (t_lo + 1 < nt) dma_step(t_lo + 1);
   if (TG) {
-    for (int i = tid; i < NWAVES * TG_RING + TS_TAB_LEN; i += MFMA_THREADS) TgBase[i] = 0.f;
+    for (int i = tid; i < 2 * TG_RING + TG_COPIES * TS_TAB_LEN; i += MFMA_THREADS) TgBase[i] = 0.f;
   }
 
   // Q and dO fragments of this lane's row (B operands): 16-byte chunk 2ks + hh of the row
@@ -3827,30 +3847,33 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
   // (timestamp-table gradient: the lane's bucket of the last block and what is summed for it)
   int sum_bucket = 0;
   float sum_s = 0.f;
+  float diag_wait = 0.f;           // (position-table gradient: diagonals that the wave's next block finishes; upper lanes 0)
+  int diag_next = 0;               // and the first key of that block
   auto block = [&](int t) {
     const int st = t % NSTAGE;
     const int kbs = t * BN;
+    if (TG) diag_next = kbs + BN;
     const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     floatx16 sacc, dpacc;
     {
-      uint4 kf[QCH];
-      const unsigned char* kr = (const unsigned char*)Ks(st) + m * (D * 2);
+      // S and dP take turns, the fragments of a product asked for AHEAD_F products ahead, in an order fixed by scheduling barriers
+      // (left to itself the compiler has one product's registers for the first chain and waits for LDS before each of it).
+      constexpr int AHEAD_F = 3;
+      const unsigned char* const kr = (const unsigned char*)Ks(st) + m * (D * 2);
+      uint4 af[AHEAD_F + 1];
+      auto ask = [&](int i) __attribute__((always_inline)) {          // product i: S for even i, dP for odd, channels 16 (i / 2) ..
+        af[i % (AHEAD_F + 1)] = *(const uint4*)(kr + (((2 * (i >> 1) + hh) ^ gk) * 16) + (i & 1) * SM::K_BYTES);
+      };
 #pragma unroll
-      for (int ks = 0; ks < QCH; ++ks) kf[ks] = *(const uint4*)(kr + (((2 * ks + hh) ^ gk) * 16));
+      for (int i = 0; i < AHEAD_F; ++i) ask(i);
 #pragma unroll
-      for (int ks = 0; ks < QCH; ++ks)
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[ks]), __builtin_bit_cast(bf16x8, qf[ks]),
-                                                       ks == 0 ? zero : sacc, 0, 0, 0);
-    }
-    {
-      uint4 vf[QCH];
-      const unsigned char* vr = (const unsigned char*)Vs(st) + m * (D * 2);
-#pragma unroll
-      for (int ks = 0; ks < QCH; ++ks) vf[ks] = *(const uint4*)(vr + (((2 * ks + hh) ^ gk) * 16));
-#pragma unroll
-      for (int ks = 0; ks < QCH; ++ks)
-        dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[ks]), __builtin_bit_cast(bf16x8, dof[ks]),
-                                                        ks == 0 ? zero : dpacc, 0, 0, 0);
+      for (int i = 0; i < 2 * QCH; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + AHEAD_F < 2 * QCH) ask(i + AHEAD_F);
+        floatx16& c = (i & 1) ? dpacc : sacc;
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i % (AHEAD_F + 1)]),
+                                                    __builtin_bit_cast(bf16x8, (i & 1) ? dof[i >> 1] : qf[i >> 1]), i < 2 ? zero : c, 0, 0, 0);
+      }
     }
     // lane holds S^T[kv = kbs + 8g + 4hh + tt][q = qrow], r = 4g + tt
     float u[16];
@@ -3894,6 +3917,7 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
         const int32_t* tk = Tk(st);
         const int2 rg = *(const int2*)(tk + BN);
         const TsEnds en = ts_ends(TsKey, tq32 - rg.y, tq32 - rg.x);
+        const int32_t* const tk_lane = tk + 4 * (lane_again() >> 5);
         if (__builtin_amdgcn_ballot_w64(!en.same) == 0) {
           const float add = en.v_near;
 #pragma unroll
@@ -3908,7 +3932,7 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           far_keys = true;
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
+            const int4 kk = *(const int4*)(tk_lane + 8 * g);
             const bool f0 = kk.x <= cut, f1 = kk.y <= cut, f2 = kk.z <= cut, f3 = kk.w <= cut;
             u[4 * g + 0] += f0 ? add_far : add_near;
             u[4 * g + 1] += f1 ? add_far : add_near;
@@ -3917,18 +3941,43 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           }
           bk_lane = en.b_near;
         } else {
+// every pair looked up, four at a time: the reads of four buckets under way together, and a group's values under way with the
+          // next group's buckets (one by one, as the compiler has them for want of registers, each waits for LDS by itself)
+          if (TG) {
+            float f[2][4], thr[2][4], val[4];
+            uint32_t below[2][4];
+            auto ask = [&](int g) __attribute__((always_inline)) {
+              const int4 kk = *(const int4*)(tk_lane + 8 * g);
+              const int d4[4] = {tq32 - kk.x, tq32 - kk.y, tq32 - kk.z, tq32 - kk.w};
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
-            if (TG) {
-              const int b0 = ts_bucket_of(TsKey, tq32 - kk.x), b1 = ts_bucket_of(TsKey, tq32 - kk.y);
-              const int b2 = ts_bucket_of(TsKey, tq32 - kk.z), b3 = ts_bucket_of(TsKey, tq32 - kk.w);
-              u[4 * g + 0] += ts_bucket_value(TsKey, b0);
-              u[4 * g + 1] += ts_bucket_value(TsKey, b1);
-              u[4 * g + 2] += ts_bucket_value(TsKey, b2);
-              u[4 * g + 3] += ts_bucket_value(TsKey, b3);
-              bkp[g] = (uint32_t)b0 | ((uint32_t)b1 << 8) | ((uint32_t)b2 << 16) | ((uint32_t)b3 << 24);
-            } else {
+              for (int t4 = 0; t4 < 4; ++t4) {
+                float& x = f[g & 1][t4];
+                x = __builtin_amdgcn_fmed3f(__builtin_fabsf((float)d4[t4]), 1.0f, (float)TS_DT_MAX);
+                const uint32_t key = (__builtin_bit_cast(uint32_t, x) >> 21) - (uint32_t)TS_KEY0;
+                below[g & 1][t4] = TsKey[TS_BKT_OFF + key];
+                thr[g & 1][t4] = *(const float*)(TsKey + (key << 3) + 4);
+              }
+            };
+            ask(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              __builtin_amdgcn_sched_barrier(0);
+              uint32_t bk[4];
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) bk[t4] = below[g & 1][t4] + (f[g & 1][t4] >= thr[g & 1][t4] ? 1u : 0u);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) val[t4] = ts_bucket_value(TsKey, (int)bk[t4]);
+              bkp[g] = bk[0] | (bk[1] << 8) | (bk[2] << 16) | (bk[3] << 24);
+              if (g < 3) ask(g + 1);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) u[4 * g + t4] += val[t4];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const int4 kk = *(const int4*)(tk_lane + 8 * g);
               u[4 * g + 0] += ts_value(ts_look(TsKey, tq32 - kk.x));
               u[4 * g + 1] += ts_value(ts_look(TsKey, tq32 - kk.y));
               u[4 * g + 2] += ts_value(ts_look(TsKey, tq32 - kk.z));
@@ -3953,6 +4002,10 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
         }
       }
     }
+    // (the wave's slots of its ring of diagonal sums, asked for ahead of their use)
+    float* const diag_slot = TgBase + (w & 1) * TG_RING + ((kbs + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_RING - 1));
+    float diag_old = 0.f;
+    if (want_dpos && lane < 32) diag_old = *diag_slot;
     float ds[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -4053,14 +4106,18 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
       up += t2;
       swap32(lo, up);
       swap16(lo, up);
-      const float diag = up + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane - 16) & 63) << 2, __builtin_bit_cast(int, lo)));
-      // the workgroup's ring of diagonal sums: this wave's diagonal X is the workgroup's X + 96 - 32 w (a lane per
-      // slot within the instruction; other waves may add to the same slots, hence the atomic form)
-      lds_atomic_add(TgBase + ((kbs + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_WG_RING - 1)), diag);
+      float diag = up + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane - 16) & 63) << 2, __builtin_bit_cast(int, lo)));
+      // lane l: the wave's diagonal 111 + (l & 48) - (l & 15) of this step.  The lower half with the last block's upper one is
+      // finished, the upper half waits.
+      diag += diag_wait;
+      diag_wait = 0.f;
+      swap32(diag, diag_wait);
+      if (lane < 32) *diag_slot = diag_old + diag;
     }
     if (want_dts) {
-      float* hist = TgBase + NWAVES * TG_RING;
+      float* hist = TgBase + 2 * TG_RING + (lane & (TG_COPIES - 1));      // entry TG_COPIES b: bucket b
       if (bk_lane >= 0) {
+        // (the two halves of the wave hold the same rows: one buckets' sum for both, in the lower one)
         // A lane's bucket changes with the step only now and then (the nearer the keys, the smaller): its sum stays in a
         // register until it does, and reaches the histogram then, by an LDS atomic of the lanes concerned.
         float s_near;
@@ -4071,76 +4128,76 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           // (two sums of their own: the near one as what the far one leaves of the total would lose its digits where the far
           // keys outweigh it, and all of them to one infinity among those.  It costs 0.8 %: B = 64 at L = 2048, d = 128, forward and
           // gradients 5001 -> 5042 us, and 5051 with sixteen comparisons at once, which spill 32 scalar registers)
-          const int32_t* tk = Tk(st);
+          const int32_t* tk = Tk(st) + 4 * (lane_again() >> 5);
           float s_far = 0.f;
           s_near = 0.f;
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            const int4 kk = *(const int4*)(tk + 8 * g + 4 * hh);
+            const int4 kk = *(const int4*)(tk + 8 * g);
             const bool f0 = kk.x <= cut, f1 = kk.y <= cut, f2 = kk.z <= cut, f3 = kk.w <= cut;
             const float *v = ds + 4 * g;
             s_far += ((f0 ? v[0] : 0.f) + (f1 ? v[1] : 0.f)) + ((f2 ? v[2] : 0.f) + (f3 ? v[3] : 0.f));
             s_near += ((f0 ? 0.f : v[0]) + (f1 ? 0.f : v[1])) + ((f2 ? 0.f : v[2]) + (f3 ? 0.f : v[3]));
             asm volatile("" : "+v"(s_far), "+v"(s_near));      // (four comparisons in scalar registers at a time, not sixteen)
           }
+          s_far = both_halves(s_far);
           if (sum_bucket == bk_lane + 1) sum_s += s_far;
-          else if (s_far != 0.f) lds_atomic_add(&hist[bk_lane + 1], s_far);
+          else if (s_far != 0.f) lds_atomic_add(&hist[TG_COPIES * (bk_lane + 1)], s_far);
         }
+        s_near = both_halves(s_near);
         if (sum_bucket != bk_lane) {
-          if (sum_s != 0.f) lds_atomic_add(&hist[sum_bucket], sum_s);
+          if (sum_s != 0.f) lds_atomic_add(&hist[TG_COPIES * sum_bucket], sum_s);
           sum_bucket = bk_lane;
           sum_s = 0.f;
         }
         sum_s += s_near;
       } else {
-        // LDS atomics cost by the lane: neighbouring keys mostly share a bucket, so each run of equal
-        // buckets is summed first, and runs that add nothing (masked pairs) are skipped
-        float carry = 0.f;
+        // neighbouring keys mostly share a bucket, so each run of equal buckets is summed first (the last one waits for the next
+        // block's first), and runs that add nothing (masked pairs) are skipped
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const uint32_t bcur = (bkp[r >> 2] >> (8 * (r & 3))) & 255u;
-          const uint32_t bnext = r < 15 ? (bkp[(r + 1) >> 2] >> (8 * ((r + 1) & 3))) & 255u : 256u;
-          carry += ds[r];
-          if (bcur != bnext) {
-            if (carry != 0.f) lds_atomic_add(&hist[bcur], carry);
-            carry = 0.f;
+          const int bcur = (int)((bkp[r >> 2] >> (8 * (r & 3))) & 255u);
+          if (bcur != sum_bucket) {
+            if (sum_s != 0.f) lds_atomic_add(&hist[TG_COPIES * sum_bucket], sum_s);
+            sum_s = 0.f;
+            sum_bucket = bcur;
           }
+          sum_s += ds[r];
         }
       }
     }
-    // K^T fragments for the last product
-    uint4 ktf[2][DVB];
+    // K^T fragments for the last product, two products ahead
     {
-      const bf16_t* kr = Ks(st) + vrow * D + 4 * (gi & 1);
+      const bf16_t* const krt = Ks(st) + vrow * D + 4 * (gi & 1);
+      uint4 pk[2], tf[3];
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc)
+        pk[cc] = uint4{pack_bf16(ds[8 * cc + 0], ds[8 * cc + 1]), pack_bf16(ds[8 * cc + 2], ds[8 * cc + 3]),
+                       pack_bf16(ds[8 * cc + 4], ds[8 * cc + 5]), pack_bf16(ds[8 * cc + 6], ds[8 * cc + 7])};
+      auto ask = [&](int i) __attribute__((always_inline)) {
+        const int cc = i / DVB, cb = 4 * ((i % DVB) ^ swz_rt_group<D>(gi));
+        const uint2 lo = lds_read_tr(krt + (16 * cc) * D + (cb + c_lo) * 8);
+        const uint2 hi = lds_read_tr(krt + (16 * cc + 8) * D + (cb + c_hi) * 8);
+        tf[i % 3] = uint4{lo.x, lo.y, hi.x, hi.y};
+      };
+      ask(0);
+      if (2 * DVB > 1) ask(1);
 #pragma unroll
-        for (int dvb = 0; dvb < DVB; ++dvb) {
-          const int cb = 4 * (dvb ^ swz_rt_group<D>(gi));
-          uint2 lo = lds_read_tr(kr + (16 * cc) * D + (cb + c_lo) * 8);
-          uint2 hi = lds_read_tr(kr + (16 * cc + 8) * D + (cb + c_hi) * 8);
-          ktf[cc][dvb] = uint4{lo.x, lo.y, hi.x, hi.y};
-        }
-    }
-#pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
-      uint4 pk;
-      pk.x = pack_bf16(ds[8 * cc + 0], ds[8 * cc + 1]);
-      pk.y = pack_bf16(ds[8 * cc + 2], ds[8 * cc + 3]);
-      pk.z = pack_bf16(ds[8 * cc + 4], ds[8 * cc + 5]);
-      pk.w = pack_bf16(ds[8 * cc + 6], ds[8 * cc + 7]);
-      const bf16x8 pb = __builtin_bit_cast(bf16x8, pk);
-#pragma unroll
-      for (int dvb = 0; dvb < DVB; ++dvb)
-        acc[dvb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ktf[cc][dvb]), pb, acc[dvb], 0, 0, 0);
+      for (int i = 0; i < 2 * DVB; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < 2 * DVB) ask(i + 2);
+        acc[i % DVB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf[i % 3]), __builtin_bit_cast(bf16x8, pk[i / DVB]),
+                                                               acc[i % DVB], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  // adds diagonals [x0, x0 + 64) of the workgroup's ring to the table in memory and clears them (one wave's job)
+  // adds diagonals [x0, x0 + 64) of the rings to the table in memory and clears them (one wave's job)
   auto flush_diag = [&](int x0) {
-    float* slot = TgBase + ((x0 + lane) & (TG_WG_RING - 1));
-    const float val = *slot;
-    *slot = 0.f;
+    float* slot = TgBase + ((x0 + lane) & (TG_RING - 1));
+    const float val = slot[0] + slot[TG_RING];
+    slot[0] = slot[TG_RING] = 0.f;
     const int idx = (p.L - 1) + (x0 + lane) - (BM - 1) - q0;
     if (val != 0.f && idx >= 0 && idx < 2 * p.L - 1)
       atomicAdd(p.dpos + (int64_t)(p.pos_heads > 1 ? h : 0) * (2 * p.L - 1) + idx, val * p.inv_n);
@@ -4152,8 +4209,8 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
   static_assert(NSTAGE == 4, "two pairs of stages");
   HSTU_WAIT_VMCNT(0);
   __syncthreads();
-  // Position-table gradient: the four waves add their blocks' diagonal sums into ONE ring of the workgroup
-  // (diagonal X = key - row + q0 + 127; the blocks of step pair (t, t + 1) touch [32 t, 32 t + 192)), and what a
+  // Position-table gradient: the four waves add their blocks' diagonal sums into the workgroup's rings
+  // (diagonal X = key - row + q0 + 127; the blocks of step pair (t, t + 1) touch [32 t, 32 t + 160)), and what a
   // pair has completed -- [32 t, 32 t + 64), final once every wave is past the pair's barrier -- goes to memory
   // at the start of the next pair, by one wave in turn.  Every workgroup of the launch adds into the one table:
   // with a ring per wave, each flushing its own 64 diagonals per pair, those adds (four times as many) cost a
@@ -4169,17 +4226,26 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     HSTU_WAIT_VMCNT(0);
     __syncthreads();
   }
+  if (want_dpos && t_lo < nt) {
+    // what waits for a block that does not come (a wave ends at most 96 keys before the tile does, so nothing of it is flushed yet)
+    if (lane < 32 && wave_live) {
+      float* slot = TgBase + (w & 1) * TG_RING + ((diag_next + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_RING - 1));
+      *slot += diag_wait;
+    }
+    __syncthreads();
+  }
   if (want_dpos && t_lo < nt && w < 3) {
-    // what the last pair left in the ring (every wave is past the loop's last barrier)
+    // what the last pair left in the rings (every wave is past the loop's last barrier)
     const int t_last = t_lo + ((nt - 1 - t_lo) & ~1);
     flush_diag(32 * t_last + 64 * w);
   }
   if (want_dts) {
-    if (sum_s != 0.f) lds_atomic_add(TgBase + NWAVES * TG_RING + sum_bucket, sum_s);
+    if (sum_s != 0.f) lds_atomic_add(TgBase + 2 * TG_RING + TG_COPIES * sum_bucket + (lane & (TG_COPIES - 1)), sum_s);
     __syncthreads();                     // the histogram is complete
-    const float* hist = TgBase + NWAVES * TG_RING;
+    const float* hist = TgBase + 2 * TG_RING;
     for (int e = tid; e < TS_TAB_LEN; e += MFMA_THREADS) {
-      const float val = hist[e];
+      const float2 two = *(const float2*)(hist + TG_COPIES * e);
+      const float val = two.x + two.y;
       if (val != 0.f) atomicAdd(p.dts + (int64_t)(p.ts_heads > 1 ? h : 0) * (p.ts_nb + 1) + (e < p.ts_nb ? e : p.ts_nb), val * p.inv_n);
     }
   }
@@ -4632,29 +4698,46 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) u[r] += add;
         } else {
-          // the 16 rows' timestamps: away from the sequence's end four consecutive words per group, one further on than an
-          // aligned read has them
-          int tqv[16];
-          if (qbs + BN < s.n_ts) {
+          // a group's rows' timestamps: away from the sequence's end four consecutive words, one further on than an aligned read
+          // has them
+          const bool inside = qbs + BN < s.n_ts;
+          auto times = [&](int g, int (&tqv)[4]) __attribute__((always_inline)) {
+            if (inside) {
+              const int32_t* const at = tqs + 8 * g + 4 * (lane_again() >> 5);
+              const int4 a = *(const int4*)at;
+              tqv[0] = a.y; tqv[1] = a.z; tqv[2] = a.w;
+              tqv[3] = at[4];
+            } else {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int4 a = *(const int4*)(tqs + 8 * g + 4 * hh);
-              tqv[4 * g] = a.y; tqv[4 * g + 1] = a.z; tqv[4 * g + 2] = a.w;
-              tqv[4 * g + 3] = tqs[8 * g + 4 * hh + 4];
+              for (int t4 = 0; t4 < 4; ++t4) tqv[t4] = tqs[tq_at(4 * g + t4) - qbs];
             }
-          } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) tqv[r] = tqs[tq_at(r) - qbs];
-          }
+          };
           if (two_buckets) {
             // one bucket boundary at most: the farther bucket exactly when tq - tk >= thr (none of the three is negative)
             const float add_near = en.v_near, add_far = en.v_far;
             const uint32_t cut = (uint32_t)en.thr + (uint32_t)tk32;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) u[r] += (uint32_t)tqv[r] >= cut ? add_far : add_near;
-          } else {
+            for (int g = 0; g < 4; ++g) {
+              int tqv[4];
+              times(g, tqv);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) u[r] += ts_value(ts_look(TsKey, tqv[r] - tk32));
+              for (int t4 = 0; t4 < 4; ++t4) u[4 * g + t4] += (uint32_t)tqv[t4] >= cut ? add_far : add_near;
+            }
+          } else {
+            // every pair looked up.  WIDE: the reads of four under way together (one by one, as the compiler has them for want of
+            // registers, each waits for LDS by itself; at smaller head dims it has them, and is better left alone)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              int tqv[4];
+              times(g, tqv);
+              TsLook look[4];
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) look[t4] = ts_look(TsKey, tqv[t4] - tk32);
+              if constexpr (WIDE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) u[4 * g + t4] += ts_value(look[t4]);
+              if constexpr (WIDE) __builtin_amdgcn_sched_barrier(0);
+            }
           }
         }
       } else {

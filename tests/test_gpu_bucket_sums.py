@@ -38,3 +38,39 @@ def test_near_bucket_keeps_its_own_sum(gpu, d, far):
     assert abs(got[0, 31] - 2.0 ** 20 * want[0, 31]) <= 1e-3 * abs(2.0 ** 20 * want[0, 31])
   else:
     assert not np.isfinite(got[0, 31])
+
+
+@pytest.mark.parametrize("d,L,causal,window,lens", [
+    (32, 1, True, None, [1]),
+    (64, 33, True, None, [33, 32]),                  # the second wave's one row; a wave's last block is its first
+    (128, 300, True, None, [300, 129, 97, 5]),       # the rings of diagonal sums begin again at 256
+    (64, 700, False, None, [700, 257]),              # every wave ends at the same step: what waits is handed on after the loop
+    (128, 520, True, 40, [520, 383]),                # a band narrower than a tile, starting and ending at another step in each wave
+    (32, 420, False, 130, [420, 31]),
+])
+def test_table_sums_are_complete(gpu, d, L, causal, window, lens):
+  """q = k = 0 and both tables 0: every logit is 0 and f' a half, dS half of a small whole number, and every sum of them exact in
+  fp32, in whatever order it is made.  So both tables' gradients are equal to the reference's, bit by bit.  An item about every hour:
+  one bucket, two and more than two to a block, and a bucket's run that goes on from one block to the next."""
+  rng = np.random.default_rng(L)
+  B, H = len(lens), 2
+  zero = np.zeros((B, L, H, d), np.float32)
+  v, dout = (rng.integers(-1, 2, (B, L, H, d)).astype(np.float32) for _ in range(2))
+  ts = 1_600_000_000 + np.cumsum(np.ceil(rng.exponential(3600.0, (B, L))).astype(np.int64), 1)
+  pos, tab = np.zeros((H, 2 * L - 1), np.float32), np.zeros((H, 129), np.float32)
+  lens = np.array(lens, np.int32)
+  want = O.hstu_attention_bwd_ref(zero, zero, v, dout, causal=causal, sliding_window_size=window, seq_lens=lens, n=1024, pos_tab=pos,
+                                  timestamps=ts, ts_tab=tab)
+  dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")
+  bf = torch.bfloat16
+  for pos_, ts_ in ((True, True), (True, False), (False, True)):
+    kw = dict(pos_bias=dev(pos)) if pos_ else {}
+    kw.update(dict(timestamps=dev(ts), ts_bias=dev(tab)) if ts_ else {})
+    variant = []
+    got = recml_amd.hstu_attention_bwd(dev(zero).to(bf), dev(zero).to(bf), dev(v).to(bf), dev(dout).to(bf), causal=causal,
+                                       sliding_window_size=window, seq_lens=dev(lens), n=1024, _variant_out=variant, **kw)
+    assert variant == ["hstu_bwd_mfma_bf16"]
+    for g, w, given in ((got[3], want[3], pos_), (got[4], want[4], ts_)):
+      assert (g is not None) == given
+      if given:
+        np.testing.assert_array_equal(g.cpu().numpy(), np.asarray(w, np.float32))
