@@ -671,6 +671,21 @@ __global__ __launch_bounds__(256, D >= 128 ? 3 : 4) void hstu_f32_fwd(const Para
     store_row<T, D>((T*)p.out + s.bo + (int64_t)qi * p.o_st, o, qi < s.n_q ? p.inv_n : 0.f, g);
 }
 
+// A block's dS to the sums along its diagonals, key - query = 4 g + r - m of lane (m, g): the four registers are brought onto 4 g - m and
+// 4 g - m + 16 by shifts within the rows of 16 lanes.  An LDS float atomic takes the CU's LDS 3 cycles a lane: 76 lanes for a block
+// instead of 256 (B = 32, L = 512, H = 8, d = 128, position table, both backward kernels: 781 -> 651 us).
+template <int CTRL>
+__device__ __forceinline__ float lanes_moved(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ void add_diagonals(float* d, const floatx4& x, int m) {
+  // register r of lane m is diagonal r - m: lane m - r's where there is one, else that of lane 16 + m - r, 16 further up
+  const float near = (x[0] + lanes_moved<0x101>(x[1])) + (lanes_moved<0x102>(x[2]) + lanes_moved<0x103>(x[3]));
+  const float far = lanes_moved<0x11f>(x[1]) + lanes_moved<0x11e>(x[2]) + lanes_moved<0x11d>(x[3]);
+  lds_add(d, near);
+  if (m >= 13) lds_add(d + 16, far);
+}
+
 template <typename T, int D, bool TAB, bool DEN>
 __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dq(const Params p, const TabArg<TAB> ta) {
   using S = Shape<D>;
@@ -745,11 +760,7 @@ __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dq(const Param
           }
           dot_cols<D>(o, t.tile(buf, 0), 16 * kg, m, g, x);
           if constexpr (TAB) {
-            if (want_pos) {
-              float* d = diag + (c0 - lo) + 4 * g + (TILE - 1) - (WROWS * w + m);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) lds_add(d + r, x[r]);
-            }
+            if (want_pos) add_diagonals(diag + (c0 - lo) + 4 * g + (TILE - 1) - (WROWS * w + m), x, m);
             if (want_ts) {
               // neighbouring pairs mostly share a bucket: a block with one bucket is summed over the wave first
               const int b0 = __builtin_amdgcn_readfirstlane(bucket[0]);

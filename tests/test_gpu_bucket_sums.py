@@ -62,14 +62,13 @@ def test_table_sums_are_complete(gpu, d, L, causal, window, lens):
   want = O.hstu_attention_bwd_ref(zero, zero, v, dout, causal=causal, sliding_window_size=window, seq_lens=lens, n=1024, pos_tab=pos,
                                   timestamps=ts, ts_tab=tab)
   dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to("cuda:0")
-  bf = torch.bfloat16
-  for pos_, ts_ in ((True, True), (True, False), (False, True)):
+  for dtype, pos_, ts_ in ((torch.bfloat16, True, True), (torch.bfloat16, True, False), (torch.bfloat16, False, True), (torch.float32, True, True)):
     kw = dict(pos_bias=dev(pos)) if pos_ else {}
     kw.update(dict(timestamps=dev(ts), ts_bias=dev(tab)) if ts_ else {})
     variant = []
-    got = recml_amd.hstu_attention_bwd(dev(zero).to(bf), dev(zero).to(bf), dev(v).to(bf), dev(dout).to(bf), causal=causal,
+    got = recml_amd.hstu_attention_bwd(dev(zero).to(dtype), dev(zero).to(dtype), dev(v).to(dtype), dev(dout).to(dtype), causal=causal,
                                        sliding_window_size=window, seq_lens=dev(lens), n=1024, _variant_out=variant, **kw)
-    assert variant == ["hstu_bwd_mfma_bf16"]
+    assert dtype == torch.float32 or variant == ["hstu_bwd_mfma_bf16"]
     for g, w, given in ((got[3], want[3], pos_), (got[4], want[4], ts_)):
       assert (g is not None) == given
       if given:
