@@ -259,6 +259,36 @@ typedef struct HstuGemmArgs {
 size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K);
 int hstu_gemm(const HstuGemmArgs* args, void* stream);
 
+/* A whole block in inference as one launch, for short sequences and narrow models (hstu.py:442-474): out = tokens + output projection of
+ * u * layer_norm(attention) with u, q, k, v = silu(layer_norm(tokens) w + bias), causal pointwise attention over alpha q k^T
+ * (+ pos_tab) with the weights scaled by inv_n and each sequence's length.  bf16 tensors and parameters, contiguous; tokens and out
+ * [B, L, width], or with seq_offsets [T, width] (sequence b from row seq_offsets[b] on, at most L rows of it).  w[i]: [width, width], the
+ * U, Q, K and V kernels; w_bias[i]: [width] or all null; w_out [width, width], b_out [width] or null; pos_tab: fp32
+ * [pos_heads, 2 L - 1] or null, pos_heads 1 or heads.  Which shapes there are: hstu_block_small_takes (1 or 0). */
+typedef struct HstuBlockSmallArgs {
+  uint32_t struct_size;   /* sizeof(HstuBlockSmallArgs) */
+  uint32_t version;       /* HSTU_BLOCK_ABI_VERSION     */
+  int32_t B, L, heads, head_dim, width, pos_heads;
+  float eps, alpha, inv_n;
+  int32_t reserved0;
+  const void* tokens;
+  void* out;
+  const int32_t* seq_lens;
+  const int32_t* seq_offsets;
+  const void* in_gamma;
+  const void* in_beta;
+  const void* w[4];
+  const void* w_bias[4];
+  const void* attn_gamma;
+  const void* attn_beta;
+  const void* w_out;
+  const void* b_out;
+  const float* pos_tab;
+} HstuBlockSmallArgs;
+
+int hstu_block_small_takes(int32_t B, int32_t L, int32_t heads, int32_t head_dim, int32_t width);
+int hstu_block_small_fwd(const HstuBlockSmallArgs* args, void* stream);
+
 int hstu_block_abi_version(void);
 const char* hstu_block_last_error(void);
 

@@ -27,6 +27,8 @@ EXPORTS = (
     "hstu_silu_bwd",
     "hstu_gemm",
     "hstu_gemm_workspace_bytes",
+    "hstu_block_small_takes",
+    "hstu_block_small_fwd",
 )
 
 

@@ -13,7 +13,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libhstu_attn.so")
 SOURCES = [os.path.join(_HERE, "csrc", "hstu_attn.hip"), os.path.join(_HERE, "csrc", "hstu_f32.hip")]
 # the block-side steps live in a library of their own
 BLOCK_LIB_PATH = os.path.join(LIB_DIR, "libhstu_block.so")
-BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip"), os.path.join(_HERE, "csrc", "hstu_gemm.hip")]
+BLOCK_SOURCES = [os.path.join(_HERE, "csrc", "hstu_block.hip"), os.path.join(_HERE, "csrc", "hstu_gemm.hip"),
+                 os.path.join(_HERE, "csrc", "hstu_block_small.hip")]
 INCLUDE = os.path.join(ROOT, "include")
 # the block's microbenchmark: a stand-alone program (its own main), evidence for what bounds the kernel
 MICRO_PATH = os.path.join(LIB_DIR, "micro_fwd_stream")

@@ -547,6 +547,35 @@ bool block_ready(const Tensor& tokens, const Tensor (&p)[P_COUNT], const BlockCa
   return true;
 }
 
+// The block as one launch, where there is one for its shape and options; false: nothing has been done.
+bool small_block(Tensor& out, const Tensor& tokens, const Tensor (&p)[P_COUNT], const BlockCall& c, const Tensor& pos, const Tensor& ts_tab, const Tensor& bias) {
+  const Options& o = c.opts;
+  const int64_t L = c.L ? c.L : o.max_len, B = c.L ? c.B : o.seq_offsets.numel() - 1;
+  if (ts_tab.defined() || bias.defined() || o.mask.defined() || o.dropout_p > 0.0 || o.window >= 0 || !o.causal || c.D != c.H * c.hd || L > 64 ||
+      c.D > 64 || B > 1 << 20 || !hstu_block_small_takes((int32_t)B, (int32_t)L, (int32_t)c.H, (int32_t)c.hd, (int32_t)c.D)) return false;
+  HstuBlockSmallArgs a;
+  memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.version = HSTU_BLOCK_ABI_VERSION;
+  a.B = (int32_t)B; a.L = (int32_t)L; a.heads = (int32_t)c.H; a.head_dim = (int32_t)c.hd; a.width = (int32_t)c.D;
+  a.eps = (float)c.eps; a.alpha = (float)o.alpha; a.inv_n = (float)(1.0 / o.n);
+  out = fresh(tokens, tokens.sizes());
+  a.tokens = tokens.const_data_ptr(); a.out = out.data_ptr();
+  if (o.seq_lens.defined()) a.seq_lens = o.seq_lens.const_data_ptr<int32_t>();
+  if (o.seq_offsets.defined()) a.seq_offsets = o.seq_offsets.const_data_ptr<int32_t>();
+  a.in_gamma = p[P_IN_G].const_data_ptr(); a.in_beta = p[P_IN_B].const_data_ptr();
+  a.attn_gamma = p[P_ATTN_G].const_data_ptr(); a.attn_beta = p[P_ATTN_B].const_data_ptr();
+  for (int i = 0; i < 4; ++i) {
+    a.w[i] = p[P_U + i].const_data_ptr();
+    if (p[P_UB + i].defined()) a.w_bias[i] = p[P_UB + i].const_data_ptr();
+  }
+  a.w_out = p[P_OUT].const_data_ptr();
+  if (p[P_OUT_B].defined()) a.b_out = p[P_OUT_B].const_data_ptr();
+  if (pos.defined()) { a.pos_tab = pos.const_data_ptr<float>(); a.pos_heads = pos.dim() == 2 ? (int32_t)pos.size(0) : 1; }
+  block_check(hstu_block_small_fwd(&a, stream_of(tokens)), "hstu_block_small_fwd");
+  return true;
+}
+
 // slice i of a projection [T, 4, H, hd], shaped as the attention takes it
 Tensor projection_slice(const Tensor& uqkv, const BlockCall& c, int i) {
   const int64_t W = c.H * c.hd;
@@ -1019,6 +1048,7 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
       HstuAttnFwdArgs a;
       const Tensor q = projection_slice(uqkv, c, 1);
       if (!fill(a, q, projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
+      if (!graph && small_block(out, tokens, p, c, pos, ts_tab, bias)) return true;
       normed = fresh(tokens, {T, D});
       norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
       if (graph) pre = at::empty_like(uqkv);
