@@ -309,6 +309,12 @@ typedef struct HstuAttnBwdArgs {
 
 int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream);
 
+/* The same where q = silu(q_pre), k = silu(k_pre), v = silu(v_pre) (the projections' activation, recml/layers/keras/hstu.py:444-449):
+ * dq, dk, dv become the gradients of q_pre, k_pre, v_pre: the rounded gradients times silu', rounded.  Each with its tensor's strides
+ * and dtype, or null (that gradient stays as hstu_attn_bwd has it).  For calls whose hstu_attn_bwd_variant is
+ * "hstu_bwd_mfma_bf16"; others are refused (HSTU_ERR_SHAPE). */
+int hstu_attn_bwd_silu(const HstuAttnBwdArgs* args, const void* q_pre, const void* k_pre, const void* v_pre, void* stream);
+
 /* Name of the kernel pair hstu_attn_bwd would launch for `args` (diagnostics;
  * static storage): "hstu_bwd_mfma_bf16", "hstu_bwd_general<float>", "hstu_bwd_general<bf16>",
  * "hstu_bwd_general<bf16, bf16 products>" or "invalid". */

@@ -163,6 +163,8 @@ def load():
     lib.hstu_embed_grad.argtypes = [C.POINTER(HstuEmbedGradArgs), C.c_void_p]
     lib.hstu_embed_grad_workspace_bytes.restype = C.c_size_t
     lib.hstu_embed_grad_workspace_bytes.argtypes = [C.c_int64, C.c_int64, C.c_int32]
+    lib.hstu_silu_bwd.restype = C.c_int
+    lib.hstu_silu_bwd.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_void_p]
     ver = lib.hstu_block_abi_version()
     if ver != ABI_VERSION:
       raise RuntimeError(f"libhstu_block.so has ABI {ver}, expected {ABI_VERSION}")

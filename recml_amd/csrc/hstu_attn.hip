@@ -3530,12 +3530,24 @@ __device__ __forceinline__ float silu_grad_log2(float u, float* fprime) {
   return sg;
 }
 
+// Two bf16 gradients times silu' at two bf16 values, rounded
+__device__ __forceinline__ uint32_t silu_bwd_pair(uint32_t d, uint32_t x) {
+  auto one = [](float dv, float xv) __attribute__((always_inline)) {
+    const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-LOG2E * xv));
+    return dv * (sg * __builtin_fmaf(xv, 1.0f - sg, 1.0f));
+  };
+  return pack_bf16(one(__builtin_bit_cast(float, d << 16), __builtin_bit_cast(float, x << 16)),
+                   one(__builtin_bit_cast(float, d & 0xffff0000u), __builtin_bit_cast(float, x & 0xffff0000u)));
+}
+
 // Turns a wave's 32 x D accumulator (lane (col m, half hh) holds channels 32 dvb + 8g + 4hh + t of
 // row m) into whole bf16 rows through the wave's own 32 x D x 2 bytes of LDS and stores rows
 // [row0, row0 + 32) that are below `rows`, rows at or past `n_live` as zeros.
+// pre (or null; laid out like dst): the rounded rows times silu'(pre), what a pass of its own over them would leave (78 k x 1536: 112 us
+// of a block's backward).
 template <int D>
 __device__ __forceinline__ void store_rows(const floatx16 (&acc)[D / 32], float scale, unsigned char* ot, bf16_t* __restrict__ dst,
-                                           int64_t row_stride, int row0, int n_live, int rows, int lane) {
+                                           const bf16_t* __restrict__ pre, int64_t row_stride, int row0, int n_live, int rows, int lane) {
   constexpr int CPR = D / 8, RPB = CPR >= 16 ? 1 : 16 / CPR;
   auto oswz = [](int row) { return (row / RPB) % CPR; };
   const int m = lane & 31, hh = lane >> 5;
@@ -3555,6 +3567,27 @@ __device__ __forceinline__ void store_rows(const floatx16 (&acc)[D / 32], float 
   }
   constexpr int ROWS_PER_STORE = 64 / CPR;
   const int rr = lane / CPR, cc = lane - rr * CPR;
+  if (pre) {
+    constexpr int N = 32 / ROWS_PER_STORE < 4 ? 32 / ROWS_PER_STORE : 4;       // rows of `pre` under way together
+#pragma unroll
+    for (int r0s = 0; r0s < 32; r0s += N * ROWS_PER_STORE) {
+      uint4 x[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int grow = row0 + r0s + i * ROWS_PER_STORE + rr;
+        x[i] = uint4{0u, 0u, 0u, 0u};
+        if (grow < n_live) x[i] = *(const uint4*)(pre + (int64_t)grow * row_stride + cc * 8);
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int row = r0s + i * ROWS_PER_STORE + rr, grow = row0 + row;
+        const uint4 val = *(const uint4*)(ot + row * (D * 2) + ((cc ^ oswz(row)) * 16));
+        const uint4 out = {silu_bwd_pair(val.x, x[i].x), silu_bwd_pair(val.y, x[i].y), silu_bwd_pair(val.z, x[i].z), silu_bwd_pair(val.w, x[i].w)};
+        if (grow < rows) *(uint4*)(dst + (int64_t)grow * row_stride + cc * 8) = out;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int r0s = 0; r0s < 32; r0s += ROWS_PER_STORE) {
     const int row = r0s + rr;
@@ -4250,7 +4283,7 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     }
   }
   // dQ^T[d][q] -> rows of dq (the ring is free: the loop ended on a barrier, no load is in flight)
-  store_rows<D>(acc, p.alpha * p.inv_n, smem + w * (32 * D * 2), dqg, p.q_st, r0, s.n_q, s.rows, lane);
+  store_rows<D>(acc, p.alpha * p.inv_n, smem + w * (32 * D * 2), dqg, p.q_pre ? (const bf16_t*)p.q_pre + s.bq : nullptr, p.q_st, r0, s.n_q, s.rows, lane);
 }
 
 // At d = 128 two 32 x 128 accumulators plus the K and V fragments are 192 registers before any
@@ -4931,6 +4964,8 @@ void hstu_bwd_dkv_mfma(const Params p) {
   }
   for (; t < nt; t += 2) block_pair(t);
 
+  const bf16_t* const k_pre = p.k_pre ? (const bf16_t*)p.k_pre + s.bk : nullptr;
+  const bf16_t* const v_pre = p.v_pre ? (const bf16_t*)p.v_pre + s.bv : nullptr;
   if (ACC_ASM) asm volatile("s_nop 15\n\ts_nop 15");   // the last product has left the pipeline before its result is read
   if constexpr (WIDE) {
     // The pair of waves on the same keys: the first sums and stores dK, the second dV; each hands the other's half over
@@ -4954,15 +4989,15 @@ void hstu_bwd_dkv_mfma(const Params p) {
     unsigned char* const ot = (unsigned char*)take;       // (read by this wave alone)
     if (qh == 0) {
       swap_halves(dka, dva);
-      store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, p.k_st, r0, s.n_kv, s.rows, lane);
+      store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, k_pre, p.k_st, r0, s.n_kv, s.rows, lane);
     } else {
       swap_halves(dva, dka);
-      store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, p.v_st, r0, s.n_kv, s.rows, lane);
+      store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, v_pre, p.v_st, r0, s.n_kv, s.rows, lane);
     }
   } else {
     unsigned char* ot = smem + w8 * (32 * D * 2);
-    store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, p.k_st, r0, s.n_kv, s.rows, lane);
-    store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, p.v_st, r0, s.n_kv, s.rows, lane);
+    store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, k_pre, p.k_st, r0, s.n_kv, s.rows, lane);
+    store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, v_pre, p.v_st, r0, s.n_kv, s.rows, lane);
   }
 }
 
@@ -5833,7 +5868,7 @@ const char* hstu_attn_bwd_variant(const HstuAttnBwdArgs* args) {
   return general_bwd_bf16_products(p) ? "hstu_bwd_general<bf16, bf16 products>" : "hstu_bwd_general<bf16>";
 }
 
-int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) {
+static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const void* k_pre, const void* v_pre, void* stream) {
   HstuAttnBwdArgs own;
   args = today(args, own);
   if (!args) return fail(HSTU_ERR_NULL, "args is null");
@@ -5854,15 +5889,27 @@ int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) {
   p.dout = args->dout; p.dq = args->dq; p.dk = args->dk; p.dv = args->dv;
   p.dpos = args->dpos_tab; p.dts = args->dts_tab;
   p.dbias = args->ddense_bias;
+  p.q_pre = q_pre; p.k_pre = k_pre; p.v_pre = v_pre;
   if (p.dbias && !p.dense_bias) return fail(HSTU_ERR_NULL, "ddense_bias needs the forward's dense_bias");
   hipStream_t st = (hipStream_t)stream;
-  if (bwd_mfma_eligible(args)) return launch_bwd_mfma(args, p, st);
+  if (bwd_mfma_eligible(args)) {
+    for (const void* x : {q_pre, k_pre, v_pre})
+      if ((uintptr_t)x & 15u) return fail(HSTU_ERR_SHAPE, "q_pre, k_pre and v_pre must be 16-byte aligned");
+    return launch_bwd_mfma(args, p, st);
+  }
+  if (q_pre || k_pre || v_pre) return fail(HSTU_ERR_SHAPE, "gradients through the activation are for the matrix-core backward's calls");
   if (f->mask_pitch > f->Lkv || f->bias_pitch > f->Lkv)
     return fail(HSTU_ERR_SHAPE, "rows of a dense operand further apart than Lkv are for the matrix-core kernels' calls");
   // (the general kernels sum the bucket table's gradient in LDS first, one float per entry)
   if (p.dts && p.ts_tab && p.ts_nb > 4095)
     return fail(HSTU_ERR_SHAPE, "the gradient of a timestamp table of more than 4096 entries is not supported, got %d", p.ts_nb + 1);
   return f->qk_dtype == HSTU_DTYPE_FP32 ? launch_bwd<float>(p, st) : launch_bwd<bf16_t>(p, st);
+}
+
+int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream) { return backward_call(args, nullptr, nullptr, nullptr, stream); }
+
+int hstu_attn_bwd_silu(const HstuAttnBwdArgs* args, const void* q_pre, const void* k_pre, const void* v_pre, void* stream) {
+  return backward_call(args, q_pre, k_pre, v_pre, stream);
 }
 
 int hstu_attn_fwd_noalloc(const HstuAttnFwdArgs* args, void* stream) {

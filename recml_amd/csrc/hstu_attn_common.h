@@ -88,6 +88,7 @@ struct Params {
   // backward pass: gradient of out in, gradients of q, k, v out (layouts of out, q, k, v), and
   // fp32 table gradients that are accumulated into (null = not wanted)
   const void* dout;
+  const void *q_pre, *k_pre, *v_pre;   // or null: q = silu(q_pre), ... and dq, dk, dv are gradients of those (matrix-core backward)
   void* dq;
   void* dk;
   void* dv;

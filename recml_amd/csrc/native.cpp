@@ -682,6 +682,7 @@ struct BlockBackward : public torch::autograd::Node {
     // attention: dq, dk, dv land next to it
     const Tensor d_attn = gate.da.view(attn.sizes());
     const Tensor pt = has_pos ? pos.unpack() : Tensor(), tt = has_ts ? ts_tab.unpack() : Tensor();
+    bool through_silu;
     {
       const Tensor q = projection_slice(uqkv, call, 1), k = projection_slice(uqkv, call, 2), v = projection_slice(uqkv, call, 3);
       HstuAttnBwdArgs b;
@@ -702,13 +703,16 @@ struct BlockBackward : public torch::autograd::Node {
         if (has_pos) { dpos = both.as_strided(pt.sizes(), pt.strides(), 0); b.dpos_tab = dpos.data_ptr<float>(); }
         if (has_ts) { dts = both.as_strided(tt.sizes(), tt.strides(), np); b.dts_tab = dts.data_ptr<float>(); }
       }
-      const int rc = hstu_attn_bwd(&b, stream_of(q));
+      // (through the projections' activation on the way, where those kernels run)
+      through_silu = w.projections && !strcmp(hstu_attn_bwd_variant(&b), "hstu_bwd_mfma_bf16");
+      const int rc = through_silu ? hstu_attn_bwd_silu(&b, at_column(pre, W), at_column(pre, 2 * W), at_column(pre, 3 * W), stream_of(q))
+                                  : hstu_attn_bwd(&b, stream_of(q));
       TORCH_CHECK(rc == HSTU_OK, "hstu_attn_bwd failed (", rc, "): ", hstu_attn_last_error());
       if (has_pos && want(P_COUNT)) r[1 + P_COUNT] = dpos;
       if (has_ts && want(P_COUNT + 1)) r[1 + P_COUNT + 1] = dts;
     }
     if (!w.projections) return r;
-    block_check(hstu_silu_bwd((void*)at_column(d_uqkv, W), 4 * W, at_column(pre, W), 4 * W, T, (int32_t)(3 * W), stream_of(x)), "hstu_silu_bwd");
+    if (!through_silu) block_check(hstu_silu_bwd((void*)at_column(d_uqkv, W), 4 * W, at_column(pre, W), 4 * W, T, (int32_t)(3 * W), stream_of(x)), "hstu_silu_bwd");
     // projections
     const Tensor dz = d_uqkv.view({T, 4 * W});
     if (w.kernels) {
