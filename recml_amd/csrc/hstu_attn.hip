@@ -1949,7 +1949,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
     // tiles (what decides which tiles are split), then the items.
     constexpr int SEG = 1024;
     __shared__ int wave_sums[4];
-    __shared__ int keys[SEG], firsts[SEG], order[SEG], tbase[SEG + 1];
+    __shared__ int keys[SEG], firsts[SEG], order[SEG], tbase[SEG + 1], level[SEG];
     const bool sorted = p.B <= SEG;
     int4* items = (int4*)(sched_out + 4);
     int walk_first = -1, walk_r = 0;      // memo of `walk` below: the first tile of the thread's run and its sequence
@@ -2059,7 +2059,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
       return c < MAX_CHUNKS ? c : MAX_CHUNKS;
     };
     // A thread's run of the segment's tiles, [f_lo, f_hi): one bisection finds the first tile's sequence, the
-    // rest follow in order.  fn(i, qt, nq, nk): index of the sequence within the segment, query tile, dimensions.
+    // rest follow in order.  fn(i, qt, nq, nk, r): index of the sequence within the segment, query tile, dimensions, place in `order`.
     auto walk = [&](int cnt, int f_lo, int f_hi, auto&& fn) {
       if (f_lo >= f_hi) return;
       // (a thread walks the same run several times over a segment: the bisection, a chain of dependent LDS reads,
@@ -2080,7 +2080,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
         int nq, nk, rows;
         dims(keys[i], nq, nk, rows);
         const int last = f_hi < t1 ? f_hi : t1;
-        for (; f < last; ++f) fn(i, (t1 - t0) - 1 - (f - t0), nq, nk);
+        for (; f < last; ++f) fn(i, (t1 - t0) - 1 - (f - t0), nq, nk, r);
       }
     };
     const int nseg = (p.B + SEG - 1) / SEG;
@@ -2092,7 +2092,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
         tiles = load_segment(sg * SEG, cnt);
         const int per = (tiles + 255) / 256;
         walk(cnt, tid * per < tiles ? tid * per : tiles, (tid + 1) * per < tiles ? (tid + 1) * per : tiles,
-             [&](int, int qt, int nq, int nk) { steps += steps_of(nq, nk, qt * BM); });
+             [&](int, int qt, int nq, int nk, int) { steps += steps_of(nq, nk, qt * BM); });
       }
       int total;
       block_scan(steps, total);
@@ -2116,16 +2116,68 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
       const int f_lo = tid * per < tiles ? tid * per : tiles, f_hi = (tid + 1) * per < tiles ? (tid + 1) * per : tiles;
       // the chunk slots this thread's tiles ask for, and where they start: a tile is split only while slots last
       int want = 0, asked = 0;
-      if (split_steps > 0)
-        walk(cnt, f_lo, f_hi, [&](int, int qt, int nq, int nk) {
+      bool split = split_steps > 0;
+      if (split && sorted) {      // (nothing to ask for where the longest sequence's keys stay below the threshold)
+        int nq, nk, rows;
+        dims(keys[order[0]], nq, nk, rows);
+        split = (nk + BN - 1) / BN > split_steps;
+      }
+      if (split)
+        walk(cnt, f_lo, f_hi, [&](int, int qt, int nq, int nk, int) {
           const int c = chunks_of(steps_of(nq, nk, qt * BM), split_steps);
           want += c > 1 ? c : 0;
         });
-      const int slot0 = split_steps > 0 ? slot_base + block_scan(want, asked) : 0;
+      const int slot0 = split ? slot_base + block_scan(want, asked) : 0;
+      if (asked == 0) {
+        // No tile is split: a tile's item lies at its number, but for the sequences from r0 on.  Those go tile index by tile index, the
+        // last first: under the causal mask that is by falling work.  (In the order above the tiles taken last are those of whole
+        // sequences, long tiles among them: a slot that draws one when the others are done runs on alone.  Forward, 8 x 2048, eight heads
+        // of 128, with two tiles a slot taken so: 145 -> 112 us; 64 x 2048: 890 -> 871; four: the same there, but 96 -> 99 instead of
+        // 94 on 128 jagged sequences of up to 1024, heads of 64: what runs together shares fewer keys through the cache.  Backward, whose
+        // kernels run fewer workgroups at once, with two / four: 568 -> 433 / 430, 3686 -> 3551 / 3510, 362 -> 350 / 328.)
+        const int per_slot = p.H >= 8 ? (p.n_slots + (p.H >> 3) - 1) / (p.H >> 3) : p.n_slots * (8 / p.H);
+        const bool by_level = sorted && p.causal && !p.mask && !p.dense_bias && p.n_qtiles <= SEG;
+        int r0 = cnt;
+        if (by_level) {
+          // r0: the last sequence with that many tiles from it on, or the first (a wave looks at 64 at a time)
+          const int most = tiles - p.level_tiles * per_slot, step = (cnt + 63) / 64, lane = tid & 63;
+          r0 = 0;
+          if (most > 0) {
+            r0 = step * (__popcll(__ballot(lane * step < cnt && tbase[lane * step < cnt ? lane * step : 0] <= most)) - 1);
+            if (step > 1) {
+              const int r = r0 + lane;
+              r0 += __popcll(__ballot(lane < step && r < cnt && tbase[r < cnt ? r : 0] <= most)) - 1;
+            }
+          }
+          // level[t]: first how many of them have a tile t (the first ones have), then the sum of those for higher t
+          for (int r = r0 + tid; r < cnt; r += 256) {
+            const int n = tbase[r + 1] - tbase[r], n_next = r + 1 < cnt ? tbase[r + 2] - tbase[r + 1] : 0;
+            for (int t = n_next; t < n; ++t) level[t] = r + 1 - r0;
+          }
+          __syncthreads();
+          const int n_max = tbase[r0 + 1] - tbase[r0];
+          for (int t0 = 0, above = 0; t0 < n_max; t0 += 256) {
+            const int t = n_max - 1 - (t0 + tid);
+            int sum;
+            const int before = above + block_scan(t >= 0 ? level[t] : 0, sum);
+            if (t >= 0) level[t] = before;
+            above += sum;
+          }
+          __syncthreads();
+        }
+        int f = f_lo;
+        walk(cnt, f_lo, f_hi, [&](int i, int qt, int, int, int r) {
+          const int at = item_base + (r < r0 ? f : tbase[r0] + level[qt] + (r - r0));
+          if (at < p.items_max) items[at] = int4{sg * SEG + i, qt | (1 << 24), firsts[i], keys[i]};
+          ++f;
+        });
+        item_base += tiles;
+        continue;
+      }
       // one walk shared by the count and the write
       auto emit = [&](int base, bool write) {
         int n = 0, slot = slot0;
-        walk(cnt, f_lo, f_hi, [&](int i, int qt, int nq, int nk) {
+        walk(cnt, f_lo, f_hi, [&](int i, int qt, int nq, int nk, int) {
           int c = chunks_of(steps_of(nq, nk, qt * BM), split_steps), ps = 0;
           if (c > 1) {
             ps = slot;
@@ -5737,6 +5789,7 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   const WorkspacePlan ws = plan_workspace(&f, false, ~(size_t)0, false);
   Params q = p;
   q.mask_pres = 1;
+  q.level_tiles = 4;
   q.no_stream = (b->fwd.flags & HSTU_FWD_COMPILER_SCHEDULED_BLOCKS) ? 1 : 0;
   if (int rc = setup_workspace(&f, ws, q, st)) return rc;
   if (q.d_qk == 128) return launch_bwd_mfma_d<128>(q, st);
@@ -5959,6 +6012,7 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // (a buffer that is missing is an error all the same: which calls use it is not the caller's to know)
       if (int rc2 = check_workspace(args, ws)) return rc2;
       if (q.whole_window && !(args->flags & HSTU_FWD_PREPARE_ONLY)) return f8 ? launch_mfma<true>(q, st) : launch_mfma<false>(q, st);
+      q.level_tiles = 2;
       if (int rc2 = setup_workspace(args, ws, q, st)) return rc2;
       if (args->flags & HSTU_FWD_PREPARE_ONLY) return HSTU_OK;
       // Resident workgroups over the work list, where that loop is built (d = 128 in bf16, lengths or no mask)

@@ -60,6 +60,7 @@ struct Params {
   // workgroup that arrives last at the tile's counter sums them and writes the rows.
   int32_t split_cap;         // chunk slots of the partial buffer (per head)
   int32_t n_slots;           // workgroups that run at once per XCD (what the split decision balances for)
+  int32_t level_tiles;       // tiles per slot that the work list's end holds by falling work (see hstu_prepare)
   const int32_t* mask_range; // workspace: per (mask batch, query tile) the first 32-key step with a kept pair and one past the last
   int32_t whole_window;      // forward: the position table as the caller gave it, no workspace (WHOLE instances)
   int32_t persist;           // forward: resident workgroups that loop over the work list

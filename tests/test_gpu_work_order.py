@@ -1,0 +1,65 @@
+"""The work list's order: every tile of every sequence is done once, whatever the lengths and wherever the part of the list that goes by
+tile index begins."""
+
+import pytest
+import torch
+
+import recml_amd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,L,H,d,kind,jagged", [
+    (1, 513, 8, 64, "full", True),               # one sequence, the shortest that has a list
+    (40, 1100, 16, 32, "full", True),            # 360 tiles, 128 (forward) and 256 (backward) of them at the list's end by tile index
+    (40, 1100, 16, 32, "mixed", True),
+    (40, 1100, 16, 32, "mixed", False),          # (padded: the rows past a length are tiles of their own, stored as zeros)
+    (6, 2300, 8, 128, "mixed", True),            # all by tile index
+    (24, 640, 2, 64, "mixed", True),             # fewer heads than XCDs
+    (9, 700, 12, 32, "none", True),              # no tokens but those of the last sequence
+    (1030, 530, 1, 32, "mixed", True),           # more sequences than are ordered at a time
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_every_tile_once(gpu, B, L, H, d, kind, jagged, causal):
+  """The backward of the batch equals, bit by bit, that of each sequence alone: its row gradients do not depend on the list.  The
+  forward's do where a tile's keys are split: sums of fp32 terms in another order, rounded to bf16: a last place of the row's largest
+  values, 2^-7 of them.  Outputs start as NaN, so that a tile left out shows."""
+  g = torch.Generator().manual_seed(B + L)
+  if kind == "full":
+    lens = torch.full((B,), L)
+  elif kind == "none":
+    lens = torch.zeros(B, dtype=torch.long)
+    lens[-1] = L
+  else:
+    lens = torch.randint(0, L + 1, (B,), generator=g)
+    for i, n in enumerate((0, 1, 127, 128, 129, L)):
+      lens[(7 * i) % B] = n
+  off = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)])
+  rows = (int(off[-1]),) if jagged else (B, L)
+  q, k, v, dout = ((torch.randn(rows + (H, d), generator=g) * 0.5).to("cuda:0", torch.bfloat16) for _ in range(4))
+  pos = (torch.randn(H, 2 * L - 1, generator=g) * 0.2).to("cuda:0")
+  kw = dict(causal=causal, alpha=d ** -0.5, n=1024, pos_bias=pos)
+  batch = dict(seq_offsets=off.int().to("cuda:0"), max_len=L) if jagged else dict(seq_lens=lens.int().to("cuda:0"))
+  nan = lambda t: torch.full_like(t, float("nan"))
+  out = recml_amd.hstu_attention(q, k, v, out=nan(q), **batch, **kw)
+  grads = [nan(q) for _ in range(3)]
+  variant = []
+  recml_amd.hstu_attention_bwd(q, k, v, dout, grads_out=grads, _variant_out=variant, **batch, **kw)
+  assert variant == ["hstu_bwd_mfma_bf16"]
+  for b in range(B) if B <= 40 else range(0, B, 41):
+    n = int(lens[b])
+    at = slice(int(off[b]), int(off[b]) + n) if jagged else (b, slice(0, n))
+    if not jagged:
+      for t in (out, *grads):
+        assert bool((t[b, n:] == 0).all())
+    if n == 0:
+      continue
+    one = dict(seq_offsets=torch.tensor([0, n], dtype=torch.int32, device="cuda:0"), max_len=L)
+    want = recml_amd.hstu_attention(q[at], k[at], v[at], **one, **kw).float()
+    scale = want.abs().amax((-1, -2), keepdim=True)
+    assert bool(((out[at].float() - want).abs() <= 2.0 ** -7 * scale).all())
+    for got, ref in zip(grads, recml_amd.hstu_attention_bwd(q[at], k[at], v[at], dout[at], table_grads=False, **one, **kw)):
+      assert torch.equal(got[at], ref)
+  if B > 40:
+    for t in (out, *grads):
+      assert bool(torch.isfinite(t).all())
