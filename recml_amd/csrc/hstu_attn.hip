@@ -1674,9 +1674,17 @@ __device__ __forceinline__ bool work_of_block(const Params& p, unsigned block, W
     work_from_item(p, item, h, wk);
     return true;
   }
-  // without a list: one entry per (sequence, head, query tile), tiles from the last one down, never split
-  const int bhk = j / p.n_qtiles;
-  const int qt = p.n_qtiles - 1 - (j - bhk * p.n_qtiles);
+  // without a list: one entry per (sequence, head, query tile), tiles from the last one down, never split; sequence by sequence or,
+  // where level_tiles asks for it, all sequences' last tiles first (see hstu_prepare)
+  int bhk, qt;
+  if (p.level_tiles) {
+    const int per_xcd = (p.B * p.H + 7) >> 3, back = j / per_xcd;
+    bhk = j - back * per_xcd;
+    qt = p.n_qtiles - 1 - back;
+  } else {
+    bhk = j / p.n_qtiles;
+    qt = p.n_qtiles - 1 - (j - bhk * p.n_qtiles);
+  }
   const int bh = bhk * 8 + xcd;
   if (bh >= p.B * p.H) return false;
   wk.b = bh / p.H; wk.h = bh - wk.b * p.H; wk.qt = qt; wk.chunk = 0; wk.n_chunks = 1; wk.pslot = 0;
@@ -5789,7 +5797,10 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   const WorkspacePlan ws = plan_workspace(&f, false, ~(size_t)0, false);
   Params q = p;
   q.mask_pres = 1;
-  q.level_tiles = 4;
+  // (without a list: a batch that the chip holds at once in the forward takes these kernels a round or two.  Causal, 32 x 512, eight heads
+  // of 64: 113 -> 85 us; 64 x up to 512, four heads: 76 -> 58; 16 x 512, eight heads of 128: 92 -> 73.  More tiles: sequence by sequence,
+  // which share their keys through the cache.)
+  q.level_tiles = ws.sched_bytes || (q.causal && (long long)q.B * q.n_qtiles * q.H <= 1024) ? 4 : 0;
   q.no_stream = (b->fwd.flags & HSTU_FWD_COMPILER_SCHEDULED_BLOCKS) ? 1 : 0;
   if (int rc = setup_workspace(&f, ws, q, st)) return rc;
   if (q.d_qk == 128) return launch_bwd_mfma_d<128>(q, st);
@@ -6012,7 +6023,7 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // (a buffer that is missing is an error all the same: which calls use it is not the caller's to know)
       if (int rc2 = check_workspace(args, ws)) return rc2;
       if (q.whole_window && !(args->flags & HSTU_FWD_PREPARE_ONLY)) return f8 ? launch_mfma<true>(q, st) : launch_mfma<false>(q, st);
-      q.level_tiles = 2;
+      q.level_tiles = ws.sched_bytes ? 2 : 0;
       if (int rc2 = setup_workspace(args, ws, q, st)) return rc2;
       if (args->flags & HSTU_FWD_PREPARE_ONLY) return HSTU_OK;
       // Resident workgroups over the work list, where that loop is built (d = 128 in bf16, lengths or no mask)

@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
     (6, 2300, 8, 128, "mixed", True),            # all by tile index
     (24, 640, 2, 64, "mixed", True),             # fewer heads than XCDs
     (9, 700, 12, 32, "none", True),              # no tokens but those of the last sequence
+    (16, 500, 4, 64, "mixed", True),             # no list: the backward takes all sequences' last tiles first
+    (15, 500, 3, 128, "mixed", False),           # the same with XCDs that have one sequence less than others
     (1030, 530, 1, 32, "mixed", True),           # more sequences than are ordered at a time
 ])
 @pytest.mark.parametrize("causal", [True, False])
