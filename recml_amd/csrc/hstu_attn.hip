@@ -1651,7 +1651,7 @@ __device__ __forceinline__ void work_from_item(const Params& p, const int4& item
 __device__ __forceinline__ bool work_of_block(const Params& p, unsigned block, Work& wk) {
   const int xcd = block & 7, j = block >> 3;
   if (p.sched) {
-    // from the work list: with H >= 8 head h runs on XCD h % 8, else 8 / H items share a round
+    // from the work list: with H >= 8 head h runs on XCD h % 8, else 8 / H items share a round (other head counts: see below)
     int it, h;
     if (p.mask || p.dense_bias) {
       // Dense operands are shared by the heads, not by the query tiles: the H workgroups of an item
@@ -1663,8 +1663,16 @@ __device__ __forceinline__ bool work_of_block(const Params& p, unsigned block, W
       const int grp = li / nq;
       it = (grp * 8 + xcd) * nq + (li - grp * nq);
     }
-    else if (p.H >= 8) { const int hx = p.H >> 3; it = j / hx; h = (j - it * hx) * 8 + xcd; }
-    else          { const int r = 8 / p.H;   it = j * r + xcd / p.H; h = xcd % p.H; }
+    else if (!(p.H & 7)) { const int hx = p.H >> 3; it = j / hx; h = (j - it * hx) * 8 + xcd; }
+    else if (p.H == 1 || p.H == 2 || p.H == 4) { const int r = 8 / p.H; it = j * r + xcd / p.H; h = xcd % p.H; }
+    else {
+      // Other head counts: with g their largest divisor of 8, a group of 8 / g items has 8 (H / g) jobs, H / g for each XCD, dealt
+      // head by head: the tiles of a (sequence, head) meet on 8 / g XCDs at most, and each takes the longest left of its share.
+      const int g = p.H & -p.H, per = 8 / g, k = p.H / g;
+      const int grp = j / k, i = xcd * k + (j - grp * k);
+      h = i / per;
+      it = grp * per + (i - h * per);
+    }
     // the item is read before the count is checked (the grid never reaches past the list's capacity):
     // both loads miss the cache, and one after the other they cost a workgroup twice the latency
     // (the dense mapping rounds its grid up to whole rounds of eight runs: indices past the capacity read item 0)
@@ -2104,9 +2112,8 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
       }
       int total;
       block_scan(steps, total);
-      // steps one slot of an XCD gets on average: with H >= 8 an XCD runs H / 8 heads of every item,
-      // else 8 / H XCDs share the items of one head
-      const long long per_xcd = p.H >= 8 ? (long long)total * (p.H >> 3) : (long long)total / (8 / p.H);
+      // steps one slot of an XCD gets on average: an XCD runs H / 8 heads of every item
+      const long long per_xcd = (long long)total * p.H / 8;
       const long long avg = (per_xcd + p.n_slots - 1) / p.n_slots;
       // A tile is split when it alone is more than twice that average: its chunks cost a round trip of
       // fp32 partial sums through memory, so tiles near the average are left whole.  (Measured, kernel
@@ -2143,7 +2150,7 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
         // of 128, with two tiles a slot taken so: 145 -> 112 us; 64 x 2048: 890 -> 871; four: the same there, but 96 -> 99 instead of
         // 94 on 128 jagged sequences of up to 1024, heads of 64: what runs together shares fewer keys through the cache.  Backward, whose
         // kernels run fewer workgroups at once, with two / four: 568 -> 433 / 430, 3686 -> 3551 / 3510, 362 -> 350 / 328.)
-        const int per_slot = p.H >= 8 ? (p.n_slots + (p.H >> 3) - 1) / (p.H >> 3) : p.n_slots * (8 / p.H);
+        const int per_slot = (8 * p.n_slots + p.H - 1) / p.H;
         const bool by_level = sorted && p.causal && !p.mask && !p.dense_bias && p.n_qtiles <= SEG;
         int r0 = cnt;
         if (by_level) {
@@ -5314,14 +5321,22 @@ WorkspacePlan plan_workspace(const HstuAttnFwdArgs* a, bool allow_split = true, 
   const int n_qtiles = (a->L + BM - 1) / BM;
   const bool jag = a->layout == HSTU_LAYOUT_JAGGED;
   // A work list built on the device spares the launch of workgroups that would find nothing to do
-  // (a jagged batch with a long maximum length and mostly short sequences is mostly such).  Its
-  // head mapping needs H to divide 8 or 8 to divide H; its builder is one workgroup.
+  // (a jagged batch with a long maximum length and mostly short sequences is mostly such), and
+  // the longest tiles go first.  Its builder is one workgroup.
   // A batch so small that one workgroup per (sequence, head, query tile) fits the chip at once, with tiles of at
   // most 16 steps, goes without: nothing is left to order or to balance, no tile is long enough for a split to pay
   // for its partial sums, and building the list would cost the call more than the kernel gains by it (measured:
   // 32 sequences of up to 512 tokens, 4 heads, d = 64: the call 28.7 -> 20.3 us, the kernel alone 19.6 -> 17.8).
   const bool small = (long long)a->B * n_qtiles * a->H <= (a->d_qk > 64 ? 512 : 1024) && a->Lkv <= 16 * BN;
-  const bool list = (a->H % 8 == 0 || 8 % a->H == 0) && a->B <= 8192 && !small;
+  // Head counts that neither divide 8 nor are divided by it have one from two rounds of tiles on, of work enough to pay for building it
+  // (and where the workspace has the room).  Forward / backward without and with one: 64 x up to 2048 of power-law length, 12 heads of
+  // 128: 282 -> 223 / 1169 -> 913 us; 30 x up to 1500, 3 of 128: 74 -> 61 / 271 -> 216; 128 x up to 1024, 3 of 64: 56 -> 54 / 190 -> 152;
+  // below the line, 64 x up to 512, 12 of 64: 32 -> 35 / 109 -> 92; 96 x up to 300, 12 of 64: 26 -> 34 / 99 -> 90; 8 x 1024, 12 of 64, one
+  // round: 38 -> 51 / 87 -> 95.
+  const bool odd_heads = a->H % 8 && 8 % a->H;
+  const long long tiles_all = (long long)a->B * n_qtiles * a->H;
+  const bool pays = tiles_all >= (a->d_qk > 64 ? 1024 : 2048) && tiles_all * ((a->Lkv + BN - 1) / BN) * a->d_qk >= 4000000;
+  bool list = a->B <= 8192 && !small && (!odd_heads || pays);
   // Key-range splitting (decided per tile by the preparation kernel, which sees the lengths) needs the list.
   // (no tile of at most 8 steps is ever split; a tile takes at most MAX_CHUNKS slots)
   const long long t128_all = jag ? a->total_tokens / BM + a->B : (long long)a->B * n_qtiles;
@@ -5367,7 +5382,12 @@ WorkspacePlan plan_workspace(const HstuAttnFwdArgs* a, bool allow_split = true, 
     if (w.total() <= max_bytes) break;
     if (w.split_cap == 0) {
       // still too large without any chunk slot: the descriptors go (every block then looks its pairs up)
-      if (!w.desc_bytes) break;
+      if (!w.desc_bytes) {
+        if (!list || !odd_heads) break;
+        list = false;
+        w.items_max = 0; w.sched_bytes = 0;
+        continue;
+      }
       w.desc_bytes = w.tquad_bytes = 0; w.desc_pitch = w.desc_tiles = 0;
       continue;
     }
@@ -5467,7 +5487,8 @@ long long mfma_grid(const Params& p) {
       const long long groups = (n + p.n_qtiles - 1) / p.n_qtiles;     // runs of n_qtiles items, eight runs a round
       return 8LL * ((groups + 7) / 8) * p.n_qtiles * p.H;
     }
-    const long long rounds = p.H >= 8 ? n * (p.H / 8) : (n + 8 / p.H - 1) / (8 / p.H);
+    const int g = p.H & 7 ? p.H & -p.H : 8, per = 8 / g;      // (see work_of_block)
+    const long long rounds = (n + per - 1) / per * (p.H / g);
     return 8LL * rounds;
   }
   return 8LL * p.n_qtiles * (((long long)p.B * p.H + 7) / 8);
@@ -5744,7 +5765,7 @@ bool bwd_mfma_eligible(const HstuAttnBwdArgs* b) {
   // q rows are addressed with 32-bit byte offsets here, like k and v rows in the forward
   if ((int64_t)f.L * f.q_stride_t * 2 >= (1LL << 31) || (int64_t)f.L * f.o_stride_t * 2 >= (1LL << 31) ||
       f.q_stride_t <= 0 || f.o_stride_t <= 0) return false;
-  const WorkspacePlan ws = plan_workspace(&f, false, ~(size_t)0, false);
+  const WorkspacePlan ws = plan_workspace(&f, false, f.workspace ? f.workspace_bytes : 0, false);
   return ws.total() == 0 || (f.workspace && f.workspace_bytes >= ws.total() && ((uintptr_t)f.workspace & 255u) == 0);
 }
 
@@ -5794,7 +5815,7 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   HstuAttnFwdArgs f = b->fwd;
   f.out = (void*)b->dout;
   f.flags &= ~HSTU_FWD_WORKSPACE_PREPARED;   // the backward lays the work list out without key-range splits
-  const WorkspacePlan ws = plan_workspace(&f, false, ~(size_t)0, false);
+  const WorkspacePlan ws = plan_workspace(&f, false, f.workspace ? f.workspace_bytes : 0, false);
   Params q = p;
   q.mask_pres = 1;
   // (without a list: a batch that the chip holds at once in the forward takes these kernels a round or two.  Causal, 32 x 512, eight heads
@@ -6032,7 +6053,7 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // end of the launch, where each workgroup finishes whatever it drew last, costs more than the items'
       // starts save: 69 -> 77 us.)  The padded layout with lengths leaves the host guessing the number of
       // items: one workgroup per item there.
-      const bool can_stay = q.sched && q.ctr && q.d_qk == 128 && !f8 && !q.mask && !q.dense_bias && q.mask_mode != HSTU_MASK_SEGMENT;
+      const bool can_stay = q.sched && q.ctr && !(q.H % 8 && 8 % q.H) && q.d_qk == 128 && !f8 && !q.mask && !q.dense_bias && q.mask_mode != HSTU_MASK_SEGMENT;
       const bool count_known = q.jagged || !q.seq_lens;
       const long long tiles = q.jagged ? args->total_tokens / BM + args->B : (long long)args->B * q.n_qtiles;
       const long long jobs_per_xcd = q.H >= 8 ? tiles * (q.H >> 3) : tiles / (8 / q.H);

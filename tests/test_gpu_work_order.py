@@ -1,10 +1,13 @@
 """The work list's order: every tile of every sequence is done once, whatever the lengths and wherever the part of the list that goes by
 tile index begins."""
 
+import ctypes
+
 import pytest
 import torch
 
 import recml_amd
+from recml_amd import _lib, hstu_ops
 
 pytestmark = pytest.mark.gpu
 
@@ -16,6 +19,9 @@ pytestmark = pytest.mark.gpu
     (40, 1100, 16, 32, "mixed", False),          # (padded: the rows past a length are tiles of their own, stored as zeros)
     (6, 2300, 8, 128, "mixed", True),            # all by tile index
     (24, 640, 2, 64, "mixed", True),             # fewer heads than XCDs
+    (40, 1100, 12, 32, "mixed", True),           # head counts dealt to the XCDs in groups of items
+    (90, 900, 3, 64, "mixed", False),
+    (31, 1000, 6, 128, "full", True),
     (9, 700, 12, 32, "none", True),              # no tokens but those of the last sequence
     (16, 500, 4, 64, "mixed", True),             # no list: the backward takes all sequences' last tiles first
     (15, 500, 3, 128, "mixed", False),           # the same with XCDs that have one sequence less than others
@@ -65,3 +71,31 @@ def test_every_tile_once(gpu, B, L, H, d, kind, jagged, causal):
   if B > 40:
     for t in (out, *grads):
       assert bool(torch.isfinite(t).all())
+
+
+def test_without_room_for_a_list(gpu):
+  """Head counts that neither divide 8 nor are divided by it: a call without a workspace, or with too little for the list, is taken."""
+  g = torch.Generator().manual_seed(3)
+  lens, L, H, d = [900, 0, 300, 1024] + 18 * [40], 1024, 12, 64
+  q, k, v = ((torch.randn(sum(lens), H, d, generator=g) * 0.5).to("cuda:0", torch.bfloat16) for _ in range(3))
+  off = torch.tensor([0] + lens, device="cuda:0").cumsum(0).int()
+  want = recml_amd.hstu_attention(q, k, v, seq_offsets=off, max_len=L).float()
+  lib = _lib.load()
+  stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+  for room in (0, 256):
+    out = torch.full_like(q, float("nan"))
+    args, keep = hstu_ops.build_args(q, k, v, out, seq_offsets=off, max_len=L)
+    assert args.workspace_bytes > 256
+    args.workspace_bytes = room
+    args.workspace = args.workspace if room else None
+    assert lib.hstu_attn_fwd(ctypes.byref(args), stream) == 0
+    assert bool(((out.float() - want).abs() <= 2.0 ** -7 * want.abs().amax((-1, -2), keepdim=True)).all())
+    bwd = _lib.HstuAttnBwdArgs(struct_size=ctypes.sizeof(_lib.HstuAttnBwdArgs), version=_lib.ABI_VERSION, fwd=args)
+    grads = [torch.full_like(q, float("nan")) for _ in range(3)]
+    bwd.dout, bwd.dq, bwd.dk, bwd.dv = v.data_ptr(), *(t.data_ptr() for t in grads)
+    assert lib.hstu_attn_bwd_variant(ctypes.byref(bwd)) == b"hstu_bwd_mfma_bf16"
+    assert lib.hstu_attn_bwd(ctypes.byref(bwd), stream) == 0
+    for got, ref in zip(grads, recml_amd.hstu_attention_bwd(q, k, v, v, seq_offsets=off, max_len=L)):
+      assert torch.equal(got, ref)
+    torch.cuda.synchronize()
+    del keep
