@@ -110,7 +110,7 @@ typedef struct HstuNormGateBwdArgs {
   float* dbeta;
   void* workspace;
   size_t workspace_bytes;
-  const void* u_pre;          /* or null.  Given: u = silu(u_pre), and du is the gradient of u_pre (u's, rounded, times silu') */
+  const void* u_pre;          /* or null.  Given: u = silu(u_pre) (and is not read), and du is the gradient of u_pre (u's, rounded, times silu') */
   int64_t u_pre_stride;
   const void* add;            /* or null.  Given: added to the rounded da (a gradient that reaches `a` another way) */
   int64_t add_stride;

@@ -217,17 +217,16 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
         if (p.u) {
           float bt[8], uu[8], y[8];
           unpack8(*(const uint4*)(p.beta + e), bt);
-          unpack8(*(const uint4*)(p.u + row * p.u_stride + e), uu);
+          // (the gate itself from u_pre too: 80 of 480 MB not read, 9.5 us less at 78 k rows of 512)
+          unpack8(p.u_pre ? *(const uint4*)(p.u_pre + row * p.u_pre_stride + e) : *(const uint4*)(p.u + row * p.u_stride + e), uu);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             y[i] = g[c][i] * __builtin_fmaf((x[c][i] - mean) * rstd, gm[i], bt[i]);
+            if (p.u_pre) {
+              y[i] = round_bf16(y[i]) * silu_grad(uu[i]);     // (du in bf16, as the attention's dq, dk, dv are)
+              uu[i] = round_bf16(silu(uu[i]));
+            }
             g[c][i] *= uu[i];
-          }
-          if (p.u_pre) {
-            float z[8];
-            unpack8(*(const uint4*)(p.u_pre + row * p.u_pre_stride + e), z);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = round_bf16(y[i]) * silu_grad(z[i]);     // (du in bf16, as the attention's dq, dk, dv are)
           }
           *(uint4*)(p.du + row * p.du_stride + e) = pack8(y);
         }
