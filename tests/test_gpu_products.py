@@ -79,6 +79,33 @@ def test_gathered_table_gradient(gpu, rows, keys, width, scale):
   assert torch.equal(out.cpu().long(), want)
 
 
+@pytest.mark.parametrize("width", [72, 136, 512])
+@pytest.mark.parametrize("scale", [1.0, 1.7])
+def test_long_runs_in_the_order_of_their_tokens(gpu, width, scale):
+  """Runs around the batches that are loaded together: every partial sum rounded to bf16, in the tokens' order, bit by bit."""
+  lens = [33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 321, 1000]
+  g = torch.Generator().manual_seed(width)
+  ids = torch.cat([torch.full((n,), k) for k, n in enumerate(lens)])
+  ids = ids[torch.randperm(len(ids), generator=g)]
+  grad = torch.randn(len(ids), width, generator=g).to(torch.bfloat16)
+  want = torch.zeros(len(lens), width, dtype=torch.bfloat16)
+  for t, k in enumerate(ids.tolist()):
+    want[k] = (want[k].float() + (grad[t].float() * scale).to(torch.bfloat16).float()).to(torch.bfloat16)
+  dev = torch.device("cuda:0")
+  d, idd, out = grad.to(dev), ids.to(dev), torch.full((len(lens), width), float("nan"), dtype=torch.bfloat16, device=dev)
+  lib = _lib_block.load()
+  ws = torch.empty(lib.hstu_embed_grad_workspace_bytes(len(ids), len(lens), width) + 256, dtype=torch.uint8, device=dev)
+  a = _lib_block.HstuEmbedGradArgs()
+  a.struct_size, a.version = C.sizeof(a), _lib_block.ABI_VERSION
+  a.rows, a.keys, a.width, a.scale = len(ids), len(lens), width, scale
+  a.g, a.g_stride, a.ids, a.out = d.data_ptr(), width, idd.data_ptr(), out.data_ptr()
+  a.workspace = (ws.data_ptr() + 255) // 256 * 256
+  a.workspace_bytes = ws.numel() - (a.workspace - ws.data_ptr())
+  assert lib.hstu_embed_grad(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+  torch.cuda.synchronize()
+  assert torch.equal(out.cpu(), want)
+
+
 @pytest.mark.parametrize("B,L,keys,width,by_position", [(128, 9, 9, 72, 2), (192, 3, 5, 136, 2), (20, 40, 40, 128, 2), (128, 9, 9, 64, 1), (30, 7, 9, 136, 1)])
 @pytest.mark.parametrize("packed", [False, True])
 def test_position_table_gradient(gpu, B, L, keys, width, by_position, packed):
