@@ -119,6 +119,8 @@ typedef struct HstuNormGateBwdArgs {
 
 size_t hstu_norm_gate_bwd_workspace_bytes(int64_t rows, int32_t width);
 int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* args, void* stream);
+/* The same with dgamma and dbeta bf16 [width]: the sums rounded (the parameters' own type). */
+int hstu_norm_gate_bwd_rounded(const HstuNormGateBwdArgs* args, void* stream);
 
 /* out[m, n] = silu(sum_k x[m, k] w[k, n] + bias[n]); x: bf16 [M, K] (row stride
  * x_stride), w: bf16 [K, N] contiguous, bias: bf16 [N] or null, out: bf16

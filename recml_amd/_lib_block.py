@@ -16,6 +16,7 @@ EXPORTS = (
     "hstu_block_last_error",
     "hstu_norm_gate_fwd",
     "hstu_norm_gate_bwd",
+    "hstu_norm_gate_bwd_rounded",
     "hstu_norm_gate_bwd_workspace_bytes",
     "hstu_gemm_silu_fwd",
     "hstu_gemm_silu_workspace_bytes",
@@ -147,6 +148,8 @@ def load():
     lib.hstu_norm_gate_fwd.argtypes = [C.POINTER(HstuNormGateArgs), C.c_void_p]
     lib.hstu_norm_gate_bwd.restype = C.c_int
     lib.hstu_norm_gate_bwd.argtypes = [C.POINTER(HstuNormGateBwdArgs), C.c_void_p]
+    lib.hstu_norm_gate_bwd_rounded.restype = C.c_int
+    lib.hstu_norm_gate_bwd_rounded.argtypes = [C.POINTER(HstuNormGateBwdArgs), C.c_void_p]
     lib.hstu_norm_gate_bwd_workspace_bytes.restype = C.c_size_t
     lib.hstu_norm_gate_bwd_workspace_bytes.argtypes = [C.c_int64, C.c_int32]
     lib.hstu_gemm_silu_fwd.restype = C.c_int

@@ -290,8 +290,9 @@ __global__ __launch_bounds__(256) void hstu_norm_gate_bwd(const NormGateBwdParam
 // [0, width) go to dgamma, [width, 2 width) to dbeta.  nb = 0 writes zeros.  A workgroup of 1024
 // threads takes 32 columns: 32 groups of threads each add every 32nd row (four sums in flight per
 // thread: the loop is nothing but dependent loads otherwise), then the groups' sums are added through LDS.
-__global__ __launch_bounds__(1024) void hstu_colsum(const float* __restrict__ part, int nb, int width, float* __restrict__ dgamma,
-                                                    float* __restrict__ dbeta) {
+template <typename T>
+__global__ __launch_bounds__(1024) void hstu_colsum(const float* __restrict__ part, int nb, int width, T* __restrict__ dgamma,
+                                                    T* __restrict__ dbeta) {
   __shared__ float red[32][33];
   const int cl = threadIdx.x & 31, rg = threadIdx.x >> 5;
   const int col = blockIdx.x * 32 + cl, n2 = 2 * width;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(1024) void hstu_colsum(const float* __restrict__ pa
     float s = 0.f;
 #pragma unroll
     for (int g = 0; g < 32; ++g) s += red[g][cl];
-    if (col < width) dgamma[col] = s; else dbeta[col - width] = s;
+    if (col < width) dgamma[col] = (T)s; else dbeta[col - width] = (T)s;
   }
 }
 
@@ -833,7 +834,10 @@ size_t hstu_norm_gate_bwd_workspace_bytes(int64_t rows, int32_t width) {
   return (size_t)norm_gate_bwd_blocks(rows, width) * 2u * (size_t)width * sizeof(float);
 }
 
-int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
+}  // extern "C"
+
+template <typename T>
+static int norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
   HstuNormGateBwdArgs own;
   a = block_today(a, own, offsetof(HstuNormGateBwdArgs, u_pre), sizeof(HstuNormGateBwdArgs));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
@@ -875,12 +879,19 @@ int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "norm-gate backward kernel launch: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(hstu_colsum, dim3((unsigned)((2 * a->width + 31) / 32)), dim3(1024), 0, st, (const float*)a->workspace, nb, a->width,
-                     a->dgamma, a->dbeta);
+  hipLaunchKernelGGL(hstu_colsum<T>, dim3((unsigned)((2 * a->width + 31) / 32)), dim3(1024), 0, st, (const float*)a->workspace, nb, a->width,
+                     (T*)a->dgamma, (T*)a->dbeta);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "column-sum kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
+
+extern "C" {
+
+int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) { return norm_gate_bwd<float>(a, stream); }
+
+// (a launch for each vector's conversion otherwise: 4 us each, twenty of them in a ranking model's step)
+int hstu_norm_gate_bwd_rounded(const HstuNormGateBwdArgs* a, void* stream) { return norm_gate_bwd<bf16_t>(a, stream); }
 
 int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   HstuEmbedNormArgs own;

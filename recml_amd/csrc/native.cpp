@@ -28,6 +28,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -443,14 +444,14 @@ void norm(const Tensor& out, Rows a, Rows u, const Tensor& gamma, const Tensor& 
   block_check(hstu_norm_gate_fwd(&g, stream_of(out)), "hstu_norm_gate_fwd");
 }
 
-// The gradients of norm(): da (and du), and the fp32 column sums [2, width] it returns.
+// The gradients of norm(): da (and du), and the column sums it returns: those of gamma and beta, fp32 or (rounded) in the parameters' bf16.
 struct NormGrad {
   Rows a, u{nullptr, 0}, dout, u_pre{nullptr, 0}, add{nullptr, 0};
   void* da; int64_t da_stride;
   void* du = nullptr; int64_t du_stride = 0;
   Tensor row_map;
 };
-Tensor norm_backward(const NormGrad& n, const Tensor& gamma, const Tensor& beta, int64_t rows, int64_t width, double eps) {
+std::pair<Tensor, Tensor> norm_backward(const NormGrad& n, const Tensor& gamma, const Tensor& beta, int64_t rows, int64_t width, double eps, bool rounded) {
   HstuNormGateBwdArgs g;
   memset(&g, 0, sizeof(g));
   g.struct_size = sizeof(g);
@@ -461,13 +462,14 @@ Tensor norm_backward(const NormGrad& n, const Tensor& gamma, const Tensor& beta,
   g.u_pre = n.u_pre.p; g.u_pre_stride = n.u_pre.stride; g.add = n.add.p; g.add_stride = n.add.stride;
   if (n.row_map.defined()) g.row_map = n.row_map.const_data_ptr<int32_t>();
   g.gamma = gamma.const_data_ptr(); g.beta = beta.const_data_ptr();
-  const Tensor sums = at::empty({2, width}, gamma.options().dtype(at::kFloat).requires_grad(false));
-  g.dgamma = sums.data_ptr<float>(); g.dbeta = g.dgamma + width;
+  const auto sums = gamma.options().dtype(rounded ? at::kBFloat16 : at::kFloat).requires_grad(false);
+  const std::pair<Tensor, Tensor> r(at::empty(gamma.sizes(), sums), at::empty(beta.sizes(), sums));
+  g.dgamma = (float*)r.first.data_ptr(); g.dbeta = (float*)r.second.data_ptr();
   const int64_t ws = (int64_t)hstu_norm_gate_bwd_workspace_bytes(rows, (int32_t)width);
   const Tensor buf = at::empty({std::max<int64_t>(ws, 16)}, gamma.options().dtype(at::kByte).requires_grad(false));
   g.workspace = buf.data_ptr(); g.workspace_bytes = (size_t)buf.numel();
-  block_check(hstu_norm_gate_bwd(&g, stream_of(gamma)), "hstu_norm_gate_bwd");
-  return sums;
+  block_check((rounded ? hstu_norm_gate_bwd_rounded : hstu_norm_gate_bwd)(&g, stream_of(gamma)), "hstu_norm_gate_bwd");
+  return r;
 }
 
 void gemm(int op, int64_t M, Rows x, std::initializer_list<const Tensor*> ws, int64_t K, int64_t N, const Tensor& out, const Tensor& bias = Tensor(),
@@ -602,9 +604,7 @@ struct NormOp {
       n.du = du_out.data_ptr(); n.du_stride = du_out.stride(0);
     }
     if (add.defined()) n.add = {add.const_data_ptr(), add.stride(0)};
-    const Tensor sums = norm_backward(n, gamma, beta, rows, W, eps);
-    dgamma = sums[0];
-    dbeta = sums[1];
+    std::tie(dgamma, dbeta) = norm_backward(n, gamma, beta, rows, W, eps, true);
   }
 };
 
@@ -676,8 +676,8 @@ struct BlockBackward : public torch::autograd::Node {
     auto rows_of = [&](const Tensor& t, int64_t stride) { return t.as_strided({T, W}, {stride, 1}, t.storage_offset()); };
     const NormOp gate(rows_of(attn, W), rows_of(uqkv, 4 * W), p[P_ATTN_G], p[P_ATTN_B], d_gated, call.eps, rows_of(d_uqkv, 4 * W), rows_of(pre, 4 * W),
                       Tensor());
-    if (want(P_ATTN_G)) r[1 + P_ATTN_G] = gate.dgamma.to(at::kBFloat16).view(p[P_ATTN_G].sizes());
-    if (want(P_ATTN_B)) r[1 + P_ATTN_B] = gate.dbeta.to(at::kBFloat16).view(p[P_ATTN_B].sizes());
+    if (want(P_ATTN_G)) r[1 + P_ATTN_G] = gate.dgamma;
+    if (want(P_ATTN_B)) r[1 + P_ATTN_B] = gate.dbeta;
     if (!w.attention) return r;
     // attention: dq, dk, dv land next to it
     const Tensor d_attn = gate.da.view(attn.sizes());
@@ -730,8 +730,8 @@ struct BlockBackward : public torch::autograd::Node {
       const Tensor d_normed = input_gradient(dz, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W);
       // (with the residual's share added)
       const NormOp in(x.view({T, D}), Tensor(), p[P_IN_G], p[P_IN_B], d_normed, call.eps, Tensor(), Tensor(), dout);
-      if (want(P_IN_G)) r[1 + P_IN_G] = in.dgamma.to(at::kBFloat16);
-      if (want(P_IN_B)) r[1 + P_IN_B] = in.dbeta.to(at::kBFloat16);
+      if (want(P_IN_G)) r[1 + P_IN_G] = in.dgamma;
+      if (want(P_IN_B)) r[1 + P_IN_B] = in.dbeta;
       if (task_should_compute_output(0)) r[0] = in.da.view(x.sizes());
     }
     return r;
@@ -817,12 +817,12 @@ struct EmbedBackward : public torch::autograd::Node {
     n.a = {x.const_data_ptr(), W};
     n.dout = {dout.const_data_ptr(), W};
     n.da = da.data_ptr(); n.da_stride = W;
-    const Tensor sums = norm_backward(n, ga, be, T, W, eps);
+    const auto sums = norm_backward(n, ga, be, T, W, eps, true);
     if (task_should_compute_output(0)) r[0] = table_gradient({vocab, 0, scale, 0}, da, ids, Tensor());
     // (packed rows gather their positions; in a padded batch the table's rows are broadcast over the sequences: one fp32 sum then)
     if (positions && task_should_compute_output(1)) r[1] = table_gradient({positions, L, 1.0, packed ? 1 : 2}, da, Tensor(), map);
-    if (task_should_compute_output(2)) r[2] = sums[0].to(ga.scalar_type()).view(ga.sizes());
-    if (task_should_compute_output(3)) r[3] = sums[1].to(be.scalar_type()).view(be.sizes());
+    if (task_should_compute_output(2)) r[2] = sums.first;
+    if (task_should_compute_output(3)) r[3] = sums.second;
     return r;
   }
 };
@@ -856,10 +856,10 @@ struct FinalNormBackward : public torch::autograd::Node {
     n.dout = {dout.const_data_ptr(), W};
     n.da = da.data_ptr(); n.da_stride = W;
     if (packed) n.row_map = row_map.unpack();
-    const Tensor sums = norm_backward(n, ga, be, rows, W, eps);
+    const auto sums = norm_backward(n, ga, be, rows, W, eps, true);
     if (task_should_compute_output(0)) r[0] = da;
-    if (task_should_compute_output(1)) r[1] = sums[0].to(ga.scalar_type()).view(ga.sizes());
-    if (task_should_compute_output(2)) r[2] = sums[1].to(be.scalar_type()).view(be.sizes());
+    if (task_should_compute_output(1)) r[1] = sums.first;
+    if (task_should_compute_output(2)) r[2] = sums.second;
     return r;
   }
 };
@@ -1126,7 +1126,8 @@ PyObject* norm_gate_bwd(PyObject*, PyObject* const* a, Py_ssize_t count) {
     for (const Tensor* t : {&u, &du, &u_pre, &add})
       if (t->defined() && !fits(*t)) Py_RETURN_NONE;
     if ((du.defined() || u_pre.defined()) && !u.defined()) Py_RETURN_NONE;
-    Tensor da, sums;
+    Tensor da;
+    std::pair<Tensor, Tensor> sums;
     without_lock(attn, [&] {
       da = fresh(attn, {rows, W});
       if (u.defined() && !du.defined()) du = fresh(attn, {rows, W});
@@ -1140,11 +1141,11 @@ PyObject* norm_gate_bwd(PyObject*, PyObject* const* a, Py_ssize_t count) {
       }
       if (u_pre.defined()) n.u_pre = {u_pre.const_data_ptr(), u_pre.stride(0)};
       if (add.defined()) n.add = {add.const_data_ptr(), add.stride(0)};
-      sums = norm_backward(n, gamma, beta, rows, W, eps);
+      sums = norm_backward(n, gamma, beta, rows, W, eps, false);
       return true;
     });
     return Py_BuildValue("(NNNN)", THPVariable_Wrap(da), du.defined() ? THPVariable_Wrap(du) : (Py_INCREF(Py_None), Py_None),
-                         THPVariable_Wrap(sums[0]), THPVariable_Wrap(sums[1]));
+                         THPVariable_Wrap(sums.first.view({W})), THPVariable_Wrap(sums.second.view({W})));
   });
 }
 

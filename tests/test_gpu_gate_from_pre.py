@@ -54,3 +54,23 @@ def test_gate_from_its_pre_activation(gpu, rows, width):
     grads.append((da, du, sums))
   for x, y in zip(*grads):
     assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("rows,width", [(0, 16), (3, 8), (1500, 72), (5000, 512)])
+def test_rounded_sums(gpu, rows, width):
+  """The parameters' gradients in bf16: the fp32 sums, rounded."""
+  lib = _lib_block.load()
+  g = torch.Generator().manual_seed(rows)
+  rn = lambda *s: torch.randn(*s, generator=g).to("cuda:0", torch.bfloat16)
+  a, dout, gamma, beta, da = rn(rows, width), rn(rows, width), rn(width), rn(width), rn(rows, width)
+  buf = torch.empty(max(int(lib.hstu_norm_gate_bwd_workspace_bytes(rows, width)), 16), dtype=torch.uint8, device="cuda:0")
+  got = []
+  for call, dtype in ((lib.hstu_norm_gate_bwd, torch.float32), (lib.hstu_norm_gate_bwd_rounded, torch.bfloat16)):
+    sums = torch.full((2, width + 4), 7.0, device="cuda:0", dtype=dtype)
+    n = _lib_block.HstuNormGateBwdArgs(struct_size=C.sizeof(_lib_block.HstuNormGateBwdArgs), version=_lib_block.ABI_VERSION, rows=rows, width=width,
+                                       eps=1e-6, a=a.data_ptr(), dout=dout.data_ptr(), a_stride=width, dout_stride=width, gamma=gamma.data_ptr(),
+                                       beta=beta.data_ptr(), da=da.data_ptr(), da_stride=width, dgamma=sums[0].data_ptr(),
+                                       dbeta=sums[1].data_ptr(), workspace=buf.data_ptr(), workspace_bytes=buf.numel())
+    assert call(C.byref(n), _stream()) == 0
+    got.append(sums)
+  assert torch.equal(got[0].to(torch.bfloat16), got[1])
