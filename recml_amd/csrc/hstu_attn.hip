@@ -6041,10 +6041,13 @@ int hstu_attn_fwd(const HstuAttnFwdArgs* args, void* stream) {
       // kernel takes the table itself, and the preparation is not launched.
       q.whole_window = ws.sched_bytes == 0 && q.pos_tab && !q.ts_tab && !q.mask && !q.dense_bias && q.mask_mode != HSTU_MASK_SEGMENT &&
                        q.Lkv <= WHOLE_KEYS;
+      // (without a list, causal, at most a round: workgroups go to an XCD's CUs in turn, and with 2, 4, ... tiles a sequence one CU got the
+      // long tiles of several.  32 x 512, eight heads of 64: 30 -> 22 us, kernel; 128 x 256, four: 20 -> 16; 256 x 512, one: 52 -> 38; 32 x up
+      // to 512, four: 15.1 -> 14.5.)
+      q.level_tiles = ws.sched_bytes || (q.causal && (long long)q.B * q.n_qtiles * q.H <= 1024) ? 2 : 0;
       // (a buffer that is missing is an error all the same: which calls use it is not the caller's to know)
       if (int rc2 = check_workspace(args, ws)) return rc2;
       if (q.whole_window && !(args->flags & HSTU_FWD_PREPARE_ONLY)) return f8 ? launch_mfma<true>(q, st) : launch_mfma<false>(q, st);
-      q.level_tiles = ws.sched_bytes ? 2 : 0;
       if (int rc2 = setup_workspace(args, ws, q, st)) return rc2;
       if (args->flags & HSTU_FWD_PREPARE_ONLY) return HSTU_OK;
       // Resident workgroups over the work list, where that loop is built (d = 128 in bf16, lengths or no mask)
