@@ -61,12 +61,16 @@ __device__ __forceinline__ const char* scalar_ptr(const void* p) {
 
 #define HSTU_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | ((((n) >> 4) & 3) << 14)) | 0x0F70)
 
-// 16 bytes that this launch does not read again: not kept in this XCD's L2, where the operands are (the reader is a later launch,
-// on any XCD).  74 k x 512 -> 2048, out alone / with the pre-activation: 240 -> 213, 282 -> 226 us.
-__device__ __forceinline__ void store_past_cache(bf16_t* to, const uint4& v) {
+// 16 bytes of the output.  PAST: this launch does not read them again and they are not kept in this XCD's L2, where the operands are (the
+// reader is a later launch, on any XCD).  74 k x 512 -> 2048, out alone / with the pre-activation: 240 -> 213, 282 -> 226 us.  Not the small
+// tiles: their outputs are small enough for the next launch to find them in a cache (18 k rows of 32 to 128: the attention behind it
+// 28.7 us with PAST, 27.3 without).
+template <bool PAST>
+__device__ __forceinline__ void store_out(bf16_t* to, const uint4& v) {
   typedef uint32_t words __attribute__((ext_vector_type(4)));
   const words x = {v.x, v.y, v.z, v.w};
-  __builtin_nontemporal_store(x, (words*)to);
+  if constexpr (PAST) __builtin_nontemporal_store(x, (words*)to);
+  else *(words*)to = x;
 }
 
 // One workgroup: a tile of 64 MB output rows x 32 NB WN output columns, 2 x WN waves of 32 MB x 32 NB.  The contraction runs in
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
           const uint4 z = pack8(x[i]);
-          if (inside(i)) store_past_cache(g.pre + (int64_t)(mb + RPI * i) * g.out_stride + n, z);
+          if (inside(i)) store_out<(MB >= 4)>(g.pre + (int64_t)(mb + RPI * i) * g.out_stride + n, z);
           unpack8(z, x[i]);
         }
       }
@@ -455,7 +459,7 @@ __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams
       bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)mb * g.out_stride + (n - osl * g.out_slab);
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
-        if (inside(i)) store_past_cache(o + (int64_t)(RPI * i) * g.out_stride, pack8(x[i]));
+        if (inside(i)) store_out<(MB >= 4)>(o + (int64_t)(RPI * i) * g.out_stride, pack8(x[i]));
     }
     __builtin_amdgcn_wave_barrier();
   }
