@@ -1965,7 +1965,8 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
     // tiles (what decides which tiles are split), then the items.
     constexpr int SEG = 1024;
     __shared__ int wave_sums[4];
-    __shared__ int keys[SEG], firsts[SEG], order[SEG], tbase[SEG + 1], level[SEG];
+    constexpr int LEVELS = 256;   // (LDS that every workgroup of the launch is given: those that read a mask need all the residency there is)
+    __shared__ int keys[SEG], firsts[SEG], order[SEG], tbase[SEG + 1], level[LEVELS];
     const bool sorted = p.B <= SEG;
     int4* items = (int4*)(sched_out + 4);
     int walk_first = -1, walk_r = 0;      // memo of `walk` below: the first tile of the thread's run and its sequence
@@ -2151,7 +2152,8 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
         // 94 on 128 jagged sequences of up to 1024, heads of 64: what runs together shares fewer keys through the cache.  Backward, whose
         // kernels run fewer workgroups at once, with two / four: 568 -> 433 / 430, 3686 -> 3551 / 3510, 362 -> 350 / 328.)
         const int per_slot = (8 * p.n_slots + p.H - 1) / p.H;
-        const bool by_level = sorted && p.causal && !p.mask && !p.dense_bias && p.n_qtiles <= SEG;
+        // (one or two tiles a sequence: nothing to gain)
+        const bool by_level = sorted && p.causal && !p.mask && !p.dense_bias && p.n_qtiles > 2 && p.n_qtiles <= LEVELS;
         int r0 = cnt;
         if (by_level) {
           // r0: the last sequence with that many tiles from it on, or the first (a wave looks at 64 at a time)
