@@ -4170,12 +4170,18 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
             float4{ds[4 * g + 0] * p.inv_n, ds[4 * g + 1] * p.inv_n, ds[4 * g + 2] * p.inv_n, ds[4 * g + 3] * p.inv_n};
       float* dbp = p.dbias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0) + (int64_t)r0 * p.Lkv + kbs;
       const int col = lane & 31;
+      // (all of them under way before the first addition: read and added one by one, each waits for LDS by itself)
+      float vals[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int rr = 2 * i + (lane >> 5), rw = 32 * w + rr;
-        const float val = *(const float*)(Bk(st) + rw * 128 + (((col >> 2) ^ (rw & 7)) * 16) + (col & 3) * 4);
-        if (val != 0.f) atomicAdd(dbp + (int64_t)rr * p.Lkv + col, val);
+        const int rw = 32 * w + 2 * i + (lane >> 5);
+        vals[i] = *(const float*)(Bk(st) + rw * 128 + (((col >> 2) ^ (rw & 7)) * 16) + (col & 3) * 4);
       }
+      __builtin_amdgcn_sched_barrier(0);
+      float* to = dbp + (int64_t)(lane >> 5) * p.Lkv + col;
+#pragma unroll
+      for (int i = 0; i < 16; ++i, to += 2 * (int64_t)p.Lkv)
+        if (vals[i] != 0.f) atomicAdd(to, vals[i]);
     }
     if (want_dpos) {
       // Pair (row m, key offset c = 8g + 4hh + tt) lies on diagonal c - m.  Within a row of 16 lanes (p = m % 16, query half
