@@ -1,9 +1,11 @@
 """A whole block in one launch (short sequences, head dims of 16) against the same block in its steps, which a call that wants gradients
 takes."""
 
+import numpy as np
 import pytest
 import torch
 
+from oracle import hstu_block_oracle as BO
 from recml_amd import _lib_block
 from recml_amd.hstu_layer import HSTUBlock
 
@@ -61,6 +63,59 @@ def test_block_in_one_launch(gpu, B, L, H, lens, pos, biases, jagged):
       got_bad = run(bad)
     for b in range(B):
       assert torch.equal(got_bad[b, :lens[b]], got[b, :lens[b]])
+
+
+@pytest.mark.parametrize("B,L,H,lens,pos,biases", [
+    (1, 1, 2, [1], None, False),
+    (3, 17, 2, [17, 16, 3], "shared", True),
+    (2, 33, 4, [33, 32], "heads", True),
+    (2, 64, 4, [64, 63], None, False),
+    (4, 50, 4, [50, 7, 50, 33], "heads", False),
+])
+def test_against_the_oracle(gpu, B, L, H, lens, pos, biases):
+  """The launch against the block in 64 bits.  Five of its values are rounded to 8 bits, one behind the other (normed; u, q, k, v; the
+  attention; gated; the output): 2^-9 / sqrt(3) each in the mean, with signs that do not agree, so sqrt(5) of that for the rows' norm:
+  2^-8.6; single values up to four times as far."""
+  assert _taken(B, L, H) == 1
+  D = 16 * H
+  g = torch.Generator().manual_seed(7 * B + L)
+  blk = HSTUBlock(D, H, dtype=BF, device=DEV, use_bias=biases, generator=g)
+  with torch.no_grad():
+    for prm in blk.parameters():
+      prm.add_((torch.randn(prm.shape, generator=g) * 0.1).to(DEV).to(BF))
+  x = torch.randn((B, L, D), generator=g).to(BF)
+  tab = None if pos is None else torch.randn((H if pos == "heads" else 1, 2 * L - 1), generator=g) * 0.3
+  with torch.no_grad():
+    got = blk(x.to(DEV), seq_lens=torch.tensor(lens, dtype=torch.int32, device=DEV), pos_bias=None if tab is None else tab.to(DEV))
+  got = got.double().cpu().numpy()
+  w = {k: v.detach().double().cpu().numpy() for k, v in blk.named_parameters()}
+  for b in range(B):
+    n = lens[b]
+    want = _oracle(x[b, :n].double().numpy(), w, H, L, tab)
+    diff = np.abs(got[b, :n] - want)
+    assert np.linalg.norm(diff) <= 2.0 ** -8 * np.linalg.norm(want)
+    assert diff.max() <= 2.0 ** -7 * np.abs(want).max()
+
+
+def _oracle(x, w, H, L, tab):
+  """What BO.hstu_block does for one sequence in a batch of length L, with a table per head (BO.hstu_block has one for all heads)."""
+  n, D = x.shape
+  hd = D // H
+  f = lambda name: w[name].reshape((D, H, hd) if name.endswith("_kernel") and name[0] in "uqkv" else (H, hd, D) if name == "output_kernel" else
+                                   (H, hd) if name.startswith("attn_ln") or (name.endswith("_bias") and name[0] in "uqkv") else (D,))
+  normed = BO.layer_norm(x, f("input_ln_gamma"), f("input_ln_beta"), 1e-6)
+  proj = {}
+  for c in "uqkv":
+    y = np.einsum("td,dnh->tnh", normed, f(c + "_kernel"))
+    proj[c] = BO.O.silu(y + f(c + "_bias") if c + "_bias" in w else y)
+  s = np.einsum("inh,jnh->nij", proj["q"], proj["k"])
+  if tab is not None:
+    i = np.arange(n)
+    s = s + tab.double().numpy()[:, (L - 1) + i[None, :] - i[:, None]]
+  p = np.where(np.tril(np.ones((n, n), bool))[None], BO.O.silu(s), 0.0) / L
+  attn = BO.layer_norm(np.einsum("nij,jnh->inh", p, proj["v"]), f("attn_ln_gamma"), f("attn_ln_beta"), 1e-6, axes=(-2, -1))
+  out = np.einsum("tnh,nhd->td", proj["u"] * attn, f("output_kernel")) + x
+  return out + f("output_bias") if "output_bias" in w else out
 
 
 def test_shapes_beside_it(gpu):

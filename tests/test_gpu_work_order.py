@@ -99,3 +99,60 @@ def test_without_room_for_a_list(gpu):
       assert torch.equal(got, ref)
     torch.cuda.synchronize()
     del keep
+
+
+def _rows_alone(kind, B, L, H, d, g, dev="cuda:0"):
+  """A batch with one kind of operand beside q, k and v, and a function that gives the operand's part for one sequence."""
+  q, k, v, dout = ((torch.randn(B, L, H, d, generator=g) * 0.5).to(dev, torch.bfloat16) for _ in range(4))
+  lens = torch.randint(1, L + 1, (B,), generator=g)
+  lens[0] = L
+  i = torch.arange(L)
+  if kind == "dense":
+    mask = ((i[None, :, None] >= i[None, None, :]) & (i[None, None, :] < lens[:, None, None])).to(dev)
+    bias = (torch.randn(B, L, L, generator=g) * 0.2).to(dev)
+    return q, k, v, dout, lambda at: dict(mask=mask[at], bias=bias[at], causal=False)
+  ids = torch.where(i[None] < (lens // 2)[:, None], 1, torch.where(i[None] < lens[:, None], 2, 0)).int().to(dev)
+  return q, k, v, dout, lambda at: dict(q_segment_ids=ids[at], kv_segment_ids=ids[at])
+
+
+@pytest.mark.parametrize("kind", ["dense", "segments"])
+@pytest.mark.parametrize("B,L,H,d", [(30, 1000, 3, 64), (12, 1024, 6, 128), (24, 640, 12, 32), (24, 640, 2, 64)])
+def test_every_tile_once_with_other_operands(gpu, kind, B, L, H, d):
+  """As above where the batch brings a dense mask and bias, or segment ids, at head counts on either side of the XCDs' eight."""
+  g = torch.Generator().manual_seed(B * L + H)
+  q, k, v, dout, part = _rows_alone(kind, B, L, H, d, g)
+  kw = dict(alpha=d ** -0.5, n=1024)
+  nan = lambda t: torch.full_like(t, float("nan"))
+  whole = slice(None)
+  out = recml_amd.hstu_attention(q, k, v, out=nan(q), **part(whole), **kw)
+  grads, variant = [nan(q) for _ in range(3)], []
+  recml_amd.hstu_attention_bwd(q, k, v, dout, grads_out=grads, _variant_out=variant, **part(whole), **kw)
+  assert variant == ["hstu_bwd_mfma_bf16"]
+  for b in range(0, B, 3):
+    at = slice(b, b + 1)
+    want = recml_amd.hstu_attention(q[at], k[at], v[at], **part(at), **kw).float()
+    assert bool(((out[at].float() - want).abs() <= 2.0 ** -7 * want.abs().amax((-1, -2), keepdim=True)).all())
+    for got, ref in zip(grads, recml_amd.hstu_attention_bwd(q[at], k[at], v[at], dout[at], **part(at), **kw)):
+      assert torch.equal(got[at], ref)
+  for t in (out, *grads):
+    assert bool(torch.isfinite(t).all())
+
+
+@pytest.mark.parametrize("H", [2, 3, 6, 12])
+def test_every_tile_once_in_fp8(gpu, H):
+  """The forward's list with 8-bit queries and keys, against each sequence alone."""
+  B, L, d = 20, 1200, 128
+  g = torch.Generator().manual_seed(H)
+  lens = torch.randint(1, L + 1, (B,), generator=g)
+  off = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)])
+  q, k = ((torch.randn(int(off[-1]), H, d, generator=g) * 0.5).to("cuda:0").to(torch.float8_e4m3fn) for _ in range(2))
+  v = torch.randn(int(off[-1]), H, d, generator=g).to("cuda:0", torch.bfloat16)
+  pos = (torch.randn(H, 2 * L - 1, generator=g) * 0.2).to("cuda:0")
+  kw = dict(alpha=d ** -0.5, n=1024, pos_bias=pos)
+  out = torch.full_like(v, float("nan"))
+  recml_amd.hstu_attention(q, k, v, out=out, seq_offsets=off.int().to("cuda:0"), max_len=L, **kw)
+  for b in range(B):
+    at = slice(int(off[b]), int(off[b + 1]))
+    one = dict(seq_offsets=torch.tensor([0, int(lens[b])], dtype=torch.int32, device="cuda:0"), max_len=L)
+    want = recml_amd.hstu_attention(q[at], k[at], v[at], **one, **kw).float()
+    assert bool(((out[at].float() - want).abs() <= 2.0 ** -7 * want.abs().amax((-1, -2), keepdim=True)).all())
