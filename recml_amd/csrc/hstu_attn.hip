@@ -4043,7 +4043,7 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
           }
           bk_lane = en.b_near;
         } else {
-// every pair looked up, four at a time: the reads of four buckets under way together, and a group's values under way with the
+          // every pair looked up, four at a time: the reads of four buckets under way together, and a group's values under way with the
           // next group's buckets (one by one, as the compiler has them for want of registers, each waits for LDS by itself)
           if (TG) {
             float f[2][4], thr[2][4], val[4];
@@ -4335,7 +4335,11 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
     __syncthreads();
   }
   if (want_dpos && t_lo < nt) {
-    // what waits for a block that does not come (a wave ends at most 96 keys before the tile does, so nothing of it is flushed yet)
+    // What waits for a block that does not come (a wave ends at most 96 keys before the tile does, so nothing of it is flushed yet).
+    // A read and a write without a lock, though waves w and w + 2 share a ring: where both have something to add their slots differ.  A
+    // live wave has run a block (a table comes with L = Lkv).  One whose last block the diagonal or the window ends waits with zeros:
+    // what waits lies above that block's diagonals c - m = 0, so above every pair the mask keeps, and it writes what it read.  Those that
+    // the sequence's end stops have the same diag_next, and slots 64 apart.
     if (lane < 32 && wave_live) {
       float* slot = TgBase + (w & 1) * TG_RING + ((diag_next + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_RING - 1));
       *slot += diag_wait;

@@ -3,8 +3,9 @@
 //
 // One workgroup per sequence of up to 64 positions, at head dims of 16 and widths of 32 and 64: everything between the block's input
 // and its output stays in LDS (95 KB).  What bounds such a block is none of its work (2 MFLOP and 45 KB a sequence) but its launches:
-// as five kernels a block of 32 sequences of 50 takes 18.1 us of the GPU and 19 of the host, as this one 8.4 and 8.  Every value that those kernels round to bf16 on its way through memory is rounded here, and none else: the weights of
-// the attention stay in fp32, as the kernels for head dims of 16 have them.
+// as five kernels a block of 32 sequences of 50 takes 18.1 us of the GPU and 19 of the host, as this one 8.4 and 8.  Every value that
+// those kernels round to bf16 on its way through memory is rounded here, and none else: the weights of the attention stay in fp32, as
+// the kernels for head dims of 16 have them.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
