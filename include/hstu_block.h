@@ -290,6 +290,12 @@ typedef struct HstuBlockSmallArgs {
 
 int hstu_block_small_takes(int32_t B, int32_t L, int32_t heads, int32_t head_dim, int32_t width);
 int hstu_block_small_fwd(const HstuBlockSmallArgs* args, void* stream);
+/* n (1 .. HSTU_BLOCK_SMALL_STACK) such blocks one behind the other in one launch: blocks[0].tokens through all of them to
+ * blocks[n - 1].out (the others' tokens and out are not looked at), then, with end_gamma and end_beta [width], a layer norm of the rows
+ * (hstu.py:619).  The blocks share everything but their parameters and eps. */
+#define HSTU_BLOCK_SMALL_STACK 16
+int hstu_block_small_stack_fwd(const HstuBlockSmallArgs* blocks, int32_t n, const void* end_gamma, const void* end_beta, float end_eps,
+                               void* stream);
 
 int hstu_block_abi_version(void);
 const char* hstu_block_last_error(void);

@@ -30,6 +30,7 @@ EXPORTS = (
     "hstu_gemm_workspace_bytes",
     "hstu_block_small_takes",
     "hstu_block_small_fwd",
+    "hstu_block_small_stack_fwd",
 )
 
 

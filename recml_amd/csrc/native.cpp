@@ -549,20 +549,37 @@ bool block_ready(const Tensor& tokens, const Tensor (&p)[P_COUNT], const BlockCa
   return true;
 }
 
-// The block as one launch, where there is one for its shape and options; false: nothing has been done.
-bool small_block(Tensor& out, const Tensor& tokens, const Tensor (&p)[P_COUNT], const BlockCall& c, const Tensor& pos, const Tensor& ts_tab, const Tensor& bias) {
+// Whether a block of these sizes and options can be part of one launch for whole blocks.
+bool small_shape(const BlockCall& c, const Tensor& ts_tab, const Tensor& bias) {
   const Options& o = c.opts;
   const int64_t L = c.L ? c.L : o.max_len, B = c.L ? c.B : o.seq_offsets.numel() - 1;
-  if (ts_tab.defined() || bias.defined() || o.mask.defined() || o.dropout_p > 0.0 || o.window >= 0 || !o.causal || c.D != c.H * c.hd || L > 64 ||
-      c.D > 64 || B > 1 << 20 || !hstu_block_small_takes((int32_t)B, (int32_t)L, (int32_t)c.H, (int32_t)c.hd, (int32_t)c.D)) return false;
-  HstuBlockSmallArgs a;
+  return !ts_tab.defined() && !bias.defined() && !o.mask.defined() && o.dropout_p == 0.0 && o.window < 0 && o.causal && c.D == c.H * c.hd && L <= 64 &&
+         c.D <= 64 && B <= 1 << 20 && hstu_block_small_takes((int32_t)B, (int32_t)L, (int32_t)c.H, (int32_t)c.hd, (int32_t)c.D);
+}
+
+// Whether its lengths or offsets and its table are as the launch reads them.
+bool small_ready(const Tensor& tokens, const BlockCall& c, const Tensor& pos) {
+  const Options& o = c.opts;
+  const auto dev = tokens.device();
+  if (o.timestamps.defined()) return false;
+  if (!c.L) {
+    if (o.max_len < 1 || o.seq_lens.defined() || !plain(o.seq_offsets, dev, at::kInt) || o.seq_offsets.dim() != 1 || o.seq_offsets.numel() < 1) return false;
+  } else if (o.max_len >= 0 || (o.seq_lens.defined() && (!plain(o.seq_lens, dev, at::kInt) || o.seq_lens.dim() != 1 || o.seq_lens.size(0) != c.B))) {
+    return false;
+  }
+  int64_t heads, width;
+  return !pos.defined() || (table(pos, dev, c.H, &heads, &width) && width == 2 * (c.L ? c.L : o.max_len) - 1);
+}
+
+void fill_small(HstuBlockSmallArgs& a, const Tensor (&p)[P_COUNT], const BlockCall& c, const Tensor& pos) {
+  const Options& o = c.opts;
   memset(&a, 0, sizeof(a));
   a.struct_size = sizeof(a);
   a.version = HSTU_BLOCK_ABI_VERSION;
-  a.B = (int32_t)B; a.L = (int32_t)L; a.heads = (int32_t)c.H; a.head_dim = (int32_t)c.hd; a.width = (int32_t)c.D;
+  a.B = (int32_t)(c.L ? c.B : o.seq_offsets.numel() - 1);
+  a.L = (int32_t)(c.L ? c.L : o.max_len);
+  a.heads = (int32_t)c.H; a.head_dim = (int32_t)c.hd; a.width = (int32_t)c.D;
   a.eps = (float)c.eps; a.alpha = (float)o.alpha; a.inv_n = (float)(1.0 / o.n);
-  out = fresh(tokens, tokens.sizes());
-  a.tokens = tokens.const_data_ptr(); a.out = out.data_ptr();
   if (o.seq_lens.defined()) a.seq_lens = o.seq_lens.const_data_ptr<int32_t>();
   if (o.seq_offsets.defined()) a.seq_offsets = o.seq_offsets.const_data_ptr<int32_t>();
   a.in_gamma = p[P_IN_G].const_data_ptr(); a.in_beta = p[P_IN_B].const_data_ptr();
@@ -574,6 +591,15 @@ bool small_block(Tensor& out, const Tensor& tokens, const Tensor (&p)[P_COUNT], 
   a.w_out = p[P_OUT].const_data_ptr();
   if (p[P_OUT_B].defined()) a.b_out = p[P_OUT_B].const_data_ptr();
   if (pos.defined()) { a.pos_tab = pos.const_data_ptr<float>(); a.pos_heads = pos.dim() == 2 ? (int32_t)pos.size(0) : 1; }
+}
+
+// The block as one launch, where there is one for its shape and options; false: nothing has been done.
+bool small_block(Tensor& out, const Tensor& tokens, const Tensor (&p)[P_COUNT], const BlockCall& c, const Tensor& pos, const Tensor& ts_tab, const Tensor& bias) {
+  if (!small_shape(c, ts_tab, bias) || !small_ready(tokens, c, pos)) return false;
+  HstuBlockSmallArgs a;
+  fill_small(a, p, c, pos);
+  out = fresh(tokens, tokens.sizes());
+  a.tokens = tokens.const_data_ptr(); a.out = out.data_ptr();
   block_check(hstu_block_small_fwd(&a, stream_of(tokens)), "hstu_block_small_fwd");
   return true;
 }
@@ -1045,6 +1071,7 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
     Tensor out, normed, pre, uqkv, attn, gated;
     const bool ok = without_lock(tokens, [&] {
       const int64_t T = c.T, D = c.D, W = c.H * c.hd;
+      if (!graph && small_block(out, tokens, p, c, pos, ts_tab, bias)) return true;
       uqkv = fresh(tokens, {T, 4, c.H, c.hd});
       if (c.L) attn = fresh(tokens, {c.B, c.L, c.H, c.hd});
       else attn = fresh(tokens, {T, c.H, c.hd});
@@ -1052,7 +1079,6 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
       HstuAttnFwdArgs a;
       const Tensor q = projection_slice(uqkv, c, 1);
       if (!fill(a, q, projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
-      if (!graph && small_block(out, tokens, p, c, pos, ts_tab, bias)) return true;
       normed = fresh(tokens, {T, D});
       norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
       if (graph) pre = at::empty_like(uqkv);
@@ -1100,6 +1126,67 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
     PyObject* const sig = PyBytes_FromStringAndSize(shared.now.data(), (Py_ssize_t)shared.now.size());
     PyObject* const buf = shared.buf.defined() ? THPVariable_Wrap(shared.buf) : (Py_INCREF(Py_None), Py_None);
     return Py_BuildValue("(NNNO)", THPVariable_Wrap(std::move(out)), sig, buf, shared.reused ? Py_True : Py_False);
+  });
+}
+
+// blocks(tokens [.., D], (params, ...), heads, head_dim, eps, alpha, n, seq_lens, seq_offsets, max_len, pos, end_gamma, end_beta, end_eps) -> out
+// or None: several blocks one behind the other as one launch (a launch for every HSTU_BLOCK_SMALL_STACK of them), and with end_gamma a layer
+// norm behind the last.  Where there is no such launch, or a gradient is asked for, the blocks are called one by one.
+PyObject* blocks(PyObject*, PyObject* const* a, Py_ssize_t count) {
+  if (count != 14) {
+    PyErr_SetString(PyExc_TypeError, "blocks takes 14 arguments");
+    return nullptr;
+  }
+  return guarded([&]() -> PyObject* {
+    Tensor tokens, pos, end_gamma, end_beta;
+    BlockCall c;
+    Options& o = c.opts;
+    double end_eps;
+    if (!tensor_arg(a[0], &tokens) || !tokens.defined() || !PyTuple_CheckExact(a[1]) || !long_arg(a[2], &c.H) || !long_arg(a[3], &c.hd) ||
+        !float_arg(a[4], &c.eps) || !float_arg(a[5], &o.alpha) || !float_arg(a[6], &o.n) || !(o.n > 0.0) || !tensor_arg(a[7], &o.seq_lens) ||
+        !tensor_arg(a[8], &o.seq_offsets) || (a[9] != Py_None && !long_arg(a[9], &o.max_len)) || !tensor_arg(a[10], &pos) ||
+        !tensor_arg(a[11], &end_gamma) || !tensor_arg(a[12], &end_beta) || !float_arg(a[13], &end_eps)) Py_RETURN_NONE;
+    const int64_t n = PyTuple_GET_SIZE(a[1]);
+    if (n < 1 || !tokens.is_cuda() || tokens.dim() != (o.seq_offsets.defined() ? 2 : 3)) Py_RETURN_NONE;
+    o.causal = true;
+    c.D = tokens.size(-1);
+    c.B = tokens.dim() == 3 ? tokens.size(0) : 0;
+    c.L = tokens.dim() == 3 ? tokens.size(1) : 0;
+    c.T = tokens.dim() == 3 ? c.B * c.L : tokens.size(0);
+    if (!small_shape(c, Tensor(), Tensor()) || !small_ready(tokens, c, pos)) Py_RETURN_NONE;
+    const auto dev = tokens.device();
+    if (end_gamma.defined() && (!ready(end_gamma, dev) || !end_beta.defined() || !ready(end_beta, dev) || end_gamma.numel() != c.D || end_beta.numel() != c.D))
+      Py_RETURN_NONE;
+    auto differentiates = [](const Tensor& t) { return wants_grad({&t}) || dual({&t}); };
+    if (differentiates(tokens) || differentiates(pos) || differentiates(end_gamma) || differentiates(end_beta)) Py_RETURN_NONE;
+    std::vector<HstuBlockSmallArgs> args((size_t)n);
+    for (int64_t i = 0; i < n; ++i) {
+      Tensor p[P_COUNT];
+      PyObject* const own = PyTuple_GET_ITEM(a[1], i);
+      if (!PyTuple_CheckExact(own) || PyTuple_GET_SIZE(own) != P_COUNT) Py_RETURN_NONE;
+      for (int j = 0; j < P_COUNT; ++j)
+        if (!tensor_arg(PyTuple_GET_ITEM(own, j), &p[j]) || differentiates(p[j])) Py_RETURN_NONE;
+      if (!block_ready(tokens, p, c, false)) Py_RETURN_NONE;
+      fill_small(args[(size_t)i], p, c, pos);        // (the caller's tuples keep the parameters)
+    }
+    Tensor out;
+    without_lock(tokens, [&] {
+      const void* from = tokens.const_data_ptr();
+      for (int64_t i = 0; i < n; i += HSTU_BLOCK_SMALL_STACK) {
+        const int64_t m = std::min<int64_t>(n - i, HSTU_BLOCK_SMALL_STACK);
+        const bool last = i + m == n;
+        // (a launch in between: in place, its workgroups read and write rows of their own sequence only)
+        if (i == 0) out = fresh(tokens, tokens.sizes());
+        args[(size_t)i].tokens = from;
+        args[(size_t)(i + m - 1)].out = out.data_ptr();
+        block_check(hstu_block_small_stack_fwd(&args[(size_t)i], (int32_t)m, last && end_gamma.defined() ? end_gamma.const_data_ptr() : nullptr,
+                                               last && end_gamma.defined() ? end_beta.const_data_ptr() : nullptr, (float)end_eps, stream_of(tokens)),
+                    "hstu_block_small_stack_fwd");
+        from = out.const_data_ptr();
+      }
+      return true;
+    });
+    return THPVariable_Wrap(std::move(out));
   });
 }
 
@@ -1400,6 +1487,7 @@ PyMethodDef methods[] = {
      "One attention forward on arguments that are ready for the kernels; None when they are not."},
 #define HSTU_FAST(name, doc) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, doc}
     HSTU_FAST(block, "One HSTU block forward (differentiable where asked)."),
+    HSTU_FAST(blocks, "Several narrow HSTU blocks in inference as one launch."),
     HSTU_FAST(norm_gate_bwd, "The gradients of the norm and gate step."),
     HSTU_FAST(embed, "The model's front end: gather, position embedding, layer norm."),
     HSTU_FAST(final_norm, "The closing layer norm, into the padded batch where asked."),

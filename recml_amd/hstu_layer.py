@@ -362,6 +362,23 @@ class HSTUBlock(torch.nn.Module):
     return self._gate_and_output(attn.reshape(T, H * hd), u.reshape(T, H * hd), tokens, fused)
 
 
+_OWN_BLOCK_FORWARDS = HSTUBlock.forward, HSTUBlock.forward_jagged
+
+
+def _is_plain_call(block, jagged) -> bool:
+  """Whether a call of the block is a call of HSTUBlock's own forward and nothing else: no subclass, no forward put in its place, and, where
+  it is called as a module (the packed form calls forward_jagged itself), no hooks on it or on all modules, and not compiled."""
+  if type(block) is not HSTUBlock or (HSTUBlock.forward, HSTUBlock.forward_jagged) != _OWN_BLOCK_FORWARDS:
+    return False
+  own = block.__dict__
+  if jagged:
+    return "forward_jagged" not in own
+  m = torch.nn.modules.module
+  return ("forward" not in own and block._compiled_call_impl is None
+          and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                   or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks))
+
+
 class HSTU(torch.nn.Module):
   """The HSTU model forward (recml/layers/keras/hstu.py:585-621): item
   embedding (x sqrt(D)) + position embedding -> final_norm -> blocks ->
@@ -436,6 +453,29 @@ class HSTU(torch.nn.Module):
       raise IndexError(f"an item id lies outside the vocabulary of {self.item_embedding.shape[0]}"
                        + ("" if self.position_embedding is None else f", or a position past the {self.position_embedding.shape[0]} there are"))
 
+  def _narrow_blocks(self, x, length, seq_lens, offsets, pos_bias, close):
+    """All blocks on x in one launch (recml_amd/csrc/hstu_block_small.hip), with `close` the closing norm behind them: narrow models in
+    inference on short sequences.  None where there is no such launch, or where somebody watches or changes the blocks' calls."""
+    if self.model_dim > 64 or not x.is_cuda or x.dtype != torch.bfloat16:
+      return None
+    blocks = self.decoder_blocks._modules.values()
+    first = next(iter(blocks), None)
+    if first is None or (close and type(self)._final_norm is not HSTU._final_norm):
+      return None
+    weights, like = [], None
+    for block in blocks:
+      if not _is_plain_call(block, offsets is not None) or (block.training and block.dropout > 0.0):
+        return None
+      kind = block.num_heads, block.head_dim, block.eps, block.scaled_pointwise_attn
+      if like is not None and kind != like:
+        return None
+      like = kind
+      weights.append(block._weights())
+    alpha, n = first._alpha_n(length)
+    gamma, beta = (self.final_norm_gamma, self.final_norm_beta) if close else (None, None)
+    return _native.blocks(x.contiguous(), tuple(weights), first.num_heads, first.head_dim, first.eps, alpha, n, seq_lens, offsets,
+                          None if offsets is None else length, pos_bias, gamma, beta, self.eps)
+
   def _head(self, x):
     out = _native.linear(x, self.reverse_embedding, True)
     return x @ self.reverse_embedding if out is None else out
@@ -469,16 +509,22 @@ class HSTU(torch.nn.Module):
     if self.training and self.dropout > 0.0:
       ticket = self._check_mask(ticket)
     x, outside = self._front_end(inputs)
-    # every block sees the same lengths, timestamps and tables: the attention prepares them once
-    batch = hstu_ops.AttentionBatch()
-    for block in self.decoder_blocks:
-      if attention_mask is not None:
-        x = block(x, attention_mask=attention_mask, batch=batch)
-      else:
-        x = block(x, seq_lens=seq_lens, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch)
-      if ticket is not None:
-        ticket = self._check_mask(ticket)
-    out = self._final_norm(x)
+    out = None
+    if attention_mask is None and timestamps is None and ts_bias is None:
+      out = self._narrow_blocks(x, x.shape[1], seq_lens, None, pos_bias, True)
+    if out is None:
+      # every block sees the same lengths, timestamps and tables: the attention prepares them once
+      batch = hstu_ops.AttentionBatch()
+      for block in self.decoder_blocks:
+        if attention_mask is not None:
+          x = block(x, attention_mask=attention_mask, batch=batch)
+        else:
+          x = block(x, seq_lens=seq_lens, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, batch=batch)
+        if ticket is not None:
+          ticket = self._check_mask(ticket)
+      out = self._final_norm(x)
+    elif ticket is not None:
+      ticket = self._check_mask(ticket)
     if self.reverse_embedding is not None:
       out = self._head(out)
     self._check_mask(ticket)
@@ -508,9 +554,11 @@ class HSTU(torch.nn.Module):
     self._check_mask(ticket)
     x, outside = self._front_end(inputs, rows, tokens)
     ts = None if timestamps is None else timestamps.reshape(-1).index_select(0, rows[:tokens])
+    narrow = self._narrow_blocks(x, L, None, offsets, pos_bias, False) if ts is None and ts_bias is None else None
     batch = hstu_ops.AttentionBatch()
-    for block in self.decoder_blocks:
+    for block in self.decoder_blocks if narrow is None else ():
       x = block.forward_jagged(x, offsets, L, pos_bias=pos_bias, timestamps=ts, ts_bias=ts_bias, batch=batch)
+    x = x if narrow is None else narrow
     if self.reverse_embedding is None:
       out = _native.final_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps, offsets, rows, B, L, True)
       if out is not None:

@@ -6,8 +6,8 @@ import pytest
 import torch
 
 from oracle import hstu_block_oracle as BO
-from recml_amd import _lib_block
-from recml_amd.hstu_layer import HSTUBlock
+from recml_amd import _lib_block, hstu_layer
+from recml_amd.hstu_layer import HSTU, HSTUBlock
 
 pytestmark = pytest.mark.gpu
 DEV, BF = "cuda:0", torch.bfloat16
@@ -121,3 +121,79 @@ def _oracle(x, w, H, L, tab):
 def test_shapes_beside_it(gpu):
   assert not any([_taken(4, 65, 4), _taken(4, 50, 8), _taken(4, 50, 1), _taken(0, 50, 4), _taken(4, 0, 4), _taken(8192, 24, 4)])
   assert _taken(8192, 50, 4) == 1
+
+
+def _model(layers, D, H, L, biases=False, seed=0):
+  g = torch.Generator().manual_seed(seed)
+  model = HSTU(vocab_size=300, max_positions=L, model_dim=D, num_heads=H, num_layers=layers, add_head=False, dtype=BF, device=DEV, seed=seed)
+  if biases:
+    model.decoder_blocks = torch.nn.ModuleList(HSTUBlock(D, H, dtype=BF, device=DEV, use_bias=True, generator=g) for _ in range(layers))
+  with torch.no_grad():
+    for prm in model.parameters():
+      prm.add_((torch.randn(prm.shape, generator=g) * 0.05).to(DEV).to(BF))
+  return model, g
+
+
+@pytest.mark.parametrize("layers,B,L,H,pos,biases,jagged", [
+    (1, 3, 17, 4, None, True, False),
+    (2, 2, 64, 2, "heads", False, False),
+    (4, 5, 50, 4, "shared", True, True),
+    (17, 2, 33, 4, "heads", False, False),               # one block more than a launch takes
+    (33, 3, 20, 2, None, False, True),                   # three launches
+])
+def test_blocks_in_one_launch_are_the_blocks_one_by_one(gpu, layers, B, L, H, pos, biases, jagged):
+  """The same bits as one launch a block, which a hook on a block (or a subclass's forward) brings back."""
+  D = 16 * H
+  model, g = _model(layers, D, H, L, biases, seed=layers)
+  ids = torch.randint(1, 300, (B, L), generator=g).to(DEV)
+  lens = torch.randint(1, L + 1, (B,), generator=g).int()
+  lens[0] = L
+  tab = None if pos is None else (torch.randn((H if pos == "heads" else 1, 2 * L - 1), generator=g) * 0.3).to(DEV)
+  calls, own = [], hstu_layer._native.block
+  with torch.no_grad(), pytest.MonkeyPatch.context() as patch:
+    patch.setattr(hstu_layer._native, "block", lambda *a: calls.append(1) or own(*a))
+    got = model(ids, seq_lens=lens.to(DEV), pos_bias=tab, jagged=jagged)
+    assert not calls
+    seen = []
+    if jagged:
+      patch.setattr(HSTUBlock, "forward_jagged", lambda self, *a, f=HSTUBlock.forward_jagged, **kw: seen.append(1) or f(self, *a, **kw))
+    else:
+      for blk in model.decoder_blocks:
+        blk.register_forward_hook(lambda *a: seen.append(1) and None)
+    want = model(ids, seq_lens=lens.to(DEV), pos_bias=tab, jagged=jagged)
+    assert len(seen) == layers and len(calls) == layers
+  # the closing norm's sums are in another order (one place of its bf16 rows); the packed form's closing norm is the same kernel
+  if jagged:
+    assert torch.equal(got, want)
+  else:
+    assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs() + 2.0 ** -20).all())
+
+
+def test_what_keeps_the_blocks_apart(gpu):
+  """Gradients, other sizes among the blocks, dropout in training, a global hook: each block is called by itself."""
+  model, g = _model(2, 32, 2, 20)
+  ids = torch.randint(1, 300, (2, 20), generator=g).to(DEV)
+  kw = dict(seq_lens=torch.tensor([20, 5], dtype=torch.int32, device=DEV))
+  calls, own = [], hstu_layer._native.block
+  with pytest.MonkeyPatch.context() as patch:
+    patch.setattr(hstu_layer._native, "block", lambda *a: calls.append(1) or own(*a))
+
+    def count(f):
+      calls.clear()
+      f()
+      return len(calls)
+
+    run = lambda: model(ids, **kw)
+    assert count(run) == 0
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert count(run) == 2
+    handle.remove()
+    model.decoder_blocks[1].eps = 1e-3
+    assert count(run) == 2
+    model.decoder_blocks[1].eps = model.decoder_blocks[0].eps
+    model.decoder_blocks[1].dropout = 0.5
+    assert count(run) == 2 and count(lambda: model.eval()(ids, **kw)) == 0
+    model.requires_grad_(True)
+    assert count(run) == 2
+    with torch.no_grad():
+      assert count(run) == 0
