@@ -61,10 +61,8 @@ __device__ __forceinline__ const char* scalar_ptr(const void* p) {
 
 #define HSTU_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt((((n) & 15) | ((((n) >> 4) & 3) << 14)) | 0x0F70)
 
-// 16 bytes of the output.  PAST: this launch does not read them again and they are not kept in this XCD's L2, where the operands are (the
-// reader is a later launch, on any XCD).  74 k x 512 -> 2048, out alone / with the pre-activation: 240 -> 213, 282 -> 226 us.  Not the small
-// tiles: their outputs are small enough for the next launch to find them in a cache (18 k rows of 32 to 128: the attention behind it
-// 28.7 us with PAST, 27.3 without).
+// 16 bytes of the output.  PAST: not kept in this XCD's L2, where the operands are (the reader is a later launch, on any XCD).  store_past
+// says for which outputs.
 template <bool PAST>
 __device__ __forceinline__ void store_out(bf16_t* to, const uint4& v) {
   typedef uint32_t words __attribute__((ext_vector_type(4)));
@@ -72,6 +70,15 @@ __device__ __forceinline__ void store_out(bf16_t* to, const uint4& v) {
   if constexpr (PAST) __builtin_nontemporal_store(x, (words*)to);
   else *(words*)to = x;
 }
+
+// Whether an output of these sizes is stored past the L2s: where it is larger than all of them together (32 MB), so that it would drive the
+// operands out and its reader would not find it there, and its rows are whole sectors of 64 bytes.  us with / without:
+//   74 k x 512 -> 2048 190 / 217, with the pre-activation 226 / 282; 78 k x 512 -> 512 57 / 59; 78 k x 64 -> 256 (40 MB) 12.3 / 14.7
+//   1600 x 64 -> 20000 (64 MB) 22.7 / 25.7
+//   rows of parts of sectors, which leave as parts of lines: 8000 x 64 -> 5000 39 / 27, 16384 x 1024 -> 1000 44 / 37
+//   below 32 MB the product gains what its reader loses (18 k x 64 -> 128 with a pass over the result 9.7 / 9.7, 6.4 k x 512 -> 2048 30.9 / 31.2;
+//   an attention behind 18 k rows of 128 28.7 / 27.3)
+bool store_past(int64_t rows, int64_t cols, int64_t stride) { return rows * cols > 16 << 20 && stride % 32 == 0; }
 
 // One workgroup: a tile of 64 MB output rows x 32 NB WN output columns, 2 x WN waves of 32 MB x 32 NB.  The contraction runs in
 // stages of 32 through a three-stage LDS ring filled by direct global -> LDS loads (two stages in flight, one barrier
@@ -93,7 +100,7 @@ __device__ __forceinline__ void store_out(bf16_t* to, const uint4& v) {
 //   OUT: what the epilogue does, known to the compiler where it is one of the products of a block: a branch between its steps keeps
 // it from ordering them across pieces (74 k x 512 -> 2048 with the activation 235 us, 194 without).
 enum { OUT_PLAIN, OUT_SILU, OUT_PRE_SILU, OUT_ADD, OUT_PARTIAL, OUT_ANY };
-template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT>
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT, bool PAST>
 __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams g) {
   constexpr int TM = 64 * MB, TN = 32 * NB * WN, WAVES = 2 * WN;
   constexpr int Q_BYTES = TM * GEMM_BK * 2, P_BYTES = TN * GEMM_BK * 2, STAGE = Q_BYTES + P_BYTES;
@@ -446,7 +453,7 @@ __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
           const uint4 z = pack8(x[i]);
-          if (inside(i)) store_out<(MB >= 4)>(g.pre + (int64_t)(mb + RPI * i) * g.out_stride + n, z);
+          if (inside(i)) store_out<PAST>(g.pre + (int64_t)(mb + RPI * i) * g.out_stride + n, z);
           unpack8(z, x[i]);
         }
       }
@@ -459,7 +466,7 @@ __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams
       bf16_t* o = (osl == 0 ? g.out[0] : osl == 1 ? g.out[1] : osl == 2 ? g.out[2] : g.out[3]) + (int64_t)mb * g.out_stride + (n - osl * g.out_slab);
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
-        if (inside(i)) store_out<(MB >= 4)>(o + (int64_t)(RPI * i) * g.out_stride, pack8(x[i]));
+        if (inside(i)) store_out<PAST>(o + (int64_t)(RPI * i) * g.out_stride, pack8(x[i]));
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -481,14 +488,23 @@ __global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
   *(uint4*)o = pack8(x);
 }
 
-template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT>
-int launch_out(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT, bool PAST>
+int launch_inst(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
   static int granted[64];
-  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT>, smem, granted)) return rc;
-  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT>), dim3(blocks), dim3(128 * WN), smem, st, g);
+  if (int rc = block_allow_lds((const void*)hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT, PAST>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_kernel<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT, PAST>), dim3(blocks), dim3(128 * WN), smem, st, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
+}
+
+template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM, int OUT>
+int launch_out(const GemmParams& g, unsigned blocks, int smem, hipStream_t st) {
+  // (weight gradients are smaller, and 64 x 64 tiles are for products that are)
+  if constexpr (!Q_T && MB >= 2) {
+    if (store_past(g.rows, g.cols, g.out_stride)) return launch_inst<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT, true>(g, blocks, smem, st);
+  }
+  return launch_inst<MB, NB, WN, Q_T, P_T, STAGES, UNIFORM, OUT, false>(g, blocks, smem, st);
 }
 
 template <int MB, int NB, int WN, bool Q_T, bool P_T, int STAGES, bool UNIFORM>

@@ -52,6 +52,19 @@ def test_block_products(gpu, M, N, K, slabs):
   _close(torch.cat(grads, 1), x.float().t() @ y.float())
 
 
+@pytest.mark.parametrize("M,N,K", [(16384, 1024, 8), (16400, 1024, 64), (16395, 1032, 64), (1025, 20000, 64), (40000, 480, 200)])
+def test_large_outputs(gpu, M, N, K):
+  """On either side of the lines of store_past (2^24 outputs; rows of whole 64-byte sectors): the same bits as the products of parts of the
+  rows, which are stored the other way and summed in the same order."""
+  g = torch.Generator(device="cuda").manual_seed(M + N)
+  x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+  w = (torch.randn(K, N, device="cuda", generator=g) * 0.1).to(torch.bfloat16)
+  got = ops.gemm_silu(x, w, None, False)
+  for at in (slice(0, 700), slice(M - 300, M)):
+    assert torch.equal(got[at], ops.gemm_silu(x[at].contiguous(), w, None, False))
+  assert bool(torch.isfinite(got).all())
+
+
 @pytest.mark.parametrize("rows,keys,width", [(0, 5, 8), (1, 1, 8), (700, 1, 136), (3000, 40, 64), (3000, 5000, 72), (4097, 257, 128)])
 @pytest.mark.parametrize("scale", [1.0, 2.0])
 def test_gathered_table_gradient(gpu, rows, keys, width, scale):
