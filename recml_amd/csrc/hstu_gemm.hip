@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "hstu_block.h"
 #include "hstu_block_common.h"
@@ -472,6 +473,235 @@ __global__ __launch_bounds__(128 * WN, 2) void hstu_gemm_kernel(const GemmParams
   }
 }
 
+// f(0), f(1), ..., f(N - 1), each index a constant (a body this long is past what the compiler unrolls)
+template <int... I, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
+
+// The forward product where whole rows of x fit a wave's registers (contractions of 256 and 512; no bias, nothing added) and the output
+// is a large one.  A wave keeps 32 rows of x as fragments and the weight goes by in LDS, 32 columns and the whole contraction a stage.  A
+// workgroup is eight waves, 256 rows; it takes a run of pieces of (256 rows, 64 columns), rows by rows: its ring of stages never empties,
+// and x is read once, or twice where a tile is two workgroups'.
+//   What bounds hstu_gemm_kernel at a short contraction is that a tile's products and its epilogue take turns (74 k x 512 -> 2048: 139 us
+// and 55).  Here the products of a column block stand beside the activation of the one before it, four outputs' steps at a time, and a
+// second wave of the SIMD beside both.  74 k x 512 -> 2048 with SiLU 197 -> 150 us, with the pre-activation 216 -> 181, plain 177 -> 142;
+// 74 k x 256 -> 1024 74 -> 51, 90 -> 65.  What is left is the matrix pipes' clock on real operands beside the bytes that move: without
+// loads of the weight 11 % less, without stores 14 %, without either 25 %.  Two blocks of 32 rows a wave, one wave per SIMD, halve the reads of LDS and are no faster (161, 191, 149; 55, 67).
+template <int K, int OUT>
+__global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams g) {
+  constexpr int NS = K / 16, STAGE = K * 64, STAGES = 3, AHEAD = 3;
+  constexpr int LP = STAGE / 8192;                       // direct loads of 1 KB per wave and stage
+  constexpr bool PRE = OUT == OUT_PRE_SILU;
+  constexpr int STORES = PRE ? 8 : 4;
+  static_assert(LP <= 4, "a step's stores follow its loads");
+  static_assert(NS % (AHEAD + 1) == 0 && 32 % NS == 0 && NS >= 16, "fragments keep their registers from step to step");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const uint32_t smem_lds = __builtin_amdgcn_groupstaticsize();
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+
+  // this workgroup's run of pairs of column blocks, XCD by XCD
+  const int pairs = g.cols >> 6;
+  const int64_t all = (int64_t)g.row_tiles * pairs;
+  const int64_t me = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int64_t first = all * me / gridDim.x, last = all * (me + 1) / gridDim.x;
+  if (first >= last) return;
+  // (scalars, which a division leaves in vector registers)
+  int rt = __builtin_amdgcn_readfirstlane((int)(first / pairs)), pc = __builtin_amdgcn_readfirstlane((int)(first - (int64_t)rt * pairs));
+  int todo = __builtin_amdgcn_readfirstlane((int)(last - first));
+
+  // ---- the weight's stages: rows of 64 bytes, piece i of a wave 16 of them
+  int sl = __builtin_amdgcn_readfirstlane(64 * pc / g.slab), sc = 64 * pc - sl * g.slab;      // slab and column of the next stage to load
+  uint32_t po[LP];
+#pragma unroll
+  for (int i = 0; i < LP; ++i) po[i] = (uint32_t)((16 * (LP * w + i) + (lane >> 2)) * (int)g.p_stride + 8 * (lane & 3)) * 2u;
+  const char* p_base;
+  auto next_columns = [&]() __attribute__((always_inline)) {
+    p_base = scalar_ptr(g.p[sl] + sc);
+    sc += 32;
+    if (sc == g.slab) {
+      sc = 0;
+      sl = (sl + 1) * g.slab == g.cols ? 0 : sl + 1;
+    }
+  };
+  auto dma = [&](int st, int i) __attribute__((always_inline)) {
+    lds_dma16(p_base, po[i], smem_lds + (uint32_t)st * STAGE + 1024u * (LP * w + i));
+  };
+
+  const int gi = lane & 15;
+  const uint32_t at_lane = (uint32_t)((8 * hh + (gi >> 2)) * 64 + 32 * ((lane >> 4) & 1) + 8 * (gi & 3));
+  bf16x8 f[AHEAD + 1];
+  auto ask = [&](int st, int s) __attribute__((always_inline)) {
+    const unsigned char* at = smem + st * STAGE + at_lane + 1024 * s;
+    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at));
+    const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at + 256));
+    struct { short4v a, b; } both = {lo, hi};
+    f[s % (AHEAD + 1)] = __builtin_bit_cast(bf16x8, both);
+  };
+
+  bf16x8 qf[NS];
+  auto load_rows = [&](int tile) __attribute__((always_inline)) {
+    int row = 256 * tile + 32 * w + l32;
+    row = row < g.rows ? row : g.rows - 1;              // (what it gives is not stored)
+    const bf16_t* at = g.q + (int64_t)row * g.q_stride + 8 * hh;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qf[s] = *(const bf16x8*)(at + 16 * s);
+  };
+  // (waited for here: left to their first use, the waits would stand in the loop and be for every younger load and store in each round)
+  auto rows_here = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+  };
+
+  // ---- the epilogue: 32 rows x 64 columns through the wave's own LDS, rows of 128 bytes, 8-byte piece c of row r at c ^ (r / 2 % 16)
+  // (written a column piece of all rows at a time, read a row at a time: all banks both ways)
+  unsigned char* const out_lds = smem + STAGES * STAGE + w * 4096;
+  unsigned char* const pre_lds = out_lds + 32768;
+  float z[4], e[4];
+  uint32_t zw[2], ow[2];
+  const int wslot = (l32 >> 1) & 15;
+  auto put = [&](unsigned char* to, int par, int q4, const uint32_t (&v)[2]) __attribute__((always_inline)) {
+    *(uint2*)(to + l32 * 128 + (((8 * par + 2 * q4 + hh) ^ wslot) * 8)) = uint2{v[0], v[1]};
+  };
+  // part `ph` of 32: eight for each four columns of a lane
+  auto epilogue = [&](const floatx16& old, auto par_, auto ph_) __attribute__((always_inline)) {
+    constexpr int ph = decltype(ph_)::value, q4 = ph >> 3, par = decltype(par_)::value;
+    constexpr bool act = OUT != OUT_PLAIN;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr ((ph & 7) == 0) z[i] = old[4 * q4 + i];
+      if constexpr ((ph & 7) == 1 && act) e[i] = -1.4426950408889634f * z[i];
+      if constexpr ((ph & 7) == 2 && act) e[i] = __builtin_amdgcn_exp2f(e[i]);
+      if constexpr ((ph & 7) == 3 && act) e[i] = 1.0f + e[i];
+      if constexpr ((ph & 7) == 4 && act) e[i] = __builtin_amdgcn_rcpf(e[i]);
+      if constexpr ((ph & 7) == 5 && act) z[i] = z[i] * e[i];
+    }
+    if constexpr (PRE && (ph & 7) == 0) {
+      // (the activation of the stored value, which is what its gradient is taken at)
+      zw[0] = pack2(z[0], z[1]);
+      zw[1] = pack2(z[2], z[3]);
+      z[0] = __builtin_bit_cast(float, zw[0] << 16);
+      z[1] = __builtin_bit_cast(float, zw[0] & 0xffff0000u);
+      z[2] = __builtin_bit_cast(float, zw[1] << 16);
+      z[3] = __builtin_bit_cast(float, zw[1] & 0xffff0000u);
+    }
+    if constexpr (PRE && (ph & 7) == 4) put(pre_lds, par, q4, zw);
+    if constexpr ((ph & 7) == 6) {
+      ow[0] = pack2(z[0], z[1]);
+      ow[1] = pack2(z[2], z[3]);
+    }
+    if constexpr ((ph & 7) == 7) put(out_lds, par, q4, ow);
+  };
+  typedef uint32_t words __attribute__((ext_vector_type(4)));
+  words rows_out[4], rows_pre[4];
+  const bool halves = (lane >> 4) & 1;                  // (of 16 bytes, in the other order)
+  auto take = [&](const unsigned char* from, int i) __attribute__((always_inline)) {
+    const int row = (lane >> 3) + 8 * i;
+    const words v = *(const words*)(from + row * 128 + (((lane & 7) ^ ((row >> 2) & 7)) * 16));
+    return words{halves ? v[2] : v[0], halves ? v[3] : v[1], halves ? v[0] : v[2], halves ? v[1] : v[3]};
+  };
+  const uint32_t out_at = (uint32_t)((32 * w + (lane >> 3)) * (int)g.out_stride + 8 * (lane & 7)) * 2u;
+  const uint32_t out_step = (uint32_t)(8 * (int)g.out_stride) * 2u;
+  // (past the L2s, see store_past; rows past the output's end lie past the buffer's: nothing is stored, and as many stores are under way)
+  bf16_t *to_out = g.out[0], *to_pre = g.pre;
+  uint32_t to_bytes = 0;
+  auto store = [&](bf16_t* base, const words& v, int i) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)to_bytes, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)(out_at + i * out_step), 0, 2);
+  };
+
+  const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  floatx16 acc_a = zero, acc_b = zero;
+  // One step: the products of a column block, the epilogue of the one before it, the stage after next on its way; in a pair's second step
+  // the rows of the pair before are stored.
+  auto step = [&](auto par_, int st, floatx16& acc, const floatx16& old) __attribute__((always_inline)) {
+    constexpr int par = decltype(par_)::value;
+    const int refill = st + 2 >= STAGES ? st + 2 - STAGES : st + 2, next = st + 1 >= STAGES ? 0 : st + 1;
+    next_columns();
+    each<NS>([&](auto s_) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_)::value, PER = 32 / NS;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (s == NS - AHEAD) {
+        // (everything asked of the stage is here, and behind the barrier everyone's is: its place can be refilled.  Younger than the next
+        // stage's loads: those of the one after it and one pair's stores)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        HSTU_WAIT_VMCNT(LP + STORES);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
+      if constexpr (s + AHEAD < NS) ask(st, s + AHEAD);
+      else ask(next, s + AHEAD - NS);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s % (AHEAD + 1)], qf[s], s == 0 ? zero : acc, 0, 0, 0);
+      if constexpr (s < LP) dma(refill, s);
+      if constexpr (par == 1) {
+        // (the first part that writes there again is the fifth)
+        each<PER>([&](auto i_) __attribute__((always_inline)) {
+          constexpr int i = s * PER + decltype(i_)::value;
+          if constexpr (i < 4) {
+            rows_out[i] = take(out_lds, i);
+            if constexpr (PRE) rows_pre[i] = take(pre_lds, i);
+          }
+        });
+        if constexpr (s >= 4 && s < 8) {
+          store(to_out, rows_out[s - 4], s - 4);
+          if constexpr (PRE) store(to_pre, rows_pre[s - 4], s - 4);
+        }
+      }
+      each<PER>([&](auto i_) __attribute__((always_inline)) {
+        epilogue(old, std::integral_constant<int, 1 - par>{}, std::integral_constant<int, s * PER + decltype(i_)::value>{});
+      });
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  next_columns();
+#pragma unroll
+  for (int i = 0; i < LP; ++i) dma(0, i);
+  next_columns();
+#pragma unroll
+  for (int i = 0; i < LP; ++i) dma(1, i);
+  load_rows(rt);
+  __builtin_amdgcn_sched_barrier(0);
+  HSTU_WAIT_VMCNT(LP + NS);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) ask(0, s);
+  rows_here();
+  int st = 0, have = rt;
+  for (; todo > 0; --todo) {
+    if (rt != have) {
+      load_rows(rt);
+      rows_here();
+      have = rt;
+    }
+    step(std::integral_constant<int, 0>{}, st, acc_a, acc_b);
+    st = st + 1 >= STAGES ? 0 : st + 1;
+    step(std::integral_constant<int, 1>{}, st, acc_b, acc_a);
+    st = st + 1 >= STAGES ? 0 : st + 1;
+    const int m0 = 256 * rt;
+    const int64_t left = ((int64_t)(g.rows - m0 < 256 ? g.rows - m0 : 256) - 1) * g.out_stride + (g.cols - 64 * pc);
+    to_out = g.out[0] + (int64_t)m0 * g.out_stride + 64 * pc;
+    to_pre = PRE ? g.pre + (int64_t)m0 * g.out_stride + 64 * pc : nullptr;
+    to_bytes = (uint32_t)(left * 2);
+    if (++pc == pairs) {
+      pc = 0;
+      ++rt;
+    }
+  }
+  each<32>([&](auto ph_) __attribute__((always_inline)) {
+    epilogue(acc_b, std::integral_constant<int, 1>{}, ph_);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    store(to_out, take(out_lds, i), i);
+    if (PRE) store(to_pre, take(pre_lds, i), i);
+  }
+  HSTU_WAIT_VMCNT(0);        // (no direct load may arrive in LDS that is another workgroup's by then)
+}
+
 // Sums the partial products of a split contraction in the order of the splits and rounds them once.
 __global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
   const int64_t per = (int64_t)g.rows * g.cols;
@@ -596,6 +826,34 @@ int pick_splits(int64_t rows, int64_t cols, int64_t depth, int* tile) {
       if (c < least) { least = c; splits = s; *tile = t; }
     }
   return splits;
+}
+
+// Whether hstu_gemm_rows_kernel takes the product: from six pieces for each of its workgroups on.  Below, reading the rows before the first
+// product (12 us, twice where a workgroup's run crosses a tile's end) costs more than is won.  us here / with the tiles, at 6.2 pieces:
+// 12800 x 512 -> 2048 40.5 / 40.7, with the pre-activation 44 / 49, 51200 x 512 -> 512 40 / 42, 51200 x 256 -> 512 25 / 30, 25600 x 256 -> 1024
+// 24 / 29; at 12.5: 25600 x 512 -> 2048 62 / 80; at 3.1: 6400 x 512 -> 2048 31 / 24, 25600 x 256 -> 512 19 / 18.
+constexpr int ROWS_GRID = 256;                 // a workgroup per CU
+bool rows_product(const GemmParams& g) {
+  return (g.depth == 256 || g.depth == 512) && !g.bias && !g.c && (g.activation || !g.pre) && g.cols % 64 == 0 && g.slab % 32 == 0 &&
+         g.out_stride < 1 << 20 && g.p_stride < 1 << 20 && (int64_t)((g.rows + 255) / 256) * (g.cols / 64) >= 6 * ROWS_GRID;
+}
+
+template <int K, int OUT>
+int launch_rows_as(GemmParams g, hipStream_t st) {
+  static int granted[64];
+  constexpr int smem = 3 * K * 64 + (OUT == OUT_PRE_SILU ? 65536 : 32768);
+  g.row_tiles = (g.rows + 255) / 256;
+  if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT>), dim3(ROWS_GRID), dim3(512), smem, st, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
+}
+template <int K>
+int launch_rows(const GemmParams& g, hipStream_t st) {
+  if (g.pre) return launch_rows_as<K, OUT_PRE_SILU>(g, st);
+  if (g.activation) return launch_rows_as<K, OUT_SILU>(g, st);
+  return launch_rows_as<K, OUT_PLAIN>(g, st);
 }
 
 // out = act(x w + c + bias) for widths that the kernel above cannot fetch 16 bytes at a time: element by element, fp32 products.  (One
@@ -770,6 +1028,7 @@ int hstu_gemm(const HstuGemmArgs* a, void* stream) {
     p.cols = p.out_slab = a->N;
     p.out_stride = a->N;
     p.depth = p.depth_per_split = a->K;
+    if (rows_product(p)) return p.depth == 512 ? launch_rows<512>(p, st) : launch_rows<256>(p, st);
     return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, true, 256, 256), p.c != nullptr));
   }
   p.cols = p.out_slab = a->K;

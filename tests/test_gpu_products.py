@@ -65,6 +65,30 @@ def test_large_outputs(gpu, M, N, K):
   assert bool(torch.isfinite(got).all())
 
 
+@pytest.mark.parametrize("M,N,K,slabs", [
+    (12289, 2048, 512, 4),     # tiles of one row at the end; runs that cross tiles, pieces that cross slabs' ends
+    (12288, 2048, 256, 1),     # whole tiles, six pieces for each workgroup
+    (36705, 704, 512, 2),      # an odd number of pieces in a tile, slabs of 352: their ends within a piece
+    (20000, 1280, 256, 4),
+])
+def test_rows_in_registers(gpu, M, N, K, slabs):
+  """Large products whose rows stay in registers: the same bits as those of parts of the rows, which go by tiles and are summed in the same
+  order; and against fp32."""
+  g = torch.Generator(device="cuda").manual_seed(M + N)
+  x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+  ws = [(torch.randn(K, N // slabs, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16) for _ in range(slabs)]
+  for kw in ({}, dict(activation=True), dict(activation=True, want_pre=True)):
+    parts = lambda r: r if isinstance(r, tuple) else (r,)
+    got = parts(ops.block_gemm(_lib_block.GEMM_NN, x, ws, **kw))
+    for at in range(0, M, 4000):
+      part = slice(at, min(at + 4000, M))
+      for a, b in zip(got, parts(ops.block_gemm(_lib_block.GEMM_NN, x[part], ws, **kw))):
+        assert torch.equal(a[part], b)
+  want = x[-300:].float() @ torch.cat(ws, 1).float()
+  _close(got[1][-300:], want)
+  _close(got[0][-300:], torch.nn.functional.silu(got[1][-300:].float()))
+
+
 @pytest.mark.parametrize("rows,keys,width", [(0, 5, 8), (1, 1, 8), (700, 1, 136), (3000, 40, 64), (3000, 5000, 72), (4097, 257, 128)])
 @pytest.mark.parametrize("scale", [1.0, 2.0])
 def test_gathered_table_gradient(gpu, rows, keys, width, scale):
