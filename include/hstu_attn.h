@@ -88,7 +88,10 @@ enum HstuFwdFlags {
    * order, the same bits out.  In the `fwd` member of hstu_attn_bwd's arguments
    * it does the same to the backward's dK/dV kernel, which runs its unmasked
    * blocks without bias as such a stream at d = 128. */
-  HSTU_FWD_COMPILER_SCHEDULED_BLOCKS = 16
+  HSTU_FWD_COMPILER_SCHEDULED_BLOCKS = 16,
+  /* In the `fwd` member of hstu_attn_bwd's arguments only: ddense_bias is
+   * written, every element of it, and need not have been cleared. */
+  HSTU_BWD_WRITE_BIAS_GRADIENT = 32
 };
 
 /* Return codes (0 = launched). */
@@ -302,7 +305,7 @@ typedef struct HstuAttnBwdArgs {
   /* Gradient of fwd.dense_bias, fp32, shaped like it ([L, Lkv] or [B, L, Lkv] by
    * fwd.dense_bias_batched): dS summed over the heads (and over the batch for a
    * shared bias), ACCUMULATED into by atomic adds like the table gradients (the
-   * caller zero-fills; null = not wanted; needs fwd.dense_bias).  jax's derivative
+   * caller zero-fills, or sets HSTU_BWD_WRITE_BIAS_GRADIENT; null = not wanted; needs fwd.dense_bias).  jax's derivative
    * of recml/layers/keras/hstu.py:373-374. */
   float* ddense_bias;
 } HstuAttnBwdArgs;

@@ -4365,6 +4365,225 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
   store_rows<D>(acc, p.alpha * p.inv_n, smem + w * (32 * D * 2), dqg, p.q_pre ? (const bf16_t*)p.q_pre + s.bq : nullptr, p.q_st, r0, s.n_q, s.rows, lane);
 }
 
+// Gradient of the dense bias, dS summed over the heads, where each sequence has a bias of its own: one workgroup per 128 query rows and 64
+// keys goes through the heads, forms S and dP again (the roundings and the sums of the kernels above), and keeps the sum
+// over the heads in registers, as it keeps its part of the bias and of the mask.  The next stage comes under the products of the one at
+// hand; masked pairs are cleared once, in the sum.
+//   As a part of the dQ kernel the gradient is H atomic additions to every element, which that kernel waits for, into a matrix that has
+// to be cleared first (16 x up to 1000, eight heads of 64: the backward call 434 us, now 319, this kernel 67 of them and dQ 109).  Tiles
+// without a kept pair are stores only.
+// A stage is 64 channels of a head.  Every operand comes by direct loads, whole lines of it: rows of Q and dO loaded as fragments would be
+// asked for 32 bytes of a line at a time (16 x up to 1000 75 us, 16 x 2048 at d = 128 450).
+template <int D>
+struct DbiasShape {
+  static constexpr int KEYS = 64, BLOCKS = KEYS / BN, CH = D < 64 ? D : 64, CHUNKS = D / CH;
+  static constexpr int K_BYTES = KEYS * CH * 2, STAGE = 2 * K_BYTES, Q_BYTES = BN * CH * 2;      // (of a wave: its 32 rows of Q, and of dO)
+  static constexpr int Q_OFF = 2 * STAGE, LDS = Q_OFF + NWAVES * 2 * Q_BYTES;
+};
+
+template <int D, bool MSK>
+__global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_bwd_dbias_mfma(const Params p) {
+  using S = DbiasShape<D>;
+  constexpr int KSTEPS = S::CH / 16, CPR = S::CH / 8, BLOCKS = S::BLOCKS;
+  constexpr int LK = S::K_BYTES / (1024 * NWAVES), LQ = S::Q_BYTES / 1024;      // direct loads of a wave and stage, per operand
+  static_assert(NWAVES * 4096 <= S::LDS, "room for the waves' blocks at the end");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 31, hh = lane >> 5;
+
+  // the tiles of 128 rows follow each other on one XCD, whose L2 has those rows; a sequence's rows are dealt to all eight, so that a long one
+  const int nk = (p.Lkv + S::KEYS - 1) / S::KEYS, j = (int)(blockIdx.x >> 3);
+  const int turn_of = __builtin_amdgcn_readfirstlane(j / nk), strip = turn_of * 8 + (int)(blockIdx.x & 7);
+  const int b = __builtin_amdgcn_readfirstlane(strip / p.n_qtiles);
+  if (b >= p.B) return;
+  // is not one XCD's work, from another tile on in each sequence, as an XCD would have the same one of all of eight tiles
+  const int qt_at = strip - b * p.n_qtiles + b % p.n_qtiles, qt = qt_at < p.n_qtiles ? qt_at : qt_at - p.n_qtiles;
+  const int q0 = qt * BM, kv0 = (j - turn_of * nk) * S::KEYS;
+  const Seq s = seq_info(p, b, 0);
+  const int win = p.window;
+  const int q_last = (q0 + BM < s.n_q ? q0 + BM : s.n_q) - 1, k_last = (kv0 + S::KEYS < s.n_kv ? kv0 + S::KEYS : s.n_kv) - 1;
+  bool live = q_last >= q0 && k_last >= kv0 && !(p.causal && kv0 > q_last) && !(win >= 0 && (k_last < q0 - win || kv0 > q_last + win));
+  if (MSK && live) {
+    const int2 mr = ((const int2*)p.mask_range)[(p.mask_batched ? b : 0) * p.n_qtiles + qt];
+    live = kv0 / BN < mr.y && kv0 / BN + BLOCKS > mr.x;
+  }
+  const int rows = p.L - q0 < BM ? p.L - q0 : BM, cols = p.Lkv - kv0 < S::KEYS ? p.Lkv - kv0 : S::KEYS;
+  float* const out = p.dbias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0) + (int64_t)q0 * p.Lkv + kv0;
+  if (!live) {
+    if (p.dbias_fresh) {
+      const int c = tid & (S::KEYS - 1);
+      for (int r = tid / S::KEYS; r < rows; r += MFMA_THREADS / S::KEYS)
+        if (c < cols) out[(int64_t)r * p.Lkv + c] = 0.f;
+    }
+    return;
+  }
+
+  const uint32_t qst_bytes = (uint32_t)p.q_st * 2u, kst_bytes = (uint32_t)p.k_st * 2u, vst_bytes = (uint32_t)p.v_st * 2u, ost_bytes = (uint32_t)p.o_st * 2u;
+  const int r0 = q0 + 32 * w, qrow = r0 + m;
+  // piece j of an operand: lane l brings 16 bytes of row (64 j + l) / CPR
+  unsigned char* const q_lds = smem + S::Q_OFF + w * (2 * S::Q_BYTES);
+  auto dma_rows = [&](int h, int c) __attribute__((always_inline)) {
+    const char* qg = (const char*)p.q + (s.bq + (int64_t)h * p.q_sh + c * S::CH) * 2;
+    const char* dg = (const char*)p.dout + (s.bo + (int64_t)h * p.o_sh + c * S::CH) * 2;
+#pragma unroll
+    for (int j = 0; j < LQ; ++j) {
+      const int row = (64 * j + lane) / CPR, pc = lane % CPR;
+      int grow = r0 + row;
+      grow = grow < s.n_q - 1 ? grow : s.n_q - 1;        // (what a row past the end gives is cleared)
+      const uint32_t sw = (uint32_t)((pc ^ swz_rt<S::CH>(row)) * 16);
+      lds_dma16(qg, (uint32_t)grow * qst_bytes + sw, q_lds + j * 1024);
+      lds_dma16(dg, (uint32_t)grow * ost_bytes + sw, q_lds + S::Q_BYTES + j * 1024);
+    }
+  };
+  auto dma_keys = [&](int h, int c, int st) __attribute__((always_inline)) {
+    const char* kg = (const char*)p.k + (s.bk + (int64_t)h * p.k_sh + c * S::CH) * 2;
+    const char* vg = (const char*)p.v + (s.bv + (int64_t)h * p.v_sh + c * S::CH) * 2;
+#pragma unroll
+    for (int r = 0; r < LK; ++r) {
+      const int j = w * LK + r;
+      const int row = (64 * j + lane) / CPR, pc = lane % CPR;
+      int grow = kv0 + row;
+      grow = grow < s.n_kv - 1 ? grow : s.n_kv - 1;
+      const uint32_t sw = (uint32_t)((pc ^ swz_rt<S::CH>(row)) * 16);
+      lds_dma16(kg, (uint32_t)grow * kst_bytes + sw, smem + st * S::STAGE + j * 1024);
+      lds_dma16(vg, (uint32_t)grow * vst_bytes + sw, smem + st * S::STAGE + S::K_BYTES + j * 1024);
+    }
+  };
+  dma_keys(0, 0, 0);
+  dma_rows(0, 0);
+
+  // the lane's part of the bias and which of its pairs are kept: register 4g + t of block kb is key kv0 + 32 kb + 8g + 4hh + t
+  float bias[BLOCKS][16], sum[BLOCKS][16];
+  uint32_t keep[BLOCKS];
+  {
+    const int row = qrow < p.L - 1 ? qrow : p.L - 1;
+    const float* bg = p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0) + (int64_t)row * p.bias_pitch;
+    const uint8_t* mg = MSK ? p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0) + (int64_t)row * p.mask_pitch : nullptr;
+    int hi = p.causal ? qrow : (win >= 0 ? qrow + win : s.n_kv - 1);
+    hi = hi < s.n_kv - 1 ? hi : s.n_kv - 1;
+    hi = qrow < s.n_q ? hi : -1;
+    const int lo = win >= 0 ? qrow - win : 0;
+#pragma unroll
+    for (int kb = 0; kb < BLOCKS; ++kb) {
+      keep[kb] = 0u;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = kv0 + 32 * kb + 8 * g + 4 * hh;
+        const float4 bv = *(const float4*)(bg + (col < p.bias_pitch - 4 ? col : p.bias_pitch - 4));
+        bias[kb][4 * g] = bv.x; bias[kb][4 * g + 1] = bv.y; bias[kb][4 * g + 2] = bv.z; bias[kb][4 * g + 3] = bv.w;
+        const uint32_t mb = MSK ? *(const uint32_t*)(mg + (col < p.mask_pitch - 4 ? col : p.mask_pitch - 4)) : ~0u;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          sum[kb][4 * g + t] = 0.f;
+          keep[kb] |= (col + t <= hi && col + t >= lo && ((mb >> (8 * t)) & 0xffu)) ? 1u << (4 * g + t) : 0u;
+        }
+      }
+    }
+  }
+  const float alpha2 = p.alpha * LOG2E;
+  const int gk = swz_rt<S::CH>(m);
+  bool any[BLOCKS];
+#pragma unroll
+  for (int kb = 0; kb < BLOCKS; ++kb) any[kb] = __builtin_amdgcn_ballot_w64(keep[kb] != 0u) != 0;
+  int st = 0;
+  for (int h = 0; h < p.H; ++h) {
+    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    floatx16 sacc[BLOCKS], dpacc[BLOCKS];
+#pragma unroll
+    for (int kb = 0; kb < BLOCKS; ++kb) sacc[kb] = dpacc[kb] = zero;
+    const uint32_t drop0 = p.drop_thr ? drop_bh_key(p.drop_key, (uint32_t)b * (uint32_t)p.H + (uint32_t)h) + (uint32_t)qrow * DROP_CI : 0u;
+#pragma unroll
+    for (int c = 0; c < S::CHUNKS; ++c) {
+      HSTU_WAIT_VMCNT(0);
+      __syncthreads();                 // this stage is here, and the other one is nobody's any more
+      uint4 qf[KSTEPS], dof[KSTEPS];
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        const unsigned char* at = q_lds + m * (S::CH * 2) + (((2 * ks + hh) ^ gk) * 16);
+        qf[ks] = *(const uint4*)at;
+        dof[ks] = *(const uint4*)(at + S::Q_BYTES);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {        // (read, before the next stage's rows come)
+        asm volatile("" : "+v"(qf[ks].x), "+v"(qf[ks].y), "+v"(qf[ks].z), "+v"(qf[ks].w));
+        asm volatile("" : "+v"(dof[ks].x), "+v"(dof[ks].y), "+v"(dof[ks].z), "+v"(dof[ks].w));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const int c_next = c + 1 < S::CHUNKS ? c + 1 : 0, h_next = c_next ? h : h + 1;
+      if (h_next < p.H) {
+        dma_keys(h_next, c_next, st ^ 1);
+        dma_rows(h_next, c_next);
+      }
+      const unsigned char* const tile = smem + st * S::STAGE + m * (S::CH * 2);
+      st ^= 1;
+#pragma unroll
+      for (int kb = 0; kb < BLOCKS; ++kb) {
+        if (any[kb]) {
+          constexpr int AHEAD_F = 3;
+          uint4 af[AHEAD_F + 1];
+          auto ask = [&](int i) __attribute__((always_inline)) {          // product i: S for even i, dP for odd, channels 16 (i / 2) ..
+            af[i % (AHEAD_F + 1)] = *(const uint4*)(tile + kb * (BN * S::CH * 2) + (((2 * (i >> 1) + hh) ^ gk) * 16) + (i & 1) * S::K_BYTES);
+          };
+#pragma unroll
+          for (int i = 0; i < AHEAD_F; ++i) ask(i);
+#pragma unroll
+          for (int i = 0; i < 2 * KSTEPS; ++i) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (i + AHEAD_F < 2 * KSTEPS) ask(i + AHEAD_F);
+            floatx16& to = (i & 1) ? dpacc[kb] : sacc[kb];
+            to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i % (AHEAD_F + 1)]),
+                                                         __builtin_bit_cast(bf16x8, (i & 1) ? dof[i >> 1] : qf[i >> 1]), to, 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if (c == S::CHUNKS - 1) {
+            float ds[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              float fp;
+              silu_grad_log2(__builtin_fmaf(bias[kb][r], LOG2E, sacc[kb][r] * alpha2), &fp);
+              ds[r] = dpacc[kb][r] * fp;
+            }
+            if (p.drop_thr) drop_apply16(ds, drop0 + (uint32_t)(kv0 + 32 * kb + 4 * hh) * DROP_CJ, DROP_CJ, p.drop_thr);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[kb][r] += ds[r];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+    }
+  }
+
+  // by rows, through 4 KB of LDS of the wave's own
+  __syncthreads();
+  unsigned char* const turn = smem + w * 4096;
+  const int col = lane & 31;
+#pragma unroll
+  for (int kb = 0; kb < BLOCKS; ++kb) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float v[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[t] = (keep[kb] >> (4 * g + t)) & 1u ? sum[kb][4 * g + t] * p.inv_n : 0.f;
+      *(float4*)(turn + m * 128 + (((2 * g + hh) ^ (m & 7)) * 16)) = float4{v[0], v[1], v[2], v[3]};
+    }
+    __builtin_amdgcn_wave_barrier();
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = 2 * i + (lane >> 5);
+      v[i] = *(const float*)(turn + r * 128 + (((col >> 2) ^ (r & 7)) * 16) + (col & 3) * 4);
+    }
+    __builtin_amdgcn_wave_barrier();
+    float* to = out + (int64_t)(32 * w + (lane >> 5)) * p.Lkv + 32 * kb + col;
+#pragma unroll
+    for (int i = 0; i < 16; ++i, to += 2 * (int64_t)p.Lkv) {
+      if (32 * w + 2 * i + (lane >> 5) >= rows || 32 * kb + col >= cols) continue;
+      if (p.dbias_fresh) *to = v[i];
+      else if (v[i] != 0.f) atomicAdd(to, v[i]);
+    }
+  }
+}
+
 // At d = 128 two 32 x 128 accumulators plus the K and V fragments are 192 registers before any
 // temporary: one workgroup per CU, the accumulators in the accumulation registers (ACC_ASM below).
 // DSPLIT = 2 would share the work of 32 keys between two waves, each accumulating dK and dV for
@@ -5815,8 +6034,36 @@ int launch_bwd_mfma_ds(const Params& q, hipStream_t st) {
   return launch_bwd_mfma_inst<D, false, false, false, SEG>(q, st);
 }
 
+// Whether the dense bias's gradient is a kernel of its own: for long rows, and matrices enough for a round of its workgroups; elsewhere the
+// additions of the dQ kernel are few and its second run over the heads is the longer way.  us for a backward call with / without, d = 64:
+// eight heads, 16 x up to 1000 319 / 434, 8 x 700 126 / 145, 1 x 2000 424 / 471 (4 x 700 117 / 123, 16 x 300 92 / 91, 64 x 256 155 / 149,
+// 32 x 256 89 / 83); two heads, 16 x 1000 142 / 155, 8 x 700 89 / 89; one, 16 x 2048 325 / 354, 16 x 1000 142 / 144.  d = 128, eight heads:
+// 16 x 2048, full, 1425 / 1626, 16 x 1000 400 / 480, 8 x 700 155 / 155.
+bool dbias_apart(const Params& p) {
+  return p.dbias && p.dense_bias && (p.dense_bias_batched || p.B == 1) && p.L >= 512 && (int64_t)p.B * p.L * p.Lkv >= 3000000;
+}
+
 template <int D>
-int launch_bwd_mfma_d(const Params& q, hipStream_t st) {
+int launch_dbias(const Params& p, hipStream_t st) {
+  using S = DbiasShape<D>;
+  const long long per_xcd = ((long long)p.B * p.n_qtiles + 7) / 8 * ((p.Lkv + S::KEYS - 1) / S::KEYS);
+  if (8 * per_xcd > 0x7fffffffLL) return fail(HSTU_ERR_SHAPE, "grid too large");
+  static int granted[2][64];
+  const auto fn = p.mask ? hstu_bwd_dbias_mfma<D, true> : hstu_bwd_dbias_mfma<D, false>;
+  if (int rc = allow_lds((const void*)fn, S::LDS, granted[p.mask ? 1 : 0])) return rc;
+  hipLaunchKernelGGL(fn, dim3((unsigned)(8 * per_xcd)), dim3(MFMA_THREADS), S::LDS, st, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward bias kernel launch: %s", hipGetErrorString(e));
+  return HSTU_OK;
+}
+
+template <int D>
+int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
+  Params q = p;
+  if (dbias_apart(q)) {
+    if (int rc = launch_dbias<D>(q, st)) return rc;
+    q.dbias = nullptr;
+  }
   if (q.mask && q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, true, true>(q, st);
   if (q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, false, true>(q, st);
   if (q.mask) return launch_bwd_mfma_inst<D, false, false, false, false, true>(q, st);
@@ -5872,6 +6119,31 @@ __global__ __launch_bounds__(256) void hstu_pad_rows(const T* __restrict__ src, 
     }
     __builtin_memcpy(dst + row * pitch + c, v, 16);
   }
+}
+
+}  // namespace
+
+namespace {
+
+// The arguments without the flags that are the backward's alone.
+const HstuAttnBwdArgs* without_bwd_flags(const HstuAttnBwdArgs* a, HstuAttnBwdArgs& own) {
+  if (!(a->fwd.flags & HSTU_BWD_WRITE_BIAS_GRADIENT)) return a;
+  if (a != &own) own = *a;
+  own.fwd.flags &= ~HSTU_BWD_WRITE_BIAS_GRADIENT;
+  return &own;
+}
+
+// (a kernel, not hipMemsetAsync: the call may be captured into a graph)
+__global__ __launch_bounds__(256) void hstu_clear(float* __restrict__ to, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) to[i] = 0.f;
+}
+int clear_floats(float* to, int64_t n, hipStream_t st) {
+  if (n <= 0) return HSTU_OK;
+  const int64_t blocks = (n + 1023) / 1024;
+  hipLaunchKernelGGL(hstu_clear, dim3((unsigned)(blocks < 16384 ? blocks : 16384)), dim3(256), 0, st, to, n);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "clear launch: %s", hipGetErrorString(e));
+  return HSTU_OK;
 }
 
 }  // namespace
@@ -5961,6 +6233,7 @@ const char* hstu_attn_bwd_variant(const HstuAttnBwdArgs* args) {
   HstuAttnBwdArgs own;
   args = today(args, own);
   if (!args || args->struct_size != sizeof(HstuAttnBwdArgs) || args->version != HSTU_ATTN_ABI_VERSION) return "invalid";
+  args = without_bwd_flags(args, own);
   HstuAttnFwdArgs probe = args->fwd;
   if (!probe.out) probe.out = (void*)args->dout;
   if (validate(&probe) != HSTU_OK || probe.qk_dtype == HSTU_DTYPE_FP8_E4M3FN) return "invalid";
@@ -5978,6 +6251,8 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
   if (args->struct_size != sizeof(HstuAttnBwdArgs) || args->version != HSTU_ATTN_ABI_VERSION)
     return fail(HSTU_ERR_VERSION, "backward args struct_size/version (%u/%u) do not match this library (%zu/%d)",
                 args->struct_size, args->version, sizeof(HstuAttnBwdArgs), HSTU_ATTN_ABI_VERSION);
+  const bool fresh = args->ddense_bias && (args->fwd.flags & HSTU_BWD_WRITE_BIAS_GRADIENT);
+  args = without_bwd_flags(args, own);
   const HstuAttnFwdArgs* f = &args->fwd;
   // the forward's own checks apply, except that its `out` is not needed
   HstuAttnFwdArgs probe = *f;
@@ -5986,7 +6261,9 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
   if (rc != HSTU_OK) return rc;
   g_err[0] = 0;
   if (f->qk_dtype == HSTU_DTYPE_FP8_E4M3FN) return fail(HSTU_ERR_DTYPE, "the backward takes fp32 or bf16 storage, not fp8 q/k");
-  if (f->B == 0 || (f->layout == HSTU_LAYOUT_JAGGED && f->total_tokens == 0)) return HSTU_OK;
+  const bool nothing = f->B == 0 || (f->layout == HSTU_LAYOUT_JAGGED && f->total_tokens == 0);
+  if (nothing && fresh && f->dense_bias) return clear_floats(args->ddense_bias, (int64_t)(f->dense_bias_batched ? f->B : 1) * f->L * f->Lkv, (hipStream_t)stream);
+  if (nothing) return HSTU_OK;
   if (!args->dout || !args->dq || !args->dk || !args->dv) return fail(HSTU_ERR_NULL, "dout, dq, dk and dv must be non-null");
   Params p = make_params(f);
   p.dout = args->dout; p.dq = args->dq; p.dk = args->dk; p.dv = args->dv;
@@ -5998,6 +6275,9 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
   if (bwd_mfma_eligible(args)) {
     for (const void* x : {q_pre, k_pre, v_pre})
       if ((uintptr_t)x & 15u) return fail(HSTU_ERR_SHAPE, "q_pre, k_pre and v_pre must be 16-byte aligned");
+    p.dbias_fresh = fresh && dbias_apart(p) ? 1 : 0;
+    if (fresh && !p.dbias_fresh)
+      if (int rc2 = clear_floats(p.dbias, (int64_t)(p.dense_bias_batched ? p.B : 1) * p.L * p.Lkv, st)) return rc2;
     return launch_bwd_mfma(args, p, st);
   }
   if (q_pre || k_pre || v_pre) return fail(HSTU_ERR_SHAPE, "gradients through the activation are for the matrix-core backward's calls");
@@ -6006,6 +6286,8 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
   // (the general kernels sum the bucket table's gradient in LDS first, one float per entry)
   if (p.dts && p.ts_tab && p.ts_nb > 4095)
     return fail(HSTU_ERR_SHAPE, "the gradient of a timestamp table of more than 4096 entries is not supported, got %d", p.ts_nb + 1);
+  if (fresh)
+    if (int rc2 = clear_floats(p.dbias, (int64_t)(p.dense_bias_batched ? p.B : 1) * p.L * p.Lkv, st)) return rc2;
   return f->qk_dtype == HSTU_DTYPE_FP32 ? launch_bwd<float>(p, st) : launch_bwd<bf16_t>(p, st);
 }
 

@@ -95,7 +95,8 @@ struct Params {
   void* dv;
   float* dpos;
   float* dts;
-  float* dbias;              // gradient of the dense bias (general backward), or null
+  float* dbias;              // gradient of the dense bias, or null
+  int32_t dbias_fresh;       // it is written, not added to
   int64_t items_max;         // capacity of the list (sizes the grid)
 };
 

@@ -384,8 +384,9 @@ struct AttentionBackward : public torch::autograd::Node {
       }
     }
     if (has_bias && task_should_compute_output(5)) {
-      dbias = at::zeros(bs.sizes(), bs.options().requires_grad(false));
+      dbias = at::empty(bs.sizes(), bs.options().requires_grad(false));
       b.ddense_bias = dbias.data_ptr<float>();
+      b.fwd.flags |= HSTU_BWD_WRITE_BIAS_GRADIENT;
     }
     const int rc = hstu_attn_bwd(&b, stream_of(t[0]));
     TORCH_CHECK(rc == HSTU_OK, "hstu_attn_bwd failed (", rc, "): ", hstu_attn_last_error());

@@ -524,6 +524,8 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
   ba.struct_size = C.sizeof(_lib.HstuAttnBwdArgs)
   ba.version = _lib.ABI_VERSION
   fa.flags |= int(_flags)       # (comparison switches of the tests)
+  if bias_grad:
+    fa.flags |= _lib.BWD_WRITE_BIAS_GRADIENT
   ba.fwd = fa
   ba.dout, ba.dq, ba.dk, ba.dv = dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
   dpos = dts = None
@@ -537,7 +539,7 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
   if bias_grad:
     if bias is None:
       raise ValueError("bias_grad=True needs a dense `bias`")
-    dbias = torch.zeros((fa.B if fa.dense_bias_batched else 1, fa.L, fa.Lkv), dtype=torch.float32, device=q.device)
+    dbias = torch.empty((fa.B if fa.dense_bias_batched else 1, fa.L, fa.Lkv), dtype=torch.float32, device=q.device)
     ba.ddense_bias = dbias.data_ptr()
   lib = _lib.load()
   if _variant_out is not None:
