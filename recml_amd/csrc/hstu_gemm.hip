@@ -479,21 +479,22 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
 
-// The forward product where whole rows of x fit a wave's registers (contractions of 256 and 512; no bias, nothing added) and the output
-// is a large one.  A wave keeps 32 rows of x as fragments and the weight goes by in LDS, 32 columns and the whole contraction a stage.  A
-// workgroup is eight waves, 256 rows; it takes a run of pieces of (256 rows, 64 columns), rows by rows: its ring of stages never empties,
-// and x is read once, or twice where a tile is two workgroups'.
+// The forward product where whole rows of x fit a wave's registers (contractions of 256 and 512, no bias) and the output is a large one.
+// A wave keeps 32 rows of x as fragments and the weight goes by in LDS, 32 columns and the whole contraction a stage.  A workgroup is eight
+// waves, 256 rows; it takes a run of pieces of (256 rows, 64 columns), rows by rows: its ring of stages never empties, and x is read once, or
+// twice where a tile is two workgroups'.
 //   What bounds hstu_gemm_kernel at a short contraction is that a tile's products and its epilogue take turns (74 k x 512 -> 2048: 139 us
 // and 55).  Here the products of a column block stand beside the activation of the one before it, four outputs' steps at a time, and a
 // second wave of the SIMD beside both.  74 k x 512 -> 2048 with SiLU 197 -> 150 us, with the pre-activation 216 -> 181, plain 177 -> 142;
-// 74 k x 256 -> 1024 74 -> 51, 90 -> 65.  What is left is the matrix pipes' clock on real operands beside the bytes that move: without
-// loads of the weight 11 % less, without stores 14 %, without either 25 %.  Two blocks of 32 rows a wave, one wave per SIMD, halve the reads of LDS and are no faster (161, 191, 149; 55, 67).
+// 74 k x 256 -> 1024 74 -> 51, 90 -> 65; added to other rows, 78 k x 512 -> 512 75 -> 66, 25.6 k x 512 -> 2048 98 -> 68.  What is left is the
+// matrix pipes' clock on real operands beside the bytes that move: without loads of the weight 11 % less, without stores 14 %, without
+// either 25 %.  Two blocks of 32 rows a wave, one wave per SIMD, halve the reads of LDS and are no faster (161, 191, 149; 55, 67).
 template <int K, int OUT>
 __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams g) {
   constexpr int NS = K / 16, STAGE = K * 64, STAGES = 3, AHEAD = 3;
   constexpr int LP = STAGE / 8192;                       // direct loads of 1 KB per wave and stage
-  constexpr bool PRE = OUT == OUT_PRE_SILU;
-  constexpr int STORES = PRE ? 8 : 4;
+  constexpr bool PRE = OUT == OUT_PRE_SILU, ADD = OUT == OUT_ADD;
+  constexpr int STORES = PRE ? 8 : 4, FROM = ADD ? 4 : 0;      // FROM: the product of a step at which its loads begin
   static_assert(LP <= 4, "a step's stores follow its loads");
   static_assert(NS % (AHEAD + 1) == 0 && 32 % NS == 0 && NS >= 16, "fragments keep their registers from step to step");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -543,7 +544,7 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   bf16x8 qf[NS];
   auto load_rows = [&](int tile) __attribute__((always_inline)) {
     int row = 256 * tile + 32 * w + l32;
-    row = row < g.rows ? row : g.rows - 1;              // (what it gives is not stored)
+    row = row < g.rows ? row : g.rows - 1;              // (what a row past the end gives is not stored)
     const bf16_t* at = g.q + (int64_t)row * g.q_stride + 8 * hh;
 #pragma unroll
     for (int s = 0; s < NS; ++s) qf[s] = *(const bf16x8*)(at + 16 * s);
@@ -556,7 +557,8 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
 
   // ---- the epilogue: 32 rows x 64 columns through the wave's own LDS, rows of 128 bytes, 8-byte piece c of row r at c ^ (r / 2 % 16)
   // (written a column piece of all rows at a time, read a row at a time: all banks both ways)
-  unsigned char* const out_lds = smem + STAGES * STAGE + w * 4096;
+  // ADD: in fp32, rows of 256 bytes, 16-byte piece c of row r at c ^ r % 16: what is added comes by rows too, and one rounding follows.
+  unsigned char* const out_lds = smem + STAGES * STAGE + w * (ADD ? 8192 : 4096);
   unsigned char* const pre_lds = out_lds + 32768;
   float z[4], e[4];
   uint32_t zw[2], ow[2];
@@ -567,7 +569,7 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   // part `ph` of 32: eight for each four columns of a lane
   auto epilogue = [&](const floatx16& old, auto par_, auto ph_) __attribute__((always_inline)) {
     constexpr int ph = decltype(ph_)::value, q4 = ph >> 3, par = decltype(par_)::value;
-    constexpr bool act = OUT != OUT_PLAIN;
+    constexpr bool act = OUT == OUT_SILU || PRE;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if constexpr ((ph & 7) == 0) z[i] = old[4 * q4 + i];
@@ -587,11 +589,12 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
       z[3] = __builtin_bit_cast(float, zw[1] & 0xffff0000u);
     }
     if constexpr (PRE && (ph & 7) == 4) put(pre_lds, par, q4, zw);
-    if constexpr ((ph & 7) == 6) {
+    if constexpr (ADD && (ph & 7) == 7) *(float4*)(out_lds + l32 * 256 + (((8 * par + 2 * q4 + hh) ^ (l32 & 15)) * 16)) = float4{z[0], z[1], z[2], z[3]};
+    if constexpr (!ADD && (ph & 7) == 6) {
       ow[0] = pack2(z[0], z[1]);
       ow[1] = pack2(z[2], z[3]);
     }
-    if constexpr ((ph & 7) == 7) put(out_lds, par, q4, ow);
+    if constexpr (!ADD && (ph & 7) == 7) put(out_lds, par, q4, ow);
   };
   typedef uint32_t words __attribute__((ext_vector_type(4)));
   words rows_out[4], rows_pre[4];
@@ -601,11 +604,29 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
     const words v = *(const words*)(from + row * 128 + (((lane & 7) ^ ((row >> 2) & 7)) * 16));
     return words{halves ? v[2] : v[0], halves ? v[3] : v[1], halves ? v[0] : v[2], halves ? v[1] : v[3]};
   };
+  words add_rows[4];
+  auto take_added = [&](int i) __attribute__((always_inline)) {
+    const int row = (lane >> 3) + 8 * i;
+    const float4 v0 = *(const float4*)(out_lds + row * 256 + (((2 * (lane & 7)) ^ (row & 15)) * 16));
+    const float4 v1 = *(const float4*)(out_lds + row * 256 + (((2 * (lane & 7) + 1) ^ (row & 15)) * 16));
+    float x[8];
+    unpack8(__builtin_bit_cast(uint4, add_rows[i]), x);
+    x[0] += v0.x; x[1] += v0.y; x[2] += v0.z; x[3] += v0.w;
+    x[4] += v1.x; x[5] += v1.y; x[6] += v1.z; x[7] += v1.w;
+    return __builtin_bit_cast(words, pack8(x));
+  };
   const uint32_t out_at = (uint32_t)((32 * w + (lane >> 3)) * (int)g.out_stride + 8 * (lane & 7)) * 2u;
   const uint32_t out_step = (uint32_t)(8 * (int)g.out_stride) * 2u;
   // (past the L2s, see store_past; rows past the output's end lie past the buffer's: nothing is stored, and as many stores are under way)
   bf16_t *to_out = g.out[0], *to_pre = g.pre;
-  uint32_t to_bytes = 0;
+  const bf16_t* from_c = g.c;
+  uint32_t to_bytes = 0, c_bytes = 0;
+  const uint32_t c_at = ADD ? (uint32_t)((32 * w + (lane >> 3)) * (int)g.c_stride + 8 * (lane & 7)) * 2u : 0u;
+  const uint32_t c_step = ADD ? (uint32_t)(8 * (int)g.c_stride) * 2u : 0u;
+  auto ask_added = [&](int i) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)from_c, 0, (int)c_bytes, 0x00020000);
+    add_rows[i] = __builtin_bit_cast(words, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(c_at + i * c_step), 0, 0));
+  };
   auto store = [&](bf16_t* base, const words& v, int i) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)to_bytes, 0x00020000);
     __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)(out_at + i * out_step), 0, 2);
@@ -624,28 +645,29 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (s == NS - AHEAD) {
         // (everything asked of the stage is here, and behind the barrier everyone's is: its place can be refilled.  Younger than the next
-        // stage's loads: those of the one after it and one pair's stores)
+        // stage's loads: those of the one after it, one pair's stores, and of what is added that pair's rows)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        HSTU_WAIT_VMCNT(LP + STORES);
+        HSTU_WAIT_VMCNT(LP + STORES + (ADD && par == 0 ? 4 : 0));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
       }
       if constexpr (s + AHEAD < NS) ask(st, s + AHEAD);
       else ask(next, s + AHEAD - NS);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s % (AHEAD + 1)], qf[s], s == 0 ? zero : acc, 0, 0, 0);
-      if constexpr (s < LP) dma(refill, s);
+      if constexpr (ADD && par == 0 && s < 4) ask_added(s);
+      if constexpr (s >= FROM && s < FROM + LP) dma(refill, s - FROM);
       if constexpr (par == 1) {
-        // (the first part that writes there again is the fifth)
+        // (the first part that writes there again is the fifth; of what is added the eighth)
         each<PER>([&](auto i_) __attribute__((always_inline)) {
           constexpr int i = s * PER + decltype(i_)::value;
           if constexpr (i < 4) {
-            rows_out[i] = take(out_lds, i);
+            rows_out[i] = ADD ? take_added(i) : take(out_lds, i);
             if constexpr (PRE) rows_pre[i] = take(pre_lds, i);
           }
         });
-        if constexpr (s >= 4 && s < 8) {
-          store(to_out, rows_out[s - 4], s - 4);
-          if constexpr (PRE) store(to_pre, rows_pre[s - 4], s - 4);
+        if constexpr (s >= FROM + 4 && s < FROM + 8) {
+          store(to_out, rows_out[s - FROM - 4], s - FROM - 4);
+          if constexpr (PRE) store(to_pre, rows_pre[s - FROM - 4], s - FROM - 4);
         }
       }
       each<PER>([&](auto i_) __attribute__((always_inline)) {
@@ -685,6 +707,10 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
     to_out = g.out[0] + (int64_t)m0 * g.out_stride + 64 * pc;
     to_pre = PRE ? g.pre + (int64_t)m0 * g.out_stride + 64 * pc : nullptr;
     to_bytes = (uint32_t)(left * 2);
+    if constexpr (ADD) {
+      from_c = g.c + (int64_t)m0 * g.c_stride + 64 * pc;
+      c_bytes = (uint32_t)((((int64_t)(g.rows - m0 < 256 ? g.rows - m0 : 256) - 1) * g.c_stride + (g.cols - 64 * pc)) * 2);
+    }
     if (++pc == pairs) {
       pc = 0;
       ++rt;
@@ -696,7 +722,8 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   });
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    store(to_out, take(out_lds, i), i);
+    if constexpr (ADD) ask_added(i);
+    store(to_out, ADD ? take_added(i) : take(out_lds, i), i);
     if (PRE) store(to_pre, take(pre_lds, i), i);
   }
   HSTU_WAIT_VMCNT(0);        // (no direct load may arrive in LDS that is another workgroup's by then)
@@ -830,18 +857,18 @@ int pick_splits(int64_t rows, int64_t cols, int64_t depth, int* tile) {
 
 // Whether hstu_gemm_rows_kernel takes the product: from six pieces for each of its workgroups on.  Below, reading the rows before the first
 // product (12 us, twice where a workgroup's run crosses a tile's end) costs more than is won.  us here / with the tiles, at 6.2 pieces:
-// 12800 x 512 -> 2048 40.5 / 40.7, with the pre-activation 44 / 49, 51200 x 512 -> 512 40 / 42, 51200 x 256 -> 512 25 / 30, 25600 x 256 -> 1024
-// 24 / 29; at 12.5: 25600 x 512 -> 2048 62 / 80; at 3.1: 6400 x 512 -> 2048 31 / 24, 25600 x 256 -> 512 19 / 18.
+// 12800 x 512 -> 2048 40.5 / 40.7, with the pre-activation 44 / 49, added to rows 43 / 50, 51200 x 512 -> 512 40 / 42 and 44 / 51, 51200 x 256
+// -> 512 25 / 30 and 29 / 35, 25600 x 256 -> 1024 24 / 29; at 12.5: 25600 x 512 -> 2048 62 / 80; at 3.1: 6400 x 512 -> 2048 31 / 24, 25600 x 256 -> 512 19 / 18.
 constexpr int ROWS_GRID = 256;                 // a workgroup per CU
 bool rows_product(const GemmParams& g) {
-  return (g.depth == 256 || g.depth == 512) && !g.bias && !g.c && (g.activation || !g.pre) && g.cols % 64 == 0 && g.slab % 32 == 0 &&
+  return (g.depth == 256 || g.depth == 512) && !g.bias && (!g.c || (!g.activation && !g.pre && g.c_stride < 1 << 20)) && (g.activation || !g.pre) && g.cols % 64 == 0 && g.slab % 32 == 0 &&
          g.out_stride < 1 << 20 && g.p_stride < 1 << 20 && (int64_t)((g.rows + 255) / 256) * (g.cols / 64) >= 6 * ROWS_GRID;
 }
 
 template <int K, int OUT>
 int launch_rows_as(GemmParams g, hipStream_t st) {
   static int granted[64];
-  constexpr int smem = 3 * K * 64 + (OUT == OUT_PRE_SILU ? 65536 : 32768);
+  constexpr int smem = 3 * K * 64 + (OUT == OUT_PRE_SILU || OUT == OUT_ADD ? 65536 : 32768);
   g.row_tiles = (g.rows + 255) / 256;
   if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT>, smem, granted)) return rc;
   hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT>), dim3(ROWS_GRID), dim3(512), smem, st, g);
@@ -851,6 +878,7 @@ int launch_rows_as(GemmParams g, hipStream_t st) {
 }
 template <int K>
 int launch_rows(const GemmParams& g, hipStream_t st) {
+  if (g.c) return launch_rows_as<K, OUT_ADD>(g, st);
   if (g.pre) return launch_rows_as<K, OUT_PRE_SILU>(g, st);
   if (g.activation) return launch_rows_as<K, OUT_SILU>(g, st);
   return launch_rows_as<K, OUT_PLAIN>(g, st);

@@ -77,12 +77,14 @@ def test_rows_in_registers(gpu, M, N, K, slabs):
   g = torch.Generator(device="cuda").manual_seed(M + N)
   x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
   ws = [(torch.randn(K, N // slabs, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16) for _ in range(slabs)]
-  for kw in ({}, dict(activation=True), dict(activation=True, want_pre=True)):
+  added = torch.randn(M, N + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :N]
+  for kw in ({}, dict(residual=added), dict(activation=True), dict(activation=True, want_pre=True)):
     parts = lambda r: r if isinstance(r, tuple) else (r,)
     got = parts(ops.block_gemm(_lib_block.GEMM_NN, x, ws, **kw))
     for at in range(0, M, 4000):
       part = slice(at, min(at + 4000, M))
-      for a, b in zip(got, parts(ops.block_gemm(_lib_block.GEMM_NN, x[part], ws, **kw))):
+      of_part = {k: v[part] if k == "residual" else v for k, v in kw.items()}
+      for a, b in zip(got, parts(ops.block_gemm(_lib_block.GEMM_NN, x[part], ws, **of_part))):
         assert torch.equal(a[part], b)
   want = x[-300:].float() @ torch.cat(ws, 1).float()
   _close(got[1][-300:], want)
