@@ -261,6 +261,26 @@ typedef struct HstuGemmArgs {
 size_t hstu_gemm_workspace_bytes(int32_t op, int64_t M, int32_t N, int32_t K);
 int hstu_gemm(const HstuGemmArgs* args, void* stream);
 
+/* The layer norm in front of a product and the product as one launch, for large batches (hstu.py:443-449): out = silu(layer_norm(x) w), the
+ * normed rows rounded as hstu_norm_gate_fwd rounds them.  bf16; x [M, K] with a row stride of whole 16 bytes, gamma and beta [K], w as in
+ * HstuGemmArgs, out [M, N] contiguous.  Which sizes there are: hstu_norm_gemm_takes (1 or 0). */
+typedef struct HstuNormGemmArgs {
+  uint32_t struct_size;   /* sizeof(HstuNormGemmArgs) */
+  uint32_t version;       /* HSTU_BLOCK_ABI_VERSION   */
+  int64_t M;
+  int32_t N, K, slabs;
+  float eps;
+  const void* x;
+  int64_t x_stride;
+  const void* gamma;
+  const void* beta;
+  const void* w[HSTU_GEMM_MAX_SLABS];
+  void* out;
+} HstuNormGemmArgs;
+
+int hstu_norm_gemm_takes(int64_t M, int32_t N, int32_t K, int32_t slabs);
+int hstu_norm_gemm(const HstuNormGemmArgs* args, void* stream);
+
 /* A whole block in inference as one launch, for short sequences and narrow models (hstu.py:442-474): out = tokens + output projection of
  * u * layer_norm(attention) with u, q, k, v = silu(layer_norm(tokens) w + bias), causal pointwise attention over alpha q k^T
  * (+ pos_tab) with the weights scaled by inv_n and each sequence's length.  bf16 tensors and parameters, contiguous; tokens and out

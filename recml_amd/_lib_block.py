@@ -28,6 +28,8 @@ EXPORTS = (
     "hstu_silu_bwd",
     "hstu_gemm",
     "hstu_gemm_workspace_bytes",
+    "hstu_norm_gemm_takes",
+    "hstu_norm_gemm",
     "hstu_block_small_takes",
     "hstu_block_small_fwd",
     "hstu_block_small_stack_fwd",
@@ -94,6 +96,15 @@ class HstuGemmArgs(C.Structure):
 
 
 GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2
+
+
+class HstuNormGemmArgs(C.Structure):
+  _fields_ = [
+      ("struct_size", C.c_uint32), ("version", C.c_uint32),
+      ("M", C.c_int64), ("N", C.c_int32), ("K", C.c_int32), ("slabs", C.c_int32), ("eps", C.c_float),
+      ("x", C.c_void_p), ("x_stride", C.c_int64), ("gamma", C.c_void_p), ("beta", C.c_void_p),
+      ("w", C.c_void_p * 4), ("out", C.c_void_p),
+  ]
 
 
 class HstuEmbedNormArgs(C.Structure):
@@ -167,6 +178,10 @@ def load():
     lib.hstu_embed_grad.argtypes = [C.POINTER(HstuEmbedGradArgs), C.c_void_p]
     lib.hstu_embed_grad_workspace_bytes.restype = C.c_size_t
     lib.hstu_embed_grad_workspace_bytes.argtypes = [C.c_int64, C.c_int64, C.c_int32]
+    lib.hstu_norm_gemm_takes.restype = C.c_int
+    lib.hstu_norm_gemm_takes.argtypes = [C.c_int64, C.c_int32, C.c_int32, C.c_int32]
+    lib.hstu_norm_gemm.restype = C.c_int
+    lib.hstu_norm_gemm.argtypes = [C.POINTER(HstuNormGemmArgs), C.c_void_p]
     lib.hstu_silu_bwd.restype = C.c_int
     lib.hstu_silu_bwd.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_void_p]
     ver = lib.hstu_block_abi_version()

@@ -33,6 +33,8 @@ struct GemmParams {
   bf16_t* pre;                       // the value before the activation is stored here as well (or null)
   const bf16_t* bias;
   const bf16_t* c;
+  const bf16_t *gamma, *beta;             // (hstu_gemm_rows_kernel: the rows' layer norm, or null)
+  float eps;
   int64_t q_stride, p_stride, out_stride, c_stride;
   int32_t rows, cols, depth;         // of the product: output rows and columns, contraction
   int32_t slab, out_slab;            // width of a slab of `p` (along the weight's n) and of `out` (along its columns)
@@ -489,7 +491,12 @@ __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence
 // 74 k x 256 -> 1024 74 -> 51, 90 -> 65; added to other rows, 78 k x 512 -> 512 75 -> 66, 25.6 k x 512 -> 2048 98 -> 68.  What is left is the
 // matrix pipes' clock on real operands beside the bytes that move: without loads of the weight 11 % less, without stores 14 %, without
 // either 25 %.  Two blocks of 32 rows a wave, one wave per SIMD, halve the reads of LDS and are no faster (161, 191, 149; 55, 67).
-template <int K, int OUT>
+//   NORM: the layer norm in front of the product on the rows in their registers.  A launch less, and the normed rows are neither written nor
+// read again; the norm's 21 instructions for two elements stand before a tile's first product, so that it takes two thirds of what it
+// saves (norm and product 78 k x 512 -> 2048 209 -> 200 us, 150 k 385 -> 354, 33 k 96 -> 93, 66 k x 256 -> 1024 72 -> 62, 100 k 93 -> 90; 13 k
+// x 512 -> 2048, where more of it is before a first product, 51 -> 55).  (A gate, and the sum of the output product, beside it do not fit the
+// registers: 110 -> 250 us.)
+template <int K, int OUT, bool NORM>
 __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams g) {
   constexpr int NS = K / 16, STAGE = K * 64, STAGES = 3, AHEAD = 3;
   constexpr int LP = STAGE / 8192;                       // direct loads of 1 KB per wave and stage
@@ -553,6 +560,47 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   auto rows_here = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+  };
+  // NORM: the rows' layer norm, as hstu_norm_gate has it (the mean, then the squares about it).  A lane holds half of its row.
+  auto both_halves = [&](float x) __attribute__((always_inline)) { return x + __shfl_xor(x, 32, 64); };
+  auto norm_rows = [&]() __attribute__((always_inline)) {
+    float sum[4] = {0.f, 0.f, 0.f, 0.f}, ss[4] = {0.f, 0.f, 0.f, 0.f};
+    // (each pass unpacks the rows again: kept from one to the next they would be two registers for each of theirs)
+    each<NS>([&](auto s_) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_)::value;
+      float x[8];
+      unpack8(__builtin_bit_cast(uint4, qf[s]), x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum[i & 3] += x[i];
+      if constexpr (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+    rows_here();
+    const float mean = both_halves((sum[0] + sum[1]) + (sum[2] + sum[3])) * (1.0f / K);
+    each<NS>([&](auto s_) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_)::value;
+      float x[8];
+      unpack8(__builtin_bit_cast(uint4, qf[s]), x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float d = x[i] - mean;
+        ss[i & 3] = __builtin_fmaf(d, d, ss[i & 3]);
+      }
+      if constexpr (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+    rows_here();
+    const float rstd = __builtin_amdgcn_rsqf(both_halves((ss[0] + ss[1]) + (ss[2] + ss[3])) * (1.0f / K) + g.eps);
+    each<NS>([&](auto s_) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_)::value;
+      float x[8], ga[8], be[8];
+      unpack8(__builtin_bit_cast(uint4, qf[s]), x);
+      unpack8(*(const uint4*)(g.gamma + 16 * s + 8 * hh), ga);
+      unpack8(*(const uint4*)(g.beta + 16 * s + 8 * hh), be);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf((x[i] - mean) * rstd, ga[i], be[i]);
+      qf[s] = __builtin_bit_cast(bf16x8, pack8(x));
+      if constexpr (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+    rows_here();
   };
 
   // ---- the epilogue: 32 rows x 64 columns through the wave's own LDS, rows of 128 bytes, 8-byte piece c of row r at c ^ (r / 2 % 16)
@@ -692,11 +740,17 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   for (int s = 0; s < AHEAD; ++s) ask(0, s);
   rows_here();
   int st = 0, have = rt;
+  bool as_stored = NORM;
   for (; todo > 0; --todo) {
     if (rt != have) {
       load_rows(rt);
       rows_here();
       have = rt;
+      as_stored = NORM;
+    }
+    if constexpr (NORM) {
+      if (as_stored) norm_rows();
+      as_stored = false;
     }
     step(std::integral_constant<int, 0>{}, st, acc_a, acc_b);
     st = st + 1 >= STAGES ? 0 : st + 1;
@@ -865,23 +919,24 @@ bool rows_product(const GemmParams& g) {
          g.out_stride < 1 << 20 && g.p_stride < 1 << 20 && (int64_t)((g.rows + 255) / 256) * (g.cols / 64) >= 6 * ROWS_GRID;
 }
 
-template <int K, int OUT>
+template <int K, int OUT, bool NORM>
 int launch_rows_as(GemmParams g, hipStream_t st) {
   static int granted[64];
   constexpr int smem = 3 * K * 64 + (OUT == OUT_PRE_SILU || OUT == OUT_ADD ? 65536 : 32768);
   g.row_tiles = (g.rows + 255) / 256;
-  if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT>, smem, granted)) return rc;
-  hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT>), dim3(ROWS_GRID), dim3(512), smem, st, g);
+  if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT, NORM>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT, NORM>), dim3(ROWS_GRID), dim3(512), smem, st, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 template <int K>
 int launch_rows(const GemmParams& g, hipStream_t st) {
-  if (g.c) return launch_rows_as<K, OUT_ADD>(g, st);
-  if (g.pre) return launch_rows_as<K, OUT_PRE_SILU>(g, st);
-  if (g.activation) return launch_rows_as<K, OUT_SILU>(g, st);
-  return launch_rows_as<K, OUT_PLAIN>(g, st);
+  if (g.gamma) return launch_rows_as<K, OUT_SILU, true>(g, st);
+  if (g.c) return launch_rows_as<K, OUT_ADD, false>(g, st);
+  if (g.pre) return launch_rows_as<K, OUT_PRE_SILU, false>(g, st);
+  if (g.activation) return launch_rows_as<K, OUT_SILU, false>(g, st);
+  return launch_rows_as<K, OUT_PLAIN, false>(g, st);
 }
 
 // out = act(x w + c + bias) for widths that the kernel above cannot fetch 16 bytes at a time: element by element, fp32 products.  (One
@@ -1063,6 +1118,42 @@ int hstu_gemm(const HstuGemmArgs* a, void* stream) {
   p.out_stride = a->K;
   p.depth = p.depth_per_split = a->N;
   return launch_sized<false, false>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, false, 256, 256), false));
+}
+
+// (from sixteen pieces a workgroup on: see NORM)
+int hstu_norm_gemm_takes(int64_t M, int32_t N, int32_t K, int32_t slabs) {
+  if (M < 1 || M > 0x3fffffff || N < 64 || slabs < 1 || slabs > HSTU_GEMM_MAX_SLABS || N % slabs) return 0;
+  GemmParams p = {};
+  p.rows = (int32_t)M; p.cols = N; p.depth = K; p.slab = p.p_stride = N / slabs; p.out_stride = N;
+  p.activation = 1;
+  return rows_product(p) && (int64_t)((p.rows + 255) / 256) * (N / 64) >= 16 * ROWS_GRID ? 1 : 0;
+}
+
+int hstu_norm_gemm(const HstuNormGemmArgs* a, void* stream) {
+  if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
+  if (a->struct_size != sizeof(HstuNormGemmArgs) || a->version != HSTU_BLOCK_ABI_VERSION)
+    return block_fail(HSTU_BLOCK_ERR_VERSION, "norm-gemm args struct_size/version (%u/%u) do not match this library (%zu/%d)", a->struct_size, a->version,
+                      sizeof(HstuNormGemmArgs), HSTU_BLOCK_ABI_VERSION);
+  if (!hstu_norm_gemm_takes(a->M, a->N, a->K, a->slabs))
+    return block_fail(HSTU_BLOCK_ERR_SHAPE, "no kernel for M=%lld N=%d K=%d in %d slabs (hstu_norm_gemm_takes)", (long long)a->M, a->N, a->K, a->slabs);
+  bool ok = a->x && a->gamma && a->beta && a->out && a->x_stride >= a->K && (a->x_stride & 7) == 0;
+  for (const void* t : {a->x, a->gamma, a->beta, (const void*)a->out}) ok = ok && block_aligned16(t);
+  for (int i = 0; i < a->slabs; ++i) ok = ok && a->w[i] && block_aligned16(a->w[i]);
+  if (!ok) return block_fail(HSTU_BLOCK_ERR_SHAPE, "operands must be present, 16-byte aligned, with row strides of whole 16-byte pieces");
+  block_clear_error();
+  GemmParams p = {};
+  p.q = (const bf16_t*)a->x; p.q_stride = a->x_stride;
+  p.gamma = (const bf16_t*)a->gamma; p.beta = (const bf16_t*)a->beta;
+  p.eps = a->eps;
+  p.splits = 1;
+  p.slab = a->N / a->slabs;
+  for (int i = 0; i < HSTU_GEMM_MAX_SLABS; ++i) p.p[i] = (const bf16_t*)a->w[i < a->slabs ? i : a->slabs - 1];
+  p.p_stride = p.slab;
+  p.rows = (int32_t)a->M; p.cols = p.out_slab = a->N; p.out_stride = a->N;
+  p.depth = p.depth_per_split = a->K;
+  p.out[0] = (bf16_t*)a->out;
+  p.activation = 1;
+  return a->K == 512 ? launch_rows<512>(p, (hipStream_t)stream) : launch_rows<256>(p, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -605,6 +605,23 @@ bool small_block(Tensor& out, const Tensor& tokens, const Tensor (&p)[P_COUNT], 
   return true;
 }
 
+// The input norm and the four projections as one launch, where there is one for their sizes; false: nothing has been done.
+bool norm_projections(const Tensor& uqkv, const Tensor& tokens, const Tensor (&p)[P_COUNT], int64_t T, int64_t D, int64_t W, double eps) {
+  if (T > 0x3fffffff || D > 512 || 4 * W > 1 << 20 || !hstu_norm_gemm_takes(T, (int32_t)(4 * W), (int32_t)D, 4)) return false;
+  HstuNormGemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.version = HSTU_BLOCK_ABI_VERSION;
+  a.M = T; a.N = (int32_t)(4 * W); a.K = (int32_t)D; a.slabs = 4; a.eps = (float)eps;
+  a.x = tokens.const_data_ptr(); a.x_stride = D;
+  a.gamma = p[P_IN_G].const_data_ptr(); a.beta = p[P_IN_B].const_data_ptr();
+  const int order[4] = {P_U, P_Q, P_K, P_V};
+  for (int i = 0; i < 4; ++i) a.w[i] = p[order[i]].const_data_ptr();
+  a.out = uqkv.data_ptr();
+  block_check(hstu_norm_gemm(&a, stream_of(tokens)), "hstu_norm_gemm");
+  return true;
+}
+
 // slice i of a projection [T, 4, H, hd], shaped as the attention takes it
 Tensor projection_slice(const Tensor& uqkv, const BlockCall& c, int i) {
   const int64_t W = c.H * c.hd;
@@ -1080,12 +1097,14 @@ PyObject* block(PyObject*, PyObject* const* a, Py_ssize_t count) {
       HstuAttnFwdArgs a;
       const Tensor q = projection_slice(uqkv, c, 1);
       if (!fill(a, q, projection_slice(uqkv, c, 2), projection_slice(uqkv, c, 3), attn, pos, ts_tab, bias, o)) return false;
-      normed = fresh(tokens, {T, D});
-      norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
-      if (graph) pre = at::empty_like(uqkv);
-      Tensor pb;
-      if (p[P_UB].defined()) pb = at::cat({p[P_UB].view({W}), p[P_QB].view({W}), p[P_KB].view({W}), p[P_VB].view({W})});
-      gemm(HSTU_GEMM_NN, T, {normed.const_data_ptr(), D}, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W, uqkv, pb, {nullptr, 0}, true, pre);
+      if (graph || p[P_UB].defined() || !norm_projections(uqkv, tokens, p, T, D, W, c.eps)) {
+        normed = fresh(tokens, {T, D});
+        norm(normed, {tokens.const_data_ptr(), D}, {nullptr, 0}, p[P_IN_G], p[P_IN_B], T, D, c.eps);
+        if (graph) pre = at::empty_like(uqkv);
+        Tensor pb;
+        if (p[P_UB].defined()) pb = at::cat({p[P_UB].view({W}), p[P_QB].view({W}), p[P_KB].view({W}), p[P_VB].view({W})});
+        gemm(HSTU_GEMM_NN, T, {normed.const_data_ptr(), D}, {&p[P_U], &p[P_Q], &p[P_K], &p[P_V]}, D, 4 * W, uqkv, pb, {nullptr, 0}, true, pre);
+      }
       if (!forward(a, q, pos, ts_tab, bias, o, share ? &shared : nullptr)) return false;
       gated = fresh(tokens, {T, W});
       norm(gated, {attn.const_data_ptr(), W}, {uqkv.const_data_ptr(), 4 * W}, p[P_ATTN_G], p[P_ATTN_B], T, W, c.eps);

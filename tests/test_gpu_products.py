@@ -91,6 +91,42 @@ def test_rows_in_registers(gpu, M, N, K, slabs):
   _close(got[0][-300:], torch.nn.functional.silu(got[1][-300:].float()))
 
 
+@pytest.mark.parametrize("M,N,K,slabs", [(32513, 2048, 512, 4), (65281, 1024, 256, 1), (58500, 1152, 512, 2)])
+def test_norm_and_product(gpu, M, N, K, slabs):
+  """The layer norm and the product as one launch, with tiles of one row at the end and runs that cross tiles, beside the two launches and
+  64 bits.  The two round the same values at the same places, but their sums go in other orders: a normed value in some thousands
+  falls on the other side of a rounding, 2^-8 of itself, so the errors are alike and few results differ."""
+  lib = _lib_block.load()
+  assert lib.hstu_norm_gemm_takes(M, N, K, slabs) == 1
+  g = torch.Generator(device="cuda").manual_seed(M)
+  x = (torch.randn(M, K + 8, device="cuda", generator=g) * 3 + 1).to(torch.bfloat16)[:, :K]
+  gamma, beta = ((torch.randn(K, device="cuda", generator=g) * 0.2 + i).to(torch.bfloat16) for i in (1, 0))
+  ws = [(torch.randn(K, N // slabs, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16) for _ in range(slabs)]
+  out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+  a = _lib_block.HstuNormGemmArgs()
+  a.struct_size, a.version = C.sizeof(a), _lib_block.ABI_VERSION
+  a.M, a.N, a.K, a.slabs, a.eps = M, N, K, slabs, 1e-6
+  a.x, a.x_stride, a.gamma, a.beta, a.out = x.data_ptr(), x.stride(0), gamma.data_ptr(), beta.data_ptr(), out.data_ptr()
+  for i, w in enumerate(ws):
+    a.w[i] = w.data_ptr()
+  assert lib.hstu_norm_gemm(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+  two = ops.block_gemm(_lib_block.GEMM_NN, ops.layer_norm(x.contiguous(), gamma, beta, 1e-6), ws, activation=True)
+  xd = x.double()
+  xd = (xd - xd.mean(1, keepdim=True)) * torch.rsqrt(xd.var(1, unbiased=False, keepdim=True) + 1e-6)
+  want = torch.nn.functional.silu((xd * gamma.double() + beta.double()) @ torch.cat(ws, 1).double())
+  err = [float((t.double() - want).norm() / want.norm()) for t in (out, two)]
+  assert err[0] <= 1.001 * err[1]
+  assert float((out != two).double().mean()) <= 1e-3
+  assert float((out.float() - two.float()).abs().max()) <= 2.0**-7 * float(two.float().abs().max())
+
+
+def test_norm_and_product_sizes(gpu):
+  takes = _lib_block.load().hstu_norm_gemm_takes
+  assert takes(78000, 2048, 512, 4) == 1 and takes(100000, 1024, 256, 4) == 1
+  assert not any([takes(13000, 2048, 512, 4), takes(78000, 2048, 384, 4), takes(78000, 2080, 512, 1), takes(0, 2048, 512, 4),
+                  takes(78000, 2048, 512, 5), takes(1 << 31, 2048, 512, 4)])
+
+
 @pytest.mark.parametrize("rows,keys,width", [(0, 5, 8), (1, 1, 8), (700, 1, 136), (3000, 40, 64), (3000, 5000, 72), (4097, 257, 128)])
 @pytest.mark.parametrize("scale", [1.0, 2.0])
 def test_gathered_table_gradient(gpu, rows, keys, width, scale):
