@@ -395,7 +395,7 @@ int check_small(const HstuBlockSmallArgs* a, bool first, bool last) {
 extern "C" {
 
 // The shapes there are, and of those the ones where this is the faster form.  A workgroup takes the time of 64 positions whatever its
-// sequence has, one a CU at width 64 (95 KB of LDS): GPU us a block in five launches / in one, 4 heads: 32 sequences of 50 18.1 / 8.4,
+// sequence has, one a CU at width 64 (107 KB of LDS): GPU us a block in five launches / in one, 4 heads: 32 sequences of 50 18.1 / 8.4,
 // 512 35.4 / 18.0, 8192 266 / 224; 1024 of 24 35 / 25, but 8192 of 24 137 / 184.
 int hstu_block_small_takes(int32_t B, int32_t L, int32_t heads, int32_t head_dim, int32_t width) {
   return head_dim == HD && (width == 32 || width == 64) && heads * head_dim == width && L >= 1 && L <= ROWS && B >= 1 && B <= 65535 && (B <= 1024 || L >= 48);
