@@ -481,7 +481,7 @@ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f)
 template <int N, typename F>
 __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
 
-// The forward product where whole rows of x fit a wave's registers (contractions of 256 and 512, no bias) and the output is a large one.
+// The products where whole rows of x fit a wave's registers (contractions of 256 and 512, no bias) and the output is a large one.
 // A wave keeps 32 rows of x as fragments and the weight goes by in LDS, 32 columns and the whole contraction a stage.  A workgroup is eight
 // waves, 256 rows; it takes a run of pieces of (256 rows, 64 columns), rows by rows: its ring of stages never empties, and x is read once, or
 // twice where a tile is two workgroups'.
@@ -496,13 +496,17 @@ __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence
 // saves (norm and product 78 k x 512 -> 2048 209 -> 200 us, 150 k 385 -> 354, 33 k 96 -> 93, 66 k x 256 -> 1024 72 -> 62, 100 k 93 -> 90; 13 k
 // x 512 -> 2048, where more of it is before a first product, 51 -> 55).  (A gate, and the sum of the output product, beside it do not fit the
 // registers: 110 -> 250 us.)
-template <int K, int OUT, bool NORM>
+//   ALONG: the input's gradient, x w^T, whose weight lies along the contraction: a stage is 32 of its rows, read as they lie.  78 k x 512 by
+// 512 60 -> 57 us, 100 k 78 -> 63, 131 k 85 -> 75, 49 k x 256 by 512 25 -> 22,
+// and where the rule begins with 512 of depth, 49 k x 512 by 256, 24 -> 24.
+template <int K, int OUT, bool NORM, bool ALONG>
 __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams g) {
   constexpr int NS = K / 16, STAGE = K * 64, STAGES = 3, AHEAD = 3;
   constexpr int LP = STAGE / 8192;                       // direct loads of 1 KB per wave and stage
   constexpr bool PRE = OUT == OUT_PRE_SILU, ADD = OUT == OUT_ADD;
   constexpr int STORES = PRE ? 8 : 4, FROM = ADD ? 4 : 0;      // FROM: the product of a step at which its loads begin
   static_assert(LP <= 4, "a step's stores follow its loads");
+  static_assert(!ALONG || (OUT == OUT_PLAIN && !NORM), "the input's gradient is a product alone");
   static_assert(NS % (AHEAD + 1) == 0 && 32 % NS == 0 && NS >= 16, "fragments keep their registers from step to step");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const uint32_t smem_lds = __builtin_amdgcn_groupstaticsize();
@@ -519,13 +523,25 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   int rt = __builtin_amdgcn_readfirstlane((int)(first / pairs)), pc = __builtin_amdgcn_readfirstlane((int)(first - (int64_t)rt * pairs));
   int todo = __builtin_amdgcn_readfirstlane((int)(last - first));
 
-  // ---- the weight's stages: rows of 64 bytes, piece i of a wave 16 of them
+  // ---- the weight's stages: 32 of its columns in rows of 64 bytes, piece i of a wave 16 rows.  ALONG: 32 of its rows, which lie along the
+  // contraction, 16-byte chunk c of row r at c ^ r % 16 (16 rows reach all banks); one slab.
   int sl = __builtin_amdgcn_readfirstlane(64 * pc / g.slab), sc = 64 * pc - sl * g.slab;      // slab and column of the next stage to load
+  int wr = 64 * pc;                                      // ALONG: and its row
+  constexpr int RC = K / 8;                              // chunks of such a row
   uint32_t po[LP];
 #pragma unroll
-  for (int i = 0; i < LP; ++i) po[i] = (uint32_t)((16 * (LP * w + i) + (lane >> 2)) * (int)g.p_stride + 8 * (lane & 3)) * 2u;
+  for (int i = 0; i < LP; ++i) {
+    const int piece = LP * w + i, row = (64 * piece + lane) / RC;
+    po[i] = ALONG ? (uint32_t)(row * (int)g.p_stride + 8 * ((lane % RC) ^ (row & 15))) * 2u
+                  : (uint32_t)((16 * piece + (lane >> 2)) * (int)g.p_stride + 8 * (lane & 3)) * 2u;
+  }
   const char* p_base;
   auto next_columns = [&]() __attribute__((always_inline)) {
+    if constexpr (ALONG) {
+      p_base = scalar_ptr(g.p[0] + (int64_t)wr * g.p_stride);
+      wr = wr + 32 == g.cols ? 0 : wr + 32;
+      return;
+    }
     p_base = scalar_ptr(g.p[sl] + sc);
     sc += 32;
     if (sc == g.slab) {
@@ -540,7 +556,12 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   const int gi = lane & 15;
   const uint32_t at_lane = (uint32_t)((8 * hh + (gi >> 2)) * 64 + 32 * ((lane >> 4) & 1) + 8 * (gi & 3));
   bf16x8 f[AHEAD + 1];
+  const uint32_t along_row = (uint32_t)(l32 * 2 * K), along_at = (uint32_t)((hh ^ (l32 & 15)) * 16);
   auto ask = [&](int st, int s) __attribute__((always_inline)) {
+    if constexpr (ALONG) {
+      f[s % (AHEAD + 1)] = *(const bf16x8*)(smem + st * STAGE + along_row + (along_at ^ (uint32_t)(32 * (s & 7))) + 256 * (s >> 3));
+      return;
+    }
     const unsigned char* at = smem + st * STAGE + at_lane + 1024 * s;
     const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at));
     const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(at + 256));
@@ -919,24 +940,25 @@ bool rows_product(const GemmParams& g) {
          g.out_stride < 1 << 20 && g.p_stride < 1 << 20 && (int64_t)((g.rows + 255) / 256) * (g.cols / 64) >= 6 * ROWS_GRID;
 }
 
-template <int K, int OUT, bool NORM>
+template <int K, int OUT, bool NORM = false, bool ALONG = false>
 int launch_rows_as(GemmParams g, hipStream_t st) {
   static int granted[64];
   constexpr int smem = 3 * K * 64 + (OUT == OUT_PRE_SILU || OUT == OUT_ADD ? 65536 : 32768);
   g.row_tiles = (g.rows + 255) / 256;
-  if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT, NORM>, smem, granted)) return rc;
-  hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT, NORM>), dim3(ROWS_GRID), dim3(512), smem, st, g);
+  if (int rc = block_allow_lds((const void*)hstu_gemm_rows_kernel<K, OUT, NORM, ALONG>, smem, granted)) return rc;
+  hipLaunchKernelGGL((hstu_gemm_rows_kernel<K, OUT, NORM, ALONG>), dim3(ROWS_GRID), dim3(512), smem, st, g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
   return HSTU_BLOCK_OK;
 }
 template <int K>
-int launch_rows(const GemmParams& g, hipStream_t st) {
+int launch_rows(const GemmParams& g, bool along, hipStream_t st) {
+  if (along) return launch_rows_as<K, OUT_PLAIN, false, true>(g, st);
   if (g.gamma) return launch_rows_as<K, OUT_SILU, true>(g, st);
-  if (g.c) return launch_rows_as<K, OUT_ADD, false>(g, st);
-  if (g.pre) return launch_rows_as<K, OUT_PRE_SILU, false>(g, st);
-  if (g.activation) return launch_rows_as<K, OUT_SILU, false>(g, st);
-  return launch_rows_as<K, OUT_PLAIN, false>(g, st);
+  if (g.c) return launch_rows_as<K, OUT_ADD>(g, st);
+  if (g.pre) return launch_rows_as<K, OUT_PRE_SILU>(g, st);
+  if (g.activation) return launch_rows_as<K, OUT_SILU>(g, st);
+  return launch_rows_as<K, OUT_PLAIN>(g, st);
 }
 
 // out = act(x w + c + bias) for widths that the kernel above cannot fetch 16 bytes at a time: element by element, fp32 products.  (One
@@ -1111,12 +1133,13 @@ int hstu_gemm(const HstuGemmArgs* a, void* stream) {
     p.cols = p.out_slab = a->N;
     p.out_stride = a->N;
     p.depth = p.depth_per_split = a->K;
-    if (rows_product(p)) return p.depth == 512 ? launch_rows<512>(p, st) : launch_rows<256>(p, st);
+    if (rows_product(p)) return p.depth == 512 ? launch_rows<512>(p, false, st) : launch_rows<256>(p, false, st);
     return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, true, 256, 256), p.c != nullptr));
   }
   p.cols = p.out_slab = a->K;
   p.out_stride = a->K;
   p.depth = p.depth_per_split = a->N;
+  if (a->slabs == 1 && rows_product(p)) return p.depth == 512 ? launch_rows<512>(p, true, st) : launch_rows<256>(p, true, st);
   return launch_sized<false, false>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, false, 256, 256), false));
 }
 
@@ -1153,7 +1176,7 @@ int hstu_norm_gemm(const HstuNormGemmArgs* a, void* stream) {
   p.depth = p.depth_per_split = a->K;
   p.out[0] = (bf16_t*)a->out;
   p.activation = 1;
-  return a->K == 512 ? launch_rows<512>(p, (hipStream_t)stream) : launch_rows<256>(p, (hipStream_t)stream);
+  return a->K == 512 ? launch_rows<512>(p, false, (hipStream_t)stream) : launch_rows<256>(p, false, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -506,7 +506,7 @@ void gemm(int op, int64_t M, Rows x, std::initializer_list<const Tensor*> ws, in
 
 // d [M, N] w^T for a weight [K, N] in slabs: the package's kernel for contractions of up to 1024 and small products, torch's
 // product (with the slabs put side by side first) for the others.  Microseconds here / there with the concatenation:
-//   N = 512 to 512     74 k rows  56 / 66, 131 k  79 / 77        N = 1024 to 256   74 k  61 / 46, 131 k  73 / 68
+//   N = 512 to 512     74 k rows  55 / 66, 131 k  75 / 77        N = 1024 to 256   74 k  61 / 46, 131 k  73 / 68
 //   N = 1024 to 1024   6.4 k  25 / 19, 19.2 k  59 / 42
 //   N = 2048 to 512    1.6 k  17 / 28, 6.4 k  28 / 27, 19.2 k  50 / 42, 74 k  173 / 185, 131 k  251 / 217
 // The library's product is the faster one at most of these, by how much depends on the rows; it is taken where it may save most of

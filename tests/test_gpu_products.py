@@ -91,6 +91,23 @@ def test_rows_in_registers(gpu, M, N, K, slabs):
   _close(got[0][-300:], torch.nn.functional.silu(got[1][-300:].float()))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (49153, 512, 512),         # a tile of one row at the end; runs that cross tiles
+    (49152, 256, 512),         # whole tiles, six pieces for each workgroup
+    (36705, 512, 704),         # an odd number of pieces in a tile
+])
+def test_rows_in_registers_gradient(gpu, M, N, K):
+  """Large input gradients, whose weights lie along the contraction: the same bits as those of parts of the rows; and against fp32."""
+  g = torch.Generator(device="cuda").manual_seed(M + N)
+  d = torch.randn(M, N + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :N]
+  w = (torch.randn(K, N, device="cuda", generator=g) * N**-0.5).to(torch.bfloat16)
+  got = ops.block_gemm(_lib_block.GEMM_NT, d, [w])
+  for at in range(0, M, 4000):
+    part = slice(at, min(at + 4000, M))
+    assert torch.equal(got[part], ops.block_gemm(_lib_block.GEMM_NT, d[part], [w]))
+  _close(got[-300:], d[-300:].float() @ w.float().t())
+
+
 @pytest.mark.parametrize("M,N,K,slabs", [(32513, 2048, 512, 4), (65281, 1024, 256, 1), (58500, 1152, 512, 2)])
 def test_norm_and_product(gpu, M, N, K, slabs):
   """The layer norm and the product as one launch, with tiles of one row at the end and runs that cross tiles, beside the two launches and
