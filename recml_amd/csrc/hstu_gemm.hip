@@ -804,6 +804,119 @@ __global__ __launch_bounds__(512, 2) void hstu_gemm_rows_kernel(const GemmParams
   HSTU_WAIT_VMCNT(0);        // (no direct load may arrive in LDS that is another workgroup's by then)
 }
 
+// A plain product of a short contraction into wide rows (the head of a narrow model), which takes the time of the output's bytes and the
+// weight's.  A workgroup stays over a run of pieces of (64 rows, 128 columns), columns by columns: the weight's columns are fragments in registers
+// for as long as the run stays in them, a wave's 32 rows of x come one piece ahead, and the only barriers stand where the columns change, so
+// that one wave's stores go beside another's products.  (The tiles of hstu_gemm_kernel each begin with loads and end with stores: 1600 x K ->
+// 20000 took 22 us at K = 8 too, where a fill of that output takes 11.)
+//   1600 x 64 -> 20000 23.3 -> 18.2 us (3.5 TB/s; without the whole lines, see `back`, 20.0), 25600 rows 257 -> 209 (4.9), 400 11.0 -> 10.8,
+// 50 10.6 -> 5.0; 50 x 64 -> 131072 43 -> 8.8, 200 x 64 -> 50000 51 -> 12.7; 1600 x 32 -> 20000 20.7 -> 15.6, x 128 29.9 -> 25.8.
+template <int K, bool PAST>
+__global__ __launch_bounds__(256, K > 64 ? 2 : 4) void hstu_gemm_short_kernel(const GemmParams g) {
+  constexpr int NS = K / 16, W_BYTES = 5 * 64 * K;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[W_BYTES + 4 * 4096];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5, half = w & 1, side = w >> 1;
+  const int steps = g.row_tiles;                         // of 64 rows
+  // Wave pairs take every second row each: rows whose stride is an odd number of half lines (the example's 20000) begin in the middle of a
+  // line by turns, and those are stored from 32 columns further left, so that whole lines are written all the same.
+  const int back = ((((uintptr_t)g.out[0] >> 6) & 1) + side * ((g.out_stride >> 5) & 1)) & 1 && g.out_stride % 32 == 0 ? 1 : 0;
+  const int64_t all = (int64_t)steps * g.col_tiles;
+  const int64_t me = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);     // XCD by XCD
+  const int64_t first = all * me / gridDim.x, last = all * (me + 1) / gridDim.x;
+  if (first >= last) return;
+  int cg = __builtin_amdgcn_readfirstlane((int)(first / steps)), at = __builtin_amdgcn_readfirstlane((int)(first - (int64_t)cg * steps));
+  int todo = __builtin_amdgcn_readfirstlane((int)(last - first));
+
+  // the weight's 128 columns and the 32 to their left as blocks of 32, in rows of 64 bytes (as hstu_gemm_rows_kernel has them)
+  const int gi = lane & 15;
+  const uint32_t at_lane = (uint32_t)((8 * hh + (gi >> 2)) * 64 + 32 * ((lane >> 4) & 1) + 8 * (gi & 3));
+  bf16x8 f[2][NS];
+  auto columns = [&]() __attribute__((always_inline)) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (20 * K + 255) / 256; ++i) {
+      const int piece = 256 * i + tid, block = piece / (4 * K), k = piece / 4 % K, col = 128 * cg - 32 + 32 * block + 8 * (piece & 3);
+      uint4 v = {0, 0, 0, 0};
+      if (piece >= 20 * K) break;
+      if (col >= 0 && col < g.cols) v = *(const uint4*)(g.p[0] + (int64_t)k * g.p_stride + col);
+      *(uint4*)(smem + piece * 16) = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const unsigned char* from = smem + (2 * half + b + 1 - back) * (K * 64) + at_lane + 1024 * s;
+        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(from));
+        const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(from + 256));
+        struct { short4v a, b; } both = {lo, hi};
+        f[b][s] = __builtin_bit_cast(bf16x8, both);
+      }
+  };
+  bf16x8 q[NS];
+  auto load_rows = [&](int step) __attribute__((always_inline)) {
+    int row = 64 * step + 2 * l32 + side;
+    row = row < g.rows ? row : g.rows - 1;              // (what a row past the end gives is not stored)
+    const bf16_t* from = g.q + (int64_t)row * g.q_stride + 8 * hh;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) q[s] = *(const bf16x8*)(from + 16 * s);
+  };
+  // (waited for behind the stores, which are younger: left to their first use in the next round the wait would be for those too)
+  auto rows_here = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(q[s]));
+  };
+
+  // a wave's 32 x 64 results: through its own LDS, as in hstu_gemm_rows_kernel, to whole rows of 128 bytes
+  unsigned char* const own = smem + W_BYTES + w * 4096;
+  const int wslot = (l32 >> 1) & 15;
+  const bool halves = (lane >> 4) & 1;
+  typedef uint32_t words __attribute__((ext_vector_type(4)));
+  const uint32_t out_at = (uint32_t)((lane >> 3) * 2 * (int)g.out_stride + 8 * (lane & 7)) * 2u, out_step = (uint32_t)(16 * (int)g.out_stride) * 2u;
+  const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+  load_rows(at);
+  columns();
+  rows_here();
+  for (; todo > 0; --todo) {
+    floatx16 acc[2] = {zero, zero};
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[b][s], q[s], acc[b], 0, 0, 0);
+    const int m0 = 64 * at + side, n0 = 128 * cg + 64 * half - 32 * back;
+    const bool turn = at + 1 == steps;
+    at = turn ? 0 : at + 1;
+    load_rows(at);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *(uint2*)(own + l32 * 128 + (((8 * b + 2 * q4 + hh) ^ wslot) * 8)) = uint2{pack2(acc[b][4 * q4], acc[b][4 * q4 + 1]), pack2(acc[b][4 * q4 + 2], acc[b][4 * q4 + 3])};
+    __builtin_amdgcn_wave_barrier();
+    // (rows and columns past the output's end lie past the buffer's)
+    const int rows_left = (g.rows - m0 + 1) >> 1;
+    const int64_t bytes = rows_left > 0 ? (((int64_t)(rows_left < 32 ? rows_left : 32) - 1) * 2 * g.out_stride + (g.cols - n0)) * 2 : 0;
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(g.out[0] + (int64_t)m0 * g.out_stride + n0, 0, bytes > 0 ? (int)bytes : 0, 0x00020000);
+    const int col = n0 + 8 * (lane & 7);
+    const bool inside = col >= 0 && col < g.cols;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (lane >> 3) + 8 * i;
+      const words v = *(const words*)(own + row * 128 + (((lane & 7) ^ ((row >> 2) & 7)) * 16));
+      const words o = {halves ? v[2] : v[0], halves ? v[3] : v[1], halves ? v[0] : v[2], halves ? v[1] : v[3]};
+      __builtin_amdgcn_raw_buffer_store_b128(o, to, (int)(inside ? out_at + i * out_step : 0x7ffffff0u), 0, PAST ? 2 : 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+    rows_here();
+    if (turn && todo > 1) {
+      ++cg;
+      columns();
+    }
+  }
+}
+
 // Sums the partial products of a split contraction in the order of the splits and rounds them once.
 __global__ __launch_bounds__(256) void hstu_gemm_reduce(const GemmParams g) {
   const int64_t per = (int64_t)g.rows * g.cols;
@@ -938,6 +1051,27 @@ constexpr int ROWS_GRID = 256;                 // a workgroup per CU
 bool rows_product(const GemmParams& g) {
   return (g.depth == 256 || g.depth == 512) && !g.bias && (!g.c || (!g.activation && !g.pre && g.c_stride < 1 << 20)) && (g.activation || !g.pre) && g.cols % 64 == 0 && g.slab % 32 == 0 &&
          g.out_stride < 1 << 20 && g.p_stride < 1 << 20 && (int64_t)((g.rows + 255) / 256) * (g.cols / 64) >= 6 * ROWS_GRID;
+}
+
+// Whether hstu_gemm_short_kernel takes the product: with rows this wide it does not lose at any number of them (1 to 25600).  Narrower ones
+// change their columns too often or leave too few of them: 800 x 64 -> 10000 10.2 us with it and 10.7 with the tiles, x 128 13.9 and 13.0;
+// 3200 x 64 -> 5008 14.9 and 13.4, 65536 x 64 -> 1024 38 and 35, x 128 52 and 41.  Rows that are no whole half lines are stored in parts of lines
+// here: with few rows alone (250 x 64 -> 16392 8.4 and 9.7, 500 10.5 and 9.9, 25600 362 and 262; 800 x 64 -> 50000 27 and 31).
+bool short_product(const GemmParams& g) {
+  return (g.depth == 32 || g.depth == 64 || g.depth == 128) && !g.bias && !g.c && !g.activation && !g.pre && g.cols >= 16384 && g.slab == g.cols &&
+         (g.out_stride % 32 == 0 || g.rows <= (g.cols >= 32768 ? 1024 : 256)) && g.out_stride < 1 << 20 && g.p_stride < 1 << 20;
+}
+
+template <int K>
+int launch_short(GemmParams g, hipStream_t st) {
+  g.row_tiles = (g.rows + 63) / 64;
+  g.col_tiles = (g.cols + 32 + 127) / 128;              // (rows that are stored from 32 columns further left)
+  const dim3 grid(256 * (K > 64 ? 2 : 4));
+  if (store_past(g.rows, g.cols, g.out_stride)) hipLaunchKernelGGL((hstu_gemm_short_kernel<K, true>), grid, dim3(256), 0, st, g);
+  else hipLaunchKernelGGL((hstu_gemm_short_kernel<K, false>), grid, dim3(256), 0, st, g);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return block_fail(HSTU_BLOCK_ERR_LAUNCH, "gemm kernel launch: %s", hipGetErrorString(e));
+  return HSTU_BLOCK_OK;
 }
 
 template <int K, int OUT, bool NORM = false, bool ALONG = false>
@@ -1134,6 +1268,7 @@ int hstu_gemm(const HstuGemmArgs* a, void* stream) {
     p.out_stride = a->N;
     p.depth = p.depth_per_split = a->K;
     if (rows_product(p)) return p.depth == 512 ? launch_rows<512>(p, false, st) : launch_rows<256>(p, false, st);
+    if (short_product(p)) return p.depth == 128 ? launch_short<128>(p, st) : p.depth == 64 ? launch_short<64>(p, st) : launch_short<32>(p, st);
     return launch_sized<false, true>(p, st, pick_tile(p.rows, p.cols, p.depth, uniform(p, true, 256, 256), p.c != nullptr));
   }
   p.cols = p.out_slab = a->K;

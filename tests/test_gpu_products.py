@@ -108,6 +108,28 @@ def test_rows_in_registers_gradient(gpu, M, N, K):
   _close(got[-300:], d[-300:].float() @ w.float().t())
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1600, 20000, 64),         # a last tile of 32 columns; every second row begins in the middle of a line
+    (900, 20000, 32),
+    (1025, 16384, 64),         # a step of one row; whole tiles
+    (1, 131080, 128),          # one row, a tile of eight columns
+    (256, 16392, 128),         # rows that are no whole sectors
+    (1023, 32776, 64),         # the same, wider, and a step without its last row
+    (2050, 16416, 128),        # a step of two rows
+])
+def test_short_contractions(gpu, M, N, K):
+  """Large products of a short contraction: the same bits as those of parts of the weight's columns, which go by tiles and are summed in
+  the same order; and against fp32."""
+  g = torch.Generator(device="cuda").manual_seed(M + N)
+  x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+  w = (torch.randn(K, N, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+  got = ops.block_gemm(_lib_block.GEMM_NN, x, [w])
+  for rows in (slice(0, 1000), slice(max(M - 1000, 0), M)):
+    for cols in (slice(0, 1024), slice(max(N - 1000, 0), N)):
+      assert torch.equal(got[rows, cols], ops.block_gemm(_lib_block.GEMM_NN, x[rows], [w[:, cols].contiguous()]))
+  _close(got, x.float() @ w.float())
+
+
 @pytest.mark.parametrize("M,N,K,slabs", [(32513, 2048, 512, 4), (65281, 1024, 256, 1), (58500, 1152, 512, 2)])
 def test_norm_and_product(gpu, M, N, K, slabs):
   """The layer norm and the product as one launch, with tiles of one row at the end and runs that cross tiles, beside the two launches and
