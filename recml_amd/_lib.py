@@ -31,6 +31,7 @@ EXPORTS = (
     "hstu_attn_fwd_variant",
     "hstu_attn_bwd",
     "hstu_attn_bwd_silu",
+    "hstu_attn_bwd_workspace_bytes",
     "hstu_attn_bwd_variant",
     "hstu_attn_bucket_thresholds",
     "hstu_attn_dropout_keep",
@@ -121,6 +122,8 @@ def load():
     lib.hstu_attn_bwd.argtypes = [C.POINTER(HstuAttnBwdArgs), C.c_void_p]
     lib.hstu_attn_bwd_silu.restype = C.c_int
     lib.hstu_attn_bwd_silu.argtypes = [C.POINTER(HstuAttnBwdArgs), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.hstu_attn_bwd_workspace_bytes.restype = C.c_size_t
+    lib.hstu_attn_bwd_workspace_bytes.argtypes = [C.POINTER(HstuAttnBwdArgs)]
     lib.hstu_attn_bwd_variant.restype = C.c_char_p
     lib.hstu_attn_bwd_variant.argtypes = [C.POINTER(HstuAttnBwdArgs)]
     lib.hstu_attn_bucket_thresholds.restype = C.c_int

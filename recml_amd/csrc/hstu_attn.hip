@@ -53,6 +53,7 @@
 #include <math.h>
 #include <stdarg.h>
 #include <stdint.h>
+#include <utility>
 #include <stdio.h>
 #include <string.h>
 
@@ -3704,6 +3705,44 @@ __device__ __forceinline__ float both_halves(float v) {
   swap32(v, z);
   return v + z;
 }
+// A block's 16 values of a lane (lane m of each half, offset c = 8g + 4hh + tt in value 4g + tt) summed along its diagonals c - m.
+// Within a row of 16 lanes (p = m % 16, query half qh = m / 16) a shift by c0 % 16, c0 = c - 4hh, brings a register's values onto
+// diagonals 16 k - p + 4hh - 16 qh: k = c0 / 16 for the lanes it keeps, one more for those that come in from the other end, so three sums
+// take all of them, by additions whose operand is shifted on the way (31, where a lane permute per value took 16 of them and as many
+// selects).
+struct DiagSums {
+  float t0 = 0.f, t1 = 0.f, t2 = 0.f;
+  template <int R>
+  __device__ __forceinline__ void add(float v) {
+    constexpr int cp = 8 * ((R >> 2) & 1) + (R & 3);
+    const float keepv = cp == 0 ? v : dpp_f<0x100 + (cp == 0 ? 1 : cp)>(v);
+    const float wrapv = cp == 0 ? 0.f : dpp_f<0x110 + (cp == 0 ? 1 : 16 - cp)>(v);
+    if constexpr (R < 8) { t0 += keepv; if constexpr (cp != 0) t1 += wrapv; }
+    else { t1 += keepv; if constexpr (cp != 0) t2 += wrapv; }
+  }
+  // lane l: diagonal (l & 48) - (l & 15) - 16 of the whole wave
+  __device__ __forceinline__ float total(int lane) {
+    // the upper half's four lanes further on (rows 2 and 3 only): then both halves are on 16 k - p - 16 qh
+    const float w0 = t0, w1 = t1;
+    t0 = dpp_upper<0x104>(t0, w0);
+    t1 = dpp_upper<0x104>(t1, w1) + dpp_upper<0x11c>(0.f, w0);
+    t2 = dpp_upper<0x104>(t2, t2) + dpp_upper<0x11c>(0.f, w1);
+    // the halves' sums; then rows [k = 0, 1, 2, -] of the lower query half in `lo`, of the upper in `up`, which lies one k
+    // further down: diagonal 16 i - 16 - p in row i of the total
+    swap32(t0, t1);
+    float lo = t0 + t1, up = 0.f;
+    swap32(t2, up);
+    up += t2;
+    swap32(lo, up);
+    swap16(lo, up);
+    return up + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane - 16) & 63) << 2, __builtin_bit_cast(int, lo)));
+  }
+};
+template <int R = 0>
+__device__ __forceinline__ void add_diagonals(DiagSums& to, const float (&ds)[16]) {
+  to.add<R>(ds[R]);
+  if constexpr (R < 15) add_diagonals<R + 1>(to, ds);
+}
 // float atomic add on an LDS location given by an ordinary pointer (named as LDS for the compiler: on
 // a pointer of unknown address space it builds a run-time dispatch that some instantiations miscompile)
 typedef __attribute__((address_space(3))) float* lds_float_ptr;
@@ -4184,37 +4223,9 @@ __global__ __launch_bounds__(MFMA_THREADS, DB ? 1 : 2) void hstu_bwd_dq_mfma(con
         if (vals[i] != 0.f) atomicAdd(to, vals[i]);
     }
     if (want_dpos) {
-      // Pair (row m, key offset c = 8g + 4hh + tt) lies on diagonal c - m.  Within a row of 16 lanes (p = m % 16, query half
-      // qh = m / 16) a shift by c0 % 16, c0 = c - 4hh, brings a register's values onto diagonals 16 k - p + 4hh - 16 qh: k = c0 / 16
-      // for the lanes it keeps, one more for those that come in from the other end, so three sums take all of them, by
-      // additions whose operand is shifted on the way (31, where a lane permute per value took 16 of them and as many selects).
-      float t0 = 0.f, t1 = 0.f, t2 = 0.f;
-#define HSTU_DIAG(G, T) { \
-      constexpr int cp = 8 * ((G) & 1) + (T); \
-      const float v = ds[4 * (G) + (T)]; \
-      const float keepv = cp == 0 ? v : dpp_f<0x100 + (cp == 0 ? 1 : cp)>(v); \
-      const float wrapv = cp == 0 ? 0.f : dpp_f<0x110 + (cp == 0 ? 1 : 16 - cp)>(v); \
-      if constexpr ((G) < 2) { t0 += keepv; if constexpr (cp != 0) t1 += wrapv; } \
-      else { t1 += keepv; if constexpr (cp != 0) t2 += wrapv; } }
-      HSTU_DIAG(0, 0) HSTU_DIAG(0, 1) HSTU_DIAG(0, 2) HSTU_DIAG(0, 3)
-      HSTU_DIAG(1, 0) HSTU_DIAG(1, 1) HSTU_DIAG(1, 2) HSTU_DIAG(1, 3)
-      HSTU_DIAG(2, 0) HSTU_DIAG(2, 1) HSTU_DIAG(2, 2) HSTU_DIAG(2, 3)
-      HSTU_DIAG(3, 0) HSTU_DIAG(3, 1) HSTU_DIAG(3, 2) HSTU_DIAG(3, 3)
-#undef HSTU_DIAG
-      // the upper half's four lanes further on (rows 2 and 3 only): then both halves are on 16 k - p - 16 qh
-      const float w0 = t0, w1 = t1;
-      t0 = dpp_upper<0x104>(t0, w0);
-      t1 = dpp_upper<0x104>(t1, w1) + dpp_upper<0x11c>(0.f, w0);
-      t2 = dpp_upper<0x104>(t2, t2) + dpp_upper<0x11c>(0.f, w1);
-      // the halves' sums; then rows [k = 0, 1, 2, -] of the lower query half in `lo`, of the upper in `up`, which lies one k
-      // further down: diagonal 16 i - 16 - p in row i of the total
-      swap32(t0, t1);
-      float lo = t0 + t1, up = 0.f;
-      swap32(t2, up);
-      up += t2;
-      swap32(lo, up);
-      swap16(lo, up);
-      float diag = up + __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane - 16) & 63) << 2, __builtin_bit_cast(int, lo)));
+      DiagSums sums;
+      add_diagonals(sums, ds);
+      float diag = sums.total(lane);
       // lane l: the wave's diagonal 111 + (l & 48) - (l & 15) of this step.  The lower half with the last block's upper one is
       // finished, the upper half waits.
       diag += diag_wait;
@@ -4614,6 +4625,19 @@ __device__ __forceinline__ void mfma_acc(floatx16& acc, bf16x8 a, bf16x8 b) {
   else asm volatile("s_nop 3\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+// dS from the dK/dV kernel to the one that forms dQ from it: blocks of 32 query rows x 32 keys, rounded to bf16 as both kernels' products take
+// them, 2 KB each.  Block (i, j) of a (sequence, head) at slot i (i + 1) / 2 + j under the causal mask, else at i n + j; a sequence's slots
+// begin where `ds_per_row` for each 32 rows before it (an upper bound) end.  Within a block, by halves of 16 rows: 32 keys of 32 bytes, a
+// key's rows in the order 0 .. 3, 8 .. 11, 4 .. 7, 12 .. 15, which is how a lane of the dK/dV kernel holds them.
+constexpr int DS_BLOCK = 32 * 32 * 2;
+__device__ __forceinline__ unsigned char* ds_blocks(const Params& p, int b, int h, const Seq& s) {
+  const int64_t rows = p.jagged ? (s.tok0 >> 5) + b : (int64_t)b * ((p.L + 31) >> 5);
+  return p.ds + (int64_t)h * p.ds_head + rows * p.ds_per_row * DS_BLOCK;
+}
+__device__ __forceinline__ uint32_t ds_block_off(const Params& p, int i, int j) {
+  return (uint32_t)(p.causal ? i * (i + 1) / 2 + j : i * p.ds_per_row + j) * (uint32_t)DS_BLOCK;
+}
+
 // Ring depth of the dK/dV kernel (see there).
 constexpr int dkv_stages(int d, bool dense_bias, bool wide) { return (d == 128 && !dense_bias && !wide) ? 6 : NSTAGE; }
 
@@ -4628,9 +4652,18 @@ struct DkvShape {
   static constexpr int NW = NWAVES * QSPLIT;             // waves per workgroup
   static constexpr int THREADS = 64 * NW;
   static constexpr int KV_BYTES = WIDE ? 2 * BM * D * 2 : 0;   // K and V rows of the tile
+  static constexpr int KV_LDS = KV_BYTES + (WIDE ? 240 : 0);   // and what brings them to a multiple of 256 bytes (from one of 16)
 };
-constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dense_bias) {
-  return d == 128 && !dense_bias && (pos || ts || seg || mask);
+// Table gradients in this kernel (DSO), as in the dQ kernel with keys and queries exchanged: rings of diagonal sums, TG_COPIES sums per
+// bucket.  WIDE: a wave takes every other step, so the diagonals that a block shares with the next one go to the ring at once (the
+// next block is another wave's), and four rings keep the eight waves of a pair of steps apart.
+template <bool WIDE>
+struct DkvTg {
+  static constexpr int RINGS = WIDE ? 4 : 2;
+  static constexpr int FLOATS = RINGS * TG_RING + TG_COPIES * TS_TAB_LEN, BYTES = FLOATS * 4;
+};
+constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dense_bias, bool dso) {
+  return d == 128 && !dense_bias && (pos || ts || seg || mask || dso);
 }
 
 // MSK: the dense keep-mask as in the other backward kernel; here a step's tile is 32 query rows x this workgroup's
@@ -4639,16 +4672,22 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
 // DB: the dense bias likewise, a step's tile of 32 rows x 128 keys (16 KB): wave w fetches rows 8w .. 8w + 7, a lane
 // reads the 16 values of its key's column (consecutive lanes, consecutive words: no swizzle needed).  The bias's
 // gradient is the other kernel's business.
-template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false>
-__global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB)>::THREADS), ((D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB)) || DB ? 1 : 2))
+template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false>
+__global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), ((D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)) || DB ? 1 : 2))
 void hstu_bwd_dkv_mfma(const Params p) {
-  constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB);
+  constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO);
   using SH = DkvShape<D, WIDE>;
   constexpr int NW = SH::NW, THREADS = SH::THREADS;
   constexpr bool ACC_ASM = SH::ACC_ASM;
+  // A block whose vector part stands between the products that do not wait for it: the activation beside dP's, the tables' gradients
+  // beside the accumulating ones.  (B = 64, L = 2048, H = 8, d = 128 with DSO, both backward kernels: both tables 3164 us with neither, 3103
+  // with both, power-law lengths 235 and 225; with the position table alone or none 2370 -> 2360, 2187 -> 2170.  Fragments two products
+  // ahead instead of three: 3156, 228.)
+  constexpr bool WOVEN = WIDE || DSO;
+  constexpr int AHEAD_R = 3, AHEAD_T = 3;      // products that the fragments of rows / of transposed rows are asked for ahead
   // A pair of blocks that needs no mask runs as one hand-scheduled instruction stream (hstu_bwd_stream_d128.inc,
   // written by gen_bwd_stream.py): the vector part of one block behind the matrix instructions of the other.
-  constexpr bool STREAM = D == 128 && !POS && !TS && !SEG && !MSK && !DB;
+  constexpr bool STREAM = D == 128 && !POS && !TS && !SEG && !MSK && !DB && !DSO;
   using SM = MfmaSmem<D, 2>;
   constexpr int CPR = SM::CPR;
   constexpr int QCH = D / 16;
@@ -4682,7 +4721,14 @@ void hstu_bwd_dkv_mfma(const Params p) {
   auto Wc = [&](int st) { return (float*)(smem + BIAS_OFF + st * BIAS_STAGE); };
   auto Tq = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0)); };
   const unsigned char* TsKey = smem + BIAS_OFF + NST * BIAS_STAGE;   // the keyed bucket table of this head
-  unsigned char* const KvLds = smem + BIAS_OFF + NST * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0);   // WIDE: [K | V], 128 rows each, swizzled like the tiles
+  // WIDE: [K | V], 128 rows each, swizzled like the tiles (and on a line of its own: an exclusive or with an address touches bits 4 to 7)
+  constexpr int KV_OFF = (BIAS_OFF + NST * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0) + (WIDE ? 255 : 0)) & (WIDE ? ~255 : ~0);
+  unsigned char* const KvLds = smem + KV_OFF;
+  float* const TgBase = (float*)(KvLds + SH::KV_BYTES);               // DSO with a table: rings of diagonal sums, then the bucket sums
+  static_assert(!DSO || (!MSK && !DB), "the logits' gradients are kept for calls without dense operands");
+  constexpr int RINGS = DkvTg<WIDE>::RINGS;
+  constexpr bool DPOS = DSO && POS, DTS = DSO && TS;
+  const bool want_dpos = DPOS && p.dpos != nullptr, want_dts = DTS && p.dts != nullptr;
 
   Work wk;
   if (!work_of_block(p, blockIdx.x, wk)) return;
@@ -4860,6 +4906,9 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i)
     if (t_lo + i < nt) dma_step(t_lo + i);
+  if (DPOS || DTS) {
+    for (int i = tid; i < DkvTg<WIDE>::FLOATS; i += THREADS) TgBase[i] = 0.f;
+  }
 
   // K and V fragments of this lane's key (B operands); WIDE: the tile's rows in LDS (rows past the sequence repeat its last)
   typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
@@ -4928,6 +4977,22 @@ void hstu_bwd_dkv_mfma(const Params p) {
   const int vc2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
   const int c_lo = vc2 ^ hh, c_hi = vc2 ^ (hh + 2);
 
+  // DSO: this wave's blocks of dS, and (timestamp table) the lane's bucket of the last block with what is summed for it, (position table)
+  // the diagonals that the wave's next block finishes
+  unsigned char* const dsg = DSO ? ds_blocks(p, b, h, s) : nullptr;
+  int sum_bucket = 0;
+  float sum_s = 0.f;
+  float diag_wait = 0.f;
+  int diag_next = 0;
+  const int ring = WIDE ? (qh == 0 ? (w & 1 ? 0 : 1) : (w & 1 ? 2 : (w == 0 ? 0 : 3))) : (w & 1);
+  // (two stores per block and wave, which end_of_pair counts)
+  auto store_ds = [&](int t, const uint4& lo, const uint4& hi) __attribute__((always_inline)) {
+    typedef uint32_t words __attribute__((ext_vector_type(4)));
+    unsigned char* const to = dsg + ds_block_off(p, t, r0 >> 5) + (m * 32 + hh * 16);
+    __builtin_nontemporal_store(words{lo.x, lo.y, lo.z, lo.w}, (words*)to);
+    __builtin_nontemporal_store(words{hi.x, hi.y, hi.z, hi.w}, (words*)(to + DS_BLOCK / 2));
+  };
+
   // One block: 32 query rows against this wave's 32 keys.  Lane (key m, half hh) holds
   // S[q = qbs + 8g + 4hh + tt][kcol], r = 4g + tt.
   auto block = [&](int t) __attribute__((always_inline)) {
@@ -4947,27 +5012,40 @@ void hstu_bwd_dkv_mfma(const Params p) {
       two_buckets = __builtin_amdgcn_ballot_w64(!en.two) == 0;
     }
     floatx16 sacc, dpacc;
-    if constexpr (WIDE) {
-      // Row m of each tile against row 32 w + m of the keys'.  The two chains take turns, and the fragments of a product are
-      // asked for two products ahead (left to itself the compiler has no registers for more than the next one, and every
-      // product waits for LDS): the order is fixed by scheduling barriers.
-      const unsigned char* const qr = (const unsigned char*)Qs(st) + m * (D * 2);
-      const unsigned char* const kr = KvLds + (32 * w + m) * (D * 2);
-      uint4 af[3], bf[3];
-      auto ask = [&](int i) __attribute__((always_inline)) {          // product i: S for even i, dP for odd, channels 16 (i / 2) ..
-        const int at = ((2 * (i >> 1) + hh) ^ gk) * 16;
-        af[i % 3] = *(const uint4*)(qr + at + (i & 1) * SM::K_BYTES);
-        bf[i % 3] = *(const uint4*)(kr + at + (i & 1) * (BM * D * 2));
-      };
-      ask(0);
-      ask(1);
+    // WOVEN: product j, S for j < QCH, then dP; its fragments are asked for two products ahead (left to itself the compiler has no
+    // registers for more than the next one, and every product waits for LDS), the order is fixed by scheduling barriers.  WIDE: row m of
+    // each tile against row 32 w + m of the keys'.
+    uint4 af[WOVEN ? AHEAD_R + 1 : 1], bf[WIDE ? AHEAD_R + 1 : 1];
+    // (Every address is one of two plus a constant after an exclusive or with another, worked out where it is used: what the compiler can
+    // see to be the same in every block it keeps, in registers that the loop does not have.)
+    uint32_t row_at = (uint32_t)(m * (D * 2) + ((hh ^ gk) * 16)), own_at = 0;
+    if constexpr (WOVEN) {
+      asm volatile("" : "+v"(row_at));
+      own_at = row_at + (uint32_t)(KvLds - smem) + (uint32_t)(32 * w * D * 2);
+      row_at += (uint32_t)(st * SM::STAGE);
+    }
+    auto ask_rows = [&](int j) __attribute__((always_inline)) {
+      if (j == QCH) asm volatile("" : "+v"(row_at), "+v"(own_at));
+      const uint32_t x = 32 * (j % QCH);
+      af[j % (AHEAD_R + 1)] = *(const uint4*)(smem + (row_at ^ x) + (j / QCH) * SM::K_BYTES);
+      if constexpr (WIDE) bf[j % (AHEAD_R + 1)] = *(const uint4*)(smem + (own_at ^ x) + (j / QCH) * (BM * D * 2));
+    };
+    auto rows_product = [&](int j, floatx16& d) __attribute__((always_inline)) {
+      uint4 own;
+      if constexpr (WIDE) own = bf[j % (AHEAD_R + 1)];
+      else own = __builtin_bit_cast(uint4, j < QCH ? hs_k[j % QCH] : hs_v[j % QCH]);
+      d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[j % (AHEAD_R + 1)]), __builtin_bit_cast(bf16x8, own), j % QCH == 0 ? zero : d, 0, 0, 0);
+    };
+    if constexpr (WOVEN) {
 #pragma unroll
-      for (int i = 0; i < 2 * QCH; ++i) {
+      for (int j = 0; j < AHEAD_R; ++j) ask_rows(j);
+#pragma unroll
+      for (int j = 0; j < QCH; ++j) {
         __builtin_amdgcn_sched_barrier(0);
-        if (i + 2 < 2 * QCH) ask(i + 2);
-        floatx16& d = (i & 1) ? dpacc : sacc;
-        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i % 3]), __builtin_bit_cast(bf16x8, bf[i % 3]), i < 2 ? zero : d, 0, 0, 0);
+        ask_rows(j + AHEAD_R);
+        rows_product(j, sacc);
       }
+      __builtin_amdgcn_sched_barrier(0);
     } else {
     {
       uint4 af[QCH];
@@ -5015,34 +5093,37 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) u[r] = __builtin_fmaf(bcol[(8 * (r >> 2) + (r & 3)) * 128], LOG2E, u[r]);
     }
+    // (the table gradients, as in the dQ kernel: the lane's 16 pairs are in bucket bk_lane >= 0, those with a bit in
+    // far_rows in the next one, or bkp has the 16 buckets)
+    uint32_t bkp[4] = {0u, 0u, 0u, 0u}, far_rows = 0u;
+    int bk_lane = -1;
+    // row i's logit takes the timestamp of row min(i + 1, last); index into this step's 36
+    auto tq_at = [&](int r) __attribute__((always_inline)) {
+      int iq = qbs + 8 * (r >> 2) + 4 * hh + (r & 3) + 1;
+      iq = iq < s.n_ts - 1 ? iq : s.n_ts - 1;
+      return iq < qbs ? qbs : iq;                 // only for rows past the sequence (masked below)
+    };
+    // a group's rows' timestamps: away from the sequence's end four consecutive words, one further on than an aligned read has them
+    auto times = [&](int g, int (&tqv)[4]) __attribute__((always_inline)) {
+      const int32_t* const tqs = Tq(st);
+      if (qbs + BN < s.n_ts) {
+        const int32_t* const at = tqs + 8 * g + 4 * (lane_again() >> 5);
+        const int4 a = *(const int4*)at;
+        tqv[0] = a.y; tqv[1] = a.z; tqv[2] = a.w;
+        tqv[3] = at[4];
+      } else {
+#pragma unroll
+        for (int t4 = 0; t4 < 4; ++t4) tqv[t4] = tqs[tq_at(4 * g + t4) - qbs];
+      }
+    };
     if (TS) {
-      const int32_t* tqs = Tq(st);
-      // row i's logit takes the timestamp of row min(i + 1, last); index into this step's 36
-      auto tq_at = [&](int r) {
-        int iq = qbs + 8 * (r >> 2) + 4 * hh + (r & 3) + 1;
-        iq = iq < s.n_ts - 1 ? iq : s.n_ts - 1;
-        return iq < qbs ? qbs : iq;                 // only for rows past the sequence (masked below)
-      };
       if (ts32) {
         if (one_bucket) {
           const float add = en.v_near;
 #pragma unroll
           for (int r = 0; r < 16; ++r) u[r] += add;
+          if (DTS) bk_lane = en.b_near;
         } else {
-          // a group's rows' timestamps: away from the sequence's end four consecutive words, one further on than an aligned read
-          // has them
-          const bool inside = qbs + BN < s.n_ts;
-          auto times = [&](int g, int (&tqv)[4]) __attribute__((always_inline)) {
-            if (inside) {
-              const int32_t* const at = tqs + 8 * g + 4 * (lane_again() >> 5);
-              const int4 a = *(const int4*)at;
-              tqv[0] = a.y; tqv[1] = a.z; tqv[2] = a.w;
-              tqv[3] = at[4];
-            } else {
-#pragma unroll
-              for (int t4 = 0; t4 < 4; ++t4) tqv[t4] = tqs[tq_at(4 * g + t4) - qbs];
-            }
-          };
           if (two_buckets) {
             // one bucket boundary at most: the farther bucket exactly when tq - tk >= thr (none of the three is negative)
             const float add_near = en.v_near, add_far = en.v_far;
@@ -5052,7 +5133,40 @@ void hstu_bwd_dkv_mfma(const Params p) {
               int tqv[4];
               times(g, tqv);
 #pragma unroll
-              for (int t4 = 0; t4 < 4; ++t4) u[4 * g + t4] += (uint32_t)tqv[t4] >= cut ? add_far : add_near;
+              for (int t4 = 0; t4 < 4; ++t4) {
+                const bool far = (uint32_t)tqv[t4] >= cut;
+                u[4 * g + t4] += far ? add_far : add_near;
+                if (DTS) far_rows |= far ? 1u << (4 * g + t4) : 0u;
+              }
+            }
+            if (DTS) {
+              bk_lane = en.b_near;
+              far_rows = en.b_far != en.b_near ? far_rows : 0u;       // (a lane whose ends share a bucket flags no row)
+            }
+          } else if (DTS) {
+            // every pair's bucket and value, four at a time (see the dQ kernel)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              int tqv[4];
+              times(g, tqv);
+              float f[4], thr[4];
+              uint32_t bk[4];
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) {
+                f[t4] = __builtin_amdgcn_fmed3f(__builtin_fabsf((float)(tqv[t4] - tk32)), 1.0f, (float)TS_DT_MAX);
+                const uint32_t key = (__builtin_bit_cast(uint32_t, f[t4]) >> 21) - (uint32_t)TS_KEY0;
+                bk[t4] = TsKey[TS_BKT_OFF + key];
+                thr[t4] = *(const float*)(TsKey + (key << 3) + 4);
+              }
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) bk[t4] += f[t4] >= thr[t4] ? 1u : 0u;
+              bkp[g] = bk[0] | (bk[1] << 8) | (bk[2] << 16) | (bk[3] << 24);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) f[t4] = ts_bucket_value(TsKey, (int)bk[t4]);
+              __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+              for (int t4 = 0; t4 < 4; ++t4) u[4 * g + t4] += f[t4];
             }
           } else {
             // every pair looked up.  WIDE: the reads of four under way together (one by one, as the compiler has them for want of
@@ -5073,10 +5187,19 @@ void hstu_bwd_dkv_mfma(const Params p) {
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) u[r] += ts_value(ts_look(TsKey, ts_clip64(tsg[tq_at(r)] - tk)));
+        for (int r = 0; r < 16; ++r) {
+          const int dt = ts_clip64(tsg[tq_at(r)] - tk);
+          if (DTS) {
+            const int bb = ts_bucket_of(TsKey, dt);
+            u[r] += ts_bucket_value(TsKey, bb);
+            bkp[r >> 2] |= (uint32_t)bb << (8 * (r & 3));
+          } else {
+            u[r] += ts_value(ts_look(TsKey, dt));
+          }
+        }
       }
     }
-    // transposed fragments of dO (for dV) and of Q (for dK); WIDE: ahead of their products
+    // transposed fragments of dO (for dV) and of Q (for dK); WOVEN: ahead of their products
     const bf16_t* const orr = Os(st) + vrow * D + 4 * (gi & 1);
     const bf16_t* const qrr = Qs(st) + vrow * D + 4 * (gi & 1);
     auto frag_tr = [&](const bf16_t* rows, int cc, int dvb) __attribute__((always_inline)) {
@@ -5085,8 +5208,8 @@ void hstu_bwd_dkv_mfma(const Params p) {
       const uint2 hi = lds_read_tr(rows + (16 * cc + 8) * D + (cb + c_hi) * 8);
       return uint4{lo.x, lo.y, hi.x, hi.y};
     };
-    uint4 otf[2][WIDE ? 1 : DVB], qtf[2][WIDE ? 1 : DVB];
-    if constexpr (!WIDE) {
+    uint4 otf[2][WOVEN ? 1 : DVB], qtf[2][WOVEN ? 1 : DVB];
+    if constexpr (!WOVEN) {
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
@@ -5096,12 +5219,29 @@ void hstu_bwd_dkv_mfma(const Params p) {
         }
     }
     float pv[16], ds[16];
+    if constexpr (WOVEN) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float fp;
-      const float sg = silu_grad_log2(u[r], &fp);
-      pv[r] = u[r] * sg;
-      ds[r] = dpacc[r] * fp;
+      for (int j = QCH; j < 2 * QCH; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + AHEAD_R < 2 * QCH) ask_rows(j + AHEAD_R);
+        rows_product(j, dpacc);
+#pragma unroll
+        for (int r = (j - QCH) * (16 / QCH); r < (j - QCH + 1) * (16 / QCH); ++r) {
+          const float sg = silu_grad_log2(u[r], &ds[r]);
+          pv[r] = u[r] * sg;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ds[r] = dpacc[r] * ds[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float fp;
+        const float sg = silu_grad_log2(u[r], &fp);
+        pv[r] = u[r] * sg;
+        ds[r] = dpacc[r] * fp;
+      }
     }
     // rows past the sequence hold a repeat of the last row: they are masked like the rest
     if ((p.causal && qbs < r0 + 31) || (qbs + 32 > s.n_q) || (r0 + 32 > s.n_kv) ||
@@ -5147,9 +5287,10 @@ void hstu_bwd_dkv_mfma(const Params p) {
       drop_apply16(pv, ds, drop_bh_key(p.drop_key, (uint32_t)b * (uint32_t)p.H + (uint32_t)h) + (uint32_t)kcol * DROP_CJ +
                                (uint32_t)(qbs + 4 * hh) * DROP_CI, DROP_CI, p.drop_thr);
     }
-    if constexpr (WIDE) {
-      // the accumulating products, dV and dK in turn, their fragments two products ahead
-      uint4 pk[2], dk4[2], tf[3];
+    if constexpr (WOVEN) {
+      // The accumulating products, dV and dK in turn, their fragments two products ahead; between them the tables' gradients: the diagonal
+      // sums in the first half, the bucket sums (a near one and a far one, see the dQ kernel) throughout.
+      uint4 pk[2], dk4[2], tf[AHEAD_T + 1];
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
         pk[cc] = uint4{pack_bf16(pv[8 * cc + 0], pv[8 * cc + 1]), pack_bf16(pv[8 * cc + 2], pv[8 * cc + 3]),
@@ -5157,18 +5298,97 @@ void hstu_bwd_dkv_mfma(const Params p) {
         dk4[cc] = uint4{pack_bf16(ds[8 * cc + 0], ds[8 * cc + 1]), pack_bf16(ds[8 * cc + 2], ds[8 * cc + 3]),
                         pack_bf16(ds[8 * cc + 4], ds[8 * cc + 5]), pack_bf16(ds[8 * cc + 6], ds[8 * cc + 7])};
       }
-      auto ask = [&](int i) __attribute__((always_inline)) { tf[i % 3] = frag_tr((i & 1) ? qrr : orr, i / (2 * DVB), (i >> 1) % DVB); };
-      ask(0);
-      ask(1);
+      float* const slot = TgBase + ring * TG_RING + ((qbs + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_RING - 1));
+      float old = 0.f, diag = 0.f, s_near = 0.f, s_far = 0.f;
+      if (DPOS) old = *slot;
+      DiagSums sums;
+      constexpr int SLOTS = 4 * DVB;
+      uint32_t tr_at = (uint32_t)(vrow * (D * 2) + 8 * (gi & 1) + 64 * swz_rt_group<D>(gi) + 16 * c_lo);
+      asm volatile("" : "+v"(tr_at));
+      tr_at += (uint32_t)(st * SM::STAGE);
+      auto ask = [&](int i) __attribute__((always_inline)) {
+        const unsigned char* const tile = smem + ((i & 1) ? 0 : SM::K_BYTES) + (16 * (i / (2 * DVB))) * (D * 2);
+        const uint32_t x = 64 * ((i >> 1) % DVB);
+        const uint2 lo = lds_read_tr((const bf16_t*)(tile + (tr_at ^ x))), hi = lds_read_tr((const bf16_t*)(tile + 8 * (D * 2) + (tr_at ^ (x ^ 32))));
+        tf[i % (AHEAD_T + 1)] = uint4{lo.x, lo.y, hi.x, hi.y};
+      };
 #pragma unroll
-      for (int i = 0; i < 4 * DVB; ++i) {
+      for (int i = 0; i < (AHEAD_T < SLOTS ? AHEAD_T : SLOTS); ++i) ask(i);
+      auto turn = [&](auto index) __attribute__((always_inline)) {
+        constexpr int i = decltype(index)::value;
         __builtin_amdgcn_sched_barrier(0);
-        if (i + 2 < 4 * DVB) ask(i + 2);
+        if constexpr (i + AHEAD_T < SLOTS) ask(i + AHEAD_T);
         const bf16x8 bb = __builtin_bit_cast(bf16x8, (i & 1) ? dk4[i / (2 * DVB)] : pk[i / (2 * DVB)]);
         floatx16& d = (i & 1) ? dka[(i >> 1) % DVB] : dva[(i >> 1) % DVB];
-        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf[i % 3]), bb, d, 0, 0, 0);
-      }
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf[i % (AHEAD_T + 1)]), bb, d, 0, 0, 0);
+        if constexpr (DPOS) {
+          constexpr int PER = 32 / SLOTS;           // of the 16 values in each of the first SLOTS / 2 turns
+          if constexpr (i < SLOTS / 2) {
+            sums.add<i * PER>(ds[i * PER]);
+            sums.add<i * PER + 1>(ds[i * PER + 1]);
+            if constexpr (PER > 2) {
+              sums.add<i * PER + 2>(ds[i * PER + 2]);
+              sums.add<i * PER + 3>(ds[i * PER + 3]);
+            }
+            if constexpr (PER > 4) {
+              sums.add<i * PER + 4>(ds[i * PER + 4]);
+              sums.add<i * PER + 5>(ds[i * PER + 5]);
+              sums.add<i * PER + 6>(ds[i * PER + 6]);
+              sums.add<i * PER + 7>(ds[i * PER + 7]);
+            }
+          }
+          if constexpr (i == SLOTS / 2) diag = sums.total(lane);
+        }
+        if constexpr (DTS) {
+          constexpr int PER = 16 / SLOTS;
+#pragma unroll
+          for (int r = i * PER; r < (i + 1) * PER; ++r) {
+            const uint32_t far_mask = (uint32_t)((int32_t)(far_rows << (31 - r)) >> 31);       // all ones in the far bucket
+            const uint32_t v = __builtin_bit_cast(uint32_t, ds[r]);
+            s_far += __builtin_bit_cast(float, v & far_mask);
+            s_near += __builtin_bit_cast(float, v & ~far_mask);
+          }
+        }
+      };
+      [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) { (turn(std::integral_constant<int, I>{}), ...); }(std::make_integer_sequence<int, SLOTS>{});
       __builtin_amdgcn_sched_barrier(0);
+      if (DSO) {
+        if (WIDE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        store_ds(t, dk4[0], dk4[1]);
+      }
+      if (want_dpos) {
+        if (WIDE) {
+          *slot = old + diag;
+        } else {
+          diag_next = qbs + BN;
+          diag += diag_wait;
+          diag_wait = 0.f;
+          swap32(diag, diag_wait);
+          if (lane < 32) *slot = old + diag;
+        }
+      }
+      if (want_dts) {
+        float* const hist = TgBase + RINGS * TG_RING + (lane & (TG_COPIES - 1));      // entry TG_COPIES b: bucket b
+        // (what is summed waits in a register until the bucket changes: the buckets of a key rise with the rows)
+        auto add_up = [&](int bucket, float v) __attribute__((always_inline)) {
+          if (sum_bucket != bucket) {
+            if (sum_s != 0.f) lds_atomic_add(&hist[TG_COPIES * sum_bucket], sum_s);
+            sum_bucket = bucket;
+            sum_s = 0.f;
+          }
+          sum_s += v;
+        };
+        if (bk_lane >= 0) {
+          // (the two halves of the wave hold the same keys: one bucket's sum for both, in the lower one)
+          s_near = both_halves(s_near);
+          s_far = both_halves(s_far);
+          add_up(bk_lane, s_near);
+          if (s_far != 0.f) add_up(bk_lane + 1, s_far);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) add_up((int)((bkp[r >> 2] >> (8 * (r & 3))) & 255u), ds[r]);
+        }
+      }
     } else {
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
@@ -5229,22 +5449,50 @@ void hstu_bwd_dkv_mfma(const Params p) {
     if (t + AHEAD + 1 < nt) { dma_step(t + AHEAD + 1); ++n; }
     return n;
   };
-  auto end_of_pair = [&](int n_sent) __attribute__((always_inline)) {
-    if (AHEAD == 2 || n_sent == 0) HSTU_WAIT_VMCNT(0);
+  auto end_of_pair = [&](int n_sent, int n_blocks = 0) __attribute__((always_inline)) {
+    if constexpr (DSO) {
+      // The pair's loads are older than its blocks' stores of dS (two each), which need not be waited for.  (WIDE: a block has waited for
+      // the loads ahead of its stores, a wave without one waits here.  As a branch that the compiler sees, this wait makes it move the
+      // accumulators at the join: 270 spilled registers.)
+      static_assert(AHEAD == 2, "the loads that a pair waits for are all older than its stores");
+      if constexpr (WIDE)
+        asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lwaited%=\n\ts_waitcnt vmcnt(0)\n.Lwaited%=:" ::"s"(__builtin_amdgcn_readfirstlane(n_blocks)) : "scc", "memory");
+      else if (n_blocks == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      else if (n_blocks == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    }
+    else if (AHEAD == 2 || n_sent == 0) HSTU_WAIT_VMCNT(0);
     else if (n_sent == 1) HSTU_WAIT_VMCNT(NDMA);
     else HSTU_WAIT_VMCNT(2 * NDMA);
     __syncthreads();
   };
+  // position-table gradient: the pair before has finished the diagonals up to its second step's (see the dQ kernel)
+  auto flush_diag = [&](int x0) __attribute__((always_inline)) {
+    float* slot = TgBase + ((x0 + lane) & (TG_RING - 1));
+    float val = 0.f;
+#pragma unroll
+    for (int i = 0; i < RINGS; ++i) {
+      val += slot[i * TG_RING];
+      slot[i * TG_RING] = 0.f;
+    }
+    const int idx = (p.L - 1) + kv0 + (BM - 1) - (x0 + lane);
+    if (val != 0.f && idx >= 0 && idx < 2 * p.L - 1)
+      atomicAdd(p.dpos + (int64_t)(p.pos_heads > 1 ? h : 0) * (2 * p.L - 1) + idx, val * p.inv_n);
+  };
   auto block_pair = [&](int t) __attribute__((always_inline)) {
+    if (want_dpos && t > t_lo && w8 == ((t >> 1) & (NW - 1))) flush_diag(32 * (t - 2));
     const int n_sent = send_ahead(t);
     if constexpr (WIDE) {
-      if (t + qh < nt && wave_live && t + qh >= t_wave && t + qh <= t_wave_end) block(t + qh);
-      end_of_pair(n_sent);
+      const bool mine = t + qh < nt && wave_live && t + qh >= t_wave && t + qh <= t_wave_end;
+      if (mine) block(t + qh);
+      end_of_pair(n_sent, mine ? 1 : 0);
       return;
     }
-    if (wave_live && t >= t_wave && t <= t_wave_end) block(t);
-    if (t + 1 < nt && wave_live && t + 1 >= t_wave && t + 1 <= t_wave_end) block(t + 1);
-    end_of_pair(n_sent);
+    const bool first = wave_live && t >= t_wave && t <= t_wave_end;
+    const bool second = t + 1 < nt && wave_live && t + 1 >= t_wave && t + 1 <= t_wave_end;
+    if (first) block(t);
+    if (second) block(t + 1);
+    end_of_pair(n_sent, (first ? 1 : 0) + (second ? 1 : 0));
   };
   HSTU_WAIT_VMCNT(0);
   __syncthreads();
@@ -5261,6 +5509,25 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
   }
   for (; t < nt; t += 2) block_pair(t);
+
+  if (want_dpos && t_lo < nt) {
+    // what waits for a block that does not come, then what the last pair left in the rings
+    if (!WIDE) {
+      if (lane < 32 && diag_wait != 0.f) lds_atomic_add(TgBase + ring * TG_RING + ((diag_next + 111 - 32 * w + (lane & 48) - (lane & 15)) & (TG_RING - 1)), diag_wait);
+      __syncthreads();
+    }
+    if (w8 < 3) flush_diag(32 * (t_lo + ((nt - 1 - t_lo) & ~1)) + 64 * w8);
+  }
+  if (want_dts) {
+    if (sum_s != 0.f) lds_atomic_add(TgBase + RINGS * TG_RING + TG_COPIES * sum_bucket + (lane & (TG_COPIES - 1)), sum_s);
+    __syncthreads();                     // the histogram is complete
+    const float* hist = TgBase + RINGS * TG_RING;
+    for (int e = tid; e < TS_TAB_LEN; e += THREADS) {
+      const float2 two = *(const float2*)(hist + TG_COPIES * e);
+      const float val = two.x + two.y;
+      if (val != 0.f) atomicAdd(p.dts + (int64_t)(p.ts_heads > 1 ? h : 0) * (p.ts_nb + 1) + (e < p.ts_nb ? e : p.ts_nb), val * p.inv_n);
+    }
+  }
 
   const bf16_t* const k_pre = p.k_pre ? (const bf16_t*)p.k_pre + s.bk : nullptr;
   const bf16_t* const v_pre = p.v_pre ? (const bf16_t*)p.v_pre + s.bv : nullptr;
@@ -5297,6 +5564,134 @@ void hstu_bwd_dkv_mfma(const Params p) {
     store_rows<D>(dka, p.alpha * p.inv_n, ot, dkg, k_pre, p.k_st, r0, s.n_kv, s.rows, lane);
     store_rows<D>(dva, p.inv_n * (1.0f / LOG2E), ot, dvg, v_pre, p.v_st, r0, s.n_kv, s.rows, lane);
   }
+}
+
+// dQ from the blocks of dS that the dK/dV kernel left (DSO): the last product of hstu_bwd_dq_mfma with its operand read instead of formed,
+// in the same order, so the same bits.  One workgroup per 128 query rows, 32 per wave; a step's K tile is shared, a wave's block of dS is
+// its own, and both come by direct loads into the ring.
+template <int D>
+struct DqDsShape {
+  static constexpr int K_BYTES = BN * D * 2;
+  static constexpr int STAGE = K_BYTES + NWAVES * DS_BLOCK;
+  static constexpr int LDS = NSTAGE * STAGE;
+};
+template <int D>
+__global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_bwd_dq_ds(const Params p) {
+  using SH = DqDsShape<D>;
+  constexpr int CPR = D / 8;
+  constexpr int DVB = D / 32;
+  constexpr int NPIECE = SH::K_BYTES / 1024;
+  constexpr int LD = NPIECE >= NWAVES ? NPIECE / NWAVES : 1;
+
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  Work wk;
+  if (!work_of_block(p, blockIdx.x, wk)) return;
+  const int b = wk.b, h = wk.h, qt = wk.qt;
+  const Seq& s = wk.s;
+  const int q0 = qt * BM;
+  if (q0 >= s.rows || wk.chunk > 0) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hh = lane >> 5;
+  const char* __restrict__ kg = (const char*)p.k + s.bk * 2;
+  bf16_t* __restrict__ dqg = (bf16_t*)p.dq + s.bq;
+  if (q0 >= s.n_q) {
+    const int rows = (s.rows - q0) < BM ? (s.rows - q0) : BM;
+    const uint4 z = {0u, 0u, 0u, 0u};
+    for (int e = tid; e < rows * (D / 8); e += MFMA_THREADS) {
+      int r = e / (D / 8), c = e - r * (D / 8);
+      *(uint4*)(dqg + (int64_t)(q0 + r) * p.q_st + c * 8) = z;
+    }
+    return;
+  }
+  const int r0 = q0 + 32 * w;
+  const bool wave_live = r0 < s.n_q;
+  const int nt = tile_steps(p, s, q0);
+  // the blocks that a wave's rows have: those that the other kernel has formed (its first and last step for each 32 keys)
+  const int win = p.window;
+  const int t_lo = (win >= 0 && q0 - win > 0) ? (q0 - win) / BN : 0;
+  int wave_last = p.causal ? r0 + 31 : (win >= 0 ? r0 + 31 + win : s.n_kv - 1);
+  wave_last = wave_last < s.n_kv - 1 ? wave_last : s.n_kv - 1;
+  if (!wave_live) wave_last = -1;
+  auto has = [&](int t) __attribute__((always_inline)) { return t < nt && t * BN <= wave_last && (win < 0 || t * BN + 31 + win >= r0); };
+
+  const uint32_t kst_bytes = (uint32_t)p.k_st * 2u;
+  const unsigned char* const dsg = ds_blocks(p, b, h, s);
+  auto dma_step = [&](int t) __attribute__((always_inline)) {
+    unsigned char* const stage = smem + (t % NSTAGE) * SH::STAGE;
+    const int kv0 = t * BN, last = s.n_kv - 1;
+#pragma unroll
+    for (int r = 0; r < LD; ++r) {
+      const int j = (w * LD + r) % NPIECE;
+      const int c = 64 * j + lane;
+      const int row = c / CPR, pc = c - row * CPR;
+      int grow = kv0 + row;
+      grow = grow < last ? grow : last;
+      lds_dma16(kg, (uint32_t)grow * kst_bytes + (uint32_t)((pc ^ swz_rt<D>(row)) * 16), stage + j * 1024);
+    }
+    if (has(t)) {
+      const unsigned char* const from = dsg + ds_block_off(p, r0 >> 5, t);
+      unsigned char* const to = stage + SH::K_BYTES + w * DS_BLOCK;
+      lds_dma16(from, (uint32_t)lane * 16u, to);
+      lds_dma16(from, (uint32_t)lane * 16u + 1024u, to + 1024);
+    }
+  };
+  if (t_lo < nt) dma_step(t_lo);
+  if (t_lo + 1 < nt) dma_step(t_lo + 1);
+
+  floatx16 acc[DVB];
+#pragma unroll
+  for (int i = 0; i < DVB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+  const int gi = lane & 15;
+  const int vrow = 4 * hh + (gi >> 2);
+  const int vc2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
+  const int c_lo = vc2 ^ hh, c_hi = vc2 ^ (hh + 2);
+  // dS: lane i of a group of 16 reads 8 bytes of key row 4hh + i / 4; the middle two of a key's four pieces are exchanged (see ds_block_off)
+  const int piece = (gi & 3) == 1 ? 2 : (gi & 3) == 2 ? 1 : gi & 3;
+  const int ds_at = ((lane >> 4) & 1) * (DS_BLOCK / 2) + vrow * 32 + piece * 8;
+
+  auto block = [&](int t) __attribute__((always_inline)) {
+    const unsigned char* const stage = smem + (t % NSTAGE) * SH::STAGE;
+    const bf16_t* const krt = (const bf16_t*)stage + vrow * D + 4 * (gi & 1);
+    const unsigned char* const dsr = stage + SH::K_BYTES + w * DS_BLOCK + ds_at;
+    uint4 pk[2], tf[3];
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc) {
+      const uint2 lo = lds_read_tr((const bf16_t*)(dsr + (16 * cc) * 32)), hi = lds_read_tr((const bf16_t*)(dsr + (16 * cc + 8) * 32));
+      pk[cc] = uint4{lo.x, lo.y, hi.x, hi.y};
+    }
+    auto ask = [&](int i) __attribute__((always_inline)) {
+      const int cc = i / DVB, cb = 4 * ((i % DVB) ^ swz_rt_group<D>(gi));
+      const uint2 lo = lds_read_tr(krt + (16 * cc) * D + (cb + c_lo) * 8);
+      const uint2 hi = lds_read_tr(krt + (16 * cc + 8) * D + (cb + c_hi) * 8);
+      tf[i % 3] = uint4{lo.x, lo.y, hi.x, hi.y};
+    };
+    ask(0);
+    if (2 * DVB > 1) ask(1);
+#pragma unroll
+    for (int i = 0; i < 2 * DVB; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + 2 < 2 * DVB) ask(i + 2);
+      acc[i % DVB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf[i % 3]), __builtin_bit_cast(bf16x8, pk[i / DVB]),
+                                                             acc[i % DVB], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  HSTU_WAIT_VMCNT(0);
+  __syncthreads();
+  // (five stages and three steps' loads under way at any time: the same 610 us at B = 64, L = 2048, d = 128, 2.2 GB of dS and 0.5 of rows)
+  for (int t = t_lo; t < nt; t += 2) {
+    if (t + 2 < nt) dma_step(t + 2);
+    if (t + 3 < nt) dma_step(t + 3);
+    if (has(t)) block(t);
+    if (has(t + 1)) block(t + 1);
+    HSTU_WAIT_VMCNT(0);
+    __syncthreads();
+  }
+  store_rows<D>(acc, p.alpha * p.inv_n, smem + w * (32 * D * 2), dqg, p.q_pre ? (const bf16_t*)p.q_pre + s.bq : nullptr, p.q_st, r0, s.n_q, s.rows, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -6005,11 +6400,11 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   const int smem = MfmaSmem<D, 2>::total(POS, TS, SEG) + (MSK ? NSTAGE * MfmaSmem<D, 2>::DM_BYTES : 0) +
                    (DB ? NSTAGE * MfmaSmem<D, 2>::DB_BYTES : 0);
   const int smem_q = smem + (TG ? BWD_TG_BYTES : 0);
-  using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB)>;
-  constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB));
+  using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, false)>;
+  constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB, false));
   const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + (MSK ? nst_kv * MfmaSmem<D, 2>::DM_BYTES : 0) +
                       (DB ? nst_kv * MfmaSmem<D, 2>::DB_BYTES : 0) +
-                      SH::KV_BYTES + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
+                      SH::KV_LDS + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
   static int granted_q[64], granted_kv[64];
   if (int rc = allow_lds((const void*)hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>, smem_q, granted_q)) return rc;
   if (int rc = allow_lds((const void*)hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>, smem_kv, granted_kv)) return rc;
@@ -6024,8 +6419,37 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   return HSTU_OK;
 }
 
+// With the logits' gradients kept between them (q.ds): dK/dV, the tables' gradients and dS, then dQ.
+template <int D, bool POS, bool TS, bool SEG>
+int launch_bwd_kept(const Params& p, hipStream_t st) {
+  using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, false, false, true)>;
+  constexpr int nst = dkv_stages(D, false, D == 128);
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + SH::KV_LDS + (TS ? nst * 16 : 0) + (POS || TS ? DkvTg<D == 128>::BYTES : 0);
+  const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, false, false, true>;
+  const auto dq = hstu_bwd_dq_ds<D>;
+  static int granted_q[64], granted_kv[64];
+  if (int rc = allow_lds((const void*)kv, smem_kv, granted_kv)) return rc;
+  if (int rc = allow_lds((const void*)dq, DqDsShape<D>::LDS, granted_q)) return rc;
+  const long long blocks = mfma_grid(p);
+  if (blocks > 0x7fffffffLL) return fail(HSTU_ERR_SHAPE, "grid too large");
+  hipLaunchKernelGGL(kv, dim3((unsigned)blocks), dim3(SH::THREADS), smem_kv, st, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dk/dv kernel launch: %s", hipGetErrorString(e));
+  hipLaunchKernelGGL(dq, dim3((unsigned)blocks), dim3(MFMA_THREADS), DqDsShape<D>::LDS, st, p);
+  e = hipGetLastError();
+  if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dq kernel launch: %s", hipGetErrorString(e));
+  return HSTU_OK;
+}
+
 template <int D, bool SEG>
 int launch_bwd_mfma_ds(const Params& q, hipStream_t st) {
+  if (q.ds) {
+    const bool pos = q.pos_tab != nullptr, ts = q.ts_tab != nullptr;
+    if (pos && ts) return launch_bwd_kept<D, true, true, SEG>(q, st);
+    if (pos) return launch_bwd_kept<D, true, false, SEG>(q, st);
+    if (ts) return launch_bwd_kept<D, false, true, SEG>(q, st);
+    return launch_bwd_kept<D, false, false, SEG>(q, st);
+  }
   const bool pos = q.pos_tab != nullptr, ts = q.ts_tab != nullptr;
   const bool tg = (pos && q.dpos) || (ts && q.dts);
   if (pos && ts) return tg ? launch_bwd_mfma_inst<D, true, true, true, SEG>(q, st) : launch_bwd_mfma_inst<D, true, true, false, SEG>(q, st);
@@ -6070,6 +6494,30 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
   return q.mask_mode == HSTU_MASK_SEGMENT ? launch_bwd_mfma_ds<D, true>(q, st) : launch_bwd_mfma_ds<D, false>(q, st);
 }
 
+// Bytes for the blocks of dS of a matrix-core backward call (see ds_blocks for the layout), 0 where each kernel forms dS for itself.  Kept, S,
+// dP and the activation are computed once instead of twice; what it costs is 2 bytes a pair and head written and read: for d = 128 always
+// less, for shorter rows only while the memory-side cache has them or both tables make the vector part long.  us, formed twice -> kept
+// (tables: none, position, timestamps, both):
+//   d = 128: 64 x 2048 2500 -> 2170, 2640 -> 2360, -, 3540 -> 3103 (2.2 GB of dS); 64 x up to 2048 of power-law length, both 260 -> 225;
+//            128 x 512 position 300 -> 264; 1 x 2048, two heads 154 -> 114; 2 x 4096 both 481 -> 384
+//   d = 64:  128 x up to 1024 (0.43 GB, 0.66 allotted) 413 -> 403, 457 -> 464, 636 -> 624, 758 -> 665; 32 x up to 512, four heads 38 -> 34,
+//            48 -> 43, 81 -> 68, 88 -> 75; 64 x up to 2048 of power-law length (0.31 GB allotted) 116 -> 114, 134 -> 122, 193 -> 168, 207 -> 182
+//   d = 32:  the same three: 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 93 -> 99, 113 -> 111,
+//            173 -> 164, 189 -> 174
+// DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
+constexpr size_t DS_MAX_BYTES = (size_t)4 << 30, DS_CACHED_BYTES = (size_t)512 << 20;
+size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
+  if (a->mask || a->dense_bias || a->L != a->Lkv) return 0;
+  const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
+  const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
+  const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
+  const bool cached = bytes <= (double)DS_CACHED_BYTES;
+  const bool pays = a->d_qk == 128 || (a->d_qk == 64 ? cached || (a->pos_tab && a->ts_tab) : cached && a->ts_tab);
+  if (!pays || bytes > (double)DS_MAX_BYTES) return 0;
+  if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
+  return (size_t)(rows * row * DS_BLOCK) * a->H;
+}
+
 int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   HstuAttnFwdArgs f = b->fwd;
   f.out = (void*)b->dout;
@@ -6083,6 +6531,8 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   q.level_tiles = ws.sched_bytes || (q.causal && (long long)q.B * q.n_qtiles * q.H <= 1024) ? 4 : 0;
   q.no_stream = (b->fwd.flags & HSTU_FWD_COMPILER_SCHEDULED_BLOCKS) ? 1 : 0;
   if (int rc = setup_workspace(&f, ws, q, st)) return rc;
+  const size_t ds = kept_ds_bytes(&f, &q.ds_head, &q.ds_per_row), at = (ws.total() + 255) / 256 * 256;
+  q.ds = ds && f.workspace && ((uintptr_t)f.workspace & 255u) == 0 && f.workspace_bytes >= at + ds ? (unsigned char*)f.workspace + at : nullptr;
   if (q.d_qk == 128) return launch_bwd_mfma_d<128>(q, st);
 #ifndef HSTU_ONLY_D128
   if (q.d_qk == 64) return launch_bwd_mfma_d<64>(q, st);
@@ -6227,6 +6677,27 @@ const char* hstu_attn_fwd_variant(const HstuAttnFwdArgs* args) {
     case V_MFMA_FP8: return "hstu_fwd_mfma_fp8";
     default: return "invalid";
   }
+}
+
+size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args) {
+  HstuAttnBwdArgs own;
+  args = today(args, own);
+  if (!args || args->struct_size != sizeof(HstuAttnBwdArgs) || args->version != HSTU_ATTN_ABI_VERSION) return 0;
+  args = without_bwd_flags(args, own);
+  HstuAttnFwdArgs f = args->fwd;
+  if (!f.out) f.out = (void*)args->dout;
+  if (validate(&f) != HSTU_OK) return 0;
+  const size_t fwd = hstu_attn_fwd_workspace_bytes(&f);
+  HstuAttnBwdArgs b = *args;
+  b.fwd = f;
+  b.fwd.workspace = (void*)256;
+  b.fwd.workspace_bytes = fwd;
+  if (!bwd_mfma_eligible(&b)) return fwd;
+  b.fwd.out = (void*)args->dout;
+  const size_t ds = kept_ds_bytes(&b.fwd, nullptr, nullptr);
+  if (!ds) return fwd;
+  const size_t own_part = (plan_workspace(&b.fwd, false, fwd, false).total() + 255) / 256 * 256;
+  return own_part + ds > fwd ? own_part + ds : fwd;
 }
 
 const char* hstu_attn_bwd_variant(const HstuAttnBwdArgs* args) {

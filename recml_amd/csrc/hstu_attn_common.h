@@ -97,6 +97,11 @@ struct Params {
   float* dts;
   float* dbias;              // gradient of the dense bias, or null
   int32_t dbias_fresh;       // it is written, not added to
+  // The logits' gradients between the two kernels of the matrix-core backward (null: each forms them for itself), see ds_block:
+  // bytes from one head's blocks to the next, and block slots for each 32 rows of queries.
+  unsigned char* ds;
+  int64_t ds_head;
+  int32_t ds_per_row;
   int64_t items_max;         // capacity of the list (sizes the grid)
 };
 

@@ -249,6 +249,21 @@ Tensor scratch_for(HstuAttnFwdArgs& a, const Tensor& like) {
   return buf;
 }
 
+// The backward's: with room for what its kernels can hand on, or without it where the device has not that much left.
+Tensor scratch_for(HstuAttnBwdArgs& b, const Tensor& like) {
+  const size_t ws = hstu_attn_bwd_workspace_bytes(&b);
+  if (!ws) return Tensor();
+  Tensor buf;
+  try {
+    buf = at::empty({(int64_t)ws}, like.options().dtype(at::kByte).requires_grad(false));
+  } catch (const c10::OutOfMemoryError&) {
+    return scratch_for(b.fwd, like);
+  }
+  b.fwd.workspace = buf.data_ptr();
+  b.fwd.workspace_bytes = ws;
+  return buf;
+}
+
 // What the calls on one batch share (recml_amd.hstu_ops.AttentionBatch): the workspace, and what it was prepared for.
 struct Shared {
   std::string prepared, now;   // signatures: of the workspace as it comes, and of this call (empty: do not share)
@@ -363,7 +378,7 @@ struct AttentionBackward : public torch::autograd::Node {
     if (has_mask_rows) rows.mask_rows = mask_rows.unpack();
     if (has_bias_rows) rows.bias_rows = bias_rows.unpack();
     pad_dense(b.fwd, rows, t[0]);
-    const Tensor scratch = scratch_for(b.fwd, t[0]);
+    const Tensor scratch = scratch_for(b, t[0]);
     Tensor g[3];
     gradient_buffers(t, g);
     b.dout = dout.const_data_ptr();
@@ -734,7 +749,7 @@ struct BlockBackward : public torch::autograd::Node {
       b.struct_size = sizeof(b);
       b.version = HSTU_ATTN_ABI_VERSION;
       TORCH_CHECK(fill(b.fwd, q, k, v, d_attn, pt, tt, Tensor(), call.opts), "the block's attention does not fit its own backward");
-      const Tensor scratch = scratch_for(b.fwd, q);
+      const Tensor scratch = scratch_for(b, q);
       b.dout = d_attn.const_data_ptr();
       b.dq = projection_slice(d_uqkv, call, 1).data_ptr();
       b.dk = projection_slice(d_uqkv, call, 2).data_ptr();

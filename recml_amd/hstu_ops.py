@@ -208,7 +208,7 @@ def build_args(q, k, v, out, *, seq_lens=None, seq_offsets=None, max_len=None,
                timestamps=None, ts_bias=None, ts_bucket_size=0.301,
                q_segment_ids=None, kv_segment_ids=None,
                sliding_window_size=None, mask=None, bias=None,
-               q_scale=None, k_scale=None, batch=None, dropout_p=0.0, dropout_seed=0, pad_dense=True):
+               q_scale=None, k_scale=None, batch=None, dropout_p=0.0, dropout_seed=0, pad_dense=True, workspace=True):
   """Validates the call and fills an HstuAttnFwdArgs.  Returns (args, keepalive)."""
   given = (seq_lens, seq_offsets, timestamps, pos_bias, ts_bias, mask)
   for name, t in (("q", q), ("k", k), ("v", v)):
@@ -392,7 +392,8 @@ def build_args(q, k, v, out, *, seq_lens=None, seq_offsets=None, max_len=None,
     _pad_dense(a, keep)
   if q.is_cuda:
     if batch is None:
-      _attach_workspace(a, keep)
+      if workspace:
+        _attach_workspace(a, keep)
     else:
       # everything the preparation reads (the dense mask included: its key-step ranges) or the workspace
       # layout depends on; segment ids (not part of it, but of the choice of kernel) rule the reuse out
@@ -509,7 +510,7 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
       q, k, v, dout, pad_dense=pad, seq_lens=seq_lens, seq_offsets=seq_offsets, max_len=max_len, n=n, alpha=alpha,
       causal=causal, pos_bias=pos_bias, timestamps=timestamps, ts_bias=ts_bias, ts_bucket_size=ts_bucket_size,
       q_segment_ids=q_segment_ids, kv_segment_ids=kv_segment_ids, sliding_window_size=sliding_window_size,
-      mask=mask, bias=bias, dropout_p=dropout_p, dropout_seed=dropout_seed)
+      mask=mask, bias=bias, dropout_p=dropout_p, dropout_seed=dropout_seed, workspace=False)
   # build_args may have made q, k, v contiguous in d: the gradients take the layout it passed on
   qi, ki, vi = _passed_inputs(keep)
   if grads_out is None:
@@ -542,6 +543,14 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
     dbias = torch.empty((fa.B if fa.dense_bias_batched else 1, fa.L, fa.Lkv), dtype=torch.float32, device=q.device)
     ba.ddense_bias = dbias.data_ptr()
   lib = _lib.load()
+  best = lib.hstu_attn_bwd_workspace_bytes(C.byref(ba))
+  if best:
+    try:
+      buf = torch.empty(best, dtype=torch.uint8, device=q.device)
+      ba.fwd.workspace, ba.fwd.workspace_bytes = buf.data_ptr(), best
+      keep.append(buf)
+    except torch.OutOfMemoryError:     # (less than the best will do)
+      _attach_workspace(ba.fwd, keep)
   if _variant_out is not None:
     _variant_out.append(lib.hstu_attn_bwd_variant(C.byref(ba)).decode())
   with torch.cuda.device(q.device):
