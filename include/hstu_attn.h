@@ -318,11 +318,12 @@ int hstu_attn_bwd(const HstuAttnBwdArgs* args, void* stream);
  * "hstu_bwd_mfma_bf16"; others are refused (HSTU_ERR_SHAPE). */
 int hstu_attn_bwd_silu(const HstuAttnBwdArgs* args, const void* q_pre, const void* k_pre, const void* v_pre, void* stream);
 
-/* Bytes of device scratch with which hstu_attn_bwd runs at its best: at least hstu_attn_fwd_workspace_bytes, and for
- * matrix-core calls without dense operands, where it pays, room for the logits' gradients, which the dK/dV kernel then leaves for the one
- * that forms dQ (2 bytes for each pair of a head in blocks of 32 x 32 on and below the diagonal, or in all without the causal mask; up to
- * 4 GiB, and none beyond).  With less, down to hstu_attn_fwd_workspace_bytes, each of the two kernels forms them: the same results up to the
- * rounding and the order of fp32 operations, and the same bits from run to run either way.  From shapes and options only, like the other. */
+/* Bytes of device scratch with which hstu_attn_bwd runs at its best: at least hstu_attn_fwd_workspace_bytes, and where it pays (matrix-core
+ * calls without dense operands; fp32 calls of head dims of 32, 64 and 128) room for the logits' gradients, which the dK/dV kernel then leaves
+ * for the one that forms dQ: 2 bytes (fp32: 4) for each pair of a head in blocks of 32 x 32 (16 x 16) on and below the diagonal, or in all
+ * without the causal mask; up to 4 GiB, and none beyond.  With less, down to hstu_attn_fwd_workspace_bytes, each of the two kernels forms
+ * them: the same results up to the rounding and the order of fp32 operations, and the same bits from run to run either way.  From shapes and
+ * options only, like the other. */
 size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args);
 
 /* Name of the kernel pair hstu_attn_bwd would launch for `args` (diagnostics;

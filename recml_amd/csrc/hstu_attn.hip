@@ -6505,7 +6505,7 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
 //   d = 32:  the same three: 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 93 -> 99, 113 -> 111,
 //            173 -> 164, 189 -> 174
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
-constexpr size_t DS_MAX_BYTES = (size_t)4 << 30, DS_CACHED_BYTES = (size_t)512 << 20;
+constexpr size_t DS_CACHED_BYTES = (size_t)512 << 20;
 size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
   if (a->mask || a->dense_bias || a->L != a->Lkv) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
@@ -6687,7 +6687,12 @@ size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args) {
   HstuAttnFwdArgs f = args->fwd;
   if (!f.out) f.out = (void*)args->dout;
   if (validate(&f) != HSTU_OK) return 0;
-  const size_t fwd = hstu_attn_fwd_workspace_bytes(&f);
+  const size_t fwd = plan_workspace(&f).total();
+  if (f.qk_dtype == HSTU_DTYPE_FP32) {
+    Params p = make_params(&f);
+    p.dout = args->dout; p.dq = args->dq; p.dk = args->dk; p.dv = args->dv;
+    return f32_takes(p, false, true) ? f32_ds_bytes(p, f.total_tokens, nullptr, nullptr) : fwd;
+  }
   HstuAttnBwdArgs b = *args;
   b.fwd = f;
   b.fwd.workspace = (void*)256;
@@ -6759,6 +6764,10 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
     return fail(HSTU_ERR_SHAPE, "the gradient of a timestamp table of more than 4096 entries is not supported, got %d", p.ts_nb + 1);
   if (fresh)
     if (int rc2 = clear_floats(p.dbias, (int64_t)(p.dense_bias_batched ? p.B : 1) * p.L * p.Lkv, st)) return rc2;
+  if (f->qk_dtype == HSTU_DTYPE_FP32 && f->workspace && ((uintptr_t)f->workspace & 255u) == 0 && f32_takes(p, false, true)) {
+    const size_t ds = f32_ds_bytes(p, f->total_tokens, &p.ds_head, &p.ds_per_row);
+    if (ds && f->workspace_bytes >= ds) p.ds = (unsigned char*)f->workspace;
+  }
   return f->qk_dtype == HSTU_DTYPE_FP32 ? launch_bwd<float>(p, st) : launch_bwd<bf16_t>(p, st);
 }
 

@@ -97,8 +97,8 @@ struct Params {
   float* dts;
   float* dbias;              // gradient of the dense bias, or null
   int32_t dbias_fresh;       // it is written, not added to
-  // The logits' gradients between the two kernels of the matrix-core backward (null: each forms them for itself), see ds_block:
-  // bytes from one head's blocks to the next, and block slots for each 32 rows of queries.
+  // The logits' gradients between the two kernels of a backward (null: each forms them for itself), see ds_blocks of either file: bytes
+  // from one head's blocks to the next, and block slots for each 32 (fp32: 16) rows of queries.
   unsigned char* ds;
   int64_t ds_head;
   int32_t ds_per_row;
@@ -208,9 +208,13 @@ __attribute__((visibility("hidden"))) int fail(int code, const char* fmt, ...);
 constexpr int LAW_THR_LEN = 256;
 __attribute__((visibility("hidden"))) int bucket_thresholds(float bucket_size, const int32_t** thr);
 
+// What the logits' gradients that a backward's kernels hand on may take of its workspace.
+constexpr size_t DS_MAX_BYTES = (size_t)4 << 30;
+
 // (hstu_f32.hip) fp32 products at d_qk = d_v in {16, 32, 64, 128} (bf16 storage: 16).  Whether a call is theirs, and the launches.
 __attribute__((visibility("hidden"))) bool f32_takes(const Params& p, bool bf16, bool backward);
 __attribute__((visibility("hidden"))) int f32_launch_fwd(const Params& p, bool bf16, hipStream_t st);
+__attribute__((visibility("hidden"))) size_t f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, int32_t* per_row);
 __attribute__((visibility("hidden"))) int f32_launch_bwd(const Params& p, bool bf16, hipStream_t st);
 
 }  // namespace hstu

@@ -4,6 +4,7 @@
 //   hstu_f32_fwd   64 query rows per workgroup, 16 per wave; keys streamed:  S^T = K Q^T, pointwise, O^T += V^T P^T
 //   hstu_f32_dq    the same rows:  S^T = K Q^T, dP^T = V dO^T, pointwise, dQ^T += K^T dS^T; the gradients of the bias tables
 //                  and of the dense bias
+//   hstu_f32_dq_ds the same from the blocks of dS that hstu_f32_dkv has left:  dQ^T += K^T dS^T
 //   hstu_f32_dkv   64 keys per workgroup, 16 per wave; query rows streamed:  S = Q K^T, dP = dO V^T, pointwise,
 //                  dV^T += dO^T P, dK^T += Q^T dS
 //
@@ -686,6 +687,70 @@ __device__ __forceinline__ void add_diagonals(float* d, const floatx4& x, int m)
   if (m >= 13) lds_add(d + 16, far);
 }
 
+// What a block's dS adds to the gradients of the biases: `diag` is the lane's place among the tile's diagonal sums, dsm LDS for a block of each
+// wave.
+template <bool TAB, bool DEN>
+__device__ __forceinline__ void bias_grads(const Params& p, const TabLds* tl_, float* diag, float* dsm, const floatx4& x, const int (&bucket)[4], bool want_pos,
+                                           bool want_ts, int b, int r0, int c0, int m, int g, int w, int lane) {
+  TabLds* const tl = const_cast<TabLds*>(tl_);
+  if constexpr (TAB) {
+    if (want_pos) add_diagonals(diag, x, m);
+    if (want_ts) {
+      // neighbouring pairs mostly share a bucket: a block with one bucket is summed over the wave first
+      const int b0 = __builtin_amdgcn_readfirstlane(bucket[0]);
+      const bool same = bucket[0] == b0 && bucket[1] == b0 && bucket[2] == b0 && bucket[3] == b0;
+      if (__builtin_amdgcn_ballot_w64(!same) == 0) {
+        float sum = (x[0] + x[1]) + (x[2] + x[3]);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+        if (lane == 0) lds_add(tl->hist + b0, sum);
+      } else {
+        float sum = x[0];
+#pragma unroll
+        for (int r = 1; r < 4; ++r) {
+          if (bucket[r] != bucket[r - 1]) { lds_add(tl->hist + bucket[r - 1], sum); sum = 0.f; }
+          sum += x[r];
+        }
+        lds_add(tl->hist + bucket[3], sum);
+      }
+    }
+  }
+  if constexpr (DEN) {
+    if (p.dbias) {
+      // the block by rows: an instruction then adds four rows of 64 bytes instead of 16 rows of 16
+      float* dw = dsm + w * (16 * 17);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dw[m * 17 + 4 * g + r] = x[r];
+      __builtin_amdgcn_wave_barrier();
+      float* dst = p.dbias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0) + (int64_t)r0 * p.Lkv + c0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = dw[(4 * i + g) * 17 + m];
+        if (v != 0.f) atomicAdd(dst + (int64_t)(4 * i + g) * p.Lkv + m, v);      // (zero wherever the pair is masked or outside)
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+// ... and the workgroup's sums to memory
+template <bool TAB>
+__device__ __forceinline__ void bias_grads_out(const Params& p, const TabArg<TAB>& ta, const TabLds* tl, const float* diag, int n_diag, bool want_pos, bool want_ts,
+                                               int h, int lo, int q0, int tid) {
+  if constexpr (TAB) {
+    if (want_pos || want_ts) {
+      __syncthreads();
+      if (want_pos) {
+        float* dst = p.dpos + (int64_t)(p.pos_heads > 1 ? h : 0) * (2 * p.L - 1);
+        const int base = (p.L - 1) + lo - q0 - (TILE - 1);
+        for (int e = tid; e < n_diag; e += 256)
+          if (diag[e] != 0.f && base + e >= 0 && base + e < 2 * p.L - 1) atomicAdd(dst + base + e, diag[e]);
+      }
+      if (want_ts && tid <= ta.top && tl->hist[tid] != 0.f)
+        atomicAdd(p.dts + (int64_t)(p.ts_heads > 1 ? h : 0) * (p.ts_nb + 1) + tid, tl->hist[tid]);
+    }
+  }
+}
+
 template <typename T, int D, bool TAB, bool DEN>
 __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dq(const Params p, const TabArg<TAB> ta) {
   using S = Shape<D>;
@@ -759,63 +824,128 @@ __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dq(const Param
             x[r] = kept(dp[r] * sg * (1.0f + u * (1.0f - sg)) * p.inv_n, keep, r);
           }
           dot_cols<D>(o, t.tile(buf, 0), 16 * kg, m, g, x);
-          if constexpr (TAB) {
-            if (want_pos) add_diagonals(diag + (c0 - lo) + 4 * g + (TILE - 1) - (WROWS * w + m), x, m);
-            if (want_ts) {
-              // neighbouring pairs mostly share a bucket: a block with one bucket is summed over the wave first
-              const int b0 = __builtin_amdgcn_readfirstlane(bucket[0]);
-              const bool same = bucket[0] == b0 && bucket[1] == b0 && bucket[2] == b0 && bucket[3] == b0;
-              if (__builtin_amdgcn_ballot_w64(!same) == 0) {
-                float sum = (x[0] + x[1]) + (x[2] + x[3]);
-#pragma unroll
-                for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
-                if (lane == 0) lds_add(tl.hist + b0, sum);
-              } else {
-                float sum = x[0];
-#pragma unroll
-                for (int r = 1; r < 4; ++r) {
-                  if (bucket[r] != bucket[r - 1]) { lds_add(tl.hist + bucket[r - 1], sum); sum = 0.f; }
-                  sum += x[r];
-                }
-                lds_add(tl.hist + bucket[3], sum);
-              }
-            }
-          }
-          if constexpr (DEN) {
-            if (p.dbias) {
-              // the block by rows: an instruction then adds four rows of 64 bytes instead of 16 rows of 16
-              float* dw = dsm + w * (16 * 17);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) dw[m * 17 + 4 * g + r] = x[r];
-              __builtin_amdgcn_wave_barrier();
-              float* dst = p.dbias + (p.dense_bias_batched ? (int64_t)b * p.L * p.Lkv : 0) + (int64_t)r0 * p.Lkv + c0;
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const float v = dw[(4 * i + g) * 17 + m];
-                if (v != 0.f) atomicAdd(dst + (int64_t)(4 * i + g) * p.Lkv + m, v);      // (zero wherever the pair is masked or outside)
-              }
-              __builtin_amdgcn_wave_barrier();
-            }
-          }
+          bias_grads<TAB, DEN>(p, tlp, diag + (c0 - lo) + 4 * g + (TILE - 1) - (WROWS * w + m), dsm, x, bucket, want_pos, want_ts, b, r0, c0, m, g, w, lane);
         }
       }
-      if constexpr (TAB) {
-        if (want_pos || want_ts) {
-          __syncthreads();
-          if (want_pos) {
-            float* dst = p.dpos + (int64_t)(p.pos_heads > 1 ? h : 0) * (2 * p.L - 1);
-            const int base = (p.L - 1) + lo - q0 - (TILE - 1);
-            for (int e = tid; e < n_diag; e += 256)
-              if (diag[e] != 0.f && base + e >= 0 && base + e < 2 * p.L - 1) atomicAdd(dst + base + e, diag[e]);
-          }
-          if (want_ts && tid <= ta.top && tl.hist[tid] != 0.f)
-            atomicAdd(p.dts + (int64_t)(p.ts_heads > 1 ? h : 0) * (p.ts_nb + 1) + tid, tl.hist[tid]);
-        }
-      }
+      bias_grads_out<TAB>(p, ta, tlp, diag, n_diag, want_pos, want_ts, h, lo, q0, tid);
     }
   }
   if (qi < s.rows)
     store_row<T, D>((T*)p.dq + s.bq + (int64_t)qi * p.q_st, o, qi < s.n_q ? p.alpha : 0.f, g);
+}
+
+// dS from hstu_f32_dkv to hstu_f32_dq_ds: blocks of 16 keys x 16 query rows, a key's 16 rows next to each other, 1 KB each.  Block (i, j) of a
+// (sequence, head) at slot i (i + 1) / 2 + j where the causal mask meets one length, else at i n + j; a sequence's slots begin where
+// `ds_per_row` for each 16 rows before it (an upper bound) end.  A block without a kept pair is neither written nor read.
+constexpr int DS_BLOCK = 16 * 16;
+__device__ __forceinline__ float* ds_blocks(const Params& p, int b, int h, const Seq& s) {
+  const int64_t rows = p.jagged ? (s.tok0 >> 4) + b : (int64_t)b * ((p.L + 15) >> 4);
+  return (float*)(p.ds + (int64_t)h * p.ds_head) + rows * p.ds_per_row * DS_BLOCK;
+}
+__device__ __forceinline__ int64_t ds_block_at(const Params& p, int i, int j) {
+  return (int64_t)(p.causal && p.L == p.Lkv ? i * (i + 1) / 2 + j : i * p.ds_per_row + j) * DS_BLOCK;
+}
+
+// The rows of hstu_f32_dq with dS read (the bits it would form): one product of three, the bias gradients as there.  Steps of 32 keys: a tile
+// of K alone is half of a step's there.  Bound by that product (B = 128,
+// L = 512, H = 8, d = 128 with segment ids: 290 us where hstu_f32_dq takes 678, and hstu_f32_dkv as long as without its stores) and below
+// d = 128 by the blocks' reads.
+template <int D, bool TAB, bool DEN>
+__global__ __launch_bounds__(256, D >= 128 && (TAB || DEN) ? 3 : 4) void hstu_f32_dq_ds(const Params p, const TabArg<TAB> ta) {
+  using S = Shape<D>;
+  constexpr int KT = 32, TILE_F = KT * D, PPW = KT * S::CPR / 64 / 4;
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  __shared__ typename std::conditional<TAB, TabLds, Nothing>::type tl;
+  __shared__ float dsm[DEN ? 4 * 16 * 17 : 1];
+  float* const diag = sm + 2 * TILE_F;
+  const int h = blockIdx.x, b = blockIdx.y, qt = gridDim.z - 1 - blockIdx.z;
+  const Seq s = seq_info(p, b, h);
+  const int q0 = qt * TILE;
+  if (q0 >= s.rows) return;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = q0 + WROWS * w, qi = r0 + m;
+  floatx4 o[S::NS];
+#pragma unroll
+  for (int x = 0; x < S::NS; ++x) o[x] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (q0 < s.n_q) {
+    int lo, hi;
+    key_range<DEN>(p, s, b, q0, tid, lo, hi);
+    if (lo < hi) {
+      const float* const kg_ = (const float*)p.k + s.bk;
+      auto fetch = [&](int kv0, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PPW; ++i) {
+          const int lin = (w + 4 * i) * 64 + lane, row = lin / S::CPR, c = (lin % S::CPR) ^ S::swz(row);
+          int j = kv0 + row;
+          j = j < s.n_kv ? j : s.n_kv - 1;          // (rows past the end repeat the last one: their pairs are 0)
+          dma16(kg_ + (int64_t)j * p.k_st + 4 * c, (uint32_t)(uintptr_t)(sm + buf * TILE_F + (lin - lane) * 4));
+        }
+      };
+      const float* const dsg = ds_blocks(p, b, h, s) + m;
+      const bool want_ts = TAB && p.dts != nullptr && p.ts_tab != nullptr;
+      const bool want_pos = TAB && p.dpos != nullptr && p.pos_tab != nullptr;
+      const int n_diag = ((hi - lo + 15) & ~15) + TILE;
+      if constexpr (TAB) {
+        if (p.ts_tab) tab_setup(p, ta, tl, h, tid);
+        if (want_pos) for (int e = tid; e < n_diag; e += 256) diag[e] = 0.f;
+      }
+      Pairs<TAB, DEN, true> pairs(p, s, b, h, qi);
+      const TabLds* tlp = nullptr;
+      if constexpr (TAB) tlp = &tl;
+      if constexpr (TAB) pairs.pos_tab = nullptr;      // (which pairs are kept and in which bucket is all that is asked)
+      if constexpr (DEN) pairs.dense = nullptr;
+      struct Block { typename Pairs<TAB, DEN, true>::Raw raw; float x[4]; } next[KT / 16];
+      auto ask = [&](Block& to, int c0) __attribute__((always_inline)) {
+        pairs.load(to.raw, c0, g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to.x[r] = 0.f;
+        if (block_live<true>(p, r0, s.n_q, c0, hi)) {
+          const float* const at = dsg + ds_block_at(p, r0 >> 4, c0 >> 4) + 64 * g;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) to.x[r] = at[16 * r];
+        }
+      };
+      fetch(lo, 0);
+#pragma unroll
+      for (int kg = 0; kg < KT / 16; ++kg) ask(next[kg], lo + 16 * kg);
+      int buf = 0;
+      for (int kv0 = lo; kv0 < hi; kv0 += KT, buf ^= 1) {
+        Block now[KT / 16];
+        dma_wait();
+#pragma unroll
+        for (int kg = 0; kg < KT / 16; ++kg) {
+          next[kg].raw.arrived();
+#pragma unroll
+          for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(next[kg].x[r]));
+          now[kg] = next[kg];
+        }
+        __syncthreads();              // the step's tile is there, and nobody reads the other buffer any more
+        if (kv0 + KT < hi) {
+#pragma unroll
+          for (int kg = 0; kg < KT / 16; ++kg) ask(next[kg], kv0 + KT + 16 * kg);
+          fetch(kv0 + KT, buf ^ 1);
+        }
+#pragma unroll
+        for (int kg = 0; kg < KT / 16; ++kg) {
+          const int c0 = kv0 + 16 * kg;
+          if (!block_live<true>(p, r0, s.n_q, c0, hi)) continue;
+          float bias[4] = {0.f, 0.f, 0.f, 0.f};
+          int bucket[4] = {0, 0, 0, 0};
+          const uint32_t keep = pairs(ta, tlp, now[kg].raw, c0, g, bias, bucket);
+          if (__builtin_amdgcn_ballot_w64(keep != 0u) == 0) continue;
+          floatx4 x;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[r] = now[kg].x[r] * p.inv_n;
+          dot_cols<D>(o, sm + buf * TILE_F, 16 * kg, m, g, x);
+          bias_grads<TAB, DEN>(p, tlp, diag + (c0 - lo) + 4 * g + (TILE - 1) - (WROWS * w + m), dsm, x, bucket, want_pos, want_ts, b, r0, c0, m, g, w, lane);
+        }
+      }
+      bias_grads_out<TAB>(p, ta, tlp, diag, n_diag, want_pos, want_ts, h, lo, q0, tid);
+    }
+  }
+  if (qi < s.rows)
+    store_row<float, D>((float*)p.dq + s.bq + (int64_t)qi * p.q_st, o, qi < s.n_q ? p.alpha : 0.f, g);
 }
 
 template <typename T, int D, bool TAB, bool DEN>
@@ -852,6 +982,7 @@ __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dkv(const Para
         if (p.ts_tab) tab_setup(p, ta, tl, h, tid);
       }
       Pairs<TAB, DEN, false> pairs(p, s, b, h, kj);
+      float* const dsg = sizeof(T) == 4 && p.ds ? ds_blocks(p, b, h, s) + 16 * m + 4 * g : nullptr;
       const TabLds* tlp = nullptr;
       if constexpr (TAB) tlp = &tl;
       typename decltype(pairs)::Raw raw[S::KG], next[S::KG];
@@ -886,6 +1017,7 @@ __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dkv(const Para
             pr[r] = kept(u * sg, keep, r);
             x[r] = kept(dp[r] * sg * (1.0f + u * (1.0f - sg)), keep, r);
           }
+          if (sizeof(T) == 4 && D >= 32 && dsg) __builtin_nontemporal_store(x, (floatx4*)(dsg + ds_block_at(p, c0 >> 4, r0 >> 4)));
           dot_cols<D>(ov, t.tile(buf, 1), 16 * kg, m, g, pr);
           dot_cols<D>(ok, t.tile(buf, 0), 16 * kg, m, g, x);
         }
@@ -940,6 +1072,15 @@ int bwd_inst(const Params& p, hipStream_t st) {
   const bool want_pos = TAB && p.dpos && p.pos_tab;
   const dim3 grid_q(p.H, p.B, (p.L + TILE - 1) / TILE), grid_k(p.H, p.B, (p.Lkv + TILE - 1) / TILE);
   const TabArg<TAB> ta = tab_arg<TAB>(p);
+  if constexpr (sizeof(T) == 4 && D >= 32) {
+    if (p.ds) {
+      hipLaunchKernelGGL((hstu_f32_dkv<T, D, TAB, DEN>), grid_k, dim3(256), smem, st, p, ta);
+      if (int rc = launched("fp32 backward dk/dv kernel")) return rc;
+      const size_t smem_q = sizeof(float) * (2 * 32 * D + (want_pos ? ((p.Lkv + 15) & ~15) + TILE + 32 : 0));
+      hipLaunchKernelGGL((hstu_f32_dq_ds<D, TAB, DEN>), grid_q, dim3(256), smem_q, st, p, ta);
+      return launched("fp32 backward dq kernel");
+    }
+  }
   hipLaunchKernelGGL((hstu_f32_dq<T, D, TAB, DEN>), grid_q, dim3(256), smem + (want_pos ? sizeof(float) * (((p.Lkv + 15) & ~15) + TILE + 32) : 0), st, p, ta);
   if (int rc = launched("fp32 backward dq kernel")) return rc;
   hipLaunchKernelGGL((hstu_f32_dkv<T, D, TAB, DEN>), grid_k, dim3(256), smem, st, p, ta);
@@ -984,6 +1125,21 @@ bool hstu::f32_takes(const Params& p, bool bf16, bool backward) {
   }
   if (p.mask && p.Lkv < 4) return false;
   return p.B <= 65535 && (p.L + TILE - 1) / TILE <= 65535 && (p.Lkv + TILE - 1) / TILE <= 65535;
+}
+// Bytes for the blocks of dS of a backward call (see ds_blocks), 0 where both kernels form them.  Kept, two of the dQ kernel's three products and
+// its activation go, for 4 bytes a pair and head written and read.  us for a backward call, formed twice -> kept:
+//   d = 128: 128 x 512 1490 -> 1191 (segment ids), 2261 -> 1731; 32 x up to 1024 with the position table 1189 -> 868; 32 x 128, four heads
+//            51 -> 41
+//   d = 64:  128 x 512 747 -> 609 (segment ids); 64 x 512 with the table 717 -> 603; 8 x 2048, both tables 1677 -> 1394; 16 x 256 52 -> 42
+//   d = 32:  128 x 512 654 -> 572; 8 x 2048, both tables 1173 -> 999; 16 x 256, four heads 36 -> 32; 32 x 128 and 4 x 64 27 -> 28
+// The last two are as long as their launches and the host's work: the line below leaves such calls (and head dims of 16) alone.
+size_t hstu::f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, int32_t* per_row) {
+  const int64_t nq = (p.L + 15) / 16, nk = (p.Lkv + 15) / 16, rows = p.jagged ? (total_tokens >> 4) + p.B : (int64_t)p.B * nq;
+  const int64_t row = p.causal && p.L == p.Lkv ? (nq + 2) / 2 : nk;        // nq (nq + 1) / 2 blocks by its nq rows
+  const double bytes = (double)rows * (double)row * (4.0 * DS_BLOCK) * p.H;
+  if (p.d_qk < 32 || bytes * p.d_qk < 2e8 || bytes > (double)DS_MAX_BYTES) return 0;
+  if (per_head) { *per_head = rows * row * (4 * DS_BLOCK); *per_row = (int32_t)row; }
+  return (size_t)(rows * row * (4 * DS_BLOCK)) * p.H;
 }
 int hstu::f32_launch_fwd(const Params& p, bool bf16, hipStream_t st) { return launch(p, bf16, false, st); }
 int hstu::f32_launch_bwd(const Params& p, bool bf16, hipStream_t st) { return launch(p, bf16, true, st); }

@@ -1,4 +1,4 @@
-"""The matrix-core backward with the logits' gradients kept between its two kernels against the one that forms them twice: what decides is
+"""The backward with the logits' gradients kept between its two kernels against the one that forms them twice, in bf16 and fp32: what decides is
 the workspace that the caller brings, and both give the same bits (but for fp32 sums that are taken in another order)."""
 
 import ctypes as C
@@ -11,14 +11,13 @@ import recml_amd
 from recml_amd import _lib
 
 pytestmark = pytest.mark.gpu
-BF = torch.bfloat16
 
 
-def _case(d, L, H, lens, *, jagged, pos, ts, seg, B):
+def _case(dtype, d, L, H, lens, *, jagged, pos, ts, seg, B):
   g = torch.Generator(device="cuda").manual_seed(d + L)
   n = np.array(lens if lens is not None else [L] * B, np.int32)
   shape = (int(n.sum()), H, d) if jagged else (B, L, H, d)
-  q, k, v, do = (torch.randn(shape, device="cuda", generator=g).mul_(0.5).to(BF) for _ in range(4))
+  q, k, v, do = (torch.randn(shape, device="cuda", generator=g).mul_(0.5).to(dtype) for _ in range(4))
   kw = {}
   if jagged:
     kw.update(seq_offsets=torch.from_numpy(np.concatenate([[0], np.cumsum(n)]).astype(np.int32)).cuda(), max_len=L)
@@ -35,7 +34,7 @@ def _case(d, L, H, lens, *, jagged, pos, ts, seg, B):
   return q, k, v, do, kw
 
 
-@pytest.mark.parametrize("d,B,L,H,lens,opt", [
+_FORMS = [
     (128, 2, 256, 8, None, {}),                                                             # whole tiles; the other side: the stream
     (128, 5, 420, 2, [420, 129, 33, 1, 256], dict(jagged=1, pos=1, ts=1)),
     (128, 5, 420, 4, [0, 420, 31, 32, 97], dict(pos=1)),                                    # a sequence without a token, block edges
@@ -49,11 +48,17 @@ def _case(d, L, H, lens, *, jagged, pos, ts, seg, B):
     (64, 3, 260, 2, None, dict(seg=1)),
     (32, 5, 420, 2, [420, 129, 33, 1, 256], dict(jagged=1, ts=1)),
     (32, 2, 333, 1, None, dict(pos=1, ts=1, sliding_window_size=50)),
-])
-def test_kept_and_formed_twice_agree(gpu, monkeypatch, d, B, L, H, lens, opt):
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,B,L,H,lens,opt", _FORMS)
+def test_kept_and_formed_twice_agree(gpu, monkeypatch, dtype, d, B, L, H, lens, opt):
+  if dtype == torch.float32:
+    H *= 16          # (small fp32 calls keep nothing)
   opt = dict(opt)
   form = {x: opt.pop(x, 0) for x in ("jagged", "pos", "ts", "seg")}
-  q, k, v, do, kw = _case(d, L, H, lens, B=B, **form)
+  q, k, v, do, kw = _case(dtype, d, L, H, lens, B=B, **form)
   kw.update(opt)
   lib = _lib.load()
   best, least = [], []
@@ -75,7 +80,7 @@ def test_kept_and_formed_twice_agree(gpu, monkeypatch, d, B, L, H, lens, opt):
   assert best[0] > least[0] + 4096
   for name, x, y, z in zip(("dq", "dk", "dv"), a, b, again):
     assert torch.equal(x, z), name
-    if (name == "dq" and form["ts"] and not form["pos"]) or (name != "dq" and d == 128 and not (form["pos"] or form["ts"] or form["seg"])):
+    if dtype == torch.bfloat16 and ((name == "dq" and form["ts"] and not form["pos"]) or (name != "dq" and d == 128 and not (form["pos"] or form["ts"] or form["seg"]))):
       # dq: a logit and its timestamp bias added with one rounding or two, which turns a bf16 rounding of dS now and then; dk, dv: fp32 sums in
       # two halves or in one.  Either shows as a last bit of single elements: far below the rounding of all of them, 2^-9 of the norm.
       assert float((x.float() - y.float()).norm()) <= 2.0 ** -9 * float(y.float().norm()), name
@@ -87,3 +92,30 @@ def test_kept_and_formed_twice_agree(gpu, monkeypatch, d, B, L, H, lens, opt):
     assert (x is None) == (y is None), name
     if x is not None:
       assert float((x - y).abs().max()) <= 1e-4 * float(y.abs().max()), name
+
+
+@pytest.mark.parametrize("d", [128, 64, 32])
+@pytest.mark.parametrize("B,L,Lkv,bias", [(2, 200, 200, True), (2, 77, 77, False), (3, 50, 130, True), (2, 130, 50, False)])
+def test_fp32_with_dense_operands(gpu, monkeypatch, d, B, L, Lkv, bias):
+  """A mask and a dense bias, keys and queries of different lengths: blocks without a kept pair are neither written nor read."""
+  g = torch.Generator(device="cuda").manual_seed(d + L)
+  H = 160
+  q, do = (torch.randn(B, L, H, d, device="cuda", generator=g) * 0.5 for _ in range(2))
+  k, v = (torch.randn(B, Lkv, H, d, device="cuda", generator=g) * 0.5 for _ in range(2))
+  mask = torch.rand(B, L, Lkv, device="cuda", generator=g) < 0.3
+  mask[:, 16:48] = False
+  mask[:, :, 16:32] = False
+  kw = dict(mask=mask, causal=False, n=float(L))
+  if bias:
+    kw.update(bias=torch.randn(B, L, Lkv, device="cuda", generator=g) * 0.3, bias_grad=True)
+  lib = _lib.load()
+  whole, best = lib.hstu_attn_bwd_workspace_bytes, []
+  monkeypatch.setattr(lib, "hstu_attn_bwd_workspace_bytes", lambda args: best.append(whole(args)) or best[-1])
+  a = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  assert best[0] > 0
+  monkeypatch.setattr(lib, "hstu_attn_bwd_workspace_bytes", lambda args: 0)
+  b = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  for x, y in zip(a[:3], b[:3]):
+    assert torch.equal(x, y)
+  if bias:      # (the heads' terms added by atomics in any order: H - 1 roundings of at most the terms' magnitudes' sum on either side)
+    assert float((a[5] - b[5]).abs().max()) <= 2 * H * 2.0 ** -24 * H * float(a[5].abs().max())
