@@ -6500,18 +6500,22 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
 // (tables: none, position, timestamps, both):
 //   d = 128: 64 x 2048 2500 -> 2170, 2640 -> 2360, -, 3540 -> 3103 (2.2 GB of dS); 64 x up to 2048 of power-law length, both 260 -> 225;
 //            128 x 512 position 300 -> 264; 1 x 2048, two heads 154 -> 114; 2 x 4096 both 481 -> 384
-//   d = 64:  128 x up to 1024 (0.43 GB, 0.66 allotted) 413 -> 403, 457 -> 464, 636 -> 624, 758 -> 665; 32 x up to 512, four heads 38 -> 34,
-//            48 -> 43, 81 -> 68, 88 -> 75; 64 x up to 2048 of power-law length (0.31 GB allotted) 116 -> 114, 134 -> 122, 193 -> 168, 207 -> 182
-//   d = 32:  the same three: 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 93 -> 99, 113 -> 111,
-//            173 -> 164, 189 -> 174
+//   d = 64:  128 x up to 1024 (0.43 GB) 413 -> 403, 457 -> 464, 636 -> 624, 758 -> 665; half as many (0.21 GB) 170 -> 184, 207 -> 218; a
+//            quarter, position 123 -> 116; 32 x up to 512, four heads 38 -> 34, 48 -> 43, 81 -> 68, 88 -> 75; 64 x up to 2048 of power-law
+//            length (0.09 GB) 104 -> 109 and 116 -> 114, 134 -> 122, 193 -> 168, 207 -> 182
+//   d = 32:  128 x up to 1024 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 x up to 512 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 64 x up to
+//            2048 93 -> 99, 113 -> 111, 173 -> 164, 189 -> 174
+// The lengths stay on the device: a batch's bytes are taken to be those of equal lengths (of power-law ones 0.04 of the 0.09 GB above).
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
-constexpr size_t DS_CACHED_BYTES = (size_t)512 << 20;
+constexpr size_t DS_CACHED_BYTES = (size_t)128 << 20;
 size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
   if (a->mask || a->dense_bias || a->L != a->Lkv) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
   const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
   const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
-  const bool cached = bytes <= (double)DS_CACHED_BYTES;
+  const int64_t n = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens / (a->B > 0 ? a->B : 1) + 31) / 32 : nb;
+  const double likely = (double)a->B * a->H * DS_BLOCK * (a->causal ? n * (n + 1) / 2 : n * n);
+  const bool cached = likely <= (double)(a->pos_tab || a->ts_tab ? DS_CACHED_BYTES : DS_CACHED_BYTES / 4);
   const bool pays = a->d_qk == 128 || (a->d_qk == 64 ? cached || (a->pos_tab && a->ts_tab) : cached && a->ts_tab);
   if (!pays || bytes > (double)DS_MAX_BYTES) return 0;
   if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
