@@ -4684,7 +4684,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
   // with both, power-law lengths 235 and 225; with the position table alone or none 2370 -> 2360, 2187 -> 2170.  Fragments two products
   // ahead instead of three: 3156, 228.)
   constexpr bool WOVEN = WIDE || DSO;
-  constexpr int AHEAD_R = 3, AHEAD_T = 3;      // products that the fragments of rows / of transposed rows are asked for ahead
+  constexpr int AHEAD_R = D / 16 < 3 ? D / 16 : 3, AHEAD_T = 3;      // products that the fragments of rows / of transposed rows are asked for ahead
   // A pair of blocks that needs no mask runs as one hand-scheduled instruction stream (hstu_bwd_stream_d128.inc,
   // written by gen_bwd_stream.py): the vector part of one block behind the matrix instructions of the other.
   constexpr bool STREAM = D == 128 && !POS && !TS && !SEG && !MSK && !DB && !DSO;
@@ -4725,7 +4725,6 @@ void hstu_bwd_dkv_mfma(const Params p) {
   constexpr int KV_OFF = (BIAS_OFF + NST * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0) + (WIDE ? 255 : 0)) & (WIDE ? ~255 : ~0);
   unsigned char* const KvLds = smem + KV_OFF;
   float* const TgBase = (float*)(KvLds + SH::KV_BYTES);               // DSO with a table: rings of diagonal sums, then the bucket sums
-  static_assert(!DSO || (!MSK && !DB), "the logits' gradients are kept for calls without dense operands");
   constexpr int RINGS = DkvTg<WIDE>::RINGS;
   constexpr bool DPOS = DSO && POS, DTS = DSO && TS;
   const bool want_dpos = DPOS && p.dpos != nullptr, want_dts = DTS && p.dts != nullptr;
@@ -5575,7 +5574,8 @@ struct DqDsShape {
   static constexpr int STAGE = K_BYTES + NWAVES * DS_BLOCK;
   static constexpr int LDS = NSTAGE * STAGE;
 };
-template <int D>
+// MSK: the blocks are those of the steps that the other kernel found in the mask's presence table; of them, those in which it keeps a pair.
+template <int D, bool MSK>
 __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_bwd_dq_ds(const Params p) {
   using SH = DqDsShape<D>;
   constexpr int CPR = D / 8;
@@ -5607,14 +5607,40 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_bwd_dq_ds(const Params p
   }
   const int r0 = q0 + 32 * w;
   const bool wave_live = r0 < s.n_q;
-  const int nt = tile_steps(p, s, q0);
+  int nt = tile_steps(p, s, q0);
   // the blocks that a wave's rows have: those that the other kernel has formed (its first and last step for each 32 keys)
   const int win = p.window;
-  const int t_lo = (win >= 0 && q0 - win > 0) ? (q0 - win) / BN : 0;
+  int t_lo = (win >= 0 && q0 - win > 0) ? (q0 - win) / BN : 0;
+  if (MSK) {
+    const int2 mr = ((const int2*)p.mask_range)[(p.mask_batched ? b : 0) * p.n_qtiles + qt];
+    t_lo = t_lo > mr.x ? t_lo : mr.x;
+    nt = nt < mr.y ? nt : mr.y;
+    nt = nt > t_lo ? nt : t_lo;
+  }
   int wave_last = p.causal ? r0 + 31 : (win >= 0 ? r0 + 31 + win : s.n_kv - 1);
   wave_last = wave_last < s.n_kv - 1 ? wave_last : s.n_kv - 1;
   if (!wave_live) wave_last = -1;
-  auto has = [&](int t) __attribute__((always_inline)) { return t < nt && t * BN <= wave_last && (win < 0 || t * BN + 31 + win >= r0); };
+  // MSK: a bit for each key tile with a pair that the wave's rows keep
+  static_assert(MASK_PRES_MAX_KT == 256, "four words of a bit for each key tile");
+  uint64_t kept0 = 0, kept1 = 0, kept2 = 0, kept3 = 0;
+  if (MSK) {
+    const int n_kt = (p.Lkv + BM - 1) / BM;
+    const uint8_t* const pres = mask_presence(p) + ((int64_t)(p.mask_batched ? b : 0) * p.n_qtiles + qt) * n_kt;
+    auto word = [&](int c) __attribute__((always_inline)) {
+      const int kt = 64 * c + lane;
+      return __builtin_amdgcn_ballot_w64(kt < n_kt && ((pres[kt < n_kt ? kt : 0] >> w) & 1));
+    };
+    kept0 = word(0);
+    if (n_kt > 64) { kept1 = word(1); kept2 = word(2); kept3 = word(3); }
+  }
+  auto has = [&](int t) __attribute__((always_inline)) {
+    if (MSK) {
+      const int c = t >> 8;
+      const uint64_t k = c == 0 ? kept0 : c == 1 ? kept1 : c == 2 ? kept2 : kept3;
+      if (!((k >> ((t >> 2) & 63)) & 1)) return false;
+    }
+    return t < nt && t * BN <= wave_last && (win < 0 || t * BN + 31 + win >= r0);
+  };
 
   const uint32_t kst_bytes = (uint32_t)p.k_st * 2u;
   const unsigned char* const dsg = ds_blocks(p, b, h, s);
@@ -6420,13 +6446,15 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
 }
 
 // With the logits' gradients kept between them (q.ds): dK/dV, the tables' gradients and dS, then dQ.
-template <int D, bool POS, bool TS, bool SEG>
+template <int D, bool POS, bool TS, bool SEG, bool MSK = false, bool DB = false>
 int launch_bwd_kept(const Params& p, hipStream_t st) {
-  using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, false, false, true)>;
-  constexpr int nst = dkv_stages(D, false, D == 128);
-  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + SH::KV_LDS + (TS ? nst * 16 : 0) + (POS || TS ? DkvTg<D == 128>::BYTES : 0);
-  const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, false, false, true>;
-  const auto dq = hstu_bwd_dq_ds<D>;
+  constexpr bool wide = dkv_wide(D, POS, TS, SEG, MSK, DB, true);
+  using SH = DkvShape<D, wide>;
+  constexpr int nst = dkv_stages(D, DB, wide);
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + (MSK ? nst * MfmaSmem<D, 2>::DM_BYTES : 0) + (DB ? nst * MfmaSmem<D, 2>::DB_BYTES : 0) +
+                      SH::KV_LDS + (TS ? nst * 16 : 0) + (POS || TS ? DkvTg<wide>::BYTES : 0);
+  const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, true>;
+  const auto dq = hstu_bwd_dq_ds<D, MSK>;
   static int granted_q[64], granted_kv[64];
   if (int rc = allow_lds((const void*)kv, smem_kv, granted_kv)) return rc;
   if (int rc = allow_lds((const void*)dq, DqDsShape<D>::LDS, granted_q)) return rc;
@@ -6458,13 +6486,15 @@ int launch_bwd_mfma_ds(const Params& q, hipStream_t st) {
   return launch_bwd_mfma_inst<D, false, false, false, SEG>(q, st);
 }
 
-// Whether the dense bias's gradient is a kernel of its own: for long rows, and matrices enough for a round of its workgroups; elsewhere the
-// additions of the dQ kernel are few and its second run over the heads is the longer way.  us for a backward call with / without, d = 64:
-// eight heads, 16 x up to 1000 319 / 434, 8 x 700 126 / 145, 1 x 2000 424 / 471 (4 x 700 117 / 123, 16 x 300 92 / 91, 64 x 256 155 / 149,
-// 32 x 256 89 / 83); two heads, 16 x 1000 142 / 155, 8 x 700 89 / 89; one, 16 x 2048 325 / 354, 16 x 1000 142 / 144.  d = 128, eight heads:
-// 16 x 2048, full, 1425 / 1626, 16 x 1000 400 / 480, 8 x 700 155 / 155.
+// Whether the dense bias's gradient is a kernel of its own: where its workgroups, which go through the heads, come to a round of the chip for
+// every eight heads or so; elsewhere the additions of the dQ kernel are few and its second run over the heads is the longer way.  (A call
+// whose gradient is apart also has its dS handed on, see kept_ds_bytes.)  us for a backward call, added by the dQ kernel / apart:
+//   eight heads, d = 64:  32 x up to 256 76 / 67, 64 x 256 124 / 107, 16 x 300 75 / 65, 4 x 700 66 / 68, 16 x 150 57 / 58; d = 32: 16 x 300
+//                         68 / 58, 8 x 512 70 / 63; d = 128: 8 x 512 89 / 86, 64 x 256 147 / 137, 4 x 300 55 / 64
+//   two heads, d = 64:    16 x up to 256 43 / 40, 8 x 700 84 / 71; one head 8 x 512 67 / 52, 16 x 1000 133 / 109
 bool dbias_apart(const Params& p) {
-  return p.dbias && p.dense_bias && (p.dense_bias_batched || p.B == 1) && p.L >= 512 && (int64_t)p.B * p.L * p.Lkv >= 3000000;
+  const int64_t tiles = (int64_t)p.B * p.n_qtiles * ((p.Lkv + 63) / 64);
+  return p.dbias && p.dense_bias && (p.dense_bias_batched || p.B == 1) && tiles >= 64 && tiles >= 28LL * p.H;
 }
 
 template <int D>
@@ -6488,6 +6518,11 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
     if (int rc = launch_dbias<D>(q, st)) return rc;
     q.dbias = nullptr;
   }
+  if (q.ds && !q.dbias) {
+    if (q.mask && q.dense_bias) return launch_bwd_kept<D, false, false, false, true, true>(q, st);
+    if (q.dense_bias) return launch_bwd_kept<D, false, false, false, false, true>(q, st);
+    if (q.mask) return launch_bwd_kept<D, false, false, false, true>(q, st);
+  }
   if (q.mask && q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, true, true>(q, st);
   if (q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, false, true>(q, st);
   if (q.mask) return launch_bwd_mfma_inst<D, false, false, false, false, true>(q, st);
@@ -6505,18 +6540,21 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
 //            length (0.09 GB) 104 -> 109 and 116 -> 114, 134 -> 122, 193 -> 168, 207 -> 182
 //   d = 32:  128 x up to 1024 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 x up to 512 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 64 x up to
 //            2048 93 -> 99, 113 -> 111, 173 -> 164, 189 -> 174
+// and with dense operands, which both kernels read, at every head dim (mask and bias, mask alone; eight heads, the bias's gradient left out):
+//   d = 128: 16 x up to 1000 310 -> 257, 206 -> 200; d = 64: 243 -> 173, 151 -> 132; d = 32: 214 -> 152, 120 -> 104; 16 x 2048, full, with the
+//            gradient 1422 -> 1282 and 1080 -> 907
 // The lengths stay on the device: a batch's bytes are taken to be those of equal lengths (of power-law ones 0.04 of the 0.09 GB above).
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
 constexpr size_t DS_CACHED_BYTES = (size_t)128 << 20;
 size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
-  if (a->mask || a->dense_bias || a->L != a->Lkv) return 0;
+  if (a->L != a->Lkv || (a->mask && (a->Lkv + BM - 1) / BM > MASK_PRES_MAX_KT)) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
   const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
   const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
   const int64_t n = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens / (a->B > 0 ? a->B : 1) + 31) / 32 : nb;
   const double likely = (double)a->B * a->H * DS_BLOCK * (a->causal ? n * (n + 1) / 2 : n * n);
   const bool cached = likely <= (double)(a->pos_tab || a->ts_tab ? DS_CACHED_BYTES : DS_CACHED_BYTES / 4);
-  const bool pays = a->d_qk == 128 || (a->d_qk == 64 ? cached || (a->pos_tab && a->ts_tab) : cached && a->ts_tab);
+  const bool pays = a->d_qk == 128 || (a->d_qk == 64 ? cached || a->dense_bias || a->mask || (a->pos_tab && a->ts_tab) : a->dense_bias || a->mask || (cached && a->ts_tab));
   if (!pays || bytes > (double)DS_MAX_BYTES) return 0;
   if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
   return (size_t)(rows * row * DS_BLOCK) * a->H;
@@ -6705,6 +6743,11 @@ size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args) {
   b.fwd.out = (void*)args->dout;
   const size_t ds = kept_ds_bytes(&b.fwd, nullptr, nullptr);
   if (!ds) return fwd;
+  if (args->ddense_bias) {               // (added by the dQ kernel: that one forms dS)
+    Params p = make_params(&b.fwd);
+    p.dbias = args->ddense_bias;
+    if (!dbias_apart(p)) return fwd;
+  }
   const size_t own_part = (plan_workspace(&b.fwd, false, fwd, false).total() + 255) / 256 * 256;
   return own_part + ds > fwd ? own_part + ds : fwd;
 }

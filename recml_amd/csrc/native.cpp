@@ -378,7 +378,6 @@ struct AttentionBackward : public torch::autograd::Node {
     if (has_mask_rows) rows.mask_rows = mask_rows.unpack();
     if (has_bias_rows) rows.bias_rows = bias_rows.unpack();
     pad_dense(b.fwd, rows, t[0]);
-    const Tensor scratch = scratch_for(b, t[0]);
     Tensor g[3];
     gradient_buffers(t, g);
     b.dout = dout.const_data_ptr();
@@ -403,6 +402,7 @@ struct AttentionBackward : public torch::autograd::Node {
       b.ddense_bias = dbias.data_ptr<float>();
       b.fwd.flags |= HSTU_BWD_WRITE_BIAS_GRADIENT;
     }
+    const Tensor scratch = scratch_for(b, t[0]);
     const int rc = hstu_attn_bwd(&b, stream_of(t[0]));
     TORCH_CHECK(rc == HSTU_OK, "hstu_attn_bwd failed (", rc, "): ", hstu_attn_last_error());
     for (int i = 0; i < 3; ++i)

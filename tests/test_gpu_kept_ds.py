@@ -119,3 +119,43 @@ def test_fp32_with_dense_operands(gpu, monkeypatch, d, B, L, Lkv, bias):
     assert torch.equal(x, y)
   if bias:      # (the heads' terms added by atomics in any order: H - 1 roundings of at most the terms' magnitudes' sum on either side)
     assert float((a[5] - b[5]).abs().max()) <= 2 * H * 2.0 ** -24 * H * float(a[5].abs().max())
+
+
+@pytest.mark.parametrize("d", [128, 64, 32])
+@pytest.mark.parametrize("B,L,lens,bias,how", [
+    (3, 420, [420, 129, 33], True, "causal"), (2, 300, None, True, "random"), (2, 300, [300, 128], False, "random"), (9, 513, None, True, "none"),
+    (1, 1100, None, False, "band"),
+])
+def test_bf16_with_dense_operands(gpu, monkeypatch, d, B, L, lens, bias, how):
+  """Blocks of the mask's tiles without a kept pair are neither written nor read."""
+  g = torch.Generator(device="cuda").manual_seed(d + L)
+  H = 2
+  q, k, v, do = (torch.randn(B, L, H, d, device="cuda", generator=g).mul_(0.5).to(torch.bfloat16) for _ in range(4))
+  i, j = torch.arange(L, device="cuda")[:, None], torch.arange(L, device="cuda")[None, :]
+  mask = {"causal": (i >= j).expand(B, L, L), "band": (i - j).abs() < 40, "none": None,
+          "random": torch.rand(B, L, L, device="cuda", generator=g) < 0.3}[how]
+  if how == "random":
+    mask[:, 32:64] = False
+    mask[:, 128:256, :128] = False
+    mask[:, :, 64:96] = False
+  kw = dict(causal=how == "none", n=float(L))
+  if mask is not None:
+    kw["mask"] = mask.contiguous()
+  if lens is not None:
+    kw["seq_lens"] = torch.tensor(lens, dtype=torch.int32, device="cuda")
+  if bias:
+    kw.update(bias=torch.randn(B, L, L, device="cuda", generator=g) * 0.3)
+  lib = _lib.load()
+  whole, best = lib.hstu_attn_bwd_workspace_bytes, []
+  monkeypatch.setattr(lib, "hstu_attn_bwd_workspace_bytes", lambda args: best.append(whole(args)) or best[-1])
+  a = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  grads = recml_amd.hstu_attention_bwd(q, k, v, do, bias_grad=bias, **kw)
+  least = lambda args: lib.hstu_attn_fwd_workspace_bytes(C.byref(args._obj.fwd))
+  monkeypatch.setattr(lib, "hstu_attn_bwd_workspace_bytes", least)
+  b = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  assert best[0] > B * H * L * L       # (two bytes for each of half the pairs at least)
+  for name, x, y, z in zip(("dq", "dk", "dv"), a, b, grads):
+    # (d = 128 without a bias table: fp32 sums in two halves or in one, see above)
+    bound = 2.0 ** -9 if d == 128 else 0.0
+    assert float((x.float() - y.float()).norm()) <= bound * float(y.float().norm()), name
+    assert float((x.float() - z.float()).norm()) <= bound * float(y.float().norm()), name
