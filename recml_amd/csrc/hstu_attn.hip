@@ -2397,11 +2397,12 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
 // DENSE (bit 0: additive bias, bit 1: keep-mask; the layer-side call of
 // recml/layers/keras/hstu.py:356-390): the step's 128 x 32 tile of the [L, Lkv] fp32 bias and / or
 // of the byte mask comes by direct loads like K and V (four per wave for the bias, one for the mask),
-// but into a single 16 KB + 4 KB buffer instead of a ring: a wave reads only the 32 rows of its own
-// queries, and the loads that bring those rows are its own, so each wave takes its part of step t into
-// registers at the start of the step and at once asks for step t + 1 into the same bytes -- no other
-// wave is involved, and the loads have the whole block and the barrier to land.  With a three-stage K / V
-// ring that is 68 KB at d = 128: two workgroups per CU.  A block whose mask tile is all zero is skipped.
+// but a wave reads only the 32 rows of its own queries, and the loads that bring those rows are its own, so each wave takes
+// its part of step t into registers at the start of the step and at once asks for a later step's into the same bytes -- no other
+// wave is involved.  Up to d = 64 one such stage of 16 KB + 4 KB (refilled for step t + 1) beside three of K and V, 44 KB: three
+// workgroups per CU.  At d = 128 two (step t + 2) beside two of K and V, 72 KB: the bias comes from memory, in rows of 128 bytes, and
+// K and V from the L2s, so the longer way is the bias's.  16 x 2048, 8 heads of 128, the call: one and three 281.6 us, two and two 271.4; with
+// the mask alone 239 and 224.  A block whose mask tile is all zero is skipped, one whose tile is all ones selects nothing.
 // Bit 2: the second product takes the activated weights as two bf16 parts, the rounded value and what the rounding left, instead of
 // the rounded value alone.  This is for calls whose rows were made longer for this kernel (mask_pitch, bias_pitch): the general kernel,
 // which they would otherwise take, multiplies 32-bit weights.
@@ -2409,8 +2410,11 @@ __global__ __launch_bounds__(256) void hstu_prepare(const Params p, float* __res
 // workgroups fit a CU once their LDS does: three stages (two steps in flight behind the one being
 // computed) instead of four take the d = 64 kernel with a position table from 43 KB to 32 KB, three
 // workgroups per CU to four (measured: 148 -> 139 us on the d = 64 benchmark shape).  At d = 128
-// registers allow two workgroups whatever the ring, and the depth makes no measurable difference.
-constexpr int fwd_stages(int d, int dense) { return (d <= 64 || dense != 0) ? 3 : 4; }
+// registers allow two workgroups whatever the ring, and the depth makes no measurable difference; with dense operands
+// it is two, and theirs the longer one.
+constexpr int fwd_stages(int d, int dense) { return dense != 0 && d == 128 ? 2 : (d <= 64 || dense != 0) ? 3 : 4; }
+// Stages of the dense operands (see there).
+constexpr int fwd_dense_stages(int d, int dense) { return dense != 0 && d == 128 ? 2 : 1; }
 constexpr int FWD_XCH_BYTES = 16;     // behind everything else in the forward kernel's LDS
 // which instances of the forward kernel are laid out for timestamp descriptors (64 bytes per wave and ring stage)
 constexpr bool fwd_takes_ts_desc(int d, bool ts, bool f8, bool seg, int dense) { return ts && d == 128 && !f8 && !seg && dense == 0; }
@@ -2468,9 +2472,10 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   const unsigned char* TsKey = smem + BIAS_OFF + NSTAGE * BIAS_STAGE;   // the keyed bucket table of this head
   constexpr int DENSE_OFF = BIAS_OFF + NSTAGE * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0) + (WHOLE ? 4 * WHOLE_COPY : 0);
   constexpr int DENSE_STAGE = SM::dense_stage(DENSE);
-  constexpr int XCH_OFF = DENSE_OFF + DENSE_STAGE;   // 16 bytes for values one lane hands to the workgroup
-  auto Db = [&]() { return smem + DENSE_OFF; };
-  auto Dm = [&]() { return smem + DENSE_OFF + ((DENSE & 1) ? SM::DB_BYTES : 0); };
+  constexpr int DSTAGES = fwd_dense_stages(D, DENSE);
+  constexpr int XCH_OFF = DENSE_OFF + DSTAGES * DENSE_STAGE;   // 16 bytes for values one lane hands to the workgroup
+  auto Db = [&](int st) { return smem + DENSE_OFF + st * DENSE_STAGE; };
+  auto Dm = [&](int st) { return smem + DENSE_OFF + st * DENSE_STAGE + ((DENSE & 1) ? SM::DB_BYTES : 0); };
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -2634,7 +2639,8 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   };
   auto dma_step = [&](const DmaCtx& c_, int t, auto st_) { dma_part(c_, t, st_, std::integral_constant<int, 3>{}); };
   // The dense operands of step t, each wave its own rows (the same number of loads whatever the step).
-  auto dense_refill = [&](const DmaCtx& c_, int t) {
+  auto dense_refill = [&](const DmaCtx& c_, int t, auto st_) {
+    constexpr int st = decltype(st_)::value;
     const int kv0 = t * BN;
     if (DENSE & 1) {
       // Bias tile: row r of the tile at LDS byte 128 r, its 16-byte chunks XOR-swizzled by r & 7
@@ -2651,7 +2657,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
         gr = gr < p.L - 1 ? gr : p.L - 1;
         int col = kv0 + 4 * (pc ^ (row & 7));
         col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
-        lds_dma16(dbg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Db() + j * 1024);
+        lds_dma16(dbg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Db(st) + j * 1024);
       }
     }
     if (DENSE & 2) {
@@ -2662,7 +2668,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       gr = gr < p.L - 1 ? gr : p.L - 1;
       int col = kv0 + 16 * (lane & 1);
       col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
-      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Dm() + w * 1024);
+      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Dm(st) + w * 1024);
     }
   };
   // The lane's share of the dense operands that have landed: 16 bias values (keys 8g + 4hh .. +3 of its
@@ -2670,16 +2676,17 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
   // here: once it is passed, the buffer may be refilled.
   float4 dbv[4];
   uint32_t mbits[4] = {0u, 0u, 0u, 0u};
-  auto dense_take = [&]() {
+  auto dense_take = [&](auto st_) {
+    constexpr int st = decltype(st_)::value;
     if (DENSE & 2) {
-      const unsigned char* mrow = Dm() + (32 * w + m) * 32 + 4 * hh;
+      const unsigned char* mrow = Dm(st) + (32 * w + m) * 32 + 4 * hh;
 #pragma unroll
       for (int g = 0; g < 4; ++g) mbits[g] = *(const uint32_t*)(mrow + 8 * g);
       asm volatile("" : "+v"(mbits[0]), "+v"(mbits[1]), "+v"(mbits[2]), "+v"(mbits[3]));
     }
     if (DENSE & 1) {
       const int row = 32 * w + m;
-      const unsigned char* brow = Db() + row * 128;
+      const unsigned char* brow = Db(st) + row * 128;
 #pragma unroll
       for (int g = 0; g < 4; ++g) dbv[g] = *(const float4*)(brow + (((2 * g + hh) ^ (row & 7)) * 16));
 #pragma unroll
@@ -2947,8 +2954,12 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       }
     }
     if (DENSE & 2) {
+      // (a tile that keeps all its pairs needs no selects: every byte of every lane has its lowest bit, as true and 1 have it)
+      const uint32_t all = mbits[0] & mbits[1] & mbits[2] & mbits[3] & 0x01010101u;
+      if (__builtin_amdgcn_ballot_w64(all != 0x01010101u) != 0) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) u[r] = ((mbits[r >> 2] >> (8 * (r & 3))) & 0xffu) ? u[r] : 0.f;
+        for (int r = 0; r < 16; ++r) u[r] = ((mbits[r >> 2] >> (8 * (r & 3))) & 0xffu) ? u[r] : 0.f;
+      }
     }
     if (drop_thr) {
       // dropout: a dropped pair is one more masked logit (the survivors' scale is in the output scale)
@@ -3325,7 +3336,7 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       }
     }
     if (t_lo < nt) dma_step(cx, t_lo, std::integral_constant<int, 0>{});
-    if (DENSE != 0 && t_lo < nt) dense_refill(cx, t_lo);
+    if (DENSE != 0 && t_lo < nt) dense_refill(cx, t_lo, std::integral_constant<int, 0>{});
     load_q(first);
     settle_q();
     if constexpr (WHOLE) {
@@ -3337,7 +3348,10 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
           if (x - c >= 0 && x < WHOLE_KEYS + BM) *(float*)(smem + BIAS_OFF + c * WHOLE_COPY + 4 * (x - c)) = whole[i] * LOG2E;
       }
     }
-    if (t_lo + 1 < nt) dma_step(cx, t_lo + 1, std::integral_constant<int, 1>{});
+    if (t_lo + 1 < nt) {
+      if constexpr (DSTAGES == 2) dense_refill(cx, t_lo + 1, std::integral_constant<int, 1>{});
+      else dma_step(cx, t_lo + 1, std::integral_constant<int, 1>{});
+    }
     if constexpr (NSTAGE > 3 && !PAIRS) {
       if (t_lo + 2 < nt) dma_step(cx, t_lo + 2, std::integral_constant<int, 2>{});
     }
@@ -3369,6 +3383,29 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
         if (t + 2 >= nt) break;
         pair(t + 2, std::integral_constant<int, 2>{});
       }
+    } else if constexpr (DENSE != 0 && DSTAGES == 2) {
+      // Step t where the dense operands have two stages and so have K and V: the wave takes its rows of step t's bias and
+      // mask tiles into registers, asks for the K / V tiles of step t + 1 (into the ring stage that the barrier before freed), then
+      // for its rows of step t + 2 into the bytes it has just read, and computes its block.  Before the barrier everything of step
+      // t + 1 has landed; the dense operands of step t + 2, the youngest loads, stay in flight.
+      static_assert(NSTAGE == 2, "one step of K / V tiles in flight");
+      if (t_lo + 1 < nt) HSTU_WAIT_VMCNT(NDENSE); else HSTU_WAIT_VMCNT(0);    // all of step t_lo
+      __syncthreads();
+      auto step = [&](int t, auto st_) {
+        constexpr int st = decltype(st_)::value;
+        const bool lv = live(t);
+        if (lv) dense_take(st_);
+        if (t + 1 < nt) dma_step(cx, t + 1, std::integral_constant<int, 1 - st>{});
+        if (t + 2 < nt) dense_refill(cx, t + 2, st_);
+        if (lv) block(t, st_);
+        if (t + 2 < nt) HSTU_WAIT_VMCNT(NDENSE); else HSTU_WAIT_VMCNT(0);
+        __syncthreads();
+      };
+      for (int t = t_lo; t < nt; t += 2) {
+        step(t, std::integral_constant<int, 0>{});
+        if (t + 1 >= nt) break;
+        step(t + 1, std::integral_constant<int, 1>{});
+      }
     } else if constexpr (DENSE != 0) {
       // Step t with dense operands: the wave takes its rows of the step's bias and mask tiles into registers,
       // asks for the next step's into the same bytes, then for the K / V tiles of step t + 2 (into the ring
@@ -3381,8 +3418,8 @@ __global__ __launch_bounds__(MFMA_THREADS, 2) void hstu_fwd_mfma_bf16(const Para
       auto step = [&](int t, auto st_) {
         constexpr int st = decltype(st_)::value;
         const bool lv = live(t);
-        if (lv) dense_take();
-        if (t + 1 < nt) dense_refill(cx, t + 1);
+        if (lv) dense_take(std::integral_constant<int, 0>{});
+        if (t + 1 < nt) dense_refill(cx, t + 1, std::integral_constant<int, 0>{});
         if (t + 2 < nt) dma_step(cx, t + 2, std::integral_constant<int, (st + 2) % NSTAGE>{});
         if (lv) block(t, st_);
         if (t + 2 < nt) HSTU_WAIT_VMCNT(NDMA); else HSTU_WAIT_VMCNT(0);
@@ -6253,7 +6290,8 @@ int launch_bwd(const Params& p, hipStream_t st) {
 template <int D, bool POS, bool TS, bool F8, bool SEG = false, int DENSE = 0, bool PERSIST = false, bool WHOLE = false>
 int launch_mfma_inst(const Params& p, hipStream_t st) {
   const int smem = MfmaSmem<D, F8 ? 1 : 2>::total(POS && !WHOLE, TS, SEG, DENSE, fwd_stages(D, DENSE)) + FWD_XCH_BYTES + (WHOLE ? 4 * WHOLE_COPY : 0) +
-                   (fwd_takes_ts_desc(D, TS, F8, SEG, DENSE) ? fwd_stages(D, DENSE) * NWAVES * 64 : 0);
+                   (fwd_takes_ts_desc(D, TS, F8, SEG, DENSE) ? fwd_stages(D, DENSE) * NWAVES * 64 : 0) +
+                   (fwd_dense_stages(D, DENSE) - 1) * MfmaSmem<D, F8 ? 1 : 2>::dense_stage(DENSE);
   static int granted[64];
   if (int rc = allow_lds((const void*)hstu_fwd_mfma_bf16<D, POS, TS, F8, SEG, DENSE, PERSIST, WHOLE>, smem, granted)) return rc;
   hipError_t e;

@@ -98,3 +98,25 @@ def test_a_mask_by_the_lowest_value(gpu, d):
     grads.append([out.detach(), *torch.autograd.grad(out, [*ts, bias], dout)])
   for a, b in zip(*grads):
     assert a.isfinite().all() and (a.float() - b.float()).norm() <= 2.0 ** -8 * b.float().norm()
+
+
+@pytest.mark.parametrize("keys", [16, 32, 48, 96, 144, 272])
+@pytest.mark.parametrize("d,with_mask,with_bias", [(128, True, True), (128, True, False), (128, False, True), (64, True, True)])
+def test_steps_of_the_dense_operands_ring(gpu, keys, d, with_mask, with_bias):
+  """One to nine steps of 32 keys, odd and even, rows at both sides of a wave's 32; mask tiles that keep all, a part (a single pair dropped
+  among them) and none, with other bytes than 1 for true.  Each of a row's activated weights and the output are rounded to bf16: 2^-8 of
+  the largest."""
+  rng = np.random.default_rng(keys + d)
+  B, L, H = 2, 161, 2
+  q = O.round_bf16(rng.standard_normal((B, L, H, d)).astype(np.float32) * 0.4)
+  k, v = (O.round_bf16(rng.standard_normal((B, keys, H, d)).astype(np.float32) * 0.4) for _ in range(2))
+  mask = np.ones((B, L, keys), np.uint8)
+  mask[0, 5, keys - 1] = 0                       # one pair of an otherwise whole tile
+  mask[0, 64:96, :16] = 0
+  mask[1, 32:64] = 0                             # a wave's tiles
+  mask[1, 128:] = rng.choice([0, 2, 255], (L - 128, keys))
+  bias = (rng.standard_normal((B, L, keys)) * 0.4).astype(np.float32) if with_bias else None
+  out = recml_amd.hstu_attention(_dev(q, bf), _dev(k, bf), _dev(v, bf), n=float(L), alpha=0.3, causal=False,
+                                 mask=_dev(mask) if with_mask else None, bias=None if bias is None else _dev(bias))
+  ref = O.pointwise_attention_dense(q * 0.3, k, v, (mask != 0).astype(np.float64) if with_mask else np.ones((B, L, keys)), bias)
+  assert _rel(out.float().cpu().numpy(), ref) <= 2 * 2.0 ** -8
