@@ -4677,6 +4677,13 @@ __device__ __forceinline__ uint32_t ds_block_off(const Params& p, int i, int j) 
 
 // Ring depth of the dK/dV kernel (see there).
 constexpr int dkv_stages(int d, bool dense_bias, bool wide) { return (d == 128 && !dense_bias && !wide) ? 6 : NSTAGE; }
+// Bytes of the dense operands in the dK/dV kernel's LDS (see there).
+constexpr int DKV_DB_STAGES = 2, DKV_DM_STAGES = 3;
+template <int D>
+constexpr int dkv_dense_bytes(bool mask, bool dense_bias, int nst) {
+  using SM = MfmaSmem<D, 2>;
+  return dense_bias ? DKV_DB_STAGES * SM::DB_BYTES + (mask ? DKV_DM_STAGES * SM::DM_BYTES : 0) : mask ? nst * SM::DM_BYTES : 0;
+}
 
 // WIDE (d = 128 without a dense bias, other than the stream's instance): eight waves, two per SIMD.  Waves w and w + 4
 // share 32 keys and take the even and the odd steps; K and V come from LDS (in registers next to the accumulators of 32
@@ -4706,11 +4713,14 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
 // MSK: the dense keep-mask as in the other backward kernel; here a step's tile is 32 query rows x this workgroup's
 // 128 keys (wave w fetches rows 8w .. 8w + 7 of it, 128 bytes each), a lane reads the 16 bytes of its key's column,
 // and the workgroup finds the query steps in which the mask keeps one of its keys by one pass over its columns.
-// DB: the dense bias likewise, a step's tile of 32 rows x 128 keys (16 KB): wave w fetches rows 8w .. 8w + 7, a lane
-// reads the 16 values of its key's column (consecutive lanes, consecutive words: no swizzle needed).  The bias's
-// gradient is the other kernel's business.
+// DB: the dense bias is 16 KB a step, and four stages of it with the mask's left one workgroup to a CU.  A wave therefore brings what
+// its own 32 keys need (32 rows of 128 bytes, and 32 of the mask's) into bytes that no other wave reads: two stages for the bias,
+// whose 16 values a lane takes into registers ahead of its block, and three for the mask, read inside it.  They are refilled without
+// regard to the other waves, and the workgroup's LDS falls from 112 to 76 KB at d = 64, two workgroups per CU (16 x up to 1000, 8 heads of
+// 64, mask and bias: the kernel 108 -> 92 us).
+// The bias's gradient is the other kernel's business.
 template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false>
-__global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), ((D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)) || DB ? 1 : 2))
+__global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), (D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO) ? 1 : 2))
 void hstu_bwd_dkv_mfma(const Params p) {
   constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO);
   using SH = DkvShape<D, WIDE>;
@@ -4731,7 +4741,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
   constexpr int DVB = D / 32;
   constexpr int NPIECE = SM::V_BYTES / 1024;
   constexpr int LD = NPIECE >= NW ? NPIECE / NW : 1;
-  constexpr int NDMA = 2 * LD + ((POS || TS) ? 1 : 0) + (SEG ? 1 : 0) + (MSK ? 1 : 0) + (DB ? 4 : 0);
+  constexpr int NDMA = 2 * LD + ((POS || TS) ? 1 : 0) + (SEG ? 1 : 0) + (MSK && !DB ? 1 : 0);
   // Ring depth: 4 stages (two pairs of steps: one at work, one on its way), or 6 where the workgroup has the CU's
   // LDS to itself anyway (d = 128) and the stages are small enough: the loads of a pair then have the time of two
   // pairs to arrive, which the hand-scheduled pairs need (one pair's time is less than a trip to memory).
@@ -4750,11 +4760,9 @@ void hstu_bwd_dkv_mfma(const Params p) {
   auto Qs = [&](int st) { return (bf16_t*)(smem + st * SM::STAGE); };
   auto Os = [&](int st) { return (bf16_t*)(smem + st * SM::STAGE + SM::K_BYTES); };
   constexpr int BIAS_OFF = NST * SM::STAGE;
-  constexpr int BIAS_STAGE = (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0) + (SEG ? SM::SEG_BYTES : 0) + (MSK ? SM::DM_BYTES : 0) +
-                             (DB ? SM::DB_BYTES : 0);
+  constexpr int BIAS_STAGE = (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0) + (SEG ? SM::SEG_BYTES : 0) + (MSK && !DB ? SM::DM_BYTES : 0);
   auto Sg = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0)); };
   auto Mk = [&](int st) { return smem + BIAS_OFF + st * BIAS_STAGE; };      // MSK (first in the stage): [32 rows][128 bytes]
-  auto Bk = [&](int st) { return smem + BIAS_OFF + st * BIAS_STAGE + (MSK ? SM::DM_BYTES : 0); };   // DB: [32 rows][128 floats]
   auto Wc = [&](int st) { return (float*)(smem + BIAS_OFF + st * BIAS_STAGE); };
   auto Tq = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0)); };
   const unsigned char* TsKey = smem + BIAS_OFF + NST * BIAS_STAGE;   // the keyed bucket table of this head
@@ -4907,7 +4915,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
         lds_dma16_at(p.q_seg + (int64_t)b * p.L, (uint32_t)g4 * 4u, smem_lds + (uint32_t)((const unsigned char*)Sg(st) - smem));
       }
     }
-    if (MSK) {
+    if (MSK && !DB) {
       // rows 8w .. 8w + 7 of the step's mask tile, eight lanes per row (16 bytes each = this tile's 128 keys); rows past
       // L and pieces past Lkv re-read bytes inside the matrix (those pairs are masked by their index)
       const uint8_t* mg = (const uint8_t*)scalar_ptr(p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0));
@@ -4917,18 +4925,42 @@ void hstu_bwd_dkv_mfma(const Params p) {
       col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
       lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Mk(st) + w * 1024);
     }
-    if (DB) {
-      // rows 8w .. 8w + 7 of the step's bias tile in four pieces of two rows (512 bytes a row = this tile's 128 keys);
-      // rows past L and pieces past Lkv re-read values inside the matrix (those pairs are masked by their index)
-      const float* bg = (const float*)scalar_ptr(p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0));
+  };
+  // DB: this wave's part of the dense operands of step t.  The bias's row 8g + 4 hh + tt stands in place 8g + 2 tt + hh, 128 bytes each, so that
+  // the two halves of the wave read neighbouring rows; the mask's rows in their order, 32 bytes each.  Rows past L and pieces past Lkv
+  // re-read values inside the matrix (those pairs are masked by their index).
+  constexpr int DENSE_OFF = BIAS_OFF + NST * BIAS_STAGE;
+  auto own_bias = [&](int t) { return smem + DENSE_OFF + ((t - t_lo) % DKV_DB_STAGES) * SM::DB_BYTES + w * (SM::DB_BYTES / NWAVES); };
+  auto own_mask = [&](int t) { return smem + DENSE_OFF + DKV_DB_STAGES * SM::DB_BYTES + ((t - t_lo) % DKV_DM_STAGES) * SM::DM_BYTES + w * (SM::DM_BYTES / NWAVES); };
+  auto dense_refill = [&](int t) __attribute__((always_inline)) {
+    const int qbs = t * BN;
+    const float* bg = (const float*)scalar_ptr(p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0));
+    int col = r0 + 4 * (lane & 7);
+    col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int gr = qbs + 8 * w + 2 * r + (lane >> 5);
-        gr = gr < p.L - 1 ? gr : p.L - 1;
-        int col = kv0 + 4 * (lane & 31);
-        col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
-        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
-      }
+    for (int r = 0; r < 4; ++r) {
+      int gr = qbs + 8 * r + 4 * ((lane >> 3) & 1) + (lane >> 4);
+      gr = gr < p.L - 1 ? gr : p.L - 1;
+      lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, own_bias(t) + r * 1024);
+    }
+    if (MSK) {
+      const uint8_t* mg = (const uint8_t*)scalar_ptr(p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0));
+      int gr = qbs + (lane >> 1);
+      gr = gr < p.L - 1 ? gr : p.L - 1;
+      int mc = r0 + 16 * (lane & 1);
+      mc = mc < p.mask_pitch - 16 ? mc : p.mask_pitch - 16;
+      lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)mc, own_mask(t));
+    }
+  };
+  // (the empty statements make the compiler wait for the values here: behind them the bytes may be refilled)
+  float dbv[DB ? 16 : 1];
+  auto dense_take = [&](int t) __attribute__((always_inline)) {
+    if constexpr (DB) {
+      const float* const bcol = (const float*)own_bias(t) + 32 * hh + m;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dbv[r] = bcol[(8 * (r >> 2) + 2 * (r & 3)) * 32];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(dbv[r]));
     }
   };
 
@@ -4942,6 +4974,10 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i)
     if (t_lo + i < nt) dma_step(t_lo + i);
+  if constexpr (DB) {
+    if (wave_live && t_lo < nt) dense_refill(t_lo);
+    if (wave_live && t_lo + 1 < nt) dense_refill(t_lo + 1);
+  }
   if (DPOS || DTS) {
     for (int i = tid; i < DkvTg<WIDE>::FLOATS; i += THREADS) TgBase[i] = 0.f;
   }
@@ -5124,10 +5160,8 @@ void hstu_bwd_dkv_mfma(const Params p) {
       for (int r = 0; r < 16; ++r) u[r] = sacc[r] * alpha2;
     }
     if (DB) {
-      // the lane's column of the bias tile: row 8g + 4hh + tt at key 32w + m
-      const float* bcol = (const float*)Bk(st) + 32 * w + m + (4 * hh) * 128;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) u[r] = __builtin_fmaf(bcol[(8 * (r >> 2) + (r & 3)) * 128], LOG2E, u[r]);
+      for (int r = 0; r < 16; ++r) u[r] = __builtin_fmaf(dbv[r], LOG2E, u[r]);
     }
     // (the table gradients, as in the dQ kernel: the lane's 16 pairs are in bucket bk_lane >= 0, those with a bit in
     // far_rows in the next one, or bkp has the 16 buckets)
@@ -5310,10 +5344,11 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
     if (MSK) {
       // the lane's column of the mask tile: byte of row 8g + 4hh + tt at key 32w + m
-      const unsigned char* mcol = Mk(st) + 32 * w + m + (4 * hh) * 128;
+      constexpr int PITCH = DB ? BN : BM;
+      const unsigned char* mcol = (DB ? own_mask(t) : Mk(st) + 32 * w) + m + (4 * hh) * PITCH;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const bool keep = mcol[(8 * (r >> 2) + (r & 3)) * 128] != 0;
+        const bool keep = mcol[(8 * (r >> 2) + (r & 3)) * PITCH] != 0;
         pv[r] = keep ? pv[r] : 0.f;
         ds[r] = keep ? ds[r] : 0.f;
       }
@@ -5526,6 +5561,19 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
     const bool first = wave_live && t >= t_wave && t <= t_wave_end;
     const bool second = t + 1 < nt && wave_live && t + 1 >= t_wave && t + 1 <= t_wave_end;
+    if constexpr (DB) {
+      if (first) dense_take(t);
+      if (wave_live && t + 2 < nt) dense_refill(t + 2);
+      if (first) block(t);
+      if (second) dense_take(t + 1);
+      if (wave_live && t + 3 < nt) {
+        if (MSK) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the mask's bytes were step t's, which its block has read)
+        dense_refill(t + 3);
+      }
+      if (second) block(t + 1);
+      end_of_pair(n_sent, second ? 1 : 0);                   // (the second block's stores are the only ones younger than every load)
+      return;
+    }
     if (first) block(t);
     if (second) block(t + 1);
     end_of_pair(n_sent, (first ? 1 : 0) + (second ? 1 : 0));
@@ -6466,8 +6514,7 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   const int smem_q = smem + (TG ? BWD_TG_BYTES : 0);
   using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, false)>;
   constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB, false));
-  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + (MSK ? nst_kv * MfmaSmem<D, 2>::DM_BYTES : 0) +
-                      (DB ? nst_kv * MfmaSmem<D, 2>::DB_BYTES : 0) +
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + dkv_dense_bytes<D>(MSK, DB, nst_kv) +
                       SH::KV_LDS + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
   static int granted_q[64], granted_kv[64];
   if (int rc = allow_lds((const void*)hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>, smem_q, granted_q)) return rc;
@@ -6489,7 +6536,7 @@ int launch_bwd_kept(const Params& p, hipStream_t st) {
   constexpr bool wide = dkv_wide(D, POS, TS, SEG, MSK, DB, true);
   using SH = DkvShape<D, wide>;
   constexpr int nst = dkv_stages(D, DB, wide);
-  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + (MSK ? nst * MfmaSmem<D, 2>::DM_BYTES : 0) + (DB ? nst * MfmaSmem<D, 2>::DB_BYTES : 0) +
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + dkv_dense_bytes<D>(MSK, DB, nst) +
                       SH::KV_LDS + (TS ? nst * 16 : 0) + (POS || TS ? DkvTg<wide>::BYTES : 0);
   const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, true>;
   const auto dq = hstu_bwd_dq_ds<D, MSK>;
