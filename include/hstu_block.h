@@ -220,6 +220,8 @@ int hstu_pack_plan(const void* lens, int32_t lens_are_64bit, int32_t B, int32_t 
 /* Lengths of an end-padded batch from its byte mask [B, L]; *bad becomes 1 when a row is not non-zero bytes followed by zeros
  * (and stays as it was otherwise). */
 int hstu_mask_lengths(const uint8_t* mask, int32_t B, int32_t L, int32_t* lens, int32_t* bad, void* stream);
+/* hstu_embed_norm_fwd and, with a mask, hstu_mask_lengths on it in the same launch. */
+int hstu_embed_norm_mask_fwd(const HstuEmbedNormArgs* args, const uint8_t* mask, int32_t B, int32_t L, int32_t* lens, int32_t* bad, void* stream);
 /* d[r, :] *= silu'(pre[r, :]) in place, bf16 rows of `width` elements. */
 int hstu_silu_bwd(void* d, int64_t d_stride, const void* pre, int64_t pre_stride, int64_t rows, int32_t width, void* stream);
 

@@ -25,6 +25,7 @@ EXPORTS = (
     "hstu_embed_grad_workspace_bytes",
     "hstu_pack_plan",
     "hstu_mask_lengths",
+    "hstu_embed_norm_mask_fwd",
     "hstu_silu_bwd",
     "hstu_gemm",
     "hstu_gemm_workspace_bytes",

@@ -344,16 +344,49 @@ struct EmbedNormParams {
   bf16_t* sums;            // the rows before the norm, for the gradients; or null
   int64_t* keys;           // the table rows taken, for the gradients; or null
   int32_t* outside;        // raised where an index lies outside its table; or null
+  const uint8_t* mask;     // or null: the batch's mask, whose lengths the first `mask_groups` workgroups write
+  int32_t* lens;
+  int32_t* bad;
+  int32_t mask_B, mask_L;
+  uint32_t mask_groups;
 };
+
+// The length of row b of an end-padded batch's mask (bytes), by one wavefront; *bad is raised by a row that is not a run of non-zero bytes
+// followed by zeros.
+__device__ __forceinline__ void mask_length(const uint8_t* __restrict__ mask, int b, int L, int lane, int32_t* __restrict__ lens, int32_t* __restrict__ bad) {
+  const uint8_t* row = mask + (int64_t)b * L;
+  int n = 0, last = -1;
+  for (int i = lane; i < L; i += 64) {
+    const bool on = row[i] != 0;
+    n += on ? 1 : 0;
+    last = on ? i : last;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    n += __shfl_xor(n, d, 64);
+    const int o = __shfl_xor(last, d, 64);
+    last = last > o ? last : o;
+  }
+  if (lane == 0) {
+    lens[b] = n;
+    if (last + 1 != n) *bad = 1;
+  }
+}
 
 // Rows on lanes as in hstu_norm_gate: a token's table row (and position row) is gathered into registers, normalised
 // there and written once.  In training the gathered rows and their ids are stored next to it (as many bytes again): the
 // backward then works on its own copies, so that neither the ids nor the tables have to stay as they were until it runs.
+// With a mask a few more workgroups count its rows: what both do is little beside a launch (32 x 50, width 64: 4.0 + 3.6 us as two).
 template <int CH, int LPR>
 __global__ __launch_bounds__(256) void hstu_embed_norm(const EmbedNormParams p) {
   constexpr int RPW = 64 / LPR;
+  if (blockIdx.x < p.mask_groups) {
+    const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (b < p.mask_B) mask_length(p.mask, b, p.mask_L, threadIdx.x & 63, p.lens, p.bad);
+    return;
+  }
   const int lane = threadIdx.x & (LPR - 1);
-  const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + ((threadIdx.x & 63) / LPR);
+  const int64_t row = ((int64_t)(blockIdx.x - p.mask_groups) * 4 + (threadIdx.x >> 6)) * RPW + ((threadIdx.x & 63) / LPR);
   if (row >= p.rows) return;
   const int64_t at = p.row_map ? p.row_map[row] : row;
   int64_t id = p.ids[at];
@@ -451,29 +484,11 @@ __global__ __launch_bounds__(256) void hstu_pack_plan_kernel(const T* __restrict
   for (int i = tid; i < n; i += 256) row_map[off + i] = b * L + i;
 }
 
-// Lengths of an end-padded batch from its mask (bytes, one row per wavefront); *bad is raised by a row that is not a
-// run of non-zero bytes followed by zeros.
+// Lengths of an end-padded batch from its mask, one row per wavefront.
 __global__ __launch_bounds__(256) void hstu_mask_lengths_kernel(const uint8_t* __restrict__ mask, int B, int L, int32_t* __restrict__ lens,
                                                          int32_t* __restrict__ bad) {
   const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (b >= B) return;
-  const uint8_t* row = mask + (int64_t)b * L;
-  int n = 0, last = -1;
-  for (int i = lane; i < L; i += 64) {
-    const bool on = row[i] != 0;
-    n += on ? 1 : 0;
-    last = on ? i : last;
-  }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    n += __shfl_xor(n, d, 64);
-    const int o = __shfl_xor(last, d, 64);
-    last = last > o ? last : o;
-  }
-  if (lane == 0) {
-    lens[b] = n;
-    if (last + 1 != n) *bad = 1;
-  }
+  if (b < B) mask_length(mask, b, L, lane, lens, bad);
 }
 
 // ---- gradients of the embedding tables ----------------------------------
@@ -893,7 +908,9 @@ int hstu_norm_gate_bwd(const HstuNormGateBwdArgs* a, void* stream) { return norm
 // (a launch for each vector's conversion otherwise: 4 us each, twenty of them in a ranking model's step)
 int hstu_norm_gate_bwd_rounded(const HstuNormGateBwdArgs* a, void* stream) { return norm_gate_bwd<bf16_t>(a, stream); }
 
-int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
+int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) { return hstu_embed_norm_mask_fwd(a, nullptr, 0, 0, nullptr, nullptr, stream); }
+
+int hstu_embed_norm_mask_fwd(const HstuEmbedNormArgs* a, const uint8_t* mask, int32_t mask_B, int32_t mask_L, int32_t* lens, int32_t* bad, void* stream) {
   HstuEmbedNormArgs own;
   a = block_today(a, own, offsetof(HstuEmbedNormArgs, row_map), offsetof(HstuEmbedNormArgs, sums));
   if (!a) return block_fail(HSTU_BLOCK_ERR_NULL, "args is null");
@@ -904,7 +921,9 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
     return block_fail(HSTU_BLOCK_ERR_SHAPE, "rows >= 0, vocab >= 1 and width a multiple of 8 in [8, 8192] expected, got rows=%lld vocab=%lld width=%d",
                 (long long)a->rows, (long long)a->vocab, a->width);
   g_err[0] = 0;
-  if (a->rows == 0) return HSTU_BLOCK_OK;
+  if (mask && (!lens || !bad)) return block_fail(HSTU_BLOCK_ERR_NULL, "lens and bad must be non-null");
+  if (mask && (mask_B < 1 || mask_L < 1)) return block_fail(HSTU_BLOCK_ERR_SHAPE, "bad batch B=%d L=%d", mask_B, mask_L);
+  if (a->rows == 0) return mask ? hstu_mask_lengths(mask, mask_B, mask_L, lens, bad, stream) : HSTU_BLOCK_OK;
   if (!a->ids || !a->table || !a->out || !a->gamma || !a->beta) return block_fail(HSTU_BLOCK_ERR_NULL, "ids, table, out, gamma and beta must be non-null");
   if ((a->pos_table != nullptr) != (a->positions != nullptr || a->L > 0) || (a->pos_table && a->n_positions < 1) || a->L < 0)
     return block_fail(HSTU_BLOCK_ERR_NULL, "pos_table and positions (or L) go together (with n_positions >= 1)");
@@ -912,7 +931,8 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
       (a->table_stride & 7) || a->table_stride < a->width)
     return block_fail(HSTU_BLOCK_ERR_SHAPE, "pointers must be 16-byte aligned, table_stride a multiple of 8 elements and >= width");
   if (a->sums && (!a->round_steps || !block_aligned16(a->sums))) return block_fail(HSTU_BLOCK_ERR_SHAPE, "sums go with round_steps and are 16-byte aligned");
-  if ((a->rows + 3) / 4 > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
+  const uint32_t mask_groups = mask ? (uint32_t)((mask_B + 3) / 4) : 0u;
+  if ((a->rows + 3) / 4 + (int64_t)mask_groups > 0x7fffffffLL) return block_fail(HSTU_BLOCK_ERR_SHAPE, "too many rows");
   EmbedNormParams p;
   p.ids = a->ids; p.positions = a->positions;
   p.table = (const bf16_t*)a->table; p.pos_table = (const bf16_t*)a->pos_table;
@@ -921,9 +941,10 @@ int hstu_embed_norm_fwd(const HstuEmbedNormArgs* a, void* stream) {
   p.width = a->width; p.eps = a->eps; p.scale = a->scale;
   p.row_map = a->row_map; p.L = a->L; p.round_steps = a->round_steps;
   p.sums = (bf16_t*)a->sums; p.keys = a->keys; p.outside = a->outside;
+  p.mask = mask; p.lens = lens; p.bad = bad; p.mask_B = mask_B; p.mask_L = mask_L; p.mask_groups = mask_groups;
   hipStream_t st = (hipStream_t)stream;
   const int lpr = lanes_per_row(a->width), per = 4 * (64 / lpr), ch = (a->width + 511) / 512;
-  const dim3 grid((unsigned)((a->rows + per - 1) / per)), block(256);
+  const dim3 grid((unsigned)((a->rows + per - 1) / per) + mask_groups), block(256);
   if (lpr == 8) hipLaunchKernelGGL((hstu_embed_norm<1, 8>), grid, block, 0, st, p);
   else if (lpr == 16) hipLaunchKernelGGL((hstu_embed_norm<1, 16>), grid, block, 0, st, p);
   else if (lpr == 32) hipLaunchKernelGGL((hstu_embed_norm<1, 32>), grid, block, 0, st, p);

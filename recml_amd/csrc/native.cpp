@@ -1321,17 +1321,24 @@ bool capturing(void* stream) {
   return hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
-// embed(ids, table, pos_table, gamma, beta, eps, scale, row_map, tokens, differentiable) -> (rows [tokens, D] (or shaped like ids), ticket)
-// or None.  Without gradients indices are clamped into their tables and the ticket is None; with them they are taken as torch's indexing
+// Whether hstu_mask_lengths reads this mask as it is.
+bool byte_mask(const Tensor& mask) {
+  return mask.is_cuda() && mask.dim() == 2 && mask.size(0) >= 1 && mask.size(1) >= 1 && mask.is_contiguous() &&
+         (mask.scalar_type() == at::kBool || mask.scalar_type() == at::kByte) && mask.numel() <= 0x7fffffff;
+}
+
+// embed(ids, table, pos_table, gamma, beta, eps, scale, row_map, tokens, differentiable, mask) -> (rows [tokens, D] (or shaped like ids), ticket),
+// with a mask shaped like ids (rows, ticket, lengths, the lengths' ticket: as from mask_lengths, in the same launch), or None.  Without gradients indices are clamped into their tables and the ticket is None; with them they are taken as torch's indexing
 // takes them, and raised(ticket) says that one lay outside.  (A captured step has no ticket: nobody can ask while it is captured.)
 PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
-  if (count != 10) {
-    PyErr_SetString(PyExc_TypeError, "embed takes 10 arguments");
+  if (count != 11) {
+    PyErr_SetString(PyExc_TypeError, "embed takes 11 arguments");
     return nullptr;
   }
   return guarded([&]() -> PyObject* {
     EmbedCall c;
-    Tensor table, pos_table, gamma, beta;
+    Tensor table, pos_table, gamma, beta, mask;
+    if (!tensor_arg(a[10], &mask)) Py_RETURN_NONE;
     if (!tensor_arg(a[0], &c.ids) || !tensor_arg(a[1], &table) || !tensor_arg(a[2], &pos_table) || !tensor_arg(a[3], &gamma) || !tensor_arg(a[4], &beta) ||
         !float_arg(a[5], &c.eps) || !float_arg(a[6], &c.scale) || !tensor_arg(a[7], &c.row_map) || !long_arg(a[8], &c.T)) Py_RETURN_NONE;
     if (!c.ids.defined() || !table.defined() || !table.is_cuda() || dual({&table, &pos_table, &gamma, &beta})) Py_RETURN_NONE;
@@ -1343,6 +1350,7 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     const bool packed = c.row_map.defined();
     // (the map's entries index ids: one with more entries is another batch's)
     if (packed && (!plain(c.row_map, dev, at::kInt) || c.row_map.numel() < c.T || c.row_map.numel() > c.ids.numel())) Py_RETURN_NONE;
+    if (mask.defined() && (packed || !byte_mask(mask) || mask.device() != dev || mask.sizes() != c.ids.sizes() || capturing(stream_of(table)))) Py_RETURN_NONE;
     if (!packed) c.T = c.ids.numel();
     const bool graph = a[9] == Py_True && wants_grad({&table, &pos_table, &gamma, &beta});
     // (a padded batch longer than the position table: torch's addition reports it)
@@ -1350,8 +1358,8 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
     c.training = graph;
     if (D % 8 || D > (graph ? 2048 : 8192) || c.T < 1 || c.L < 1 || gamma.numel() != D || beta.numel() != D || c.ids.numel() > (1 << 30) ||
         (graph && (table.size(0) > (1 << 30)))) Py_RETURN_NONE;
-    Tensor out, sums, keys;
-    std::unique_ptr<Word> outside;
+    Tensor out, sums, keys, lens;
+    std::unique_ptr<Word> outside, bad;
     without_lock(table, [&] {
       out = packed ? fresh(table, {c.T, D}) : fresh(table, {c.ids.size(0), c.L, D});
       HstuEmbedNormArgs e;
@@ -1367,8 +1375,15 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
           e.outside = outside->host.data_ptr<int32_t>();
         }
       }
-      block_check(hstu_embed_norm_fwd(&e, stream_of(table)), "hstu_embed_norm_fwd");
+      if (mask.defined()) {
+        lens = at::empty({mask.size(0)}, mask.options().dtype(at::kInt));
+        bad = std::make_unique<Word>(mask);
+      }
+      block_check(hstu_embed_norm_mask_fwd(&e, mask.defined() ? (const uint8_t*)mask.const_data_ptr() : nullptr, (int32_t)c.ids.size(0), (int32_t)c.L,
+                                           bad ? lens.data_ptr<int32_t>() : nullptr, bad ? bad->host.data_ptr<int32_t>() : nullptr, stream_of(table)),
+                  "hstu_embed_norm_fwd");
       if (outside) outside->record(stream_of(table));
+      if (bad) bad->record(stream_of(table));
       return true;
     });
     if (graph) {
@@ -1387,7 +1402,13 @@ PyObject* embed(PyObject*, PyObject* const* a, Py_ssize_t count) {
       torch::autograd::set_history(out, node);
     }
     PyObject* const ticket = outside ? ticket_of(std::move(outside)) : (Py_INCREF(Py_None), Py_None);
-    return ticket ? Py_BuildValue("(NN)", THPVariable_Wrap(std::move(out)), ticket) : nullptr;
+    if (!ticket || !bad) return ticket ? Py_BuildValue("(NN)", THPVariable_Wrap(std::move(out)), ticket) : nullptr;
+    PyObject* const end = ticket_of(std::move(bad));
+    if (!end) {
+      Py_DECREF(ticket);
+      return nullptr;
+    }
+    return Py_BuildValue("(NNNN)", THPVariable_Wrap(std::move(out)), ticket, THPVariable_Wrap(std::move(lens)), end);
   });
 }
 
@@ -1500,8 +1521,7 @@ PyObject* mask_lengths(PyObject*, PyObject* const* a, Py_ssize_t count) {
   }
   return guarded([&]() -> PyObject* {
     Tensor mask;
-    if (!tensor_arg(a[0], &mask) || !mask.defined() || !mask.is_cuda() || mask.dim() != 2 || mask.size(0) < 1 || mask.size(1) < 1 || !mask.is_contiguous() ||
-        (mask.scalar_type() != at::kBool && mask.scalar_type() != at::kByte) || mask.numel() > 0x7fffffff) Py_RETURN_NONE;
+    if (!tensor_arg(a[0], &mask) || !mask.defined() || !byte_mask(mask)) Py_RETURN_NONE;
     Tensor lens;
     auto word = without_lock(mask, [&] {
       lens = at::empty({mask.size(0)}, mask.options().dtype(at::kInt));

@@ -418,14 +418,18 @@ class HSTU(torch.nn.Module):
       return hstu_block_ops.layer_norm(x, self.final_norm_gamma, self.final_norm_beta, self.eps)
     return F.layer_norm(x, (D,), self.final_norm_gamma, self.final_norm_beta, self.eps)
 
+  def _embed(self, ids, row_map, tokens, mask):
+    return _native.embed(ids if ids.dtype == torch.int64 and ids.is_contiguous() else ids.to(torch.int64).contiguous(), self.item_embedding,
+                         self.position_embedding, self.final_norm_gamma, self.final_norm_beta, self.eps,
+                         self.model_dim ** 0.5 if self.scale_by_sqrt_dim else 1.0, row_map, tokens, True, mask)
+
   def _front_end(self, ids, row_map=None, tokens=0):
     """Gather, scale, position embedding and final_norm (hstu.py:593-601): in bf16 on a GPU one pass, and one each for the
     gradients of the norm and of the tables.  ids [B, L]; the packed form with `row_map` (its `tokens` first entries).
     Returns the rows and, with gradients, a ticket for _check_indices."""
     table, positions = self.item_embedding, self.position_embedding
     scale, length = self.model_dim ** 0.5 if self.scale_by_sqrt_dim else 1.0, ids.shape[1]
-    got = _native.embed(ids if ids.dtype == torch.int64 and ids.is_contiguous() else ids.to(torch.int64).contiguous(), table, positions,
-                      self.final_norm_gamma, self.final_norm_beta, self.eps, scale, row_map, tokens, True)
+    got = self._embed(ids, row_map, tokens, None)
     x, ticket = (None, None) if got is None else got
     if x is None:
       where = None if row_map is None else row_map[:tokens].to(torch.int64)
@@ -490,7 +494,7 @@ class HSTU(torch.nn.Module):
     for padding.  Rows past a sequence's length are then returned as zeros, whereas the padded
     form (like the reference) carries the padded positions' own embeddings through the blocks.
     """
-    ticket = None
+    ticket = front = None
     if attention_mask is not None:
       if jagged or pos_bias is not None or ts_bias is not None or seq_lens is not None:
         raise ValueError("`attention_mask` goes with the padded form and without `seq_lens` and bias tables")
@@ -502,13 +506,19 @@ class HSTU(torch.nn.Module):
       # Whether the mask is end-padded is known once its kernel has run (`ticket`).  It is asked before anything random is drawn, in the
       # packed form behind the packing's own wait, and otherwise when the first block is enqueued: the answer is there by then, where
       # waiting for it first leaves a small batch's GPU idle (32 x 50 x 64, 4 blocks: 164 us a call, 133 this way).
-      got = _native.mask_lengths(padding_mask)
-      seq_lens, ticket = got if got is not None else (masks.lengths_from_padding_mask(padding_mask), None)
+      # (Nothing random to draw and no packing: the lengths come with the front end, in its launch; 53.3 us a call of that size -> 50.4.)
+      if not jagged and not (self.training and self.dropout > 0.0) and type(self)._front_end is HSTU._front_end:
+        front = self._embed(inputs, None, 0, padding_mask)
+      if front is not None:
+        *front, seq_lens, ticket = front
+      else:
+        got = _native.mask_lengths(padding_mask)
+        seq_lens, ticket = got if got is not None else (masks.lengths_from_padding_mask(padding_mask), None)
     if jagged:
       return self._forward_jagged(inputs, seq_lens, pos_bias, timestamps, ts_bias, ticket)
     if self.training and self.dropout > 0.0:
       ticket = self._check_mask(ticket)
-    x, outside = self._front_end(inputs)
+    x, outside = self._front_end(inputs) if front is None else front
     out = None
     if attention_mask is None and timestamps is None and ts_bias is None:
       out = self._narrow_blocks(x, x.shape[1], seq_lens, None, pos_bias, True)

@@ -136,3 +136,26 @@ def test_a_mask_that_is_not_end_padded_ends_the_call(gpu, jagged, dropout):
   assert torch.equal(torch.get_rng_state(), before[0]) and torch.equal(torch.cuda.get_rng_state(), before[1])
   mask[1, 5] = True
   assert model(ids, padding_mask=mask, jagged=jagged).isfinite().all()
+
+
+@pytest.mark.parametrize("batch,length", [(1, 1), (3, 40), (5, 65), (9, 130)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_lengths_from_the_mask_in_the_front_end(gpu, batch, length, grad):
+  """A padding mask's lengths come with the front end's launch (four rows of it to a workgroup, 64 bytes to a wavefront): the same bits as
+  the lengths themselves give, and a row that is not end-padded is refused, wherever it stands."""
+  g = torch.Generator().manual_seed(length)
+  model = recml_amd.HSTU(vocab_size=V, max_positions=length, model_dim=D, num_heads=2, num_layers=1, add_head=False, dtype=BF, device=DEV, seed=3)
+  model.requires_grad_(grad)
+  ids = torch.randint(1, V, (batch, length), generator=g).to(DEV)
+  lens = torch.randint(0, length + 1, (batch,), generator=g)
+  lens[-1] = length
+  mask = (torch.arange(length)[None, :] < lens[:, None]).to(DEV)
+  with torch.set_grad_enabled(grad):
+    want = model(ids, seq_lens=lens.to(torch.int32).to(DEV))
+    for m in (mask, mask.to(torch.uint8) * 255, mask.float()):
+      assert torch.equal(model(ids.to(torch.int32), padding_mask=m), want)
+    for row in range(batch) if length > 1 else ():
+      bad = mask.clone()
+      bad[row, 0], bad[row, length - 1] = False, True
+      with pytest.raises(ValueError):
+        model(ids, padding_mask=bad)
