@@ -4729,8 +4729,10 @@ void hstu_bwd_dkv_mfma(const Params p) {
   // A block whose vector part stands between the products that do not wait for it: the activation beside dP's, the tables' gradients
   // beside the accumulating ones.  (B = 64, L = 2048, H = 8, d = 128 with DSO, both backward kernels: both tables 3164 us with neither, 3103
   // with both, power-law lengths 235 and 225; with the position table alone or none 2370 -> 2360, 2187 -> 2170.  Fragments two products
-  // ahead instead of three: 3156, 228.)
-  constexpr bool WOVEN = WIDE || DSO;
+  // ahead instead of three: 3156, 228.)  Without DSO where it is the faster order: heads of 64 without a table, the call for 64 x 2048 1401 -> 1354 us,
+  // 128 x up to 1024 470 -> 454, with segment ids 965 -> 895; heads of 32 with both tables, 64 x 2048 1998 -> 1832, 192 x up to 1024 942 -> 867.
+  // (Heads of 64 with the position table 496 and 496, of 32 with timestamps alone 716 and 741.)
+  constexpr bool WOVEN = WIDE || DSO || (!MSK && !DB && ((D == 64 && !POS && !TS) || (D == 32 && POS && TS)));
   constexpr int AHEAD_R = D / 16 < 3 ? D / 16 : 3, AHEAD_T = 3;      // products that the fragments of rows / of transposed rows are asked for ahead
   // A pair of blocks that needs no mask runs as one hand-scheduled instruction stream (hstu_bwd_stream_d128.inc,
   // written by gen_bwd_stream.py): the vector part of one block behind the matrix instructions of the other.

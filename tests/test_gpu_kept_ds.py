@@ -48,6 +48,8 @@ _FORMS = [
     (64, 3, 260, 2, None, dict(seg=1)),
     (32, 5, 420, 2, [420, 129, 33, 1, 256], dict(jagged=1, ts=1)),
     (32, 2, 333, 1, None, dict(pos=1, ts=1, sliding_window_size=50)),
+    (64, 4, 300, 4, [300, 129, 33, 1], dict(jagged=1)),                                     # the order of the kept form on both sides
+    (32, 4, 300, 4, [300, 129, 33, 1], dict(jagged=1, pos=1, ts=1)),
 ]
 
 
