@@ -4698,7 +4698,7 @@ struct DkvShape {
   static constexpr int KV_BYTES = WIDE ? 2 * BM * D * 2 : 0;   // K and V rows of the tile
   static constexpr int KV_LDS = KV_BYTES + (WIDE ? 240 : 0);   // and what brings them to a multiple of 256 bytes (from one of 16)
 };
-// Table gradients in this kernel (DSO), as in the dQ kernel with keys and queries exchanged: rings of diagonal sums, TG_COPIES sums per
+// Table gradients in this kernel (DSO, TG), as in the dQ kernel with keys and queries exchanged: rings of diagonal sums, TG_COPIES sums per
 // bucket.  WIDE: a wave takes every other step, so the diagonals that a block shares with the next one go to the ring at once (the
 // next block is another wave's), and four rings keep the eight waves of a pair of steps apart.
 template <bool WIDE>
@@ -4719,7 +4719,7 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
 // regard to the other waves, and the workgroup's LDS falls from 112 to 76 KB at d = 64, two workgroups per CU (16 x up to 1000, 8 heads of
 // 64, mask and bias: the kernel 108 -> 92 us).
 // The bias's gradient is the other kernel's business.
-template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false>
+template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false, bool TG = false>
 __global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), (D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO) ? 1 : 2))
 void hstu_bwd_dkv_mfma(const Params p) {
   constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO);
@@ -4771,9 +4771,10 @@ void hstu_bwd_dkv_mfma(const Params p) {
   // WIDE: [K | V], 128 rows each, swizzled like the tiles (and on a line of its own: an exclusive or with an address touches bits 4 to 7)
   constexpr int KV_OFF = (BIAS_OFF + NST * BIAS_STAGE + (TS ? SM::TAB_BYTES : 0) + (WIDE ? 255 : 0)) & (WIDE ? ~255 : ~0);
   unsigned char* const KvLds = smem + KV_OFF;
-  float* const TgBase = (float*)(KvLds + SH::KV_BYTES);               // DSO with a table: rings of diagonal sums, then the bucket sums
+  float* const TgBase = (float*)(KvLds + SH::KV_BYTES);               // TG: rings of diagonal sums, then the bucket sums
   constexpr int RINGS = DkvTg<WIDE>::RINGS;
-  constexpr bool DPOS = DSO && POS, DTS = DSO && TS;
+  static_assert(!TG || (DSO && (POS || TS)), "the tables' gradients are formed where dS is handed on");
+  constexpr bool DPOS = TG && POS, DTS = TG && TS;
   const bool want_dpos = DPOS && p.dpos != nullptr, want_dts = DTS && p.dts != nullptr;
 
   Work wk;
@@ -5051,8 +5052,8 @@ void hstu_bwd_dkv_mfma(const Params p) {
   const int vc2 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
   const int c_lo = vc2 ^ hh, c_hi = vc2 ^ (hh + 2);
 
-  // DSO: this wave's blocks of dS, and (timestamp table) the lane's bucket of the last block with what is summed for it, (position table)
-  // the diagonals that the wave's next block finishes
+  // DSO: this wave's blocks of dS, and (TG) the lane's bucket of the last block with what is summed for it, the diagonals that the wave's
+  // next block finishes
   unsigned char* const dsg = DSO ? ds_blocks(p, b, h, s) : nullptr;
   int sum_bucket = 0;
   float sum_s = 0.f;
@@ -6533,14 +6534,16 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
 }
 
 // With the logits' gradients kept between them (q.ds): dK/dV, the tables' gradients and dS, then dQ.
-template <int D, bool POS, bool TS, bool SEG, bool MSK = false, bool DB = false>
+// TG: a table's gradient is wanted.  Without one (frozen tables) an instance that neither sums nor has the rings: us, 64 x up to 2048 of
+// power-law length, eight heads, both tables: d = 128 396 -> 377, d = 64 290 -> 266, d = 32 256 -> 240; 128 x up to 1024, d = 64 626 -> 571.
+template <int D, bool POS, bool TS, bool TG, bool SEG, bool MSK = false, bool DB = false>
 int launch_bwd_kept(const Params& p, hipStream_t st) {
   constexpr bool wide = dkv_wide(D, POS, TS, SEG, MSK, DB, true);
   using SH = DkvShape<D, wide>;
   constexpr int nst = dkv_stages(D, DB, wide);
   const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + dkv_dense_bytes<D>(MSK, DB, nst) +
-                      SH::KV_LDS + (TS ? nst * 16 : 0) + (POS || TS ? DkvTg<wide>::BYTES : 0);
-  const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, true>;
+                      SH::KV_LDS + (TS ? nst * 16 : 0) + (TG ? DkvTg<wide>::BYTES : 0);
+  const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, true, TG>;
   const auto dq = hstu_bwd_dq_ds<D, MSK>;
   static int granted_q[64], granted_kv[64];
   if (int rc = allow_lds((const void*)kv, smem_kv, granted_kv)) return rc;
@@ -6558,15 +6561,14 @@ int launch_bwd_kept(const Params& p, hipStream_t st) {
 
 template <int D, bool SEG>
 int launch_bwd_mfma_ds(const Params& q, hipStream_t st) {
-  if (q.ds) {
-    const bool pos = q.pos_tab != nullptr, ts = q.ts_tab != nullptr;
-    if (pos && ts) return launch_bwd_kept<D, true, true, SEG>(q, st);
-    if (pos) return launch_bwd_kept<D, true, false, SEG>(q, st);
-    if (ts) return launch_bwd_kept<D, false, true, SEG>(q, st);
-    return launch_bwd_kept<D, false, false, SEG>(q, st);
-  }
   const bool pos = q.pos_tab != nullptr, ts = q.ts_tab != nullptr;
   const bool tg = (pos && q.dpos) || (ts && q.dts);
+  if (q.ds) {
+    if (pos && ts) return tg ? launch_bwd_kept<D, true, true, true, SEG>(q, st) : launch_bwd_kept<D, true, true, false, SEG>(q, st);
+    if (pos) return tg ? launch_bwd_kept<D, true, false, true, SEG>(q, st) : launch_bwd_kept<D, true, false, false, SEG>(q, st);
+    if (ts) return tg ? launch_bwd_kept<D, false, true, true, SEG>(q, st) : launch_bwd_kept<D, false, true, false, SEG>(q, st);
+    return launch_bwd_kept<D, false, false, false, SEG>(q, st);
+  }
   if (pos && ts) return tg ? launch_bwd_mfma_inst<D, true, true, true, SEG>(q, st) : launch_bwd_mfma_inst<D, true, true, false, SEG>(q, st);
   if (pos) return tg ? launch_bwd_mfma_inst<D, true, false, true, SEG>(q, st) : launch_bwd_mfma_inst<D, true, false, false, SEG>(q, st);
   if (ts) return tg ? launch_bwd_mfma_inst<D, false, true, true, SEG>(q, st) : launch_bwd_mfma_inst<D, false, true, false, SEG>(q, st);
@@ -6606,9 +6608,9 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
     q.dbias = nullptr;
   }
   if (q.ds && !q.dbias) {
-    if (q.mask && q.dense_bias) return launch_bwd_kept<D, false, false, false, true, true>(q, st);
-    if (q.dense_bias) return launch_bwd_kept<D, false, false, false, false, true>(q, st);
-    if (q.mask) return launch_bwd_kept<D, false, false, false, true>(q, st);
+    if (q.mask && q.dense_bias) return launch_bwd_kept<D, false, false, false, false, true, true>(q, st);
+    if (q.dense_bias) return launch_bwd_kept<D, false, false, false, false, false, true>(q, st);
+    if (q.mask) return launch_bwd_kept<D, false, false, false, false, true>(q, st);
   }
   if (q.mask && q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, true, true>(q, st);
   if (q.dense_bias) return launch_bwd_mfma_inst<D, false, false, false, false, false, true>(q, st);

@@ -53,6 +53,22 @@ _FORMS = [
 ]
 
 
+@pytest.mark.parametrize("d", [128, 64, 32])
+@pytest.mark.parametrize("form", [dict(jagged=1, pos=1, ts=1), dict(jagged=1, ts=1), dict(pos=1), dict(jagged=1, pos=1, ts=1, dropout_p=0.3, dropout_seed=5),
+                                  dict(pos=1, ts=1, sliding_window_size=70), dict(pos=1, causal=False)])
+def test_frozen_tables(gpu, monkeypatch, d, form):
+  """No table's gradient wanted: an instance without the sums for them, and the same bits of dq, dk and dv."""
+  opt = dict(form)
+  form = {x: opt.pop(x, 0) for x in ("jagged", "pos", "ts", "seg")}
+  q, k, v, do, kw = _case(torch.bfloat16, d, 420, 4, [420, 129, 33, 1, 0, 256], B=6, **form)
+  kw.update(opt)
+  want = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  got = recml_amd.hstu_attention_bwd(q, k, v, do, table_grads=False, **kw)
+  assert got[3] is None and got[4] is None
+  for name, x, y in zip(("dq", "dk", "dv"), got, want):
+    assert torch.equal(x, y), name
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("d,B,L,H,lens,opt", _FORMS)
 def test_kept_and_formed_twice_agree(gpu, monkeypatch, dtype, d, B, L, H, lens, opt):
