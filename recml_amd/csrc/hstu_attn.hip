@@ -51,6 +51,7 @@
 
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <algorithm>
 #include <stdarg.h>
 #include <stdint.h>
 #include <utility>
@@ -6618,33 +6619,44 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
   return q.mask_mode == HSTU_MASK_SEGMENT ? launch_bwd_mfma_ds<D, true>(q, st) : launch_bwd_mfma_ds<D, false>(q, st);
 }
 
+// Pairs of one head that the index rules keep in a batch, as far as shapes and options say (the lengths are the device's): equal lengths in the
+// padded layout, and in the jagged one lengths of mean m whose mean square is halfway between m m and m L, what they have when none is
+// longer than L.  (Against U{L/8 .. L} and a power law of exponent 1.2 from 16, 16 to 128 sequences of up to 256 to 4096: 5 % low to 21 %
+// high.  By m m alone the power law's batches came out at less than half of what they are.)
+double likely_pairs(const HstuAttnFwdArgs* a) {
+  const bool jagged = a->layout == HSTU_LAYOUT_JAGGED;
+  const double mean = jagged && a->B > 0 ? std::min((double)a->total_tokens / a->B, (double)a->L) : (double)a->L;
+  const double square = 0.5 * mean * (mean + a->L);
+  return (double)a->B * (a->causal ? 0.5 * square + 16.0 * mean : square);        // (whole blocks of 32 x 32 on the diagonal)
+}
+
 // Bytes for the blocks of dS of a matrix-core backward call (see ds_blocks for the layout), 0 where each kernel forms dS for itself.  Kept, S,
 // dP and the activation are computed once instead of twice; what it costs is 2 bytes a pair and head written and read: for d = 128 always
 // less, for shorter rows only while the memory-side cache has them or both tables make the vector part long.  us, formed twice -> kept
-// (tables: none, position, timestamps, both):
-//   d = 128: 64 x 2048 2500 -> 2170, 2640 -> 2360, -, 3540 -> 3103 (2.2 GB of dS); 64 x up to 2048 of power-law length, both 260 -> 225;
+// (tables: none, position, timestamps, both; a table's gradient wanted; MB of dS):
+//   d = 128: 64 x 2048 2500 -> 2170, 2640 -> 2360, -, 3540 -> 3103 (2200 MB); 64 x up to 2048 of power-law length, both 536 -> 456;
 //            128 x 512 position 300 -> 264; 1 x 2048, two heads 154 -> 114; 2 x 4096 both 481 -> 384
-//   d = 64:  128 x up to 1024 (0.43 GB) 413 -> 403, 457 -> 464, 636 -> 624, 758 -> 665; half as many (0.21 GB) 170 -> 184, 207 -> 218; a
-//            quarter, position 123 -> 116; 32 x up to 512, four heads 38 -> 34, 48 -> 43, 81 -> 68, 88 -> 75; 64 x up to 2048 of power-law
-//            length (0.09 GB) 104 -> 109 and 116 -> 114, 134 -> 122, 193 -> 168, 207 -> 182
-//   d = 32:  128 x up to 1024 262 -> 315, 302 -> 356, 437 -> 467, 575 -> 597; 32 x up to 512 32 -> 31, 41 -> 42, 73 -> 65, 79 -> 70; 64 x up to
-//            2048 93 -> 99, 113 -> 111, 173 -> 164, 189 -> 174
+//   d = 64, eight heads:  32 x up to 512, four heads (20) 39 -> 36, 45 -> 40, 84 -> 68, 88 -> 75; 128 x up to 256 (38) 72 -> 67, 81 -> 76, 113 -> 96,
+//            126 -> 99; 64 x up to 500 (66) 81 -> 76; 128 x up to 500 (128) 137 -> 153, 158 -> 172, 249 -> 240, 300 -> 260; 32 x up to 1024 (147)
+//            117 -> 121, 138 -> 135, 213 -> 194, 247 -> 213; 48 x (207) -, 182 -> 204, 279 -> 278, 341 -> 303; power-law lengths, 64 x up to 2048
+//            (268) 188 -> 208, 215 -> 237, 311 -> 312, 376 -> 341; 16 x up to 4096 (280) -, 237 -> 231, 330 -> 307, 365 -> 336; 128 x up to
+//            2048 (340) -, 276 -> 310, 410 -> 410, 493 -> 447
+//   d = 32:  32 x up to 512, four heads (20) -, 38 -> 36, 64 -> 54, 67 -> 56; 128 x up to 500 (128) -, 122 -> 124, 206 -> 191, 238 (its older
+//            order) -> 230; 32 x up to 1024 (147) -, 110 -> 111, 176 -> 168, 203 -> 200; 48 x (207) -, 143 -> 149, 214 -> 219, 271 -> 272; 64 x up to 2048,
+//            power law (268) -, 170 -> 184, 248 -> 248, 303 -> 311
 // and with dense operands, which both kernels read, at every head dim (mask and bias, mask alone; eight heads, the bias's gradient left out):
 //   d = 128: 16 x up to 1000 310 -> 257, 206 -> 200; d = 64: 243 -> 173, 151 -> 132; d = 32: 214 -> 152, 120 -> 104; 16 x 2048, full, with the
 //            gradient 1422 -> 1282 and 1080 -> 907
-// The lengths stay on the device: a batch's bytes are taken to be those of equal lengths (of power-law ones 0.04 of the 0.09 GB above).
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
-constexpr size_t DS_CACHED_BYTES = (size_t)128 << 20;
 size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
   if (a->L != a->Lkv || (a->mask && (a->Lkv + BM - 1) / BM > MASK_PRES_MAX_KT)) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
   const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
   const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
-  const int64_t n = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens / (a->B > 0 ? a->B : 1) + 31) / 32 : nb;
-  const double likely = (double)a->B * a->H * DS_BLOCK * (a->causal ? n * (n + 1) / 2 : n * n);
-  const bool cached = likely <= (double)(a->pos_tab || a->ts_tab ? DS_CACHED_BYTES : DS_CACHED_BYTES / 4);
-  const bool pays = a->d_qk == 128 || (a->d_qk == 64 ? cached || a->dense_bias || a->mask || (a->pos_tab && a->ts_tab) : a->dense_bias || a->mask || (cached && a->ts_tab));
-  if (!pays || bytes > (double)DS_MAX_BYTES) return 0;
+  const double likely_mb = likely_pairs(a) * a->H * 2.0 / (1 << 20);
+  const bool dense = a->mask || a->dense_bias;
+  const double up_to_mb = a->d_qk == 128 || dense ? HUGE_VAL : a->d_qk == 64 ? (a->ts_tab ? (a->pos_tab ? HUGE_VAL : 288.0) : 96.0) : a->ts_tab ? 160.0 : 0.0;
+  if (likely_mb > up_to_mb || bytes > (double)DS_MAX_BYTES) return 0;
   if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
   return (size_t)(rows * row * DS_BLOCK) * a->H;
 }
