@@ -4711,6 +4711,15 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
   return d == 128 && !dense_bias && (pos || ts || seg || mask || dso);
 }
 
+// Forms in which, without DSO, the vector part stands between the products, us for the call: heads of 64 without a table, 64 x 2048
+// 1401 -> 1354, 128 x up to 1024 470 -> 454, with segment ids 965 -> 895; heads of 32 with both tables, 64 x 2048 1998 -> 1832, 192 x up to
+// 1024 942 -> 867.  (Heads of 64 with the position table 496 and 496, of 32 with timestamps alone 716 and 741; the others were not tried.)
+// It lengthens a step, though: calls whose longest tile ends last keep the other order.  4 x 2048, four heads of 64: 116 and 125; 2 x 8192,
+// two heads: 404 and 441; 16 x up to 4096 of power-law length, eight heads of 32 with both tables: 331 and 348.
+constexpr bool dkv_takes_turns(int d, bool pos, bool ts, bool mask, bool dense_bias) {
+  return !mask && !dense_bias && ((d == 64 && !pos && !ts) || (d == 32 && pos && ts));
+}
+
 // MSK: the dense keep-mask as in the other backward kernel; here a step's tile is 32 query rows x this workgroup's
 // 128 keys (wave w fetches rows 8w .. 8w + 7 of it, 128 bytes each), a lane reads the 16 bytes of its key's column,
 // and the workgroup finds the query steps in which the mask keeps one of its keys by one pass over its columns.
@@ -4720,7 +4729,7 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
 // regard to the other waves, and the workgroup's LDS falls from 112 to 76 KB at d = 64, two workgroups per CU (16 x up to 1000, 8 heads of
 // 64, mask and bias: the kernel 108 -> 92 us).
 // The bias's gradient is the other kernel's business.
-template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false, bool TG = false>
+template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false, bool TG = false, bool CHAIN = false>
 __global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), (D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO) ? 1 : 2))
 void hstu_bwd_dkv_mfma(const Params p) {
   constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO);
@@ -4730,10 +4739,9 @@ void hstu_bwd_dkv_mfma(const Params p) {
   // A block whose vector part stands between the products that do not wait for it: the activation beside dP's, the tables' gradients
   // beside the accumulating ones.  (B = 64, L = 2048, H = 8, d = 128 with DSO, both backward kernels: both tables 3164 us with neither, 3103
   // with both, power-law lengths 235 and 225; with the position table alone or none 2370 -> 2360, 2187 -> 2170.  Fragments two products
-  // ahead instead of three: 3156, 228.)  Without DSO where it is the faster order: heads of 64 without a table, the call for 64 x 2048 1401 -> 1354 us,
-  // 128 x up to 1024 470 -> 454, with segment ids 965 -> 895; heads of 32 with both tables, 64 x 2048 1998 -> 1832, 192 x up to 1024 942 -> 867.
-  // (Heads of 64 with the position table 496 and 496, of 32 with timestamps alone 716 and 741.)
-  constexpr bool WOVEN = WIDE || DSO || (!MSK && !DB && ((D == 64 && !POS && !TS) || (D == 32 && POS && TS)));
+  // ahead instead of three: 3156, 228.)  Without DSO where it is the faster order (dkv_takes_turns) and not the longest tile's chain of steps but
+  // the matrix cores bound the call (CHAIN: they do not, see chain_bound).
+  constexpr bool WOVEN = WIDE || DSO || (dkv_takes_turns(D, POS, TS, MSK, DB) && !CHAIN);
   constexpr int AHEAD_R = D / 16 < 3 ? D / 16 : 3, AHEAD_T = 3;      // products that the fragments of rows / of transposed rows are asked for ahead
   // A pair of blocks that needs no mask runs as one hand-scheduled instruction stream (hstu_bwd_stream_d128.inc,
   // written by gen_bwd_stream.py): the vector part of one block behind the matrix instructions of the other.
@@ -6520,15 +6528,19 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB, false));
   const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + dkv_dense_bytes<D>(MSK, DB, nst_kv) +
                       SH::KV_LDS + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
-  static int granted_q[64], granted_kv[64];
+  static int granted_q[64], granted_kv[2][64];
+  const bool chain = dkv_takes_turns(D, POS, TS, MSK, DB) && p.chain_bound;
+  void (*kv)(Params) = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>;
+  if constexpr (dkv_takes_turns(D, POS, TS, MSK, DB))
+    if (chain) kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, false, false, true>;
   if (int rc = allow_lds((const void*)hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>, smem_q, granted_q)) return rc;
-  if (int rc = allow_lds((const void*)hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>, smem_kv, granted_kv)) return rc;
+  if (int rc = allow_lds((const void*)kv, smem_kv, granted_kv[chain])) return rc;
   const long long blocks = mfma_grid(p);
   if (blocks > 0x7fffffffLL) return fail(HSTU_ERR_SHAPE, "grid too large");
   hipLaunchKernelGGL((hstu_bwd_dq_mfma<D, POS, TS, TG, SEG, MSK, DB>), dim3((unsigned)blocks), dim3(MFMA_THREADS), smem_q, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dq kernel launch: %s", hipGetErrorString(e));
-  hipLaunchKernelGGL((hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB>), dim3((unsigned)blocks), dim3(SH::THREADS), smem_kv, st, p);
+  hipLaunchKernelGGL(kv, dim3((unsigned)blocks), dim3(SH::THREADS), smem_kv, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(HSTU_ERR_LAUNCH, "backward dk/dv kernel launch: %s", hipGetErrorString(e));
   return HSTU_OK;
@@ -6630,6 +6642,13 @@ double likely_pairs(const HstuAttnFwdArgs* a) {
   return (double)a->B * (a->causal ? 0.5 * square + 16.0 * mean : square);        // (whole blocks of 32 x 32 on the diagonal)
 }
 
+// Whether a backward call lasts as long as its longest tile rather than as its work: what the 256 CUs' two workgroups each have to do is less
+// than 0.7 of the steps of a tile that meets every row.  (d = 64 without a table, dK/dV's two orders, see dkv_takes_turns, by that ratio: 0.25
+// + 8 to 9 %, 0.5 + 4 to 7 %, 0.66 + 5 %, 0.77 - 1 %, 0.85 - 6 %, 1.0 - 3 to 5 %.)
+bool chain_bound(const HstuAttnFwdArgs* a) {
+  return likely_pairs(a) * a->H / (BM * BN) / 512.0 < 0.7 * ((a->L + BN - 1) / BN);
+}
+
 // Bytes for the blocks of dS of a matrix-core backward call (see ds_blocks for the layout), 0 where each kernel forms dS for itself.  Kept, S,
 // dP and the activation are computed once instead of twice; what it costs is 2 bytes a pair and head written and read: for d = 128 always
 // less, for shorter rows only while the memory-side cache has them or both tables make the vector part long.  us, formed twice -> kept
@@ -6641,21 +6660,24 @@ double likely_pairs(const HstuAttnFwdArgs* a) {
 //            117 -> 121, 138 -> 135, 213 -> 194, 247 -> 213; 48 x (207) -, 182 -> 204, 279 -> 278, 341 -> 303; power-law lengths, 64 x up to 2048
 //            (268) 188 -> 208, 215 -> 237, 311 -> 312, 376 -> 341; 16 x up to 4096 (280) -, 237 -> 231, 330 -> 307, 365 -> 336; 128 x up to
 //            2048 (340) -, 276 -> 310, 410 -> 410, 493 -> 447
-//   d = 32:  32 x up to 512, four heads (20) -, 38 -> 36, 64 -> 54, 67 -> 56; 128 x up to 500 (128) -, 122 -> 124, 206 -> 191, 238 (its older
-//            order) -> 230; 32 x up to 1024 (147) -, 110 -> 111, 176 -> 168, 203 -> 200; 48 x (207) -, 143 -> 149, 214 -> 219, 271 -> 272; 64 x up to 2048,
-//            power law (268) -, 170 -> 184, 248 -> 248, 303 -> 311
+//   d = 32:  32 x up to 512, four heads (20) -, 38 -> 36, 64 -> 54, 67 -> 56; 128 x up to 500 (128) -, 122 -> 124, 206 -> 191, 224 -> 231; 16 x
+//            1024 (138) -, 100 -> 102, 142 -> 151, 165 -> 177; 32 x up to 1024 (147) -, 110 -> 111, 176 -> 168, 196 -> 199; 48 x (207) -, 143 ->
+//            149, 214 -> 219, 253 -> 272; 64 x up to 2048, power law (268) -, 170 -> 184, 248 -> 248, 285 -> 311
+//   and at d = 64 with a position table whose gradient is wanted, whatever the bytes, where the longest tile is what lasts (chain_bound): 16 x up to
+//            4096 as above; 4 x 4096, four heads (264) 266 -> 246; 16 x up to 4096, two heads 264 -> 254
 // and with dense operands, which both kernels read, at every head dim (mask and bias, mask alone; eight heads, the bias's gradient left out):
 //   d = 128: 16 x up to 1000 310 -> 257, 206 -> 200; d = 64: 243 -> 173, 151 -> 132; d = 32: 214 -> 152, 120 -> 104; 16 x 2048, full, with the
 //            gradient 1422 -> 1282 and 1080 -> 907
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
-size_t kept_ds_bytes(const HstuAttnFwdArgs* a, int64_t* per_head, int32_t* per_row) {
+size_t kept_ds_bytes(const HstuAttnFwdArgs* a, bool dpos, int64_t* per_head, int32_t* per_row) {
   if (a->L != a->Lkv || (a->mask && (a->Lkv + BM - 1) / BM > MASK_PRES_MAX_KT)) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
   const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
   const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
   const double likely_mb = likely_pairs(a) * a->H * 2.0 / (1 << 20);
   const bool dense = a->mask || a->dense_bias;
-  const double up_to_mb = a->d_qk == 128 || dense ? HUGE_VAL : a->d_qk == 64 ? (a->ts_tab ? (a->pos_tab ? HUGE_VAL : 288.0) : 96.0) : a->ts_tab ? 160.0 : 0.0;
+  const bool always = a->d_qk == 128 || dense || (a->d_qk == 64 && a->pos_tab && (a->ts_tab || (dpos && chain_bound(a))));
+  const double up_to_mb = always ? HUGE_VAL : a->d_qk == 64 ? (a->ts_tab ? 288.0 : 100.0) : a->ts_tab ? 131.0 : 0.0;
   if (likely_mb > up_to_mb || bytes > (double)DS_MAX_BYTES) return 0;
   if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
   return (size_t)(rows * row * DS_BLOCK) * a->H;
@@ -6673,8 +6695,9 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   // which share their keys through the cache.)
   q.level_tiles = ws.sched_bytes || (q.causal && (long long)q.B * q.n_qtiles * q.H <= 1024) ? 4 : 0;
   q.no_stream = (b->fwd.flags & HSTU_FWD_COMPILER_SCHEDULED_BLOCKS) ? 1 : 0;
+  q.chain_bound = chain_bound(&f) ? 1 : 0;
   if (int rc = setup_workspace(&f, ws, q, st)) return rc;
-  const size_t ds = kept_ds_bytes(&f, &q.ds_head, &q.ds_per_row), at = (ws.total() + 255) / 256 * 256;
+  const size_t ds = kept_ds_bytes(&f, q.dpos != nullptr, &q.ds_head, &q.ds_per_row), at = (ws.total() + 255) / 256 * 256;
   q.ds = ds && f.workspace && ((uintptr_t)f.workspace & 255u) == 0 && f.workspace_bytes >= at + ds ? (unsigned char*)f.workspace + at : nullptr;
   if (q.d_qk == 128) return launch_bwd_mfma_d<128>(q, st);
 #ifndef HSTU_ONLY_D128
@@ -6842,7 +6865,7 @@ size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args) {
   b.fwd.workspace_bytes = fwd;
   if (!bwd_mfma_eligible(&b)) return fwd;
   b.fwd.out = (void*)args->dout;
-  const size_t ds = kept_ds_bytes(&b.fwd, nullptr, nullptr);
+  const size_t ds = kept_ds_bytes(&b.fwd, args->dpos_tab != nullptr, nullptr, nullptr);
   if (!ds) return fwd;
   if (args->ddense_bias) {               // (added by the dQ kernel: that one forms dS)
     Params p = make_params(&b.fwd);

@@ -64,6 +64,7 @@ struct Params {
   const int32_t* mask_range; // workspace: per (mask batch, query tile) the first 32-key step with a kept pair and one past the last
   int32_t whole_window;      // forward: the position table as the caller gave it, no workspace (WHOLE instances)
   int32_t persist;           // forward: resident workgroups that loop over the work list
+  int32_t chain_bound;       // backward: its longest tile is what lasts (picks dK/dV's order of products)
   int32_t no_stream;         // forward: interior steps through the compiler-scheduled block code too (a comparison switch)
   int32_t mask_pres;         // the preparation also fills the dense mask's presence table (the backward asks for it)
   // Dropout on the attention weights: pair (b, h, i, j) is kept when drop_hash(...) >= drop_thr (0: no dropout).

@@ -44,9 +44,13 @@ def room_for_kept(b):
     # lengths of one mean: a batch of power-law lengths holds two to three times the pairs of one of equal lengths
     (64, 64, 2048, 350, "pos", False), (64, 128, 500, 281, "pos", False), (64, 128, 256, 144, "pos", True), (64, 64, 2048, 350, "", False),
     (64, 64, 2048, 350, "ts", True), (64, 64, 2048, 350, "pos ts", True), (64, 128, 2048, 290, "ts", False),
-    (32, 64, 2048, 350, "ts", False), (32, 64, 2048, 350, "pos ts", False), (32, 32, 1024, 580, "ts", True), (32, 32, 1024, 580, "pos", False),
+    (32, 64, 2048, 350, "ts", False), (32, 64, 2048, 350, "pos ts", False), (32, 128, 1024, 170, "ts", True), (32, 16, 1024, 1024, "ts", False), (32, 128, 1024, 170, "pos", False),
     (128, 64, 2048, 350, "", True), (128, 64, 2048, 350, "pos ts", True),
+    # one long sequence's tile lasts longer than a round of the chip
+    (64, 16, 4096, 900, "pos", True), (64, 16, 4096, 900, "pos frozen", False), (64, 16, 4096, 900, "", False), (32, 16, 4096, 900, "pos ts", False),
 ])
 def test_kept_by_the_bytes_that_a_batch_is_likely_to_have(d, B, L, mean, tables, kept):
   b = backward_args(B, L, 8, d, tokens=B * mean, pos="pos" in tables, ts="ts" in tables)
+  if "frozen" in tables:
+    b.dpos_tab = b.dts_tab = None
   assert (room_for_kept(b) > 0) == kept

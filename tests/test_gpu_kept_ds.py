@@ -53,6 +53,25 @@ _FORMS = [
 ]
 
 
+@pytest.mark.parametrize("d,form", [(64, {}), (64, dict(seg=1)), (64, dict(causal=False)), (64, dict(dropout_p=0.2, dropout_seed=3)), (32, dict(pos=1, ts=1)),
+                                    (32, dict(pos=1, ts=1, causal=False)), (32, dict(jagged=1, pos=1, ts=1, sliding_window_size=40))])
+@pytest.mark.parametrize("B,L,H", [(3, 420, 2), (100, 60, 24), (33, 100, 32)])
+def test_both_orders_of_products(gpu, monkeypatch, d, form, B, L, H):
+  """With dS formed twice the order of dK/dV's products and vector part goes by whether the longest tile or the work lasts longer (the first batch;
+  the other two): the same bits of all gradients as with the order of the kept form."""
+  opt = dict(form)
+  form = {x: opt.pop(x, 0) for x in ("jagged", "pos", "ts", "seg")}
+  rng = np.random.default_rng(B)
+  q, k, v, do, kw = _case(torch.bfloat16, d, L, H, None if form["seg"] else [L] + [int(x) for x in rng.integers(0, L + 1, B - 1)], B=B, **form)
+  kw.update(opt)
+  lib = _lib.load()
+  a = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  monkeypatch.setattr(lib, "hstu_attn_bwd_workspace_bytes", lambda args: lib.hstu_attn_fwd_workspace_bytes(C.byref(args._obj.fwd)))
+  b = recml_amd.hstu_attention_bwd(q, k, v, do, **kw)
+  for name, x, y in zip(("dq", "dk", "dv"), a, b):
+    assert torch.equal(x, y), name
+
+
 @pytest.mark.parametrize("d", [128, 64, 32])
 @pytest.mark.parametrize("form", [dict(jagged=1, pos=1, ts=1), dict(jagged=1, ts=1), dict(pos=1), dict(jagged=1, pos=1, ts=1, dropout_p=0.3, dropout_seed=5),
                                   dict(pos=1, ts=1, sliding_window_size=70), dict(pos=1, causal=False)])
