@@ -4664,16 +4664,16 @@ __device__ __forceinline__ void mfma_acc(floatx16& acc, bf16x8 a, bf16x8 b) {
 }
 
 // dS from the dK/dV kernel to the one that forms dQ from it: blocks of 32 query rows x 32 keys, rounded to bf16 as both kernels' products take
-// them, 2 KB each.  Block (i, j) of a (sequence, head) at slot i (i + 1) / 2 + j under the causal mask, else at i n + j; a sequence's slots
-// begin where `ds_per_row` for each 32 rows before it (an upper bound) end.  Within a block, by halves of 16 rows: 32 keys of 32 bytes, a
+// them, 2 KB each, a (sequence, head)'s in the slots of DsRows; a sequence's slots
+// begin where `per_row` for each 32 rows before it (an upper bound) end.  Within a block, by halves of 16 rows: 32 keys of 32 bytes, a
 // key's rows in the order 0 .. 3, 8 .. 11, 4 .. 7, 12 .. 15, which is how a lane of the dK/dV kernel holds them.
 constexpr int DS_BLOCK = 32 * 32 * 2;
 __device__ __forceinline__ unsigned char* ds_blocks(const Params& p, int b, int h, const Seq& s) {
   const int64_t rows = p.jagged ? (s.tok0 >> 5) + b : (int64_t)b * ((p.L + 31) >> 5);
-  return p.ds + (int64_t)h * p.ds_head + rows * p.ds_per_row * DS_BLOCK;
+  return p.ds + (int64_t)h * p.ds_head + rows * p.ds_rows.per_row * DS_BLOCK;
 }
 __device__ __forceinline__ uint32_t ds_block_off(const Params& p, int i, int j) {
-  return (uint32_t)(p.causal ? i * (i + 1) / 2 + j : i * p.ds_per_row + j) * (uint32_t)DS_BLOCK;
+  return (uint32_t)((p.ds_rows.step < 0 ? i * (i + 1) / 2 : i * p.ds_rows.step) + p.ds_rows.shift + j) * (uint32_t)DS_BLOCK;
 }
 
 // Ring depth of the dK/dV kernel (see there).
@@ -6632,21 +6632,29 @@ int launch_bwd_mfma_d(const Params& p, hipStream_t st) {
 }
 
 // Pairs of one head that the index rules keep in a batch, as far as shapes and options say (the lengths are the device's): equal lengths in the
-// padded layout, and in the jagged one lengths of mean m whose mean square is halfway between m m and m L, what they have when none is
-// longer than L.  (Against U{L/8 .. L} and a power law of exponent 1.2 from 16, 16 to 128 sequences of up to 256 to 4096: 5 % low to 21 %
-// high.  By m m alone the power law's batches came out at less than half of what they are.)
+// padded layout, and in the jagged one half of the tokens in sequences of the mean length m and half in ones of length L, which without a window
+// is a mean square halfway between m m and m L, what lengths have when none is longer than L.  (Against U{L/8 .. L} and a power law of exponent
+// 1.2 from 16, 16 to 128 sequences of up to 256 to 4096: 5 % low to 21 % high.  By m m alone the power law's batches came out at less
+// than half of what they are.)  Whole blocks of 32 x 32 on the diagonal and at the window's ends.
 double likely_pairs(const HstuAttnFwdArgs* a) {
   const bool jagged = a->layout == HSTU_LAYOUT_JAGGED;
   const double mean = jagged && a->B > 0 ? std::min((double)a->total_tokens / a->B, (double)a->L) : (double)a->L;
-  const double square = 0.5 * mean * (mean + a->L);
-  return (double)a->B * (a->causal ? 0.5 * square + 16.0 * mean : square);        // (whole blocks of 32 x 32 on the diagonal)
+  const int window = effective_window(a);
+  auto of_length = [&](double n) {
+    const double all = a->causal ? 0.5 * n * n + 16.0 * n : n * n, x = window + 1.0;
+    if (window < 0 || x >= n) return all;
+    const double side = n * x - 0.5 * x * x;
+    return std::min(all, (a->causal ? side : 2.0 * side - n) + 32.0 * n);
+  };
+  return 0.5 * a->B * (of_length(mean) + mean / a->L * of_length(a->L));
 }
 
 // Whether a backward call lasts as long as its longest tile rather than as its work: what the 256 CUs' two workgroups each have to do is less
-// than 0.7 of the steps of a tile that meets every row.  (d = 64 without a table, dK/dV's two orders, see dkv_takes_turns, by that ratio: 0.25
+// than 0.7 of the steps of a tile that meets every row (or those of its window).  (d = 64 without a table, dK/dV's two orders, see dkv_takes_turns, by that ratio: 0.25
 // + 8 to 9 %, 0.5 + 4 to 7 %, 0.66 + 5 %, 0.77 - 1 %, 0.85 - 6 %, 1.0 - 3 to 5 %.)
 bool chain_bound(const HstuAttnFwdArgs* a) {
-  return likely_pairs(a) * a->H / (BM * BN) / 512.0 < 0.7 * ((a->L + BN - 1) / BN);
+  const int window = effective_window(a), rows = window < 0 ? a->L : std::min((int64_t)a->L, BM + (int64_t)window * (a->causal ? 1 : 2));
+  return likely_pairs(a) * a->H / (BM * BN) / 512.0 < 0.7 * ((rows + BN - 1) / BN);
 }
 
 // Bytes for the blocks of dS of a matrix-core backward call (see ds_blocks for the layout), 0 where each kernel forms dS for itself.  Kept, S,
@@ -6668,19 +6676,22 @@ bool chain_bound(const HstuAttnFwdArgs* a) {
 // and with dense operands, which both kernels read, at every head dim (mask and bias, mask alone; eight heads, the bias's gradient left out):
 //   d = 128: 16 x up to 1000 310 -> 257, 206 -> 200; d = 64: 243 -> 173, 151 -> 132; d = 32: 214 -> 152, 120 -> 104; 16 x 2048, full, with the
 //            gradient 1422 -> 1282 and 1080 -> 907
+//   A sliding window's dS is its band, and so are the bytes (eight heads, window; none, position, timestamps, both): d = 128: 16 x 2048, 128,
+//            270 -> 194, 229 -> 206, 311 -> 275, 333 -> 288; 8 x 8192, 256 (0.3 GB) 652 -> 465; d = 64: 16 x 2048, 128, 105 -> 111, 124 -> 124, 206 ->
+//            188, 236 -> 200; 4 x 8192, 256, 137 -> 138, 161 -> 161, 258 -> 253, 306 -> 271; d = 32: 16 x 2048, 128, -, 97 -> 97, 155 -> 149, 182 -> 185
 // DS_MAX_BYTES bounds what a call's scratch may grow by (the largest above takes half of it).
-size_t kept_ds_bytes(const HstuAttnFwdArgs* a, bool dpos, int64_t* per_head, int32_t* per_row) {
+size_t kept_ds_bytes(const HstuAttnFwdArgs* a, bool dpos, int64_t* per_head, DsRows* in_head) {
   if (a->L != a->Lkv || (a->mask && (a->Lkv + BM - 1) / BM > MASK_PRES_MAX_KT)) return 0;
   const int64_t nb = (a->L + 31) / 32, rows = a->layout == HSTU_LAYOUT_JAGGED ? (a->total_tokens >> 5) + a->B : (int64_t)a->B * nb;
-  const int64_t row = a->causal ? (nb + 2) / 2 : nb;                 // nb (nb + 1) / 2 blocks or nb nb, by its nb rows
-  const double bytes = (double)rows * (double)row * DS_BLOCK * a->H;
+  const DsRows slots = ds_row_slots(nb, nb, a->causal != 0, a->causal != 0, effective_window(a), 32);
+  const double bytes = (double)rows * slots.per_row * DS_BLOCK * a->H;
   const double likely_mb = likely_pairs(a) * a->H * 2.0 / (1 << 20);
   const bool dense = a->mask || a->dense_bias;
   const bool always = a->d_qk == 128 || dense || (a->d_qk == 64 && a->pos_tab && (a->ts_tab || (dpos && chain_bound(a))));
   const double up_to_mb = always ? HUGE_VAL : a->d_qk == 64 ? (a->ts_tab ? 288.0 : 100.0) : a->ts_tab ? 131.0 : 0.0;
   if (likely_mb > up_to_mb || bytes > (double)DS_MAX_BYTES) return 0;
-  if (per_head) { *per_head = rows * row * DS_BLOCK; *per_row = (int32_t)row; }
-  return (size_t)(rows * row * DS_BLOCK) * a->H;
+  if (per_head) { *per_head = rows * slots.per_row * DS_BLOCK; *in_head = slots; }
+  return (size_t)(rows * slots.per_row * DS_BLOCK) * a->H;
 }
 
 int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
@@ -6697,7 +6708,7 @@ int launch_bwd_mfma(const HstuAttnBwdArgs* b, const Params& p, hipStream_t st) {
   q.no_stream = (b->fwd.flags & HSTU_FWD_COMPILER_SCHEDULED_BLOCKS) ? 1 : 0;
   q.chain_bound = chain_bound(&f) ? 1 : 0;
   if (int rc = setup_workspace(&f, ws, q, st)) return rc;
-  const size_t ds = kept_ds_bytes(&f, q.dpos != nullptr, &q.ds_head, &q.ds_per_row), at = (ws.total() + 255) / 256 * 256;
+  const size_t ds = kept_ds_bytes(&f, q.dpos != nullptr, &q.ds_head, &q.ds_rows), at = (ws.total() + 255) / 256 * 256;
   q.ds = ds && f.workspace && ((uintptr_t)f.workspace & 255u) == 0 && f.workspace_bytes >= at + ds ? (unsigned char*)f.workspace + at : nullptr;
   if (q.d_qk == 128) return launch_bwd_mfma_d<128>(q, st);
 #ifndef HSTU_ONLY_D128
@@ -6936,7 +6947,7 @@ static int backward_call(const HstuAttnBwdArgs* args, const void* q_pre, const v
   if (fresh)
     if (int rc2 = clear_floats(p.dbias, (int64_t)(p.dense_bias_batched ? p.B : 1) * p.L * p.Lkv, st)) return rc2;
   if (f->qk_dtype == HSTU_DTYPE_FP32 && f->workspace && ((uintptr_t)f->workspace & 255u) == 0 && f32_takes(p, false, true)) {
-    const size_t ds = f32_ds_bytes(p, f->total_tokens, &p.ds_head, &p.ds_per_row);
+    const size_t ds = f32_ds_bytes(p, f->total_tokens, &p.ds_head, &p.ds_rows);
     if (ds && f->workspace_bytes >= ds) p.ds = (unsigned char*)f->workspace;
   }
   return f->qk_dtype == HSTU_DTYPE_FP32 ? launch_bwd<float>(p, st) : launch_bwd<bf16_t>(p, st);

@@ -16,6 +16,12 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// Where the blocks of the logits' gradients of one (sequence, head) lie that a backward's kernels hand on: row i's block j at slot
+// i * step + shift + j, with step < 0 at i (i + 1) / 2 + j; `per_row` slots are allotted for each row of blocks.
+struct DsRows {
+  int32_t per_row, step, shift;
+};
+
 struct Params {
   const void* q;
   const void* k;
@@ -99,10 +105,10 @@ struct Params {
   float* dbias;              // gradient of the dense bias, or null
   int32_t dbias_fresh;       // it is written, not added to
   // The logits' gradients between the two kernels of a backward (null: each forms them for itself), see ds_blocks of either file: bytes
-  // from one head's blocks to the next, and block slots for each 32 (fp32: 16) rows of queries.
+  // from one head's blocks to the next, and where in it a block lies.
   unsigned char* ds;
   int64_t ds_head;
-  int32_t ds_per_row;
+  DsRows ds_rows;
   int64_t items_max;         // capacity of the list (sizes the grid)
 };
 
@@ -211,11 +217,25 @@ __attribute__((visibility("hidden"))) int bucket_thresholds(float bucket_size, c
 
 // What the logits' gradients that a backward's kernels hand on may take of its workspace.
 constexpr size_t DS_MAX_BYTES = (size_t)4 << 30;
+// Their slots where a sequence has up to nq x nk blocks of `size` rows and keys: those on and below the diagonal (triangle), all, or, where
+// that is fewer, the band that a window leaves, from ceil(window / size) blocks before the diagonal to as many behind it (causal: to the
+// diagonal itself).
+inline DsRows ds_row_slots(int64_t nq, int64_t nk, bool triangle, bool causal, int window, int size) {
+  DsRows r;
+  r.per_row = (int32_t)(triangle ? (nq + 2) / 2 : nk);              // nq (nq + 1) / 2 blocks by its nq rows
+  r.step = triangle ? -1 : r.per_row;
+  r.shift = 0;
+  if (window >= 0) {
+    const int64_t reach = ((int64_t)window + size - 1) / size, band = causal ? reach + 1 : 2 * reach + 1;
+    if (band < r.per_row) { r.per_row = (int32_t)band; r.step = (int32_t)band - 1; r.shift = (int32_t)reach; }
+  }
+  return r;
+}
 
 // (hstu_f32.hip) fp32 products at d_qk = d_v in {16, 32, 64, 128} (bf16 storage: 16).  Whether a call is theirs, and the launches.
 __attribute__((visibility("hidden"))) bool f32_takes(const Params& p, bool bf16, bool backward);
 __attribute__((visibility("hidden"))) int f32_launch_fwd(const Params& p, bool bf16, hipStream_t st);
-__attribute__((visibility("hidden"))) size_t f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, int32_t* per_row);
+__attribute__((visibility("hidden"))) size_t f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, DsRows* in_head);
 __attribute__((visibility("hidden"))) int f32_launch_bwd(const Params& p, bool bf16, hipStream_t st);
 
 }  // namespace hstu

@@ -834,16 +834,15 @@ __global__ __launch_bounds__(256, D >= 128 ? 2 : 3) void hstu_f32_dq(const Param
     store_row<T, D>((T*)p.dq + s.bq + (int64_t)qi * p.q_st, o, qi < s.n_q ? p.alpha : 0.f, g);
 }
 
-// dS from hstu_f32_dkv to hstu_f32_dq_ds: blocks of 16 keys x 16 query rows, a key's 16 rows next to each other, 1 KB each.  Block (i, j) of a
-// (sequence, head) at slot i (i + 1) / 2 + j where the causal mask meets one length, else at i n + j; a sequence's slots begin where
-// `ds_per_row` for each 16 rows before it (an upper bound) end.  A block without a kept pair is neither written nor read.
+// dS from hstu_f32_dkv to hstu_f32_dq_ds: blocks of 16 keys x 16 query rows, a key's 16 rows next to each other, 1 KB each, a
+// (sequence, head)'s in the slots of DsRows; a sequence's slots begin where `per_row` for each 16 rows before it (an upper bound) end.  A block without a kept pair is neither written nor read.
 constexpr int DS_BLOCK = 16 * 16;
 __device__ __forceinline__ float* ds_blocks(const Params& p, int b, int h, const Seq& s) {
   const int64_t rows = p.jagged ? (s.tok0 >> 4) + b : (int64_t)b * ((p.L + 15) >> 4);
-  return (float*)(p.ds + (int64_t)h * p.ds_head) + rows * p.ds_per_row * DS_BLOCK;
+  return (float*)(p.ds + (int64_t)h * p.ds_head) + rows * p.ds_rows.per_row * DS_BLOCK;
 }
 __device__ __forceinline__ int64_t ds_block_at(const Params& p, int i, int j) {
-  return (int64_t)(p.causal && p.L == p.Lkv ? i * (i + 1) / 2 + j : i * p.ds_per_row + j) * DS_BLOCK;
+  return (int64_t)((p.ds_rows.step < 0 ? i * (i + 1) / 2 : i * p.ds_rows.step) + p.ds_rows.shift + j) * DS_BLOCK;
 }
 
 // The rows of hstu_f32_dq with dS read (the bits it would form): one product of three, the bias gradients as there.  Steps of 32 keys: a tile
@@ -1132,14 +1131,16 @@ bool hstu::f32_takes(const Params& p, bool bf16, bool backward) {
 //            51 -> 41
 //   d = 64:  128 x 512 747 -> 609 (segment ids); 64 x 512 with the table 717 -> 603; 8 x 2048, both tables 1677 -> 1394; 16 x 256 52 -> 42
 //   d = 32:  128 x 512 654 -> 572; 8 x 2048, both tables 1173 -> 999; 16 x 256, four heads 36 -> 32; 32 x 128 and 4 x 64 27 -> 28
-// The last two are as long as their launches and the host's work: the line below leaves such calls (and head dims of 16) alone.
-size_t hstu::f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, int32_t* per_row) {
+//   a window's band, eight heads: 16 x 2048, window 256: d = 128 1163 -> 881, d = 64 590 -> 454, d = 32 317 -> 262; 8 x 256, four heads, window
+//            32: d = 128 38 -> 31, d = 64 27 -> 27
+// Those of 27 us are as long as their launches and the host's work: the line below leaves such calls (and head dims of 16) alone.
+size_t hstu::f32_ds_bytes(const Params& p, int64_t total_tokens, int64_t* per_head, DsRows* in_head) {
   const int64_t nq = (p.L + 15) / 16, nk = (p.Lkv + 15) / 16, rows = p.jagged ? (total_tokens >> 4) + p.B : (int64_t)p.B * nq;
-  const int64_t row = p.causal && p.L == p.Lkv ? (nq + 2) / 2 : nk;        // nq (nq + 1) / 2 blocks by its nq rows
-  const double bytes = (double)rows * (double)row * (4.0 * DS_BLOCK) * p.H;
+  const DsRows slots = ds_row_slots(nq, nk, p.causal && p.L == p.Lkv, p.causal != 0, p.window, 16);
+  const double bytes = (double)rows * slots.per_row * (4.0 * DS_BLOCK) * p.H;
   if (p.d_qk < 32 || bytes * p.d_qk < 2e8 || bytes > (double)DS_MAX_BYTES) return 0;
-  if (per_head) { *per_head = rows * row * (4 * DS_BLOCK); *per_row = (int32_t)row; }
-  return (size_t)(rows * row * (4 * DS_BLOCK)) * p.H;
+  if (per_head) { *per_head = rows * slots.per_row * (4 * DS_BLOCK); *in_head = slots; }
+  return (size_t)(rows * slots.per_row * (4 * DS_BLOCK)) * p.H;
 }
 int hstu::f32_launch_fwd(const Params& p, bool bf16, hipStream_t st) { return launch(p, bf16, false, st); }
 int hstu::f32_launch_bwd(const Params& p, bool bf16, hipStream_t st) { return launch(p, bf16, true, st); }

@@ -54,3 +54,27 @@ def test_kept_by_the_bytes_that_a_batch_is_likely_to_have(d, B, L, mean, tables,
   if "frozen" in tables:
     b.dpos_tab = b.dts_tab = None
   assert (room_for_kept(b) > 0) == kept
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,L,H,window", [(7, 8192, 8, 256), (24, 8192, 8, 256), (2, 4096, 8, 0), (16, 2048, 8, 31), (16, 2048, 8, 32), (16, 2048, 8, 33), (4, 1000, 8, 100)])
+def test_a_window_takes_its_band(B, L, H, window, causal, fp32):
+  """Blocks that a sliding window leaves have a slot, not all below the diagonal: a long windowed call stays far below the 4 GiB that are the most."""
+  size, block = (16, 1024) if fp32 else (32, 2048)
+  n, reach = -(-L // size), -(-window // size)
+  band = (reach + 1 if causal else 2 * reach + 1) * n * B * H * block
+  b = backward_args(B, L, H, 128, causal=causal, window=window, fp32=fp32, pos=not fp32)
+  least = _lib.load().hstu_attn_fwd_workspace_bytes(C.byref(b.fwd))
+  assert band <= least + room_for_kept(b) <= band + least + 512
+  # a window as wide as the triangle or the square needs no more than they do
+  whole = room_for_kept(backward_args(1, 512, H, 128, causal=causal, fp32=fp32))
+  assert room_for_kept(backward_args(1, 512, H, 128, causal=causal, window=500, fp32=fp32)) == whole > 0
+
+
+def test_a_window_leaves_the_cached_head_dims_their_band():
+  """Heads of 64 and 32 hand dS on while a likely batch's fit the caches: with a window that is its band."""
+  for d in (64, 32):
+    assert room_for_kept(backward_args(16, 2048, 8, d, tokens=16 * 2048, ts=True)) == 0 or d == 64
+    assert room_for_kept(backward_args(32, 2048, 8, d, tokens=32 * 2048, ts=True)) == 0
+    assert room_for_kept(backward_args(32, 2048, 8, d, tokens=32 * 2048, ts=True, window=64)) > 0

@@ -41,6 +41,10 @@ _FORMS = [
     (128, 3, 300, 3, [300, 128, 5], dict(ts=1, causal=False)),                              # rectangular blocks, no list
     (128, 2, 400, 2, [400, 333], dict(pos=1, sliding_window_size=37)),
     (128, 2, 400, 2, None, dict(causal=False, sliding_window_size=150)),
+    (128, 2, 333, 2, [333, 290], dict(sliding_window_size=0)),                               # bands of one block a row and of two, a row more than the last
+    (128, 3, 333, 2, [333, 64, 33], dict(jagged=1, pos=1, ts=1, sliding_window_size=31)),
+    (64, 3, 420, 2, [420, 97, 300], dict(jagged=1, pos=1, sliding_window_size=32, causal=False)),
+    (64, 2, 420, 2, [420, 333], dict(pos=1, ts=1, sliding_window_size=33)),
     (128, 3, 260, 2, None, dict(seg=1)),
     (128, 3, 300, 2, [300, 200, 64], dict(jagged=1, pos=1, ts=1, dropout_p=0.3, dropout_seed=7)),
     (64, 5, 420, 8, [420, 129, 33, 1, 256], dict(jagged=1, pos=1, ts=1)),
@@ -92,7 +96,7 @@ def test_frozen_tables(gpu, monkeypatch, d, form):
 @pytest.mark.parametrize("d,B,L,H,lens,opt", _FORMS)
 def test_kept_and_formed_twice_agree(gpu, monkeypatch, dtype, d, B, L, H, lens, opt):
   if dtype == torch.float32:
-    H *= 16          # (small fp32 calls keep nothing)
+    H *= 64 if "sliding_window_size" in opt else 16          # (small fp32 calls keep nothing: below 2e8 bytes of blocks times the head dim)
   opt = dict(opt)
   form = {x: opt.pop(x, 0) for x in ("jagged", "pos", "ts", "seg")}
   q, k, v, do, kw = _case(dtype, d, L, H, lens, B=B, **form)
