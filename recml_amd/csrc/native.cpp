@@ -749,7 +749,6 @@ struct BlockBackward : public torch::autograd::Node {
       b.struct_size = sizeof(b);
       b.version = HSTU_ATTN_ABI_VERSION;
       TORCH_CHECK(fill(b.fwd, q, k, v, d_attn, pt, tt, Tensor(), call.opts), "the block's attention does not fit its own backward");
-      const Tensor scratch = scratch_for(b, q);
       b.dout = d_attn.const_data_ptr();
       b.dq = projection_slice(d_uqkv, call, 1).data_ptr();
       b.dk = projection_slice(d_uqkv, call, 2).data_ptr();
@@ -762,6 +761,7 @@ struct BlockBackward : public torch::autograd::Node {
         if (has_pos) { dpos = both.as_strided(pt.sizes(), pt.strides(), 0); b.dpos_tab = dpos.data_ptr<float>(); }
         if (has_ts) { dts = both.as_strided(tt.sizes(), tt.strides(), np); b.dts_tab = dts.data_ptr<float>(); }
       }
+      const Tensor scratch = scratch_for(b, q);       // (goes by the gradients that are wanted, too)
       // (through the projections' activation on the way, where those kernels run)
       through_silu = w.projections && !strcmp(hstu_attn_bwd_variant(&b), "hstu_bwd_mfma_bf16");
       const int rc = through_silu ? hstu_attn_bwd_silu(&b, at_column(pre, W), at_column(pre, 2 * W), at_column(pre, 3 * W), stream_of(q))
