@@ -257,7 +257,11 @@ Tensor scratch_for(HstuAttnBwdArgs& b, const Tensor& like) {
   try {
     buf = at::empty({(int64_t)ws}, like.options().dtype(at::kByte).requires_grad(false));
   } catch (const c10::OutOfMemoryError&) {
-    return scratch_for(b.fwd, like);
+    const uint32_t flags = b.fwd.flags;
+    b.fwd.flags &= ~HSTU_BWD_WRITE_BIAS_GRADIENT;       // (the forward's question knows no flag of the backward's)
+    buf = scratch_for(b.fwd, like);
+    b.fwd.flags = flags;
+    return buf;
   }
   b.fwd.workspace = buf.data_ptr();
   b.fwd.workspace_bytes = ws;

@@ -549,8 +549,11 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
       buf = torch.empty(best, dtype=torch.uint8, device=q.device)
       ba.fwd.workspace, ba.fwd.workspace_bytes = buf.data_ptr(), best
       keep.append(buf)
-    except torch.OutOfMemoryError:     # (less than the best will do)
-      _attach_workspace(ba.fwd, keep)
+    except torch.OutOfMemoryError:     # (less than the best will do; the forward's question knows no flag of the backward's)
+      fa = ba.fwd
+      flags, fa.flags = fa.flags, fa.flags & ~_lib.BWD_WRITE_BIAS_GRADIENT
+      _attach_workspace(fa, keep)
+      fa.flags = flags
   if _variant_out is not None:
     _variant_out.append(lib.hstu_attn_bwd_variant(C.byref(ba)).decode())
   with torch.cuda.device(q.device):

@@ -6,6 +6,69 @@ import torch
 import recml_amd
 
 pytestmark = pytest.mark.gpu
+MB = 1 << 20
+
+
+@pytest.fixture
+def share():
+  """Leaves the process so many bytes beyond those it has; the whole device again afterwards."""
+  total = torch.cuda.get_device_properties(0).total_memory
+
+  def leave(n):
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + n) / total)
+
+  yield leave
+  torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def _inputs(B, L, H=8, d=128, dense=False):
+  g = torch.Generator(device="cuda").manual_seed(L)
+  t = [torch.randn(B, L, H, d, device="cuda", generator=g).mul_(0.5).to(torch.bfloat16) for _ in range(4)]
+  bias = torch.randn((B, L, L) if dense else (H, 2 * L - 1), device="cuda", generator=g) * 0.3
+  return t, dict(bias=bias, n=float(L)) if dense else dict(pos_bias=bias)
+
+
+def _gradients(t, kw, native):
+  """dq, dk, dv and the bias's, by the call's autograd node or by the backward's own entry."""
+  q, k, v, do = t
+  if not native:
+    got = recml_amd.hstu_attention_bwd(q, k, v, do, **kw, bias_grad="bias" in kw)
+    return *got[:3], got[5 if "bias" in kw else 3]
+  wrt = [x.detach().requires_grad_() for x in (q, k, v)]
+  name = next(iter(kw))
+  kw = {**kw, name: kw[name].detach().requires_grad_()}
+  out = recml_amd.hstu_attention_autograd(*wrt, **kw)
+  assert out.grad_fn.name() == "HstuAttentionBackward"
+  return torch.autograd.grad(out, (*wrt, kw[name]), do)
+
+
+def _same(a, b):
+  for x, y in zip(a[:3], b[:3]):
+    assert torch.equal(x, y)
+  # (fp32 sums of the same terms in another order, as where the two forms of the backward are compared)
+  assert float((a[3] - b[3]).abs().max()) <= 1e-4 * float(b[3].abs().max())
+
+
+def _failed():
+  s = torch.cuda.memory_stats()
+  return s["num_alloc_retries"], s["num_ooms"]
+
+
+@pytest.mark.parametrize("native,dense,left", [(True, False, 78), (False, False, 62), (True, True, 96), (False, True, 82)])
+def test_an_allocation_that_fails(gpu, share, native, dense, left):
+  """The call goes on without what there is no memory for, also with a dense bias's gradient (a flag of the backward's): 14 MB for each of dq, dk,
+  dv (and the output), 20 for the bias's gradient, and the 38 or so of dS do not fit."""
+  t, kw = _inputs(8, 768, dense=dense)
+  want = _gradients(t, kw, native)
+  share(left * MB)
+  before = _failed()
+  got = _gradients(t, kw, native)
+  torch.cuda.synchronize()
+  assert _failed()[1] == before[1] + 1
+  torch.cuda.set_per_process_memory_fraction(1.0)
+  _same(got, want)
 
 
 @pytest.mark.parametrize("wanted", [True, False])
