@@ -55,5 +55,5 @@ def _first_call(name):
   return call
 
 
-_FUNCTIONS = ("attention", "block", "blocks", "embed", "final_norm", "linear", "pack", "mask_lengths", "raised", "norm_gate_bwd")
-attention, block, blocks, embed, final_norm, linear, pack, mask_lengths, raised, norm_gate_bwd = (_first_call(n) for n in _FUNCTIONS)
+_FUNCTIONS = ("attention", "block", "blocks", "embed", "final_norm", "linear", "pack", "mask_lengths", "raised", "norm_gate_bwd", "has_room")
+attention, block, blocks, embed, final_norm, linear, pack, mask_lengths, raised, norm_gate_bwd, has_room = (_first_call(n) for n in _FUNCTIONS)

@@ -15,6 +15,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <hip/hip_runtime.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/edge.h>
 #include <torch/csrc/autograd/function.h>
@@ -249,14 +250,43 @@ Tensor scratch_for(HstuAttnFwdArgs& a, const Tensor& like) {
   return buf;
 }
 
-// The backward's: with room for what its kernels can hand on, or without it where the device has not that much left.
+// Whether the device has room for a buffer that a call can do without: in one piece among those that the caching allocator holds, or beside
+// them within the process's share.  One that has not makes the allocator wait for the device and give back all that it holds before it fails;
+// a training step near the memory's end would do so in every layer's backward.  (Buffers below 64 MB are simply asked for; so are those of
+// other allocators, which have no such cache.)
+bool has_room(c10::DeviceIndex device, size_t bytes) {
+  constexpr size_t SMALL = (size_t)64 << 20, GRAIN = (size_t)2 << 20;
+  if (bytes < SMALL) return true;
+  try {
+    auto* const allocator = c10::hip::HIPCachingAllocator::get();
+    if (allocator->name() != "native") return true;
+    size_t piece = 1;
+    allocator->cacheInfo(device, &piece);
+    if (piece >= bytes) return true;
+    const c10::DeviceGuard guard(c10::Device(c10::kCUDA, device));
+    size_t left = 0, all = 0;
+    if (hipMemGetInfo(&left, &all) != hipSuccess) return true;
+    const double share = allocator->getMemoryFraction(device) * (double)all -
+                         (double)allocator->getDeviceStats(device).reserved_bytes[0].current;
+    return left >= bytes + GRAIN && share >= (double)(bytes + GRAIN);
+  } catch (const c10::Error&) {
+    return true;
+  }
+}
+
+// The backward's: with room for what its kernels can hand on, or without it where the device has not that much left.  Asked for last, so that
+// nothing that the call cannot do without comes after it.
 Tensor scratch_for(HstuAttnBwdArgs& b, const Tensor& like) {
   const size_t ws = hstu_attn_bwd_workspace_bytes(&b);
   if (!ws) return Tensor();
   Tensor buf;
-  try {
-    buf = at::empty({(int64_t)ws}, like.options().dtype(at::kByte).requires_grad(false));
-  } catch (const c10::OutOfMemoryError&) {
+  if (has_room(like.device().index(), ws)) {
+    try {
+      buf = at::empty({(int64_t)ws}, like.options().dtype(at::kByte).requires_grad(false));
+    } catch (const c10::OutOfMemoryError&) {
+    }
+  }
+  if (!buf.defined()) {
     const uint32_t flags = b.fwd.flags;
     b.fwd.flags &= ~HSTU_BWD_WRITE_BIAS_GRADIENT;       // (the forward's question knows no flag of the backward's)
     buf = scratch_for(b.fwd, like);
@@ -1541,6 +1571,18 @@ PyObject* mask_lengths(PyObject*, PyObject* const* a, Py_ssize_t count) {
   });
 }
 
+// has_room(device index, bytes): whether a buffer that a call can do without should be asked for.
+PyObject* room(PyObject*, PyObject* const* a, Py_ssize_t count) {
+  if (count != 2) {
+    PyErr_SetString(PyExc_TypeError, "has_room takes 2 arguments");
+    return nullptr;
+  }
+  const long device = PyLong_AsLong(a[0]);
+  const long long bytes = PyLong_AsLongLong(a[1]);
+  if (PyErr_Occurred()) return nullptr;
+  return guarded([&]() -> PyObject* { return PyBool_FromLong(has_room((c10::DeviceIndex)device, (size_t)bytes)); });
+}
+
 PyMethodDef methods[] = {
     {"attention", (PyCFunction)(void (*)(void))attention, METH_FASTCALL,
      "One attention forward on arguments that are ready for the kernels; None when they are not."},
@@ -1553,6 +1595,7 @@ PyMethodDef methods[] = {
     HSTU_FAST(linear, "A matrix product with gradients."),
     HSTU_FAST(pack, "The packed form of a padded batch."),
     HSTU_FAST(mask_lengths, "Lengths of an end-padded batch from its mask."),
+    {"has_room", (PyCFunction)(void (*)(void))room, METH_FASTCALL, "Whether the device has room for a buffer that a call can do without."},
     {"raised", raised, METH_O, "Whether the kernel behind a ticket found what it looks for (waits for that kernel)."},
     {nullptr, nullptr, 0, nullptr},
 };

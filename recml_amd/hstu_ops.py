@@ -545,12 +545,17 @@ def hstu_attention_bwd(q, k, v, dout, *, seq_lens=None, seq_offsets=None, max_le
   lib = _lib.load()
   best = lib.hstu_attn_bwd_workspace_bytes(C.byref(ba))
   if best:
-    try:
-      buf = torch.empty(best, dtype=torch.uint8, device=q.device)
-      ba.fwd.workspace, ba.fwd.workspace_bytes = buf.data_ptr(), best
+    buf = None
+    if _native.has_room(q.get_device(), best) is not False:
+      try:
+        buf = torch.empty(best, dtype=torch.uint8, device=q.device)
+      except torch.OutOfMemoryError:
+        pass
+    fa = ba.fwd
+    if buf is not None:
+      fa.workspace, fa.workspace_bytes = buf.data_ptr(), best
       keep.append(buf)
-    except torch.OutOfMemoryError:     # (less than the best will do; the forward's question knows no flag of the backward's)
-      fa = ba.fwd
+    else:                              # (less than the best will do; the forward's question knows no flag of the backward's)
       flags, fa.flags = fa.flags, fa.flags & ~_lib.BWD_WRITE_BIAS_GRADIENT
       _attach_workspace(fa, keep)
       fa.flags = flags

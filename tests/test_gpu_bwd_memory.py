@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import recml_amd
+from recml_amd import _native
 
 pytestmark = pytest.mark.gpu
 MB = 1 << 20
@@ -12,6 +13,8 @@ MB = 1 << 20
 @pytest.fixture
 def share():
   """Leaves the process so many bytes beyond those it has; the whole device again afterwards."""
+  torch.cuda.synchronize()
+  torch.cuda.empty_cache()                # (so that the test's tensors have pieces of their own)
   total = torch.cuda.get_device_properties(0).total_memory
 
   def leave(n):
@@ -24,9 +27,9 @@ def share():
 
 
 def _inputs(B, L, H=8, d=128, dense=False):
-  g = torch.Generator(device="cuda").manual_seed(L)
-  t = [torch.randn(B, L, H, d, device="cuda", generator=g).mul_(0.5).to(torch.bfloat16) for _ in range(4)]
-  bias = torch.randn((B, L, L) if dense else (H, 2 * L - 1), device="cuda", generator=g) * 0.3
+  g = torch.Generator().manual_seed(L)      # (on the host, for the same reason)
+  t = [torch.randn(B, L, H, d, generator=g).mul_(0.5).to(torch.bfloat16).cuda() for _ in range(4)]
+  bias = (torch.randn((B, L, L) if dense else (H, 2 * L - 1), generator=g) * 0.3).cuda()
   return t, dict(bias=bias, n=float(L)) if dense else dict(pos_bias=bias)
 
 
@@ -56,9 +59,35 @@ def _failed():
   return s["num_alloc_retries"], s["num_ooms"]
 
 
+@pytest.mark.parametrize("native,left", [(True, 232), (False, 200)])
+def test_no_room_is_not_asked_for(gpu, share, native, left):
+  """What the caching allocator holds is not given back for a buffer that the call can do without: 32 MB for each of dq, dk, dv (and the output),
+  136 for dS."""
+  t, kw = _inputs(16, 1024)
+  want = _gradients(t, kw, native)
+  share(left * MB)
+  before = _failed()
+  got = _gradients(t, kw, native)
+  torch.cuda.synchronize()
+  assert _failed() == before
+  torch.cuda.set_per_process_memory_fraction(1.0)
+  _same(got, want)
+
+
+def test_room(gpu, share):
+  index = torch.cuda.current_device()
+  share(300 * MB)
+  assert _native.has_room(index, 280 * MB) and not _native.has_room(index, 310 * MB)
+  held = torch.empty(200 * MB, dtype=torch.uint8, device="cuda")
+  assert not _native.has_room(index, 200 * MB) and _native.has_room(index, 96 * MB) and _native.has_room(index, 63 * MB)
+  del held
+  assert _native.has_room(index, 200 * MB)              # (a piece that the allocator holds)
+  assert not _native.has_room(index, 203 * MB)
+
+
 @pytest.mark.parametrize("native,dense,left", [(True, False, 78), (False, False, 62), (True, True, 96), (False, True, 82)])
 def test_an_allocation_that_fails(gpu, share, native, dense, left):
-  """The call goes on without what there is no memory for, also with a dense bias's gradient (a flag of the backward's): 14 MB for each of dq, dk,
+  """Buffers below 64 MB are asked for without a look.  The call goes on without what there is no memory for, also with a dense bias's gradient (a flag of the backward's): 14 MB for each of dq, dk,
   dv (and the output), 20 for the bias's gradient, and the 38 or so of dS do not fit."""
   t, kw = _inputs(8, 768, dense=dense)
   want = _gradients(t, kw, native)
