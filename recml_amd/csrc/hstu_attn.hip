@@ -4678,12 +4678,14 @@ __device__ __forceinline__ uint32_t ds_block_off(const Params& p, int i, int j) 
 
 // Ring depth of the dK/dV kernel (see there).
 constexpr int dkv_stages(int d, bool dense_bias, bool wide) { return (d == 128 && !dense_bias && !wide) ? 6 : NSTAGE; }
-// Bytes of the dense operands in the dK/dV kernel's LDS (see there).
+// Whether a wave brings its own part of the dense operands, and their bytes in the dK/dV kernel's LDS (see there).
+constexpr bool dkv_own_dense(int d, bool dense_bias, bool ds_out) { return dense_bias && (d < 128 || ds_out); }
 constexpr int DKV_DB_STAGES = 2, DKV_DM_STAGES = 3;
 template <int D>
-constexpr int dkv_dense_bytes(bool mask, bool dense_bias, int nst) {
+constexpr int dkv_dense_bytes(bool mask, bool dense_bias, bool ds_out, int nst) {
   using SM = MfmaSmem<D, 2>;
-  return dense_bias ? DKV_DB_STAGES * SM::DB_BYTES + (mask ? DKV_DM_STAGES * SM::DM_BYTES : 0) : mask ? nst * SM::DM_BYTES : 0;
+  return dkv_own_dense(D, dense_bias, ds_out) ? DKV_DB_STAGES * SM::DB_BYTES + (mask ? DKV_DM_STAGES * SM::DM_BYTES : 0)
+                                              : nst * ((mask ? SM::DM_BYTES : 0) + (dense_bias ? SM::DB_BYTES : 0));
 }
 
 // WIDE (d = 128 without a dense bias, other than the stream's instance): eight waves, two per SIMD.  Waves w and w + 4
@@ -4727,12 +4729,14 @@ constexpr bool dkv_takes_turns(int d, bool pos, bool ts, bool mask, bool dense_b
 // its own 32 keys need (32 rows of 128 bytes, and 32 of the mask's) into bytes that no other wave reads: two stages for the bias,
 // whose 16 values a lane takes into registers ahead of its block, and three for the mask, read inside it.  They are refilled without
 // regard to the other waves, and the workgroup's LDS falls from 112 to 76 KB at d = 64, two workgroups per CU (16 x up to 1000, 8 heads of
-// 64, mask and bias: the kernel 108 -> 92 us).
+// 64, mask and bias: the kernel 108 -> 92 us).  At d = 128 without DSO the accumulators leave room for one workgroup whatever the LDS, and bias and
+// mask ride in the workgroup's ring (mask and bias with the bias's gradient, eight heads, 1 x 1000, the call: 214 us with a wave's own, 202 this way;
+// 1 x 300 59.7 and 56.5).
 // The bias's gradient is the other kernel's business.
 template <int D, bool POS, bool TS, bool SEG = false, bool MSK = false, bool DB = false, bool DSO = false, bool TG = false, bool CHAIN = false>
 __global__ __launch_bounds__((DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, DSO)>::THREADS), (D == 128 && !dkv_wide(D, POS, TS, SEG, MSK, DB, DSO) ? 1 : 2))
 void hstu_bwd_dkv_mfma(const Params p) {
-  constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO);
+  constexpr bool WIDE = dkv_wide(D, POS, TS, SEG, MSK, DB, DSO), OWN = dkv_own_dense(D, DB, DSO);
   using SH = DkvShape<D, WIDE>;
   constexpr int NW = SH::NW, THREADS = SH::THREADS;
   constexpr bool ACC_ASM = SH::ACC_ASM;
@@ -4752,7 +4756,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
   constexpr int DVB = D / 32;
   constexpr int NPIECE = SM::V_BYTES / 1024;
   constexpr int LD = NPIECE >= NW ? NPIECE / NW : 1;
-  constexpr int NDMA = 2 * LD + ((POS || TS) ? 1 : 0) + (SEG ? 1 : 0) + (MSK && !DB ? 1 : 0);
+  constexpr int NDMA = 2 * LD + ((POS || TS) ? 1 : 0) + (SEG ? 1 : 0) + (MSK && !OWN ? 1 : 0) + (DB && !OWN ? 4 : 0);
   // Ring depth: 4 stages (two pairs of steps: one at work, one on its way), or 6 where the workgroup has the CU's
   // LDS to itself anyway (d = 128) and the stages are small enough: the loads of a pair then have the time of two
   // pairs to arrive, which the hand-scheduled pairs need (one pair's time is less than a trip to memory).
@@ -4771,9 +4775,11 @@ void hstu_bwd_dkv_mfma(const Params p) {
   auto Qs = [&](int st) { return (bf16_t*)(smem + st * SM::STAGE); };
   auto Os = [&](int st) { return (bf16_t*)(smem + st * SM::STAGE + SM::K_BYTES); };
   constexpr int BIAS_OFF = NST * SM::STAGE;
-  constexpr int BIAS_STAGE = (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0) + (SEG ? SM::SEG_BYTES : 0) + (MSK && !DB ? SM::DM_BYTES : 0);
+  constexpr int BIAS_STAGE = (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0) + (SEG ? SM::SEG_BYTES : 0) + (MSK && !OWN ? SM::DM_BYTES : 0) +
+                             (DB && !OWN ? SM::DB_BYTES : 0);
   auto Sg = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0) + (TS ? TQ_BYTES : 0)); };
   auto Mk = [&](int st) { return smem + BIAS_OFF + st * BIAS_STAGE; };      // MSK (first in the stage): [32 rows][128 bytes]
+  auto Bk = [&](int st) { return smem + BIAS_OFF + st * BIAS_STAGE + (MSK ? SM::DM_BYTES : 0); };   // DB: [32 rows][128 floats]
   auto Wc = [&](int st) { return (float*)(smem + BIAS_OFF + st * BIAS_STAGE); };
   auto Tq = [&](int st) { return (int32_t*)(smem + BIAS_OFF + st * BIAS_STAGE + (POS ? SM::POS_BYTES : 0)); };
   const unsigned char* TsKey = smem + BIAS_OFF + NST * BIAS_STAGE;   // the keyed bucket table of this head
@@ -4927,7 +4933,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
         lds_dma16_at(p.q_seg + (int64_t)b * p.L, (uint32_t)g4 * 4u, smem_lds + (uint32_t)((const unsigned char*)Sg(st) - smem));
       }
     }
-    if (MSK && !DB) {
+    if (MSK && !OWN) {
       // rows 8w .. 8w + 7 of the step's mask tile, eight lanes per row (16 bytes each = this tile's 128 keys); rows past
       // L and pieces past Lkv re-read bytes inside the matrix (those pairs are masked by their index)
       const uint8_t* mg = (const uint8_t*)scalar_ptr(p.mask + (p.mask_batched ? (int64_t)b * p.L * p.mask_pitch : 0));
@@ -4937,8 +4943,20 @@ void hstu_bwd_dkv_mfma(const Params p) {
       col = col < p.mask_pitch - 16 ? col : p.mask_pitch - 16;
       lds_dma16(mg, (uint32_t)gr * (uint32_t)p.mask_pitch + (uint32_t)col, Mk(st) + w * 1024);
     }
+    if (DB && !OWN) {
+      // the bias's likewise, in four pieces of two rows (512 bytes a row)
+      const float* bg = (const float*)scalar_ptr(p.dense_bias + (p.dense_bias_batched ? (int64_t)b * p.L * p.bias_pitch : 0));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        int gr = qbs + 8 * w + 2 * r + (lane >> 5);
+        gr = gr < p.L - 1 ? gr : p.L - 1;
+        int col = kv0 + 4 * (lane & 31);
+        col = col < p.bias_pitch - 4 ? col : p.bias_pitch - 4;
+        lds_dma16(bg, ((uint32_t)gr * (uint32_t)p.bias_pitch + (uint32_t)col) * 4u, Bk(st) + (4 * w + r) * 1024);
+      }
+    }
   };
-  // DB: this wave's part of the dense operands of step t.  The bias's row 8g + 4 hh + tt stands in place 8g + 2 tt + hh, 128 bytes each, so that
+  // OWN: this wave's part of the dense operands of step t.  The bias's row 8g + 4 hh + tt stands in place 8g + 2 tt + hh, 128 bytes each, so that
   // the two halves of the wave read neighbouring rows; the mask's rows in their order, 32 bytes each.  Rows past L and pieces past Lkv
   // re-read values inside the matrix (those pairs are masked by their index).
   constexpr int DENSE_OFF = BIAS_OFF + NST * BIAS_STAGE;
@@ -4965,9 +4983,9 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
   };
   // (the empty statements make the compiler wait for the values here: behind them the bytes may be refilled)
-  float dbv[DB ? 16 : 1];
+  float dbv[OWN ? 16 : 1];
   auto dense_take = [&](int t) __attribute__((always_inline)) {
-    if constexpr (DB) {
+    if constexpr (OWN) {
       const float* const bcol = (const float*)own_bias(t) + 32 * hh + m;
 #pragma unroll
       for (int r = 0; r < 16; ++r) dbv[r] = bcol[(8 * (r >> 2) + 2 * (r & 3)) * 32];
@@ -4986,7 +5004,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i)
     if (t_lo + i < nt) dma_step(t_lo + i);
-  if constexpr (DB) {
+  if constexpr (OWN) {
     if (wave_live && t_lo < nt) dense_refill(t_lo);
     if (wave_live && t_lo + 1 < nt) dense_refill(t_lo + 1);
   }
@@ -5171,9 +5189,14 @@ void hstu_bwd_dkv_mfma(const Params p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) u[r] = sacc[r] * alpha2;
     }
-    if (DB) {
+    if constexpr (OWN) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) u[r] = __builtin_fmaf(dbv[r], LOG2E, u[r]);
+    } else if constexpr (DB) {
+      // the lane's column of the bias tile: row 8g + 4hh + tt at key 32w + m
+      const float* const bcol = (const float*)Bk(st) + 32 * w + m + (4 * hh) * BM;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) u[r] = __builtin_fmaf(bcol[(8 * (r >> 2) + (r & 3)) * BM], LOG2E, u[r]);
     }
     // (the table gradients, as in the dQ kernel: the lane's 16 pairs are in bucket bk_lane >= 0, those with a bit in
     // far_rows in the next one, or bkp has the 16 buckets)
@@ -5356,8 +5379,8 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
     if (MSK) {
       // the lane's column of the mask tile: byte of row 8g + 4hh + tt at key 32w + m
-      constexpr int PITCH = DB ? BN : BM;
-      const unsigned char* mcol = (DB ? own_mask(t) : Mk(st) + 32 * w) + m + (4 * hh) * PITCH;
+      constexpr int PITCH = OWN ? BN : BM;
+      const unsigned char* mcol = (OWN ? own_mask(t) : Mk(st) + 32 * w) + m + (4 * hh) * PITCH;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const bool keep = mcol[(8 * (r >> 2) + (r & 3)) * PITCH] != 0;
@@ -5573,7 +5596,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
     }
     const bool first = wave_live && t >= t_wave && t <= t_wave_end;
     const bool second = t + 1 < nt && wave_live && t + 1 >= t_wave && t + 1 <= t_wave_end;
-    if constexpr (DB) {
+    if constexpr (OWN) {
       if (first) dense_take(t);
       if (wave_live && t + 2 < nt) dense_refill(t + 2);
       if (first) block(t);
@@ -6526,7 +6549,7 @@ int launch_bwd_mfma_inst(const Params& p, hipStream_t st) {
   const int smem_q = smem + (TG ? BWD_TG_BYTES : 0);
   using SH = DkvShape<D, dkv_wide(D, POS, TS, SEG, MSK, DB, false)>;
   constexpr int nst_kv = dkv_stages(D, DB, dkv_wide(D, POS, TS, SEG, MSK, DB, false));
-  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + dkv_dense_bytes<D>(MSK, DB, nst_kv) +
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst_kv) + dkv_dense_bytes<D>(MSK, DB, false, nst_kv) +
                       SH::KV_LDS + (TS ? nst_kv * 16 : 0);     // one more 16-byte piece of timestamp operands per stage
   static int granted_q[64], granted_kv[2][64];
   const bool chain = dkv_takes_turns(D, POS, TS, MSK, DB) && p.chain_bound;
@@ -6554,7 +6577,7 @@ int launch_bwd_kept(const Params& p, hipStream_t st) {
   constexpr bool wide = dkv_wide(D, POS, TS, SEG, MSK, DB, true);
   using SH = DkvShape<D, wide>;
   constexpr int nst = dkv_stages(D, DB, wide);
-  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + dkv_dense_bytes<D>(MSK, DB, nst) +
+  const int smem_kv = MfmaSmem<D, 2>::total(POS, TS, SEG, 0, nst) + dkv_dense_bytes<D>(MSK, DB, true, nst) +
                       SH::KV_LDS + (TS ? nst * 16 : 0) + (TG ? DkvTg<wide>::BYTES : 0);
   const auto kv = hstu_bwd_dkv_mfma<D, POS, TS, SEG, MSK, DB, true, TG>;
   const auto dq = hstu_bwd_dq_ds<D, MSK>;
