@@ -1,4 +1,4 @@
-"""The dense bias's gradient of long rows, which has a kernel of its own, against the fp32 kernels on the same values."""
+"""The dense bias's gradient, which has a kernel of its own where there are tiles enough, against the fp32 kernels on the same values."""
 
 import pytest
 import torch
@@ -35,8 +35,14 @@ def _call(B, L, H, d, kind, seed=0):
     (3, 1024, 2, 128, "mask"),           # two stages a head
     (12, 520, 2, 32, "lengths"),
     (5, 900, 3, 64, "window"),           # with dropout
-    (12, 512, 1, 64, "full"),            # the smallest that has it
+    (12, 512, 1, 64, "full"),
     (1, 1800, 2, 128, "shared"),
+    # short rows of many sequences: one step, less than a tile, odd lengths
+    (64, 30, 2, 64, "mask"), (64, 31, 2, 128, "lengths"), (100, 17, 1, 32, "window"),
+    (64, 100, 2, 32, "lengths"), (40, 97, 2, 128, "mask"), (33, 127, 2, 64, "window"),
+    (16, 201, 3, 64, "window"), (12, 267, 2, 128, "mask"), (16, 155, 4, 32, "full"),
+    (14, 150, 3, 64, "lengths"), (13, 150, 3, 64, "lengths"),              # 28 tiles of 128 x 64 a head, and less: added by the dQ kernel
+    (64, 60, 1, 128, "mask"), (63, 60, 1, 128, "mask"),                  # 64 tiles, and less
 ])
 def test_against_fp32(gpu, B, L, H, d, kind):
   """Both form S and dP from the same values in fp32 sums of d terms and add H of their products in fp32: relative differences of some
@@ -51,7 +57,12 @@ def test_against_fp32(gpu, B, L, H, d, kind):
   diff = (got - want).double()
   assert float(diff.norm()) <= 1e-5 * float(want.double().norm())
   assert float(diff.abs().max()) <= 2.0**-15 * float(want.abs().max())
-  assert torch.equal(got, recml_amd.hstu_attention_bwd(q, k, v, dout, bias_grad=True, **kw)[5])
+  again = recml_amd.hstu_attention_bwd(q, k, v, dout, bias_grad=True, **kw)[5]
+  tiles = B * ((L + 127) // 128) * ((L + 63) // 64)
+  if tiles >= max(64, 28 * H):
+    assert torch.equal(got, again)
+  else:      # (the dQ kernel's additions come in any order: H - 1 roundings of at most the terms' magnitudes' sum on either side)
+    assert float((got - again).abs().max()) <= 2 * H * 2.0**-24 * H * float(got.abs().max())
 
 
 @pytest.mark.parametrize("B,L", [(12, 520), (2, 200)])
