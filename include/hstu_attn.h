@@ -267,8 +267,8 @@ int hstu_attn_fwd_noalloc(const HstuAttnFwdArgs* args, void* stream);
 
 /* Backward of the same op: gradients of sum(out * dout) with respect to q, k, v
  * and the two bias tables.  `fwd` describes the forward call (its `out` is
- * not used; its `workspace`, sized by hstu_attn_fwd_workspace_bytes, is
- * overwritten when the matrix-core kernels run, see below).  dout has the
+ * not used; its `workspace`, 256-byte aligned, of hstu_attn_bwd_workspace_bytes
+ * or at the least hstu_attn_fwd_workspace_bytes, is overwritten, see below).  dout has the
  * layout, dtype and strides of out;
  * dq, dk, dv those of q, k, v and are fully written (rows past a sequence's
  * length as zeros).  dpos_tab / dts_tab are fp32 tables shaped like pos_tab /
@@ -280,8 +280,8 @@ int hstu_attn_fwd_noalloc(const HstuAttnFwdArgs* args, void* stream);
  * at most 4096 entries.)  fp32 or bf16
  * storage, every option of the forward, fp32 arithmetic; fp8 q/k is not
  * supported.  bf16 calls that meet the conditions of the
- * matrix-core forward (without a dense mask or bias, and with keys and
- * queries of one length), pass 16-byte aligned gradient buffers and bring
+ * matrix-core forward (a dense mask or bias among them) with keys and
+ * queries of one length, pass 16-byte aligned gradient buffers and bring
  * the workspace run on the matrix cores instead (bf16 products, fp32
  * accumulation, table gradients included); every other bf16 call whose head
  * dims are multiples of 16 up to 128 and whose q, k, v, dout rows lie on

@@ -4715,7 +4715,9 @@ constexpr bool dkv_wide(int d, bool pos, bool ts, bool seg, bool mask, bool dens
 
 // Forms in which, without DSO, the vector part stands between the products, us for the call: heads of 64 without a table, 64 x 2048
 // 1401 -> 1354, 128 x up to 1024 470 -> 454, with segment ids 965 -> 895; heads of 32 with both tables, 64 x 2048 1998 -> 1832, 192 x up to
-// 1024 942 -> 867.  (Heads of 64 with the position table 496 and 496, of 32 with timestamps alone 716 and 741; the others were not tried.)
+// 1024 942 -> 867.  The other forms with the tables frozen, dS formed twice, 64 x 2048 / 128 x up to 1024: heads of 64 with positions 1481 ->
+// 1493 / 382 -> 384, timestamps 1820 -> 1811 / 517 -> 514, both 2029 -> 2032 / 583 -> 581; heads of 32 without a table 1010 -> 1017 / 239 -> 243, with
+// segment ids 1080 -> 1070 / 640 -> 621, positions 1090 -> 1076 / 262 -> 260, timestamps 1291 -> 1341 / 349 -> 365.
 // It lengthens a step, though: calls whose longest tile ends last keep the other order.  4 x 2048, four heads of 64: 116 and 125; 2 x 8192,
 // two heads: 404 and 441; 16 x up to 4096 of power-law length, eight heads of 32 with both tables: 331 and 348.
 constexpr bool dkv_takes_turns(int d, bool pos, bool ts, bool mask, bool dense_bias) {
@@ -5114,7 +5116,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
       two_buckets = __builtin_amdgcn_ballot_w64(!en.two) == 0;
     }
     floatx16 sacc, dpacc;
-    // WOVEN: product j, S for j < QCH, then dP; its fragments are asked for two products ahead (left to itself the compiler has no
+    // WOVEN: product j, S for j < QCH, then dP; its fragments are asked for AHEAD_R products ahead (left to itself the compiler has no
     // registers for more than the next one, and every product waits for LDS), the order is fixed by scheduling barriers.  WIDE: row m of
     // each tile against row 32 w + m of the keys'.
     uint4 af[WOVEN ? AHEAD_R + 1 : 1], bf[WIDE ? AHEAD_R + 1 : 1];
@@ -5394,7 +5396,7 @@ void hstu_bwd_dkv_mfma(const Params p) {
                                (uint32_t)(qbs + 4 * hh) * DROP_CI, DROP_CI, p.drop_thr);
     }
     if constexpr (WOVEN) {
-      // The accumulating products, dV and dK in turn, their fragments two products ahead; between them the tables' gradients: the diagonal
+      // The accumulating products, dV and dK in turn, their fragments AHEAD_T products ahead; between them the tables' gradients: the diagonal
       // sums in the first half, the bucket sums (a near one and a far one, see the dQ kernel) throughout.
       uint4 pk[2], dk4[2], tf[AHEAD_T + 1];
 #pragma unroll
