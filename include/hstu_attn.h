@@ -322,8 +322,8 @@ int hstu_attn_bwd_silu(const HstuAttnBwdArgs* args, const void* q_pre, const voi
  * calls, with dense operands too; fp32 calls of head dims of 32, 64 and 128) room for the logits' gradients, which the dK/dV kernel then leaves
  * for the one that forms dQ: 2 bytes (fp32: 4) for each pair of a head in blocks of 32 x 32 (16 x 16) on and below the diagonal, in all
  * without the causal mask, or in the window's band; up to 4 GiB, and none beyond.  With less, down to hstu_attn_fwd_workspace_bytes, each of the two kernels forms
- * them: the same results up to the rounding and the order of fp32 operations, and the same bits from run to run either way.  From shapes and
- * options only, like the other. */
+ * them: the same results up to the rounding and the order of fp32 operations, and the same bits of dq, dk and dv from run to run either way.
+ * From shapes, options and which gradients are asked for (their addresses set or null). */
 size_t hstu_attn_bwd_workspace_bytes(const HstuAttnBwdArgs* args);
 
 /* Name of the kernel pair hstu_attn_bwd would launch for `args` (diagnostics;

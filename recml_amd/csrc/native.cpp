@@ -45,6 +45,11 @@ void* stream_of(const Tensor& t) {
   return (void*)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
+bool capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // ---------------------------------------------------------------------------
 // arguments
 // ---------------------------------------------------------------------------
@@ -263,6 +268,7 @@ bool has_room(c10::DeviceIndex device, size_t bytes) {
     size_t piece = 1;
     allocator->cacheInfo(device, &piece);
     if (piece >= bytes) return true;
+    if (capturing((void*)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream())) return true;      // (nothing else is asked of the runtime then)
     const c10::DeviceGuard guard(c10::Device(c10::kCUDA, device));
     size_t left = 0, all = 0;
     if (hipMemGetInfo(&left, &all) != hipSuccess) return true;
@@ -1348,11 +1354,6 @@ PyObject* raised(PyObject*, PyObject* ticket) {
     Py_END_ALLOW_THREADS
     return PyBool_FromLong(value != 0);
   });
-}
-
-bool capturing(void* stream) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
 // Whether hstu_mask_lengths reads this mask as it is.

@@ -100,6 +100,29 @@ def test_an_allocation_that_fails(gpu, share, native, dense, left):
   _same(got, want)
 
 
+def test_captured(gpu):
+  """A backward whose scratch is large enough to be looked for, in a graph: every replay as the call itself."""
+  t, kw = _inputs(16, 1024)
+  want = _gradients(t, kw, False)
+  side = torch.cuda.Stream()
+  side.wait_stream(torch.cuda.current_stream())
+  with torch.cuda.stream(side):
+    _gradients(t, kw, False)
+  torch.cuda.current_stream().wait_stream(side)
+  torch.cuda.empty_cache()                # (no piece of that size to be found)
+  graph = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(graph):
+    got = _gradients(t, kw, False)
+  for _ in range(3):
+    for x in got:
+      x.fill_(7.0)
+    graph.replay()
+    torch.cuda.synchronize()
+    _same(got, want)
+    t[0].mul_(-1.0)
+    want = _gradients(t, kw, False)
+
+
 @pytest.mark.parametrize("wanted", [True, False])
 def test_a_block_asks_for_what_its_attention_takes(gpu, wanted):
   """Heads of 64 with a position table: whether dS is handed on goes by whether the table's gradient is wanted, so a block asks once all of
